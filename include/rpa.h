@@ -313,6 +313,13 @@ RPA_API int rpa_attention_noalloc(const RpaParams* p, void* stream);
  */
 RPA_API int rpa_kv_write(const RpaParams* p, const void* keys, const void* values, void* stream);
 
+/*
+ * rpa_kv_write and rpa_attention as one call: ragged_paged_attention as the reference's layers call it
+ * (ragged_paged_attention_v3.py:1667-2097 writes the new tokens and attends to them in one kernel).  keys / values:
+ * [T, Hkv, D] in the cache dtype, or both NULL when the cache already holds every token.
+ */
+RPA_API int rpa_attention_update(const RpaParams* p, const void* keys, const void* values, void* stream);
+
 /* Absorbed-MLA decode, see RpaMlaParams: every sequence contributes exactly one query token. */
 RPA_API int rpa_mla_decode(const RpaMlaParams* p, void* stream);
 
@@ -335,6 +342,13 @@ RPA_API int rpa_mla_describe_plan(const RpaMlaParams* p, int token_rows, char* b
  * [T, rope_dim]; token j of sequence i goes to position kv_len_i - q_len_i + j.
  */
 RPA_API int rpa_mla_kv_write(const RpaMlaParams* p, const void* new_kv_c, const void* new_k_pe, void* stream);
+
+/*
+ * rpa_mla_kv_write and rpa_mla_decode (token_rows = 0) or rpa_mla_attention (token_rows = 1) as one call; the new rows
+ * may both be NULL when the cache already holds every token.
+ */
+RPA_API int rpa_mla_attention_update(const RpaMlaParams* p, const void* new_kv_c, const void* new_k_pe, int token_rows,
+                             void* stream);
 
 #ifdef __cplusplus
 }

@@ -11,6 +11,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "librpa_mi355.so")
+TORCH_LIB_PATH = os.path.join(_HERE, "lib", "rpa_torch.so")
 
 RPA_KV_BF16 = 0
 RPA_KV_FP8_E4M3 = 1
@@ -54,6 +55,8 @@ EXPORTED_SYMBOLS = (
     "rpa_mla_attention",
     "rpa_mla_kv_write",
     "rpa_mla_describe_plan",
+    "rpa_attention_update",
+    "rpa_mla_attention_update",
 )
 
 
@@ -195,12 +198,37 @@ def load() -> ctypes.CDLL:
     lib.rpa_mla_attention.argtypes = [P(RpaMlaParams), ctypes.c_void_p]
     lib.rpa_mla_kv_write.restype = ctypes.c_int
     lib.rpa_mla_kv_write.argtypes = [P(RpaMlaParams), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+    lib.rpa_attention_update.restype = ctypes.c_int
+    lib.rpa_attention_update.argtypes = [P(RpaParams), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+    lib.rpa_mla_attention_update.restype = ctypes.c_int
+    lib.rpa_mla_attention_update.argtypes = [P(RpaMlaParams), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p]
     lib.rpa_describe_plan.restype = ctypes.c_int
     lib.rpa_describe_plan.argtypes = [P(RpaParams), ctypes.c_char_p, ctypes.c_size_t]
     lib.rpa_mla_describe_plan.restype = ctypes.c_int
     lib.rpa_mla_describe_plan.argtypes = [P(RpaMlaParams), ctypes.c_int, ctypes.c_char_p, ctypes.c_size_t]
     _lib = lib
     return lib
+
+
+_torch = None
+
+
+def load_torch():
+    """The native host path of the operators (csrc/rpa_torch.cpp), built next to the library."""
+    global _torch
+    if _torch is None:
+        import importlib.machinery
+        import importlib.util
+
+        load()
+        if not os.path.exists(TORCH_LIB_PATH):
+            raise RpaLibraryMissing(
+                f"{TORCH_LIB_PATH} not found: build it with `python sglang-jax_amd/build.py` (or __graft_entry__.build())")
+        loader = importlib.machinery.ExtensionFileLoader("rpa_torch", TORCH_LIB_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("rpa_torch", loader))
+        loader.exec_module(module)
+        _torch = module
+    return _torch
 
 
 class RpaError(ValueError):

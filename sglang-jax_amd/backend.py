@@ -27,6 +27,7 @@ from dataclasses import dataclass, field
 import numpy as np
 import torch
 
+from . import _lib
 from .mla import mla_ragged_paged_attention
 from .ragged_paged_attention import ragged_paged_attention
 
@@ -313,6 +314,18 @@ class FlashAttention:
         elif hasattr(token_to_kv_pool, "remap_cache_loc") and self.page_size == 1:
             page_indices = token_to_kv_pool.remap_cache_loc(page_indices, layer.layer_id)
         xai = getattr(layer, "xai_temperature_len", -1)
+        xai = xai if xai is not None and xai > 0 else None
+        soft_cap = getattr(layer, "logit_cap", None) or None
+        softmax_dtype = getattr(layer, "softmax_dtype", None)
+        if causal or md.custom_mask is None:
+            out = _lib.load_torch().attention(
+                q, k, v, kv_cache_fused, md.seq_lens, page_indices, md.cu_q_lens, md.cu_kv_lens, md.host_distribution,
+                attention_sink, causal, scale, window, soft_cap, None, None, None, None, xai, softmax_dtype, None,
+                md.max_kv_len, md.max_q_len, 0, md.host_seq_lens, head_dim)
+            if out is not None:
+                if type(out) is int:
+                    _lib.check(out)
+                return out if out.dim() == 2 else out.reshape(out.shape[0], -1), kv_cache_fused
         T = q.shape[0]
         out, cache = ragged_paged_attention(
             q.reshape(T, -1, head_dim),
@@ -329,9 +342,9 @@ class FlashAttention:
             causal=causal,
             sm_scale=scale,
             sliding_window=window,
-            soft_cap=getattr(layer, "logit_cap", None) or None,
-            xai_temperature_len=xai if xai is not None and xai > 0 else None,
-            softmax_dtype=getattr(layer, "softmax_dtype", None),
+            soft_cap=soft_cap,
+            xai_temperature_len=xai,
+            softmax_dtype=softmax_dtype,
             max_kv_len=md.max_kv_len,
             max_q_len=md.max_q_len,
             host_kv_lens=md.host_seq_lens,

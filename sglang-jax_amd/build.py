@@ -23,6 +23,10 @@ SOURCES = ["rpa_capi.hip", "rpa_decode.hip", "rpa_prefill.hip", "rpa_prefill_pip
 CEILINGS_SOURCE = "rpa_ceilings.hip"
 CEILINGS_LIB_PATH = os.path.join(OUT_DIR, "librpa_ceilings.so")
 
+# the host path of the Python operators (argument reading, output, launch): CPU code only, against torch's headers
+TORCH_SOURCE = "rpa_torch.cpp"
+TORCH_LIB_PATH = os.path.join(OUT_DIR, "rpa_torch.so")
+
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950",
@@ -63,6 +67,21 @@ def source_hash() -> str:
     return h.hexdigest()
 
 
+def torch_command(out: str) -> list:
+    """How rpa_torch.so is compiled and linked against torch and the attention library (found next to it)."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    return ["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(x for d in inc for x in ("-isystem", d)),
+            os.path.join(CSRC, TORCH_SOURCE), "-o", out, "-L" + OUT_DIR, "-l:" + os.path.basename(LIB_PATH),
+            "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10", "-Wl,-rpath,$ORIGIN"]
+
+
 def build(verbose: bool = False, extra_flags=()) -> str:
     os.makedirs(OUT_DIR, exist_ok=True)
     objs = []
@@ -81,6 +100,9 @@ def build(verbose: bool = False, extra_flags=()) -> str:
         tmp = path + ".tmp"
         _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *members, "-o", tmp])
         os.replace(tmp, path)
+    tmp = TORCH_LIB_PATH + ".tmp"
+    _run(torch_command(tmp))
+    os.replace(tmp, TORCH_LIB_PATH)
     objs.append(ceil_obj)
     if not extra_flags:
         with open(HASH_PATH, "w") as f:

@@ -820,6 +820,14 @@ int rpa_kv_write(const RpaParams* p, const void* keys, const void* values, void*
   return check_hip(rpa::launch_kv_write(a, static_cast<hipStream_t>(stream)), "rpa_kv_write");
 }
 
+int rpa_attention_update(const RpaParams* p, const void* keys, const void* values, void* stream) {
+  if (keys || values) {
+    const int rc = rpa_kv_write(p, keys, values, stream);
+    if (rc != RPA_OK) return rc;
+  }
+  return rpa_attention(p, stream);
+}
+
 // ---------------------------------------------------------------- MLA ----
 
 static int mla_wgs();
@@ -1025,6 +1033,15 @@ int rpa_mla_kv_write(const RpaMlaParams* p, const void* new_kv_c, const void* ne
   a.row_stride = p->row_stride;
   a.rope_offset = p->rope_offset;
   return check_hip(rpa::launch_mla_kv_write(a, static_cast<hipStream_t>(stream)), "rpa_mla_kv_write");
+}
+
+int rpa_mla_attention_update(const RpaMlaParams* p, const void* new_kv_c, const void* new_k_pe, int token_rows,
+                             void* stream) {
+  if (new_kv_c || new_k_pe) {
+    const int rc = rpa_mla_kv_write(p, new_kv_c, new_k_pe, stream);
+    if (rc != RPA_OK) return rc;
+  }
+  return mla_run(p, stream, token_rows != 0);
 }
 
 }  // extern "C"

@@ -55,6 +55,14 @@ def mla_ragged_paged_attention(
     ``new_kv_c`` / ``new_k_pe`` may be None when the cache already holds all ``kv_len``
     tokens.  A decode batch (``distribution = (n, n, n)``) takes the one-row-per-sequence
     entry point; anything else (prefill chunks, mixed) runs one row per query token."""
+    native = _lib.load_torch().mla(
+        ql_nope, q_pe, new_kv_c, new_k_pe, cache_kv, kv_lens, page_indices, cu_q_lens, cu_kv_lens, distribution, sm_scale,
+        sliding_window, soft_cap, mask_value, q_scale, k_scale, v_scale, max_kv_len, num_splits, sum_kv_len)
+    if native is not None:
+        if type(native) is int:
+            _lib.check(native)
+        return native, cache_kv if cache_kv.dim() == 3 else cache_kv.view(cache_kv.shape[0], -1, cache_kv.shape[3])
+    # anything but the common form of a call: conversions, and the words of what is wrong
     _require_gpu(ql_nope, "ql_nope")
     _require_gpu(cache_kv, "cache_kv")
     if ql_nope.dim() != 3:
@@ -157,7 +165,7 @@ def mla_ragged_paged_attention(
         _lib.check(lib.rpa_mla_kv_write(ctypes.byref(p), nk.data_ptr(), nr.data_ptr(), stream))
     need = (lib.rpa_mla_workspace_bytes if decode_only else lib.rpa_mla_attention_workspace_bytes)(ctypes.byref(p))
     if need:
-        ws = _workspace(device, need)
+        ws = _workspace(ql_nope, need)
         p.workspace = ws.data_ptr()
         p.workspace_bytes = ws.numel()
     _lib.check((lib.rpa_mla_decode if decode_only else lib.rpa_mla_attention)(ctypes.byref(p), stream))

@@ -31,17 +31,10 @@ from ._lib import RpaParams
 # rpa_v3:47
 DEFAULT_MASK_VALUE = -0.7 * float(np.finfo(np.float32).max)
 
-_workspaces: dict = {}
 
-
-def _workspace(device, nbytes: int) -> torch.Tensor:
-    """Grow-only scratch for the split-KV partials, one per device and stream."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
+def _workspace(tensor, nbytes: int) -> torch.Tensor:
+    """Grow-only scratch for the split-KV partials, one per device and stream (of ``tensor``'s device)."""
+    return _lib.load_torch().workspace(tensor, nbytes)
 
 
 def _ptr(t):
@@ -315,7 +308,7 @@ class RpaCall:
         self.workspace = None
         if need:
             self.workspace = (torch.empty(need, dtype=torch.uint8, device=self.device) if own_workspace
-                              else _workspace(self.device, need))
+                              else _workspace(queries, need))
             p.workspace = self.workspace.data_ptr()
             p.workspace_bytes = self.workspace.numel()
         self.params = p
@@ -398,6 +391,16 @@ def ragged_paged_attention(
     bound) and the kernels read the batch composition themselves, as the jitted reference does
     (rpa_v3:1676): one prepared call serves every batch of a bucket.
     """
+    if out_dtype in (None, torch.bfloat16) and not (skip_kv_mask or validate_values) and (causal or custom_mask is None):
+        out = _lib.load_torch().attention(
+            queries, keys, values, kv_cache_fused, kv_lens, page_indices, cu_q_lens, cu_kv_lens, distribution,
+            attention_sink, causal, sm_scale, sliding_window, soft_cap, mask_value, q_scale, k_scale, v_scale,
+            xai_temperature_len, softmax_dtype, chunk_prefill_size, max_kv_len, max_q_len, num_splits, host_kv_lens, 0)
+        if out is not None:
+            if type(out) is int:
+                _lib.check(out)
+            return out, kv_cache_fused
+    # anything but the common form of a call: conversions, and the words of what is wrong
     _require_gpu(queries, "queries")
     _require_gpu(kv_cache_fused, "kv_cache_fused")
     device = queries.device
