@@ -39,6 +39,7 @@ const Tuning& tuning() {
   geti("RPA_DECODE_WAVES_PER_WG", t.decode_waves_per_wg);
   geti("RPA_DECODE_WAVE_CAPACITY", t.decode_wave_capacity);
   geti("RPA_DECODE_MERGE_IN_KERNEL", t.decode_merge_in_kernel);
+  geti("RPA_DECODE_LDS_KB", t.decode_lds_kb);
   geti("RPA_MASK_BITS", t.mask_bits);
   geti("RPA_PREFILL_ROWS256", t.prefill_rows256);
   geti("RPA_PREFILL_STAGED", t.prefill_staged);
@@ -227,6 +228,23 @@ int decode_waves_per_wg(const RpaParams* p);
 int decode_wgs(const RpaParams* p);
 int64_t decode_kv_bytes(const RpaParams* p);
 
+// Whether the fixed plan's pieces come out even enough.  Its launch starts streaming about 4 us earlier than the balanced
+// one (no prefix sum, no piece to look up), but what its pieces leave uneven is lost: with one piece per slot at best
+// (72 MB), on rows of nearly one length (mean at least 0.7 of the longest), or cut finely (24 pieces), the start wins.
+// 128 rows of 256..512 tokens x 2 heads 25.0 -> 19.0 us, 16 x 1024 x 8 heads 23.9 -> 18.5, 16 x 2048..16384 x 2 heads
+// 39.2 -> 35.3; beyond: 16 x 512..4096 x 8 heads 40.2 balanced against 47.8.
+bool fixed_is_even(const RpaParams* p, const SplitPlan& fixed) {
+  const int64_t bytes = decode_kv_bytes(p);
+  if (bytes <= (72ll << 20)) return true;
+  // many short rows, none of them cut: the dispatcher evens them out, and nothing is left to merge (250 rows of 100..200
+  // tokens x 8 heads 42.5 -> 32.3 us, 500 x 200..400 x 2 heads 43.8 -> 32.7; rows of up to 600 tokens about level)
+  if (fixed.splits <= 1 && (int64_t)p->max_kv_len * 2 * p->head_dim * esize_of(p->kv_dtype) <= (256ll << 10) && p->max_kv_len > 0)
+    return true;
+  if (p->sliding_window > 0 || p->sum_decode_kv_len <= 0 || p->max_kv_len <= 0) return false;
+  if (fixed.splits >= 24 && bytes <= (256ll << 20)) return true;
+  return bytes <= (128ll << 20) && p->sum_decode_kv_len * 10 >= (int64_t)p->decode_end * p->max_kv_len * 7;
+}
+
 bool use_balanced(const RpaParams* p, const SplitPlan& fixed) {
   if (!decode_balanced()) return false;
   if (p->num_splits == 1) return false;  // the caller asked for whole rows: one launch, no merge pass
@@ -236,6 +254,7 @@ bool use_balanced(const RpaParams* p, const SplitPlan& fixed) {
   // (128 rows of 128..4096 tokens: 228 -> 205 us, 200 rows of 1000..3000: 351 -> 295 us).
   if (fixed.splits <= 1 && decode_kv_bytes(p) < (64ll << 20)) return false;
   if (p->num_splits > 0) return true;
+  if (fixed_is_even(p, fixed)) return false;
   // too little work to hand every workgroup its minimum piece: latency-bound, keep the launch count low
   const int64_t bound = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages,
                                      p->cu_kv_lens != nullptr);
@@ -290,6 +309,12 @@ int decode_wave_capacity(const RpaParams* p) {
   const int cus = wave_capacity() / 8;
   const int nw = decode_waves_per_wg(p);
   return std::max(nw, cus * decode_shape(p).resident_x8 / 8 / nw * nw);
+}
+
+// Waves of a workgroup of the fixed plan: two up to 256 MB (its pieces spread over more CUs), else the shape table's.
+int decode_fixed_waves(const RpaParams* p) {
+  const int nw = decode_waves_per_wg(p);
+  return rpa::tuning().decode_waves_per_wg > 0 || decode_kv_bytes(p) >= (256ll << 20) ? nw : std::min(nw, 2);
 }
 
 int decode_wgs(const RpaParams* p) { return std::max(1, decode_wave_capacity(p) / decode_waves_per_wg(p)); }
@@ -355,6 +380,9 @@ int rows256(const RpaParams* p, int seq_begin, int seq_end, void* stream, int di
 }
 
 }  // namespace
+
+constexpr int kTokenRows = 64;                  // query tokens
+constexpr int64_t kTokenRowBytes = 64ll << 20;  // what they read, every token its whole row
 
 // ---- rpa_attention_noalloc: the split-KV workspace as a static device array ----
 // Every GPU the library is loaded on holds one copy of the array until the process ends.
@@ -514,6 +542,8 @@ std::atomic<unsigned long long> g_decode_generation{1};
 }  // namespace
 
 static size_t prefill_optional_workspace(const RpaParams* p);
+static bool takes_token_rows(const RpaParams* p);
+static size_t token_row_workspace(const RpaParams* p);
 
 // What the decode partition cannot run without.
 static size_t required_workspace_bytes(const RpaParams* p_in) {
@@ -531,7 +561,8 @@ static size_t required_workspace_bytes(const RpaParams* p_in) {
 
 size_t rpa_workspace_bytes(const RpaParams* p) {
   if (!p) return 0;
-  return std::max(required_workspace_bytes(p), prefill_optional_workspace(p));
+  const size_t need = std::max(required_workspace_bytes(p), prefill_optional_workspace(p));
+  return takes_token_rows(p) ? std::max(need, token_row_workspace(p)) : need;
 }
 
 int rpa_gather_pages(const RpaParams* p, int32_t seq, void* k_out, void* v_out, int32_t max_tokens,
@@ -553,16 +584,45 @@ int rpa_gather_pages(const RpaParams* p, int32_t seq, void* k_out, void* v_out, 
   return check_hip(rpa::launch_gather(a, static_cast<hipStream_t>(stream)), "rpa_gather_pages");
 }
 
-int rpa_decode(const RpaParams* p_in, void* stream) {
-  int rc = rpa_validate(p_in);
-  if (rc != RPA_OK) return rc;
-  const RpaParams pv = planning_view(p_in);
+// The row kernels' view of a call whose query tokens are all rows of their own.
+static RpaParams token_row_view(const RpaParams* p) {
+  RpaParams q = *p;
+  q.decode_end = p->num_tokens;
+  q.sum_decode_kv_len = 0;
+  q.num_splits = 0;
+  return q;
+}
+
+// Whether a call that may hold chunks runs with a row per query token on the decode kernels: a few tokens on short
+// contexts, where what counts is launches (cache write, decode rows, their merge, chunks, their merge: 5 x 3 us of host
+// time against 2) and not that a chunk's prefix is read once per token.  (RPA_PREFILL_SPLITS asks for the prefill kernels.)
+static bool takes_token_rows(const RpaParams* p) {
+  if (p->head_dim != 128 || p->mask_mode != RPA_MASK_CAUSAL || p->num_splits > 0 || p->num_tokens <= 0 ||
+      p->num_tokens > kTokenRows || rpa::tuning().prefill_splits >= 0 || (!p->distribution && p->num_seqs <= p->decode_end))
+    return false;
+  const RpaParams v = token_row_view(p);
+  return decode_kv_bytes(&v) <= kTokenRowBytes;
+}
+static size_t token_row_workspace(const RpaParams* p) {
+  const RpaParams v = token_row_view(p);
+  const SplitPlan sp = decode_plan(&v);
+  return sp.splits <= 1 ? 0 : (size_t)v.decode_end * sp.splits * v.num_q_heads * (v.head_dim + 2) * sizeof(float);
+}
+
+// Decode rows; with keys / values the rows' own tokens are not in the cache yet and are written by these kernels.
+// token_rows: every query token of the call is a row (takes_token_rows).
+static int decode_rows(const RpaParams* p_in, const void* keys, const void* values, bool token_rows, void* stream) {
+  const RpaParams pv = token_rows ? token_row_view(p_in) : planning_view(p_in);
   const RpaParams* p = &pv;
   if (p->decode_end <= 0) return RPA_OK;
   if (p->mask_mode == RPA_MASK_CUSTOM) return RPA_OK;  // masked rows all go through the prefill kernel
   if (p->head_dim == 256) return rows256(p, 0, p->decode_end, stream, p->distribution ? 1 : 0);
   const SplitPlan sp = decode_plan(p);
   rpa::DecodeArgs a;
+  a.new_k = static_cast<const char*>(keys);
+  a.new_v = static_cast<const char*>(values);
+  a.token_rows = token_rows ? 1 : 0;
+  a.num_seqs = p->num_seqs;
   a.q = static_cast<const uint16_t*>(p->q);
   a.out = static_cast<uint16_t*>(p->out);
   a.kv = kv_addr(p);
@@ -583,9 +643,9 @@ int rpa_decode(const RpaParams* p_in, void* stream) {
   a.merge_counters = nullptr;
   a.generation = 0;
   a.dist = p->distribution;
-  a.balanced = use_balanced(p, sp) ? 1 : 0;
+  a.balanced = (!token_rows && use_balanced(p, sp)) ? 1 : 0;
   a.num_wgs = decode_wgs(p);
-  a.waves_per_wg = decode_waves_per_wg(p);
+  a.waves_per_wg = a.balanced ? decode_waves_per_wg(p) : decode_fixed_waves(p);
   a.min_blocks_per_wave = std::max(1, rpa::tuning().decode_min_chunk / 32);
   a.forced_blocks_per_wave = 0;
   if (p->num_splits > 0) {  // the caller pins the partition: about num_splits pieces for the longest row
@@ -613,13 +673,18 @@ int rpa_decode(const RpaParams* p_in, void* stream) {
       a.generation = (g_decode_generation.fetch_add(1, std::memory_order_relaxed) % ((1ull << 48) - 1)) + 1;
     }
   } else if (sp.splits > 1) {
-    const size_t need = required_workspace_bytes(p);
+    const size_t need = token_rows ? token_row_workspace(p_in) : required_workspace_bytes(p);
     if (!p->workspace || p->workspace_bytes < need)
       return fail(RPA_EINVAL_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, p->workspace_bytes);
     a.ws_o = static_cast<float*>(p->workspace);
     a.ws_ml = a.ws_o + (size_t)p->decode_end * sp.splits * p->num_q_heads * p->head_dim;
   }
   return check_hip(rpa::launch_decode(a, static_cast<hipStream_t>(stream)), "rpa_decode");
+}
+
+int rpa_decode(const RpaParams* p, void* stream) {
+  const int rc = rpa_validate(p);
+  return rc != RPA_OK ? rc : decode_rows(p, nullptr, nullptr, false, stream);
 }
 
 // The prefill kernels' view of a call; false when the call has no chunk for them.
@@ -725,11 +790,44 @@ int rpa_prefill(const RpaParams* p, void* stream) {
   return check_hip(rpa::launch_prefill(a, static_cast<hipStream_t>(stream)), "rpa_prefill");
 }
 
-int rpa_attention(const RpaParams* p, void* stream) {
-  int rc = rpa_decode(p, stream);
+// Whether the decode kernels read their rows' new tokens from the caller's keys / values and write them into the cache
+// (not the 256-wide rows, nor the balanced plan on pages smaller than a block).
+static bool decode_takes_new_tokens(const RpaParams* p_in) {
+  if (p_in->head_dim != 128 || p_in->mask_mode == RPA_MASK_CUSTOM) return false;
+  if (p_in->page_size % 32 == 0) return true;
+  const RpaParams p = planning_view(p_in);
+  return !use_balanced(&p, decode_plan(&p));
+}
+
+static int write_new_tokens(const RpaParams* p, const void* keys, const void* values, bool skip_decode_rows, void* stream) {
+  rpa::KvWriteArgs a;
+  a.kv = kv_addr(p);
+  a.pt = page_table(p);
+  a.keys = static_cast<const char*>(keys);
+  a.values = static_cast<const char*>(values);
+  a.num_seqs = p->num_seqs;
+  a.dist = p->distribution;
+  a.Hkv = p->num_kv_heads;
+  a.head_bytes = p->head_dim * esize_of(p->kv_dtype);
+  a.num_tokens = p->num_tokens;
+  a.skip_decode_rows = skip_decode_rows ? 1 : 0;
+  a.seq_begin = skip_decode_rows && !p->distribution ? p->decode_end : 0;
+  return check_hip(rpa::launch_kv_write(a, static_cast<hipStream_t>(stream)), "rpa_kv_write");
+}
+
+int rpa_attention_update(const RpaParams* p, const void* keys, const void* values, void* stream) {
+  int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
+  if (!keys != !values) return fail(RPA_EINVAL_NULL, "keys and values must be given together");
+  if (takes_token_rows(p) && p->workspace_bytes >= token_row_workspace(p)) return decode_rows(p, keys, values, true, stream);
+  const bool fused = keys && decode_takes_new_tokens(p);
+  if (keys && !fused && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
+  if ((rc = decode_rows(p, fused ? keys : nullptr, fused ? values : nullptr, false, stream)) != RPA_OK) return rc;
+  if (fused && (rc = write_new_tokens(p, keys, values, true, stream)) != RPA_OK) return rc;
   return rpa_prefill(p, stream);
 }
+
+int rpa_attention(const RpaParams* p, void* stream) { return rpa_attention_update(p, nullptr, nullptr, stream); }
 
 int rpa_describe_plan(const RpaParams* p_in, char* buf, size_t len) {
   int rc = rpa_validate(p_in);
@@ -756,7 +854,7 @@ int rpa_describe_plan(const RpaParams* p_in, char* buf, size_t len) {
       const SplitPlan sp = decode_plan(p);
       const bool bal = use_balanced(p, sp);
       put("decode: shape=%s kernel=%s rows=%d waves_per_wg=%d", r.name,
-          bal ? "rpa_decode_balanced_kernel" : "rpa_decode_splitkv_kernel", p->decode_end, decode_waves_per_wg(p));
+          bal ? "rpa_decode_balanced_kernel" : "rpa_decode_splitkv_kernel", p->decode_end, bal ? decode_waves_per_wg(p) : decode_fixed_waves(p));
       if (bal) put(" resident_waves=%d merge=rpa_combine_balanced_kernel", decode_wave_capacity(p));
       else put(" pieces_per_row=%d chunk=%d merge=%s", sp.splits, sp.chunk, sp.splits > 1 ? "rpa_combine_kernel" : "none");
     }
@@ -807,25 +905,7 @@ int rpa_kv_write(const RpaParams* p, const void* keys, const void* values, void*
   int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
   if (!keys || !values) return fail(RPA_EINVAL_NULL, "keys/values is NULL");
-  rpa::KvWriteArgs a;
-  a.kv = kv_addr(p);
-  a.pt = page_table(p);
-  a.keys = static_cast<const char*>(keys);
-  a.values = static_cast<const char*>(values);
-  a.num_seqs = p->num_seqs;
-  a.dist = p->distribution;
-  a.Hkv = p->num_kv_heads;
-  a.head_bytes = p->head_dim * esize_of(p->kv_dtype);
-  a.num_tokens = p->num_tokens;
-  return check_hip(rpa::launch_kv_write(a, static_cast<hipStream_t>(stream)), "rpa_kv_write");
-}
-
-int rpa_attention_update(const RpaParams* p, const void* keys, const void* values, void* stream) {
-  if (keys || values) {
-    const int rc = rpa_kv_write(p, keys, values, stream);
-    if (rc != RPA_OK) return rc;
-  }
-  return rpa_attention(p, stream);
+  return write_new_tokens(p, keys, values, false, stream);
 }
 
 // ---------------------------------------------------------------- MLA ----

@@ -67,7 +67,21 @@ struct SeqView {
   int32_t page_size;
   int32_t page_shift;  // >= 0 when page_size is a power of two
   int32_t last_tok;    // kv_len - 1
+  // Tokens from fresh_first on are not in the cache yet: they come from the caller's new rows (DecodeArgs.new_k / new_v),
+  // fresh_row = row of token fresh_first and this kv head there.  kNoFresh: all are in the cache.
+  int32_t fresh_first;
+  int32_t fresh_row;
 };
+
+constexpr int kNoFresh = 0x7fffffff;
+
+// A wave-uniform condition the optimiser knows nothing else about: without it the rare branches on "this block ends the
+// row" are threaded through the whole block's code, which doubles it (8.3 k against 4.5 k instructions).
+__device__ __forceinline__ bool rare(bool cond) {
+  int v = __builtin_amdgcn_readfirstlane(cond);
+  asm("" : "+s"(v));
+  return v != 0;
+}
 
 __device__ __forceinline__ int page_slot_of(const SeqView& s, int tok) {
   return s.page_shift >= 0 ? (tok >> s.page_shift) : (tok / s.page_size);
@@ -81,12 +95,39 @@ __device__ __forceinline__ int page_slot_of(const SeqView& s, int tok) {
 // memory, a dependent round trip in front of the block's loads.
 // (A compile-time choice: with both lookups in the code the compiler's wait-count bookkeeping sees a possible
 // page-id load behind every block and drains the whole queue in front of each block's use.)
-template <bool FP8, bool UNIFORM_PAGE, bool WINDOW = false>
-__device__ __forceinline__ void load_block(KvRegs<FP8>& r, const SeqView& s, const KvAddr& kv,
-                                           const char* kh, const char* vh, int tb, int page, int c, int g,
+// FRESH: the row's last tokens may come from the caller's new rows instead (SeqView.fresh_first).
+template <bool FP8, bool UNIFORM_PAGE, bool WINDOW = false, bool FRESH = false>
+__device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, int page, int c, int g,
                                            const int32_t* win = nullptr, int win_first = 0) {
+  const KvAddr& kv = a.kv;
   constexpr int kLaneK = FP8 ? 32 : 16;  // byte offset step of lane group g inside a K row
   constexpr int kLaneV = FP8 ? 8 : 16;   // byte offset step of lane c inside a V row
+  // A block that reaches into the new tokens (the last one of a row): an address of its own per token row.  The
+  // number of loads is that of the other branch, so the counted waits behind it stay the same.
+  if (FRESH && rare(tb + kBlk > s.fresh_first)) {
+    const int block_slot = UNIFORM_PAGE ? page_slot_of(s, tb) : 0;
+    auto row_of = [&](int tok, const char* cached, const char* fresh) __attribute__((always_inline)) -> const char* {
+      tok = min(tok, s.last_tok);
+      const int slot = UNIFORM_PAGE ? block_slot : page_slot_of(s, tok);
+      const int pg = UNIFORM_PAGE ? page : WINDOW ? win[slot - win_first] : s.pages[slot];
+      const char* old_at = cached + (int64_t)pg * kv.page_stride + (int64_t)((tok - slot * s.page_size) * kv.tok_stride);
+      const char* new_at = fresh + (int64_t)(s.fresh_row + (tok - s.fresh_first) * a.Hkv) * (FP8 ? 128 : 256);
+      return tok >= s.fresh_first ? new_at : old_at;
+    };
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const char* kp = row_of(tb + b * 16 + c, kh, a.new_k) + g * kLaneK;
+#pragma unroll
+      for (int st = 0; st < (FP8 ? 2 : 4); ++st) r.k[b][st] = RPA_KV_LD16(kp + st * (FP8 ? 16 : 64));
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const char* vp = row_of(tb + tok_slot(g, i), vh, a.new_v) + c * kLaneV;
+      if constexpr (FP8) r.v[i] = RPA_KV_LD8(vp);
+      else r.v[i] = RPA_KV_LD16(vp);
+    }
+    return;
+  }
   if constexpr (UNIFORM_PAGE) {
     // the whole block lies in one page whose id the caller fetched a block ahead
     const int slot = page_slot_of(s, tb);
@@ -138,6 +179,39 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const SeqView& s, con
       if constexpr (FP8) r.v[i] = RPA_KV_LD8(vp);
       else r.v[i] = RPA_KV_LD16(vp);
     }
+  }
+}
+
+// Leave a row's new token, its last one, in the cache: the registers of the block that ends the row hold it (token t of
+// the block), K dims of token 16b + c in lanes (c, g), V rows of slot i in lanes (., g).  kh / vh: this kv head's rows of
+// the page, tin: the token's place in it.
+template <bool FP8>
+__device__ __forceinline__ void store_new_token(const KvRegs<FP8>& r, const KvAddr& kv, const char* kh, const char* vh,
+                                                int page, int tin, int t, int c, int g) {
+  const int64_t at = (int64_t)page * kv.page_stride + (int64_t)(tin * kv.tok_stride);
+  char* kp = const_cast<char*>(kh) + at;
+  char* vp = const_cast<char*>(vh) + at;
+  // (branches on t, which is the same in every lane: selects between the registers would take their address)
+  constexpr int kN = FP8 ? 2 : 4, kStep = FP8 ? 16 : 64;
+  t = __builtin_amdgcn_readfirstlane(t);
+  if (c == (t & 15)) {
+    kp += g * (FP8 ? 32 : 16);
+    if (t < 16) {
+#pragma unroll
+      for (int st = 0; st < kN; ++st) st16(kp + st * kStep, r.k[0][st]);
+    } else {
+#pragma unroll
+      for (int st = 0; st < kN; ++st) st16(kp + st * kStep, r.k[1][st]);
+    }
+  }
+  if (g == ((t >> 2) & 3)) {
+    const int i = (t & 3) + (t < 16 ? 0 : 4);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (i == k) {
+        if constexpr (FP8) *reinterpret_cast<u32x2_t*>(vp + c * 8) = r.v[k];
+        else st16(vp + c * 16, r.v[k]);
+      }
   }
 }
 
@@ -380,10 +454,18 @@ __device__ __forceinline__ void write_rows(const DecodeArgs& a, const f32x4_t (&
   }
 }
 
-// One wave, one (sequence, kv head, group of 16 query heads), tokens [t_begin, t_end).
+// One row: query token tq of sequence seq, which sees kv_len tokens; new tokens start at position fresh_first, whose
+// query token is fresh_tq.
+struct RowRef {
+  int seq, tq, kv_len, fresh_first, fresh_tq;
+};
+
+// One wave, one (row, kv head, group of 16 query heads), tokens [t_begin, t_end).
 template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP>
-__device__ __forceinline__ void decode_segment(const DecodeArgs& a, int seq, int hk, int rg, int kv_len, int t_lo,
+__device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef& row, int hk, int rg, int t_lo,
                                                int t_begin, int t_end, const PartDest dest, int lane) {
+  const int kv_len = row.kv_len;
+  const int seq = __builtin_amdgcn_readfirstlane(row.seq);
   const int c = lane & 15, g = lane >> 4;
   const int nblk = (t_end - t_begin + kBlk - 1) / kBlk;
 
@@ -394,15 +476,16 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, int seq, int
   // Sequence metadata and page ids go through the scalar cache: nothing writes them while the
   // kernel runs, and a scalar load is not counted by vmcnt, so waiting for a page id never
   // drains the block prefetch issued just before it.
-  seq = __builtin_amdgcn_readfirstlane(seq);
   sv.pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (scalar_load_i32(a.pt.cu_kv_lens + seq) / a.pt.page_size)
                                                   : (int64_t)seq * a.pt.pages_per_seq);
 
   const char* kh = a.kv.k_base + (int64_t)hk * a.kv.head_stride;
   const char* vh = a.kv.v_base + (int64_t)hk * a.kv.head_stride;
+  sv.fresh_first = a.new_k ? row.fresh_first : kNoFresh;
+  sv.fresh_row = row.fresh_tq * a.Hkv + hk;
 
   // ---- Q^T operands: column c = query head (row0 + 16*mt + c) of this kv head ----
-  const int tq = scalar_load_i32(a.pt.cu_q_lens + seq);
+  const int tq = row.tq;
   const int row0 = rg * 16 * MT;
   u32x4_t qB[MT][4];
   load_queries<MT, FP8>(a, tq, hk, row0, c, g, qB);
@@ -462,56 +545,93 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, int seq, int
       }
     }
   };
+  auto leave_new_token = [&](const KvRegs<FP8>& r, int tb) __attribute__((always_inline)) {
+    if (rare(a.new_k && tb + kBlk > sv.last_tok)) {
+      const int slot = __builtin_amdgcn_readfirstlane(page_slot_of(sv, sv.last_tok));
+      store_new_token<FP8>(r, a.kv, kh, vh, scalar_load_i32(sv.pages + slot), sv.last_tok - slot * sv.page_size,
+                           sv.last_tok - tb, c, g);
+    }
+  };
   KvRegs<FP8> ra, rb;
   int pg_next = page_of(block_tok(1));
   cover(t_begin);
-  load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(ra, sv, a.kv, kh, vh, t_begin, page_of(t_begin), c, g, win, win_first);
+  load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true>(ra, a, sv, kh, vh, t_begin, page_of(t_begin), c, g, win, win_first);
   for (int blk = 0; blk < nblk; blk += 2) {
     cover(block_tok(blk + 1));
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(rb, sv, a.kv, kh, vh, block_tok(blk + 1), pg_next, c, g, win, win_first);
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true>(rb, a, sv, kh, vh, block_tok(blk + 1), pg_next, c, g, win, win_first);
     pg_next = page_of(block_tok(blk + 2));
+    leave_new_token(ra, t_begin + blk * kBlk);
     compute_block<MT, FP8, CAP>(ra, qB, acc, m, l, so, t_begin + blk * kBlk, g);
     if (blk + 1 >= nblk) break;
     cover(block_tok(blk + 2));
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(ra, sv, a.kv, kh, vh, block_tok(blk + 2), pg_next, c, g, win, win_first);
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true>(ra, a, sv, kh, vh, block_tok(blk + 2), pg_next, c, g, win, win_first);
     pg_next = page_of(block_tok(blk + 3));
+    leave_new_token(rb, t_begin + (blk + 1) * kBlk);
     compute_block<MT, FP8, CAP>(rb, qB, acc, m, l, so, t_begin + (blk + 1) * kBlk, g);
   }
 
   write_rows<MT>(a, acc, m, l, tq, hk, row0, dest, c, g);
 }
 
-// ---- fixed split plan: grid = (max_splits * decode rows, 1, head groups * row groups), splits fastest (rows do
+__device__ __forceinline__ int owner_of_token(const int32_t* cu_q_lens, int num_seqs, int tok) {
+  int lo = 0, hi = num_seqs;  // last i with cu_q_lens[i] <= tok (zero-length sequences are skipped)
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (cu_q_lens[mid] <= tok) lo = mid; else hi = mid;
+  }
+  return lo;
+}
+
+// Row `index` of the fixed plan: decode row `index`, or (token_rows) query token `index` of whatever sequence owns it.
+// false: nothing there.
+__device__ __forceinline__ bool fixed_row(const DecodeArgs& a, int index, RowRef& row) {
+  if (a.token_rows) {
+    const int seqs = a.dist ? min(a.num_seqs, scalar_load_i32(a.dist + 2)) : a.num_seqs;
+    if (index >= scalar_load_i32(a.pt.cu_q_lens + seqs)) return false;
+    row.tq = index;
+    row.seq = __builtin_amdgcn_readfirstlane(owner_of_token(a.pt.cu_q_lens, seqs, index));
+    row.fresh_tq = scalar_load_i32(a.pt.cu_q_lens + row.seq);
+    row.fresh_first = scalar_load_i32(a.pt.kv_lens + row.seq) - (scalar_load_i32(a.pt.cu_q_lens + row.seq + 1) - row.fresh_tq);
+    row.kv_len = row.fresh_first + (index - row.fresh_tq) + 1;
+    return row.fresh_first >= 0;
+  }
+  // (static-shape mode: the number of decode rows comes from the device)
+  if (index >= (a.dist ? min(a.num_rows, scalar_load_i32(a.dist)) : a.num_rows)) return false;
+  row.seq = index;
+  row.kv_len = scalar_load_i32(a.pt.kv_lens + index);
+  row.tq = row.fresh_tq = scalar_load_i32(a.pt.cu_q_lens + index);
+  row.fresh_first = row.kv_len - 1;
+  return row.kv_len > 0;
+}
+
+// ---- fixed split plan: grid = (max_splits * rows, 1, head groups * row groups), splits fastest (rows do
 // not sit on a grid dimension of their own: that one ends at 65535); block = NW waves
 template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP>
-__global__ __launch_bounds__(256, 2) void rpa_decode_splitkv_kernel(const DecodeArgs a_in) {
-  DecodeArgs a = a_in;  // static-shape mode: the number of decode rows comes from the device
-  if (a.dist) a.num_rows = min(a.num_rows, scalar_load_i32(a.dist));
+__global__ __launch_bounds__(256, 2) void rpa_decode_splitkv_kernel(const DecodeArgs a) {
   const int nsp = max(a.max_splits, 1);
-  const int seq = (int)(blockIdx.x / (unsigned)nsp);
-  const int split = (int)blockIdx.x - seq * nsp;
-  if (seq >= a.num_rows) return;
+  const int index = (int)(blockIdx.x / (unsigned)nsp);
+  const int split = (int)blockIdx.x - index * nsp;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nw = blockDim.x >> 6;
   const int head_groups = (a.Hkv + nw - 1) / nw;
   const int hg = blockIdx.z % head_groups;
   const int rg = blockIdx.z / head_groups;
   const int hk = hg * nw + wave;
-  if (hk >= a.Hkv) return;
+  RowRef row;
+  if (hk >= a.Hkv || !fixed_row(a, index, row)) return;
 
-  const int kv_len = a.pt.kv_lens[seq];
-  const int t_lo = (a.sm.window > 0) ? max(0, kv_len - a.sm.window) : 0;
+  const int t_lo = (a.sm.window > 0) ? max(0, row.kv_len - a.sm.window) : 0;
   const int t0 = t_lo & ~(kBlk - 1);
   const int t_begin = t0 + split * a.chunk;
-  if (t_begin >= kv_len) return;
+  if (t_begin >= row.kv_len) return;
   // the last split runs to kv_len even if the host's length bound was too small
-  const int t_end = (split == a.max_splits - 1) ? kv_len : min(kv_len, t_begin + a.chunk);
+  const int t_end = (split == a.max_splits - 1) ? row.kv_len : min(row.kv_len, t_begin + a.chunk);
   PartDest dest;
   dest.final_rows = a.max_splits == 1;
   dest.by_head = true;
-  dest.base = ((int64_t)seq * a.max_splits + split) * a.Hq;
-  decode_segment<MT, FP8, UNIFORM_PAGE, CAP>(a, seq, hk, rg, kv_len, t_lo, t_begin, t_end, dest, lane);
+  dest.base = ((int64_t)index * a.max_splits + split) * a.Hq;
+  decode_segment<MT, FP8, UNIFORM_PAGE, CAP>(a, row, hk, rg, t_lo, t_begin, t_end, dest, lane);
 }
 
 // ---- balanced plan ------------------------------------------------------------------------
@@ -731,6 +851,7 @@ __device__ __forceinline__ void merge_unit(const DecodeArgs& a, const PendingMer
 // are requested right behind that first block.  A piece border costs no round trip to memory,
 // and neither does a block: under load a small dependent load waits behind megabytes of queued
 // KV traffic (10 us and more), so there are none after the first block.
+// New tokens (a.new_k) are taken where pages hold whole blocks; with smaller pages there is no register left for it.
 template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool MERGE>
 __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const DecodeArgs a_in) {
   DecodeArgs a = a_in;  // static-shape mode: the number of decode rows comes from the device
@@ -821,12 +942,14 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
     p.final_rows = (blk == 0) && (take == r.nb);
     return p;
   };
-  auto view_of = [&](const RowMeta& r) {
+  auto view_of = [&](const RowMeta& r, int hk) {
     SeqView sv;
     sv.page_size = page_size;
     sv.page_shift = page_shift;
     sv.last_tok = r.kv_len - 1;
     sv.pages = a.pt.page_indices + r.page0;
+    sv.fresh_first = (UNIFORM_PAGE && a.new_k) ? r.kv_len - 1 : kNoFresh;
+    sv.fresh_row = r.tq * a.Hkv + hk;
     return sv;
   };
   auto slot_of_tok = [&](int tok) { return page_shift >= 0 ? (tok >> page_shift) : (tok / page_size); };
@@ -857,9 +980,9 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
   KvRegs<FP8> ra, rb;
   bool in_b = false;  // which register set holds the block about to be consumed
   {
-    const SeqView sv = view_of(cur.row);
     const int hk = min(cur.hk, a.Hkv - 1);
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(ra, sv, a.kv, a.kv.k_base + (int64_t)hk * a.kv.head_stride,
+    const SeqView sv = view_of(cur.row, hk);
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE>(ra, a, sv, a.kv.k_base + (int64_t)hk * a.kv.head_stride,
                                   a.kv.v_base + (int64_t)hk * a.kv.head_stride, cur.t_first,
                                   page_in(win, cur.t_first), c, g, lanes_win(win), win.first);
   }
@@ -868,7 +991,7 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
   for (;;) {
     // ---- this piece
     const int hk = min(cur.hk, a.Hkv - 1);
-    const SeqView sv = view_of(cur.row);
+    const SeqView sv = view_of(cur.row, hk);
     const char* kh = a.kv.k_base + (int64_t)hk * a.kv.head_stride;
     const char* vh = a.kv.v_base + (int64_t)hk * a.kv.head_stride;
     requantise_queries<MT, FP8>(a, qB);
@@ -925,8 +1048,8 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
         const int x_next = x + cur.nblk;
         nxt = make_piece(nrow, nunit, 0, min(nrow.nb, x_end - x_next));
         request_window<kWin>(a, nrow, nwin, slot_of_tok(nxt.t_first), page_shift, lane);
-        nsv = view_of(nrow);
         const int nhk = min(nxt.hk, a.Hkv - 1);
+        nsv = view_of(nrow, nhk);
         nkh = a.kv.k_base + (int64_t)nhk * a.kv.head_stride;
         nvh = a.kv.v_base + (int64_t)nhk * a.kv.head_stride;
       }
@@ -945,11 +1068,15 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
         // The next piece's window was requested at block resolve_at, in front of that block's
         // prefetch.  Two blocks later a wait for younger loads has passed; earlier it has not.
         if (i <= resolve_at + 1) wait_all_loads();
-        load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(fill, nsv, a.kv, nkh, nvh, nxt.t_first, page_in(nwin, nxt.t_first), c, g,
+        load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE>(fill, a, nsv, nkh, nvh, nxt.t_first, page_in(nwin, nxt.t_first), c, g,
                                       lanes_win(nwin), nwin.first);
       } else {
         const int ptb = last ? tb : tb + kBlk;
-        load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(fill, sv, a.kv, kh, vh, ptb, page_in(win, ptb), c, g, lanes_win(win), win.first);
+        load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE>(fill, a, sv, kh, vh, ptb, page_in(win, ptb), c, g, lanes_win(win), win.first);
+      }
+      if (UNIFORM_PAGE && rare(a.new_k && tb + kBlk > sv.last_tok)) {  // the block that ends the row
+        const int slot = slot_of_tok(sv.last_tok);
+        store_new_token<FP8>(use, a.kv, kh, vh, page_in(win, sv.last_tok), sv.last_tok - slot * page_size, sv.last_tok - tb, c, g);
       }
       compute_block<MT, FP8, CAP>(use, qB, acc, m, l, so, tb, g);
     };
@@ -1072,11 +1199,10 @@ __device__ __forceinline__ void merge_few(const DecodeArgs& a, int n, int lane, 
 }
 
 template <int HD = 128, typename SlotOf>
-__device__ __forceinline__ void merge_rows(const DecodeArgs& a, int seq, int head, int n, int lane, SlotOf slot_of) {
+__device__ __forceinline__ void merge_rows(const DecodeArgs& a, int tq, int head, int n, int lane, SlotOf slot_of) {
   constexpr int kDpl = HD / 64;  // dims per lane
   typedef float fvec_t __attribute__((ext_vector_type(kDpl)));
   const int d = lane * kDpl;
-  const int tq = scalar_load_i32(a.pt.cu_q_lens + seq);
   float mstar = -INFINITY, den = 0.f;
   float acc[kDpl];
 #pragma unroll
@@ -1159,7 +1285,7 @@ __global__ __launch_bounds__(64) void rpa_combine_balanced_kernel(const DecodeAr
     const int part = ((int64_t)wj * pw >= first_block) ? 0 : 1;
     return (((int64_t)wj * nw + wv) * 2 + part) * 16 + r16;
   };
-  merge_rows(a, seq, head, n, lane, slot_of);
+  merge_rows(a, scalar_load_i32(a.pt.cu_q_lens + seq), head, n, lane, slot_of);
 }
 
 // ---- head_dim 256 ---------------------------------------------------------------------------
@@ -1170,15 +1296,6 @@ __global__ __launch_bounds__(64) void rpa_combine_balanced_kernel(const DecodeAr
 // over both halves, each half has its own accumulators.  No split over tokens, no prefetch
 // ahead of the block being consumed, and a chunk's tokens each stream the prefix again: this
 // path exists so that 256-dim heads work, it is not tuned.
-__device__ __forceinline__ int owner_of_token(const int32_t* cu_q_lens, int num_seqs, int tok) {
-  int lo = 0, hi = num_seqs;  // last i with cu_q_lens[i] <= tok (zero-length sequences are skipped)
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (cu_q_lens[mid] <= tok) lo = mid; else hi = mid;
-  }
-  return lo;
-}
-
 // grid = (token rows, Hkv, row groups of 16 query heads); block = one wave.
 // With the composition on the device (a.dist) seq_end is only a bound: dist_role 1 = the decode partition
 // [0, dist[0]), 2 = everything behind it [dist[0], dist[2]) (custom-mask calls: [0, dist[2])).
@@ -1220,6 +1337,7 @@ __global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int
   sv.page_size = a.pt.page_size;
   sv.page_shift = ((sv.page_size & (sv.page_size - 1)) == 0) ? (31 - __builtin_clz(sv.page_size)) : -1;
   sv.last_tok = t_hi - 1;
+  sv.fresh_first = kNoFresh;
   sv.pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (a.pt.cu_kv_lens[seq] / a.pt.page_size)
                                                   : (int64_t)seq * a.pt.pages_per_seq);
   constexpr int kHalfB = FP8 ? 128 : 256;  // bytes of 128 cached elements
@@ -1275,8 +1393,8 @@ __global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int
       win = win_ids;
     }
     KvRegs<FP8> r0, r1;
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(r0, sv, a.kv, kh, vh, tb, page, c, g, win, win_first);
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(r1, sv, a.kv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(r0, a, sv, kh, vh, tb, page, c, g, win, win_first);
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(r1, a, sv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
     f32x4_t s[2];
     {
       u32x4_t kA[2][4];
@@ -1375,19 +1493,17 @@ __global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int
 // with shuffles, then the weights are broadcast lane by lane while the partial
 // rows stream in with independent loads.
 template <int HD>
-__global__ __launch_bounds__(64) void rpa_combine_kernel(const DecodeArgs a_in) {
-  DecodeArgs a = a_in;  // static-shape mode: the number of decode rows comes from the device
-  if (a.dist) a.num_rows = min(a.num_rows, scalar_load_i32(a.dist));
-  const int seq = (int)(blockIdx.x / (unsigned)a.Hq);  // grid.x = Hq * rows, heads fastest
-  const int head = (int)blockIdx.x - seq * a.Hq;
-  if (seq >= a.num_rows) return;
+__global__ __launch_bounds__(64) void rpa_combine_kernel(const DecodeArgs a) {
+  const int index = (int)(blockIdx.x / (unsigned)a.Hq);  // grid.x = Hq * rows, heads fastest
+  const int head = (int)blockIdx.x - index * a.Hq;
+  RowRef row;
+  if (!fixed_row(a, index, row)) return;
   const int lane = threadIdx.x;
-  const int kv_len = a.pt.kv_lens[seq];
-  const int t0 = first_block_token(kv_len, a.sm.window);
-  const int n = min(a.max_splits, (kv_len - t0 + a.chunk - 1) / a.chunk);
+  const int t0 = first_block_token(row.kv_len, a.sm.window);
+  const int n = min(a.max_splits, (row.kv_len - t0 + a.chunk - 1) / a.chunk);
   if (n <= 0) return;
-  const int64_t base = ((int64_t)seq * a.max_splits) * a.Hq + head;
-  merge_rows<HD>(a, seq, head, n, lane, [&](int j) -> int64_t { return base + (int64_t)j * a.Hq; });
+  const int64_t base = ((int64_t)index * a.max_splits) * a.Hq + head;
+  merge_rows<HD>(a, row.tq, head, n, lane, [&](int j) -> int64_t { return base + (int64_t)j * a.Hq; });
 }
 
 // One thread copies one 16-byte piece of one gathered row.
@@ -1417,11 +1533,12 @@ __global__ __launch_bounds__(256) void rpa_gather_kernel(const GatherArgs a) {
 __global__ __launch_bounds__(256) void rpa_kv_write_kernel(const KvWriteArgs a_in) {
   KvWriteArgs a = a_in;
   if (a.dist) a.num_seqs = min(a.num_seqs, a.dist[2]);
+  if (a.dist && a.skip_decode_rows) a.seq_begin = min(a.num_seqs, a.dist[0]);
   const int pieces = a.Hkv * a.head_bytes / 16;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int total_tokens = min(a.num_tokens, a.pt.cu_q_lens[a.num_seqs]);
-  if (idx >= (int64_t)total_tokens * pieces) return;
-  const int t = (int)(idx / pieces);
+  const int t = (int)(idx / pieces) + (a.seq_begin > 0 ? a.pt.cu_q_lens[a.seq_begin] : 0);
+  if (t >= total_tokens) return;
   const int byte = (int)(idx % pieces) * 16;
   int lo = 0, hi = a.num_seqs;  // last i with cu_q_lens[i] <= t
   while (hi - lo > 1) {
@@ -1447,11 +1564,18 @@ __global__ __launch_bounds__(256) void rpa_kv_write_kernel(const KvWriteArgs a_i
 
 template <bool FP8, bool UNIFORM, bool CAP>
 void launch_decode_variant(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t st) {
+  // LDS nobody uses keeps four waves on a CU, one per SIMD: without it the dispatcher doubles workgroups up on some CUs
+  // while others stand idle, and a CU draws about 39 bytes per ns at most (fixed plan, 128 rows of 256..2048 tokens x 2
+  // heads 47.7 -> 35.6 us; balanced, 56 rows of 512..4096 x 8 heads 99.3 -> 98.3).  Not for grids of many rounds, whose
+  // workgroups' starts have to overlap.
+  const bool one_round = (int64_t)grid.x * grid.z * (block.x / 64) <= 2048;
+  const int forced = tuning().decode_lds_kb;
+  const unsigned lds = forced >= 0 ? (unsigned)forced << 10 : !one_round ? 0u : block.x >= 256 ? 84u << 10 : block.x >= 128 ? 54u << 10 : 34u << 10;
   if (a.balanced && a.merge_counters)
-    hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, FP8, UNIFORM, CAP, true>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, FP8, UNIFORM, CAP, true>), grid, block, lds, st, a);
   else if (a.balanced)
-    hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, FP8, UNIFORM, CAP, false>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((rpa_decode_splitkv_kernel<1, FP8, UNIFORM, CAP>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, FP8, UNIFORM, CAP, false>), grid, block, lds, st, a);
+  else hipLaunchKernelGGL((rpa_decode_splitkv_kernel<1, FP8, UNIFORM, CAP>), grid, block, lds, st, a);
 }
 
 hipError_t launch_decode_mt(const DecodeArgs& a, dim3 grid, dim3 block, bool uniform, hipStream_t st) {
@@ -1531,8 +1655,8 @@ hipError_t launch_rows256(const DecodeArgs& a, int seq_begin, int seq_end, int m
 }
 
 hipError_t launch_kv_write(const KvWriteArgs& a, hipStream_t stream) {
-  if (a.num_tokens <= 0 || a.num_seqs <= 0) return hipSuccess;
-  const int64_t total = (int64_t)a.num_tokens * (a.Hkv * a.head_bytes / 16);
+  if (a.num_tokens <= 0 || a.num_seqs <= a.seq_begin) return hipSuccess;
+  const int64_t total = (int64_t)(a.num_tokens - a.seq_begin) * (a.Hkv * a.head_bytes / 16);
   const int blocks = (int)((total + 255) / 256);
   hipLaunchKernelGGL(rpa_kv_write_kernel, dim3(blocks), dim3(256), 0, stream, a);
   return hipGetLastError();

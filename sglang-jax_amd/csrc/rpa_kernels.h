@@ -76,6 +76,12 @@ struct DecodeArgs {
   // device i32[3] (decode_end, prefill_end, num_seqs) or nullptr: when given, num_rows is only a bound
   // and the rows to process are [0, min(num_rows, dist[0]))
   const int32_t* dist;
+  // New tokens that are not in the cache yet, [T, Hkv, D] in its element type, or nullptr: the kernel reads them from
+  // here and leaves each in its cache slot
+  const char* new_k;
+  const char* new_v;
+  int32_t token_rows;    // fixed plan: rows are the query tokens of sequences [0, num_seqs), of any length
+  int32_t num_seqs;      // token_rows: sequences (with dist: a bound on dist[2])
 };
 
 struct PrefillArgs {
@@ -130,6 +136,10 @@ struct KvWriteArgs {
   int32_t head_bytes;
   int32_t num_tokens;
   const int32_t* dist;  // device i32[3] or nullptr: when given, num_seqs is only a bound on dist[2]
+  // decode rows whose tokens the decode kernel writes itself are left out: sequences [0, seq_begin), with dist
+  // (skip_decode_rows) sequences [0, dist[0])
+  int32_t seq_begin;
+  int32_t skip_decode_rows;
 };
 
 struct MlaDecodeArgs {

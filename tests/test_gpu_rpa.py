@@ -1497,3 +1497,72 @@ def test_kv_range_pieces_with_the_composition_on_the_device(pkg, wl, gpu, monkey
         assert_parity(cut.float(), want.float(), **BF16_TOL)
         assert_parity(whole.float(), want.float(), **BF16_TOL)
         assert not torch.equal(cut, whole), "the bounds were expected to cut this launch"
+
+
+# ------------------------------------------------------------------ new tokens taken by the decode kernels themselves
+def with_new_tokens(b):
+    """(keys, values, cache): the batch's query tokens as new K / V rows, and a cache whose slots of those tokens and
+    whose unused slots hold NaN (fp8: its NaN byte): nothing may be read from there, each new slot must be written."""
+    P, n = b.page_size, int(b.distribution[2])
+    fp8 = b.kv_cache.dtype != torch.bfloat16
+    full = b.kv_cache.view(torch.uint8 if fp8 else torch.int16)
+    cache = torch.full_like(full, 0x7F if fp8 else 0x7FC0)
+    rows = []
+    for i in range(n):
+        kv, q = int(b.kv_lens[i]), int(b.cu_q_lens[i + 1] - b.cu_q_lens[i])
+        first = int(b.cu_kv_lens[i]) // P
+        for t in range(kv):
+            page = int(b.page_indices[first + t // P])
+            if t < kv - q:
+                cache[page, t % P] = full[page, t % P]
+            else:
+                rows.append(full[page, t % P])
+    new = torch.stack(rows).view(b.kv_cache.dtype)
+    return new[:, 0::2].contiguous(), new[:, 1::2].contiguous(), cache.view(b.kv_cache.dtype)
+
+
+EDGE_KV = [1, 2, 31, 32, 33, 63, 64, 65, 127, 129, 255, 300]
+NEW_TOKEN_CASES = {
+    # name: (q_lens, kv_lens, Hq, Hkv, P, window, composition on the device)
+    "edges": ([1] * 12, EDGE_KV, 16, 8, 64, None, False),
+    "edges_small_pages": ([1] * 12, EDGE_KV, 8, 1, 16, None, False),
+    "edges_window": ([1] * 12, EDGE_KV, 40, 2, 32, 33, False),  # 20 query heads per kv head: two groups walk the row
+    "odd_heads": ([1] * 5, [40, 7, 900, 64, 1], 9, 3, 64, None, False),
+    "cut_rows": ([1] * 3, [5000, 33, 4097], 8, 2, 64, None, False),
+    "many_short_rows": ([1] * 300, [1 + (7 * i) % 150 for i in range(300)], 16, 8, 64, None, False),
+    "balanced": ([1] * 40, [1 + (911 * i) % 4000 for i in range(40)], 32, 8, 64, None, False),
+    "balanced_small_pages": ([1] * 40, [1 + (911 * i) % 4000 for i in range(40)], 32, 8, 16, None, False),
+    "token_rows": ([1, 1, 3, 1, 17], [64, 1, 40, 33, 17], 16, 8, 16, None, True),
+    "token_rows_host": ([1, 5, 32], [65, 5, 97], 8, 2, 64, 40, False),
+    "mixed": ([1, 1, 70, 130], [500, 33, 200, 130], 8, 2, 64, None, False),
+    "mixed_on_the_device": ([1, 1, 70, 130], [500, 33, 200, 130], 8, 2, 64, None, True),
+}
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("case", list(NEW_TOKEN_CASES))
+def test_new_tokens_are_attended_to_and_left_in_the_cache(pkg, wl, gpu, case, fp8):
+    q_lens, kv_lens, Hq, Hkv, P, window, on_device = NEW_TOKEN_CASES[case]
+    say(f"new tokens {case} fp8={fp8}")
+    b = wl.make_batch("new_tokens", q_lens, kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=311,
+                      kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16, sliding_window=window)
+    want = oracle_out(b)
+    keys, values, cache = with_new_tokens(b)
+    g, cache = b.to(gpu), cache.to(gpu)
+    dist = g.distribution if on_device else b.distribution.numpy()
+    bounds = {} if on_device else dict(max_kv_len=max(kv_lens), max_q_len=max(q_lens), host_kv_lens=b.kv_lens.numpy())
+    out, after = pkg.ragged_paged_attention(
+        g.q, keys.to(gpu), values.to(gpu), cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, dist,
+        sm_scale=b.sm_scale, sliding_window=window, k_scale=g.k_scale, v_scale=g.v_scale, **bounds)
+    torch.cuda.synchronize()
+    assert_parity(out.cpu().float(), want.float(), **(FP8_TOL if fp8 else BF16_TOL))
+    bits = torch.uint8 if fp8 else torch.int16
+    got, full = after.cpu().view(bits), b.kv_cache.view(bits)
+    _, _, before = with_new_tokens(b)
+    expect = before.view(bits).clone()
+    for i, kv in enumerate(kv_lens):
+        first = int(b.cu_kv_lens[i]) // P
+        for t in range(kv - q_lens[i], kv):
+            page = int(b.page_indices[first + t // P])
+            expect[page, t % P] = full[page, t % P]
+    assert torch.equal(got, expect)  # every new slot written, nothing else touched
