@@ -350,6 +350,30 @@ RPA_API int rpa_mla_kv_write(const RpaMlaParams* p, const void* new_kv_c, const 
 RPA_API int rpa_mla_attention_update(const RpaMlaParams* p, const void* new_kv_c, const void* new_k_pe, int token_rows,
                              void* stream);
 
+/*
+ * Sparse absorbed-MLA attention (kernels/dsa/sparse_mla.py:63-297): every query token attends to its own selection of
+ * its sequence's cached tokens, as if it were a decode row over a page table of the selection.
+ *   k_pages_max > 0   whole pages (sparse_mla.py:63-203, decode rows): the distinct pages the selection touches, ascending,
+ *                     at most k_pages_max - 1 of them, then the page of the new token, into which the new row is written.
+ *                     The last page of the cache is the padding target.
+ *   k_pages_max == 0  single tokens (sparse_mla.py:206-297): the valid entries of the selection, which come first; the
+ *                     new row stands for the last of them and the cache is not written.
+ * `p` is the batch as rpa_mla_decode takes it (ragged page table; kv_lens, cu_q_lens of num_seqs sequences; max_kv_len
+ * and sum_kv_len are not read).  The new rows may both be NULL when the cache already holds every token.
+ */
+typedef struct RpaMlaSparse {
+  const int32_t* topk;       /* i32[T, topk_stride]: positions in the sequence, -1 = unused */
+  int32_t topk_count;        /* entries of a row that are read */
+  int32_t topk_stride;
+  int32_t topk_is_pages;     /* whole pages: the entries are pages of the sequence already */
+  int32_t pages_per_seq;
+  int32_t k_pages_max;
+  int32_t num_page_indices;  /* entries of p->page_indices */
+} RpaMlaSparse;
+RPA_API size_t rpa_mla_sparse_workspace_bytes(const RpaMlaParams* p, const RpaMlaSparse* s);
+RPA_API int rpa_mla_sparse_attention(const RpaMlaParams* p, const RpaMlaSparse* s, const void* new_kv_c,
+                                     const void* new_k_pe, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -57,6 +57,8 @@ EXPORTED_SYMBOLS = (
     "rpa_mla_describe_plan",
     "rpa_attention_update",
     "rpa_mla_attention_update",
+    "rpa_mla_sparse_workspace_bytes",
+    "rpa_mla_sparse_attention",
 )
 
 

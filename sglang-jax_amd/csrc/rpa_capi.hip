@@ -988,7 +988,7 @@ size_t rpa_mla_attention_workspace_bytes(const RpaMlaParams* p) {
   return mla_workspace(p, p ? p->num_tokens : 0, true);
 }
 
-static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows) {
+static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const char* extra_rows = nullptr) {
   int rc = mla_validate(p);
   if (rc != RPA_OK) return rc;
   if (p->num_seqs <= 0) return RPA_OK;
@@ -998,6 +998,7 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows) {
   if (rows <= 0) return RPA_OK;
   const SplitPlan sp = mla_plan(p, rows);
   rpa::MlaDecodeArgs a;
+  a.extra_rows = extra_rows;
   a.ql_nope = static_cast<const uint16_t*>(p->ql_nope);
   a.q_pe = static_cast<const uint16_t*>(p->q_pe);
   a.out = static_cast<uint16_t*>(p->out);
@@ -1122,6 +1123,99 @@ int rpa_mla_attention_update(const RpaMlaParams* p, const void* new_kv_c, const 
     if (rc != RPA_OK) return rc;
   }
   return mla_run(p, stream, token_rows != 0);
+}
+
+// ---- sparse attention: the dense kernels over a page table per query token ----
+namespace {
+// The call the dense kernels see: a decode row per query token.
+RpaMlaParams sparse_view(const RpaMlaParams* p, const RpaMlaSparse* s) {
+  RpaMlaParams v = *p;
+  const bool rows = s->k_pages_max <= 0;
+  v.num_seqs = p->num_tokens;
+  v.cu_kv_lens = nullptr;
+  if (rows) v.page_size = 1;
+  v.pages_per_seq = rows ? s->topk_count : s->k_pages_max;
+  v.max_kv_len = v.pages_per_seq * v.page_size;
+  v.sum_kv_len = 0;
+  v.num_splits = 0;
+  v.distribution = nullptr;
+  return v;
+}
+
+// Workspace: what the view's plan needs, then the tables.
+struct SparseLayout {
+  size_t kv_lens, cu_q, table, extra, total;
+};
+SparseLayout sparse_layout(const RpaMlaParams* p, const RpaMlaSparse* s, const RpaMlaParams& view) {
+  auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+  const size_t T = (size_t)p->num_tokens;
+  SparseLayout l;
+  l.kv_lens = up(rpa_mla_workspace_bytes(&view));
+  l.cu_q = l.kv_lens + up(T * sizeof(int32_t));
+  l.table = l.cu_q + up((T + 1) * sizeof(int32_t));
+  l.extra = l.table + up(T * view.pages_per_seq * sizeof(int32_t));
+  l.total = l.extra + (s->k_pages_max > 0 ? 0 : (T + 1) * p->row_stride * (p->cache_dtype == RPA_KV_FP8_E4M3 ? 1 : 2));
+  return l;
+}
+}  // namespace
+
+size_t rpa_mla_sparse_workspace_bytes(const RpaMlaParams* p, const RpaMlaSparse* s) {
+  if (!p || !s || p->num_tokens <= 0) return 0;
+  return sparse_layout(p, s, sparse_view(p, s)).total;
+}
+
+int rpa_mla_sparse_attention(const RpaMlaParams* p, const RpaMlaSparse* s, const void* new_kv_c, const void* new_k_pe,
+                             void* stream) {
+  int rc = mla_validate(p);
+  if (rc != RPA_OK) return rc;
+  if (!s || !s->topk || !p->cu_kv_lens) return fail(RPA_EINVAL_NULL, "a selection and a ragged page table are needed");
+  if (!new_kv_c != !new_k_pe) return fail(RPA_EINVAL_NULL, "new_kv_c and new_k_pe must be given together");
+  if (p->num_tokens <= 0 || p->num_seqs <= 0) return RPA_OK;
+  const bool rows = s->k_pages_max <= 0;
+  if (s->topk_count < (s->topk_is_pages ? 0 : 1) || s->topk_stride < s->topk_count || s->num_page_indices <= 0 || (!rows && s->pages_per_seq <= 0) ||
+      (rows && s->topk_is_pages))
+    return fail(RPA_EINVAL_SHAPE, "selection of %d entries (stride %d), %d pages per sequence, %d page ids", s->topk_count,
+                s->topk_stride, s->pages_per_seq, s->num_page_indices);
+  if ((int64_t)p->total_pages * p->page_size > 0x7fffffffLL || (int64_t)s->k_pages_max * p->page_size > 0x7fffffffLL)
+    return fail(RPA_EUNSUPPORTED, "%d pages of %d tokens: more than 2^31 rows", p->total_pages, p->page_size);
+  RpaMlaParams v = sparse_view(p, s);
+  const SparseLayout l = sparse_layout(p, s, v);
+  if (!p->workspace || p->workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(p->workspace) & 15) != 0)
+    return fail(RPA_EINVAL_WORKSPACE, "workspace of %zu bytes needed (aligned to 16), %zu given", l.total, p->workspace_bytes);
+  char* ws = static_cast<char*>(p->workspace);
+  rpa::SparseMlaArgs a;
+  a.pt.kv_lens = p->kv_lens;
+  a.pt.page_indices = p->page_indices;
+  a.pt.cu_q_lens = p->cu_q_lens;
+  a.pt.cu_kv_lens = p->cu_kv_lens;
+  a.pt.pages_per_seq = 0;
+  a.pt.page_size = p->page_size;
+  a.num_page_indices = s->num_page_indices;
+  a.num_tokens = p->num_tokens;
+  a.num_seqs = p->num_seqs;
+  a.topk = s->topk;
+  a.topk_count = s->topk_count;
+  a.topk_stride = s->topk_stride;
+  a.topk_is_pages = s->topk_is_pages;
+  a.pages_per_seq = s->pages_per_seq;
+  a.k_pages_max = rows ? 0 : s->k_pages_max;
+  a.total_pages = p->total_pages;
+  a.cache = static_cast<char*>(const_cast<void*>(p->cache_kv));
+  a.row_stride = p->row_stride;
+  a.rope_offset = p->rope_offset;
+  a.fp8 = p->cache_dtype == RPA_KV_FP8_E4M3 ? 1 : 0;
+  a.new_kv_c = static_cast<const char*>(new_kv_c);
+  a.new_k_pe = static_cast<const char*>(new_k_pe);
+  a.table = reinterpret_cast<int32_t*>(ws + l.table);
+  a.kv_len_out = reinterpret_cast<int32_t*>(ws + l.kv_lens);
+  a.cu_q_out = reinterpret_cast<int32_t*>(ws + l.cu_q);
+  a.extra = ws + l.extra;
+  if ((rc = check_hip(rpa::launch_sparse_table(a, static_cast<hipStream_t>(stream)), "rpa sparse table")) != RPA_OK) return rc;
+  v.kv_lens = a.kv_len_out;
+  v.cu_q_lens = a.cu_q_out;
+  v.page_indices = a.table;
+  v.workspace_bytes = l.kv_lens;
+  return mla_run(&v, stream, false, rows ? a.extra : nullptr);
 }
 
 }  // extern "C"

@@ -170,6 +170,8 @@ struct MlaDecodeArgs {
   float out_scale;    // finished rows are multiplied by it (v_scale; 1 when off)
   const int32_t* dist;  // device i32[3] or nullptr: when given, num_seqs is only a bound on dist[2]
   int32_t fp8;          // cache rows are e4m3 bytes (row_stride / rope_offset stay in elements)
+  // pages -1, -2, ... of the page table are pages 0, 1, ... of this buffer (pages under 32 tokens only), or nullptr
+  const char* extra_rows;
 };
 
 struct MlaWriteArgs {
@@ -183,6 +185,27 @@ struct MlaWriteArgs {
   int32_t row_stride;
   int32_t rope_offset;
   const int32_t* dist;  // device i32[3] or nullptr: when given, num_seqs is only a bound on dist[2]
+};
+
+struct SparseMlaArgs {
+  PageTable pt;              // of the batch: ragged table (cu_kv_lens)
+  int32_t num_page_indices;  // entries of pt.page_indices
+  int32_t num_tokens;
+  int32_t num_seqs;
+  const int32_t* topk;       // [T, topk_stride], the first topk_count of a row are read; -1 = unused
+  int32_t topk_count, topk_stride;
+  int32_t topk_is_pages;     // entries are pages of the sequence, not tokens
+  int32_t pages_per_seq;
+  int32_t k_pages_max;       // > 0: tables of whole pages; 0: tables of single rows
+  int32_t total_pages;
+  char* cache;               // whole pages: the new rows are written here
+  int32_t row_stride, rope_offset, fp8;
+  const char* new_kv_c;      // [T, 512] in the cache's element type, or nullptr: the cache holds them already
+  const char* new_k_pe;      // [T, 64]
+  int32_t* table;            // [T, k_pages_max or topk_count]
+  int32_t* kv_len_out;       // [T]
+  int32_t* cu_q_out;         // [T + 1]
+  char* extra;               // single rows: [T + 1] rows, the new ones and one of zeros
 };
 
 hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream);
@@ -205,6 +228,7 @@ ShapeKey mla_shape_key(const MlaDecodeArgs& a);
 unsigned mla_shape_skip(const Tuning& tune);
 // how query tokens of a chunk share a workgroup (0: they do not; 1, 2: eight waves; 3: wide workgroups)
 int mla_token_group_mode(const MlaDecodeArgs& a, const Tuning& tune, const ShapeRule& shape);
+hipError_t launch_sparse_table(const SparseMlaArgs& a, hipStream_t stream);
 hipError_t launch_mla_kv_write(const MlaWriteArgs& a, hipStream_t stream);
 
 }  // namespace rpa

@@ -93,13 +93,21 @@ __device__ __forceinline__ int tok_of(int g, int i) {
   return 16 * (i >> 2) + 4 * g + (i & 3);
 }
 
+// Pages that are no whole number of tiles: the ids of a tile's pages arrive in LDS by a copy of their own
+// (global_load_lds_dword, entry i = page slot of the tile's first token + i), two tiles ahead of the tile's rows, in
+// a ring of kIdSlots tiles; the lanes look their rows' pages up there.  An id in a register would be a load that the
+// next tile's copies depend on, behind which the copies in flight drain, and a window over many tiles (what was here
+// before) drains them each time it moves: every 128 tokens where a page is a single row.
+constexpr int kIdSlots = 8;
+constexpr int kIdEntries = 64;  // at most 33 pages meet a tile
+
+typedef __attribute__((address_space(3))) int32_t* lds_i32_t;
+
 struct Src {
   const int32_t* pages;
-  // pages smaller than a tile: the wave's LDS window of this row's page ids (entry 0 = page slot win_first),
-  // which the lanes look their rows' pages up in; fetched from memory per tile they would be a load the next
-  // tile's copies depend on, behind which the copies in flight drain
-  const int32_t* win;
-  int32_t win_first;
+  lds_i32_t ids;       // the ring
+  const char* extra;   // pages -1, -2, ... of the table are pages 0, 1, ... here (sparse attention's new rows)
+  int32_t t_begin;     // first token of the segment: tile k of the ring starts at t_begin + 32 k
   int32_t page_size, page_shift, last_tok;
   int64_t page_stride;  // bytes
   int32_t row_bytes;    // bytes between tokens of a page
@@ -108,6 +116,29 @@ struct Src {
 
 __device__ __forceinline__ int page_slot(const Src& s, int tok) {
   return s.page_shift >= 0 ? (tok >> s.page_shift) : (tok / s.page_size);
+}
+
+// Ring slot of the page ids of the tile at `tb` (a multiple of 32 tokens behind t_begin), and the id of page slot
+// `ps` in it.
+__device__ __forceinline__ int id_slot(const Src& s, int tb) { return ((tb - s.t_begin) / kTok) & (kIdSlots - 1); }
+
+__device__ __forceinline__ int page_in_ring(const Src& s, int tb, int ps) {
+  return s.ids[id_slot(s, tb) * kIdEntries + ps - page_slot(s, tb)];
+}
+
+// First byte of page `pg`.
+template <bool UNIFORM>
+__device__ __forceinline__ const char* page_base(const Src& s, const char* cache, int pg) {
+  if constexpr (UNIFORM) return cache + (int64_t)pg * s.page_stride;
+  else return (pg < 0 ? s.extra : cache) + (int64_t)(pg < 0 ? ~pg : pg) * s.page_stride;
+}
+
+// Request the page ids of the tile at `tb` (past the end: of the last tile, like the rows).
+__device__ __forceinline__ void copy_tile_ids(const Src& s, int tb, int lane) {
+  tb = min(tb, s.last_tok & ~(kTok - 1));
+  const uint32_t dst = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s.ids + id_slot(s, tb) * kIdEntries));
+  const int32_t* src = s.pages + min(page_slot(s, tb) + lane, page_slot(s, s.last_tok));
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(src) : "memory", "m0");
 }
 
 // A lane's 5 chunks of a tile: position p = 64*(5*wave + n) + lane; row p / 74, chunk
@@ -163,8 +194,8 @@ __device__ __forceinline__ void copy_tile(char* slot, const Src& s, const char* 
     chunk_of<CPW>(s, wave, lane, n, row, inner);
     const int tok = min(tb + row, s.last_tok);
     const int ps = page_slot(s, tok);
-    const int pg = UNIFORM ? page : s.win[ps - s.win_first];
-    const char* src = cache + (int64_t)pg * s.page_stride + (int64_t)(tok - ps * s.page_size) * s.row_bytes + inner;
+    const int pg = UNIFORM ? page : page_in_ring(s, tb, ps);
+    const char* src = page_base<UNIFORM>(s, cache, pg) + (int64_t)(tok - ps * s.page_size) * s.row_bytes + inner;
     async_copy16(src, slot + copy_block<CPW>(wave, n) * 1024);
   }
 }
@@ -202,8 +233,8 @@ __device__ __forceinline__ void copy_tile_f8(char* stage, const Src& s, const ch
     } else {  // last, partial tile (rows clamped to the last valid token) or pages smaller than a tile
       const int tok = min(tb + row, s.last_tok);
       const int ps = page_slot(s, tok);
-      const int pg = UNIFORM ? page : s.win[ps - s.win_first];
-      async_copy16(cache + (int64_t)pg * s.page_stride + (int64_t)(tok - ps * s.page_size) * s.row_bytes + inner,
+      const int pg = UNIFORM ? page : page_in_ring(s, tb, ps);
+      async_copy16(page_base<UNIFORM>(s, cache, pg) + (int64_t)(tok - ps * s.page_size) * s.row_bytes + inner,
                    stage + blk * 1024);
     }
   }
@@ -318,7 +349,8 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  static_assert(DS == 1 || (UNIFORM && !PIPE), "shared tiles: compiled loop, whole tiles per page (LDS for the partial scores)");
+  static_assert(DS == 1 || !PIPE, "shared tiles: compiled loop (LDS for the partial scores)");
+  static_assert(UNIFORM || !PIPE, "the assembly loop takes one page per tile");
   static_assert(!TG || DS == 1, "token groups: one wave per (token, block of 16 heads)");
   const int sub = wave % DS;                       // this wave's place among the DS waves of its block of heads
   // token groups: a wave past the group's last real token repeats that token's work and writes nothing
@@ -344,20 +376,10 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   src.row_bytes = a.row_stride * (FP8 ? 1 : 2);
   src.page_stride = (int64_t)src.row_bytes * a.pt.page_size;
   src.rope_byte = a.rope_offset * (FP8 ? 1 : 2);
-  src.win = nullptr;
-  src.win_first = 0;
-  __shared__ int32_t page_windows[UNIFORM ? 1 : 8][UNIFORM ? 1 : kWinSmallPages];  // [wave][entry]
-  auto cover = [&](int tb) __attribute__((always_inline)) {  // make the wave's window hold the pages of tile tb
-    if constexpr (!UNIFORM) {
-      tb = min(tb, src.last_tok & ~(kTok - 1));
-      if (!src.win || page_slot(src, min(tb + kTok - 1, src.last_tok)) - src.win_first >= kWinSmallPages) {
-        src.win_first = __builtin_amdgcn_readfirstlane(page_slot(src, tb));
-        copy_page_window<kWinSmallPages>(src.pages, page_slot(src, src.last_tok), page_windows[wave], src.win_first, lane);
-        wait_all_loads();
-        src.win = page_windows[wave];
-      }
-    }
-  };
+  __shared__ int32_t id_ring[UNIFORM ? 1 : kIdSlots * kIdEntries];
+  src.ids = (lds_i32_t)id_ring;
+  src.extra = a.extra_rows;
+  src.t_begin = t_begin;
   auto page_of = [&](int tb) -> int {
     if constexpr (UNIFORM) {
       tb = min(tb, src.last_tok & ~(kTok - 1));
@@ -400,9 +422,14 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
 
   // ---- pipeline: copies run three tiles ahead of the MFMAs (4-slot ring, 148 of the CU's 160 KiB:
   // 111 KiB per CU in flight, which is what HBM latency under load asks for) ----
+  if constexpr (!UNIFORM) {
+    // every wave requests the ids for itself (the same bytes to the same place): no barrier in front of their use
+#pragma unroll
+    for (int k = 0; k < 5; ++k) copy_tile_ids(src, t_begin + k * kTok, lane);
+    wait_all_loads();
+  }
   int pg_next = page_of(t_begin + 3 * kTok);
   auto stage_of = [&](int i) -> char* { return i == 0 ? slot2 : (i == 1 ? slot2 + kF8StageB : slot3); };
-  cover(t_begin);  // (the first three tiles never span a window's 256 pages)
   if constexpr (FP8) {
     copy_tile_f8<UNIFORM>(stage_of(0), src, a.cache, t_begin, wave, lane, page_of(t_begin));
     copy_tile_f8<UNIFORM>(stage_of(1), src, a.cache, t_begin + kTok, wave, lane, page_of(t_begin + kTok));
@@ -419,6 +446,8 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   for (int ks = 0; ks < 18; ++ks) asm volatile("" ::"v"(qB[ks]));
   // wait for the first tile (all but the 10 newest copies), then meet
   constexpr int kAhead = 2 * (FP8 ? kF8CopiesPerWave : kCopiesPerWave);  // copies of the two tiles behind the next one
+  // in the loop a step's id request precedes its copies: the ids it has to wait for are older than both tiles' copies
+  constexpr int kAheadLoop = kAhead + (UNIFORM ? 0 : 1);
   __builtin_amdgcn_s_waitcnt(0x0F70 | kAhead);
   __syncthreads();
   auto bare_barrier = [&]() {
@@ -443,7 +472,7 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
     const int k_off_t = PIPE ? (c_t * kRowB + g_t * 16) : k_off;
     const int v_off_t = PIPE ? ((4 * g_t + (c_t >> 2)) * kRowB + (c_t & 3) * 8) : v_off;
     // `fill` held tile tb - 32, which every wave finished before the last barrier
-    cover(tb + 3 * kTok);
+    if constexpr (!UNIFORM) copy_tile_ids(src, tb + 5 * kTok, lane_t);
     if constexpr (FP8) copy_tile_f8<UNIFORM>(fill, src, a.cache, tb + 3 * kTok, wave, lane_t, pg_next);
     else copy_tile<UNIFORM>(fill, src, a.cache, tb + 3 * kTok, wave, lane_t, pg_next);
     pg_next = page_of(tb + 4 * kTok);
@@ -549,7 +578,7 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
     // wait for ALL outstanding copies, which would shorten the prefetch distance to one tile.
     // Every LDS read of this tile has returned (its MFMA consumed it) before the barrier, and
     // each wave has waited for its own share of the next tile, so no fence is needed.
-    __builtin_amdgcn_s_waitcnt(0x0F70 | kAhead);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | kAheadLoop);
     bare_barrier();
     if constexpr (FP8) expand(next_stage, next_slot);  // tile tb + 32 becomes bf16 rows
   };
@@ -1061,7 +1090,7 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
 // grid = windows of 128 / Hq consecutive query tokens of the call.  A window that lies inside one sequence is one
 // group; one that spans a border between sequences (the end of a chunk, decode rows of one token each) runs one
 // group per sequence, one after the other.
-template <bool PIPE, bool FP8>
+template <bool UNIFORM, bool PIPE, bool FP8>
 __global__ __launch_bounds__(512, 2) void rpa_mla_token_group_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char slot0[kSlotB];
   __shared__ __attribute__((aligned(1024))) char slot1[kSlotB];
@@ -1097,7 +1126,7 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_token_group_kernel(const MlaDe
       MlaDest dest;
       dest.final_rows = true;
       dest.base = 0;
-      mla_segment<true, false, PIPE, FP8, 1, true>(a, mr, 0, t_lo, t_lo & ~(kTok - 1), mr.kv_len, dest, slot0, slot1, slot2,
+      mla_segment<UNIFORM, false, PIPE, FP8, 1, true>(a, mr, 0, t_lo, t_lo & ~(kTok - 1), mr.kv_len, dest, slot0, slot1, slot2,
                                                    slot3, n);
     }
     t += n;
@@ -1476,7 +1505,7 @@ int mla_token_group_mode(const MlaDecodeArgs& a, const Tuning& tune, const Shape
       tune.mla_token_groups == 0 || (128 % a.Hq) != 0 || a.Hq < 16 || a.num_rows < 4 * a.num_seqs)
     return 0;
   const int P = a.pt.page_size;
-  const bool pipe_ok = tune.mla_pipe != 0 && (P & (P - 1)) == 0 && (int64_t)a.row_stride * 2 * P < (int64_t(1) << 32);
+  const bool pipe_ok = tune.mla_pipe != 0 && (P & (P - 1)) == 0 && (P % kTok) == 0 && (int64_t)a.row_stride * 2 * P < (int64_t(1) << 32);
   if (!pipe_ok) return 1;
   if (!a.fp8 && a.sm.window <= 0 && tune.mla_wide != 0 && tune.mla_wide != 32) return 3;
   return 2;
@@ -1507,20 +1536,27 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
       return hipGetLastError();
     }
     if (a.fp8) {
-      if (pipe_ok) hipLaunchKernelGGL((rpa_mla_token_group_kernel<true, true>), tg_grid, block, 0, stream, a);
-      else hipLaunchKernelGGL((rpa_mla_token_group_kernel<false, true>), tg_grid, block, 0, stream, a);
+      if (pipe_ok) hipLaunchKernelGGL((rpa_mla_token_group_kernel<true, true, true>), tg_grid, block, 0, stream, a);
+      else if (uniform) hipLaunchKernelGGL((rpa_mla_token_group_kernel<true, false, true>), tg_grid, block, 0, stream, a);
+      else hipLaunchKernelGGL((rpa_mla_token_group_kernel<false, false, true>), tg_grid, block, 0, stream, a);
     } else {
-      if (pipe_ok) hipLaunchKernelGGL((rpa_mla_token_group_kernel<true, false>), tg_grid, block, 0, stream, a);
-      else hipLaunchKernelGGL((rpa_mla_token_group_kernel<false, false>), tg_grid, block, 0, stream, a);
+      if (pipe_ok) hipLaunchKernelGGL((rpa_mla_token_group_kernel<true, true, false>), tg_grid, block, 0, stream, a);
+      else if (uniform) hipLaunchKernelGGL((rpa_mla_token_group_kernel<true, false, false>), tg_grid, block, 0, stream, a);
+      else hipLaunchKernelGGL((rpa_mla_token_group_kernel<false, false, false>), tg_grid, block, 0, stream, a);
     }
     return hipGetLastError();
   }
   if (ds != 1) {
-#define RPA_MLA_DS(KERNEL, GRID, F8)                                                                                  \
+#define RPA_MLA_DS_U(KERNEL, GRID, U, F8)                                                                            \
   do {                                                                                                                \
-    if (ds == 8) hipLaunchKernelGGL((KERNEL<true, false, false, F8, 8>), GRID, block, 0, stream, a);                 \
-    else if (ds == 4) hipLaunchKernelGGL((KERNEL<true, false, false, F8, 4>), GRID, block, 0, stream, a);            \
-    else hipLaunchKernelGGL((KERNEL<true, false, false, F8, 2>), GRID, block, 0, stream, a);                         \
+    if (ds == 8) hipLaunchKernelGGL((KERNEL<U, false, false, F8, 8>), GRID, block, 0, stream, a);                    \
+    else if (ds == 4) hipLaunchKernelGGL((KERNEL<U, false, false, F8, 4>), GRID, block, 0, stream, a);               \
+    else hipLaunchKernelGGL((KERNEL<U, false, false, F8, 2>), GRID, block, 0, stream, a);                            \
+  } while (0)
+#define RPA_MLA_DS(KERNEL, GRID, F8)                                                                                 \
+  do {                                                                                                                \
+    if (uniform) RPA_MLA_DS_U(KERNEL, GRID, true, F8);                                                                \
+    else RPA_MLA_DS_U(KERNEL, GRID, false, F8);                                                                       \
   } while (0)
     if (a.balanced) {
       const dim3 bgrid(a.num_wgs);
@@ -1534,6 +1570,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     if (a.fp8) RPA_MLA_DS(rpa_mla_decode_kernel, grid, true);
     else RPA_MLA_DS(rpa_mla_decode_kernel, grid, false);
 #undef RPA_MLA_DS
+#undef RPA_MLA_DS_U
     hipError_t es = hipGetLastError();
     if (es != hipSuccess) return es;
     if (a.max_splits > 1) {

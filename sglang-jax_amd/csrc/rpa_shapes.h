@@ -111,14 +111,14 @@ constexpr ShapeRule kShapeRules[] = {
    kKernelMlaWide, 1, 128, 32, 4, 8, 1, 12, "every operand fragment feeds two matrix instructions: C5 226 -> 205 us, prefill chunks 48 -> 55 % of peak; a row switch costs 22 us = 12 tiles (C5 197 -> 191 us against 5)"},
   {"mla_pipe", kStageMla, 0, 576, 128, 0, 128, 0, 0, kOptSoftCap | kOptAsmPages,
    kKernelMlaPipe, 1, 128, 32, 8, 8, 1, 12, "e4m3 latents (bytes staged and expanded once per tile) and RPA_MLA_WIDE=0"},
-  {"mla_shared_16", kStageMla, 0, 576, 1, 16, 0, 0, 0, kOptSoftCap | kOptOddPages,
+  {"mla_shared_16", kStageMla, 0, 576, 1, 16, 0, 0, 0, kOptSoftCap,
    kKernelMlaShared, 1, 16, 32, 8, 8, 8, 8, "a tensor-parallel share of the heads: 64 rows x 8192 tokens 146 -> 120 us"},
-  {"mla_shared_32", kStageMla, 0, 576, 17, 32, 0, 0, 0, kOptSoftCap | kOptOddPages,
+  {"mla_shared_32", kStageMla, 0, 576, 17, 32, 0, 0, 0, kOptSoftCap,
    kKernelMlaShared, 1, 32, 32, 8, 8, 4, 8, "144 -> 126 us"},
-  {"mla_shared_64", kStageMla, 0, 576, 33, 64, 0, 0, 0, kOptSoftCap | kOptOddPages,
+  {"mla_shared_64", kStageMla, 0, 576, 33, 64, 0, 0, 0, kOptSoftCap,
    kKernelMlaShared, 1, 64, 32, 8, 8, 2, 8, "159 -> 147 us"},
   {"mla_compiled", kStageMla, 0, 576, 0, 0, 0, 0, 0, 0,
-   kKernelMlaCompiled, 1, 128, 32, 8, 8, 1, 5, "soft cap, pages under 32 tokens, head counts that are no multiple of 128"},
+   kKernelMlaCompiled, 1, 128, 32, 8, 8, 1, 5, "soft cap; more than 64 heads on pages under 32 tokens or in a count that is no multiple of 128"},
 };
 // clang-format on
 

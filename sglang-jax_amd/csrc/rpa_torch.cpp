@@ -306,6 +306,54 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// The tensors of an absorbed-MLA call: queries, latent cache, new rows.
+struct MlaTensors {
+  const at::Tensor *q, *q_pe, *cache;
+  at::Tensor new_c, new_r;
+  // false: not in the common form
+  bool read(PyObject* const* a, RpaMlaParams& p) {
+    q = tensor(a[0]), q_pe = tensor(a[1]), cache = tensor(a[4]);
+    if (!(q && q_pe && cache && q->is_cuda())) return false;
+    const at::Device dev = q->device();
+    const at::ScalarType kv_type = cache->scalar_type();
+    if (!(q->scalar_type() == at::kBFloat16 && q_pe->scalar_type() == at::kBFloat16 && q->dim() == 3 && q_pe->dim() == 3 &&
+          q->is_contiguous() && q_pe->is_contiguous() && q_pe->device() == dev && q->size(0) == q_pe->size(0) &&
+          q->size(1) == q_pe->size(1)))
+      return false;
+    if (!(cache->device() == dev && cache->is_contiguous() && (cache->dim() == 3 || cache->dim() == 4) &&
+          (kv_type == at::kBFloat16 || kv_type == at::kFloat8_e4m3fn)))
+      return false;
+    const int64_t T = q->size(0), lkv = q->size(2), rope = q_pe->size(2), width = cache->size(-1);
+    if (width == lkv + rope) p.rope_offset = (int32_t)lkv;
+    else if (width == (lkv + 127) / 128 * 128 + (rope + 127) / 128 * 128) p.rope_offset = (int32_t)((lkv + 127) / 128 * 128);
+    else return false;
+    if (!none(a[2])) {
+      const at::Tensor *c = tensor(a[2]), *r = tensor(a[3]);
+      if (!(c && r && c->device() == dev && r->device() == dev && c->scalar_type() == kv_type && r->scalar_type() == kv_type &&
+            c->dim() == 2 && r->dim() == 2 && c->size(0) == T && r->size(0) == T && c->size(1) == lkv && r->size(1) == rope))
+        return false;
+      new_c = c->contiguous();
+      new_r = r->contiguous();
+    } else if (!none(a[3])) {
+      return false;
+    }
+    p.ql_nope = q->const_data_ptr();
+    p.q_pe = q_pe->const_data_ptr();
+    p.cache_kv = cache->const_data_ptr();
+    p.num_tokens = (int32_t)T;
+    p.num_q_heads = (int32_t)q->size(1);
+    p.lkv_dim = (int32_t)lkv;
+    p.rope_dim = (int32_t)rope;
+    p.row_stride = (int32_t)width;
+    p.page_size = (int32_t)(cache->dim() == 3 ? cache->size(1) : cache->size(1) * cache->size(2));
+    p.total_pages = (int32_t)cache->size(0);
+    p.cache_dtype = kv_type == at::kBFloat16 ? RPA_KV_BF16 : RPA_KV_FP8_E4M3;
+    return true;
+  }
+  const void* new_c_ptr() const { return new_c.defined() ? new_c.const_data_ptr() : nullptr; }
+  const void* new_r_ptr() const { return new_r.defined() ? new_r.const_data_ptr() : nullptr; }
+};
+
 // mla(ql_nope, q_pe, new_kv_c, new_k_pe, cache, kv_lens, page_indices, cu_q_lens, cu_kv_lens, distribution, sm_scale,
 //     sliding_window, soft_cap, mask_value, q_scale, k_scale, v_scale, max_kv_len, num_splits, sum_kv_len)
 // -> output, a status below 0, or None.
@@ -315,33 +363,10 @@ PyObject* mla(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     PyErr_SetString(PyExc_TypeError, "mla takes 20 arguments");
     return nullptr;
   }
-  const at::Tensor *q = tensor(a[0]), *q_pe = tensor(a[1]), *cache = tensor(a[4]);
-  COMMON(q && q_pe && cache && q->is_cuda());
-  const at::Device dev = q->device();
-  const at::ScalarType kv_type = cache->scalar_type();
-  COMMON(q->scalar_type() == at::kBFloat16 && q_pe->scalar_type() == at::kBFloat16 && q->dim() == 3 && q_pe->dim() == 3 &&
-         q->is_contiguous() && q_pe->is_contiguous() && q_pe->device() == dev && q->size(0) == q_pe->size(0) &&
-         q->size(1) == q_pe->size(1));
-  COMMON(cache->device() == dev && cache->is_contiguous() && (cache->dim() == 3 || cache->dim() == 4) &&
-         (kv_type == at::kBFloat16 || kv_type == at::kFloat8_e4m3fn));
-  const int64_t T = q->size(0), Hq = q->size(1), lkv = q->size(2), rope = q_pe->size(2);
-  const int64_t width = cache->size(-1), page = cache->dim() == 3 ? cache->size(1) : cache->size(1) * cache->size(2);
   RpaMlaParams p = {};
-  if (width == lkv + rope) p.rope_offset = (int32_t)lkv;
-  else if (width == (lkv + 127) / 128 * 128 + (rope + 127) / 128 * 128) p.rope_offset = (int32_t)((lkv + 127) / 128 * 128);
-  else Py_RETURN_NONE;
-
-  at::Tensor new_c, new_r;
-  if (!none(a[2])) {
-    const at::Tensor *c = tensor(a[2]), *r = tensor(a[3]);
-    COMMON(c && r && c->device() == dev && r->device() == dev && c->scalar_type() == kv_type &&
-           r->scalar_type() == kv_type && c->dim() == 2 && r->dim() == 2 && c->size(0) == T && r->size(0) == T &&
-           c->size(1) == lkv && r->size(1) == rope);
-    new_c = c->contiguous();
-    new_r = r->contiguous();
-  } else {
-    COMMON(none(a[3]));
-  }
+  MlaTensors x;
+  COMMON(x.read(a, p));
+  const at::Device dev = x.q->device();
   const at::Tensor* kv_lens = on_device(a[5], dev, at::kInt);
   const at::Tensor* pages = on_device(a[6], dev, at::kInt);
   const at::Tensor* cu_q = on_device(a[7], dev, at::kInt);
@@ -383,33 +408,72 @@ PyObject* mla(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     p.sum_kv_len = v;
   }
 
-  at::Tensor out = at::empty_like(*q);
+  at::Tensor out = at::empty_like(*x.q);
   void* stream = stream_of(dev);
-  p.ql_nope = q->const_data_ptr();
-  p.q_pe = q_pe->const_data_ptr();
   p.out = out.data_ptr();
-  p.cache_kv = cache->const_data_ptr();
   p.kv_lens = kv_lens->const_data_ptr<int32_t>();
   p.page_indices = pages->const_data_ptr<int32_t>();
   p.cu_q_lens = cu_q->const_data_ptr<int32_t>();
   p.distribution = dist.device;
-  p.num_tokens = (int32_t)T;
   p.num_seqs = dist.device ? (int32_t)kv_lens->size(0) : (int32_t)dist.k;
-  p.num_q_heads = (int32_t)Hq;
-  p.lkv_dim = (int32_t)lkv;
-  p.rope_dim = (int32_t)rope;
-  p.row_stride = (int32_t)width;
-  p.page_size = (int32_t)page;
-  p.total_pages = (int32_t)cache->size(0);
-  p.cache_dtype = kv_type == at::kBFloat16 ? RPA_KV_BF16 : RPA_KV_FP8_E4M3;
   if (const size_t need = decode_only ? rpa_mla_workspace_bytes(&p) : rpa_mla_attention_workspace_bytes(&p)) {
     at::Tensor& ws = workspace(dev, stream, need);
     p.workspace = ws.data_ptr();
     p.workspace_bytes = (size_t)ws.numel();
   }
-  const void* cp = new_c.defined() ? new_c.const_data_ptr() : nullptr;
-  const void* rp = new_r.defined() ? new_r.const_data_ptr() : nullptr;
-  const int rc = without_gil([&] { return rpa_mla_attention_update(&p, cp, rp, decode_only ? 0 : 1, stream); });
+  const int rc = without_gil([&] { return rpa_mla_attention_update(&p, x.new_c_ptr(), x.new_r_ptr(), decode_only ? 0 : 1, stream); });
+  if (rc != RPA_OK) return PyLong_FromLong(rc);
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// sparse_mla(ql_nope, q_pe, new_kv_c, new_k_pe, cache, kv_lens, topk, topk_is_pages, page_indices, cu_q_lens, cu_kv_lens,
+//            sm_scale, page_size, pages_per_seq, k_pages_max)
+// -> output, a status below 0, or None.  k_pages_max 0: single tokens, else whole pages.
+PyObject* sparse_mla(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 15) {
+    PyErr_SetString(PyExc_TypeError, "sparse_mla takes 15 arguments");
+    return nullptr;
+  }
+  RpaMlaParams p = {};
+  MlaTensors x;
+  COMMON(x.read(a, p));
+  const at::Device dev = x.q->device();
+  const at::Tensor* kv_lens = on_device(a[5], dev, at::kInt);
+  const at::Tensor* topk = on_device(a[6], dev, at::kInt);
+  const at::Tensor* pages = on_device(a[8], dev, at::kInt);
+  const at::Tensor* cu_q = on_device(a[9], dev, at::kInt);
+  const at::Tensor* cu_kv = on_device(a[10], dev, at::kInt);
+  COMMON(kv_lens && topk && pages && cu_q && cu_kv && kv_lens->dim() == 1 && topk->dim() == 2 &&
+         topk->size(0) == x.q->size(0) && cu_q->numel() == kv_lens->size(0) + 1 && cu_kv->numel() == kv_lens->size(0) + 1);
+  RpaMlaSparse s = {};
+  int64_t page, per_seq, most;
+  double scale;
+  COMMON(real(a[11], scale) && whole(a[12], page) && whole(a[13], per_seq) && whole(a[14], most));
+  COMMON(page == p.page_size && most >= 0 && topk->size(1) <= INT32_MAX && pages->numel() <= INT32_MAX);
+  s.topk = topk->const_data_ptr<int32_t>();
+  s.topk_is_pages = PyObject_IsTrue(a[7]) == 1;
+  s.topk_stride = (int32_t)topk->size(1);
+  // precomputed pages: the last of a row's k_pages_max entries is the new token's
+  s.topk_count = s.topk_is_pages ? (int32_t)std::min<int64_t>(s.topk_stride, most - 1) : s.topk_stride;
+  s.pages_per_seq = (int32_t)per_seq;
+  s.k_pages_max = (int32_t)most;
+  s.num_page_indices = (int32_t)pages->numel();
+  p.sm_scale = (float)scale;
+  p.kv_lens = kv_lens->const_data_ptr<int32_t>();
+  p.page_indices = pages->const_data_ptr<int32_t>();
+  p.cu_q_lens = cu_q->const_data_ptr<int32_t>();
+  p.cu_kv_lens = cu_kv->const_data_ptr<int32_t>();
+  p.num_seqs = (int32_t)kv_lens->size(0);
+  at::Tensor out = at::empty_like(*x.q);
+  void* stream = stream_of(dev);
+  p.out = out.data_ptr();
+  const size_t need = rpa_mla_sparse_workspace_bytes(&p, &s);
+  at::Tensor& ws = workspace(dev, stream, need);
+  p.workspace = ws.data_ptr();
+  p.workspace_bytes = (size_t)ws.numel();
+  const int rc = without_gil([&] { return rpa_mla_sparse_attention(&p, &s, x.new_c_ptr(), x.new_r_ptr(), stream); });
   if (rc != RPA_OK) return PyLong_FromLong(rc);
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
@@ -431,6 +495,7 @@ PyObject* py_workspace(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 PyMethodDef kMethods[] = {
     {"attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(attention)), METH_FASTCALL, nullptr},
     {"mla", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(mla)), METH_FASTCALL, nullptr},
+    {"sparse_mla", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(sparse_mla)), METH_FASTCALL, nullptr},
     {"workspace", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(py_workspace)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -1,7 +1,7 @@
 """Sparse absorbed-MLA (DeepSeek sparse attention) on the dense MLA kernels: the reference's
 ``python/sgl_jax/srt/kernels/dsa/sparse_mla.py`` re-indexes the page table (or gathers rows) and
-hands the result to its dense kernel; the same is done here in front of
-``mla_ragged_paged_attention`` (mla.py, HIP kernels behind ``rpa_mla_*``).  All index work stays
+hands the result to its dense kernel; here ``rpa_mla_sparse_attention`` writes one page table per query
+token and runs the dense kernel over it, three launches in all.  All index work stays
 on the device (no host reads), so a call can sit inside a captured step.
 
 * ``compute_topk_pages``     sparse_mla.py:35-60   unique pages a top-k list touches
@@ -13,7 +13,7 @@ from __future__ import annotations
 
 import torch
 
-from .mla import mla_ragged_paged_attention
+from . import _lib
 from .ragged_paged_attention import _i32, _require_gpu
 
 
@@ -46,100 +46,51 @@ def compute_topk_pages(topk_indices, *, page_size: int, pages_per_seq: int, k_pa
     return torch.where(col < n_hit[:, None], hit, torch.full_like(hit, -1)).to(torch.int32)
 
 
+def _sparse(ql_nope, q_pe, new_kv_c, new_k_pe, cache_kv, kv_lens, topk, topk_is_pages, page_indices, cu_q_lens,
+            cu_kv_lens, sm_scale, page_size, pages_per_seq, k_pages_max):
+    """The table of every query token's selection and the dense kernel over it (csrc/rpa_dsa.hip, rpa_mla.hip)."""
+    native = _lib.load_torch().sparse_mla
+    rest = (sm_scale, page_size, pages_per_seq, k_pages_max)
+    o = native(ql_nope, q_pe, new_kv_c, new_k_pe, cache_kv, kv_lens, topk, topk_is_pages, page_indices, cu_q_lens,
+               cu_kv_lens, *rest)
+    if o is None:  # host metadata, wide indices, strided rows: brought into the common form
+        _require_gpu(ql_nope, "ql_nope")
+        _require_gpu(cache_kv, "cache_kv")
+        dev = ql_nope.device
+        o = native(ql_nope.contiguous(), q_pe.contiguous(), new_kv_c, new_k_pe, cache_kv, _i32(kv_lens, dev),
+                   topk.to(dev).to(torch.int32).contiguous(), topk_is_pages, _i32(page_indices, dev).reshape(-1),
+                   _i32(cu_q_lens, dev), _i32(cu_kv_lens, dev), *rest)
+        if o is None:
+            raise ValueError(f"Expected bfloat16 queries [T, heads, lkv] and [T, heads, rope], a contiguous bfloat16 or float8_e4m3fn "
+                             f"cache of pages of {page_size} rows of lkv + rope elements (or each rounded up to 128), new rows of the "
+                             f"cache's dtype and one row of indices per query token; got {tuple(ql_nope.shape)} {ql_nope.dtype}, "
+                             f"{tuple(q_pe.shape)} {q_pe.dtype}, {tuple(cache_kv.shape)} {cache_kv.dtype}, {tuple(topk.shape)}")
+    if type(o) is int:
+        _lib.check(o)
+    return o
+
+
 def sparse_mla_page_level(ql_nope, q_pe, new_kv_c, new_k_pe, cache_kv, kv_lens, topk_indices, page_indices,
                           cu_q_lens, cu_kv_lens, distribution, topk_pages=None, *, sm_scale: float, page_size: int,
                           pages_per_seq: int, kv_lora_rank: int, k_pages_max: int = 64, **_tile_hints):
     """Decode (one query token per sequence): attends the whole pages that ``topk_indices``
-    touches plus the page of the new token, which goes last so that the kernel's cache write
+    touches (or ``topk_pages`` names) plus the page of the new token, which goes last so that the new row
     lands in the true slot (sparse_mla.py:63-203).  Returns ``(o_latent, cache_kv)``; the last
     page of the cache is the padding target, as in the reference."""
-    _require_gpu(ql_nope, "ql_nope")
-    dev = ql_nope.device
-    T = ql_nope.shape[0]
-    kv_lens_d, page_d = _i32(kv_lens, dev).to(torch.int64), _i32(page_indices, dev).reshape(-1).to(torch.int64)
-    cu_q_d, cu_kv_d = _i32(cu_q_lens, dev).to(torch.int64), _i32(cu_kv_lens, dev).to(torch.int64)
-    S = kv_lens_d.shape[0]
-    tok = torch.arange(T, device=dev)
-    seq_id = torch.clamp(torch.searchsorted(cu_q_d[1:].contiguous(), tok, right=True), 0, S - 1)
-    tok_valid = kv_lens_d[seq_id] > 0
-    seq_page_start = cu_kv_d[seq_id] // page_size
-    new_abs = torch.clamp(kv_lens_d[seq_id] - 1, min=0)
-    new_page_local = new_abs // page_size
-    new_off = new_abs % page_size
-    kp = k_pages_max
-    if topk_pages is not None:
-        raw = topk_pages.to(dev).to(torch.int64)[:, : kp - 1]
-        ok = (raw >= 0) & (raw != new_page_local[:, None])
-        n_hit = torch.clamp(ok.sum(dim=1), max=kp - 1)
-        big = torch.iinfo(torch.int32).max
-        hit = torch.sort(torch.where(ok, raw, torch.full_like(raw, big)), dim=1).values
-        if hit.shape[1] < kp - 1:
-            hit = torch.nn.functional.pad(hit, (0, kp - 1 - hit.shape[1]))
-    else:
-        idx = topk_indices.to(dev).to(torch.int64)
-        valid = idx >= 0
-        page_local = torch.where(valid, idx // page_size, torch.full_like(idx, pages_per_seq))
-        mask = torch.zeros((T, pages_per_seq + 1), dtype=torch.bool, device=dev)
-        mask.scatter_(1, page_local, torch.ones_like(page_local, dtype=torch.bool))
-        mask = mask[:, :pages_per_seq]
-        mask &= torch.arange(pages_per_seq, device=dev)[None, :] != new_page_local[:, None]
-        n_hit = torch.clamp(mask.sum(dim=1), max=kp - 1)
-        hit = _first_hits(mask, min(kp - 1, pages_per_seq))
-        if hit.shape[1] < kp - 1:
-            hit = torch.nn.functional.pad(hit, (0, kp - 1 - hit.shape[1]))
-    n_used = n_hit + 1
-    col = torch.arange(kp, device=dev)[None, :]
-    hit_p = torch.nn.functional.pad(hit, (0, 1))
-    sp_local = torch.where(col < n_hit[:, None], hit_p,
-                           torch.where(col == n_hit[:, None], new_page_local[:, None], torch.zeros_like(hit_p)))
-    gather_at = torch.clamp(seq_page_start[:, None] + sp_local, 0, page_d.numel() - 1)
-    sentinel = cache_kv.shape[0] - 1
-    sp_phys = torch.where((col < n_used[:, None]) & tok_valid[:, None], page_d[gather_at],
-                          torch.full_like(gather_at, sentinel))
-    sp_kv_len = (n_hit * page_size + new_off + 1).to(torch.int32)
-    sp_cu_q = torch.arange(T + 1, dtype=torch.int32, device=dev)
-    sp_cu_kv = sp_cu_q * (kp * page_size)
-    o, cache_out = mla_ragged_paged_attention(
-        ql_nope, q_pe, new_kv_c, new_k_pe, cache_kv, sp_kv_len, sp_phys.reshape(-1).to(torch.int32), sp_cu_q,
-        sp_cu_kv, (T, T, T), sm_scale=sm_scale, sliding_window=None, soft_cap=None,
-        max_kv_len=kp * page_size, sum_kv_len=0)
-    return o[..., :kv_lora_rank], cache_out
+    pre = topk_pages is not None
+    o = _sparse(ql_nope, q_pe, new_kv_c, new_k_pe, cache_kv, kv_lens, topk_pages if pre else topk_indices, pre, page_indices,
+                cu_q_lens, cu_kv_lens, sm_scale, page_size, pages_per_seq, k_pages_max)
+    cache_out = cache_kv if cache_kv.dim() == 3 else cache_kv.view(cache_kv.shape[0], -1, cache_kv.shape[3])
+    return o if o.shape[-1] == kv_lora_rank else o[..., :kv_lora_rank], cache_out
 
 
 def sparse_mla_via_dense(ql_nope, q_pe, new_kv_c, new_k_pe, cache_kv, kv_lens, topk_indices, page_indices,
                          cu_q_lens, cu_kv_lens, distribution, *, sm_scale: float, page_size: int,
                          pages_per_seq: int, kv_lora_rank: int, **_tile_hints) -> torch.Tensor:
-    """Token-level sparse attention for any T: the k selected rows of every query token are
-    gathered into a temporary paged buffer (k rows = one short "sequence" per token) and the
-    dense kernel runs over it with ``kv_len`` = number of valid entries; the new token's row
-    replaces the last valid entry, as the dense kernel's cache write does in the reference
-    (sparse_mla.py:206-297).  Valid entries must come first in each row."""
-    _require_gpu(ql_nope, "ql_nope")
-    dev = ql_nope.device
-    T = ql_nope.shape[0]
-    cache3 = cache_kv.view(cache_kv.shape[0], -1, cache_kv.shape[-1]) if cache_kv.dim() == 4 else cache_kv
-    width = cache3.shape[-1]
-    idx = topk_indices.to(dev).to(torch.int64)
-    k = idx.shape[1]
-    kv_lens_d, page_d = _i32(kv_lens, dev).to(torch.int64), _i32(page_indices, dev).reshape(-1).to(torch.int64)
-    cu_q_d, cu_kv_d = _i32(cu_q_lens, dev).to(torch.int64), _i32(cu_kv_lens, dev).to(torch.int64)
-    S = kv_lens_d.shape[0]
-    seq_id = torch.clamp(torch.searchsorted(cu_q_d[1:].contiguous(), torch.arange(T, device=dev), right=True), 0, S - 1)
-    seq_page_start = cu_kv_d[seq_id] // page_size
-    valid = idx >= 0
-    safe = torch.where(valid, idx, torch.zeros_like(idx))
-    phys = page_d[torch.clamp(seq_page_start[:, None] + safe // page_size, 0, page_d.numel() - 1)]
-    slot = phys * page_size + safe % page_size
-    rows = cache3.reshape(-1, width).index_select(0, slot.reshape(-1)).reshape(T, k, width)
-    rows = torch.where(valid[..., None], rows, torch.zeros_like(rows))
-    n_tmp = -(-k // page_size)
-    tmp = torch.zeros((T * n_tmp + 1, page_size, width), dtype=cache3.dtype, device=dev)
-    tmp[: T * n_tmp].view(T, n_tmp * page_size, width)[:, :k] = rows
-    tmp_kv_lens = valid.sum(dim=1).to(torch.int32)
-    tmp_pages = torch.arange(T * n_tmp, dtype=torch.int32, device=dev)
-    tmp_cu_q = torch.arange(T + 1, dtype=torch.int32, device=dev)
-    tmp_cu_kv = tmp_cu_q * (n_tmp * page_size)
-    o, _ = mla_ragged_paged_attention(
-        ql_nope, q_pe, new_kv_c, new_k_pe, tmp, tmp_kv_lens, tmp_pages, tmp_cu_q, tmp_cu_kv, (T, T, T),
-        sm_scale=sm_scale, sliding_window=None, soft_cap=None, max_kv_len=n_tmp * page_size, sum_kv_len=0)
-    return o[..., :kv_lora_rank]
+    """Token-level sparse attention for any T: the k selected rows of every query token are one short
+    "sequence" of pages of a single row, ``kv_len`` = number of valid entries; the new token's row
+    stands for the last valid entry, where the dense kernel's cache write puts it in the reference
+    (sparse_mla.py:206-297; the reference gathers the rows first).  Valid entries must come first in each row."""
+    o = _sparse(ql_nope, q_pe, new_kv_c, new_k_pe, cache_kv, kv_lens, topk_indices, False, page_indices, cu_q_lens, cu_kv_lens,
+                sm_scale, page_size, pages_per_seq, 0)
+    return o if o.shape[-1] == kv_lora_rank else o[..., :kv_lora_rank]

@@ -121,3 +121,51 @@ def test_page_level_selection(pkg, wl, gpu, precomputed):
     torch.cuda.synchronize()
     assert_parity(got.cpu().float(), want.float(), **TOL)
     assert torch.equal(cache_out.cpu(), b.cache_kv)  # every new row back in its slot, nothing else touched
+
+
+@pytest.mark.parametrize("level", ["page", "token"])
+@pytest.mark.parametrize("P,Hq,k,dtype", [(16, 16, 2048, "bf16"), (64, 64, 300, "bf16"), (16, 128, 33, "bf16"), (24, 40, 65, "bf16"),
+                                          (128, 32, 512, "e4m3"), (16, 128, 96, "e4m3")])
+def test_selections_of_every_shape(pkg, wl, gpu, level, P, Hq, k, dtype):
+    """Head counts of every workgroup shape, pages below and above a tile, selections that end inside one, rows cut in pieces;
+    lengths from one token to far more than the selection."""
+    kv_lens, kp = [1, 2, 31, P, P + 1, 700, 5003], 40
+    b = batch(wl, kv_lens, P, 83, Hq=Hq)
+    topk_np = draw_topk(kv_lens, k, 8)
+    S, pps = len(kv_lens), -(-max(kv_lens) // P)
+    pages = torch.cat([b.page_indices, torch.zeros(pps, dtype=torch.int32)])
+    dt = torch.float8_e4m3fn if dtype == "e4m3" else torch.bfloat16
+    stored = b.cache_kv.to(dt)
+    ref_cache = stored.to(torch.bfloat16)
+    say(f"dsa {level} P={P} Hq={Hq} k={k} {dtype}")
+    if level == "token":
+        want = sparse_mla_ref(torch.cat([b.ql_nope, b.q_pe], dim=-1), ref_cache, b.kv_lens, torch.from_numpy(topk_np), pages,
+                              b.cu_q_lens, b.cu_kv_lens, [S, S, S], sm_scale=b.sm_scale, pages_per_seq=pps, v_dim=512)
+    else:
+        sp_len, sp_pages = page_level_metadata_ref(b.kv_lens.numpy(), topk_np, b.page_indices.numpy(), b.cu_q_lens.numpy(),
+                                                   b.cu_kv_lens.numpy(), page_size=P, pages_per_seq=pps, k_pages_max=kp,
+                                                   sentinel_page=stored.shape[0] - 1)
+        want, _ = ref_mla_ragged_paged_attention(
+            b.ql_nope, b.q_pe, None, None, ref_cache, torch.from_numpy(sp_len), torch.from_numpy(sp_pages).reshape(-1),
+            torch.arange(S + 1, dtype=torch.int32), [S, S, S], sm_scale=b.sm_scale)
+    new_c = torch.zeros(S, 512, dtype=torch.bfloat16).to(dt)
+    new_r = torch.zeros(S, 64, dtype=torch.bfloat16).to(dt)
+    cache, o = stored.clone(), 0
+    for i, n in enumerate(kv_lens):
+        page, off = int(b.page_indices[o + (n - 1) // P]), (n - 1) % P
+        new_c[i], new_r[i] = cache[page, off, :512], cache[page, off, 512:]
+        cache.view(torch.uint8)[page, off] = 0
+        o += -(-n // P)
+    g, cache = b.to(gpu), cache.to(gpu)
+    args = (g.ql_nope, g.q_pe, new_c.to(gpu), new_r.to(gpu), cache, g.kv_lens, torch.from_numpy(topk_np).to(gpu), g.page_indices,
+            g.cu_q_lens, g.cu_kv_lens, (S, S, S))
+    common = dict(sm_scale=b.sm_scale, page_size=P, pages_per_seq=pps, kv_lora_rank=512)
+    if level == "token":
+        before = cache.view(torch.uint8).clone()
+        got = pkg.sparse_mla_via_dense(*args, **common)
+        assert torch.equal(cache.view(torch.uint8), before)
+    else:
+        got, cache_out = pkg.sparse_mla_page_level(*args, k_pages_max=kp, **common)
+        assert torch.equal(cache_out.cpu().view(torch.uint8), stored.view(torch.uint8))
+    torch.cuda.synchronize()
+    assert_parity(got.cpu().float(), want.float(), **TOL)
