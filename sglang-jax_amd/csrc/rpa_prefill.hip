@@ -36,77 +36,19 @@ using namespace pf;
 namespace {
 
 
-// ---- fp8 rows into the same LDS layout (the 256-wide heads' fp8 path) ----
-// Thread tid stages a quarter of K row and V row (tid >> 2): HD / 4 bytes of e4m3 each, loaded
-// two tiles ahead into registers, widened to bf16 and written one tile ahead to the chunk
-// positions the asynchronous copy would have used, so the products read both caches alike.
-template <int HD>
-struct Fp8Stage {
-  u32x4_t k[HD / 64], v[HD / 64];
-};
-
-template <bool UNIFORM>
-__device__ __forceinline__ int32_t fp8_fetch_page(const TileSrc& s, int tb, int tid) {
-  tb = min(tb, s.last_tok & ~(kBN - 1));
-  if constexpr (UNIFORM) {
-    return scalar_load_i32(s.pages + __builtin_amdgcn_readfirstlane(page_slot(s, tb)));
-  } else {
-    return s.pages[page_slot(s, min(tb + (tid >> 2), s.last_tok))];
-  }
-}
-
-template <bool UNIFORM, int HD>
-__device__ __forceinline__ void fp8_gload(Fp8Stage<HD>& st, const TileSrc& s, const KvAddr& kv, const char* kh,
-                                          const char* vh, int tb, int tid, int32_t page) {
-  tb = min(tb, s.last_tok & ~(kBN - 1));  // past the end: re-read the last tile
-  const int64_t ro = row_offset<UNIFORM>(s, kv, tb, tb + (tid >> 2), page) + (tid & 3) * (HD / 4);
-#pragma unroll
-  for (int i = 0; i < HD / 64; ++i) {
-    st.k[i] = ld16(kh + ro + i * 16);
-    st.v[i] = ld16(vh + ro + i * 16);
-  }
-}
-
-template <int HD>
-__device__ __forceinline__ void fp8_lstore(const Fp8Stage<HD>& st, char* lds_k, char* lds_v, int tid) {
-  const int t = tid >> 2;
-  char* kr = lds_k + t * Tile<HD>::kRowB;
-  char* vr = lds_v + t * Tile<HD>::kRowB;
-  const int ks = t & 15, vs = (t & 3) << 2;
-#pragma unroll
-  for (int i = 0; i < HD / 64; ++i) {
-    const int j = (tid & 3) * (HD / 32) + 2 * i;  // the first of the two bf16 chunks these 16 bytes widen to
-    {
-      const u32x2_t a = fp8x4_to_bf16x4(st.k[i][0]), b = fp8x4_to_bf16x4(st.k[i][1]);
-      const u32x2_t c = fp8x4_to_bf16x4(st.k[i][2]), d = fp8x4_to_bf16x4(st.k[i][3]);
-      lds_st16(kr + ((j ^ ks) << 4), u32x4_t{a[0], a[1], b[0], b[1]});
-      lds_st16(kr + (((j + 1) ^ ks) << 4), u32x4_t{c[0], c[1], d[0], d[1]});
-    }
-    {
-      const u32x2_t a = fp8x4_to_bf16x4(st.v[i][0]), b = fp8x4_to_bf16x4(st.v[i][1]);
-      const u32x2_t c = fp8x4_to_bf16x4(st.v[i][2]), d = fp8x4_to_bf16x4(st.v[i][3]);
-      lds_st16(vr + ((j ^ vs) << 4), u32x4_t{a[0], a[1], b[0], b[1]});
-      lds_st16(vr + (((j + 1) ^ vs) << 4), u32x4_t{c[0], c[1], d[0], d[1]});
-    }
-  }
-}
-
 // EXT compiles in the rarely used options (temperature factor, custom mask / no mask); the
 // plain causal instantiation keeps its scale in a scalar register and its mask test to one compare.
-// HD = 256 doubles the rows in LDS (two 64 KiB slots), the Q^T operands and the accumulators: one
-// workgroup per CU, one wave per SIMD with up to 512 registers.
-// FP8: an e4m3 cache staged through registers into the same LDS layout (see above).
 // HEADS4: the short-chunk tile (chunks of at most 64 tokens: a verify step, a short prompt).  A workgroup owns 32
 // query positions of FOUR query heads of a kv head, one head per wave, instead of 128 positions of one head:
 // such chunks then fill their tiles, and the four waves still share every K/V tile.
-template <bool UNIFORM, bool CAP, bool EXT, int HD = 128, bool FP8 = false, bool HEADS4 = false>
-__global__ __launch_bounds__(256, (HD == 128 ? 2 : 1)) void rpa_prefill_async_kernel(const PrefillArgs a_in, int tiles, int nseq,
-                                                                                  bool by_level) {
+template <bool UNIFORM, bool CAP, bool EXT, bool HEADS4 = false>
+__global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const PrefillArgs a_in, int tiles, int nseq, bool by_level) {
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
     a.seq_end = min(a.seq_end, scalar_load_i32(a.dist + 2));
   }
+  constexpr int HD = 128;
   using T = Tile<HD>;
   constexpr int kRowB = T::kRowB;
   constexpr int kTileB = T::kTileB;
@@ -118,7 +60,6 @@ __global__ __launch_bounds__(256, (HD == 128 ? 2 : 1)) void rpa_prefill_async_ke
   __shared__ __attribute__((aligned(1024))) char lds_v0[kTileB];
   __shared__ __attribute__((aligned(1024))) char lds_v1[kTileB];
 
-  static_assert(!HEADS4 || (HD == 128 && !FP8), "the short-chunk tile exists for 128-wide heads on bf16 caches");
   constexpr int BM = HEADS4 ? 32 : kBM;  // query positions per workgroup
   Work w = decompose(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
   if (!w.valid) return;
@@ -147,7 +88,7 @@ __global__ __launch_bounds__(256, (HD == 128 ? 2 : 1)) void rpa_prefill_async_ke
     for (int ks = 0; ks < T::kSteps; ++ks) qB[ks] = ld16(qp + ks * 16);
     if (EXT && a.sm.q_scale > 0.f) {
 #pragma unroll
-      for (int ks = 0; ks < T::kSteps; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, FP8);
+      for (int ks = 0; ks < T::kSteps; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, false);
     }
   }
   Softmax<CAP> sm;
@@ -210,42 +151,24 @@ __global__ __launch_bounds__(256, (HD == 128 ? 2 : 1)) void rpa_prefill_async_ke
   }
 
   // ---- pipeline: page ids two tiles ahead, the asynchronous copy one tile ahead ----
-  AsyncOffsets<HD> ofs;
+  const AsyncOffsets<HD> ofs = make_async_offsets<HD>(a.kv, wave, lane);
   AsyncPages<UNIFORM, HD> pg;
-  Fp8Stage<HD> stg;     // FP8: rows of the tile after the next one
-  int32_t fp8_page = 0;  // FP8: page of this thread's row in the tile loaded next
-  if constexpr (FP8) {
-    fp8_page = fp8_fetch_page<UNIFORM>(src, t_lo, tid);
-    fp8_gload<UNIFORM, HD>(stg, src, a.kv, kh, vh, t_lo, tid, fp8_page);
-    fp8_page = fp8_fetch_page<UNIFORM>(src, t_lo + kBN, tid);
-    fp8_lstore<HD>(stg, lds_k0, lds_v0, tid);
-    fp8_gload<UNIFORM, HD>(stg, src, a.kv, kh, vh, t_lo + kBN, tid, fp8_page);
-    fp8_page = fp8_fetch_page<UNIFORM>(src, t_lo + 2 * kBN, tid);
-  } else {
-    ofs = make_async_offsets<HD>(a.kv, wave, lane);
-    async_fetch_pages<UNIFORM, HD>(pg, src, t_lo, wave, lane);
-    async_copy_tile<UNIFORM, HD>(lds_k0, lds_v0, src, a.kv, kh, vh, t_lo, wave, lane, pg, ofs);
-    async_fetch_pages<UNIFORM, HD>(pg, src, t_lo + kBN, wave, lane);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the copies have landed in LDS
-  }
+  async_fetch_pages<UNIFORM, HD>(pg, src, t_lo, wave, lane);
+  async_copy_tile<UNIFORM, HD>(lds_k0, lds_v0, src, a.kv, kh, vh, t_lo, wave, lane, pg, ofs);
+  async_fetch_pages<UNIFORM, HD>(pg, src, t_lo + kBN, wave, lane);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the copies have landed in LDS
   __syncthreads();
 
   // one tile: consume (lds_k, lds_v), fill (nxt_k, nxt_v) with the tile after it
   auto tile_step = [&](const char* lds_k, const char* lds_v, char* nxt_k, char* nxt_v, int tb) {
     uint64_t mask_word = 0;  // a caller's mask turned into bits by the pre-pass: one word per lane and tile
-    if constexpr (EXT && HD == 128) {
+    if constexpr (EXT) {
       if (mc.mode == 1 && mc.bits) mask_word = mc.bits[min(tb >> 6, mc.bit_words - 1)];
     }
     if (tb + kBN < t_hi) {
       // the other slot was last read before the barrier that ended the previous tile
-      if constexpr (FP8) {
-        fp8_lstore<HD>(stg, nxt_k, nxt_v, tid);
-        fp8_gload<UNIFORM, HD>(stg, src, a.kv, kh, vh, tb + 2 * kBN, tid, fp8_page);
-        fp8_page = fp8_fetch_page<UNIFORM>(src, tb + 3 * kBN, tid);
-      } else {
-        async_copy_tile<UNIFORM, HD>(nxt_k, nxt_v, src, a.kv, kh, vh, tb + kBN, wave, lane, pg, ofs);
-        async_fetch_pages<UNIFORM, HD>(pg, src, tb + 2 * kBN, wave, lane);
-      }
+      async_copy_tile<UNIFORM, HD>(nxt_k, nxt_v, src, a.kv, kh, vh, tb + kBN, wave, lane, pg, ofs);
+      async_fetch_pages<UNIFORM, HD>(pg, src, tb + 2 * kBN, wave, lane);
     }
     // visible to this wave?  causal: some token <= last row's position; window: some token
     // newer than the first row's horizon
@@ -280,7 +203,7 @@ __global__ __launch_bounds__(256, (HD == 128 ? 2 : 1)) void rpa_prefill_async_ke
             }
       }
     }
-    if constexpr (!FP8) __builtin_amdgcn_s_waitcnt(0x0F70);  // the next tile has landed
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // the next tile has landed
     __syncthreads();
   };
   for (int tb = t_lo; tb < t_hi; tb += 2 * kBN) {
@@ -291,6 +214,377 @@ __global__ __launch_bounds__(256, (HD == 128 ? 2 : 1)) void rpa_prefill_async_ke
   if (a.kv_splits > 1) write_partial_rows<T::kDimTiles>(a, w, wr, O, l, h, m * sm.sc2, split);
   else write_rows<T::kDimTiles>(a, w, wr, O, l, h, m * sm.sc2);
 }
+
+}  // namespace
+
+// ==================================================================== 256-wide heads
+// A workgroup owns 128 query positions of one query head with EIGHT waves of 16 positions (16x16x32 matrix
+// instructions), two waves per SIMD.  A wave holds Q^T of its positions (32 registers), O^T (64), the scores of a 64-token
+// tile (16) and the probabilities of the one before.  With four waves of 32 positions and 512 registers, what was here
+// before, a lone wave per SIMD had its operand reads and its exponentials exposed, and the compiler moved operands through
+// the accumulation registers and drained the loads in flight to make room.  The price is LDS: every wave reads the whole
+// K and V tile, 512 KiB per tile and CU, 2300 clocks (3.7 per ds_read_b128, 2.6 per transposing read) against 2048 of the
+// matrix pipe.  Counters (e4m3, soft cap, window): LDS 31 %, vector pipe 30 %, matrix pipe 20 % of the clocks, a quarter
+// lost to the packing of 704 workgroups on 256 CUs: no pipe is full, the waves of a CU go through its phases together.
+// (Eight waves as pairs that share 32 positions, one set of scores each, and exchange their probabilities through LDS --
+// half the reads -- spilled 50 registers at 256: 423 us.)
+// Measured: 6 chunks of 300 .. 1500 tokens x 16 heads, e4m3, soft cap, window 1024 (89 GFLOP) 424 -> 258 us; 3 bf16 prompts of
+// 1490 .. 2883 tokens x 16 heads on 16-token pages 182 -> 135 us.
+namespace {
+
+constexpr int kWRowB = 512;                // a K or V row in LDS
+constexpr int kWTileB = kBN * kWRowB;      // 32 KiB
+typedef __attribute__((address_space(3))) char* lds_ptr_t;  // the ring is addressed by offset: a tile's halves are an xor apart
+
+__device__ __forceinline__ u32x4_t ring_ld16(uint32_t at) {
+  return *reinterpret_cast<__attribute__((address_space(3))) const u32x4_t*>((lds_ptr_t)(uintptr_t)at);
+}
+__device__ __forceinline__ void ring_st16(uint32_t at, u32x4_t v) {
+  *reinterpret_cast<__attribute__((address_space(3))) u32x4_t*>((lds_ptr_t)(uintptr_t)at) = v;
+}
+__device__ __forceinline__ u32x2_t ring_tr16(uint32_t at) {
+  typedef __attribute__((address_space(3))) s16x4_t* ptr_t;
+  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr_t)(uintptr_t)at));
+}
+__device__ __forceinline__ const void* ring_ptr(uint32_t at) { return (const void*)(lds_ptr_t)(uintptr_t)at; }
+
+// bf16 rows: every wave copies 4 x 64 chunks of 16 bytes of K and of V (two rows per copy instruction); chunk j of row t
+// sits at chunk position j ^ swizzle(t), K: t & 15, V: 4 (t & 3) + 2 ((t >> 2) & 1) -- 32 lanes of a transposing read
+// meet rows t .. t + 7 in the same 32 bytes, and every bank once.
+// e4m3 rows: their bytes arrive in LDS as they are, two tiles ahead, in an area of the wave's own (2 x 1 KiB of K, of V):
+// a lane copies the 16 bytes that it later widens, so nothing but the wave's own wait stands between the two and no
+// register holds them on the way.  Piece p of a row (16 bytes) widens to chunks 2p and 2p + 1.
+__device__ __forceinline__ int wide_v_swizzle(int t) { return ((t & 3) << 2) | ((t >> 1) & 2); }
+
+template <bool UNIFORM, bool FP8>
+struct WideFeed {
+  static constexpr int N = FP8 ? 2 : 4;  // copy instructions per wave, for K and for V
+  int32_t id[UNIFORM ? 1 : N];           // pages of this lane's rows in the tile copied next
+
+  __device__ __forceinline__ static int row(int n, int wave, int lane) {
+    return FP8 ? wave * 8 + n * 4 + (lane >> 4) : wave * 8 + n * 2 + (lane >> 5);
+  }
+  __device__ __forceinline__ void fetch_pages(const TileSrc& s, int tb, int wave, int lane) {
+    tb = min(tb, s.last_tok & ~(kBN - 1));
+    if constexpr (UNIFORM) {
+      id[0] = scalar_load_i32(s.pages + __builtin_amdgcn_readfirstlane(page_slot(s, tb)));
+    } else {
+#pragma unroll
+      for (int n = 0; n < N; ++n) id[n] = s.pages[page_slot(s, min(tb + row(n, wave, lane), s.last_tok))];
+    }
+  }
+  // K (or V) rows to `at` (FP8: the bytes to the staging area at `at`)
+  __device__ __forceinline__ void copy(bool is_v, uint32_t at, const TileSrc& s, const KvAddr& kv, const char* base, int tb, int wave,
+                                       int lane) {
+    tb = min(tb, s.last_tok & ~(kBN - 1));  // past the end: re-copy the last tile
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int t = row(n, wave, lane);
+      const int64_t ro = row_offset<UNIFORM>(s, kv, tb, tb + t, id[UNIFORM ? 0 : n]);
+      const int j = FP8 ? (lane & 15) : (lane & 31) ^ (is_v ? wide_v_swizzle(t) : t & 15);
+      async_copy16(base + ro + j * 16, ring_ptr(at + (wave * N + n) * 1024));
+    }
+  }
+  // FP8: the staged bytes of this wave's rows -> bf16 rows of a tile (16 lanes of a row write chunks two apart: all banks)
+  __device__ __forceinline__ static void widen(uint32_t stage, uint32_t at, bool is_v, int wave, int lane) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int t = row(n, wave, lane), j = 2 * (lane & 15), swz = is_v ? wide_v_swizzle(t) : t & 15;
+      const u32x4_t x = ring_ld16(stage + (wave * N + n) * 1024 + lane * 16);
+      const u32x2_t a = fp8x4_to_bf16x4(x[0]), b = fp8x4_to_bf16x4(x[1]), c = fp8x4_to_bf16x4(x[2]), d = fp8x4_to_bf16x4(x[3]);
+      ring_st16(at + t * kWRowB + ((j ^ swz) << 4), u32x4_t{a[0], a[1], b[0], b[1]});
+      ring_st16(at + t * kWRowB + (((j + 1) ^ swz) << 4), u32x4_t{c[0], c[1], d[0], d[1]});
+    }
+  }
+};
+
+template <bool UNIFORM, bool CAP, bool EXT, bool FP8>
+__global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillArgs a_in, int tiles, int nseq, bool by_level) {
+  PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
+  if (a.dist) {
+    a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
+    a.seq_end = min(a.seq_end, scalar_load_i32(a.dist + 2));
+  }
+  __shared__ __attribute__((aligned(65536))) char ring[4 * kWTileB];  // K, K, V, V
+  __shared__ __attribute__((aligned(1024))) char stage[FP8 ? kWTileB : 16];  // K bytes, V bytes
+
+  const Work w = decompose(a, tiles, nseq, by_level, kBM, 1);
+  if (!w.valid) return;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const TileSrc src = make_src(a, w);
+  const char* kh = a.kv.k_base + (int64_t)w.hk * a.kv.head_stride;
+  const char* vh = a.kv.v_base + (int64_t)w.hk * a.kv.head_stride;
+
+  // this wave's positions: [r_lo, r_hi] of the chunk, lane column c = position r_lo + c
+  const int r_lo = w.q_start + wave * 16, r_hi = min(r_lo + 15, w.q_len - 1);
+  const bool active = r_lo < w.q_len;
+  const int row = r_lo + c, qpos = w.prefix + row;
+  const int W_ = a.sm.window;
+
+  const int wg_r_hi = min(w.q_start + kBM, w.q_len) - 1;
+  const bool causal = !EXT || a.sm.mask_mode == 0;
+  MaskCtx mc;
+  mc.mode = 0;
+  if constexpr (EXT) mc = make_mask_ctx(a, w, row);
+  int t_hi = causal ? min(w.kv_len, w.prefix + wg_r_hi + 1) : w.kv_len;  // exclusive
+  int t_lo = 0;
+  if (W_ > 0) t_lo = max(0, w.prefix + w.q_start - W_ + 1) & ~(kBN - 1);
+  int split = 0;
+  if (a.kv_splits > 1 && !kv_piece(a, t_lo, t_hi, split)) t_hi = t_lo;  // under-filled launch, nothing left for this piece
+
+  // ---- Q^T operands: column c = position, k-step ks covers dims 32 ks + 8 g ..
+  u32x4_t qB[8];
+  {
+    const uint16_t* qp = a.q + ((int64_t)(w.qg0 + min(row, w.q_len - 1)) * a.Hq + w.head) * 256 + g * 8;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qB[ks] = ld16(qp + ks * 32);
+    if (EXT && a.sm.q_scale > 0.f) {
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, FP8);
+    }
+  }
+  const float scale = a.sm.sm_scale * (a.k_scale ? a.k_scale[w.hk] : 1.0f) * ((EXT && a.sm.q_scale > 0.f) ? a.sm.q_scale : 1.0f);
+  const float temp = EXT ? xai_factor(qpos, a.sm.xai_len) : 1.0f;  // per position
+  const float sc2 = CAP ? 1.0f : scale * kLog2e * temp;            // score -> log2 units (soft-capped scores are there already)
+
+  f32x4_t O[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) O[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = kMaxFloor, l = 0.f;
+
+  // ---- operand addresses: K row 16 b + c, chunk (4 ks + g) ^ c; V^T of dims 16 j .., token 4 g + (c >> 2) (+ 16 for the
+  // second half of the k-step): chunk 2 j + ((c & 3) >> 1) before the swizzle, 8 bytes (c & 1) of it
+  const uint32_t ring_at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)ring);
+  const uint32_t stage_k = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)stage), stage_v = stage_k + kWTileB / 2;
+  uint32_t koff[4], voff[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) koff[i] = ring_at + c * kWRowB + (((4 * i + g) ^ c) << 4);  // steps 4 .. 7: 256 bytes on
+#pragma unroll
+  for (int i = 0; i < 8; ++i)  // dims 128 ..: 256 bytes on
+    voff[i] = ring_at + 2 * kWTileB + (4 * g + (c >> 2)) * kWRowB + (((2 * i + ((c & 3) >> 1)) ^ ((c >> 2) << 2) ^ ((g & 1) << 1)) << 4) + ((c & 1) << 3);
+
+  auto scores = [&](f32x4_t (&S)[4]) __attribute__((always_inline)) {  // tokens 16 b + 4 g + r
+#pragma unroll
+    for (int b = 0; b < 4; ++b) S[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) S[b] = mfma16(ring_ld16(koff[ks & 3] + (ks >> 2) * 256 + b * (16 * kWRowB)), qB[ks], S[b]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) koff[i] ^= kWTileB;
+  };
+  auto cap_scores = [&](f32x4_t (&S)[4]) __attribute__((always_inline)) {
+    if constexpr (CAP) {
+      const float cap = a.sm.soft_cap;
+      if (cap != 0.f && !a.sm.round_logits) {
+        // cap tanh(s scale / cap) temp log2e = k2 - 2 k2 / (2^(s k1) + 1)
+        const float k1 = scale / cap * (2.0f * kLog2e), k2 = cap * temp * kLog2e;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            S[b][r] = __builtin_fmaf(__builtin_amdgcn_rcpf(fast_exp2(S[b][r] * k1) + 1.0f), -2.0f * k2, k2);
+      } else {
+        const float inv_cap = cap != 0.f ? 1.0f / cap : 0.f;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float x = S[b][r] * scale;
+            if (cap != 0.f) x = soft_cap_f(x, cap, inv_cap);
+            x = x * temp;
+            if (a.sm.round_logits) x = round_logit(x, a.sm.round_logits);
+            S[b][r] = x * kLog2e;
+          }
+      }
+    }
+  };
+  auto mask_scores = [&](f32x4_t (&S)[4], int tb) __attribute__((always_inline)) {
+    if ((causal ? (tb + kBN - 1 > w.prefix + r_lo) : (mc.mode == 1 || tb + kBN > w.kv_len)) ||
+        (W_ > 0 && tb <= w.prefix + r_hi - W_)) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int tok = tb + 16 * b + 4 * g + r;
+          bool masked;
+          if (!EXT || mc.mode == 0) masked = tok > qpos;
+          else masked = (tok >= mc.kv_len) || (mc.mode == 1 && mc.row[tok] < 1);
+          masked = masked || (W_ > 0 && tok <= qpos - W_);
+          S[b][r] = masked ? kMaskRaw : S[b][r];
+        }
+    }
+  };
+  // probabilities as bf16 pairs, the B operands of the second product; the row sum is taken over the rounded pairs
+  u32x4_t pB[2];
+  auto probabilities = [&](const f32x4_t (&S)[4], u32x4_t (&p)[2]) __attribute__((always_inline)) {
+    const float neg_m = -m * sc2;
+    const bf16x2_t ones = {(__bf16)1.0f, (__bf16)1.0f};
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; r += 2) {
+        const uint32_t x = pack_bf16x2(fast_exp2(__builtin_fmaf(S[b][r], sc2, neg_m)), fast_exp2(__builtin_fmaf(S[b][r + 1], sc2, neg_m)));
+        l = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, x), ones, l, false);
+        p[b >> 1][(b & 1) * 2 + (r >> 1)] = x;
+      }
+  };
+  // the running max goes stale by up to 2^kMaxSlack before what was taken against it follows (see softmax_tile)
+  auto raise_max = [&](const f32x4_t (&S)[4]) __attribute__((always_inline)) {
+    float mx = fmaxf(S[0][0], S[0][1]);
+#pragma unroll
+    for (int i = 2; i < 16; i += 2) mx = __builtin_fmaxf(__builtin_fmaxf(mx, S[i >> 2][i & 3]), S[i >> 2][(i & 3) + 1]);
+    mx = swap_max(swap16_max(mx));
+    if (__builtin_amdgcn_ballot_w64((mx - m) * sc2 > kMaxSlack) != 0) {
+      const float m_new = fmaxf(m, mx);
+      const float alpha = fast_exp2((m - m_new) * sc2);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) O[j] *= alpha;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)  // the probabilities that wait for their half of the second product
+        pB[1][i] = pack_bf16x2(bf16_lo_to_f32(pB[1][i]) * alpha, bf16_hi_to_f32(pB[1][i]) * alpha);
+    }
+  };
+  auto second_product = [&](int kk) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const uint32_t vt = voff[j & 7] + (j >> 3) * 256 + kk * (32 * kWRowB);
+      const u32x2_t lo = ring_tr16(vt);
+      const u32x2_t hi = ring_tr16(vt + 16 * kWRowB);
+      O[j] = mfma16(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pB[kk], O[j]);
+    }
+  };
+
+  // ---- K runs a tile ahead of V.  Step i: K of tile i + 2 and V of tile i + 1 are requested; scores of tile i + 1, whose
+  // soft cap and exponentials run beside the two halves of the second product of tile i
+  if (t_lo < t_hi) {
+    const int n = __builtin_amdgcn_readfirstlane((t_hi - t_lo + kBN - 1) / kBN);
+    WideFeed<UNIFORM, FP8> fk, fv;  // their page ids
+    uint32_t k_fill = ring_at, v_fill = ring_at + 3 * kWTileB;
+    fk.fetch_pages(src, t_lo, wave, lane);
+    fv.fetch_pages(src, t_lo + kBN, wave, lane);
+    if constexpr (FP8) {
+      fk.copy(false, stage_k, src, a.kv, kh, t_lo, wave, lane);
+      fk.copy(true, stage_v, src, a.kv, vh, t_lo, wave, lane);
+      fk.fetch_pages(src, t_lo + 2 * kBN, wave, lane);
+      wait_all_loads();
+      fk.widen(stage_k, ring_at, false, wave, lane);
+      fk.widen(stage_v, ring_at + 2 * kWTileB, true, wave, lane);
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the bytes have been read
+      fv.copy(false, stage_k, src, a.kv, kh, t_lo + kBN, wave, lane);
+      fv.copy(true, stage_v, src, a.kv, vh, t_lo + kBN, wave, lane);
+      wait_all_loads();
+      fk.widen(stage_k, ring_at + kWTileB, false, wave, lane);
+      __builtin_amdgcn_s_waitcnt(0xC07F);
+      fk.copy(false, stage_k, src, a.kv, kh, t_lo + 2 * kBN, wave, lane);
+      fv = fk;
+      fk.fetch_pages(src, t_lo + 3 * kBN, wave, lane);
+    } else {
+      fk.copy(false, ring_at, src, a.kv, kh, t_lo, wave, lane);
+      fk.copy(true, ring_at + 2 * kWTileB, src, a.kv, vh, t_lo, wave, lane);
+      fv.copy(false, ring_at + kWTileB, src, a.kv, kh, t_lo + kBN, wave, lane);
+      fk.fetch_pages(src, t_lo + 2 * kBN, wave, lane);
+      wait_all_loads();
+    }
+    __syncthreads();
+    auto next = [&](int tb) __attribute__((always_inline)) {
+      if constexpr (FP8) {
+        wait_all_loads();  // this wave's bytes: K of tile i + 2, V of tile i + 1
+        fk.widen(stage_k, k_fill, false, wave, lane);
+        fk.widen(stage_v, v_fill, true, wave, lane);
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        fk.copy(false, stage_k, src, a.kv, kh, tb + 3 * kBN, wave, lane);
+        fv.copy(true, stage_v, src, a.kv, vh, tb + 2 * kBN, wave, lane);
+        fv = fk;
+        fk.fetch_pages(src, tb + 4 * kBN, wave, lane);
+      } else {
+        fk.copy(false, k_fill, src, a.kv, kh, tb + 2 * kBN, wave, lane);
+        fv.copy(true, v_fill, src, a.kv, vh, tb + kBN, wave, lane);
+        fv = fk;
+        fk.fetch_pages(src, tb + 3 * kBN, wave, lane);
+      }
+      k_fill ^= kWTileB;
+      v_fill ^= kWTileB;
+    };
+    auto meet = [&]() __attribute__((always_inline)) {
+      if constexpr (!FP8) wait_all_loads();  // this wave's copies have landed
+      __syncthreads();
+    };
+    if (__builtin_amdgcn_readfirstlane(!active)) {  // positions past the chunk's end: this wave only copies
+      for (int i = 0; i + 1 < n; ++i) {
+        if (i == 0) __syncthreads();
+        next(t_lo + i * kBN);
+        meet();
+      }
+    } else {
+      {
+        f32x4_t S[4];
+        scores(S);
+        cap_scores(S);
+        mask_scores(S, t_lo);
+        pB[1] = u32x4_t{0u, 0u, 0u, 0u};
+        raise_max(S);
+        probabilities(S, pB);
+      }
+      // (tiles that none of a wave's positions sees are not skipped: the other waves of the workgroup are at work on them)
+      for (int i = 0; i + 1 < n; ++i) {
+        const int tb = t_lo + i * kBN;
+        // (K of tile 0 is free once every wave has taken its scores of it)
+        if (i == 0) __syncthreads();
+        next(tb);
+        f32x4_t S[4];
+        scores(S);
+        cap_scores(S);
+        second_product(0);
+        mask_scores(S, tb + kBN);
+        raise_max(S);
+        u32x4_t p_next[2];
+        probabilities(S, p_next);
+        second_product(1);
+        pB[0] = p_next[0];
+        pB[1] = p_next[1];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) voff[k] ^= kWTileB;
+        meet();
+      }
+      second_product(0);
+      second_product(1);
+    }
+    if constexpr (FP8) wait_all_loads();  // (bytes requested past the end)
+  }
+
+  // ---- lane (c, g) holds position r_lo + c, dims 16 j + 4 g + r
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (!active || row >= w.q_len) return;
+  const int64_t out_row = (int64_t)(w.qg0 + row) * a.Hq + w.head;
+  if (a.kv_splits > 1) {
+    const int64_t slot = out_row * a.kv_splits + split;
+    float* op = a.ws_o + slot * 256 + 4 * g;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) *reinterpret_cast<f32x4_t*>(op + 16 * j) = O[j];
+    if (g == 0) {
+      a.ws_ml[slot * 2] = fmaxf(m * sc2, kNoReference);
+      a.ws_ml[slot * 2 + 1] = l;
+    }
+    return;
+  }
+  const float vs = a.v_scale ? a.v_scale[w.hk] : 1.0f;
+  const float inv = a.sm.sink ? vs * sink_inverse(m * sc2, l, sink_logit(a.sm.sink, a.sm.round_logits, w.head)) : vs / l;
+  uint16_t* op = a.out + out_row * 256 + 4 * g;
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    *reinterpret_cast<u32x2_t*>(op + 16 * j) = u32x2_t{pack_bf16x2(O[j][0] * inv, O[j][1] * inv), pack_bf16x2(O[j][2] * inv, O[j][3] * inv)};
+}
+
+}  // namespace
+
+namespace {
 
 // ==================================================================== staged path (fp8 cache)
 constexpr int kKPitch = 272;  // bytes per K row in LDS (256 + 16 pad: conflict-free b128 reads)
@@ -647,11 +941,9 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL((rpa_prefill_staged_kernel<true, U, C, E, true>), g, blk, 0, stream, a, tiles, nseq, by_level)
 #define RPA_ASYNC(U, C, E) hipLaunchKernelGGL((rpa_prefill_async_kernel<U, C, E>), g, blk, 0, stream, a, tiles, nseq, by_level)
 #define RPA_ASYNC_HEADS4(U, C, E) \
-  hipLaunchKernelGGL((rpa_prefill_async_kernel<U, C, E, 128, false, true>), g, blk, 0, stream, a, tiles, nseq, by_level)
-#define RPA_ASYNC256(U, C, E) \
-  hipLaunchKernelGGL((rpa_prefill_async_kernel<U, C, E, 256>), g, blk, 0, stream, a, tiles, nseq, by_level)
-#define RPA_ASYNC256_FP8(U, C, E) \
-  hipLaunchKernelGGL((rpa_prefill_async_kernel<U, C, E, 256, true>), g, blk, 0, stream, a, tiles, nseq, by_level)
+  hipLaunchKernelGGL((rpa_prefill_async_kernel<U, C, E, true>), g, blk, 0, stream, a, tiles, nseq, by_level)
+#define RPA_WIDE(F, U, C, E) \
+  hipLaunchKernelGGL((rpa_prefill_wide_kernel<U, C, E, F>), g, dim3(512), 0, stream, a, tiles, nseq, by_level)
 #define RPA_PICK(M, ...)                                            \
   switch ((uniform ? 4 : 0) | (cap ? 2 : 0) | (ext ? 1 : 0)) {        \
     case 0: M(__VA_ARGS__ false, false, false); break;              \
@@ -663,13 +955,15 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
     case 6: M(__VA_ARGS__ true, true, false); break;                \
     default: M(__VA_ARGS__ true, true, true); break;                \
   }
+#define RPA_WIDE_FP8(U, C, E) RPA_WIDE(true, U, C, E)
+#define RPA_WIDE_BF16(U, C, E) RPA_WIDE(false, U, C, E)
 #define RPA_STAGED_FP8(U, C, E) RPA_STAGED(true, U, C, E)
 #define RPA_STAGED_BF16(U, C, E) RPA_STAGED(false, U, C, E)
   if (a.head_dim == 256) {
     if (a.fp8) {
-      RPA_PICK(RPA_ASYNC256_FP8, )
+      RPA_PICK(RPA_WIDE_FP8, )
     } else {
-      RPA_PICK(RPA_ASYNC256, )
+      RPA_PICK(RPA_WIDE_BF16, )
     }
   } else if (heads4 && a.fp8) {
     RPA_PICK(RPA_STAGED_FP8_HEADS4, )
@@ -689,8 +983,9 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
 #undef RPA_ASYNC
 #undef RPA_ASYNC_HEADS4
 #undef RPA_STAGED_FP8_HEADS4
-#undef RPA_ASYNC256
-#undef RPA_ASYNC256_FP8
+#undef RPA_WIDE
+#undef RPA_WIDE_FP8
+#undef RPA_WIDE_BF16
   return cut ? launch_prefill_combine(a, stream) : hipGetLastError();
 }
 

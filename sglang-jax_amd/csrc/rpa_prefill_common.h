@@ -174,6 +174,12 @@ __device__ __forceinline__ float swap_max(float x) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+// the same over lanes 16 apart
+__device__ __forceinline__ float swap16_max(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // Which tokens a query row may see.  mode 0: causal (token <= row position); mode 1: the
 // caller's mask row (>= 1 keeps), mode 2: everything; modes 1 and 2 still hide the tokens of a
 // partial last tile beyond kv_len.  The sliding window applies on top in every mode.
@@ -209,19 +215,7 @@ __device__ __forceinline__ void softmax_tile(f32x16_t (&S)[2], f32x16_t (&O)[ND]
                                              const Softmax<CAP>& sm, bool need_mask, int tb, int h, int qpos,
                                              int window, u32x4_t (&pB)[2][2], const MaskCtx& mc,
                                              uint64_t mask_word = 0) {
-  if constexpr (CAP && ND != 4) {
-    // 256-wide heads: one loop with run-time choices (those kernels have no register to spare for variants)
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        float x = S[mt][v] * sm.scale;
-        if (sm.cap != 0.f) x = soft_cap_f(x, sm.cap, sm.inv_cap);
-        x = x * sm.temp;
-        if (sm.round_mode) x = round_logit(x, sm.round_mode);
-        S[mt][v] = x * kLog2e;
-      }
-  } else if constexpr (CAP) {
+  if constexpr (CAP) {
     if (sm.cap != 0.f && !sm.round_mode) {
       // soft cap alone (the usual case), constants folded: five instructions per score.
       // cap tanh(s scale / cap) temp log2e = k2 - 2 k2 / (2^(s k1) + 1)
@@ -231,6 +225,18 @@ __device__ __forceinline__ void softmax_tile(f32x16_t (&S)[2], f32x16_t (&O)[ND]
 #pragma unroll
         for (int v = 0; v < 16; ++v)
           S[mt][v] = __builtin_fmaf(__builtin_amdgcn_rcpf(fast_exp2(S[mt][v] * k1) + 1.0f), -2.0f * k2, k2);
+    } else if constexpr (ND != 4) {
+      // 256-wide heads, logits that are rounded: one loop with run-time choices
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          float x = S[mt][v] * sm.scale;
+          if (sm.cap != 0.f) x = soft_cap_f(x, sm.cap, sm.inv_cap);
+          x = x * sm.temp;
+          if (sm.round_mode) x = round_logit(x, sm.round_mode);
+          S[mt][v] = x * kLog2e;
+        }
     } else {
       // the general path: soft cap (if any), temperature, then the logit rounded to the softmax dtype.  One loop
       // per combination, so that no score pays for a choice that is the same for the whole call.

@@ -985,6 +985,17 @@ def test_head_dim_256_fp8_chunks_flash_kernel_against_row_kernel(pkg, wl, gpu, P
     assert not torch.equal(flash, rows)  # two kernels: the last bits differ somewhere
 
 
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("P,cap,window", [(64, None, None), (64, 30.0, 100), (16, None, 64), (24, 50.0, None)])
+def test_head_dim_256_chunks_at_the_edges_of_a_tile(pkg, wl, gpu, P, cap, window, kv_dtype):
+    """Chunks whose waves end inside, at and behind a block of 16 positions and of 128, contexts of one to a few 64-token tiles
+    and ranges that begin inside one."""
+    q_lens, kv_lens = [2, 15, 16, 17, 127, 128, 129, 64, 65], [2, 64, 65, 128, 127, 129, 400, 192, 65]
+    b = batch256(wl, "d256edge", q_lens, kv_lens, 97, Hq=4, Hkv=2, P=P, kv_dtype=kv_dtype, sliding_window=window, soft_cap=cap)
+    say(f"case d256 tile edges P={P} cap={cap} window={window} {kv_dtype}")
+    assert_parity(gpu_out(pkg, b, gpu).float(), oracle_out(b).float(), **(FP8_TOL if kv_dtype != torch.bfloat16 else BF16_TOL))
+
+
 def test_head_dim_256_cache_write_and_gather(pkg, wl, gpu):
     """The new-token write and the page gather take any head width (bit-exact)."""
     q_lens, kv_lens = [1, 7], [33, 40]
