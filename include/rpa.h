@@ -137,7 +137,8 @@ typedef struct RpaParams {
   const int32_t* custom_mask;   /* device i32, flat: sequence i, query row j, token t at
                                    cu_mask_lens[i] + j * row_width_i + t; >= 1 keeps, < 1 masks (:154-163).
                                    Read only when mask_mode == RPA_MASK_CUSTOM */
-  const int32_t* cu_mask_lens;  /* device i32[S+1]: cumulative q_len_i * row_width_i (:123-129, 1801-1806) */
+  const int32_t* cu_mask_lens;  /* device i32[S+1]: cumulative q_len_i * row_width_i (:123-129, 1801-1806); may be NULL
+                                   where rpa_mask_needs_starts() says so */
   float xai_temperature_len;    /* > 0: logits of a query at position p > len are multiplied by
                                    log2(p) / log2(len) (:171-177); 0 => off.  With soft_cap set as well
                                    the factor multiplies the capped logit, the order of
@@ -163,6 +164,10 @@ typedef struct RpaParams {
    * Neither mode limits the sequences or tokens of a call beyond int32: rows are folded onto the first
    * grid dimension. */
   const int32_t* distribution;
+  /* Elements of a row of q, out, keys and values where that is less than the cache's head_dim (the reference pads heads
+   * to a multiple of 128, rpa_v3:1187-1241): a multiple of 8 (e4m3: 16), head_dim - q_head_dim < 128; 0 = head_dim.
+   * The rest of a cached row is zero, is written as zeros with the new tokens and adds nothing. */
+  int32_t q_head_dim;
 } RpaParams;
 
 /*
@@ -319,6 +324,10 @@ RPA_API int rpa_kv_write(const RpaParams* p, const void* keys, const void* value
  * [T, Hkv, D] in the cache dtype, or both NULL when the cache already holds every token.
  */
 RPA_API int rpa_attention_update(const RpaParams* p, const void* keys, const void* values, void* stream);
+
+/* Whether a RPA_MASK_CUSTOM call needs cu_mask_lens: 0 where the mask is turned into bits first (128-wide heads, max_kv_len
+ * given, rpa_workspace_bytes() of workspace), which finds the starts of the sequences' rows by itself. */
+RPA_API int rpa_mask_needs_starts(const RpaParams* p);
 
 /* Absorbed-MLA decode, see RpaMlaParams: every sequence contributes exactly one query token. */
 RPA_API int rpa_mla_decode(const RpaMlaParams* p, void* stream);

@@ -57,6 +57,7 @@ EXPORTED_SYMBOLS = (
     "rpa_mla_describe_plan",
     "rpa_attention_update",
     "rpa_mla_attention_update",
+    "rpa_mask_needs_starts",
     "rpa_mla_sparse_workspace_bytes",
     "rpa_mla_sparse_attention",
 )
@@ -104,6 +105,7 @@ class RpaParams(ctypes.Structure):
         ("softmax_dtype", ctypes.c_int32),
         ("q_scale", ctypes.c_float),
         ("distribution", ctypes.c_void_p),
+        ("q_head_dim", ctypes.c_int32),
     ]
 
 

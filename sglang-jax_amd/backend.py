@@ -317,15 +317,14 @@ class FlashAttention:
         xai = xai if xai is not None and xai > 0 else None
         soft_cap = getattr(layer, "logit_cap", None) or None
         softmax_dtype = getattr(layer, "softmax_dtype", None)
-        if causal or md.custom_mask is None:
-            out = _lib.load_torch().attention(
-                q, k, v, kv_cache_fused, md.seq_lens, page_indices, md.cu_q_lens, md.cu_kv_lens, md.host_distribution,
-                attention_sink, causal, scale, window, soft_cap, None, None, None, None, xai, softmax_dtype, None,
-                md.max_kv_len, md.max_q_len, 0, md.host_seq_lens, head_dim)
-            if out is not None:
-                if type(out) is int:
-                    _lib.check(out)
-                return out if out.dim() == 2 else out.reshape(out.shape[0], -1), kv_cache_fused
+        out = _lib.load_torch().attention(
+            q, k, v, kv_cache_fused, md.seq_lens, page_indices, md.cu_q_lens, md.cu_kv_lens, md.host_distribution,
+            attention_sink, causal, scale, window, soft_cap, None, None, None, None, xai, softmax_dtype, None,
+            md.max_kv_len, md.max_q_len, 0, md.host_seq_lens, head_dim, md.custom_mask, False)
+        if out is not None:
+            if type(out) is int:
+                _lib.check(out)
+            return out if out.dim() == 2 else out.reshape(out.shape[0], -1), kv_cache_fused
         T = q.shape[0]
         out, cache = ragged_paged_attention(
             q.reshape(T, -1, head_dim),

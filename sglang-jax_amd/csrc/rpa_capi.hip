@@ -81,6 +81,19 @@ int fail(int code, const char* fmt, ...) {
 
 constexpr float kDefaultMask = -0.7f * 3.4028234663852886e38f;
 
+// Bytes of a custom mask as one bit per pair; 0: the kernels read the caller's i32 words (no bound on the lengths, 256-wide
+// heads, a batch too large, RPA_MASK_BITS=0).
+size_t mask_bits_bytes(const RpaParams* p) {
+  if (p->mask_mode != RPA_MASK_CUSTOM || p->head_dim != 128 || p->max_kv_len <= 0 || p->num_tokens <= 0 || rpa::tuning().mask_bits == 0)
+    return 0;
+  const size_t bytes = (size_t)p->num_tokens * ((p->max_kv_len + 63) / 64) * sizeof(uint64_t);
+  return bytes > ((size_t)256 << 20) ? 0 : bytes;
+}
+bool mask_as_bits(const RpaParams* p) { return mask_bits_bytes(p) != 0; }
+
+// elements of a row of queries, keys, values and outputs
+int q_dim_of(const RpaParams* p) { return p->q_head_dim > 0 ? p->q_head_dim : p->head_dim; }
+
 int esize_of(int kv_dtype) { return kv_dtype == RPA_KV_FP8_E4M3 ? 1 : 2; }
 
 rpa::KvAddr kv_addr(const RpaParams* p) {
@@ -280,7 +293,7 @@ int64_t decode_kv_bytes(const RpaParams* p) {
     tokens = (int64_t)p->decode_end * kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages,
                                                    p->cu_kv_lens != nullptr);
   if (p->sliding_window > 0) tokens = std::min(tokens, (int64_t)p->decode_end * (p->sliding_window + 31));
-  return tokens * 2 * p->num_kv_heads * p->head_dim * esize_of(p->kv_dtype);
+  return tokens * 2 * p->num_kv_heads * (q_dim_of(p) == 64 && p->kv_dtype == RPA_KV_BF16 ? 64 : p->head_dim) * esize_of(p->kv_dtype);
 }
 
 // The decode rows' row of the shape table (rpa_shapes.h): waves of a workgroup = neighbouring kv heads walked
@@ -359,6 +372,7 @@ int rows256(const RpaParams* p, int seq_begin, int seq_end, void* stream, int di
   a.Hq = p->num_q_heads;
   a.Hkv = p->num_kv_heads;
   a.G = p->num_q_heads / p->num_kv_heads;
+  a.q_dim = q_dim_of(p);
   a.fp8 = p->kv_dtype == RPA_KV_FP8_E4M3;
   a.dist = dist_role ? p->distribution : nullptr;
   // decode rows are one token each; other sequences are bounded by the tokens of the call
@@ -423,6 +437,9 @@ int rpa_validate(const RpaParams* p) {
   if (p->num_q_heads % p->num_kv_heads != 0)
     return fail(RPA_EINVAL_HEADS, "expected num_q_heads=%d to be divisible by num_kv_heads=%d",
                 p->num_q_heads, p->num_kv_heads);
+  if (p->q_head_dim != 0 && (p->q_head_dim < 0 || p->q_head_dim > p->head_dim || p->head_dim - p->q_head_dim >= 128 ||
+                             p->q_head_dim * esize_of(p->kv_dtype) % 16 != 0 || p->q_head_dim % 8 != 0))
+    return fail(RPA_EUNSUPPORTED, "q_head_dim=%d: multiples of 8 (e4m3: 16) that round up to head_dim=%d", p->q_head_dim, p->head_dim);
   if (p->head_dim != 128 && p->head_dim != 256)
     return fail(RPA_EUNSUPPORTED, "head_dim=%d: 128 and 256 are built", p->head_dim);
   if (p->kv_dtype != RPA_KV_BF16 && p->kv_dtype != RPA_KV_FP8_E4M3)
@@ -445,8 +462,8 @@ int rpa_validate(const RpaParams* p) {
   if (p->mask_value > 0.0f) return fail(RPA_EINVAL_SHAPE, "mask_value=%g must be negative", p->mask_value);
   if (p->mask_mode < RPA_MASK_CAUSAL || p->mask_mode > RPA_MASK_NONE)
     return fail(RPA_EINVAL_SHAPE, "mask_mode=%d is not an RpaMaskMode", p->mask_mode);
-  if (p->mask_mode == RPA_MASK_CUSTOM && (!p->custom_mask || !p->cu_mask_lens))
-    return fail(RPA_EINVAL_NULL, "RPA_MASK_CUSTOM needs custom_mask and cu_mask_lens");
+  if (p->mask_mode == RPA_MASK_CUSTOM && (!p->custom_mask || (!p->cu_mask_lens && !mask_as_bits(p))))
+    return fail(RPA_EINVAL_NULL, "RPA_MASK_CUSTOM needs custom_mask and, where the mask is not turned into bits, cu_mask_lens");
   if (p->mask_mode == RPA_MASK_CUSTOM && p->mask_rows_page_aligned && !p->cu_kv_lens)
     return fail(RPA_EINVAL_NULL, "page-aligned mask rows need cu_kv_lens");
   if (p->softmax_dtype != RPA_SOFTMAX_F32 && p->softmax_dtype != RPA_SOFTMAX_BF16 && p->softmax_dtype != RPA_SOFTMAX_F16)
@@ -634,6 +651,7 @@ static int decode_rows(const RpaParams* p_in, const void* keys, const void* valu
   a.Hq = p->num_q_heads;
   a.Hkv = p->num_kv_heads;
   a.G = p->num_q_heads / p->num_kv_heads;
+  a.q_dim = q_dim_of(p);
   a.chunk = sp.chunk;
   a.max_splits = sp.splits;
   a.fp8 = p->kv_dtype == RPA_KV_FP8_E4M3;
@@ -706,6 +724,7 @@ static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a) {
   a.Hq = p->num_q_heads;
   a.Hkv = p->num_kv_heads;
   a.G = p->num_q_heads / p->num_kv_heads;
+  a.q_dim = q_dim_of(p);
   a.max_q_len = p->max_q_len > 0 ? p->max_q_len : p->num_tokens;
   a.max_kv_len = p->max_kv_len > 0 ? p->max_kv_len : 0;
   a.fp8 = p->kv_dtype == RPA_KV_FP8_E4M3;
@@ -732,12 +751,8 @@ PrefillWorkspace prefill_workspace(const RpaParams* p, const rpa::PrefillArgs& a
   w.splits = rpa::prefill_kv_splits(a);
   w.split_bytes = rpa::prefill_split_workspace_bytes(a, w.splits);
   w.bits_offset = (w.split_bytes + 255) & ~(size_t)255;
-  if (p->mask_mode == RPA_MASK_CUSTOM && p->head_dim == 128 && p->max_kv_len > 0 && p->num_tokens > 0 &&
-      rpa::tuning().mask_bits != 0) {
-    w.pitch = (p->max_kv_len + 63) / 64;
-    w.bits_bytes = (size_t)p->num_tokens * w.pitch * sizeof(uint64_t);
-    if (w.bits_bytes > ((size_t)256 << 20)) w.bits_bytes = 0;  // a batch this large keeps the i32 words
-  }
+  w.bits_bytes = mask_bits_bytes(p);
+  w.pitch = w.bits_bytes ? (p->max_kv_len + 63) / 64 : 0;
   w.total = w.bits_bytes ? w.bits_offset + w.bits_bytes : w.split_bytes;
   return w;
 }
@@ -787,13 +802,23 @@ int rpa_prefill(const RpaParams* p, void* stream) {
       a.mask_pitch = w.pitch;
     }
   }
+  if (p->mask_mode == RPA_MASK_CUSTOM && !p->cu_mask_lens && !a.mask_bits)
+    return fail(RPA_EINVAL_WORKSPACE, "a mask without cu_mask_lens needs rpa_workspace_bytes() of workspace");
   return check_hip(rpa::launch_prefill(a, static_cast<hipStream_t>(stream)), "rpa_prefill");
+}
+
+int rpa_mask_needs_starts(const RpaParams* p) { return p && p->mask_mode == RPA_MASK_CUSTOM && !mask_as_bits(p) ? 1 : 0; }
+
+// (narrow heads: only the kernels that know of the zeros behind 64 dims)
+static bool rows_take_new_tokens(const RpaParams* p) {
+  const int d = q_dim_of(p);
+  return d == p->head_dim || (d == 64 && p->kv_dtype == RPA_KV_BF16 && rpa::tuning().decode_merge_in_kernel == 0);
 }
 
 // Whether the decode kernels read their rows' new tokens from the caller's keys / values and write them into the cache
 // (not the 256-wide rows, nor the balanced plan on pages smaller than a block).
 static bool decode_takes_new_tokens(const RpaParams* p_in) {
-  if (p_in->head_dim != 128 || p_in->mask_mode == RPA_MASK_CUSTOM) return false;
+  if (p_in->head_dim != 128 || p_in->mask_mode == RPA_MASK_CUSTOM || !rows_take_new_tokens(p_in)) return false;
   if (p_in->page_size % 32 == 0) return true;
   const RpaParams p = planning_view(p_in);
   return !use_balanced(&p, decode_plan(&p));
@@ -809,6 +834,7 @@ static int write_new_tokens(const RpaParams* p, const void* keys, const void* va
   a.dist = p->distribution;
   a.Hkv = p->num_kv_heads;
   a.head_bytes = p->head_dim * esize_of(p->kv_dtype);
+  a.src_head_bytes = q_dim_of(p) * esize_of(p->kv_dtype);
   a.num_tokens = p->num_tokens;
   a.skip_decode_rows = skip_decode_rows ? 1 : 0;
   a.seq_begin = skip_decode_rows && !p->distribution ? p->decode_end : 0;
@@ -819,7 +845,11 @@ int rpa_attention_update(const RpaParams* p, const void* keys, const void* value
   int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
   if (!keys != !values) return fail(RPA_EINVAL_NULL, "keys and values must be given together");
-  if (takes_token_rows(p) && p->workspace_bytes >= token_row_workspace(p)) return decode_rows(p, keys, values, true, stream);
+  if (takes_token_rows(p) && p->workspace_bytes >= token_row_workspace(p)) {
+    const bool with_rows = keys && rows_take_new_tokens(p);
+    if (keys && !with_rows && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
+    return decode_rows(p, with_rows ? keys : nullptr, with_rows ? values : nullptr, true, stream);
+  }
   const bool fused = keys && decode_takes_new_tokens(p);
   if (keys && !fused && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
   if ((rc = decode_rows(p, fused ? keys : nullptr, fused ? values : nullptr, false, stream)) != RPA_OK) return rc;

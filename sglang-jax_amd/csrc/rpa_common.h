@@ -130,6 +130,11 @@ __device__ __forceinline__ void async_copy16(const void* gsrc, const void* lds_b
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0v), "v"(gsrc) : "memory", "m0");
 }
 
+// Eight query elements from dim d of a row of q_dim (a multiple of 8); dims past it are zero.
+__device__ __forceinline__ u32x4_t ld_query(const uint16_t* row, int d, int q_dim) {
+  return d < q_dim ? *reinterpret_cast<const u32x4_t*>(row + d) : u32x4_t{0u, 0u, 0u, 0u};
+}
+
 // 16-byte global loads / stores.
 __device__ __forceinline__ u32x4_t ld16(const void* p) { return *reinterpret_cast<const u32x4_t*>(p); }
 __device__ __forceinline__ u32x2_t ld8(const void* p) { return *reinterpret_cast<const u32x2_t*>(p); }

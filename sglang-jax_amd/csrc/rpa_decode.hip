@@ -96,12 +96,19 @@ __device__ __forceinline__ int page_slot_of(const SeqView& s, int tok) {
 // (A compile-time choice: with both lookups in the code the compiler's wait-count bookkeeping sees a possible
 // page-id load behind every block and drains the whole queue in front of each block's use.)
 // FRESH: the row's last tokens may come from the caller's new rows instead (SeqView.fresh_first).
-template <bool FP8, bool UNIFORM_PAGE, bool WINDOW = false, bool FRESH = false>
+// HALF (bf16): heads of 64 dims in rows of 128 whose second half is zero: it is not read.
+template <bool FP8, bool UNIFORM_PAGE, bool WINDOW = false, bool FRESH = false, bool HALF = false>
 __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, int page, int c, int g,
                                            const int32_t* win = nullptr, int win_first = 0) {
   const KvAddr& kv = a.kv;
   constexpr int kLaneK = FP8 ? 32 : 16;  // byte offset step of lane group g inside a K row
   constexpr int kLaneV = FP8 ? 8 : 16;   // byte offset step of lane c inside a V row
+  constexpr int kSteps = HALF ? 2 : 4;   // k-steps of the first product
+  auto ld_v = [&](const char* p) __attribute__((always_inline)) {
+    if constexpr (HALF) return c < 8 ? RPA_KV_LD16(p) : u32x4_t{0u, 0u, 0u, 0u};
+    else if constexpr (FP8) return RPA_KV_LD8(p);
+    else return RPA_KV_LD16(p);
+  };
   // A block that reaches into the new tokens (the last one of a row): an address of its own per token row.  The
   // number of loads is that of the other branch, so the counted waits behind it stay the same.
   if (FRESH && rare(tb + kBlk > s.fresh_first)) {
@@ -111,20 +118,19 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
       const int slot = UNIFORM_PAGE ? block_slot : page_slot_of(s, tok);
       const int pg = UNIFORM_PAGE ? page : WINDOW ? win[slot - win_first] : s.pages[slot];
       const char* old_at = cached + (int64_t)pg * kv.page_stride + (int64_t)((tok - slot * s.page_size) * kv.tok_stride);
-      const char* new_at = fresh + (int64_t)(s.fresh_row + (tok - s.fresh_first) * a.Hkv) * (FP8 ? 128 : 256);
+      const char* new_at = fresh + (int64_t)(s.fresh_row + (tok - s.fresh_first) * a.Hkv) * (FP8 || HALF ? 128 : 256);
       return tok >= s.fresh_first ? new_at : old_at;
     };
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       const char* kp = row_of(tb + b * 16 + c, kh, a.new_k) + g * kLaneK;
 #pragma unroll
-      for (int st = 0; st < (FP8 ? 2 : 4); ++st) r.k[b][st] = RPA_KV_LD16(kp + st * (FP8 ? 16 : 64));
+      for (int st = 0; st < (FP8 ? 2 : kSteps); ++st) r.k[b][st] = RPA_KV_LD16(kp + st * (FP8 ? 16 : 64));
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const char* vp = row_of(tb + tok_slot(g, i), vh, a.new_v) + c * kLaneV;
-      if constexpr (FP8) r.v[i] = RPA_KV_LD8(vp);
-      else r.v[i] = RPA_KV_LD16(vp);
+      r.v[i] = ld_v(vp);
     }
     return;
   }
@@ -143,15 +149,14 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
         r.k[b][1] = RPA_KV_LD16(kp + off + 16);
       } else {
 #pragma unroll
-        for (int st = 0; st < 4; ++st) r.k[b][st] = RPA_KV_LD16(kp + off + st * 64);
+        for (int st = 0; st < kSteps; ++st) r.k[b][st] = RPA_KV_LD16(kp + off + st * 64);
       }
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int tin = min(tb + tok_slot(g, i), s.last_tok) - t0;
       const uint32_t off = (uint32_t)(tin * kv.tok_stride + c * kLaneV);
-      if constexpr (FP8) r.v[i] = RPA_KV_LD8(vp + off);
-      else r.v[i] = RPA_KV_LD16(vp + off);
+      r.v[i] = ld_v(vp + off);
     }
   } else {
 #pragma unroll
@@ -166,7 +171,7 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
         r.k[b][1] = RPA_KV_LD16(kp + 16);
       } else {
 #pragma unroll
-        for (int st = 0; st < 4; ++st) r.k[b][st] = RPA_KV_LD16(kp + st * 64);
+        for (int st = 0; st < kSteps; ++st) r.k[b][st] = RPA_KV_LD16(kp + st * 64);
       }
     }
 #pragma unroll
@@ -176,8 +181,7 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
       const int page = WINDOW ? win[slot - win_first] : s.pages[slot];
       const char* vp = vh + (int64_t)page * kv.page_stride +
                        (int64_t)((tok - slot * s.page_size) * kv.tok_stride + c * kLaneV);
-      if constexpr (FP8) r.v[i] = RPA_KV_LD8(vp);
-      else r.v[i] = RPA_KV_LD16(vp);
+      r.v[i] = ld_v(vp);
     }
   }
 }
@@ -185,14 +189,14 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
 // Leave a row's new token, its last one, in the cache: the registers of the block that ends the row hold it (token t of
 // the block), K dims of token 16b + c in lanes (c, g), V rows of slot i in lanes (., g).  kh / vh: this kv head's rows of
 // the page, tin: the token's place in it.
-template <bool FP8>
+template <bool FP8, bool HALF = false>
 __device__ __forceinline__ void store_new_token(const KvRegs<FP8>& r, const KvAddr& kv, const char* kh, const char* vh,
                                                 int page, int tin, int t, int c, int g) {
   const int64_t at = (int64_t)page * kv.page_stride + (int64_t)(tin * kv.tok_stride);
   char* kp = const_cast<char*>(kh) + at;
   char* vp = const_cast<char*>(vh) + at;
   // (branches on t, which is the same in every lane: selects between the registers would take their address)
-  constexpr int kN = FP8 ? 2 : 4, kStep = FP8 ? 16 : 64;
+  constexpr int kN = FP8 || HALF ? 2 : 4, kStep = FP8 ? 16 : 64;
   t = __builtin_amdgcn_readfirstlane(t);
   if (c == (t & 15)) {
     kp += g * (FP8 ? 32 : 16);
@@ -202,6 +206,10 @@ __device__ __forceinline__ void store_new_token(const KvRegs<FP8>& r, const KvAd
     } else {
 #pragma unroll
       for (int st = 0; st < kN; ++st) st16(kp + st * kStep, r.k[1][st]);
+    }
+    if constexpr (HALF) {
+      st16(kp + 128, u32x4_t{0u, 0u, 0u, 0u});
+      st16(kp + 192, u32x4_t{0u, 0u, 0u, 0u});
     }
   }
   if (g == ((t >> 2) & 3)) {
@@ -227,7 +235,7 @@ struct ScoreOpts {
 };
 
 // K operands (A of S^T = K Q^T) of one 32-token block: [token half][k step]
-template <bool FP8>
+template <bool FP8, bool HALF = false>
 __device__ __forceinline__ void k_operands(const KvRegs<FP8>& r, u32x4_t (&kA)[2][4]) {
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
@@ -242,7 +250,7 @@ __device__ __forceinline__ void k_operands(const KvRegs<FP8>& r, u32x4_t (&kA)[2
       }
     } else {
 #pragma unroll
-      for (int st = 0; st < 4; ++st) kA[b][st] = r.k[b][st];
+      for (int st = 0; st < (HALF ? 2 : 4); ++st) kA[b][st] = r.k[b][st];
     }
   }
 }
@@ -278,12 +286,12 @@ __device__ __forceinline__ void v_operands(const KvRegs<FP8>& r, u32x4_t (&vA)[8
   }
 }
 
-template <int MT, bool FP8, bool CAP>
+template <int MT, bool FP8, bool CAP, bool HALF = false>
 __device__ __forceinline__ void compute_block(const KvRegs<FP8>& r, const u32x4_t (&qB)[MT][4],
                                               f32x4_t (&acc)[MT][8], float (&m)[MT], float (&l)[MT],
                                               const ScoreOpts& so, int tb, int g) {
   u32x4_t kA[2][4];
-  k_operands<FP8>(r, kA);
+  k_operands<FP8, HALF>(r, kA);
   u32x4_t vA[8];
   v_operands<FP8>(r, vA);
   const bool need_mask = (tb + kBlk > so.kv_len) || (tb < so.t_lo);
@@ -294,7 +302,7 @@ __device__ __forceinline__ void compute_block(const KvRegs<FP8>& r, const u32x4_
     for (int b = 0; b < 2; ++b) {
       s[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int st = 0; st < 4; ++st) s[b] = mfma16(kA[b][st], qB[mt][st], s[b]);
+      for (int st = 0; st < (HALF ? 2 : 4); ++st) s[b] = mfma16(kA[b][st], qB[mt][st], s[b]);
     }
     float x[8];
 #pragma unroll
@@ -377,11 +385,11 @@ __device__ __forceinline__ void load_queries(const DecodeArgs& a, int tq, int hk
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int row = row0 + mt * 16 + c;
-    const uint16_t* qp = a.q + ((int64_t)tq * a.Hq + (int64_t)hk * a.G + row) * 128;
+    const uint16_t* qp = a.q + ((int64_t)tq * a.Hq + (int64_t)hk * a.G + row) * a.q_dim;
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
       const int d0 = FP8 ? (g * 32 + st * 8) : (st * 32 + g * 8);
-      qB[mt][st] = (row < a.G) ? ld16(qp + d0) : u32x4_t{0u, 0u, 0u, 0u};
+      qB[mt][st] = ld_query(qp, row < a.G ? d0 : a.q_dim, a.q_dim);
     }
   }
 }
@@ -413,9 +421,10 @@ __device__ __forceinline__ void write_rows(const DecodeArgs& a, const f32x4_t (&
     const int head = hk * a.G + row;
     if (dest.final_rows) {
       const float inv = a.sm.sink ? vs * sink_inverse(m[mt], lt, sink_logit(a.sm.sink, a.sm.round_logits, head)) : vs / lt;
-      uint16_t* op = a.out + ((int64_t)tq * a.Hq + head) * 128 + g * 32;
+      uint16_t* op = a.out + ((int64_t)tq * a.Hq + head) * a.q_dim + g * 32;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
+        if (g * 32 + r * 8 >= a.q_dim) break;
         u32x4_t w;
 #pragma unroll
         for (int jp = 0; jp < 4; ++jp)
@@ -461,7 +470,7 @@ struct RowRef {
 };
 
 // One wave, one (row, kv head, group of 16 query heads), tokens [t_begin, t_end).
-template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP>
+template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool HALF>
 __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef& row, int hk, int rg, int t_lo,
                                                int t_begin, int t_end, const PartDest dest, int lane) {
   const int kv_len = row.kv_len;
@@ -548,26 +557,26 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
   auto leave_new_token = [&](const KvRegs<FP8>& r, int tb) __attribute__((always_inline)) {
     if (rare(a.new_k && tb + kBlk > sv.last_tok)) {
       const int slot = __builtin_amdgcn_readfirstlane(page_slot_of(sv, sv.last_tok));
-      store_new_token<FP8>(r, a.kv, kh, vh, scalar_load_i32(sv.pages + slot), sv.last_tok - slot * sv.page_size,
+      store_new_token<FP8, HALF>(r, a.kv, kh, vh, scalar_load_i32(sv.pages + slot), sv.last_tok - slot * sv.page_size,
                            sv.last_tok - tb, c, g);
     }
   };
   KvRegs<FP8> ra, rb;
   int pg_next = page_of(block_tok(1));
   cover(t_begin);
-  load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true>(ra, a, sv, kh, vh, t_begin, page_of(t_begin), c, g, win, win_first);
+  load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true, HALF>(ra, a, sv, kh, vh, t_begin, page_of(t_begin), c, g, win, win_first);
   for (int blk = 0; blk < nblk; blk += 2) {
     cover(block_tok(blk + 1));
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true>(rb, a, sv, kh, vh, block_tok(blk + 1), pg_next, c, g, win, win_first);
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true, HALF>(rb, a, sv, kh, vh, block_tok(blk + 1), pg_next, c, g, win, win_first);
     pg_next = page_of(block_tok(blk + 2));
     leave_new_token(ra, t_begin + blk * kBlk);
-    compute_block<MT, FP8, CAP>(ra, qB, acc, m, l, so, t_begin + blk * kBlk, g);
+    compute_block<MT, FP8, CAP, HALF>(ra, qB, acc, m, l, so, t_begin + blk * kBlk, g);
     if (blk + 1 >= nblk) break;
     cover(block_tok(blk + 2));
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true>(ra, a, sv, kh, vh, block_tok(blk + 2), pg_next, c, g, win, win_first);
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true, HALF>(ra, a, sv, kh, vh, block_tok(blk + 2), pg_next, c, g, win, win_first);
     pg_next = page_of(block_tok(blk + 3));
     leave_new_token(rb, t_begin + (blk + 1) * kBlk);
-    compute_block<MT, FP8, CAP>(rb, qB, acc, m, l, so, t_begin + (blk + 1) * kBlk, g);
+    compute_block<MT, FP8, CAP, HALF>(rb, qB, acc, m, l, so, t_begin + (blk + 1) * kBlk, g);
   }
 
   write_rows<MT>(a, acc, m, l, tq, hk, row0, dest, c, g);
@@ -606,7 +615,7 @@ __device__ __forceinline__ bool fixed_row(const DecodeArgs& a, int index, RowRef
 
 // ---- fixed split plan: grid = (max_splits * rows, 1, head groups * row groups), splits fastest (rows do
 // not sit on a grid dimension of their own: that one ends at 65535); block = NW waves
-template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP>
+template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool HALF = false>
 __global__ __launch_bounds__(256, 2) void rpa_decode_splitkv_kernel(const DecodeArgs a) {
   const int nsp = max(a.max_splits, 1);
   const int index = (int)(blockIdx.x / (unsigned)nsp);
@@ -631,7 +640,7 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_splitkv_kernel(const Decode
   dest.final_rows = a.max_splits == 1;
   dest.by_head = true;
   dest.base = ((int64_t)index * a.max_splits + split) * a.Hq;
-  decode_segment<MT, FP8, UNIFORM_PAGE, CAP>(a, row, hk, rg, t_lo, t_begin, t_end, dest, lane);
+  decode_segment<MT, FP8, UNIFORM_PAGE, CAP, HALF>(a, row, hk, rg, t_lo, t_begin, t_end, dest, lane);
 }
 
 // ---- balanced plan ------------------------------------------------------------------------
@@ -836,8 +845,8 @@ __device__ __forceinline__ void merge_unit(const DecodeArgs& a, const PendingMer
   for (int i = 0; i < 16; ++i) {
     const float inv = __shfl(inv_r, i);
     if (i < pm.rows) {
-      uint32_t* op = reinterpret_cast<uint32_t*>(a.out + ((int64_t)pm.tq * a.Hq + pm.head0 + i) * 128 + 2 * lane);
-      *op = pack_bf16x2(acc[i][0] * inv, acc[i][1] * inv);
+      uint32_t* op = reinterpret_cast<uint32_t*>(a.out + ((int64_t)pm.tq * a.Hq + pm.head0 + i) * a.q_dim + 2 * lane);
+      if (2 * lane < a.q_dim) *op = pack_bf16x2(acc[i][0] * inv, acc[i][1] * inv);
     }
   }
   if (lane == 0) __hip_atomic_store(pm.ctr, generation << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -852,7 +861,7 @@ __device__ __forceinline__ void merge_unit(const DecodeArgs& a, const PendingMer
 // and neither does a block: under load a small dependent load waits behind megabytes of queued
 // KV traffic (10 us and more), so there are none after the first block.
 // New tokens (a.new_k) are taken where pages hold whole blocks; with smaller pages there is no register left for it.
-template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool MERGE>
+template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool MERGE, bool HALF = false>
 __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const DecodeArgs a_in) {
   DecodeArgs a = a_in;  // static-shape mode: the number of decode rows comes from the device
   if (a.dist) a.num_rows = min(a.num_rows, scalar_load_i32(a.dist));
@@ -982,7 +991,7 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
   {
     const int hk = min(cur.hk, a.Hkv - 1);
     const SeqView sv = view_of(cur.row, hk);
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE>(ra, a, sv, a.kv.k_base + (int64_t)hk * a.kv.head_stride,
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE, HALF>(ra, a, sv, a.kv.k_base + (int64_t)hk * a.kv.head_stride,
                                   a.kv.v_base + (int64_t)hk * a.kv.head_stride, cur.t_first,
                                   page_in(win, cur.t_first), c, g, lanes_win(win), win.first);
   }
@@ -1068,17 +1077,17 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
         // The next piece's window was requested at block resolve_at, in front of that block's
         // prefetch.  Two blocks later a wait for younger loads has passed; earlier it has not.
         if (i <= resolve_at + 1) wait_all_loads();
-        load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE>(fill, a, nsv, nkh, nvh, nxt.t_first, page_in(nwin, nxt.t_first), c, g,
+        load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE, HALF>(fill, a, nsv, nkh, nvh, nxt.t_first, page_in(nwin, nxt.t_first), c, g,
                                       lanes_win(nwin), nwin.first);
       } else {
         const int ptb = last ? tb : tb + kBlk;
-        load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE>(fill, a, sv, kh, vh, ptb, page_in(win, ptb), c, g, lanes_win(win), win.first);
+        load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE, HALF>(fill, a, sv, kh, vh, ptb, page_in(win, ptb), c, g, lanes_win(win), win.first);
       }
       if (UNIFORM_PAGE && rare(a.new_k && tb + kBlk > sv.last_tok)) {  // the block that ends the row
         const int slot = slot_of_tok(sv.last_tok);
-        store_new_token<FP8>(use, a.kv, kh, vh, page_in(win, sv.last_tok), sv.last_tok - slot * page_size, sv.last_tok - tb, c, g);
+        store_new_token<FP8, HALF>(use, a.kv, kh, vh, page_in(win, sv.last_tok), sv.last_tok - slot * page_size, sv.last_tok - tb, c, g);
       }
-      compute_block<MT, FP8, CAP>(use, qB, acc, m, l, so, tb, g);
+      compute_block<MT, FP8, CAP, HALF>(use, qB, acc, m, l, so, tb, g);
     };
     // the piece's first block sits in ra or in rb, wherever the piece before it ended
     {
@@ -1250,7 +1259,8 @@ __device__ __forceinline__ void merge_rows(const DecodeArgs& a, int tq, int head
     }
   }
   const float inv = a.sm.sink ? sink_inverse(mstar, den, sink_logit(a.sm.sink, a.sm.round_logits, head)) : 1.0f / den;
-  uint32_t* op = reinterpret_cast<uint32_t*>(a.out + ((int64_t)tq * a.Hq + head) * HD + d);
+  if (d >= a.q_dim) return;
+  uint32_t* op = reinterpret_cast<uint32_t*>(a.out + ((int64_t)tq * a.Hq + head) * a.q_dim + d);
 #pragma unroll
   for (int e = 0; e < kDpl; e += 2) op[e / 2] = pack_bf16x2(acc[e] * inv, acc[e + 1] * inv);
 }
@@ -1348,13 +1358,13 @@ __global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int
   const int row = rg * 16 + c;
   u32x4_t qB[2][4];
   {
-    const uint16_t* qp = a.q + ((int64_t)tok_row * a.Hq + (int64_t)hk * a.G + min(row, a.G - 1)) * 256;
+    const uint16_t* qp = a.q + ((int64_t)tok_row * a.Hq + (int64_t)hk * a.G + min(row, a.G - 1)) * a.q_dim;
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
         const int d0 = hf * 128 + (FP8 ? (g * 32 + st * 8) : (st * 32 + g * 8));
-        qB[hf][st] = ld16(qp + d0);
+        qB[hf][st] = ld_query(qp, d0, a.q_dim);
         if (a.sm.q_scale > 0.f) qB[hf][st] = requantise_q(qB[hf][st], a.sm.q_scale, FP8);
       }
   }
@@ -1475,11 +1485,12 @@ __global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int
     return;
   }
   const float inv = a.sm.sink ? vs * sink_inverse(m, l, sink_logit(a.sm.sink, a.sm.round_logits, head)) : vs / l;
-  uint16_t* op = a.out + ((int64_t)tok_row * a.Hq + head) * 256 + g * 32;
+  uint16_t* op = a.out + ((int64_t)tok_row * a.Hq + head) * a.q_dim + g * 32;
 #pragma unroll
   for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
+      if (hf * 128 + g * 32 + r * 8 >= a.q_dim) break;
       u32x4_t w;
 #pragma unroll
       for (int jp = 0; jp < 4; ++jp) w[jp] = pack_bf16x2(acc[hf][2 * jp][r] * inv, acc[hf][2 * jp + 1][r] * inv);
@@ -1557,9 +1568,10 @@ __global__ __launch_bounds__(256) void rpa_kv_write_kernel(const KvWriteArgs a_i
   const int64_t off = (int64_t)pages[slot] * a.kv.page_stride +
                       (int64_t)(pos - slot * a.pt.page_size) * a.kv.tok_stride +
                       (int64_t)head * a.kv.head_stride + inner;
-  const int64_t src = (int64_t)t * a.Hkv * a.head_bytes + byte;
-  st16(const_cast<char*>(a.kv.k_base) + off, ld16(a.keys + src));
-  st16(const_cast<char*>(a.kv.v_base) + off, ld16(a.values + src));
+  const int64_t src = ((int64_t)t * a.Hkv + head) * a.src_head_bytes + inner;
+  const bool real = inner < a.src_head_bytes;  // (a narrow head's row ends in zeros)
+  st16(const_cast<char*>(a.kv.k_base) + off, real ? ld16(a.keys + src) : u32x4_t{0u, 0u, 0u, 0u});
+  st16(const_cast<char*>(a.kv.v_base) + off, real ? ld16(a.values + src) : u32x4_t{0u, 0u, 0u, 0u});
 }
 
 template <bool FP8, bool UNIFORM, bool CAP>
@@ -1571,6 +1583,14 @@ void launch_decode_variant(const DecodeArgs& a, dim3 grid, dim3 block, hipStream
   const bool one_round = (int64_t)grid.x * grid.z * (block.x / 64) <= 2048;
   const int forced = tuning().decode_lds_kb;
   const unsigned lds = forced >= 0 ? (unsigned)forced << 10 : !one_round ? 0u : block.x >= 256 ? 84u << 10 : block.x >= 128 ? 54u << 10 : 34u << 10;
+  // heads of 64 dims (rows of 128, the second half zero): half the bytes.  (Not with the opt-in merge inside the kernel.)
+  if constexpr (!FP8) {
+    if (a.q_dim == 64 && !(a.balanced && a.merge_counters)) {
+      if (a.balanced) hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, false, UNIFORM, CAP, false, true>), grid, block, lds, st, a);
+      else hipLaunchKernelGGL((rpa_decode_splitkv_kernel<1, false, UNIFORM, CAP, true>), grid, block, lds, st, a);
+      return;
+    }
+  }
   if (a.balanced && a.merge_counters)
     hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, FP8, UNIFORM, CAP, true>), grid, block, lds, st, a);
   else if (a.balanced)

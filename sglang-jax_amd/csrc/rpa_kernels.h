@@ -58,6 +58,7 @@ struct DecodeArgs {
   float* ws_ml;  // [num_rows, max_splits, Hq, 2]  (running max in log2 units, sum)
   int32_t num_rows;  // decode sequences
   int32_t Hq, Hkv, G;
+  int32_t q_dim;       // elements of a row of q, out, new_k, new_v (<= the head dim of the cache, whose rest is zero)
   int32_t chunk;       // fixed plan: kv tokens per split (multiple of 32)
   int32_t max_splits;  // fixed plan: grid.x
   int32_t fp8;
@@ -94,6 +95,7 @@ struct PrefillArgs {
   const float* v_scale;
   int32_t seq_begin, seq_end;  // sequences [seq_begin, seq_end)
   int32_t Hq, Hkv, G;
+  int32_t q_dim;       // elements of a row of q and out (<= head_dim)
   int32_t max_q_len;
   int32_t max_kv_len;  // host bound on kv_len of these sequences, 0 = unknown
   int32_t fp8;
@@ -134,6 +136,7 @@ struct KvWriteArgs {
   int32_t num_seqs;
   int32_t Hkv;
   int32_t head_bytes;
+  int32_t src_head_bytes;  // of a head in keys / values (<= head_bytes; the rest of the cached row is set to zero)
   int32_t num_tokens;
   const int32_t* dist;  // device i32[3] or nullptr: when given, num_seqs is only a bound on dist[2]
   // decode rows whose tokens the decode kernel writes itself are left out: sequences [0, seq_begin), with dist

@@ -83,9 +83,9 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
   u32x4_t qB[T::kSteps];
   {
     const int rr = min(wr.row, w.q_len - 1);
-    const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * HD + h * 8;
+    const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * a.q_dim;
 #pragma unroll
-    for (int ks = 0; ks < T::kSteps; ++ks) qB[ks] = ld16(qp + ks * 16);
+    for (int ks = 0; ks < T::kSteps; ++ks) qB[ks] = ld_query(qp, ks * 16 + h * 8, a.q_dim);
     if (EXT && a.sm.q_scale > 0.f) {
 #pragma unroll
       for (int ks = 0; ks < T::kSteps; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, false);
@@ -338,9 +338,9 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillA
   // ---- Q^T operands: column c = position, k-step ks covers dims 32 ks + 8 g ..
   u32x4_t qB[8];
   {
-    const uint16_t* qp = a.q + ((int64_t)(w.qg0 + min(row, w.q_len - 1)) * a.Hq + w.head) * 256 + g * 8;
+    const uint16_t* qp = a.q + ((int64_t)(w.qg0 + min(row, w.q_len - 1)) * a.Hq + w.head) * a.q_dim;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qB[ks] = ld16(qp + ks * 32);
+    for (int ks = 0; ks < 8; ++ks) qB[ks] = ld_query(qp, ks * 32 + g * 8, a.q_dim);
     if (EXT && a.sm.q_scale > 0.f) {
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, FP8);
@@ -576,10 +576,11 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillA
   }
   const float vs = a.v_scale ? a.v_scale[w.hk] : 1.0f;
   const float inv = a.sm.sink ? vs * sink_inverse(m * sc2, l, sink_logit(a.sm.sink, a.sm.round_logits, w.head)) : vs / l;
-  uint16_t* op = a.out + out_row * 256 + 4 * g;
+  uint16_t* op = a.out + out_row * a.q_dim + 4 * g;
 #pragma unroll
   for (int j = 0; j < 16; ++j)
-    *reinterpret_cast<u32x2_t*>(op + 16 * j) = u32x2_t{pack_bf16x2(O[j][0] * inv, O[j][1] * inv), pack_bf16x2(O[j][2] * inv, O[j][3] * inv)};
+    if (16 * j + 4 * g < a.q_dim)
+      *reinterpret_cast<u32x2_t*>(op + 16 * j) = u32x2_t{pack_bf16x2(O[j][0] * inv, O[j][1] * inv), pack_bf16x2(O[j][2] * inv, O[j][3] * inv)};
 }
 
 }  // namespace
@@ -732,9 +733,9 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const Prefil
   u32x4_t qB[8];
   {
     const int rr = min(wr.row, w.q_len - 1);
-    const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * 128 + h * 8;
+    const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * a.q_dim;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qB[ks] = ld16(qp + ks * 16);
+    for (int ks = 0; ks < 8; ++ks) qB[ks] = ld_query(qp, ks * 16 + h * 8, a.q_dim);
     if (EXT && a.sm.q_scale > 0.f) {
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, FP8);
@@ -856,7 +857,20 @@ __global__ __launch_bounds__(256) void rpa_mask_bits_kernel(const PrefillArgs a)
   const int seq = mask_owner_of_token(a.pt.cu_q_lens, seq_end, token);
   const int kv_len = a.pt.kv_lens[seq];
   const int width = a.sm.mask_rows_page_aligned ? (a.pt.cu_kv_lens[seq + 1] - a.pt.cu_kv_lens[seq]) : kv_len;
-  const int32_t* row = a.sm.custom_mask + a.sm.cu_mask_lens[seq] + (int64_t)(token - a.pt.cu_q_lens[seq]) * width;
+  // where the sequence's rows start: given, or the sum over the sequences before it (cheap beside the rows themselves, and
+  // the caller is spared a scan of its own)
+  int64_t first = 0;
+  if (a.sm.cu_mask_lens) {
+    first = a.sm.cu_mask_lens[seq];
+  } else {
+    for (int s = (int)(threadIdx.x & 63); s < seq; s += 64) {
+      const int n = a.pt.cu_q_lens[s + 1] - a.pt.cu_q_lens[s];
+      first += (int64_t)n * (a.sm.mask_rows_page_aligned ? a.pt.cu_kv_lens[s + 1] - a.pt.cu_kv_lens[s] : a.pt.kv_lens[s]);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off);
+  }
+  const int32_t* row = a.sm.custom_mask + first + (int64_t)(token - a.pt.cu_q_lens[seq]) * width;
   uint64_t* out = a.mask_bits + (int64_t)token * a.mask_pitch;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int words = min((kv_len + 63) >> 6, a.mask_pitch);

@@ -199,7 +199,7 @@ __device__ __forceinline__ MaskCtx make_mask_ctx(const PrefillArgs& a, const Wor
   mc.bits = nullptr;
   mc.bit_words = a.mask_pitch;
   if (mc.mode == 1 && a.mask_bits) mc.bits = a.mask_bits + (int64_t)(w.qg0 + min(row, w.q_len - 1)) * a.mask_pitch;
-  if (mc.mode == 1) {
+  if (mc.mode == 1 && a.sm.cu_mask_lens) {
     const int width = a.sm.mask_rows_page_aligned ? (a.pt.cu_kv_lens[w.seq + 1] - a.pt.cu_kv_lens[w.seq]) : w.kv_len;
     mc.row = a.sm.custom_mask + a.sm.cu_mask_lens[w.seq] + (int64_t)min(row, w.q_len - 1) * width;
   }
@@ -328,11 +328,12 @@ __device__ __forceinline__ void write_rows(const PrefillArgs& a, const Work& w, 
   if (!wr.active || wr.row >= w.q_len) return;
   const float vs = a.v_scale ? a.v_scale[w.hk] : 1.0f;
   const float inv = a.sm.sink ? vs * sink_inverse(m2, l, sink_logit(a.sm.sink, a.sm.round_logits, w.head)) : vs / l;
-  uint16_t* op = a.out + ((int64_t)(w.qg0 + wr.row) * a.Hq + w.head) * (ND * 32) + 4 * h;
+  uint16_t* op = a.out + ((int64_t)(w.qg0 + wr.row) * a.Hq + w.head) * a.q_dim + 4 * h;
 #pragma unroll
   for (int d = 0; d < ND; ++d)
 #pragma unroll
     for (int vq = 0; vq < 4; ++vq) {
+      if (d * 32 + vq * 8 >= a.q_dim) break;
       u32x2_t o = {pack_bf16x2(O[d][4 * vq + 0] * inv, O[d][4 * vq + 1] * inv),
                    pack_bf16x2(O[d][4 * vq + 2] * inv, O[d][4 * vq + 3] * inv)};
       *reinterpret_cast<u32x2_t*>(op + d * 32 + vq * 8) = o;
@@ -468,7 +469,8 @@ static __global__ __launch_bounds__(64) void rpa_prefill_combine_kernel(const Pr
   }
   const float vs = a.v_scale ? a.v_scale[head / a.G] : 1.0f;
   const float inv = a.sm.sink ? vs * sink_inverse(mstar, den, sink_logit(a.sm.sink, a.sm.round_logits, head)) : vs / den;
-  uint32_t* op = reinterpret_cast<uint32_t*>(a.out + ((int64_t)token * a.Hq + head) * HD + kDpl * lane);
+  if (kDpl * lane >= a.q_dim) return;
+  uint32_t* op = reinterpret_cast<uint32_t*>(a.out + ((int64_t)token * a.Hq + head) * a.q_dim + kDpl * lane);
 #pragma unroll
   for (int e = 0; e < kDpl; e += 2) op[e / 2] = pack_bf16x2(acc[e] * inv, acc[e + 1] * inv);
 }

@@ -356,10 +356,10 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
     const int row = r_lo + 32 * q + c;
     b[q].qpos = w.prefix + row;
     const int rr = min(row, w.q_len - 1);
-    const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * 128 + h * 8;
+    const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * a.q_dim;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      const u32x4_t x = ld16(qp + ks * 16);
+      const u32x4_t x = ld_query(qp, ks * 16 + h * 8, a.q_dim);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         b[q].Q[4 * ks + e] = pack_bf16x2(bf16_lo_to_f32(x[e]) * sc2, bf16_hi_to_f32(x[e]) * sc2);

@@ -160,13 +160,13 @@ int without_gil(F f) {
 
 // attention(q, k, v, cache, kv_lens, page_indices, cu_q_lens, cu_kv_lens, distribution, attention_sink, causal, sm_scale,
 //           sliding_window, soft_cap, mask_value, q_scale, k_scale, v_scale, xai_temperature_len, softmax_dtype,
-//           chunk_prefill_size, max_kv_len, max_q_len, num_splits, host_kv_lens, head_dim)
+//           chunk_prefill_size, max_kv_len, max_q_len, num_splits, host_kv_lens, head_dim, custom_mask, mask_aligned)
 // -> output, a status below 0, or None.  head_dim 0: q, k, v are [T, heads, D]; else they may be [T, heads * D], and
-// so is the output.
+// so is the output.  custom_mask is read where causal is false.
 PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  if (nargs != 26) {
-    PyErr_SetString(PyExc_TypeError, "attention takes 26 arguments");
+  if (nargs != 28) {
+    PyErr_SetString(PyExc_TypeError, "attention takes 28 arguments");
     return nullptr;
   }
   const at::Tensor* q = tensor(a[0]);
@@ -179,14 +179,17 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   int64_t head_dim;
   COMMON(whole(a[25], head_dim));
   const int64_t D = cache->size(3), T = q->size(0), Hkv = cache->size(2) / 2;
-  COMMON(D == 128 || D == 256);
+  COMMON((D == 128 || D == 256) && (q->dim() == 2 || q->dim() == 3));
+  // rows narrower than the cache's (which end in zeros)
+  const int64_t row = q->dim() == 3 ? q->size(2) : head_dim;
+  COMMON(row > 0 && row <= D && D - row < 128 && row % (kv_type == at::kBFloat16 ? 8 : 16) == 0);
   int64_t Hq;
   if (q->dim() == 3) {
-    COMMON(q->size(2) == D && (head_dim == 0 || head_dim == D));
+    COMMON(head_dim == 0 || head_dim == row);
     Hq = q->size(1);
   } else {
-    COMMON(q->dim() == 2 && head_dim == D && q->size(1) % D == 0);
-    Hq = q->size(1) / D;
+    COMMON(q->size(1) % row == 0);
+    Hq = q->size(1) / row;
   }
   COMMON(Hkv > 0 && cache->size(2) % 2 == 0 && Hq > 0 && Hq % Hkv == 0);
 
@@ -195,7 +198,7 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const at::Tensor *k = tensor(a[1]), *v = tensor(a[2]);
     COMMON(k && v && k->device() == dev && v->device() == dev && k->scalar_type() == kv_type &&
            v->scalar_type() == kv_type && k->sizes() == v->sizes() && k->dim() == q->dim() && k->size(0) == T);
-    COMMON(k->dim() == 3 ? (k->size(1) == Hkv && k->size(2) == D) : k->size(1) == Hkv * D);
+    COMMON(k->dim() == 3 ? (k->size(1) == Hkv && k->size(2) == row) : k->size(1) == Hkv * row);
     keys = k->contiguous();
     values = v->contiguous();
   } else {
@@ -222,6 +225,14 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   const int causal = PyObject_IsTrue(a[10]);
   COMMON(causal >= 0);
   p.mask_mode = causal ? RPA_MASK_CAUSAL : RPA_MASK_NONE;
+  if (!causal && !none(a[26])) {
+    const at::Tensor* mask = on_device(a[26], dev, at::kInt);
+    const int aligned = PyObject_IsTrue(a[27]);
+    COMMON(mask && aligned >= 0);
+    p.mask_mode = RPA_MASK_CUSTOM;
+    p.custom_mask = mask->const_data_ptr<int32_t>();
+    p.mask_rows_page_aligned = aligned;
+  }
   double d;
   COMMON(real(a[11], d));
   p.sm_scale = (float)d;
@@ -289,10 +300,12 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   p.num_q_heads = (int32_t)Hq;
   p.num_kv_heads = (int32_t)Hkv;
   p.head_dim = (int32_t)D;
+  p.q_head_dim = (int32_t)row;
   p.page_size = (int32_t)cache->size(1);
   p.total_pages = (int32_t)cache->size(0);
   p.layout = RPA_LAYOUT_FUSED;
   p.kv_dtype = kv_type == at::kBFloat16 ? RPA_KV_BF16 : RPA_KV_FP8_E4M3;
+  COMMON(!rpa_mask_needs_starts(&p));
   if (const size_t need = rpa_workspace_bytes(&p)) {
     at::Tensor& ws = workspace(dev, stream, need);
     p.workspace = ws.data_ptr();

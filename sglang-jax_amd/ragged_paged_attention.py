@@ -391,11 +391,12 @@ def ragged_paged_attention(
     bound) and the kernels read the batch composition themselves, as the jitted reference does
     (rpa_v3:1676): one prepared call serves every batch of a bucket.
     """
-    if out_dtype in (None, torch.bfloat16) and not (skip_kv_mask or validate_values) and (causal or custom_mask is None):
+    if out_dtype in (None, torch.bfloat16) and not (skip_kv_mask or validate_values):
         out = _lib.load_torch().attention(
             queries, keys, values, kv_cache_fused, kv_lens, page_indices, cu_q_lens, cu_kv_lens, distribution,
             attention_sink, causal, sm_scale, sliding_window, soft_cap, mask_value, q_scale, k_scale, v_scale,
-            xai_temperature_len, softmax_dtype, chunk_prefill_size, max_kv_len, max_q_len, num_splits, host_kv_lens, 0)
+            xai_temperature_len, softmax_dtype, chunk_prefill_size, max_kv_len, max_q_len, num_splits, host_kv_lens, 0,
+            custom_mask, mask_aligned_to_cu_kv)
         if out is not None:
             if type(out) is int:
                 _lib.check(out)

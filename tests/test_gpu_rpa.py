@@ -351,6 +351,33 @@ def test_wider_query_dtypes_come_back_in_their_own_type(pkg, wl, gpu, q_dtype):
     assert_parity(out.cpu().float(), want.float(), **BF16_TOL)
 
 
+@pytest.mark.parametrize("head_dim,P,kv_lens,window,cap", [
+    (64, 16, [1, 2, 17, 33, 64, 300], None, None), (64, 64, [1, 32, 33, 700, 64, 129], 100, None), (64, 24, [40, 5, 2000], None, 30.0),
+    (64, 64, [9000, 8191, 300, 12000, 1, 31, 5000, 2500] * 4, None, None), (96, 32, [1, 70, 600, 33], None, None)])
+def test_narrow_heads_decode_rows(pkg, wl, gpu, head_dim, P, kv_lens, window, cap):
+    """Decode rows of heads of 64 dims (half of a cached row is read) and of 96 on a pool of 128-wide rows: short rows, rows cut
+    in pieces, the balanced plan; the new tokens are written with zeros behind them, whatever was there."""
+    Hq, Hkv, S = 16, 4, len(kv_lens)
+    b = wl.make_batch("narrow_rows", [1] * S, kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=head_dim, page_size=P, seed=74,
+                      sliding_window=window, soft_cap=cap)
+    want = oracle_out(b)
+    full = torch.nn.functional.pad(b.kv_cache, (0, 128 - head_dim))
+    holed, table = full.clone(), b.padded_page_table()
+    keys, vals = torch.empty(S, Hkv, head_dim, dtype=torch.bfloat16), torch.empty(S, Hkv, head_dim, dtype=torch.bfloat16)
+    for i, n in enumerate(kv_lens):
+        page, row = int(table[i, (n - 1) // P]), (n - 1) % P
+        keys[i], vals[i] = b.kv_cache[page, row, 0::2], b.kv_cache[page, row, 1::2]
+        holed[page, row] = 7.0
+    say(f"case narrow rows D={head_dim} P={P} rows={S} window={window} cap={cap}")
+    g, cache = b.to(gpu), holed.to(gpu)
+    out, _ = pkg.ragged_paged_attention(g.q, keys.to(gpu), vals.to(gpu), cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens,
+                                        (S, S, S), None, sm_scale=b.sm_scale, sliding_window=window, soft_cap=cap,
+                                        max_kv_len=max(kv_lens), max_q_len=1, host_kv_lens=np.array(kv_lens, dtype=np.int32))
+    torch.cuda.synchronize()
+    assert torch.equal(cache.cpu().view(torch.int16), full.view(torch.int16))
+    assert_parity(out.cpu().float(), want.float(), **BF16_TOL)
+
+
 @pytest.mark.parametrize("head_dim,aligned_pool", [(64, True), (64, False), (96, True), (80, False), (192, True), (192, False)])
 def test_head_dims_that_are_not_a_multiple_of_128(pkg, wl, gpu, head_dim, aligned_pool):
     """rpa_v3:1187-1241, 1270-1296: queries, new tokens and narrow caches run zero-padded to the next
