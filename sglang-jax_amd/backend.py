@@ -247,6 +247,25 @@ class FlashAttentionMetadata:
     host_seq_lens: np.ndarray | None = field(default=None, repr=False)
 
 
+def _native_metadata(batch, page_size: int, device, mixed: bool):
+    """The metadata of a batch in its common form (integer arrays of one rank, no sliding-window pool) in native code:
+    one pass over the host arrays and one upload.  None: anything else."""
+    mode = _mode_name(batch.forward_mode)
+    seq_lens = batch.seq_lens
+    if mode not in ("EXTEND", "DECODE") or not isinstance(seq_lens, np.ndarray) or seq_lens.dtype != np.int32:
+        return None
+    if (getattr(batch, "per_dp_bs_size", None) or len(seq_lens)) != len(seq_lens) or device.type != "cuda":
+        return None
+    x = _lib.load_torch().metadata(mode == "DECODE", seq_lens, batch.cache_loc, getattr(batch, "extend_seq_lens", None),
+                                   page_size, mixed, torch.cuda.current_device() if device.index is None else device.index)
+    if x is None:
+        return None
+    return FlashAttentionMetadata(
+        cu_q_lens=x[0], cu_kv_lens=x[1], page_indices=x[2], seq_lens=x[3], distribution=x[4],
+        host_distribution=np.array(x[5], dtype=np.int32), max_kv_len=x[6], max_q_len=x[7], sum_visible=x[8],
+        host_seq_lens=seq_lens)
+
+
 class FlashAttention:
     """One-GPU counterpart of the reference's ``FlashAttention`` backend."""
 
@@ -263,6 +282,10 @@ class FlashAttention:
     def get_forward_metadata(self, batch) -> FlashAttentionMetadata:
         if getattr(batch, "dp_size", 1) != 1:
             raise NotImplementedError("one GPU: data-parallel sections (dp_size > 1) are not built")
+        if self.swa_index_mapping is None:
+            md = _native_metadata(batch, self.page_size, self.device, mixed=False)
+            if md is not None:
+                return md
         host = build_forward_metadata(
             forward_mode=batch.forward_mode,
             seq_lens=batch.seq_lens,
@@ -381,6 +404,9 @@ class MLAAttentionBackend:
     def get_forward_metadata(self, batch) -> FlashAttentionMetadata:
         if getattr(batch, "dp_size", 1) != 1:
             raise NotImplementedError("one GPU: data-parallel sections (dp_size > 1) are not built")
+        md = _native_metadata(batch, self.page_size, self.device, mixed=True)
+        if md is not None:
+            return md
         host = build_forward_metadata(
             forward_mode=batch.forward_mode,
             seq_lens=batch.seq_lens,

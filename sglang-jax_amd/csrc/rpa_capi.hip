@@ -807,6 +807,12 @@ int rpa_prefill(const RpaParams* p, void* stream) {
   return check_hip(rpa::launch_prefill(a, static_cast<hipStream_t>(stream)), "rpa_prefill");
 }
 
+int rpa_upload_i32(int32_t* dst, const int32_t* src, int32_t n, void* stream) {
+  if (n <= 0) return RPA_OK;
+  if (!dst || !src) return fail(RPA_EINVAL_NULL, "dst/src is NULL");
+  return check_hip(rpa::launch_upload(dst, src, n, static_cast<hipStream_t>(stream)), "rpa_upload_i32");
+}
+
 int rpa_mask_needs_starts(const RpaParams* p) { return p && p->mask_mode == RPA_MASK_CUSTOM && !mask_as_bits(p) ? 1 : 0; }
 
 // (narrow heads: only the kernels that know of the zeros behind 64 dims)

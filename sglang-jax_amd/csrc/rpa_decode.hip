@@ -21,6 +21,7 @@
 // GQA: the G query heads of a kv head are the (zero padded) 16 columns of Q^T.
 
 #include <cstdlib>
+#include <cstring>
 
 #include "rpa_common.h"
 #include "rpa_kernels.h"
@@ -1642,6 +1643,31 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
     e = hipGetLastError();
   }
   return e;
+}
+
+// A few KB of host words as kernel arguments: the words ride in the packet's argument buffer and the store is one more
+// kernel of the stream, where a copy is a hand-over to a copy engine and back (five small copies of a step's metadata took
+// 20 us of host time and 4 us of the GPU's each).  Up to three launches; beyond, a copy costs less.
+namespace {
+constexpr int kUploadWords = 896;  // 3.5 KB: under the 4 KB that arguments may take
+struct UploadWords {
+  int32_t w[kUploadWords];
+};
+__global__ __launch_bounds__(256) void rpa_upload_kernel(int32_t* dst, int n, const UploadWords words) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) dst[i] = words.w[i];
+}
+}  // namespace
+
+hipError_t launch_upload(int32_t* dst, const int32_t* src, int n, hipStream_t stream) {
+  if (n > 3 * kUploadWords) return hipMemcpyAsync(dst, src, (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, stream);
+  UploadWords words;
+  for (int at = 0; at < n; at += kUploadWords) {
+    const int m = min(n - at, kUploadWords);
+    memcpy(words.w, src + at, (size_t)m * sizeof(int32_t));
+    hipLaunchKernelGGL(rpa_upload_kernel, dim3((m + 255) / 256), dim3(256), 0, stream, dst + at, m, words);
+  }
+  return hipGetLastError();
 }
 
 hipError_t launch_gather(const GatherArgs& a, hipStream_t stream) {

@@ -217,6 +217,8 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream);
 // bytes of workspace that takes.
 int prefill_kv_splits(const PrefillArgs& a);
 size_t prefill_split_workspace_bytes(const PrefillArgs& a, int splits);
+// n host words to device memory, in stream order; the source may be reused at once
+hipError_t launch_upload(int32_t* dst, const int32_t* src, int n, hipStream_t stream);
 hipError_t launch_gather(const GatherArgs& a, hipStream_t stream);
 // head_dim 256: every query token of sequences [seq_begin, seq_end) as a row of its own; at most
 // max_token_rows tokens (a host bound) are covered.  With a.dist set, seq_end is a bound and dist_role says

@@ -9,6 +9,7 @@
 // but the split-KV workspace, one grow-only buffer per (device, stream).
 
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/DynamicTypes.h>
@@ -18,6 +19,7 @@
 #include <algorithm>
 #include <map>
 #include <utility>
+#include <vector>
 
 #include "../../include/rpa.h"
 
@@ -492,6 +494,70 @@ PyObject* sparse_mla(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// metadata(decode, seq_lens, cache_loc, extend_seq_lens, page_size, extend_is_mixed, device index)
+// -> (cu_q_lens, cu_kv_lens, page_indices, seq_lens, distribution on the device, distribution as a tuple, max_kv_len,
+// max_q_len, sum of visible lengths), or None: what build_forward_metadata works out for one data-parallel rank, in one
+// pass over the host arrays and one upload.
+PyObject* metadata(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 7) {
+    PyErr_SetString(PyExc_TypeError, "metadata takes 7 arguments");
+    return nullptr;
+  }
+  const bool decode = PyObject_IsTrue(a[0]) == 1, mixed = PyObject_IsTrue(a[5]) == 1;
+  HostInts lens, loc, ext;
+  int64_t P, index;
+  COMMON(lens.open(a[1]) && loc.open(a[2]) && (decode || (!none(a[3]) && ext.open(a[3]))) && whole(a[4], P) && P > 0 && whole(a[6], index));
+  const int64_t S = lens.size(), np = (loc.size() + P - 1) / P;
+  COMMON(S > 0 && (decode || ext.size() == S) && np <= INT32_MAX / 2);
+  // (16-byte aligned pieces of one buffer)
+  auto up4 = [](int64_t n) { return (n + 3) & ~(int64_t)3; };
+  const int64_t at_q = 0, at_kv = up4(S + 1), at_len = at_kv + up4(S + 1), at_dist = at_len + up4(S), at_page = at_dist + 4;
+  const int64_t total = at_page + np;
+  std::vector<int32_t> w((size_t)total);
+  int64_t cu_q = 0, cu_kv = 0, n = 0, max_kv = INT64_MIN, max_q = INT64_MIN;
+  for (int64_t s = 0; s < S; ++s) {
+    const int64_t kv = lens.at(s), q = decode ? 1 : ext.at(s);
+    COMMON(kv >= 0 && kv <= INT32_MAX - P && q >= 0);
+    cu_q += q;
+    cu_kv += (kv + P - 1) / P * P;
+    COMMON(cu_q <= INT32_MAX && cu_kv <= INT32_MAX);
+    w[at_q + s + 1] = (int32_t)cu_q;
+    w[at_kv + s + 1] = (int32_t)cu_kv;
+    w[at_len + s] = (int32_t)kv;
+    n += kv > 0;
+    max_kv = std::max(max_kv, kv);
+    max_q = std::max(max_q, q);
+  }
+  int64_t visible = 0;
+  for (int64_t s = 0; s < n; ++s) {
+    const int64_t q = decode ? 1 : ext.at(s);
+    visible += q * lens.at(s) - q * (q - 1) / 2;
+  }
+  const int32_t first = decode ? (int32_t)n : 0, mid = !decode && mixed ? 0 : (int32_t)n;
+  w[at_dist] = first, w[at_dist + 1] = mid, w[at_dist + 2] = (int32_t)n;
+  for (int64_t i = 0; i < np; ++i) {
+    const int64_t slot = loc.at(i * P);
+    COMMON(slot >= 0 && slot <= INT32_MAX);
+    w[at_page + i] = (int32_t)(slot / P);
+  }
+  const at::Device dev(at::kCUDA, (c10::DeviceIndex)index);
+  const c10::DeviceGuard guard(dev);
+  at::Tensor base = at::empty({total}, at::TensorOptions().dtype(at::kInt).device(dev));
+  const int rc = rpa_upload_i32(base.data_ptr<int32_t>(), w.data(), (int32_t)total, stream_of(dev));
+  COMMON(rc == RPA_OK);
+  const int64_t from[5] = {at_q, at_kv, at_page, at_len, at_dist}, size[5] = {S + 1, S + 1, np, S, 3};
+  PyObject* out = PyTuple_New(9);
+  if (!out) return nullptr;
+  for (int i = 0; i < 5; ++i) PyTuple_SET_ITEM(out, i, THPVariable_Wrap(base.narrow(0, from[i], size[i])));
+  PyTuple_SET_ITEM(out, 5, Py_BuildValue("(iii)", first, mid, (int)n));
+  PyTuple_SET_ITEM(out, 6, PyLong_FromLongLong(max_kv));
+  PyTuple_SET_ITEM(out, 7, PyLong_FromLongLong(max_q));
+  PyTuple_SET_ITEM(out, 8, PyLong_FromLongLong(visible));
+  return out;
+  END_HANDLE_TH_ERRORS
+}
+
 // workspace(tensor on the device, bytes) -> the buffer of its device's current stream, at least that long
 PyObject* py_workspace(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -509,6 +575,7 @@ PyMethodDef kMethods[] = {
     {"attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(attention)), METH_FASTCALL, nullptr},
     {"mla", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(mla)), METH_FASTCALL, nullptr},
     {"sparse_mla", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(sparse_mla)), METH_FASTCALL, nullptr},
+    {"metadata", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(metadata)), METH_FASTCALL, nullptr},
     {"workspace", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(py_workspace)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -174,3 +174,25 @@ def test_mla_backend_extend_then_decode(pkg, gpu):
     for s_ in range(2):
         say(f"mla decode {s_}")
         step(pkg.ForwardMode.DECODE, [1, 1, 1])
+
+
+@pytest.mark.parametrize("P,lens", [(16, [1]), (16, [17, 0, 5]), (1, [300, 800, 500]), (16, [9000, 40000, 7, 0])])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_metadata_in_one_upload(pkg, gpu, P, lens, mixed):
+    """The native metadata against the numpy builder, from one launch's worth of words to more than kernel arguments carry."""
+    rng = np.random.default_rng(5)
+    kv = np.array(lens, dtype=np.int32)
+    pages = rng.permutation(int((-(-kv // P)).sum()) + 3).astype(np.int32)
+    loc = (pages[: int((-(-kv // P)).sum())].astype(np.int64)[:, None] * P + np.arange(P)).reshape(-1).astype(np.int32)
+    for mode, ext in ((pkg.ForwardMode.DECODE, None), (pkg.ForwardMode.EXTEND, np.minimum(kv, 5))):
+        batch = SimpleNamespace(forward_mode=mode, seq_lens=kv, cache_loc=loc, extend_seq_lens=ext, dp_size=1, per_dp_bs_size=len(kv))
+        backend = (pkg.MLAAttentionBackend(16, 512, 128, 64, 128, page_size=P, device=gpu) if mixed and P > 1
+                   else pkg.FlashAttention(8, 2, 128, page_size=P, device=gpu))
+        md = backend.get_forward_metadata(batch)
+        want = pkg.build_forward_metadata(forward_mode=mode, seq_lens=kv, cache_loc=loc, extend_seq_lens=ext, page_size=P,
+                                          extend_distribution_is_mixed=isinstance(backend, pkg.MLAAttentionBackend))
+        for name in ("cu_q_lens", "cu_kv_lens", "page_indices", "seq_lens", "distribution"):
+            got = getattr(md, name)
+            assert got.dtype == torch.int32 and np.array_equal(got.cpu().numpy(), want[name]), name
+        assert np.array_equal(md.host_distribution, want["distribution"])
+        assert md.max_kv_len == kv.max() and md.max_q_len == (1 if ext is None else ext.max())
