@@ -326,7 +326,7 @@ RPA_API int rpa_kv_write(const RpaParams* p, const void* keys, const void* value
 RPA_API int rpa_attention_update(const RpaParams* p, const void* keys, const void* values, void* stream);
 
 /* n words of host memory to device memory in stream order (a batch's metadata); the source may be reused at once. */
-RPA_API int rpa_upload_i32(int32_t* dst, const int32_t* src, int32_t n, void* stream);
+RPA_API int rpa_upload_words(int32_t* dst, const int32_t* src, int32_t n, void* stream);
 
 /* Whether a RPA_MASK_CUSTOM call needs cu_mask_lens: 0 where the mask is turned into bits first (128-wide heads, max_kv_len
  * given, rpa_workspace_bytes() of workspace), which finds the starts of the sequences' rows by itself. */

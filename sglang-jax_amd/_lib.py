@@ -58,7 +58,7 @@ EXPORTED_SYMBOLS = (
     "rpa_attention_update",
     "rpa_mla_attention_update",
     "rpa_mask_needs_starts",
-    "rpa_upload_i32",
+    "rpa_upload_words",
     "rpa_mla_sparse_workspace_bytes",
     "rpa_mla_sparse_attention",
 )

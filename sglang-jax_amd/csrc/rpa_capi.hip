@@ -183,8 +183,9 @@ int wave_capacity() {
   return cap;
 }
 
+// one_round: the slots are all there is (one workgroup per CU), and a piece too many costs a round of its own.
 SplitPlan plan_splits(int64_t max_len, int window, int64_t units, int64_t work, int forced, int min_chunk,
-                      int capacity) {
+                      int capacity, bool one_round = false) {
   int64_t eff = max_len;
   if (window > 0 && eff > (int64_t)window + 31) eff = (int64_t)window + 31;
   if (eff < 1) eff = 1;
@@ -208,6 +209,9 @@ SplitPlan plan_splits(int64_t max_len, int window, int64_t units, int64_t work, 
   }
   chunk = (chunk + 31) / 32 * 32;
   if (chunk < 32) chunk = 32;
+  // (37 rows of 1024 tokens: 7 pieces of 160 are 259 workgroups, 56 us; 6 of 192 are 222, 43 us)
+  if (one_round && forced <= 0 && uniform && units <= capacity)
+    while ((eff + chunk - 1) / chunk * units > capacity) chunk += 32;
   int64_t splits = (eff + chunk - 1) / chunk;
   if (splits < 1) splits = 1;
   SplitPlan sp;
@@ -807,10 +811,10 @@ int rpa_prefill(const RpaParams* p, void* stream) {
   return check_hip(rpa::launch_prefill(a, static_cast<hipStream_t>(stream)), "rpa_prefill");
 }
 
-int rpa_upload_i32(int32_t* dst, const int32_t* src, int32_t n, void* stream) {
+int rpa_upload_words(int32_t* dst, const int32_t* src, int32_t n, void* stream) {
   if (n <= 0) return RPA_OK;
   if (!dst || !src) return fail(RPA_EINVAL_NULL, "dst/src is NULL");
-  return check_hip(rpa::launch_upload(dst, src, n, static_cast<hipStream_t>(stream)), "rpa_upload_i32");
+  return check_hip(rpa::launch_upload(dst, src, n, static_cast<hipStream_t>(stream)), "rpa_upload_words");
 }
 
 int rpa_mask_needs_starts(const RpaParams* p) { return p && p->mask_mode == RPA_MASK_CUSTOM && !mask_as_bits(p) ? 1 : 0; }
@@ -958,7 +962,7 @@ static SplitPlan mla_plan(const RpaMlaParams* p, int64_t rows) {
   int64_t work = p->sum_kv_len > 0 ? p->sum_kv_len * groups : 0;
   if (p->sliding_window > 0) work = 0;
   return plan_splits(bound, p->sliding_window, units, work, p->num_splits,
-                     rpa::tuning().mla_min_chunk, mla_wgs());
+                     rpa::tuning().mla_min_chunk, mla_wgs(), true);
 }
 
 static int mla_validate(const RpaMlaParams* p) {
@@ -1171,8 +1175,12 @@ RpaMlaParams sparse_view(const RpaMlaParams* p, const RpaMlaSparse* s) {
   v.cu_kv_lens = nullptr;
   if (rows) v.page_size = 1;
   v.pages_per_seq = rows ? s->topk_count : s->k_pages_max;
-  v.max_kv_len = v.pages_per_seq * v.page_size;
-  v.sum_kv_len = 0;
+  // a selection is as long as it can be, or as its sequence is: rows of one length, as far as the host knows (the fixed plan's
+  // even pieces, 32 rows x 4096 tokens 52.5 -> 46 us against the balanced plan)
+  int64_t bound = (int64_t)v.pages_per_seq * v.page_size;
+  if (s->pages_per_seq > 0) bound = std::min(bound, (int64_t)s->pages_per_seq * p->page_size);
+  v.max_kv_len = (int32_t)bound;
+  v.sum_kv_len = p->num_tokens * bound;
   v.num_splits = 0;
   v.distribution = nullptr;
   return v;

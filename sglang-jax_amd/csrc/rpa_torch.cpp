@@ -544,7 +544,7 @@ PyObject* metadata(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   const at::Device dev(at::kCUDA, (c10::DeviceIndex)index);
   const c10::DeviceGuard guard(dev);
   at::Tensor base = at::empty({total}, at::TensorOptions().dtype(at::kInt).device(dev));
-  const int rc = rpa_upload_i32(base.data_ptr<int32_t>(), w.data(), (int32_t)total, stream_of(dev));
+  const int rc = rpa_upload_words(base.data_ptr<int32_t>(), w.data(), (int32_t)total, stream_of(dev));
   COMMON(rc == RPA_OK);
   const int64_t from[5] = {at_q, at_kv, at_page, at_len, at_dist}, size[5] = {S + 1, S + 1, np, S, 3};
   PyObject* out = PyTuple_New(9);
