@@ -168,6 +168,9 @@ typedef struct RpaParams {
    * to a multiple of 128, rpa_v3:1187-1241): a multiple of 8 (e4m3: 16), head_dim - q_head_dim < 128; 0 = head_dim.
    * The rest of a cached row is zero, is written as zeros with the new tokens and adds nothing. */
   int32_t q_head_dim;
+  /* 1: no sequence of the call has tokens in the cache before its new ones (kv_len == query tokens, known on the host).
+   * rpa_attention_update then attends to the keys / values it is given and fills the cache beside that. */
+  int32_t prompts_only;
 } RpaParams;
 
 /*

@@ -107,6 +107,7 @@ class RpaParams(ctypes.Structure):
         ("q_scale", ctypes.c_float),
         ("distribution", ctypes.c_void_p),
         ("q_head_dim", ctypes.c_int32),
+        ("prompts_only", ctypes.c_int32),
     ]
 
 

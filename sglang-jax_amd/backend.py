@@ -244,6 +244,7 @@ class FlashAttentionMetadata:
     max_kv_len: int = 0
     max_q_len: int = 0
     sum_visible: int = 0
+    no_prefix: bool = False  # every sequence is a prompt whose tokens are all new
     host_seq_lens: np.ndarray | None = field(default=None, repr=False)
 
 
@@ -262,7 +263,7 @@ def _native_metadata(batch, page_size: int, device, mixed: bool):
         return None
     return FlashAttentionMetadata(
         cu_q_lens=x[0], cu_kv_lens=x[1], page_indices=x[2], seq_lens=x[3], distribution=x[4],
-        host_distribution=np.array(x[5], dtype=np.int32), max_kv_len=x[6], max_q_len=x[7], sum_visible=x[8],
+        host_distribution=np.array(x[5], dtype=np.int32), max_kv_len=x[6], max_q_len=x[7], sum_visible=x[8], no_prefix=x[9],
         host_seq_lens=seq_lens)
 
 
@@ -343,7 +344,7 @@ class FlashAttention:
         out = _lib.load_torch().attention(
             q, k, v, kv_cache_fused, md.seq_lens, page_indices, md.cu_q_lens, md.cu_kv_lens, md.host_distribution,
             attention_sink, causal, scale, window, soft_cap, None, None, None, None, xai, softmax_dtype, None,
-            md.max_kv_len, md.max_q_len, 0, md.host_seq_lens, head_dim, md.custom_mask, False)
+            md.max_kv_len, md.max_q_len, 0, md.host_seq_lens, head_dim, md.custom_mask, False, md.no_prefix)
         if out is not None:
             if type(out) is int:
                 _lib.check(out)

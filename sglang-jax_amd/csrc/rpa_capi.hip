@@ -709,8 +709,32 @@ int rpa_decode(const RpaParams* p, void* stream) {
   return rc != RPA_OK ? rc : decode_rows(p, nullptr, nullptr, false, stream);
 }
 
+static rpa::KvWriteArgs kv_write_args(const RpaParams* p, const void* keys, const void* values) {
+  rpa::KvWriteArgs a = {};
+  a.kv = kv_addr(p);
+  a.pt = page_table(p);
+  a.keys = static_cast<const char*>(keys);
+  a.values = static_cast<const char*>(values);
+  a.num_seqs = p->num_seqs;
+  a.dist = p->distribution;
+  a.Hkv = p->num_kv_heads;
+  a.head_bytes = p->head_dim * esize_of(p->kv_dtype);
+  a.src_head_bytes = q_dim_of(p) * esize_of(p->kv_dtype);
+  a.num_tokens = p->num_tokens;
+  return a;
+}
+
+// Whether a call's chunks are prompts whose keys and values, every token of them, the caller brings along: the kernels
+// then read those rows and not the cache (whatever its pages are like), and write the cache beside the attention.
+static bool takes_fresh_prompts(const RpaParams* p) {
+  return p->prompts_only && !p->distribution && p->decode_end == 0 && p->mask_mode != RPA_MASK_CUSTOM && q_dim_of(p) == p->head_dim &&
+         p->num_seqs > 0 && p->num_tokens > 0 && !(p->head_dim == 256 && rpa::tuning().prefill_rows256 != 0) &&
+         (int64_t)p->num_tokens * p->num_kv_heads * p->head_dim * esize_of(p->kv_dtype) < (int64_t(1) << 31);
+}
+
 // The prefill kernels' view of a call; false when the call has no chunk for them.
-static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a) {
+// fresh: a prompt's keys / values, which the kernels read in place of the cache (takes_fresh_prompts).
+static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a, const void* keys = nullptr, const void* values = nullptr) {
   const bool dyn = p->distribution != nullptr;
   if (!dyn && p->num_seqs <= p->decode_end && p->mask_mode != RPA_MASK_CUSTOM) return false;
   if (dyn && p->num_seqs <= 0) return false;
@@ -738,6 +762,22 @@ static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a) {
   a.ws_ml = nullptr;
   a.mask_bits = nullptr;
   a.mask_pitch = 0;
+  a.rows_are_new = 0;
+  a.write_blocks = a.write_tokens = 0;
+  a.write = {};
+  if (takes_fresh_prompts(p)) {
+    a.write = kv_write_args(p, keys, values);
+    // two tokens per wave on a small launch, where the attention's own workgroups leave CUs idle
+    a.write_tokens = p->num_tokens <= 2048 ? 8 : 32;
+    a.write_blocks = (p->num_tokens + a.write_tokens - 1) / a.write_tokens;
+    a.rows_are_new = 1;
+    a.kv.k_base = static_cast<const char*>(keys);
+    a.kv.v_base = static_cast<const char*>(values);
+    a.kv.head_stride = p->head_dim * esize_of(p->kv_dtype);
+    a.kv.tok_stride = p->num_kv_heads * a.kv.head_stride;
+    a.kv.page_stride = 0;  // (the id of the one page, whatever the table holds, adds nothing)
+    a.pt.page_size = 1 << 30;
+  }
   return true;
 }
 
@@ -771,11 +811,11 @@ static size_t prefill_optional_workspace(const RpaParams* p) {
   return prefill_workspace(p, a).total;
 }
 
-int rpa_prefill(const RpaParams* p, void* stream) {
+static int prefill_run(const RpaParams* p, const void* keys, const void* values, void* stream) {
   int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
   rpa::PrefillArgs a;
-  if (!prefill_args(p, a)) return RPA_OK;
+  if (!prefill_args(p, a, keys, values)) return RPA_OK;
   // 256-wide heads take the flash kernel (two 128-dim halves per row, one workgroup per CU; e4m3
   // caches staged through registers); RPA_PREFILL_ROWS256=1 sends them through the row kernel
   if (p->head_dim == 256 && rpa::tuning().prefill_rows256 != 0)
@@ -817,6 +857,13 @@ int rpa_upload_words(int32_t* dst, const int32_t* src, int32_t n, void* stream) 
   return check_hip(rpa::launch_upload(dst, src, n, static_cast<hipStream_t>(stream)), "rpa_upload_words");
 }
 
+int rpa_prefill(const RpaParams* p, void* stream) {
+  if (!p || !p->prompts_only) return prefill_run(p, nullptr, nullptr, stream);
+  RpaParams q = *p;  // the new tokens are in the cache already
+  q.prompts_only = 0;
+  return prefill_run(&q, nullptr, nullptr, stream);
+}
+
 int rpa_mask_needs_starts(const RpaParams* p) { return p && p->mask_mode == RPA_MASK_CUSTOM && !mask_as_bits(p) ? 1 : 0; }
 
 // (narrow heads: only the kernels that know of the zeros behind 64 dims)
@@ -835,17 +882,7 @@ static bool decode_takes_new_tokens(const RpaParams* p_in) {
 }
 
 static int write_new_tokens(const RpaParams* p, const void* keys, const void* values, bool skip_decode_rows, void* stream) {
-  rpa::KvWriteArgs a;
-  a.kv = kv_addr(p);
-  a.pt = page_table(p);
-  a.keys = static_cast<const char*>(keys);
-  a.values = static_cast<const char*>(values);
-  a.num_seqs = p->num_seqs;
-  a.dist = p->distribution;
-  a.Hkv = p->num_kv_heads;
-  a.head_bytes = p->head_dim * esize_of(p->kv_dtype);
-  a.src_head_bytes = q_dim_of(p) * esize_of(p->kv_dtype);
-  a.num_tokens = p->num_tokens;
+  rpa::KvWriteArgs a = kv_write_args(p, keys, values);
   a.skip_decode_rows = skip_decode_rows ? 1 : 0;
   a.seq_begin = skip_decode_rows && !p->distribution ? p->decode_end : 0;
   return check_hip(rpa::launch_kv_write(a, static_cast<hipStream_t>(stream)), "rpa_kv_write");
@@ -860,6 +897,7 @@ int rpa_attention_update(const RpaParams* p, const void* keys, const void* value
     if (keys && !with_rows && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
     return decode_rows(p, with_rows ? keys : nullptr, with_rows ? values : nullptr, true, stream);
   }
+  if (keys && takes_fresh_prompts(p)) return prefill_run(p, keys, values, stream);
   const bool fused = keys && decode_takes_new_tokens(p);
   if (keys && !fused && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
   if ((rc = decode_rows(p, fused ? keys : nullptr, fused ? values : nullptr, false, stream)) != RPA_OK) return rc;

@@ -85,6 +85,24 @@ struct DecodeArgs {
   int32_t num_seqs;      // token_rows: sequences (with dist: a bound on dist[2])
 };
 
+// New tokens on their way into the cache.
+struct KvWriteArgs {
+  KvAddr kv;  // bases are written through
+  PageTable pt;
+  const char* keys;    // [T, Hkv, D] cache dtype
+  const char* values;
+  int32_t num_seqs;
+  int32_t Hkv;
+  int32_t head_bytes;
+  int32_t src_head_bytes;  // of a head in keys / values (<= head_bytes; the rest of the cached row is set to zero)
+  int32_t num_tokens;
+  const int32_t* dist;  // device i32[3] or nullptr: when given, num_seqs is only a bound on dist[2]
+  // decode rows whose tokens the decode kernel writes itself are left out: sequences [0, seq_begin), with dist
+  // (skip_decode_rows) sequences [0, dist[0])
+  int32_t seq_begin;
+  int32_t skip_decode_rows;
+};
+
 struct PrefillArgs {
   const uint16_t* q;
   uint16_t* out;
@@ -114,6 +132,11 @@ struct PrefillArgs {
   // rpa_mask_bits_kernel in front of the attention kernels; nullptr: the kernels read the caller's i32 words
   uint64_t* mask_bits;
   int32_t mask_pitch;
+  // Prompts without a prefix: kv addresses the caller's new rows (a sequence's start at its first query token, one huge
+  // page), and the last write_blocks workgroups of the grid put them into the cache, write_tokens each.
+  int32_t rows_are_new;
+  int32_t write_blocks, write_tokens;
+  KvWriteArgs write;
 };
 
 struct GatherArgs {
@@ -126,23 +149,6 @@ struct GatherArgs {
   void* k_out;
   void* v_out;
   int32_t max_tokens;
-};
-
-struct KvWriteArgs {
-  KvAddr kv;  // bases are written through
-  PageTable pt;
-  const char* keys;    // [T, Hkv, D] cache dtype
-  const char* values;
-  int32_t num_seqs;
-  int32_t Hkv;
-  int32_t head_bytes;
-  int32_t src_head_bytes;  // of a head in keys / values (<= head_bytes; the rest of the cached row is set to zero)
-  int32_t num_tokens;
-  const int32_t* dist;  // device i32[3] or nullptr: when given, num_seqs is only a bound on dist[2]
-  // decode rows whose tokens the decode kernel writes itself are left out: sequences [0, seq_begin), with dist
-  // (skip_decode_rows) sequences [0, dist[0])
-  int32_t seq_begin;
-  int32_t skip_decode_rows;
 };
 
 struct MlaDecodeArgs {

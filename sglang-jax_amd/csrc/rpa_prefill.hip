@@ -43,6 +43,7 @@ namespace {
 // such chunks then fill their tiles, and the four waves still share every K/V tile.
 template <bool UNIFORM, bool CAP, bool EXT, bool HEADS4 = false>
 __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const PrefillArgs a_in, int tiles, int nseq, bool by_level) {
+  if (writes_new_tokens(a_in)) return;
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
@@ -69,8 +70,8 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
   if constexpr (HEADS4) w.head += wave;  // this wave's head
   const int c = lane & 31, h = lane >> 5;
   const TileSrc src = make_src(a, w);
-  const char* kh = a.kv.k_base + (int64_t)w.hk * a.kv.head_stride;
-  const char* vh = a.kv.v_base + (int64_t)w.hk * a.kv.head_stride;
+  const char* kh = head_rows(a, w, a.kv.k_base);
+  const char* vh = head_rows(a, w, a.kv.v_base);
 
   WaveRows wr;
   wr.r_lo = w.q_start + (HEADS4 ? 0 : wave * 32);
@@ -300,6 +301,7 @@ struct WideFeed {
 
 template <bool UNIFORM, bool CAP, bool EXT, bool FP8>
 __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillArgs a_in, int tiles, int nseq, bool by_level) {
+  if (writes_new_tokens(a_in)) return;
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
@@ -315,8 +317,8 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillA
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   const TileSrc src = make_src(a, w);
-  const char* kh = a.kv.k_base + (int64_t)w.hk * a.kv.head_stride;
-  const char* vh = a.kv.v_base + (int64_t)w.hk * a.kv.head_stride;
+  const char* kh = head_rows(a, w, a.kv.k_base);
+  const char* vh = head_rows(a, w, a.kv.v_base);
 
   // this wave's positions: [r_lo, r_hi] of the chunk, lane column c = position r_lo + c
   const int r_lo = w.q_start + wave * 16, r_hi = min(r_lo + 15, w.q_len - 1);
@@ -703,6 +705,7 @@ __device__ __forceinline__ void tile_lstore(const Stage<FP8>& st, char* lds_k, c
 
 template <bool FP8, bool UNIFORM, bool CAP, bool EXT, bool HEADS4 = false>
 __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const PrefillArgs a_in, int tiles, int nseq, bool by_level) {
+  if (writes_new_tokens(a_in)) return;
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
@@ -719,8 +722,8 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const Prefil
   if constexpr (HEADS4) w.head += wave;
   const int c = lane & 31, h = lane >> 5;
   const TileSrc src = make_src(a, w);
-  const char* kh = a.kv.k_base + (int64_t)w.hk * a.kv.head_stride;
-  const char* vh = a.kv.v_base + (int64_t)w.hk * a.kv.head_stride;
+  const char* kh = head_rows(a, w, a.kv.k_base);
+  const char* vh = head_rows(a, w, a.kv.v_base);
 
   WaveRows wr;
   wr.r_lo = w.q_start + (HEADS4 ? 0 : wave * 32);
@@ -936,7 +939,7 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
   if (by_level) tiles = levels;
   const int64_t units = (int64_t)nseq * a.Hkv;
   const int64_t grid = (units >= 8 ? ((units + 7) / 8) * 8 : units) * (heads4 ? a.G / 4 : a.G) * tiles;
-  if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+  if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   const bool uniform = (a.pt.page_size % kBN) == 0;
   // soft cap and logit rounding share the general score path
   const bool cap = a.sm.soft_cap != 0.f || a.sm.round_logits != 0;
@@ -947,7 +950,7 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
   }
   const bool cut = a.kv_splits > 1;  // pieces of the K/V ranges on the second grid dimension, then the merge
   if (cut && (!a.ws_o || !a.ws_ml || a.kv_splits > 64)) return hipErrorInvalidValue;
-  const dim3 g((unsigned)grid, cut ? (unsigned)a.kv_splits : 1u), blk(256);
+  const dim3 g((unsigned)(grid + a.write_blocks), cut ? (unsigned)a.kv_splits : 1u), blk(256);
   const bool ext = a.sm.xai_len > 0.f || a.sm.mask_mode != 0 || a.sm.q_scale > 0.f;
 #define RPA_STAGED(F, U, C, E) \
   hipLaunchKernelGGL((rpa_prefill_staged_kernel<F, U, C, E>), g, blk, 0, stream, a, tiles, nseq, by_level)

@@ -296,6 +296,7 @@ template <bool WIN, int NQ, bool HEADS4 = false, bool SPLIT = false>
 __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kernel(const PrefillArgs a_in, int tiles, int nseq,
                                                                                  bool by_level, float row_sum_limit,
                                                                                  bool masked_steps) {
+  if (writes_new_tokens(a_in)) return;
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
@@ -313,8 +314,8 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
   if constexpr (HEADS4) w.head += wave;  // this wave's head
   const int c = lane & 31, h = lane >> 5;
   const TileSrc src = make_src(a, w);
-  const char* kh = a.kv.k_base + (int64_t)w.hk * a.kv.head_stride;
-  const char* vh = a.kv.v_base + (int64_t)w.hk * a.kv.head_stride;
+  const char* kh = head_rows(a, w, a.kv.k_base);
+  const char* vh = head_rows(a, w, a.kv.v_base);
   typedef __attribute__((address_space(3))) char* lds_ptr_t;
   const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)lds);
 
@@ -562,12 +563,12 @@ hipError_t launch_prefill_pipe(const PrefillArgs& a, int nseq, bool level_order,
   if (by_level) tiles = levels;
   const int64_t units = (int64_t)nseq * a.Hkv;
   const int64_t grid = (units >= 8 ? ((units + 7) / 8) * 8 : units) * (heads4 ? a.G / 4 : a.G) * tiles;
-  if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  const dim3 g((unsigned)grid), blk(256);
+  if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+  const dim3 g((unsigned)(grid + a.write_blocks)), blk(256);
   const bool win = a.sm.window > 0;
   if (a.kv_splits > 1 && nq == 1) {  // pieces of the K/V ranges, then the merge
     if (!a.ws_o || !a.ws_ml || a.kv_splits > 64) return hipErrorInvalidValue;
-    const dim3 gs((unsigned)grid, (unsigned)a.kv_splits);
+    const dim3 gs((unsigned)(grid + a.write_blocks), (unsigned)a.kv_splits);
 #define RPA_LAUNCH_SPLIT(W, H4) \
   hipLaunchKernelGGL((rpa_prefill_pipe_kernel<W, 1, H4, true>), gs, blk, 0, stream, a, tiles, nseq, by_level, limit, masked)
     if (heads4) {

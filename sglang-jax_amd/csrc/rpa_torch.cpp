@@ -162,13 +162,14 @@ int without_gil(F f) {
 
 // attention(q, k, v, cache, kv_lens, page_indices, cu_q_lens, cu_kv_lens, distribution, attention_sink, causal, sm_scale,
 //           sliding_window, soft_cap, mask_value, q_scale, k_scale, v_scale, xai_temperature_len, softmax_dtype,
-//           chunk_prefill_size, max_kv_len, max_q_len, num_splits, host_kv_lens, head_dim, custom_mask, mask_aligned)
+//           chunk_prefill_size, max_kv_len, max_q_len, num_splits, host_kv_lens, head_dim, custom_mask, mask_aligned,
+//           prompts_only)
 // -> output, a status below 0, or None.  head_dim 0: q, k, v are [T, heads, D]; else they may be [T, heads * D], and
 // so is the output.  custom_mask is read where causal is false.
 PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  if (nargs != 28) {
-    PyErr_SetString(PyExc_TypeError, "attention takes 28 arguments");
+  if (nargs != 29) {
+    PyErr_SetString(PyExc_TypeError, "attention takes 29 arguments");
     return nullptr;
   }
   const at::Tensor* q = tensor(a[0]);
@@ -308,6 +309,7 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   p.layout = RPA_LAYOUT_FUSED;
   p.kv_dtype = kv_type == at::kBFloat16 ? RPA_KV_BF16 : RPA_KV_FP8_E4M3;
   COMMON(!rpa_mask_needs_starts(&p));
+  p.prompts_only = keys.defined() && PyObject_IsTrue(a[28]) == 1;
   if (const size_t need = rpa_workspace_bytes(&p)) {
     at::Tensor& ws = workspace(dev, stream, need);
     p.workspace = ws.data_ptr();
@@ -496,7 +498,7 @@ PyObject* sparse_mla(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 
 // metadata(decode, seq_lens, cache_loc, extend_seq_lens, page_size, extend_is_mixed, device index)
 // -> (cu_q_lens, cu_kv_lens, page_indices, seq_lens, distribution on the device, distribution as a tuple, max_kv_len,
-// max_q_len, sum of visible lengths), or None: what build_forward_metadata works out for one data-parallel rank, in one
+// max_q_len, sum of visible lengths, whether no sequence has a prefix), or None: what build_forward_metadata works out for one data-parallel rank, in one
 // pass over the host arrays and one upload.
 PyObject* metadata(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -515,6 +517,7 @@ PyObject* metadata(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   const int64_t at_q = 0, at_kv = up4(S + 1), at_len = at_kv + up4(S + 1), at_dist = at_len + up4(S), at_page = at_dist + 4;
   const int64_t total = at_page + np;
   std::vector<int32_t> w((size_t)total);
+  bool no_prefix = !decode;
   int64_t cu_q = 0, cu_kv = 0, n = 0, max_kv = INT64_MIN, max_q = INT64_MIN;
   for (int64_t s = 0; s < S; ++s) {
     const int64_t kv = lens.at(s), q = decode ? 1 : ext.at(s);
@@ -526,6 +529,7 @@ PyObject* metadata(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     w[at_kv + s + 1] = (int32_t)cu_kv;
     w[at_len + s] = (int32_t)kv;
     n += kv > 0;
+    no_prefix = no_prefix && q == kv;
     max_kv = std::max(max_kv, kv);
     max_q = std::max(max_q, q);
   }
@@ -547,13 +551,14 @@ PyObject* metadata(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   const int rc = rpa_upload_words(base.data_ptr<int32_t>(), w.data(), (int32_t)total, stream_of(dev));
   COMMON(rc == RPA_OK);
   const int64_t from[5] = {at_q, at_kv, at_page, at_len, at_dist}, size[5] = {S + 1, S + 1, np, S, 3};
-  PyObject* out = PyTuple_New(9);
+  PyObject* out = PyTuple_New(10);
   if (!out) return nullptr;
   for (int i = 0; i < 5; ++i) PyTuple_SET_ITEM(out, i, THPVariable_Wrap(base.narrow(0, from[i], size[i])));
   PyTuple_SET_ITEM(out, 5, Py_BuildValue("(iii)", first, mid, (int)n));
   PyTuple_SET_ITEM(out, 6, PyLong_FromLongLong(max_kv));
   PyTuple_SET_ITEM(out, 7, PyLong_FromLongLong(max_q));
   PyTuple_SET_ITEM(out, 8, PyLong_FromLongLong(visible));
+  PyTuple_SET_ITEM(out, 9, PyBool_FromLong(no_prefix));
   return out;
   END_HANDLE_TH_ERRORS
 }

@@ -396,7 +396,7 @@ def ragged_paged_attention(
             queries, keys, values, kv_cache_fused, kv_lens, page_indices, cu_q_lens, cu_kv_lens, distribution,
             attention_sink, causal, sm_scale, sliding_window, soft_cap, mask_value, q_scale, k_scale, v_scale,
             xai_temperature_len, softmax_dtype, chunk_prefill_size, max_kv_len, max_q_len, num_splits, host_kv_lens, 0,
-            custom_mask, mask_aligned_to_cu_kv)
+            custom_mask, mask_aligned_to_cu_kv, False)
         if out is not None:
             if type(out) is int:
                 _lib.check(out)

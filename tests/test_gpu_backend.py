@@ -196,3 +196,38 @@ def test_metadata_in_one_upload(pkg, gpu, P, lens, mixed):
             assert got.dtype == torch.int32 and np.array_equal(got.cpu().numpy(), want[name]), name
         assert np.array_equal(md.host_distribution, want["distribution"])
         assert md.max_kv_len == kv.max() and md.max_q_len == (1 if ext is None else ext.max())
+
+
+@pytest.mark.parametrize("P,D,Hq,Hkv,dtype,window,cap", [
+    (64, 128, 8, 2, torch.bfloat16, None, None), (16, 128, 16, 4, torch.bfloat16, 100, None), (1, 128, 8, 4, torch.bfloat16, None, 30.0),
+    (24, 256, 8, 2, torch.bfloat16, None, None), (16, 128, 8, 1, torch.float8_e4m3fn, None, None),
+    (64, 256, 4, 2, torch.float8_e4m3fn, 64, 50.0)])
+@pytest.mark.parametrize("lens", [[1003], [130, 1, 70, 300, 64], [2500, 129]])
+def test_prompts_attend_to_the_rows_they_bring(pkg, gpu, P, D, Hq, Hkv, dtype, window, cap, lens):
+    """Prompts without a prefix read the caller's keys and values and fill the cache beside the attention; the functional
+    operator on the same batch writes first and reads the cache."""
+    gen = torch.Generator().manual_seed(3)
+    rng = np.random.default_rng(4)
+    kv = np.array(lens, dtype=np.int32)
+    n = int((-(-kv // P)).sum())
+    pages = rng.permutation(n + 2)[:n].astype(np.int32)
+    loc = (pages.astype(np.int64)[:, None] * P + np.arange(P)).reshape(-1).astype(np.int32)
+    T = int(kv.sum())
+    cache = torch.full((n + 2, P, 2 * Hkv, D), 3.0).to(dtype).to(gpu)
+    other = cache.clone()
+    q = torch.randn(T, Hq, D, generator=gen).to(torch.bfloat16).to(gpu)
+    k, v = (torch.randn(T, Hkv, D, generator=gen).to(dtype).to(gpu) for _ in range(2))
+    backend = pkg.FlashAttention(Hq, Hkv, D, page_size=P, device=gpu)
+    batch = SimpleNamespace(forward_mode=pkg.ForwardMode.EXTEND, seq_lens=kv, cache_loc=loc, extend_seq_lens=kv, dp_size=1,
+                            per_dp_bs_size=len(kv))
+    md = backend.forward_metadata = backend.get_forward_metadata(batch)
+    assert md.no_prefix
+    layer = SimpleNamespace(layer_id=0, scaling=D ** -0.5, head_dim=D, sliding_window_size=window, logit_cap=cap)
+    say(f"prompts P={P} D={D} {dtype} window={window} cap={cap} {lens}")
+    out, _ = backend(q.view(T, -1), k.view(T, -1), v.view(T, -1), layer, batch, SimpleNamespace(get_fused_kv_buffer=lambda i: cache))
+    want, _ = pkg.ragged_paged_attention(q, k, v, other, md.seq_lens, md.page_indices, md.cu_q_lens, md.cu_kv_lens, md.host_distribution,
+                                         sm_scale=D ** -0.5, sliding_window=window, soft_cap=cap, max_kv_len=md.max_kv_len,
+                                         max_q_len=md.max_q_len)
+    torch.cuda.synchronize()
+    assert torch.equal(cache.view(torch.uint8), other.view(torch.uint8))
+    assert_parity(out.view(T, Hq, D).cpu().float(), want.cpu().float(), **TOL)
