@@ -38,6 +38,7 @@ const Tuning& tuning() {
   geti("RPA_DECODE_BALANCED", t.decode_balanced);
   geti("RPA_DECODE_WAVES_PER_WG", t.decode_waves_per_wg);
   geti("RPA_DECODE_WAVE_CAPACITY", t.decode_wave_capacity);
+  geti("RPA_DECODE_ROW_KB", t.decode_row_kb);
   geti("RPA_DECODE_MERGE_IN_KERNEL", t.decode_merge_in_kernel);
   geti("RPA_DECODE_LDS_KB", t.decode_lds_kb);
   geti("RPA_MASK_BITS", t.mask_bits);
@@ -230,8 +231,30 @@ SplitPlan decode_plan(const RpaParams* p) {
   const int64_t units = (int64_t)p->decode_end * per_row;
   int64_t work = p->sum_decode_kv_len > 0 ? p->sum_decode_kv_len * per_row : 0;
   if (p->sliding_window > 0) work = 0;  // visible lengths are not the raw lengths
-  return plan_splits(bound, p->sliding_window, units, work, p->num_splits,
-                     rpa::tuning().decode_min_chunk, decode_wave_capacity(p));
+  SplitPlan sp = plan_splits(bound, p->sliding_window, units, work, p->num_splits,
+                             rpa::tuning().decode_min_chunk, decode_wave_capacity(p));
+  // Short pieces of small batches: 128 or 256 tokens where that gives all pieces, counted by the longest row, a wave slot at
+  // once, at two waves per CU for bf16 (a workgroup that finds its row ended still takes its turn at the dispatcher), or
+  // where a row's partials outgrow the merge.  4 rows of 1000..4095 tokens x 8 heads 22.8 us at 64, 16.9 at 128, 14.6 at
+  // 256; e4m3 8 rows of 500..2047 17.8 / 13.1 / 13.8; one row of 16000 x 1 head 21.3 -> 15.1.  From about 160 tokens on
+  // the pieces fill the chip and longer ones lose; bf16 on pages under a block, whose tokens cost more, gains by the merge only.
+  if (p->num_splits > 0 || sp.splits <= 1 || sp.chunk > 128) return sp;
+  int64_t eff = std::max<int64_t>(bound, 1);
+  if (p->sliding_window > 0) eff = std::min(eff, (int64_t)p->sliding_window + 31);
+  const bool fp8 = p->kv_dtype == RPA_KV_FP8_E4M3, small_pages = p->page_size % 32 != 0;
+  const int64_t slots = decode_wave_capacity(p), most = fp8 || small_pages ? slots : slots / 2;
+  auto splits = [&](int chunk) { return (eff + chunk - 1) / chunk; };
+  auto crowded = [&](int chunk) {
+    return splits(chunk) * units > slots * 3 / 4 && (fp8 ? chunk < 128 : !small_pages);
+  };
+  int chunk = 64;
+  while (chunk < sp.chunk) chunk *= 2;
+  while (chunk < 256 && (splits(chunk) > 64 || crowded(chunk))) chunk *= 2;
+  if (chunk > sp.chunk && splits(chunk) * units <= most && (!small_pages || fp8 || splits(sp.chunk) > 64)) {
+    sp.chunk = chunk;
+    sp.splits = (int)splits(chunk);
+  }
+  return sp;
 }
 
 // Balanced decode plan: a fixed number of waves (every wave slot of the GPU once) share the
@@ -287,6 +310,20 @@ bool use_balanced(const RpaParams* p, const SplitPlan& fixed) {
   // the window most rows are clipped and the batch is as good as uniform
   if (p->sliding_window > 0 && p->sum_decode_kv_len >= (int64_t)p->decode_end * p->sliding_window) return false;
   return true;
+}
+
+// Whether rpa_decode_row_kernel takes the rows: what a workgroup cannot read in the time that a merge pass costs loses (a CU
+// draws about 39 bytes per ns), and a second round of them does.  Up to 255 tokens or a window of 224 in bf16, twice that in
+// e4m3: 10.2 -> 7.5 us for a few rows (the second launch is the host's time too), 64 rows of 64..255 x 4 heads 15.7 -> 12.1;
+// 511 tokens: 9.8 against 11.0.
+bool rows_in_one_workgroup(const RpaParams* p, const SplitPlan& fixed) {
+  if (fixed.splits <= 1 || p->num_splits > 0) return false;
+  int64_t longest = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages, p->cu_kv_lens != nullptr);
+  if (p->sliding_window > 0) longest = std::min(longest, (int64_t)p->sliding_window + 31);
+  const int64_t bytes = longest * 2 * (q_dim_of(p) == 64 && p->kv_dtype == RPA_KV_BF16 ? 64 : p->head_dim) * esize_of(p->kv_dtype);
+  const int64_t units = (int64_t)p->decode_end * p->num_kv_heads * ((p->num_q_heads / p->num_kv_heads + 15) / 16);
+  const int kb = rpa::tuning().decode_row_kb >= 0 ? rpa::tuning().decode_row_kb : 128;
+  return bytes <= ((int64_t)kb << 10) && units <= wave_capacity() / 8;
 }
 
 // Bytes of KV the decode rows will read, as far as the host knows (its sum of lengths, or rows
@@ -576,7 +613,7 @@ static size_t required_workspace_bytes(const RpaParams* p_in) {
   const SplitPlan sp = decode_plan(p);
   if (use_balanced(p, sp))
     return balanced_layout(p).total;
-  if (sp.splits <= 1) return 0;
+  if (sp.splits <= 1 || rows_in_one_workgroup(p, sp)) return 0;
   return (size_t)p->decode_end * sp.splits * p->num_q_heads * (p->head_dim + 2) * sizeof(float);
 }
 
@@ -627,7 +664,7 @@ static bool takes_token_rows(const RpaParams* p) {
 static size_t token_row_workspace(const RpaParams* p) {
   const RpaParams v = token_row_view(p);
   const SplitPlan sp = decode_plan(&v);
-  return sp.splits <= 1 ? 0 : (size_t)v.decode_end * sp.splits * v.num_q_heads * (v.head_dim + 2) * sizeof(float);
+  return sp.splits <= 1 || rows_in_one_workgroup(&v, sp) ? 0 : (size_t)v.decode_end * sp.splits * v.num_q_heads * (v.head_dim + 2) * sizeof(float);
 }
 
 // Decode rows; with keys / values the rows' own tokens are not in the cache yet and are written by these kernels.
@@ -667,6 +704,7 @@ static int decode_rows(const RpaParams* p_in, const void* keys, const void* valu
   a.dist = p->distribution;
   a.balanced = (!token_rows && use_balanced(p, sp)) ? 1 : 0;
   a.num_wgs = decode_wgs(p);
+  a.whole_rows = (!a.balanced && rows_in_one_workgroup(p, sp)) ? 1 : 0;
   a.waves_per_wg = a.balanced ? decode_waves_per_wg(p) : decode_fixed_waves(p);
   a.min_blocks_per_wave = std::max(1, rpa::tuning().decode_min_chunk / 32);
   a.forced_blocks_per_wave = 0;
@@ -694,7 +732,7 @@ static int decode_rows(const RpaParams* p_in, const void* keys, const void* valu
       // look like this call's
       a.generation = (g_decode_generation.fetch_add(1, std::memory_order_relaxed) % ((1ull << 48) - 1)) + 1;
     }
-  } else if (sp.splits > 1) {
+  } else if (sp.splits > 1 && !a.whole_rows) {
     const size_t need = token_rows ? token_row_workspace(p_in) : required_workspace_bytes(p);
     if (!p->workspace || p->workspace_bytes < need)
       return fail(RPA_EINVAL_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, p->workspace_bytes);
@@ -931,10 +969,12 @@ int rpa_describe_plan(const RpaParams* p_in, char* buf, size_t len) {
     } else {
       const SplitPlan sp = decode_plan(p);
       const bool bal = use_balanced(p, sp);
-      put("decode: shape=%s kernel=%s rows=%d waves_per_wg=%d", r.name,
+      if (!bal && rows_in_one_workgroup(p, sp))
+        put("decode: shape=%s kernel=rpa_decode_row_kernel rows=%d", r.name, p->decode_end);
+      else put("decode: shape=%s kernel=%s rows=%d waves_per_wg=%d", r.name,
           bal ? "rpa_decode_balanced_kernel" : "rpa_decode_splitkv_kernel", p->decode_end, bal ? decode_waves_per_wg(p) : decode_fixed_waves(p));
       if (bal) put(" resident_waves=%d merge=rpa_combine_balanced_kernel", decode_wave_capacity(p));
-      else put(" pieces_per_row=%d chunk=%d merge=%s", sp.splits, sp.chunk, sp.splits > 1 ? "rpa_combine_kernel" : "none");
+      else if (!rows_in_one_workgroup(p, sp)) put(" pieces_per_row=%d chunk=%d merge=%s", sp.splits, sp.chunk, sp.splits > 1 ? "rpa_combine_kernel" : "none");
     }
     put(" workspace=%zu\n", required_workspace_bytes(p_in));
   }

@@ -45,6 +45,8 @@ namespace rpa {
 namespace {
 
 constexpr int kBlk = 32;
+constexpr int kRowWaves = 8;    // rpa_decode_row_kernel: waves of a workgroup
+constexpr int kRowPitch = 132;  // its partial rows in LDS: 128 floats and 16 bytes, so that neighbouring heads' banks differ
 
 __device__ __forceinline__ int tok_slot(int g, int i) {
   return (i < 4) ? (g * 4 + i) : (16 + g * 4 + (i - 4));
@@ -470,10 +472,11 @@ struct RowRef {
   int seq, tq, kv_len, fresh_first, fresh_tq;
 };
 
-// One wave, one (row, kv head, group of 16 query heads), tokens [t_begin, t_end).
-template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool HALF>
+// One wave, one (row, kv head, group of 16 query heads), tokens [t_begin, t_end): unnormalised output rows, maxima, sums.
+template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool HALF, int WAVES>
 __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef& row, int hk, int rg, int t_lo,
-                                               int t_begin, int t_end, const PartDest dest, int lane) {
+                                               int t_begin, int t_end, f32x4_t (&acc)[MT][8], float (&m)[MT], float (&l)[MT],
+                                               int lane) {
   const int kv_len = row.kv_len;
   const int seq = __builtin_amdgcn_readfirstlane(row.seq);
   const int c = lane & 15, g = lane >> 4;
@@ -515,8 +518,6 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
   so.t_lo = t_lo;
   so.kv_len = kv_len;
 
-  f32x4_t acc[MT][8];
-  float m[MT], l[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     m[mt] = -INFINITY;
@@ -540,7 +541,7 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
   // trip in front of every block's loads, behind which the loads already in flight had to drain (page size
   // 16: 2.6 TB/s where pages of 64 stream 5.8).  The window moves on every kWinSmallPages pages, at the
   // price of one drained queue.
-  __shared__ int32_t seg_windows[UNIFORM_PAGE ? 1 : 4][UNIFORM_PAGE ? 1 : kWinSmallPages];  // [wave][entry]
+  __shared__ int32_t seg_windows[UNIFORM_PAGE ? 1 : WAVES][UNIFORM_PAGE ? 1 : kWinSmallPages];  // [wave][entry]
   const int32_t* win = nullptr;
   int win_first = 0;
   auto cover = [&](int tb) __attribute__((always_inline)) {  // make the window hold the pages of block tb
@@ -579,8 +580,6 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
     leave_new_token(rb, t_begin + (blk + 1) * kBlk);
     compute_block<MT, FP8, CAP, HALF>(rb, qB, acc, m, l, so, t_begin + (blk + 1) * kBlk, g);
   }
-
-  write_rows<MT>(a, acc, m, l, tq, hk, row0, dest, c, g);
 }
 
 __device__ __forceinline__ int owner_of_token(const int32_t* cu_q_lens, int num_seqs, int tok) {
@@ -641,7 +640,77 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_splitkv_kernel(const Decode
   dest.final_rows = a.max_splits == 1;
   dest.by_head = true;
   dest.base = ((int64_t)index * a.max_splits + split) * a.Hq;
-  decode_segment<MT, FP8, UNIFORM_PAGE, CAP, HALF>(a, row, hk, rg, t_lo, t_begin, t_end, dest, lane);
+  f32x4_t acc[MT][8];
+  float m[MT], l[MT];
+  decode_segment<MT, FP8, UNIFORM_PAGE, CAP, HALF, 4>(a, row, hk, rg, t_lo, t_begin, t_end, acc, m, l, lane);
+  write_rows<MT>(a, acc, m, l, row.tq, hk, rg * 16 * MT, dest, lane & 15, lane >> 4);
+}
+
+// ---- short rows: grid = (rows, 1, kv heads * row groups); one workgroup of kRowWaves waves deals a row's blocks out among
+// them and merges their partial rows in LDS.  Bound by latency: the split kernel and its merge are two launches, each about
+// 4 us from its start to its first useful load; here the merge is two barriers and 8 KB of LDS per 2 query heads.  8 waves:
+// the registers allow two per SIMD, and a row of 255 tokens is then one 32-token block each.  A few rows of up to 255
+// tokens: 10.2 -> 7.5 us.
+template <bool FP8, bool UNIFORM_PAGE, bool CAP, bool HALF = false>
+__global__ __launch_bounds__(kRowWaves * 64, 2) void rpa_decode_row_kernel(const DecodeArgs a) {
+  extern __shared__ float row_parts[];  // [wave][query head of the group][kRowPitch]
+  __shared__ float row_ml[kRowWaves][16][2];
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hk = (int)blockIdx.z % a.Hkv, rg = (int)blockIdx.z / a.Hkv;
+  RowRef row;
+  if (!fixed_row(a, (int)blockIdx.x, row)) return;
+  const int t_lo = (a.sm.window > 0) ? max(0, row.kv_len - a.sm.window) : 0;
+  const int t0 = t_lo & ~(kBlk - 1);
+  const int piece = ((row.kv_len - t0 + kBlk - 1) / kBlk + kRowWaves - 1) / kRowWaves * kBlk;
+  const int used = (row.kv_len - t0 + piece - 1) / piece;  // waves with work
+  const int heads = min(16, a.G - rg * 16);
+  f32x4_t acc[1][8];
+  float m[1], l[1];
+  if (wave < used) {
+    const int t_begin = t0 + wave * piece;
+    decode_segment<1, FP8, UNIFORM_PAGE, CAP, HALF, kRowWaves>(a, row, hk, rg, t_lo, t_begin, min(row.kv_len, t_begin + piece),
+                                                               acc, m, l, lane);
+    float lt = l[0];
+    lt += __shfl_xor(lt, 16);
+    lt += __shfl_xor(lt, 32);
+    if (g == 0) {
+      row_ml[wave][c][0] = m[0];
+      row_ml[wave][c][1] = lt;
+    }
+  }
+  __syncthreads();
+  if (wave < used && c < heads) {
+    float top = row_ml[0][c][0];
+    for (int w = 1; w < used; ++w) top = fmaxf(top, row_ml[w][c][0]);
+    const float share = fast_exp2(m[0] - top);
+    float* to = row_parts + (wave * heads + c) * kRowPitch + g * 32;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      *reinterpret_cast<f32x4_t*>(to + r * 8) =
+          f32x4_t{acc[0][0][r], acc[0][1][r], acc[0][2][r], acc[0][3][r]} * share;
+      *reinterpret_cast<f32x4_t*>(to + r * 8 + 4) =
+          f32x4_t{acc[0][4][r], acc[0][5][r], acc[0][6][r], acc[0][7][r]} * share;
+    }
+  }
+  __syncthreads();
+  const float vs = a.v_scale ? a.v_scale[hk] : 1.0f;
+  for (int at = (int)threadIdx.x; at < heads * 64; at += kRowWaves * 64) {
+    const int h = at >> 6, d = (at & 63) * 2;  // two dims of one query head
+    const int head = hk * a.G + rg * 16 + h;
+    float top = row_ml[0][h][0];
+    for (int w = 1; w < used; ++w) top = fmaxf(top, row_ml[w][h][0]);
+    float den = 0.f, x = 0.f, y = 0.f;
+    for (int w = 0; w < used; ++w) {
+      den += row_ml[w][h][1] * fast_exp2(row_ml[w][h][0] - top);
+      const float* from = row_parts + (w * heads + h) * kRowPitch + d;
+      x += from[0];
+      y += from[1];
+    }
+    const float inv = a.sm.sink ? vs * sink_inverse(top, den, sink_logit(a.sm.sink, a.sm.round_logits, head)) : vs / den;
+    if (d < a.q_dim)
+      *reinterpret_cast<uint32_t*>(a.out + ((int64_t)row.tq * a.Hq + head) * a.q_dim + d) = pack_bf16x2(x * inv, y * inv);
+  }
 }
 
 // ---- balanced plan ------------------------------------------------------------------------
@@ -1584,6 +1653,18 @@ void launch_decode_variant(const DecodeArgs& a, dim3 grid, dim3 block, hipStream
   const bool one_round = (int64_t)grid.x * grid.z * (block.x / 64) <= 2048;
   const int forced = tuning().decode_lds_kb;
   const unsigned lds = forced >= 0 ? (unsigned)forced << 10 : !one_round ? 0u : block.x >= 256 ? 84u << 10 : block.x >= 128 ? 54u << 10 : 34u << 10;
+  if (a.whole_rows) {
+    // (one workgroup per CU, too)
+    const unsigned parts = std::max(84u << 10, (unsigned)(kRowWaves * min(a.G, 16) * kRowPitch * sizeof(float)));
+    if constexpr (!FP8) {
+      if (a.q_dim == 64) {
+        hipLaunchKernelGGL((rpa_decode_row_kernel<false, UNIFORM, CAP, true>), grid, block, parts, st, a);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((rpa_decode_row_kernel<FP8, UNIFORM, CAP>), grid, block, parts, st, a);
+    return;
+  }
   // heads of 64 dims (rows of 128, the second half zero): half the bytes.  (Not with the opt-in merge inside the kernel.)
   if constexpr (!FP8) {
     if (a.q_dim == 64 && !(a.balanced && a.merge_counters)) {
@@ -1632,6 +1713,8 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
       hipLaunchKernelGGL(rpa_combine_balanced_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(64), 0, stream, a);
     return hipGetLastError();
   }
+  if (a.whole_rows)
+    return launch_decode_mt(a, dim3((unsigned)a.num_rows, 1, (unsigned)(a.Hkv * row_groups)), dim3(kRowWaves * 64), uniform, stream);
   if ((int64_t)a.max_splits * a.num_rows > 0x7fffffffLL || (int64_t)a.Hq * a.num_rows > 0x7fffffffLL)
     return hipErrorInvalidValue;
   dim3 grid((unsigned)max(a.max_splits, 1) * (unsigned)a.num_rows, 1, head_groups * row_groups);

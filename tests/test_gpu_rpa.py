@@ -1604,3 +1604,22 @@ def test_new_tokens_are_attended_to_and_left_in_the_cache(pkg, wl, gpu, case, fp
             page = int(b.page_indices[first + t // P])
             expect[page, t % P] = full[page, t % P]
     assert torch.equal(got, expect)  # every new slot written, nothing else touched
+
+
+@pytest.mark.parametrize("Hq,Hkv,P,kv_dtype,window", [
+    (16, 8, 64, torch.bfloat16, None), (40, 2, 16, torch.bfloat16, None), (12, 1, 24, torch.float8_e4m3fn, None),
+    (16, 2, 64, torch.float8_e4m3fn, 200), (8, 8, 128, torch.bfloat16, 65)])
+def test_short_rows_in_one_workgroup(pkg, wl, gpu, monkeypatch, Hq, Hkv, P, kv_dtype, window):
+    """Rows of up to 255 tokens (or a short window of longer ones) finish in one launch, their pieces merged in LDS: lengths
+    around a block and around the eight waves' share, against the oracle and against split rows, with a sink."""
+    lens = [1, 31, 32, 33, 96, 224, 255] if window is None else [1, 64, 65, 200, 4000, 231, 8]
+    b = wl.make_batch("short", [1] * len(lens), lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=311,
+                      kv_dtype=kv_dtype, sliding_window=window)
+    tol = BF16_TOL if kv_dtype == torch.bfloat16 else FP8_TOL
+    say(f"short rows {Hq}/{Hkv} P={P} {kv_dtype} window={window}")
+    assert_parity(gpu_out(pkg, b, gpu).float(), oracle_out(b).float(), **tol)
+    sink = torch.from_numpy(np.random.RandomState(5).randn(Hq).astype(np.float32))
+    got = gpu_out(pkg, b, gpu, attention_sink=sink)
+    assert_parity(got.float(), oracle_out(b, attention_sink=sink).float(), **tol)
+    monkeypatch.setenv("RPA_DECODE_ROW_KB", "0")
+    torch.testing.assert_close(gpu_out(pkg, b, gpu, attention_sink=sink).float(), got.float(), rtol=1e-2, atol=4e-3)
