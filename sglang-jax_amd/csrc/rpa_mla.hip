@@ -423,7 +423,8 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   // ---- pipeline: copies run three tiles ahead of the MFMAs (4-slot ring, 148 of the CU's 160 KiB:
   // 111 KiB per CU in flight, which is what HBM latency under load asks for) ----
   if constexpr (!UNIFORM) {
-    // every wave requests the ids for itself (the same bytes to the same place): no barrier in front of their use
+    // every wave requests the ids for itself (the same bytes to the same place): no barrier in front of their use.  (Nor in
+    // front of the requests: every wave has drained the last segment's, see the end of this function.)
 #pragma unroll
     for (int k = 0; k < 5; ++k) copy_tile_ids(src, t_begin + k * kTok, lane);
     wait_all_loads();
@@ -710,6 +711,10 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
     }
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);  // drain the copies issued past the end
+  // The ring of page ids is one for all waves: the next segment of this workgroup (another piece, another sequence)
+  // requests its first ids only when no wave has one of this segment's on its way, which would overwrite them behind the
+  // other waves' backs.  (The tiles need no such barrier: a wave's late copies land only where its own next ones follow.)
+  if constexpr (!UNIFORM) bare_barrier();
 
   // ---- epilogue: lane (c, g) holds head head0+c, dims 16j + 4g + r in acc[j][r] ----
   l += __shfl_xor(l, 16);

@@ -75,6 +75,30 @@ def test_mla_long_rows_on_pages_smaller_than_a_tile(pkg, wl, gpu, P, f8):
     assert_parity(run_gpu(pkg, b, gpu).float(), ref(b).float(), **TOL)
 
 
+@pytest.mark.parametrize("P,Hq,cap", [(1, 16, None), (8, 48, None), (16, 24, None), (16, 80, None), (16, 128, 30.0)])
+@pytest.mark.parametrize("f8", [False, True])
+def test_mla_rows_that_follow_each_other_in_a_workgroup_on_small_pages(pkg, wl, gpu, P, Hq, cap, f8):
+    """Pages under a tile, several pieces or sequences per workgroup: the ring of page ids in LDS is the whole
+    workgroup's, and a row's first ids may be requested only when no wave has one of the row before on its way.  Head
+    counts that leave waves without heads (they run ahead) among them; decode rows on the balanced plan, then one group of
+    query tokens over many short sequences.  Every launch gives the same bits."""
+    kw = dict(num_q_heads=Hq, lkv_dim=512, rope_dim=64, page_size=P, sm_scale=192 ** -0.5, soft_cap=cap,
+              kv_dtype=torch.float8_e4m3fn if f8 else torch.bfloat16)
+    ref = fp8_oracle if f8 else oracle
+    rng = np.random.default_rng(P + Hq)
+    rows = [int(x) for x in rng.integers(1, 450, size=300)]
+    q_lens = [int(x) for x in rng.integers(4, 8, size=40)]
+    chunks = [q + int(x) for q, x in zip(q_lens, rng.integers(0, 300, size=40))]
+    for name, ql, kl in (("rows", [1] * len(rows), rows), ("chunks", q_lens, chunks)):
+        say(f"mla small pages, rows in a row P={P} Hq={Hq} cap={cap} f8={f8} {name}")
+        b = wl.make_mla_batch("mla_in_a_row_" + name, ql, kl, seed=440 + P + Hq, **kw)
+        T = sum(ql)
+        first = run_gpu(pkg, b, gpu)[:T]
+        assert_parity(first.float(), ref(b)[:T].float(), **TOL)
+        for _ in range(6):
+            assert torch.equal(first, run_gpu(pkg, b, gpu)[:T])
+
+
 @pytest.mark.parametrize("Hq", [8, 16, 32, 48, 64])
 @pytest.mark.parametrize("f8", [False, True])
 def test_mla_waves_share_tiles_when_heads_are_few(pkg, wl, gpu, monkeypatch, Hq, f8):
