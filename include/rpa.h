@@ -122,8 +122,8 @@ typedef struct RpaParams {
   int32_t num_splits;         /* decode split-KV count per sequence; 0 => automatic */
   /* ---- options ---- */
   int32_t sliding_window;     /* 0 => off */
-  float sm_scale;             /* the pipelined prefill kernel (bf16 cache, 128-wide heads, causal, no option)
-                                 multiplies the bf16 queries by sm_scale * log2(e) and rounds them to bf16 once,
+  float sm_scale;             /* the pipelined prefill kernel (bf16 cache on pages of 2^k >= 64 tokens, 128-wide
+                                 heads, causal, no option) multiplies the bf16 queries by sm_scale * log2(e) and rounds them to bf16 once,
                                  where the reference scales the f32 scores (:149): element-wise inside the
                                  reference's rtol = atol = 2e-2, and at most 1.5e-2 of a row's norm on rows whose
                                  weight sits on one or two keys (1e-2 for every other path) */

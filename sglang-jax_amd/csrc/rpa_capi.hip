@@ -801,6 +801,7 @@ static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a, const void* ke
   a.mask_bits = nullptr;
   a.mask_pitch = 0;
   a.rows_are_new = 0;
+  a.page_options = rpa::page_options(p->page_size, a.kv.page_stride, 64);
   a.write_blocks = a.write_tokens = 0;
   a.write = {};
   if (takes_fresh_prompts(p)) {
@@ -814,7 +815,7 @@ static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a, const void* ke
     a.kv.head_stride = p->head_dim * esize_of(p->kv_dtype);
     a.kv.tok_stride = p->num_kv_heads * a.kv.head_stride;
     a.kv.page_stride = 0;  // (the id of the one page, whatever the table holds, adds nothing)
-    a.pt.page_size = 1 << 30;
+    a.pt.page_size = 1 << 30;  // (a.page_options stay the cache's)
   }
   return true;
 }

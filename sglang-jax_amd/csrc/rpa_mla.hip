@@ -1487,9 +1487,7 @@ ShapeKey mla_shape_key(const MlaDecodeArgs& a) {
   k.kv_bits = a.fp8 ? 8 : 16;
   k.head_dim = 576;
   k.heads = a.Hq;
-  k.options = (a.sm.soft_cap != 0.f ? kOptSoftCap : 0u) | ((P % kTok) != 0 ? kOptOddPages : 0u) |
-              ((P & (P - 1)) != 0 ? kOptNotPow2Pages : 0u) |
-              ((int64_t)a.row_stride * 2 * P >= (int64_t(1) << 32) ? kOptWidePages : 0u);
+  k.options = (a.sm.soft_cap != 0.f ? kOptSoftCap : 0u) | page_options(P, (int64_t)a.row_stride * 2 * P, kTok);
   return k;
 }
 

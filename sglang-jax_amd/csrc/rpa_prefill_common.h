@@ -385,7 +385,6 @@ __device__ __forceinline__ void write_rows(const PrefillArgs& a, const Work& w, 
 // = 32 | 128 and RPA_PREFILL_PIPE_NQ=2 decide the short-chunk question by hand.
 inline ShapeKey prefill_shape_key(const PrefillArgs& a) {
   const Tuning& tune = tuning();
-  const int P = a.pt.page_size;
   ShapeKey k = {};
   k.stage = kStagePrefill;
   k.kv_bits = a.fp8 ? 8 : 16;
@@ -396,9 +395,7 @@ inline ShapeKey prefill_shape_key(const PrefillArgs& a) {
   else if (tune.prefill_pipe_tile != 0 || tune.prefill_pipe_nq == 2) k.max_q_len = 0;
   k.options = ((a.sm.soft_cap != 0.f || a.sm.round_logits != 0) ? kOptSoftCap : 0u) |
               (a.sm.mask_mode != 0 ? kOptMaskOther : 0u) | (a.sm.xai_len > 0.f ? kOptTemperature : 0u) |
-              (a.sm.q_scale > 0.f ? kOptQScale : 0u) | ((P % kBN) != 0 ? kOptOddPages : 0u) |
-              ((P & (P - 1)) != 0 ? kOptNotPow2Pages : 0u) |
-              (a.kv.page_stride >= (int64_t(1) << 32) ? kOptWidePages : 0u);
+              (a.sm.q_scale > 0.f ? kOptQScale : 0u) | a.page_options;
   return k;
 }
 

@@ -73,6 +73,12 @@ struct ShapeRule {
   const char* why;         // the measurement behind the row
 };
 
+// The options that a cache's pages set: tokens of a page, its bytes, K/V tokens of the stage's tile.
+inline unsigned page_options(int page_size, int64_t page_bytes, int tile) {
+  return ((page_size % tile) != 0 ? kOptOddPages : 0u) | ((page_size & (page_size - 1)) != 0 ? kOptNotPow2Pages : 0u) |
+         (page_bytes >= (int64_t(1) << 32) ? kOptWidePages : 0u);
+}
+
 constexpr unsigned kOptAsmPages = kOptOddPages | kOptWidePages | kOptNotPow2Pages;
 constexpr unsigned kOptPlainOnly = kOptSoftCap | kOptMaskOther | kOptTemperature | kOptQScale | kOptAsmPages;
 

@@ -231,3 +231,55 @@ def test_prompts_attend_to_the_rows_they_bring(pkg, gpu, P, D, Hq, Hkv, dtype, w
     torch.cuda.synchronize()
     assert torch.equal(cache.view(torch.uint8), other.view(torch.uint8))
     assert_parity(out.view(T, Hq, D).cpu().float(), want.cpu().float(), **TOL)
+
+
+def attention64(q, k, v, lens, scale, window=None):
+    """Prompts without a prefix in 64 bits: [T, Hq, D] of q [T, Hq, D], k / v [T, Hkv, D]."""
+    q, k, v = q.cpu().double(), k.cpu().double(), v.cpu().double()
+    g = q.shape[1] // k.shape[1]
+    out, at = [], 0
+    for n in lens:
+        s = slice(at, at + n)
+        at += n
+        kk, vv = (x[s].repeat_interleave(g, dim=1).transpose(0, 1) for x in (k, v))
+        x = q[s].transpose(0, 1) @ kk.transpose(1, 2) * scale
+        row, col = torch.arange(n)[:, None], torch.arange(n)[None, :]
+        x = x.masked_fill((col > row) | (col <= row - (window or n + 1)), -torch.inf)
+        out.append((torch.softmax(x, dim=-1) @ vv).transpose(0, 1))
+    return torch.cat(out)
+
+
+# The 2-norm of the whole error over that of the result.  Scores scaled in 32 bits: probabilities and results rounded to
+# bf16 once (each up to 2^-8 of the value, 2^-8 / sqrt(12) / ~0.72 = 1.6e-3 on average over the mantissas): 2.2e-3 together
+# where few keys carry a row, less where many do.  Queries rounded to bf16 a second time (pages of 2^k >= 64 tokens: the
+# assembly kernel) move every logit by 1.6e-3 of its own terms, 2 units of spread here: 3.2e-3 more.
+@pytest.mark.parametrize("P,bound", [(1, 2.4e-3), (16, 2.4e-3), (24, 2.4e-3), (96, 2.4e-3), (64, 4.4e-3)])
+@pytest.mark.parametrize("lens", [[1003], [130, 1, 70, 300, 64]])
+def test_prompts_keep_the_precision_of_their_pages(pkg, gpu, P, bound, lens):
+    """What reads the caller's rows suits any pages, but a kernel that rounds more is not chosen for that: prompts on pages
+    that the assembly kernel does not take scale their scores in 32 bits, as the cache's rows do.  Against 64 bits, logits
+    of a few units, through the layer call and through the operator that reads the cache."""
+    gen = torch.Generator().manual_seed(11)
+    Hq, Hkv, D = 8, 2, 128
+    kv = np.array(lens, dtype=np.int32)
+    n = int((-(-kv // P)).sum())
+    pages = np.random.default_rng(4).permutation(n + 2)[:n].astype(np.int32)
+    loc = (pages.astype(np.int64)[:, None] * P + np.arange(P)).reshape(-1).astype(np.int32)
+    T = int(kv.sum())
+    cache = torch.zeros(n + 2, P, 2 * Hkv, D, dtype=torch.bfloat16, device=gpu)
+    q = (2 * torch.randn(T, Hq, D, generator=gen)).to(torch.bfloat16).to(gpu)
+    k, v = (torch.randn(T, Hkv, D, generator=gen).to(torch.bfloat16).to(gpu) for _ in range(2))
+    backend = pkg.FlashAttention(Hq, Hkv, D, page_size=P, device=gpu)
+    batch = SimpleNamespace(forward_mode=pkg.ForwardMode.EXTEND, seq_lens=kv, cache_loc=loc, extend_seq_lens=kv, dp_size=1,
+                            per_dp_bs_size=len(kv))
+    md = backend.forward_metadata = backend.get_forward_metadata(batch)
+    layer = SimpleNamespace(layer_id=0, scaling=D ** -0.5, head_dim=D, sliding_window_size=None, logit_cap=None)
+    say(f"prompt precision P={P} {lens}")
+    out, _ = backend(q.view(T, -1), k.view(T, -1), v.view(T, -1), layer, batch, SimpleNamespace(get_fused_kv_buffer=lambda i: cache))
+    old, _ = pkg.ragged_paged_attention(q, None, None, cache, md.seq_lens, md.page_indices, md.cu_q_lens, md.cu_kv_lens,
+                                        md.host_distribution, sm_scale=D ** -0.5, max_kv_len=md.max_kv_len, max_q_len=md.max_q_len)
+    want = attention64(q, k, v, lens, D ** -0.5)
+    for name, got in (("layer", out.view(T, Hq, D)), ("cache", old)):
+        err = float((got.cpu().double() - want).norm() / want.norm())
+        say(f"  {name} {err:.3e}")
+        assert err <= bound, (name, err)
