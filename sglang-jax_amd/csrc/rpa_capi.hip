@@ -1031,6 +1031,17 @@ int rpa_kv_write(const RpaParams* p, const void* keys, const void* values, void*
 
 static int mla_wgs();
 
+// The smallest piece of a row.  Partial rows are bf16, so a row that is cut is rounded once more than a whole one: batches of
+// rows up to 256 tokens are left whole (their result is 2.3e-3 from the 64-bit one, in pieces of 64 it was 2.8e-3).  That is
+// also the faster plan from 16 rows on (128 heads, rows of 100..255 tokens: 64 rows 36.0 -> 32.4 us, 200 rows 64.1 -> 36.5),
+// but not for a few (4 rows 25.3 -> 29.1; 16 heads 16.3 -> 20.6).
+constexpr int kMlaWholeRow = 256;
+static int mla_min_piece(const RpaMlaParams* p) {
+  int64_t longest = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages, p->cu_kv_lens != nullptr);
+  if (p->sliding_window > 0) longest = std::min(longest, (int64_t)p->sliding_window + 31);
+  return longest <= kMlaWholeRow ? kMlaWholeRow : std::max(1, rpa::tuning().mla_min_chunk);
+}
+
 static SplitPlan mla_plan(const RpaMlaParams* p, int64_t rows) {
   const int64_t bound = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages,
                                      p->cu_kv_lens != nullptr);
@@ -1041,7 +1052,7 @@ static SplitPlan mla_plan(const RpaMlaParams* p, int64_t rows) {
   int64_t work = p->sum_kv_len > 0 ? p->sum_kv_len * groups : 0;
   if (p->sliding_window > 0) work = 0;
   return plan_splits(bound, p->sliding_window, units, work, p->num_splits,
-                     rpa::tuning().mla_min_chunk, mla_wgs(), true);
+                     mla_min_piece(p), mla_wgs(), true);
 }
 
 static int mla_validate(const RpaMlaParams* p) {
@@ -1085,7 +1096,7 @@ static bool mla_use_balanced(const RpaMlaParams* p, const SplitPlan& fixed, bool
   const int64_t bound = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages,
                                      p->cu_kv_lens != nullptr);
   const int64_t units = (p->num_q_heads + 127) / 128;
-  const int64_t min_tiles = std::max(1, rpa::tuning().mla_min_chunk / 32);
+  const int64_t min_tiles = std::max(1, mla_min_piece(p) / 32);
   if ((int64_t)p->num_seqs * ((bound + 31) / 32) * units <= (int64_t)mla_wgs() * min_tiles) return false;
   const bool equal_lengths = p->sum_kv_len > 0 && p->max_kv_len > 0 &&
                              p->sum_kv_len == (int64_t)p->num_seqs * p->max_kv_len;
@@ -1149,7 +1160,7 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const c
   a.cu_tiles = nullptr;
   a.balanced = mla_use_balanced(p, sp, token_rows) ? 1 : 0;
   a.num_wgs = mla_wgs();
-  a.min_tiles_per_wg = std::max(1, rpa::tuning().mla_min_chunk / 32);
+  a.min_tiles_per_wg = std::max(1, mla_min_piece(p) / 32);
   a.forced_tiles_per_wg = 0;
   a.piece_pad = rpa::tuning().mla_piece_pad >= 0
                     ? rpa::tuning().mla_piece_pad

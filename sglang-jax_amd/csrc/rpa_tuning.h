@@ -30,7 +30,7 @@ struct Tuning {
   int prefill_pipe_masked = 1;      // RPA_PREFILL_PIPE_MASKED    0: the steps on the causal diagonal through compiled code
   int prefill_splits = -1;          // RPA_PREFILL_SPLITS         -1: cost model; 0 | 1 never; n forces n pieces
   // ---- absorbed MLA (rpa_mla.hip)
-  int mla_min_chunk = 64;           // RPA_MLA_MIN_CHUNK          smallest piece, tokens (3 rows of 1479 x 128 heads 38.7 us at 256, 28.7 at 64)
+  int mla_min_chunk = 64;           // RPA_MLA_MIN_CHUNK          smallest piece of a row of more than 256 tokens (3 rows of 1479 x 128 heads 38.7 us at 256, 28.7 at 64)
   int mla_wg_capacity = 0;          // RPA_MLA_WG_CAPACITY        0: one workgroup per CU
   int mla_balanced = 1;             // RPA_MLA_BALANCED
   int mla_piece_pad = -1;           // RPA_MLA_PIECE_PAD          -1: the shape table's; tiles a workgroup pays for starting another row

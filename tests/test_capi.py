@@ -412,6 +412,34 @@ def test_shape_table_environment_overrides(pkg, monkeypatch):
     assert "rpa_decode_balanced_kernel" in d(p)
 
 
+def _mla_params(pkg, Hq, P=64, fp8=False, S=64, T=64, max_kv=16384, sum_kv=590000, soft_cap=0.0, window=0):
+    p = pkg._lib.RpaMlaParams()
+    for f in ("ql_nope", "q_pe", "out", "cache_kv", "kv_lens", "page_indices", "cu_q_lens", "cu_kv_lens"):
+        setattr(p, f, 0x1000)
+    p.num_tokens, p.num_seqs, p.num_q_heads = T, S, Hq
+    p.lkv_dim, p.rope_dim, p.page_size, p.total_pages = 512, 64, P, 1 << 16
+    p.row_stride, p.rope_offset = 576, 512
+    p.max_kv_len, p.sum_kv_len, p.sm_scale, p.soft_cap, p.sliding_window = max_kv, sum_kv, 0.07, soft_cap, window
+    p.cache_dtype = pkg._lib.RPA_KV_FP8_E4M3 if fp8 else pkg._lib.RPA_KV_BF16
+    return p
+
+
+@pytest.mark.parametrize("S", [1, 4, 37, 64, 200, 256])
+@pytest.mark.parametrize("Hq,fp8", [(16, False), (64, False), (128, False), (128, True)])
+def test_mla_rows_of_up_to_256_tokens_are_left_whole(pkg, S, Hq, fp8):
+    """Partial rows are bf16: a row that fits one piece of 256 tokens is not cut, whatever idles (nor are a few rows that a
+    window clips to that); a longer one is."""
+    for longest, window, most, cut in ((64, 0, 256, False), (65, 0, 256, False), (256, 0, 256, False), (4000, 225, 4, False),
+                                       (2000, 0, 64, True)):
+        if S > most:
+            continue
+        seen = min(longest, window or longest)
+        for total in (S * seen, S * seen - S // 2, 0):
+            d = pkg._lib.describe_mla_plan(_mla_params(pkg, Hq, fp8=fp8, S=S, T=S, max_kv=longest, sum_kv=total, window=window), False)
+            whole = "plan=fixed pieces_per_row=1 " in d and " workspace=0" in d
+            assert whole != cut, (longest, window, total, d)
+
+
 def test_mla_shape_table_rows(pkg, monkeypatch):
     def params(Hq, P=64, fp8=False, S=64, T=64, max_kv=16384, sum_kv=590000, soft_cap=0.0):
         p = pkg._lib.RpaMlaParams()

@@ -99,6 +99,32 @@ def test_mla_rows_that_follow_each_other_in_a_workgroup_on_small_pages(pkg, wl, 
             assert torch.equal(first, run_gpu(pkg, b, gpu)[:T])
 
 
+def mla_attention64(b):
+    """Decode rows in 64 bits: [S, Hq, 512]."""
+    pages = torch.as_tensor(b.padded_page_indices()).reshape(len(b.meta["kv_lens"]), -1)
+    rows = b.cache_kv.double().reshape(-1, b.cache_kv.shape[-1])
+    out = []
+    for s, n in enumerate(b.meta["kv_lens"]):
+        t = torch.arange(n)
+        x = rows[pages[s][t // b.page_size].long() * b.page_size + t % b.page_size]
+        logits = torch.cat([b.ql_nope[s], b.q_pe[s]], dim=-1).double() @ x.T * b.sm_scale
+        out.append(torch.softmax(logits, dim=-1) @ x[:, :512])
+    return torch.stack(out)
+
+
+@pytest.mark.parametrize("Hq,S,longest", [(128, 64, 256), (128, 5, 200), (64, 40, 256), (16, 3, 90)])
+def test_mla_short_rows_are_rounded_once(pkg, wl, gpu, Hq, S, longest):
+    """Rows of up to 256 tokens are not cut: the 2-norm of the error is that of bf16 probabilities and of one rounding
+    of the result (2^-8 / sqrt(12) / ~0.72 = 1.6e-3 each, 2.3e-3 together; bf16 partial rows add another 1.6e-3: 2.8e-3)."""
+    lens = [longest] + [int(x) for x in np.random.default_rng(S).integers(65, longest + 1, size=S - 1)]
+    b = wl.make_mla_batch("mla_short", [1] * S, lens, num_q_heads=Hq, lkv_dim=512, rope_dim=64, page_size=64, seed=450 + S,
+                          sm_scale=192 ** -0.5)
+    want = mla_attention64(b)
+    err = float((run_gpu(pkg, b, gpu).double() - want).norm() / want.norm())
+    say(f"mla short rows Hq={Hq} S={S} up to {longest}: {err:.3e}")
+    assert err <= 2.4e-3
+
+
 @pytest.mark.parametrize("Hq", [8, 16, 32, 48, 64])
 @pytest.mark.parametrize("f8", [False, True])
 def test_mla_waves_share_tiles_when_heads_are_few(pkg, wl, gpu, monkeypatch, Hq, f8):
