@@ -434,23 +434,23 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillA
         p[b >> 1][(b & 1) * 2 + (r >> 1)] = x;
       }
   };
-  // the running max goes stale by up to 2^kMaxSlack before what was taken against it follows (see softmax_tile)
-  auto raise_max = [&](const f32x4_t (&S)[4]) __attribute__((always_inline)) {
+  // The running max goes stale by up to 2^kMaxSlack before what was taken against it follows (see softmax_tile).  The
+  // probabilities whose half of the second product is still to come are bf16 and stay what they are (multiplied here they
+  // would be rounded again, which l would not): O follows behind that product, when the caller multiplies it by the
+  // factor returned.
+  auto raise_max = [&](const f32x4_t (&S)[4]) __attribute__((always_inline)) -> float {
     float mx = fmaxf(S[0][0], S[0][1]);
 #pragma unroll
     for (int i = 2; i < 16; i += 2) mx = __builtin_fmaxf(__builtin_fmaxf(mx, S[i >> 2][i & 3]), S[i >> 2][(i & 3) + 1]);
     mx = swap_max(swap16_max(mx));
+    float alpha = 1.0f;
     if (__builtin_amdgcn_ballot_w64((mx - m) * sc2 > kMaxSlack) != 0) {
       const float m_new = fmaxf(m, mx);
-      const float alpha = fast_exp2((m - m_new) * sc2);
+      alpha = fast_exp2((m - m_new) * sc2);
       m = m_new;
       l *= alpha;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) O[j] *= alpha;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)  // the probabilities that wait for their half of the second product
-        pB[1][i] = pack_bf16x2(bf16_lo_to_f32(pB[1][i]) * alpha, bf16_hi_to_f32(pB[1][i]) * alpha);
     }
+    return alpha;
   };
   auto second_product = [&](int kk) __attribute__((always_inline)) {
 #pragma unroll
@@ -529,8 +529,7 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillA
         scores(S);
         cap_scores(S);
         mask_scores(S, t_lo);
-        pB[1] = u32x4_t{0u, 0u, 0u, 0u};
-        raise_max(S);
+        raise_max(S);  // (O is zero)
         probabilities(S, pB);
       }
       // (tiles that none of a wave's positions sees are not skipped: the other waves of the workgroup are at work on them)
@@ -544,10 +543,14 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillA
         cap_scores(S);
         second_product(0);
         mask_scores(S, tb + kBN);
-        raise_max(S);
+        const float alpha = raise_max(S);
         u32x4_t p_next[2];
         probabilities(S, p_next);
         second_product(1);
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+          for (int j = 0; j < 16; ++j) O[j] *= alpha;
+        }
         pB[0] = p_next[0];
         pB[1] = p_next[1];
 #pragma unroll

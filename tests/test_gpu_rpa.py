@@ -1023,6 +1023,39 @@ def test_head_dim_256_chunks_at_the_edges_of_a_tile(pkg, wl, gpu, P, cap, window
     assert_parity(gpu_out(pkg, b, gpu).float(), oracle_out(b).float(), **(FP8_TOL if kv_dtype != torch.bfloat16 else BF16_TOL))
 
 
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("P", [64, 16])
+def test_head_dim_256_probabilities_are_rounded_once(pkg, gpu, kv_dtype, P):
+    """A maximum that rises by more than the slack between two tiles, while half of the first tile's probabilities still
+    wait for their product: they are bf16 and are not rounded a second time against the new maximum.  64 equal keys (p = 1,
+    values 1 in their second half), then one key s = 8.02 .. 8.98 (powers of two) above them whose value is 0:
+    32 / (64 + 2^s) to the last bit of bf16, wherever that is not a tie."""
+    rows, kv_len, D = 128, 320, 256
+    s = torch.linspace(8.02, 8.98, rows, dtype=torch.float64) * math.log(2.0)
+    q = torch.zeros(rows, 1, D)
+    q[:, 0, 0] = s.to(torch.bfloat16)  # a logit as the sum of two bf16 numbers
+    q[:, 0, 2] = (s - q[:, 0, 0].double()).to(torch.bfloat16)
+    q[:, 0, 1] = 1.0
+    logit = q[:, 0, 0].double() + q[:, 0, 2].double()
+    cache = torch.zeros(kv_len // P, P, 2, D)
+    k, v = (cache.view(-1, 2, D)[:, i] for i in (0, 1))
+    k[64:, 1] = -104.0  # everything behind the first tile, ...
+    k[100] = 0.0  # ... but the key that carries the row
+    k[100, 0] = k[100, 2] = 1.0
+    v[32:64] = 1.0
+    say(f"d256 risen maximum {kv_dtype} P={P}")
+    d = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)  # noqa: E731
+    out, _ = pkg.ragged_paged_attention(
+        q.to(torch.bfloat16).to(gpu), None, None, cache.to(kv_dtype).to(gpu), d([kv_len]), torch.arange(kv_len // P, dtype=torch.int32, device=gpu),
+        d([0, rows]), d([0, kv_len]), np.array([0, 0, 1], dtype=np.int32), sm_scale=1.0, max_kv_len=kv_len, max_q_len=rows)
+    want = 32.0 / (64.0 + torch.exp(logit))
+    ulp = 2.0 ** (torch.floor(torch.log2(want)) - 7)
+    err = (out[:, 0, 0].cpu().double() - want).abs() / ulp
+    say(f"  {float(err.max()):.3f} units of the last place")
+    assert float(err.max()) <= 0.51
+    assert torch.equal(out[:, 0, :1].expand(-1, D), out[:, 0])
+
+
 def test_head_dim_256_cache_write_and_gather(pkg, wl, gpu):
     """The new-token write and the page gather take any head width (bit-exact)."""
     q_lens, kv_lens = [1, 7], [33, 40]
