@@ -136,11 +136,12 @@ struct PrefillArgs {
   // Prompts without a prefix: kv addresses the caller's new rows (a sequence's start at its first query token, one huge
   // page), and the last write_blocks workgroups of the grid put them into the cache, write_tokens each.
   int32_t rows_are_new;
-  // ShapeOption bits of the cache's pages.  They choose the kernel also where it reads the caller's rows, which would suit
-  // any: the assembly kernel rounds the scaled queries to bf16, and pages that it does not take never had that
-  uint32_t page_options;
   int32_t write_blocks, write_tokens;
   KvWriteArgs write;
+  // ShapeOption bits of the cache's pages (for the launchers).  They choose the kernel also where it reads the caller's
+  // rows, which would suit any: the assembly kernel rounds the scaled queries to bf16, and pages that it does not take
+  // never had that
+  uint32_t page_options;
 };
 
 struct GatherArgs {
