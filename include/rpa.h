@@ -328,7 +328,8 @@ RPA_API int rpa_kv_write(const RpaParams* p, const void* keys, const void* value
  */
 RPA_API int rpa_attention_update(const RpaParams* p, const void* keys, const void* values, void* stream);
 
-/* n words of host memory to device memory in stream order (a batch's metadata); the source may be reused at once. */
+/* n words of host memory to device memory in stream order (a batch's metadata); the source may be reused at once, the
+ * destination is whole once the stream has come that far: work on other streams waits for an event behind it. */
 RPA_API int rpa_upload_words(int32_t* dst, const int32_t* src, int32_t n, void* stream);
 
 /* Whether a RPA_MASK_CUSTOM call needs cu_mask_lens: 0 where the mask is turned into bits first (128-wide heads, max_kv_len

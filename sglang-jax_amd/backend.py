@@ -14,7 +14,8 @@ The batch, layer and KV pool are duck-typed exactly as the reference reads them:
   (mem_cache/memory_pool.py:566-611).
 
 The metadata arithmetic is pure numpy (no device needed); ``get_forward_metadata`` then
-uploads it once per forward pass and every layer call reuses it.  Host-side bounds
+uploads it once per forward pass, in the order of torch's current stream, and every layer call
+on that stream reuses it.  Host-side bounds
 (``max_kv_len``, ``max_q_len``, the decode work sum) travel with the metadata because the
 library sizes its launch grids from them without reading device memory.
 """
@@ -230,7 +231,11 @@ def build_verify_metadata(
 
 @dataclass
 class FlashAttentionMetadata:
-    """Built once per forward pass, reused by every layer (flashattention_backend.py:72-120)."""
+    """Built once per forward pass, reused by every layer (flashattention_backend.py:72-120).
+
+    The device tensors are written in the order of the stream that is current when they are built, and the host does not
+    wait for them: a layer call on another stream has to be ordered behind that one (``other.wait_stream(stream)`` or an
+    event), like any tensor that torch makes on one stream and reads on another."""
 
     cu_q_lens: torch.Tensor | None = None
     cu_kv_lens: torch.Tensor | None = None

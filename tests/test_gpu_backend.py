@@ -283,3 +283,55 @@ def test_prompts_keep_the_precision_of_their_pages(pkg, gpu, P, bound, lens):
         err = float((got.cpu().double() - want).norm() / want.norm())
         say(f"  {name} {err:.3e}")
         assert err <= bound, (name, err)
+
+
+@pytest.mark.parametrize("mla", [False, True])
+def test_metadata_arrives_in_the_order_of_its_stream(pkg, gpu, mla):
+    """Metadata built on one stream, behind work that is still running there, and read on another that waits for the first
+    (the host does not wait, so without that the words need not be there)."""
+    P, rng = 16, np.random.default_rng(6 + mla)
+    kv = np.array([700, 33, 1500, 1], dtype=np.int32)
+    n = int((-(-kv // P)).sum())
+    pages = rng.permutation(n).astype(np.int32) + 1
+    loc = (pages.astype(np.int64)[:, None] * P + np.arange(P)).reshape(-1).astype(np.int32)
+    batch = SimpleNamespace(forward_mode=pkg.ForwardMode.DECODE, seq_lens=kv, cache_loc=loc, extend_seq_lens=None, dp_size=1,
+                            per_dp_bs_size=len(kv))
+    backend = (pkg.MLAAttentionBackend(16, 512, 128, 64, 128, page_size=P, device=gpu) if mla
+               else pkg.FlashAttention(8, 2, 128, page_size=P, device=gpu))
+    one, two = torch.cuda.Stream(gpu), torch.cuda.Stream(gpu)
+    torch.cuda.synchronize()
+    say(f"metadata on two streams mla={mla}")
+    with torch.cuda.stream(one):
+        torch.cuda._sleep(50_000_000)  # some 20 ms
+        md = backend.get_forward_metadata(batch)
+    two.wait_stream(one)
+    with torch.cuda.stream(two):
+        got = {name: getattr(md, name).cpu().numpy() for name in ("page_indices", "seq_lens", "cu_q_lens", "cu_kv_lens", "distribution")}
+    torch.cuda.synchronize()
+    want = pkg.build_forward_metadata(forward_mode=pkg.ForwardMode.DECODE, seq_lens=kv, cache_loc=loc, page_size=P)
+    for name, x in got.items():
+        assert np.array_equal(x, want[name]), name
+
+
+def test_metadata_inside_a_captured_graph(pkg, gpu):
+    """Under capture the upload becomes part of the graph; every replay leaves the same words."""
+    P = 16
+    kv = np.array([40, 7, 100], dtype=np.int32)
+    n = int((-(-kv // P)).sum())
+    loc = (np.arange(n, dtype=np.int64)[::-1, None] * P + np.arange(P)).reshape(-1).astype(np.int32)
+    batch = SimpleNamespace(forward_mode=pkg.ForwardMode.DECODE, seq_lens=kv, cache_loc=loc, extend_seq_lens=None, dp_size=1,
+                            per_dp_bs_size=len(kv))
+    backend = pkg.FlashAttention(8, 2, 128, page_size=P, device=gpu)
+    want = pkg.build_forward_metadata(forward_mode=pkg.ForwardMode.DECODE, seq_lens=kv, cache_loc=loc, page_size=P)
+    backend.get_forward_metadata(batch)
+    torch.cuda.synchronize()
+    say("metadata under capture")
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        md = backend.get_forward_metadata(batch)
+    for _ in range(3):
+        md.page_indices.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(md.page_indices.cpu().numpy(), want["page_indices"])
+        assert np.array_equal(md.cu_kv_lens.cpu().numpy(), want["cu_kv_lens"])
