@@ -119,6 +119,10 @@ __device__ __forceinline__ int32_t scalar_load_i32(const int32_t* p) {
   return *reinterpret_cast<const_ptr_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+__device__ __forceinline__ float scalar_load_f32(const float* p) {
+  return __int_as_float(scalar_load_i32(reinterpret_cast<const int32_t*>(p)));
+}
+
 // Asynchronous 16-byte copy global -> LDS (global_load_lds_dwordx4): lane l's 16 bytes land at
 // lds_base + 16*l; the data never touches a VGPR and completion is counted by vmcnt.  Issued as
 // inline assembly so that the compiler does not model it as an LDS store: it would otherwise
@@ -133,6 +137,20 @@ __device__ __forceinline__ void async_copy16(const void* gsrc, const void* lds_b
 // Eight query elements from dim d of a row of q_dim (a multiple of 8); dims past it are zero.
 __device__ __forceinline__ u32x4_t ld_query(const uint16_t* row, int d, int q_dim) {
   return d < q_dim ? *reinterpret_cast<const u32x4_t*>(row + d) : u32x4_t{0u, 0u, 0u, 0u};
+}
+
+// The N groups of eight that lane group g holds of a row that has D elements in the cache: dims D / N i + 8 g ..
+// A row of full width is asked for once and not load by load: its loads go out together.
+template <int N, int D>
+__device__ __forceinline__ void ld_query_row(u32x4_t (&q)[N], const uint16_t* row, int g, int q_dim) {
+  constexpr int kStep = D / N;
+  if (q_dim == D) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) q[i] = *reinterpret_cast<const u32x4_t*>(row + i * kStep + g * 8);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) q[i] = ld_query(row, i * kStep + g * 8, q_dim);
+  }
 }
 
 // 16-byte global loads / stores.

@@ -43,7 +43,6 @@ namespace {
 // such chunks then fill their tiles, and the four waves still share every K/V tile.
 template <bool UNIFORM, bool CAP, bool EXT, bool HEADS4 = false>
 __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const PrefillArgs a_in, int tiles, int nseq, bool by_level) {
-  if (writes_new_tokens(a_in)) return;
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
@@ -63,7 +62,10 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
 
   constexpr int BM = HEADS4 ? 32 : kBM;  // query positions per workgroup
   Work w = decompose(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
-  if (!w.valid) return;
+  if (!w.valid) {
+    write_new_tokens(a_in);
+    return;
+  }
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -85,15 +87,14 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
   {
     const int rr = min(wr.row, w.q_len - 1);
     const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * a.q_dim;
-#pragma unroll
-    for (int ks = 0; ks < T::kSteps; ++ks) qB[ks] = ld_query(qp, ks * 16 + h * 8, a.q_dim);
+    ld_query_row<T::kSteps, HD>(qB, qp, h, a.q_dim);
     if (EXT && a.sm.q_scale > 0.f) {
 #pragma unroll
       for (int ks = 0; ks < T::kSteps; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, false);
     }
   }
   Softmax<CAP> sm;
-  sm.scale = a.sm.sm_scale * (a.k_scale ? a.k_scale[w.hk] : 1.0f) *
+  sm.scale = a.sm.sm_scale * (a.k_scale ? scalar_load_f32(a.k_scale + w.hk) : 1.0f) *
              ((EXT && a.sm.q_scale > 0.f) ? a.sm.q_scale : 1.0f);
   sm.cap = a.sm.soft_cap;
   sm.inv_cap = (sm.cap != 0.f) ? 1.0f / sm.cap : 0.f;
@@ -301,7 +302,6 @@ struct WideFeed {
 
 template <bool UNIFORM, bool CAP, bool EXT, bool FP8>
 __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillArgs a_in, int tiles, int nseq, bool by_level) {
-  if (writes_new_tokens(a_in)) return;
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
@@ -311,7 +311,10 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillA
   __shared__ __attribute__((aligned(1024))) char stage[FP8 ? kWTileB : 16];  // K bytes, V bytes
 
   const Work w = decompose(a, tiles, nseq, by_level, kBM, 1);
-  if (!w.valid) return;
+  if (!w.valid) {
+    write_new_tokens(a_in);
+    return;
+  }
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -341,14 +344,13 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillA
   u32x4_t qB[8];
   {
     const uint16_t* qp = a.q + ((int64_t)(w.qg0 + min(row, w.q_len - 1)) * a.Hq + w.head) * a.q_dim;
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qB[ks] = ld_query(qp, ks * 32 + g * 8, a.q_dim);
+    ld_query_row<8, 256>(qB, qp, g, a.q_dim);
     if (EXT && a.sm.q_scale > 0.f) {
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, FP8);
     }
   }
-  const float scale = a.sm.sm_scale * (a.k_scale ? a.k_scale[w.hk] : 1.0f) * ((EXT && a.sm.q_scale > 0.f) ? a.sm.q_scale : 1.0f);
+  const float scale = a.sm.sm_scale * (a.k_scale ? scalar_load_f32(a.k_scale + w.hk) : 1.0f) * ((EXT && a.sm.q_scale > 0.f) ? a.sm.q_scale : 1.0f);
   const float temp = EXT ? xai_factor(qpos, a.sm.xai_len) : 1.0f;  // per position
   const float sc2 = CAP ? 1.0f : scale * kLog2e * temp;            // score -> log2 units (soft-capped scores are there already)
 
@@ -579,7 +581,7 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillA
     }
     return;
   }
-  const float vs = a.v_scale ? a.v_scale[w.hk] : 1.0f;
+  const float vs = a.v_scale ? scalar_load_f32(a.v_scale + w.hk) : 1.0f;
   const float inv = a.sm.sink ? vs * sink_inverse(m * sc2, l, sink_logit(a.sm.sink, a.sm.round_logits, w.head)) : vs / l;
   uint16_t* op = a.out + out_row * a.q_dim + 4 * g;
 #pragma unroll
@@ -708,7 +710,6 @@ __device__ __forceinline__ void tile_lstore(const Stage<FP8>& st, char* lds_k, c
 
 template <bool FP8, bool UNIFORM, bool CAP, bool EXT, bool HEADS4 = false>
 __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const PrefillArgs a_in, int tiles, int nseq, bool by_level) {
-  if (writes_new_tokens(a_in)) return;
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
@@ -719,7 +720,10 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const Prefil
 
   constexpr int BM = HEADS4 ? 32 : kBM;  // the short-chunk tile: 32 positions x 4 heads, one head per wave
   Work w = decompose(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
-  if (!w.valid) return;
+  if (!w.valid) {
+    write_new_tokens(a_in);
+    return;
+  }
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   if constexpr (HEADS4) w.head += wave;
@@ -740,15 +744,14 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const Prefil
   {
     const int rr = min(wr.row, w.q_len - 1);
     const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * a.q_dim;
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qB[ks] = ld_query(qp, ks * 16 + h * 8, a.q_dim);
+    ld_query_row<8, 128>(qB, qp, h, a.q_dim);
     if (EXT && a.sm.q_scale > 0.f) {
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, FP8);
     }
   }
   Softmax<CAP> sm;
-  sm.scale = a.sm.sm_scale * (a.k_scale ? a.k_scale[w.hk] : 1.0f) *
+  sm.scale = a.sm.sm_scale * (a.k_scale ? scalar_load_f32(a.k_scale + w.hk) : 1.0f) *
              ((EXT && a.sm.q_scale > 0.f) ? a.sm.q_scale : 1.0f);
   sm.cap = a.sm.soft_cap;
   sm.inv_cap = (sm.cap != 0.f) ? 1.0f / sm.cap : 0.f;

@@ -103,9 +103,11 @@ __device__ __forceinline__ Work decompose(const PrefillArgs& a, int tiles, int n
   w.head = w.hk * a.G + gi;
   w.seq = a.seq_begin + si;
   if (w.seq >= a.seq_end) return w;  // the grid was sized for a bound on the number of sequences
-  w.qg0 = a.pt.cu_q_lens[w.seq];
-  w.q_len = a.pt.cu_q_lens[w.seq + 1] - w.qg0;
-  w.kv_len = a.pt.kv_lens[w.seq];
+  // (scalar loads, said explicitly here and below: in a kernel that also writes the cache the compiler takes no ordinary
+  // load for one of memory that stays as it is, and fetches the lengths through the vector memory pipe)
+  w.qg0 = scalar_load_i32(a.pt.cu_q_lens + w.seq);
+  w.q_len = scalar_load_i32(a.pt.cu_q_lens + w.seq + 1) - w.qg0;
+  w.kv_len = scalar_load_i32(a.pt.kv_lens + w.seq);
   w.prefix = w.kv_len - w.q_len;
   int tile = tiles - 1 - tile_rev;
   if (by_level) tile -= (max(w.prefix, 0) + bm - 1) / bm;
@@ -122,11 +124,12 @@ __device__ __forceinline__ const char* head_rows(const PrefillArgs& a, const Wor
 
 // The workgroups behind those of the attention itself leave the new tokens in the cache: a wave takes a token at a time.
 // The attention does not wait for them (it reads the caller's rows), and a launch in front of it is saved: 4.3 us of the 25
-// that a prompt of 1003 tokens on 8 heads took.  true: this workgroup was one of them.
-__device__ __forceinline__ bool writes_new_tokens(const PrefillArgs& a) {
+// that a prompt of 1003 tokens on 8 heads took.  Called by the workgroups that decompose() finds no tile for, as it does for
+// those behind the attention's (a question in front of it is a load that every workgroup waits for: 2.5 us of the 317 of a
+// mixed batch that writes nothing here).
+__device__ __forceinline__ void write_new_tokens(const PrefillArgs& a) {
   const int first = (int)gridDim.x - a.write_blocks;
-  if ((int)blockIdx.x < first) return false;
-  if (blockIdx.y != 0) return true;
+  if ((int)blockIdx.x < first || blockIdx.y != 0) return;
   const KvWriteArgs& wr = a.write;
   const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
   const int t0 = ((int)blockIdx.x - first) * a.write_tokens;
@@ -152,7 +155,6 @@ __device__ __forceinline__ bool writes_new_tokens(const PrefillArgs& a) {
       st16(const_cast<char*>(wr.kv.v_base) + at, ld16(wr.values + from + b));
     }
   }
-  return true;
 }
 
 __device__ __forceinline__ TileSrc make_src(const PrefillArgs& a, const Work& w) {
@@ -160,7 +162,7 @@ __device__ __forceinline__ TileSrc make_src(const PrefillArgs& a, const Work& w)
   src.page_size = a.pt.page_size;
   src.page_shift = ((src.page_size & (src.page_size - 1)) == 0) ? (31 - __builtin_clz(src.page_size)) : -1;
   src.last_tok = w.kv_len - 1;
-  src.pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (a.pt.cu_kv_lens[w.seq] / a.pt.page_size)
+  src.pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (scalar_load_i32(a.pt.cu_kv_lens + w.seq) / a.pt.page_size)
                                                   : (int64_t)w.seq * a.pt.pages_per_seq);
   return src;
 }
@@ -366,7 +368,7 @@ __device__ __forceinline__ void write_rows(const PrefillArgs& a, const Work& w, 
                                            const f32x16_t (&O)[ND], float l, int h, float m2) {
   l += __shfl_xor(l, 32);
   if (!wr.active || wr.row >= w.q_len) return;
-  const float vs = a.v_scale ? a.v_scale[w.hk] : 1.0f;
+  const float vs = a.v_scale ? scalar_load_f32(a.v_scale + w.hk) : 1.0f;
   const float inv = a.sm.sink ? vs * sink_inverse(m2, l, sink_logit(a.sm.sink, a.sm.round_logits, w.head)) : vs / l;
   uint16_t* op = a.out + ((int64_t)(w.qg0 + wr.row) * a.Hq + w.head) * a.q_dim + 4 * h;
 #pragma unroll

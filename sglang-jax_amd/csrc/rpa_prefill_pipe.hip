@@ -296,7 +296,6 @@ template <bool WIN, int NQ, bool HEADS4 = false, bool SPLIT = false>
 __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kernel(const PrefillArgs a_in, int tiles, int nseq,
                                                                                  bool by_level, float row_sum_limit,
                                                                                  bool masked_steps) {
-  if (writes_new_tokens(a_in)) return;
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
@@ -307,7 +306,10 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
   __shared__ __attribute__((aligned(1024))) char lds[4 * kTileB];
 
   Work w = decompose(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
-  if (!w.valid) return;
+  if (!w.valid) {
+    write_new_tokens(a_in);
+    return;
+  }
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -324,7 +326,7 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
   const int r_hi = min(r_lo + 32 * NQ - 1, w.q_len - 1);
   const bool active = r_lo < w.q_len;
   const int W_ = WIN ? a.sm.window : 0;
-  const float sc2 = a.sm.sm_scale * (a.k_scale ? a.k_scale[w.hk] : 1.0f) * kLog2e;
+  const float sc2 = a.sm.sm_scale * (a.k_scale ? scalar_load_f32(a.k_scale + w.hk) : 1.0f) * kLog2e;
 
   const int wg_r_hi = min(w.q_start + BM, w.q_len) - 1;
   int t_hi = min(w.kv_len, w.prefix + wg_r_hi + 1);  // exclusive
@@ -358,13 +360,13 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
     b[q].qpos = w.prefix + row;
     const int rr = min(row, w.q_len - 1);
     const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * a.q_dim;
+    u32x4_t x[8];
+    ld_query_row<8, 128>(x, qp, h, a.q_dim);
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-      const u32x4_t x = ld_query(qp, ks * 16 + h * 8, a.q_dim);
+    for (int ks = 0; ks < 8; ++ks)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        b[q].Q[4 * ks + e] = pack_bf16x2(bf16_lo_to_f32(x[e]) * sc2, bf16_hi_to_f32(x[e]) * sc2);
-    }
+        b[q].Q[4 * ks + e] = pack_bf16x2(bf16_lo_to_f32(x[ks][e]) * sc2, bf16_hi_to_f32(x[ks][e]) * sc2);
 #pragma unroll
     for (int d = 0; d < 4; ++d) b[q].O[d] = kZero16;
     b[q].S[0] = b[q].S[1] = b[q].NM = kZero16;
