@@ -937,7 +937,11 @@ int rpa_attention_update(const RpaParams* p, const void* keys, const void* value
     return decode_rows(p, with_rows ? keys : nullptr, with_rows ? values : nullptr, true, stream);
   }
   if (keys && takes_fresh_prompts(p)) return prefill_run(p, keys, values, stream);
-  const bool fused = keys && decode_takes_new_tokens(p);
+  // (with chunks behind the rows their tokens need a launch anyway, and it takes the rows' along: 317.1 -> 316.7 us, 47.3 ->
+  // 47.1, 162.7 -> 162.3 for mixed batches.  With the composition on the device there are chunks in few calls, and the launch
+  // for them ends at once: 30 rows of 100..700 tokens in a bucket of 32 24.4 -> 22.6 us)
+  const bool chunks = !p->distribution && p->num_seqs > p->decode_end;
+  const bool fused = keys && !chunks && decode_takes_new_tokens(p);
   if (keys && !fused && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
   if ((rc = decode_rows(p, fused ? keys : nullptr, fused ? values : nullptr, false, stream)) != RPA_OK) return rc;
   if (fused && (rc = write_new_tokens(p, keys, values, true, stream)) != RPA_OK) return rc;
