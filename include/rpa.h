@@ -76,7 +76,11 @@ typedef enum RpaLayout {
   RPA_LAYOUT_FUSED = 0,
   /* two buffers k_pages, v_pages [pages, P, Hkv, D]
    * (kernels/ragged_paged_attention/ragged_paged_attention_v3.py:96-97) */
-  RPA_LAYOUT_SPLIT = 1
+  RPA_LAYOUT_SPLIT = 1,
+  /* added to one of the two: the caller's RpaParams has the fields behind `distribution`, q_head_dim and prompts_only.
+   * Without it they are taken as 0 and not read, so that a caller compiled against a header that did not have them
+   * keeps working */
+  RPA_PARAMS_TAIL = 0x100
 } RpaLayout;
 
 /*
@@ -103,13 +107,14 @@ typedef struct RpaParams {
   int32_t num_seqs;           /* S = distribution[2]: sequences to process */
   int32_t num_q_heads;        /* Hq */
   int32_t num_kv_heads;       /* Hkv, Hq % Hkv == 0 */
-  int32_t head_dim;           /* D: 128 or 256.  Narrower heads (64, 80, 96, 192 ...) run zero-padded to the next
-                               * multiple of 128 exactly as in the reference (rpa_v3:1187-1241 pads the queries,
-                               * memory_pool.py:70 stores aligned rows); the caller pads, as the host mirror does */
+  int32_t head_dim;           /* D of the cache's rows: 128 or 256.  Narrower heads (64, 80, 96, 192 ...) are stored
+                               * zero-padded to the next multiple of 128 as in the reference (memory_pool.py:70; the
+                               * reference pads the queries too, rpa_v3:1187-1241).  q, out, keys and values either
+                               * come padded, or in their own width with q_head_dim (below) */
   int32_t page_size;          /* P */
   int32_t total_pages;
   int32_t pages_per_seq;      /* row stride of the padded table (cu_kv_lens == NULL) */
-  int32_t layout;             /* RpaLayout */
+  int32_t layout;             /* RpaLayout, + RPA_PARAMS_TAIL where the last two fields are set */
   int32_t kv_dtype;           /* RpaKvDtype */
   /* ---- batch composition: distribution = (decode_end, prefill_end, num_seqs)
    *      (ragged_paged_attention_v3.py:82-91); sequences [0, decode_end) have
@@ -164,6 +169,7 @@ typedef struct RpaParams {
    * Neither mode limits the sequences or tokens of a call beyond int32: rows are folded onto the first
    * grid dimension. */
   const int32_t* distribution;
+  /* ---- read only with RPA_PARAMS_TAIL in `layout` ---- */
   /* Elements of a row of q, out, keys and values where that is less than the cache's head_dim (the reference pads heads
    * to a multiple of 128, rpa_v3:1187-1241): a multiple of 8 (e4m3: 16), head_dim - q_head_dim < 128; 0 = head_dim.
    * The rest of a cached row is zero, is written as zeros with the new tokens and adds nothing. */

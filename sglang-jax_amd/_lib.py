@@ -17,6 +17,7 @@ RPA_KV_BF16 = 0
 RPA_KV_FP8_E4M3 = 1
 RPA_LAYOUT_FUSED = 0
 RPA_LAYOUT_SPLIT = 1
+RPA_PARAMS_TAIL = 0x100  # added to the layout: q_head_dim and prompts_only of RpaParams are set (else they are not read)
 
 STATUS_NAMES = {
     0: "RPA_OK",

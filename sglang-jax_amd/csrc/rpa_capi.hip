@@ -8,6 +8,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -92,6 +93,22 @@ size_t mask_bits_bytes(const RpaParams* p) {
 }
 bool mask_as_bits(const RpaParams* p) { return mask_bits_bytes(p) != 0; }
 
+// A caller's parameters as this build knows them.  The fields behind `distribution` came later: a caller compiled against
+// an earlier header passes a struct that ends there, and nothing behind that is read unless `layout` says it is (rpa.h).
+// Every entry point starts with one of these and works on its copy.
+struct OwnParams {
+  RpaParams own = {};
+  const RpaParams* p = nullptr;  // nullptr where the caller's is
+  explicit OwnParams(const RpaParams* given) {
+    if (!given) return;
+    const bool tail = given->layout == (RPA_LAYOUT_FUSED | RPA_PARAMS_TAIL) || given->layout == (RPA_LAYOUT_SPLIT | RPA_PARAMS_TAIL);
+    memcpy(&own, given, tail ? sizeof(own) : offsetof(RpaParams, q_head_dim));
+    if (own.layout == RPA_LAYOUT_FUSED || own.layout == RPA_LAYOUT_SPLIT) own.layout |= RPA_PARAMS_TAIL;  // the copy has them
+    p = &own;
+  }
+};
+int layout_of(const RpaParams* p) { return p->layout & ~RPA_PARAMS_TAIL; }
+
 // elements of a row of queries, keys, values and outputs
 int q_dim_of(const RpaParams* p) { return p->q_head_dim > 0 ? p->q_head_dim : p->head_dim; }
 
@@ -102,7 +119,7 @@ rpa::KvAddr kv_addr(const RpaParams* p) {
   const int es = esize_of(p->kv_dtype);
   const int64_t D = p->head_dim, H = p->num_kv_heads, P = p->page_size;
   kv.k_base = static_cast<const char*>(p->kv_cache);
-  if (p->layout == RPA_LAYOUT_FUSED) {
+  if (layout_of(p) == RPA_LAYOUT_FUSED) {
     kv.v_base = kv.k_base + D * es;
     kv.head_stride = (int32_t)(2 * D * es);
     kv.tok_stride = (int32_t)(2 * H * D * es);
@@ -468,7 +485,9 @@ int rpa_version(void) { return RPA_VERSION; }
 
 const char* rpa_last_error(void) { return g_err; }
 
-int rpa_validate(const RpaParams* p) {
+int rpa_validate(const RpaParams* given) {
+  const OwnParams in(given);
+  const RpaParams* p = in.p;
   if (!p) return fail(RPA_EINVAL_NULL, "params is NULL");
   if (p->num_tokens < 0 || p->num_seqs < 0 || p->num_q_heads <= 0 || p->num_kv_heads <= 0 ||
       p->head_dim <= 0 || p->page_size <= 0 || p->total_pages <= 0)
@@ -485,9 +504,9 @@ int rpa_validate(const RpaParams* p) {
     return fail(RPA_EUNSUPPORTED, "head_dim=%d: 128 and 256 are built", p->head_dim);
   if (p->kv_dtype != RPA_KV_BF16 && p->kv_dtype != RPA_KV_FP8_E4M3)
     return fail(RPA_EINVAL_DTYPE, "kv_dtype=%d is not a floating point cache dtype", p->kv_dtype);
-  if (p->layout != RPA_LAYOUT_FUSED && p->layout != RPA_LAYOUT_SPLIT)
+  if (layout_of(p) != RPA_LAYOUT_FUSED && layout_of(p) != RPA_LAYOUT_SPLIT)
     return fail(RPA_EINVAL_SHAPE, "layout=%d unknown", p->layout);
-  if (p->layout == RPA_LAYOUT_SPLIT && !p->v_pages)
+  if (layout_of(p) == RPA_LAYOUT_SPLIT && !p->v_pages)
     return fail(RPA_EINVAL_NULL, "split layout needs v_pages");
   if (p->sliding_window < 0) return fail(RPA_EINVAL_WINDOW, "sliding_window=%d must be positive", p->sliding_window);
   if (std::isnan(p->soft_cap)) return fail(RPA_EINVAL_SOFTCAP, "soft_cap must not be NaN");
@@ -516,9 +535,11 @@ int rpa_validate(const RpaParams* p) {
   return RPA_OK;
 }
 
-int rpa_validate_host(const RpaParams* p, const int32_t* kv_lens, const int32_t* page_indices,
+int rpa_validate_host(const RpaParams* given, const int32_t* kv_lens, const int32_t* page_indices,
                       int64_t num_page_indices, const int32_t* cu_q_lens, const int32_t* cu_kv_lens,
                       const int32_t* distribution) {
+  const OwnParams in(given);
+  const RpaParams* p = in.p;
   int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
   if (!kv_lens || !page_indices || !cu_q_lens) return fail(RPA_EINVAL_NULL, "host metadata is NULL");
@@ -617,14 +638,18 @@ static size_t required_workspace_bytes(const RpaParams* p_in) {
   return (size_t)p->decode_end * sp.splits * p->num_q_heads * (p->head_dim + 2) * sizeof(float);
 }
 
-size_t rpa_workspace_bytes(const RpaParams* p) {
+size_t rpa_workspace_bytes(const RpaParams* given) {
+  const OwnParams in(given);
+  const RpaParams* p = in.p;
   if (!p) return 0;
   const size_t need = std::max(required_workspace_bytes(p), prefill_optional_workspace(p));
   return takes_token_rows(p) ? std::max(need, token_row_workspace(p)) : need;
 }
 
-int rpa_gather_pages(const RpaParams* p, int32_t seq, void* k_out, void* v_out, int32_t max_tokens,
+int rpa_gather_pages(const RpaParams* given, int32_t seq, void* k_out, void* v_out, int32_t max_tokens,
                      void* stream) {
+  const OwnParams in(given);
+  const RpaParams* p = in.p;
   int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
   if (seq < 0 || seq >= p->num_seqs) return fail(RPA_EINVAL_SHAPE, "seq=%d out of [0, %d)", seq, p->num_seqs);
@@ -742,7 +767,9 @@ static int decode_rows(const RpaParams* p_in, const void* keys, const void* valu
   return check_hip(rpa::launch_decode(a, static_cast<hipStream_t>(stream)), "rpa_decode");
 }
 
-int rpa_decode(const RpaParams* p, void* stream) {
+int rpa_decode(const RpaParams* given, void* stream) {
+  const OwnParams in(given);
+  const RpaParams* p = in.p;
   const int rc = rpa_validate(p);
   return rc != RPA_OK ? rc : decode_rows(p, nullptr, nullptr, false, stream);
 }
@@ -896,14 +923,16 @@ int rpa_upload_words(int32_t* dst, const int32_t* src, int32_t n, void* stream) 
   return check_hip(rpa::launch_upload(dst, src, n, static_cast<hipStream_t>(stream)), "rpa_upload_words");
 }
 
-int rpa_prefill(const RpaParams* p, void* stream) {
-  if (!p || !p->prompts_only) return prefill_run(p, nullptr, nullptr, stream);
-  RpaParams q = *p;  // the new tokens are in the cache already
-  q.prompts_only = 0;
-  return prefill_run(&q, nullptr, nullptr, stream);
+int rpa_prefill(const RpaParams* given, void* stream) {
+  OwnParams in(given);
+  in.own.prompts_only = 0;  // the new tokens are in the cache already
+  return prefill_run(in.p, nullptr, nullptr, stream);
 }
 
-int rpa_mask_needs_starts(const RpaParams* p) { return p && p->mask_mode == RPA_MASK_CUSTOM && !mask_as_bits(p) ? 1 : 0; }
+int rpa_mask_needs_starts(const RpaParams* given) {
+  const OwnParams in(given);
+  return in.p && in.p->mask_mode == RPA_MASK_CUSTOM && !mask_as_bits(in.p) ? 1 : 0;
+}
 
 // (narrow heads: only the kernels that know of the zeros behind 64 dims)
 static bool rows_take_new_tokens(const RpaParams* p) {
@@ -927,7 +956,9 @@ static int write_new_tokens(const RpaParams* p, const void* keys, const void* va
   return check_hip(rpa::launch_kv_write(a, static_cast<hipStream_t>(stream)), "rpa_kv_write");
 }
 
-int rpa_attention_update(const RpaParams* p, const void* keys, const void* values, void* stream) {
+int rpa_attention_update(const RpaParams* given, const void* keys, const void* values, void* stream) {
+  const OwnParams in(given);
+  const RpaParams* p = in.p;
   int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
   if (!keys != !values) return fail(RPA_EINVAL_NULL, "keys and values must be given together");
@@ -950,7 +981,9 @@ int rpa_attention_update(const RpaParams* p, const void* keys, const void* value
 
 int rpa_attention(const RpaParams* p, void* stream) { return rpa_attention_update(p, nullptr, nullptr, stream); }
 
-int rpa_describe_plan(const RpaParams* p_in, char* buf, size_t len) {
+int rpa_describe_plan(const RpaParams* given, char* buf, size_t len) {
+  const OwnParams in(given);
+  const RpaParams* p_in = in.p;
   int rc = rpa_validate(p_in);
   if (rc != RPA_OK) return rc;
   if (!buf || len == 0) return fail(RPA_EINVAL_NULL, "buf is NULL or empty");
@@ -1001,7 +1034,9 @@ int rpa_describe_plan(const RpaParams* p_in, char* buf, size_t len) {
 
 size_t rpa_noalloc_max_workspace_bytes(void) { return kNoAllocScratchBytes; }
 
-int rpa_attention_noalloc(const RpaParams* p, void* stream) {
+int rpa_attention_noalloc(const RpaParams* given, void* stream) {
+  const OwnParams in(given);
+  const RpaParams* p = in.p;
   int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
   const size_t need = required_workspace_bytes(p);  // (a prefill launch cuts its K/V ranges only if the array has the room)
@@ -1024,7 +1059,9 @@ int rpa_attention_noalloc(const RpaParams* p, void* stream) {
   return rpa_attention(&q, stream);
 }
 
-int rpa_kv_write(const RpaParams* p, const void* keys, const void* values, void* stream) {
+int rpa_kv_write(const RpaParams* given, const void* keys, const void* values, void* stream) {
+  const OwnParams in(given);
+  const RpaParams* p = in.p;
   int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
   if (!keys || !values) return fail(RPA_EINVAL_NULL, "keys/values is NULL");

@@ -306,7 +306,7 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   p.q_head_dim = (int32_t)row;
   p.page_size = (int32_t)cache->size(1);
   p.total_pages = (int32_t)cache->size(0);
-  p.layout = RPA_LAYOUT_FUSED;
+  p.layout = RPA_LAYOUT_FUSED | RPA_PARAMS_TAIL;
   p.kv_dtype = kv_type == at::kBFloat16 ? RPA_KV_BF16 : RPA_KV_FP8_E4M3;
   COMMON(!rpa_mask_needs_starts(&p));
   p.prompts_only = keys.defined() && PyObject_IsTrue(a[28]) == 1;

@@ -129,6 +129,39 @@ def base_params(pkg):
     return p
 
 
+def test_a_caller_of_the_earlier_struct_is_read_no_further_than_it_reaches(pkg):
+    """RpaParams grew two fields behind `distribution`: they are read where the layout says that they are there, else taken as
+    0 whatever lies behind the caller's struct."""
+    lib, tail = pkg._lib.load(), pkg._lib.RPA_PARAMS_TAIL
+    P = pkg._lib.RpaParams
+    old_size = P.q_head_dim.offset
+    assert old_size == P.distribution.offset + 8
+
+    def answers(p):
+        buf = ctypes.create_string_buffer(1024)
+        ref = ctypes.cast(ctypes.addressof(p), ctypes.POINTER(P))
+        n = lib.rpa_describe_plan(ref, buf, len(buf))
+        return lib.rpa_validate(ref), lib.rpa_workspace_bytes(ref), lib.rpa_mask_needs_starts(ref), n, buf.value
+
+    for layout in (pkg._lib.RPA_LAYOUT_FUSED, pkg._lib.RPA_LAYOUT_SPLIT):
+        p = base_params(pkg)
+        p.layout, p.v_pages = layout, 0x1000
+        want = answers(p)
+        assert want[0] == 0 and want[3] > 0
+        for rest in (b"\xff" * 64, b"\x40\0\0\0\x01\0\0\0" * 8):  # -1, -1, ...; 64, 1, ...
+            assert answers(ctypes.create_string_buffer(bytes(p)[:old_size] + rest)) == want
+        # the same fields where the caller says that they are there
+        p.layout = layout | tail
+        assert answers(p) == want
+        p.q_head_dim = -1
+        assert status(pkg, lib.rpa_validate(ctypes.byref(p))) == "RPA_EUNSUPPORTED"
+        p.q_head_dim = 64
+        assert lib.rpa_validate(ctypes.byref(p)) == 0
+    for layout in (2, 0x102, 0x200, -1):
+        p.layout = layout
+        assert status(pkg, lib.rpa_validate(ctypes.byref(p))) == "RPA_EINVAL_SHAPE"
+
+
 def status(pkg, code):
     return pkg._lib.STATUS_NAMES[code]
 
