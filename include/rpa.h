@@ -295,7 +295,10 @@ RPA_API int rpa_attention(const RpaParams* p, void* stream);
 /*
  * Which launch shape a call would take, as text: the row of the library's shape table (kernel family, query
  * positions x query heads x K/V tokens per workgroup, waves walked together, resident waves), the split plan
- * of the decode rows and the workspace behind it.  The counterpart of the reference's get_tuned_block_sizes /
+ * of the decode rows and the workspace behind it, and who leaves the new tokens of rpa_attention_update in the cache.
+ * "whole call" stands in front where rpa_attention and rpa_attention_update run every query token as a row of the decode
+ * kernels (few tokens on short contexts, workspace of rpa_workspace_bytes()); "decode" and "prefill" are then what
+ * rpa_decode and rpa_prefill take.  The counterpart of the reference's get_tuned_block_sizes /
  * get_default_block_sizes, which answer the same question for its tile table
  * (kernels/ragged_paged_attention/tuned_block_sizes_v3.py:2163-2229, ragged_paged_attention_v3.py:1490-1638).
  * Host arithmetic only (no launch, no device read).  Writes at most len - 1 characters plus a NUL into buf and

@@ -956,6 +956,15 @@ static int write_new_tokens(const RpaParams* p, const void* keys, const void* va
   return check_hip(rpa::launch_kv_write(a, static_cast<hipStream_t>(stream)), "rpa_kv_write");
 }
 
+// Whether the decode rows of a call write their tokens themselves.  (With chunks behind the rows their tokens need a launch
+// anyway, and it takes the rows' along: 317.1 -> 316.7 us, 47.3 -> 47.1, 162.7 -> 162.3 for mixed batches.  With the
+// composition on the device there are chunks in few calls, and the launch for them ends at once: 30 rows of 100..700 tokens
+// in a bucket of 32 24.4 -> 22.6 us.)
+static bool decode_rows_write(const RpaParams* p) {
+  const bool chunks = !p->distribution && p->num_seqs > p->decode_end;
+  return !chunks && decode_takes_new_tokens(p);
+}
+
 int rpa_attention_update(const RpaParams* given, const void* keys, const void* values, void* stream) {
   const OwnParams in(given);
   const RpaParams* p = in.p;
@@ -968,11 +977,7 @@ int rpa_attention_update(const RpaParams* given, const void* keys, const void* v
     return decode_rows(p, with_rows ? keys : nullptr, with_rows ? values : nullptr, true, stream);
   }
   if (keys && takes_fresh_prompts(p)) return prefill_run(p, keys, values, stream);
-  // (with chunks behind the rows their tokens need a launch anyway, and it takes the rows' along: 317.1 -> 316.7 us, 47.3 ->
-  // 47.1, 162.7 -> 162.3 for mixed batches.  With the composition on the device there are chunks in few calls, and the launch
-  // for them ends at once: 30 rows of 100..700 tokens in a bucket of 32 24.4 -> 22.6 us)
-  const bool chunks = !p->distribution && p->num_seqs > p->decode_end;
-  const bool fused = keys && !chunks && decode_takes_new_tokens(p);
+  const bool fused = keys && decode_rows_write(p);
   if (keys && !fused && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
   if ((rc = decode_rows(p, fused ? keys : nullptr, fused ? values : nullptr, false, stream)) != RPA_OK) return rc;
   if (fused && (rc = write_new_tokens(p, keys, values, true, stream)) != RPA_OK) return rc;
@@ -999,22 +1004,26 @@ int rpa_describe_plan(const RpaParams* given, char* buf, size_t len) {
     if (n > 0) at += (size_t)n;
   };
   buf[0] = 0;
+  auto put_rows = [&](const char* what, const RpaParams* v, bool token_rows, size_t workspace) {
+    const rpa::ShapeRule& r = decode_shape(v);
+    const SplitPlan sp = decode_plan(v);
+    const bool bal = !token_rows && use_balanced(v, sp), whole = !bal && rows_in_one_workgroup(v, sp);
+    put("%s: shape=%s kernel=%s rows=%d", what, r.name,
+        whole ? "rpa_decode_row_kernel" : bal ? "rpa_decode_balanced_kernel" : "rpa_decode_splitkv_kernel", v->decode_end);
+    if (!whole) put(" waves_per_wg=%d", bal ? decode_waves_per_wg(v) : decode_fixed_waves(v));
+    if (bal) put(" resident_waves=%d merge=rpa_combine_balanced_kernel", decode_wave_capacity(v));
+    else if (!whole) put(" pieces_per_row=%d chunk=%d merge=%s", sp.splits, sp.chunk, sp.splits > 1 ? "rpa_combine_kernel" : "none");
+    put(" workspace=%zu\n", workspace);
+  };
+  if (takes_token_rows(p_in)) {
+    const RpaParams v = token_row_view(p_in);
+    put_rows("whole call", &v, true, token_row_workspace(p_in));
+  }
   if (p->decode_end > 0 && p->mask_mode != RPA_MASK_CUSTOM) {
-    const rpa::ShapeRule& r = decode_shape(p);
-    if (p->head_dim == 256) {
-      const SplitPlan sp = rows256_plan(p);
-      put("decode: shape=%s kernel=rpa_rows256_kernel rows=%d pieces_per_row=%d", r.name, p->decode_end, sp.splits);
-    } else {
-      const SplitPlan sp = decode_plan(p);
-      const bool bal = use_balanced(p, sp);
-      if (!bal && rows_in_one_workgroup(p, sp))
-        put("decode: shape=%s kernel=rpa_decode_row_kernel rows=%d", r.name, p->decode_end);
-      else put("decode: shape=%s kernel=%s rows=%d waves_per_wg=%d", r.name,
-          bal ? "rpa_decode_balanced_kernel" : "rpa_decode_splitkv_kernel", p->decode_end, bal ? decode_waves_per_wg(p) : decode_fixed_waves(p));
-      if (bal) put(" resident_waves=%d merge=rpa_combine_balanced_kernel", decode_wave_capacity(p));
-      else if (!rows_in_one_workgroup(p, sp)) put(" pieces_per_row=%d chunk=%d merge=%s", sp.splits, sp.chunk, sp.splits > 1 ? "rpa_combine_kernel" : "none");
-    }
-    put(" workspace=%zu\n", required_workspace_bytes(p_in));
+    if (p->head_dim == 256)
+      put("decode: shape=%s kernel=rpa_rows256_kernel rows=%d pieces_per_row=%d workspace=%zu\n", decode_shape(p).name, p->decode_end,
+          rows256_plan(p).splits, required_workspace_bytes(p_in));
+    else put_rows("decode", p, false, required_workspace_bytes(p_in));
   }
   rpa::PrefillArgs a;
   if (prefill_args(p_in, a)) {
@@ -1022,13 +1031,21 @@ int rpa_describe_plan(const RpaParams* given, char* buf, size_t len) {
       put("prefill: kernel=rpa_rows256_kernel (RPA_PREFILL_ROWS256)\n");
     } else {
       const rpa::ShapeRule& r = rpa::prefill_shape_of(a);
-      const char* kernel = r.kernel == rpa::kKernelPrefillPipe ? "rpa_prefill_pipe_kernel"
-                           : (r.kernel == rpa::kKernelPrefillStaged ? "rpa_prefill_staged_kernel" : "rpa_prefill_async_kernel");
+      const char* kernel = r.kernel == rpa::kKernelPrefillPipe     ? "rpa_prefill_pipe_kernel"
+                           : r.kernel == rpa::kKernelPrefillStaged ? "rpa_prefill_staged_kernel"
+                           : r.kernel == rpa::kKernelPrefillWide   ? "rpa_prefill_async_kernel_wide"
+                                                                   : "rpa_prefill_async_kernel";
       const PrefillWorkspace w = prefill_workspace(p_in, a);
       put("prefill: shape=%s kernel=%s tile=%dx%dx%d kv_pieces_with_workspace=%d mask_bits=%s optional_workspace=%zu\n",
           r.name, kernel, r.tile_q, r.tile_heads, r.tile_kv, w.splits, w.bits_bytes ? "yes" : "no", w.total);
     }
   }
+  const bool rows = takes_token_rows(p_in), prompts = !rows && takes_fresh_prompts(p_in);
+  const bool by_rows = rows ? rows_take_new_tokens(p_in) : !prompts && decode_rows_write(p_in);
+  put("new tokens: written by %s\n", prompts                            ? "workgroups of the prefill launch, which reads the caller's rows"
+                                     : !by_rows                         ? "rpa_kv_write_kernel, in front"
+                                     : p_in->distribution && !rows      ? "the decode kernels, those of chunks by rpa_kv_write_kernel"
+                                                                        : "the decode kernels");
   return (int)std::min<size_t>(at, 0x7fffffff);
 }
 

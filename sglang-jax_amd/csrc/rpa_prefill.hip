@@ -301,7 +301,7 @@ struct WideFeed {
 };
 
 template <bool UNIFORM, bool CAP, bool EXT, bool FP8>
-__global__ __launch_bounds__(512, 2) void rpa_prefill_wide_kernel(const PrefillArgs a_in, int tiles, int nseq, bool by_level) {
+__global__ __launch_bounds__(512, 2) void rpa_prefill_async_kernel_wide(const PrefillArgs a_in, int tiles, int nseq, bool by_level) {
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
@@ -966,7 +966,7 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
 #define RPA_ASYNC_HEADS4(U, C, E) \
   hipLaunchKernelGGL((rpa_prefill_async_kernel<U, C, E, true>), g, blk, 0, stream, a, tiles, nseq, by_level)
 #define RPA_WIDE(F, U, C, E) \
-  hipLaunchKernelGGL((rpa_prefill_wide_kernel<U, C, E, F>), g, dim3(512), 0, stream, a, tiles, nseq, by_level)
+  hipLaunchKernelGGL((rpa_prefill_async_kernel_wide<U, C, E, F>), g, dim3(512), 0, stream, a, tiles, nseq, by_level)
 #define RPA_PICK(M, ...)                                            \
   switch ((uniform ? 4 : 0) | (cap ? 2 : 0) | (ext ? 1 : 0)) {        \
     case 0: M(__VA_ARGS__ false, false, false); break;              \

@@ -33,6 +33,7 @@ enum ShapeKernel : int {
   kKernelRows256,         // rpa_rows256_kernel
   kKernelPrefillPipe,     // rpa_prefill_pipe_kernel (assembly steady state)
   kKernelPrefillAsync,    // rpa_prefill_async_kernel (compiled, global -> LDS copies)
+  kKernelPrefillWide,     // rpa_prefill_async_kernel_wide (256-wide heads: eight waves of 16 positions)
   kKernelPrefillStaged,   // rpa_prefill_staged_kernel (rows through registers: fp8 caches)
   kKernelMlaWide,         // rpa_mla_*_wide_kernel: four waves x 32 heads, every tile in the assembly loop
   kKernelMlaPipe,         // rpa_mla_*_kernel, eight waves x 16 heads, assembly steady state
@@ -101,9 +102,9 @@ constexpr ShapeRule kShapeRules[] = {
   {"prefill_pipe", kStagePrefill, 16, 128, 0, 0, 0, 0, 0, kOptPlainOnly,
    kKernelPrefillPipe, 128, 1, 64, 4, 16, 1, 0, "assembly steady state: C2 295 -> 236 us"},
   {"prefill_256_fp8", kStagePrefill, 8, 256, 0, 0, 0, 0, 0, 0,
-   kKernelPrefillAsync, 128, 1, 64, 8, 8, 1, 0, "e4m3 bytes staged in LDS and widened into the bf16 tiles; soft cap and window 424 -> 258 us"},
+   kKernelPrefillWide, 128, 1, 64, 8, 8, 1, 0, "e4m3 bytes staged in LDS and widened into the bf16 tiles; soft cap and window 424 -> 258 us"},
   {"prefill_256", kStagePrefill, 16, 256, 0, 0, 0, 0, 0, 0,
-   kKernelPrefillAsync, 128, 1, 64, 8, 8, 1, 0, "eight waves of 16 positions, one workgroup per CU: 182 -> 135 us"},
+   kKernelPrefillWide, 128, 1, 64, 8, 8, 1, 0, "eight waves of 16 positions, one workgroup per CU: 182 -> 135 us"},
   {"prefill_fp8_short", kStagePrefill, 8, 128, 0, 0, 4, 64, 0, 0,
    kKernelPrefillStaged, 32, 4, 64, 4, 16, 1, 0, "short-chunk tile of the register-staged kernel"},
   {"prefill_fp8", kStagePrefill, 8, 128, 0, 0, 0, 0, 0, 0,

@@ -429,6 +429,34 @@ def test_shape_table_rows_of_the_benchmark_configurations(pkg):
     assert "shape=decode_256 kernel=rpa_rows256_kernel" in wide and "shape=prefill_256 kernel=rpa_prefill_async_kernel" in wide
 
 
+def test_described_plan_names_what_runs(pkg):
+    """The kernels of a whole call beside those of its partitions, the 256-wide prefill kernel by its name, and who leaves
+    the new tokens in the cache."""
+    d, tail = pkg._lib.describe_plan, pkg._lib.RPA_PARAMS_TAIL
+    wide = d(_shape_params(pkg, S=6, decode_end=4, T=304, Hq=16, Hkv=4, D=256, max_q=200, max_kv=900, sum_dec=3000))
+    assert "kernel=rpa_prefill_async_kernel_wide " in wide and "whole call" not in wide
+    # decode rows only: their kernels write the tokens; with chunks behind them, or 256-wide heads, a launch in front does
+    rows = dict(S=64, decode_end=64, T=64, Hq=32, Hkv=8, max_kv=4000, sum_dec=130000)
+    assert d(_shape_params(pkg, **rows)).endswith("new tokens: written by the decode kernels\n")
+    assert "written by rpa_kv_write_kernel, in front" in d(_shape_params(pkg, D=256, **rows))
+    mixed = dict(S=64, decode_end=56, T=8760, Hq=32, Hkv=8, max_q=2048, max_kv=4096, sum_dec=130000)
+    assert "written by rpa_kv_write_kernel, in front" in d(_shape_params(pkg, **mixed))
+    bucket = d(_shape_params(pkg, distribution=0x1000, **mixed))
+    assert "the decode kernels, those of chunks by rpa_kv_write_kernel" in bucket and "whole call" not in bucket
+    # a few query tokens on short contexts: rows of the decode kernels, chunk or not
+    few = d(_shape_params(pkg, S=3, decode_end=1, T=20, Hq=16, Hkv=8, P=16, max_q=12, max_kv=500, sum_dec=300))
+    assert few.startswith("whole call: shape=decode_bf16_stream kernel=rpa_decode_splitkv_kernel rows=20 ")
+    assert "\nprefill: shape=prefill_options" in few and few.endswith("written by the decode kernels\n")
+    # prompts without a prefix read the caller's rows; the kernel is that of the cache's pages all the same
+    prompt = dict(S=1, decode_end=0, T=1003, Hq=8, Hkv=2, max_q=1003, max_kv=1003, prompts_only=1)
+    for P, kernel in ((64, "shape=prefill_pipe kernel=rpa_prefill_pipe_kernel"), (16, "shape=prefill_options kernel=rpa_prefill_async_kernel "),
+                      (96, "shape=prefill_options kernel=rpa_prefill_async_kernel ")):
+        text = d(_shape_params(pkg, P=P, layout=tail, **prompt))
+        assert kernel in text and "written by workgroups of the prefill launch, which reads the caller's rows" in text
+        text = d(_shape_params(pkg, P=P, **prompt))  # (the promise is not read without the flag)
+        assert kernel in text and "written by rpa_kv_write_kernel, in front" in text
+
+
 def test_shape_table_environment_overrides(pkg, monkeypatch):
     d = pkg._lib.describe_plan
     p = _shape_params(pkg, S=64, decode_end=56, T=8760, Hq=32, Hkv=8, max_q=2048, max_kv=4096, sum_dec=130000)
