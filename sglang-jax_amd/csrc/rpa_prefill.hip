@@ -48,10 +48,6 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
     a.seq_end = min(a.seq_end, scalar_load_i32(a.dist + 2));
   }
-  constexpr int HD = 128;
-  using T = Tile<HD>;
-  constexpr int kRowB = T::kRowB;
-  constexpr int kTileB = T::kTileB;
   // Four separate arrays (not one indexed array): the compiler can then prove that the
   // asynchronous copy into one ring slot does not alias the LDS reads of the other slot and
   // does not drain the vector-memory queue in the middle of a tile.
@@ -83,14 +79,14 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
   wr.qpos = w.prefix + wr.row;
   const int W_ = a.sm.window;
 
-  u32x4_t qB[T::kSteps];
+  u32x4_t qB[kSteps];
   {
     const int rr = min(wr.row, w.q_len - 1);
     const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * a.q_dim;
-    ld_query_row<T::kSteps, HD>(qB, qp, h, a.q_dim);
+    ld_query_row<kSteps, kHeadDim>(qB, qp, h, a.q_dim);
     if (EXT && a.sm.q_scale > 0.f) {
 #pragma unroll
-      for (int ks = 0; ks < T::kSteps; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, false);
+      for (int ks = 0; ks < kSteps; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, false);
     }
   }
   Softmax<CAP> sm;
@@ -105,9 +101,9 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
     sm.round_mode = a.sm.round_logits;
   }
 
-  f32x16_t O[T::kDimTiles];
+  f32x16_t O[kDimTiles];
 #pragma unroll
-  for (int d = 0; d < T::kDimTiles; ++d)
+  for (int d = 0; d < kDimTiles; ++d)
 #pragma unroll
     for (int v = 0; v < 16; ++v) O[d][v] = 0.f;
   float m = kMaxFloor, l = 0.f;
@@ -122,7 +118,7 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
   if (W_ > 0) t_lo = max(0, w.prefix + w.q_start - W_ + 1) & ~(kBN - 1);
   int split = 0;
   if (a.kv_splits > 1 && !kv_piece(a, t_lo, t_hi, split)) {  // under-filled launch, nothing left for this piece
-    write_empty_partial_rows<T::kDimTiles>(a, w, wr, h, split);
+    write_empty_partial_rows(a, w, wr, h, split);
     return;
   }
 
@@ -140,24 +136,24 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
   // The swizzled offsets are kept in registers for the whole loop (12 of them) instead of being
   // recomputed in front of each of the 48 LDS reads of a tile; slot bases and row steps fold
   // into the instructions' immediate offsets.
-  int koff[T::kSteps], voff[T::kDimTiles];
+  int koff[kSteps], voff[kDimTiles];
 #pragma unroll
-  for (int ks = 0; ks < T::kSteps; ++ks) {
+  for (int ks = 0; ks < kSteps; ++ks) {
     koff[ks] = k_row + ((ks * 32) ^ k_swz);
     asm volatile("" : "+v"(koff[ks]));
   }
 #pragma unroll
-  for (int d = 0; d < T::kDimTiles; ++d) {
+  for (int d = 0; d < kDimTiles; ++d) {
     voff[d] = v_row + v_in + ((d * 64) ^ v_swz);
     asm volatile("" : "+v"(voff[d]));
   }
 
   // ---- pipeline: page ids two tiles ahead, the asynchronous copy one tile ahead ----
-  const AsyncOffsets<HD> ofs = make_async_offsets<HD>(a.kv, wave, lane);
-  AsyncPages<UNIFORM, HD> pg;
-  async_fetch_pages<UNIFORM, HD>(pg, src, t_lo, wave, lane);
-  async_copy_tile<UNIFORM, HD>(lds_k0, lds_v0, src, a.kv, kh, vh, t_lo, wave, lane, pg, ofs);
-  async_fetch_pages<UNIFORM, HD>(pg, src, t_lo + kBN, wave, lane);
+  const AsyncOffsets ofs = make_async_offsets(a.kv, wave, lane);
+  AsyncPages<UNIFORM> pg;
+  async_fetch_pages<UNIFORM>(pg, src, t_lo, wave, lane);
+  async_copy_tile<UNIFORM>(lds_k0, lds_v0, src, a.kv, kh, vh, t_lo, wave, lane, pg, ofs);
+  async_fetch_pages<UNIFORM>(pg, src, t_lo + kBN, wave, lane);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the copies have landed in LDS
   __syncthreads();
 
@@ -169,8 +165,8 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
     }
     if (tb + kBN < t_hi) {
       // the other slot was last read before the barrier that ended the previous tile
-      async_copy_tile<UNIFORM, HD>(nxt_k, nxt_v, src, a.kv, kh, vh, tb + kBN, wave, lane, pg, ofs);
-      async_fetch_pages<UNIFORM, HD>(pg, src, tb + 2 * kBN, wave, lane);
+      async_copy_tile<UNIFORM>(nxt_k, nxt_v, src, a.kv, kh, vh, tb + kBN, wave, lane, pg, ofs);
+      async_fetch_pages<UNIFORM>(pg, src, tb + 2 * kBN, wave, lane);
     }
     // visible to this wave?  causal: some token <= last row's position; window: some token
     // newer than the first row's horizon
@@ -185,19 +181,19 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
         S[0] = mfma32(lds_ld16(lds_k + koff[0]), qB[0], kZero16);  // zero accumulator as an inline constant
         S[1] = mfma32(lds_ld16(lds_k + koff[0] + 32 * kRowB), qB[0], kZero16);
 #pragma unroll
-        for (int ks = 1; ks < T::kSteps; ++ks) {
+        for (int ks = 1; ks < kSteps; ++ks) {
           S[0] = mfma32(lds_ld16(lds_k + koff[ks]), qB[ks], S[0]);
           S[1] = mfma32(lds_ld16(lds_k + koff[ks] + 32 * kRowB), qB[ks], S[1]);
         }
         u32x4_t pB[2][2];
-        softmax_tile<CAP, EXT, T::kDimTiles>(S, O, m, l, sm, need_mask, tb, h, wr.qpos, W_, pB, mc, mask_word);
+        softmax_tile<CAP, EXT>(S, O, m, l, sm, need_mask, tb, h, wr.qpos, W_, pB, mc, mask_word);
         // independent accumulator chains (dim tiles), issued round-robin
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
           for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-            for (int d = 0; d < T::kDimTiles; ++d) {
+            for (int d = 0; d < kDimTiles; ++d) {
               const char* vt = lds_v + voff[d] + (mt * 32 + kk * 16) * kRowB;
               const u32x2_t lo = lds_tr16(vt);
               const u32x2_t hi = lds_tr16(vt + 8 * kRowB);
@@ -213,8 +209,8 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
     if (tb + kBN >= t_hi) break;
     tile_step(lds_k1, lds_v1, lds_k0, lds_v0, tb + kBN);
   }
-  if (a.kv_splits > 1) write_partial_rows<T::kDimTiles>(a, w, wr, O, l, h, m * sm.sc2, split);
-  else write_rows<T::kDimTiles>(a, w, wr, O, l, h, m * sm.sc2);
+  if (a.kv_splits > 1) write_partial_rows(a, w, wr, O, l, h, m * sm.sc2, split);
+  else write_rows(a, w, wr, O, l, h, m * sm.sc2);
 }
 
 }  // namespace
@@ -779,7 +775,7 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const Prefil
   if (W_ > 0) t_lo = max(0, w.prefix + w.q_start - W_ + 1) & ~(kBN - 1);
   int split = 0;
   if (a.kv_splits > 1 && !kv_piece(a, t_lo, t_hi, split)) {  // under-filled launch, nothing left for this piece
-    write_empty_partial_rows<4>(a, w, wr, h, split);
+    write_empty_partial_rows(a, w, wr, h, split);
     return;
   }
 
@@ -835,7 +831,7 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const Prefil
     }
     __syncthreads();
   }
-  if (a.kv_splits > 1) write_partial_rows<4>(a, w, wr, O, l, h, m * sm.sc2, split);
+  if (a.kv_splits > 1) write_partial_rows(a, w, wr, O, l, h, m * sm.sc2, split);
   else write_rows(a, w, wr, O, l, h, m * sm.sc2);
 }
 

@@ -14,6 +14,16 @@ namespace pf {
 constexpr int kBM = 128;  // query rows per workgroup
 constexpr int kBN = 64;   // kv tokens per tile
 
+// A tile of 128-wide heads in LDS: rows stay row-major and unpadded (256-wide heads have a kernel and a layout of their own)
+constexpr int kHeadDim = 128;
+constexpr int kRowB = kHeadDim * 2;      // one K or V row of a head, bf16
+constexpr int kTileB = kBN * kRowB;      // 16 KiB
+constexpr int kChunks = kHeadDim / 8;    // 16-byte chunks per row
+constexpr int kSteps = kHeadDim / 16;    // k-steps of the first product
+constexpr int kDimTiles = kHeadDim / 32; // 32-dim output tiles of the second product
+constexpr int kCopies = kChunks / 4;     // copy instructions per wave, for K and for V
+constexpr int kRowsPerCopy = 64 / kChunks;
+
 __device__ __forceinline__ u32x4_t lds_ld16(const char* p) { return *reinterpret_cast<const u32x4_t*>(p); }
 __device__ __forceinline__ void lds_st16(char* p, u32x4_t v) { *reinterpret_cast<u32x4_t*>(p) = v; }
 
@@ -196,15 +206,14 @@ constexpr float kMaskRaw = -3.0e38f;
 // of O happens a handful of times per row instead of once per tile.
 constexpr float kMaxSlack = 8.0f;
 
-template <int ND>
-__device__ __forceinline__ void update_running_max(float mx, float& m, float& l, f32x16_t (&O)[ND], float sc2) {
+__device__ __forceinline__ void update_running_max(float mx, float& m, float& l, f32x16_t (&O)[kDimTiles], float sc2) {
   if (__builtin_amdgcn_ballot_w64((mx - m) * sc2 > kMaxSlack) != 0) {
     const float m_new = fmaxf(m, mx);
     const float alpha = fast_exp2((m - m_new) * sc2);
     m = m_new;
     l *= alpha;
 #pragma unroll
-    for (int d = 0; d < ND; ++d)
+    for (int d = 0; d < kDimTiles; ++d)
 #pragma unroll
       for (int v = 0; v < 16; ++v) O[d][v] *= alpha;
   }
@@ -252,8 +261,8 @@ __device__ __forceinline__ MaskCtx make_mask_ctx(const PrefillArgs& a, const Wor
 // caller fetches at the top of the tile's step, in FRONT of the next tile's copy: loads return in order, so
 // the wait for it leaves the copy in flight.  Without the bits, one 4-byte load per score, here, behind the
 // first product (which waits for the copy as well).
-template <bool CAP, bool EXT, int ND = 4>
-__device__ __forceinline__ void softmax_tile(f32x16_t (&S)[2], f32x16_t (&O)[ND], float& m, float& l,
+template <bool CAP, bool EXT>
+__device__ __forceinline__ void softmax_tile(f32x16_t (&S)[2], f32x16_t (&O)[kDimTiles], float& m, float& l,
                                              const Softmax<CAP>& sm, bool need_mask, int tb, int h, int qpos,
                                              int window, u32x4_t (&pB)[2][2], const MaskCtx& mc,
                                              uint64_t mask_word = 0) {
@@ -267,18 +276,6 @@ __device__ __forceinline__ void softmax_tile(f32x16_t (&S)[2], f32x16_t (&O)[ND]
 #pragma unroll
         for (int v = 0; v < 16; ++v)
           S[mt][v] = __builtin_fmaf(__builtin_amdgcn_rcpf(fast_exp2(S[mt][v] * k1) + 1.0f), -2.0f * k2, k2);
-    } else if constexpr (ND != 4) {
-      // 256-wide heads, logits that are rounded: one loop with run-time choices
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          float x = S[mt][v] * sm.scale;
-          if (sm.cap != 0.f) x = soft_cap_f(x, sm.cap, sm.inv_cap);
-          x = x * sm.temp;
-          if (sm.round_mode) x = round_logit(x, sm.round_mode);
-          S[mt][v] = x * kLog2e;
-        }
     } else {
       // the general path: soft cap (if any), temperature, then the logit rounded to the softmax dtype.  One loop
       // per combination, so that no score pays for a choice that is the same for the whole call.
@@ -305,7 +302,7 @@ __device__ __forceinline__ void softmax_tile(f32x16_t (&S)[2], f32x16_t (&O)[ND]
       }
     }
   }
-  if (EXT && ND == 4 && need_mask && mc.mode == 1 && mc.bits) {  // (128-wide heads: the 256-wide kernels have no register to spare)
+  if (EXT && need_mask && mc.mode == 1 && mc.bits) {
     // the caller's mask as bits: the tile's 64 tokens are one word, fetched by the caller at the top of the step
     const uint32_t half[2] = {(uint32_t)mask_word >> (4 * h), (uint32_t)(mask_word >> 32) >> (4 * h)};
 #pragma unroll
@@ -338,7 +335,7 @@ __device__ __forceinline__ void softmax_tile(f32x16_t (&S)[2], f32x16_t (&O)[ND]
     else mx = __builtin_fmaxf(mx, S[1][v]);
   }
   mx = swap_max(mx);
-  update_running_max<ND>(mx, m, l, O, sm.sc2);
+  update_running_max(mx, m, l, O, sm.sc2);
   const float neg_m = -m * sm.sc2;
   // probabilities go straight into bf16 pairs (the B operands of the second product); the row
   // sum is taken over the rounded pairs, one dot instruction per pair
@@ -363,16 +360,15 @@ __device__ __forceinline__ void softmax_tile(f32x16_t (&S)[2], f32x16_t (&O)[ND]
 }
 
 // lane (c, h) holds query row c, dims 32d + 8*(v/4) + 4h + v%4 in O[d][v]
-template <int ND = 4>
 __device__ __forceinline__ void write_rows(const PrefillArgs& a, const Work& w, const WaveRows& wr,
-                                           const f32x16_t (&O)[ND], float l, int h, float m2) {
+                                           const f32x16_t (&O)[kDimTiles], float l, int h, float m2) {
   l += __shfl_xor(l, 32);
   if (!wr.active || wr.row >= w.q_len) return;
   const float vs = a.v_scale ? scalar_load_f32(a.v_scale + w.hk) : 1.0f;
   const float inv = a.sm.sink ? vs * sink_inverse(m2, l, sink_logit(a.sm.sink, a.sm.round_logits, w.head)) : vs / l;
   uint16_t* op = a.out + ((int64_t)(w.qg0 + wr.row) * a.Hq + w.head) * a.q_dim + 4 * h;
 #pragma unroll
-  for (int d = 0; d < ND; ++d)
+  for (int d = 0; d < kDimTiles; ++d)
 #pragma unroll
     for (int vq = 0; vq < 4; ++vq) {
       if (d * 32 + vq * 8 >= a.q_dim) break;
@@ -432,16 +428,15 @@ __device__ __forceinline__ bool kv_piece(const PrefillArgs& a, int& t_lo, int& t
 }
 
 // lane (c, h) holds query row c, dims 32d + 8*(v/4) + 4h + v%4 in O[d][v]
-template <int ND>
 __device__ __forceinline__ void write_partial_rows(const PrefillArgs& a, const Work& w, const WaveRows& wr,
-                                                   const f32x16_t (&O)[ND], float l, int h, float m2, int split) {
+                                                   const f32x16_t (&O)[kDimTiles], float l, int h, float m2, int split) {
   typedef float f32x4_t __attribute__((ext_vector_type(4)));
   l += __shfl_xor(l, 32);
   if (!wr.active || wr.row >= w.q_len) return;
   const int64_t slot = ((int64_t)(w.qg0 + wr.row) * a.Hq + w.head) * a.kv_splits + split;
-  float* op = a.ws_o + slot * (ND * 32) + 4 * h;
+  float* op = a.ws_o + slot * kHeadDim + 4 * h;
 #pragma unroll
-  for (int d = 0; d < ND; ++d)
+  for (int d = 0; d < kDimTiles; ++d)
 #pragma unroll
     for (int vq = 0; vq < 4; ++vq)
       *reinterpret_cast<f32x4_t*>(op + d * 32 + vq * 8) =
@@ -452,13 +447,12 @@ __device__ __forceinline__ void write_partial_rows(const PrefillArgs& a, const W
   }
 }
 
-template <int ND>
 __device__ __forceinline__ void write_empty_partial_rows(const PrefillArgs& a, const Work& w, const WaveRows& wr, int h,
                                                          int split) {
-  f32x16_t zero[ND];
+  f32x16_t zero[kDimTiles];
 #pragma unroll
-  for (int d = 0; d < ND; ++d) zero[d] = kZero16;
-  write_partial_rows<ND>(a, w, wr, zero, 0.f, h, kNoReference, split);
+  for (int d = 0; d < kDimTiles; ++d) zero[d] = kZero16;
+  write_partial_rows(a, w, wr, zero, 0.f, h, kNoReference, split);
 }
 
 // Merge the kv_splits partial rows of one (query token, query head): out = sum_j O_j 2^(m_j - m*) /
@@ -568,37 +562,24 @@ inline int kv_pieces(const PrefillArgs& a, int nseq, int bm, int heads, double t
 }
 
 // ==================================================================== async path (bf16 cache)
-// Geometry of a tile for head dim HD (128 or 256): rows stay row-major and unpadded in LDS.
-template <int HD>
-struct Tile {
-  static constexpr int kRowB = HD * 2;          // one K or V row of a head, bf16
-  static constexpr int kTileB = kBN * kRowB;    // 16 or 32 KiB
-  static constexpr int kChunks = HD / 8;        // 16-byte chunks per row
-  static constexpr int kSteps = HD / 16;        // k-steps of the first product
-  static constexpr int kDimTiles = HD / 32;     // 32-dim output tiles of the second product
-  static constexpr int kCopies = kChunks / 4;   // copy instructions per wave, for K and for V
-  static constexpr int kRowsPerCopy = 64 / kChunks;
-};
-
 // 16-byte chunk j of row t sits at chunk position j ^ swizzle(t):
 //   K: swizzle = t & 15      (ds_read_b128: 16 consecutive tokens -> 16 distinct chunk columns)
 //   V: swizzle = 4 * (t & 3) (transposing read: 4 consecutive tokens -> 4 distinct 64-byte windows)
-template <bool UNIFORM, int HD>
+template <bool UNIFORM>
 struct AsyncPages {
-  int32_t id[UNIFORM ? 1 : Tile<HD>::kCopies];
+  int32_t id[UNIFORM ? 1 : kCopies];
 };
 
-template <bool UNIFORM, int HD>
-__device__ __forceinline__ void async_fetch_pages(AsyncPages<UNIFORM, HD>& pg, const TileSrc& s, int tb, int wave,
+template <bool UNIFORM>
+__device__ __forceinline__ void async_fetch_pages(AsyncPages<UNIFORM>& pg, const TileSrc& s, int tb, int wave,
                                                   int lane) {
-  using T = Tile<HD>;
   tb = min(tb, s.last_tok & ~(kBN - 1));
   if constexpr (UNIFORM) {
     pg.id[0] = scalar_load_i32(s.pages + __builtin_amdgcn_readfirstlane(page_slot(s, tb)));
   } else {
 #pragma unroll
-    for (int n = 0; n < T::kCopies; ++n) {
-      const int t = (wave * T::kCopies + n) * T::kRowsPerCopy + lane / T::kChunks;
+    for (int n = 0; n < kCopies; ++n) {
+      const int t = (wave * kCopies + n) * kRowsPerCopy + lane / kChunks;
       pg.id[n] = s.pages[page_slot(s, min(tb + t, s.last_tok))];
     }
   }
@@ -608,30 +589,26 @@ __device__ __forceinline__ void async_fetch_pages(AsyncPages<UNIFORM, HD>& pg, c
 // lane of the tile, i.e. row p / kChunks, chunk column p % kChunks.  For a full tile inside one
 // page the byte offset of a lane's chunk from the tile's first row never changes: it is computed
 // once (AsyncOffsets) and a copy costs no vector ALU work, only a scalar tile base.
-template <int HD>
 struct AsyncOffsets {
-  uint32_t k[Tile<HD>::kCopies], v[Tile<HD>::kCopies];
+  uint32_t k[kCopies], v[kCopies];
 };
 
-template <int HD>
-__device__ __forceinline__ AsyncOffsets<HD> make_async_offsets(const KvAddr& kv, int wave, int lane) {
-  using T = Tile<HD>;
-  AsyncOffsets<HD> o;
-  const int cp = lane % T::kChunks;
+__device__ __forceinline__ AsyncOffsets make_async_offsets(const KvAddr& kv, int wave, int lane) {
+  AsyncOffsets o;
+  const int cp = lane % kChunks;
 #pragma unroll
-  for (int n = 0; n < T::kCopies; ++n) {
-    const int t = (wave * T::kCopies + n) * T::kRowsPerCopy + lane / T::kChunks;
+  for (int n = 0; n < kCopies; ++n) {
+    const int t = (wave * kCopies + n) * kRowsPerCopy + lane / kChunks;
     o.k[n] = (uint32_t)(t * kv.tok_stride + ((cp ^ (t & 15)) << 4));
     o.v[n] = (uint32_t)(t * kv.tok_stride + ((cp ^ ((t & 3) << 2)) << 4));
   }
   return o;
 }
 
-template <bool UNIFORM, int HD>
+template <bool UNIFORM>
 __device__ __forceinline__ void async_copy_tile(char* lds_k, char* lds_v, const TileSrc& s, const KvAddr& kv,
                                                 const char* kh, const char* vh, int tb, int wave, int lane,
-                                                const AsyncPages<UNIFORM, HD>& pg, const AsyncOffsets<HD>& ofs) {
-  using T = Tile<HD>;
+                                                const AsyncPages<UNIFORM>& pg, const AsyncOffsets& ofs) {
   typedef const __attribute__((address_space(1))) void* gptr_t;
   typedef __attribute__((address_space(3))) void* lptr_t;
   tb = min(tb, s.last_tok & ~(kBN - 1));  // past the end: re-copy the last tile
@@ -642,8 +619,8 @@ __device__ __forceinline__ void async_copy_tile(char* lds_k, char* lds_v, const 
       const char* kb = kh + base;
       const char* vb = vh + base;
 #pragma unroll
-      for (int n = 0; n < T::kCopies; ++n) {
-        const int blk = wave * T::kCopies + n;
+      for (int n = 0; n < kCopies; ++n) {
+        const int blk = wave * kCopies + n;
         __builtin_amdgcn_global_load_lds((gptr_t)(kb + ofs.k[n]), (lptr_t)(lds_k + blk * 1024), 16, 0, 0);
         __builtin_amdgcn_global_load_lds((gptr_t)(vb + ofs.v[n]), (lptr_t)(lds_v + blk * 1024), 16, 0, 0);
       }
@@ -651,11 +628,11 @@ __device__ __forceinline__ void async_copy_tile(char* lds_k, char* lds_v, const 
     }
   }
   // last, partial tile (rows clamped to the last valid token) or pages smaller than a tile
-  const int cp = lane % T::kChunks;
+  const int cp = lane % kChunks;
 #pragma unroll
-  for (int n = 0; n < T::kCopies; ++n) {
-    const int blk = wave * T::kCopies + n;
-    const int t = blk * T::kRowsPerCopy + lane / T::kChunks;
+  for (int n = 0; n < kCopies; ++n) {
+    const int blk = wave * kCopies + n;
+    const int t = blk * kRowsPerCopy + lane / kChunks;
     const int64_t ro = row_offset<UNIFORM>(s, kv, tb, tb + t, pg.id[UNIFORM ? 0 : n]);
     const int jk = cp ^ (t & 15);
     const int jv = cp ^ ((t & 3) << 2);

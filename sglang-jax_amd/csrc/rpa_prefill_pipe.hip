@@ -46,8 +46,6 @@ using namespace pf;
 
 namespace {
 
-constexpr int kRowB = 256;               // bytes of one K or V row of a head
-constexpr int kTileB = kBN * kRowB;      // 16 KiB
 constexpr int kHalfB = 32 * kRowB;       // byte distance between the halves of a tile
 constexpr int kKSlot = 0;                // ring slots inside the LDS array: K0 K1 V0 V1
 constexpr int kVSlot = 2 * kTileB;
@@ -343,7 +341,7 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
         wr.active = wr.r_lo < w.q_len;
         wr.row = wr.r_lo + c;
         wr.qpos = w.prefix + wr.row;
-        write_empty_partial_rows<4>(a, w, wr, h, split);
+        write_empty_partial_rows(a, w, wr, h, split);
       }
       return;
     }
@@ -404,7 +402,7 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
     for (int ks = 0; ks < 8; ++ks) sh.koff[ks] = (int)lds_base + kKSlot + k_row + ((ks * 32) ^ k_swz);
 #pragma unroll
     for (int d = 0; d < 4; ++d) sh.voff[d] = (int)lds_base + kVSlot + v_row + v_in + ((d * 64) ^ v_swz);
-    const AsyncOffsets<128> ofs = make_async_offsets<128>(a.kv, wave, lane);
+    const AsyncOffsets ofs = make_async_offsets(a.kv, wave, lane);
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       sh.ofs_k[n] = ofs.k[n];
@@ -522,8 +520,8 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
     wr.active = wr.r_lo < w.q_len;
     wr.row = wr.r_lo + c;
     wr.qpos = b[q].qpos;
-    if constexpr (SPLIT) write_partial_rows<4>(a, w, wr, b[q].O, b[q].l, h, b[q].seen != 0.f ? b[q].m : kNoReference, split);
-    else write_rows<4>(a, w, wr, b[q].O, b[q].l, h, b[q].m);
+    if constexpr (SPLIT) write_partial_rows(a, w, wr, b[q].O, b[q].l, h, b[q].seen != 0.f ? b[q].m : kNoReference, split);
+    else write_rows(a, w, wr, b[q].O, b[q].l, h, b[q].m);
   }
 }
 
