@@ -205,7 +205,7 @@ def test_metadata_in_one_upload(pkg, gpu, P, lens, mixed):
 @pytest.mark.parametrize("lens", [[1003], [130, 1, 70, 300, 64], [2500, 129]])
 def test_prompts_attend_to_the_rows_they_bring(pkg, gpu, P, D, Hq, Hkv, dtype, window, cap, lens):
     """Prompts without a prefix read the caller's keys and values and fill the cache beside the attention; the functional
-    operator on the same batch writes first and reads the cache."""
+    operator on the same batch writes first and reads the cache.  Both against 64 bits."""
     gen = torch.Generator().manual_seed(3)
     rng = np.random.default_rng(4)
     kv = np.array(lens, dtype=np.int32)
@@ -231,11 +231,14 @@ def test_prompts_attend_to_the_rows_they_bring(pkg, gpu, P, D, Hq, Hkv, dtype, w
     torch.cuda.synchronize()
     assert torch.equal(cache.view(torch.uint8), other.view(torch.uint8))
     assert_parity(out.view(T, Hq, D).cpu().float(), want.cpu().float(), **TOL)
+    exact = attention64(q, k, v, lens, D ** -0.5, window, cap)
+    assert_parity(out.view(T, Hq, D), exact, **TOL)
+    assert_parity(want, exact, **TOL)
 
 
-def attention64(q, k, v, lens, scale, window=None):
+def attention64(q, k, v, lens, scale, window=None, cap=None):
     """Prompts without a prefix in 64 bits: [T, Hq, D] of q [T, Hq, D], k / v [T, Hkv, D]."""
-    q, k, v = q.cpu().double(), k.cpu().double(), v.cpu().double()
+    q, k, v = (x.cpu().float().double() for x in (q, k, v))
     g = q.shape[1] // k.shape[1]
     out, at = [], 0
     for n in lens:
@@ -243,6 +246,7 @@ def attention64(q, k, v, lens, scale, window=None):
         at += n
         kk, vv = (x[s].repeat_interleave(g, dim=1).transpose(0, 1) for x in (k, v))
         x = q[s].transpose(0, 1) @ kk.transpose(1, 2) * scale
+        x = cap * torch.tanh(x / cap) if cap else x
         row, col = torch.arange(n)[:, None], torch.arange(n)[None, :]
         x = x.masked_fill((col > row) | (col <= row - (window or n + 1)), -torch.inf)
         out.append((torch.softmax(x, dim=-1) @ vv).transpose(0, 1))
