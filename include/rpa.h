@@ -14,6 +14,8 @@
  *     the legacy default stream), so calls are graph-capturable;
  *   - functions return RPA_OK (0) or a negative RpaStatus; rpa_last_error()
  *     returns a thread-local, human readable description of the last failure;
+ *   - calls may come from several threads; the launches of two calls on one workspace do not mix, but
+ *     calls that share a workspace are still ordered by the caller: on one stream, or by events;
  *   - metadata (kv_lens, page_indices, cu_q_lens, cu_kv_lens) is read on the
  *     device only.  Host copies can be checked with rpa_validate_host().
  */

@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 
 #include "../../include/rpa.h"
 #include "rpa_kernels.h"
@@ -80,6 +81,19 @@ int fail(int code, const char* fmt, ...) {
   va_end(ap);
   return code;
 }
+
+// Held while a call's launches are enqueued: several threads may share a stream and with it a workspace, and between the
+// launch that leaves partial rows there and the one that merges them no other call's may come.
+class WorkspaceTurn {
+ public:
+  explicit WorkspaceTurn(const void* workspace) {
+    static std::mutex turns[16];
+    if (workspace) lock_ = std::unique_lock<std::mutex>(turns[(reinterpret_cast<uintptr_t>(workspace) >> 9) & 15]);
+  }
+
+ private:
+  std::unique_lock<std::mutex> lock_;
+};
 
 constexpr float kDefaultMask = -0.7f * 3.4028234663852886e38f;
 
@@ -771,7 +785,9 @@ int rpa_decode(const RpaParams* given, void* stream) {
   const OwnParams in(given);
   const RpaParams* p = in.p;
   const int rc = rpa_validate(p);
-  return rc != RPA_OK ? rc : decode_rows(p, nullptr, nullptr, false, stream);
+  if (rc != RPA_OK) return rc;
+  const WorkspaceTurn turn(p->workspace);
+  return decode_rows(p, nullptr, nullptr, false, stream);
 }
 
 static rpa::KvWriteArgs kv_write_args(const RpaParams* p, const void* keys, const void* values) {
@@ -923,10 +939,18 @@ int rpa_upload_words(int32_t* dst, const int32_t* src, int32_t n, void* stream) 
   return check_hip(rpa::launch_upload(dst, src, n, static_cast<hipStream_t>(stream)), "rpa_upload_words");
 }
 
+// The new tokens are in the cache already.
+static int prefill_cached(const RpaParams* p, void* stream) {
+  if (!p || !p->prompts_only) return prefill_run(p, nullptr, nullptr, stream);
+  RpaParams q = *p;
+  q.prompts_only = 0;
+  return prefill_run(&q, nullptr, nullptr, stream);
+}
+
 int rpa_prefill(const RpaParams* given, void* stream) {
-  OwnParams in(given);
-  in.own.prompts_only = 0;  // the new tokens are in the cache already
-  return prefill_run(in.p, nullptr, nullptr, stream);
+  const OwnParams in(given);
+  const WorkspaceTurn turn(in.p ? in.p->workspace : nullptr);
+  return prefill_cached(in.p, stream);
 }
 
 int rpa_mask_needs_starts(const RpaParams* given) {
@@ -971,6 +995,7 @@ int rpa_attention_update(const RpaParams* given, const void* keys, const void* v
   int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
   if (!keys != !values) return fail(RPA_EINVAL_NULL, "keys and values must be given together");
+  const WorkspaceTurn turn(p->workspace);
   if (takes_token_rows(p) && p->workspace_bytes >= token_row_workspace(p)) {
     const bool with_rows = keys && rows_take_new_tokens(p);
     if (keys && !with_rows && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
@@ -981,7 +1006,7 @@ int rpa_attention_update(const RpaParams* given, const void* keys, const void* v
   if (keys && !fused && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
   if ((rc = decode_rows(p, fused ? keys : nullptr, fused ? values : nullptr, false, stream)) != RPA_OK) return rc;
   if (fused && (rc = write_new_tokens(p, keys, values, true, stream)) != RPA_OK) return rc;
-  return rpa_prefill(p, stream);
+  return prefill_cached(p, stream);
 }
 
 int rpa_attention(const RpaParams* p, void* stream) { return rpa_attention_update(p, nullptr, nullptr, stream); }
@@ -1276,9 +1301,15 @@ int rpa_mla_describe_plan(const RpaMlaParams* p, int token_rows, char* buf, size
                   mla_workspace(p, rows, token_rows != 0));
 }
 
-int rpa_mla_decode(const RpaMlaParams* p, void* stream) { return mla_run(p, stream, false); }
+int rpa_mla_decode(const RpaMlaParams* p, void* stream) {
+  const WorkspaceTurn turn(p ? p->workspace : nullptr);
+  return mla_run(p, stream, false);
+}
 
-int rpa_mla_attention(const RpaMlaParams* p, void* stream) { return mla_run(p, stream, true); }
+int rpa_mla_attention(const RpaMlaParams* p, void* stream) {
+  const WorkspaceTurn turn(p ? p->workspace : nullptr);
+  return mla_run(p, stream, true);
+}
 
 int rpa_mla_kv_write(const RpaMlaParams* p, const void* new_kv_c, const void* new_k_pe, void* stream) {
   int rc = mla_validate(p);
@@ -1306,6 +1337,7 @@ int rpa_mla_kv_write(const RpaMlaParams* p, const void* new_kv_c, const void* ne
 
 int rpa_mla_attention_update(const RpaMlaParams* p, const void* new_kv_c, const void* new_k_pe, int token_rows,
                              void* stream) {
+  const WorkspaceTurn turn(p ? p->workspace : nullptr);
   if (new_kv_c || new_k_pe) {
     const int rc = rpa_mla_kv_write(p, new_kv_c, new_k_pe, stream);
     if (rc != RPA_OK) return rc;
@@ -1374,6 +1406,7 @@ int rpa_mla_sparse_attention(const RpaMlaParams* p, const RpaMlaSparse* s, const
   const SparseLayout l = sparse_layout(p, s, v);
   if (!p->workspace || p->workspace_bytes < l.total || (reinterpret_cast<uintptr_t>(p->workspace) & 15) != 0)
     return fail(RPA_EINVAL_WORKSPACE, "workspace of %zu bytes needed (aligned to 16), %zu given", l.total, p->workspace_bytes);
+  const WorkspaceTurn turn(p->workspace);
   char* ws = static_cast<char*>(p->workspace);
   rpa::SparseMlaArgs a;
   a.pt.kv_lens = p->kv_lens;

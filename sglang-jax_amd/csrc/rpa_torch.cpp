@@ -25,8 +25,9 @@
 
 namespace {
 
-// ---- the workspace, shared with the Python side (`workspace()` below); touched under the GIL only
-at::Tensor& workspace(const at::Device& dev, void* stream, size_t bytes) {
+// ---- the workspace, shared with the Python side (`workspace()` below); the map is touched under the GIL only.  A call holds
+// on to the buffer it was given: without the GIL, while it launches, another thread's call on the same stream may grow it.
+at::Tensor workspace(const at::Device& dev, void* stream, size_t bytes) {
   static auto* pool = new std::map<std::pair<int, void*>, at::Tensor>;  // never destroyed: tensors outlive no device
   at::Tensor& t = (*pool)[{dev.index(), stream}];
   if (!t.defined() || (size_t)t.numel() < bytes)
@@ -310,8 +311,9 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   p.kv_dtype = kv_type == at::kBFloat16 ? RPA_KV_BF16 : RPA_KV_FP8_E4M3;
   COMMON(!rpa_mask_needs_starts(&p));
   p.prompts_only = keys.defined() && PyObject_IsTrue(a[28]) == 1;
+  at::Tensor ws;
   if (const size_t need = rpa_workspace_bytes(&p)) {
-    at::Tensor& ws = workspace(dev, stream, need);
+    ws = workspace(dev, stream, need);
     p.workspace = ws.data_ptr();
     p.workspace_bytes = (size_t)ws.numel();
   }
@@ -433,8 +435,9 @@ PyObject* mla(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   p.cu_q_lens = cu_q->const_data_ptr<int32_t>();
   p.distribution = dist.device;
   p.num_seqs = dist.device ? (int32_t)kv_lens->size(0) : (int32_t)dist.k;
+  at::Tensor ws;
   if (const size_t need = decode_only ? rpa_mla_workspace_bytes(&p) : rpa_mla_attention_workspace_bytes(&p)) {
-    at::Tensor& ws = workspace(dev, stream, need);
+    ws = workspace(dev, stream, need);
     p.workspace = ws.data_ptr();
     p.workspace_bytes = (size_t)ws.numel();
   }
@@ -487,7 +490,7 @@ PyObject* sparse_mla(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   void* stream = stream_of(dev);
   p.out = out.data_ptr();
   const size_t need = rpa_mla_sparse_workspace_bytes(&p, &s);
-  at::Tensor& ws = workspace(dev, stream, need);
+  const at::Tensor ws = workspace(dev, stream, need);
   p.workspace = ws.data_ptr();
   p.workspace_bytes = (size_t)ws.numel();
   const int rc = without_gil([&] { return rpa_mla_sparse_attention(&p, &s, x.new_c_ptr(), x.new_r_ptr(), stream); });

@@ -339,3 +339,50 @@ def test_metadata_inside_a_captured_graph(pkg, gpu):
         torch.cuda.synchronize()
         assert np.array_equal(md.page_indices.cpu().numpy(), want["page_indices"])
         assert np.array_equal(md.cu_kv_lens.cpu().numpy(), want["cu_kv_lens"])
+
+
+def test_threads_share_a_stream_and_its_workspace(pkg, gpu):
+    """Layer calls of two threads on one stream: the launches of a call (partial rows, then their merge) stay together on the
+    workspace that they share, and a call keeps the buffer it was given while the other one's grows it."""
+    import threading
+
+    Hq, Hkv, D, P = 8, 2, 128, 64
+    stream = torch.cuda.Stream(gpu)
+
+    def prepare(seed, lens):
+        gen = torch.Generator().manual_seed(seed)
+        kv = np.array(lens, dtype=np.int32)
+        n = int((-(-kv // P)).sum())
+        pages = np.random.default_rng(seed).permutation(n).astype(np.int32)
+        loc = (pages.astype(np.int64)[:, None] * P + np.arange(P)).reshape(-1).astype(np.int32)
+        cache = torch.randn(n, P, 2 * Hkv, D, generator=gen).to(torch.bfloat16).to(gpu)
+        q, k, v = (torch.randn(len(lens), h * D, generator=gen).to(torch.bfloat16).to(gpu) for h in (Hq, Hkv, Hkv))
+        backend = pkg.FlashAttention(Hq, Hkv, D, page_size=P, device=gpu)
+        batch = SimpleNamespace(forward_mode=pkg.ForwardMode.DECODE, seq_lens=kv, cache_loc=loc, extend_seq_lens=None, dp_size=1,
+                                per_dp_bs_size=len(lens))
+        backend.forward_metadata = backend.get_forward_metadata(batch)
+        layer = SimpleNamespace(layer_id=0, scaling=D ** -0.5, head_dim=D, sliding_window_size=None, logit_cap=None)
+        pool = SimpleNamespace(get_fused_kv_buffer=lambda i: cache)
+        return lambda: backend(q, k, v, layer, batch, pool)[0]
+
+    rng = np.random.default_rng(2)
+    calls = [prepare(1, [3000, 4100]), prepare(2, [int(x) for x in rng.integers(600, 6000, size=90)])]
+    torch.cuda.synchronize()
+    want = [c() for c in calls]
+    torch.cuda.synchronize()
+    got = [[], []]
+
+    def work(i):
+        with torch.cuda.stream(stream):
+            for _ in range(150):
+                got[i].append(calls[i]())
+
+    say("two threads on one stream")
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert len(got[i]) == 150 and all(torch.equal(x, want[i]) for x in got[i])
