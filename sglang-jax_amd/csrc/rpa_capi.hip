@@ -806,7 +806,8 @@ static rpa::KvWriteArgs kv_write_args(const RpaParams* p, const void* keys, cons
 }
 
 // Whether a call's chunks are prompts whose keys and values, every token of them, the caller brings along: the kernels
-// then read those rows and not the cache (whatever its pages are like), and write the cache beside the attention.
+// then read those rows and not the cache, and write the cache beside the attention.  (1003 tokens x 8 heads on 16-token
+// pages 32.2 -> 24.3 us, on pages of 64, which the assembly kernel takes, 27.0 -> 22.1.)
 static bool takes_fresh_prompts(const RpaParams* p) {
   return p->prompts_only && !p->distribution && p->decode_end == 0 && p->mask_mode != RPA_MASK_CUSTOM && q_dim_of(p) == p->head_dim &&
          p->num_seqs > 0 && p->num_tokens > 0 && !(p->head_dim == 256 && rpa::tuning().prefill_rows256 != 0) &&

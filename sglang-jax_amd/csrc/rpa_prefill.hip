@@ -222,12 +222,13 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
 // before, a lone wave per SIMD had its operand reads and its exponentials exposed, and the compiler moved operands through
 // the accumulation registers and drained the loads in flight to make room.  The price is LDS: every wave reads the whole
 // K and V tile, 512 KiB per tile and CU, 2300 clocks (3.7 per ds_read_b128, 2.6 per transposing read) against 2048 of the
-// matrix pipe.  Counters (e4m3, soft cap, window): LDS 31 %, vector pipe 30 %, matrix pipe 20 % of the clocks, a quarter
-// lost to the packing of 704 workgroups on 256 CUs: no pipe is full, the waves of a CU go through its phases together.
+// matrix pipe.  Counters (e4m3, soft cap, window): LDS 27 %, vector pipe 26 %, matrix pipe 17 % of the launch's clocks, for
+// 64 % of which the CUs hold their waves (704 workgroups on 256 CUs pack badly): no pipe is full, the waves of a CU go
+// through its phases together.
 // (Eight waves as pairs that share 32 positions, one set of scores each, and exchange their probabilities through LDS --
 // half the reads -- spilled 50 registers at 256: 423 us.)
-// Measured: 6 chunks of 300 .. 1500 tokens x 16 heads, e4m3, soft cap, window 1024 (89 GFLOP) 424 -> 258 us; 3 bf16 prompts of
-// 1490 .. 2883 tokens x 16 heads on 16-token pages 182 -> 135 us.
+// Measured: 6 chunks of 300 .. 1500 tokens x 16 heads, e4m3, soft cap, window 1024 (89 GFLOP) 424 -> 262 us; 3 bf16 prompts of
+// 1490 .. 2883 tokens x 16 heads on 16-token pages 198 -> 152 us with the cache write.
 namespace {
 
 constexpr int kWRowB = 512;                // a K or V row in LDS
@@ -545,14 +546,15 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_async_kernel_wide(const Pr
         u32x4_t p_next[2];
         probabilities(S, p_next);
         second_product(1);
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-#pragma unroll
-          for (int j = 0; j < 16; ++j) O[j] *= alpha;
-        }
         pB[0] = p_next[0];
         pB[1] = p_next[1];
 #pragma unroll
         for (int k = 0; k < 8; ++k) voff[k] ^= kWTileB;
+        // (here and not right behind the product: 3 bf16 prompts 153.7 -> 151.4 us, 64-token pages 375.6 -> 377.6)
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+          for (int j = 0; j < 16; ++j) O[j] *= alpha;
+        }
         meet();
       }
       second_product(0);
