@@ -1730,7 +1730,8 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
 
 // A few KB of host words as kernel arguments: the words ride in the packet's argument buffer and the store is one more
 // kernel of the stream, where a copy is a hand-over to a copy engine and back (five small copies of a step's metadata took
-// 20 us of host time and 4 us of the GPU's each).  Up to three launches; beyond, a copy costs less.
+// 20 us of host time and 4 us of the GPU's each).  Up to three launches; beyond, a copy costs less (host memory that is not
+// pinned is staged before the call returns).
 namespace {
 constexpr int kUploadWords = 896;  // 3.5 KB: under the 4 KB that arguments may take
 struct UploadWords {
@@ -1743,7 +1744,14 @@ __global__ __launch_bounds__(256) void rpa_upload_kernel(int32_t* dst, int n, co
 }  // namespace
 
 hipError_t launch_upload(int32_t* dst, const int32_t* src, int n, hipStream_t stream) {
-  if (n > 3 * kUploadWords) return hipMemcpyAsync(dst, src, (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, stream);
+  if (n > 3 * kUploadWords) {
+    // (not into a graph: a replay would read the host memory again, and the caller may have let go of it)
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(stream, &capture);
+    if (e != hipSuccess) return e;
+    if (capture == hipStreamCaptureStatusNone)
+      return hipMemcpyAsync(dst, src, (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, stream);
+  }
   UploadWords words;
   for (int at = 0; at < n; at += kUploadWords) {
     const int m = min(n - at, kUploadWords);

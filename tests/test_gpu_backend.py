@@ -317,10 +317,11 @@ def test_metadata_arrives_in_the_order_of_its_stream(pkg, gpu, mla):
         assert np.array_equal(x, want[name]), name
 
 
-def test_metadata_inside_a_captured_graph(pkg, gpu):
-    """Under capture the upload becomes part of the graph; every replay leaves the same words."""
-    P = 16
-    kv = np.array([40, 7, 100], dtype=np.int32)
+@pytest.mark.parametrize("P,lens", [(16, [40, 7, 100]), (1, [4000, 1, 2500])])
+def test_metadata_inside_a_captured_graph(pkg, gpu, P, lens):
+    """Under capture the upload becomes part of the graph, words and all (also more of them than an eager call sends as kernel
+    arguments); every replay leaves the same ones."""
+    kv = np.array(lens, dtype=np.int32)
     n = int((-(-kv // P)).sum())
     loc = (np.arange(n, dtype=np.int64)[::-1, None] * P + np.arange(P)).reshape(-1).astype(np.int32)
     batch = SimpleNamespace(forward_mode=pkg.ForwardMode.DECODE, seq_lens=kv, cache_loc=loc, extend_seq_lens=None, dp_size=1,
@@ -329,12 +330,13 @@ def test_metadata_inside_a_captured_graph(pkg, gpu):
     want = pkg.build_forward_metadata(forward_mode=pkg.ForwardMode.DECODE, seq_lens=kv, cache_loc=loc, page_size=P)
     backend.get_forward_metadata(batch)
     torch.cuda.synchronize()
-    say("metadata under capture")
+    say(f"metadata under capture P={P}")
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
         md = backend.get_forward_metadata(batch)
     for _ in range(3):
         md.page_indices.zero_()
+        backend.get_forward_metadata(batch)  # (eager work between the replays)
         g.replay()
         torch.cuda.synchronize()
         assert np.array_equal(md.page_indices.cpu().numpy(), want["page_indices"])
