@@ -388,3 +388,72 @@ def test_threads_share_a_stream_and_its_workspace(pkg, gpu):
     torch.cuda.synchronize()
     for i in range(2):
         assert len(got[i]) == 150 and all(torch.equal(x, want[i]) for x in got[i])
+
+
+FORMS = {
+    "plain": {}, "host_metadata": {}, "strided_new_tokens": {}, "narrow_cache_rows": {}, "f32_queries": {}, "cache_only": {},
+    "distribution_on_the_device": {}, "distribution_as_a_tuple": {}, "sink_per_head": {}, "scalar_sink": {},
+    "per_head_scales": {}, "scalar_scales": dict(k_scale=0.5, v_scale=2.0), "window": dict(sliding_window=np.int64(40)),
+    "cap": dict(soft_cap=20), "bf16_logits": dict(softmax_dtype=torch.bfloat16), "no_mask": dict(causal=0), "bool_mask": {},
+    "int_mask": {}, "bounds": dict(max_kv_len=np.int32(900), max_q_len=200, num_splits=3),
+    # refused, with the same words
+    "zero_window": dict(sliding_window=0), "zero_cap": dict(soft_cap=0.0), "positive_mask_value": dict(mask_value=1.0),
+    "f64_softmax": dict(softmax_dtype=torch.float64), "wrong_scales": {}, "wide_metadata": {}, "chunk_of_nothing": dict(chunk_prefill_size=0)}
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.bfloat16), (256, torch.float8_e4m3fn)])
+def test_native_calls_equal_the_general_ones(pkg, gpu, monkeypatch, form, D, dtype):
+    """The native reader of a call's arguments against the general Python code, over the forms that it takes or leaves to it:
+    the same rows and cache, or the same refusal."""
+    P, Hq, Hkv, lens, new = 16, 8, 2, [700, 31, 400, 260], [1, 1, 130, 200]
+    kv, cu = np.array(lens, dtype=np.int32), np.concatenate([[0], np.cumsum(new)]).astype(np.int32)
+    counts, T = -(-kv // P), sum(new)
+    n = int(counts.sum())
+    gen = torch.Generator().manual_seed(9)
+    rnd = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    rows = -(-D // 128) * 128 if form != "narrow_cache_rows" else D
+    cache = torch.zeros(n, P, 2 * Hkv, rows)
+    cache[..., :D] = rnd(n, P, 2 * Hkv, D)
+    cache = cache.to(dtype).to(gpu)
+    q = rnd(T, Hq, D).to(torch.float32 if form == "f32_queries" else torch.bfloat16).to(gpu)
+    kv_new = rnd(T, 2 * Hkv, D).to(dtype).to(gpu)
+    k, v = kv_new[:, :Hkv], kv_new[:, Hkv:]
+    if form != "strided_new_tokens":
+        k, v = k.contiguous(), v.contiguous()
+    if form == "cache_only":
+        k = v = None
+    meta = [kv, np.random.default_rng(1).permutation(n).astype(np.int32), cu, np.concatenate([[0], np.cumsum(counts * P)]).astype(np.int32)]
+    if form == "wide_metadata":
+        meta[0] = kv.astype(np.int64)
+    if form != "host_metadata":
+        meta = [torch.from_numpy(x).to(gpu) for x in meta]
+    dist = np.array([2, 2, 4], dtype=np.int32)
+    dist = {"distribution_on_the_device": torch.from_numpy(dist).to(gpu), "distribution_as_a_tuple": (2, 2, 4)}.get(form, dist)
+    mask = (torch.rand(int((np.array(new) * kv).sum()), generator=gen) < 0.7).to(gpu) if form.endswith("_mask") and form != "no_mask" else None
+    sink = {"sink_per_head": rnd(Hq).to(gpu), "scalar_sink": 0.5}.get(form)
+    kw = dict(sm_scale=D ** -0.5, **FORMS[form])
+    if mask is not None:
+        kw["causal"] = 0
+        mask = mask.to(torch.int32) if form == "int_mask" else mask
+    if form in ("per_head_scales", "wrong_scales"):
+        kw.update(k_scale=(torch.rand(Hkv + (form == "wrong_scales"), generator=gen) + 0.5).to(gpu), v_scale=(torch.rand(Hkv, generator=gen) + 0.5).to(gpu))
+    native = pkg._lib.load_torch()
+    general = SimpleNamespace(attention=lambda *a: None, workspace=native.workspace)
+    say(f"forms {form} D={D} {dtype}")
+    results = []
+    for module in (native, general):
+        monkeypatch.setattr(pkg._lib, "_torch", module)
+        own = cache.clone()
+        try:
+            out, _ = pkg.ragged_paged_attention(q, k, v, own, *meta, dist, mask, sink, **kw)
+            torch.cuda.synchronize()
+            results.append((out.cpu(), own.view(torch.uint8).cpu()))
+        except (ValueError, NotImplementedError) as e:
+            results.append((type(e), str(e)))
+    (a, b), (c, d) = results
+    if isinstance(b, str) or isinstance(d, str):
+        assert (a, b) == (c, d)
+        return
+    assert torch.equal(b, d) and a.dtype == c.dtype
+    assert_parity(a.float(), c.float(), **TOL)
