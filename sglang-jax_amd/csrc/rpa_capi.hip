@@ -52,6 +52,7 @@ const Tuning& tuning() {
   geti("RPA_PREFILL_PIPE_NQ", t.prefill_pipe_nq);
   geti("RPA_PREFILL_PIPE_MASKED", t.prefill_pipe_masked);
   geti("RPA_PREFILL_SPLITS", t.prefill_splits);
+  geti("RPA_PREFILL_PACKED", t.prefill_packed);
   geti("RPA_MLA_MIN_CHUNK", t.mla_min_chunk);
   geti("RPA_MLA_WG_CAPACITY", t.mla_wg_capacity);
   geti("RPA_MLA_BALANCED", t.mla_balanced);
@@ -861,6 +862,8 @@ static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a, const void* ke
     a.kv.page_stride = 0;  // (the id of the one page, whatever the table holds, adds nothing)
     a.pt.page_size = 1 << 30;  // (a.page_options stay the cache's)
   }
+  // (not where the caller pins the partition: such a call agrees bit for bit with one whose composition is on the device)
+  a.packed = p->num_splits == 0 ? rpa::prefill_packed_pieces(a) : 0;
   return true;
 }
 
@@ -1064,6 +1067,8 @@ int rpa_describe_plan(const RpaParams* given, char* buf, size_t len) {
       const PrefillWorkspace w = prefill_workspace(p_in, a);
       put("prefill: shape=%s kernel=%s tile=%dx%dx%d kv_pieces_with_workspace=%d mask_bits=%s optional_workspace=%zu\n",
           r.name, kernel, r.tile_q, r.tile_heads, r.tile_kv, w.splits, w.bits_bytes ? "yes" : "no", w.total);
+      if (a.packed)
+        put("prefill, small launch: kernel=rpa_prefill_packed_kernel instead, columns=%d tile=%dx%dx32\n", 32, 32 / a.G, a.G);
     }
   }
   const bool rows = takes_token_rows(p_in), prompts = !rows && takes_fresh_prompts(p_in);

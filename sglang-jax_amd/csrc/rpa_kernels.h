@@ -142,6 +142,7 @@ struct PrefillArgs {
   // rows, which would suit any: the assembly kernel rounds the scaled queries to bf16, and pages that it does not take
   // never had that
   uint32_t page_options;
+  int32_t packed;  // rpa_prefill_packed_kernel takes the call, K/V ranges in so many pieces where there is room for them; 0 = not
 };
 
 struct GatherArgs {
@@ -227,6 +228,7 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream);
 // How many pieces launch_prefill would cut the K/V ranges into if it had the workspace (1 = no cut), and the
 // bytes of workspace that takes.
 int prefill_kv_splits(const PrefillArgs& a);
+int prefill_packed_pieces(const PrefillArgs& a);
 size_t prefill_split_workspace_bytes(const PrefillArgs& a, int splits);
 // n host words to device memory, in stream order; the source may be reused at once
 hipError_t launch_upload(int32_t* dst, const int32_t* src, int n, hipStream_t stream);

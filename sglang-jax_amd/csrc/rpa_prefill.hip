@@ -881,11 +881,19 @@ __global__ __launch_bounds__(256) void rpa_mask_bits_kernel(const PrefillArgs a)
   uint64_t* out = a.mask_bits + (int64_t)token * a.mask_pitch;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int words = min((kv_len + 63) >> 6, a.mask_pitch);
-  for (int k = wave; k < words; k += 4) {
-    const int t = 64 * k + lane;
-    const int v = (t < kv_len) ? row[t] : 0;
-    const uint64_t keep = __ballot(v >= 1);
-    if (lane == 0) out[k] = keep;
+  // eight words of a wave requested at a time: one after the other, a row of 16000 was 60 round trips to memory
+  for (int k0 = wave; k0 < words; k0 += 32) {
+    int v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int t = 64 * (k0 + 4 * i) + lane;
+      v[i] = (t < kv_len) ? row[t] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint64_t keep = __ballot(v[i] >= 1);
+      if (lane == 0 && k0 + 4 * i < words) out[k0 + 4 * i] = keep;
+    }
   }
 }
 
@@ -915,11 +923,15 @@ const ShapeRule& prefill_shape_of(const PrefillArgs& a) {
 }
 
 int prefill_kv_splits(const PrefillArgs& a) {
+  return a.packed ? a.packed : prefill_unpacked_kv_splits(a, nullptr);
+}
+
+int prefill_unpacked_kv_splits(const PrefillArgs& a, double* us) {
   const int nseq = a.seq_end - a.seq_begin;
-  if (takes_pipe_kernel(a)) return prefill_pipe_kv_splits(a, nseq);
+  if (takes_pipe_kernel(a)) return prefill_pipe_kv_splits(a, nseq, us);
   // the compiled kernels: a tile takes about 1.1 us alone on its CU (2.2 us for 256-wide heads)
   const bool heads4 = compiled_short_chunk_tile(a);
-  return kv_pieces(a, nseq, heads4 ? 32 : kBM, heads4 ? 4 : 1, a.head_dim == 256 ? 2.2 : 1.1);
+  return kv_pieces(a, nseq, heads4 ? 32 : kBM, heads4 ? 4 : 1, a.head_dim == 256 ? 2.2 : 1.1, us);
 }
 
 size_t prefill_split_workspace_bytes(const PrefillArgs& a, int splits) {
@@ -929,6 +941,13 @@ size_t prefill_split_workspace_bytes(const PrefillArgs& a, int splits) {
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
   const int nseq = a.seq_end - a.seq_begin;
   if (nseq <= 0 || a.max_q_len <= 0) return hipSuccess;
+  if (a.packed) {
+    if (a.sm.mask_mode == 1) {
+      hipError_t e = launch_mask_bits(a, stream);
+      if (e != hipSuccess) return e;
+    }
+    return launch_prefill_packed(a, nseq, stream);
+  }
   if (takes_pipe_kernel(a)) {
     return launch_prefill_pipe(a, nseq, tuning().prefill_level_order != 0, stream);
   }

@@ -526,11 +526,11 @@ inline hipError_t launch_prefill_combine(const PrefillArgs& a, hipStream_t strea
 // way to memory and back (~0.29 ns per (token, head, piece) of 128 dims).  A cut must save at least 2 us,
 // leaves no piece under four tiles and makes at most 64 pieces.  bm / heads: query positions and query heads
 // per workgroup.  RPA_PREFILL_SPLITS: 0 / 1 never, n forces n.
-inline int kv_pieces(const PrefillArgs& a, int nseq, int bm, int heads, double tile_us) {
+inline int kv_pieces(const PrefillArgs& a, int nseq, int bm, int heads, double tile_us, double* us_of_best = nullptr) {
   // (with the composition on the device nseq, max_q_len, max_kv_len and num_tokens are bounds: a launch that is
   // under-filled even by its bounds is cut, and every workgroup fits the piece count to its own range)
   if (nseq <= 0 || a.max_q_len <= 0 || a.max_kv_len <= 0 || a.num_tokens <= 0) return 1;
-  const int forced = tuning().prefill_splits;
+  const int forced = us_of_best ? -1 : tuning().prefill_splits;  // (who asks for the time asks for the model's plan)
   if (forced == 0 || forced == 1) return 1;
   if (forced > 1) return std::min(forced, 64);
   const int64_t tokens = std::max<int64_t>(1, (int64_t)a.num_tokens - a.seq_begin);
@@ -557,6 +557,12 @@ inline int kv_pieces(const PrefillArgs& a, int nseq, int bm, int heads, double t
       best_us = us;
       best = n;
     }
+  }
+  if (us_of_best) {
+    // (for the time and not only the choice: workgroups beyond one per CU cost what a mean range costs, not the longest)
+    const double mean = std::min<double>(longest, std::max(1.0, a.max_kv_len - 0.5 * (a.max_q_len - 1))) / longest;
+    const double w = (double)wgs * best, rate = w <= 192 ? 1.0 : w <= 512 ? 1.0 + (w - 192) * (1.6 / 320) : 2.6 * (w / 512);
+    *us_of_best = tile_us * chain / best * std::max(1.0, rate * mean * 1.15) + (best > 1 ? 1.5 + per_piece * best : 0.0);
   }
   return best;
 }
@@ -645,6 +651,11 @@ __device__ __forceinline__ void async_copy_tile(char* lds_k, char* lds_v, const 
 // rpa_prefill_pipe.hip: the software-pipelined kernel for the plain causal bf16 case
 bool prefill_pipe_applies(const PrefillArgs& a);
 hipError_t launch_prefill_pipe(const PrefillArgs& a, int nseq, bool level_order, hipStream_t stream);
-int prefill_pipe_kv_splits(const PrefillArgs& a, int nseq);
+int prefill_pipe_kv_splits(const PrefillArgs& a, int nseq, double* us = nullptr);
+
+// rpa_prefill_packed.hip: 32 (position, head) columns per workgroup, whose waves walk different tiles
+hipError_t launch_prefill_packed(const PrefillArgs& a, int nseq, hipStream_t stream);
+// pieces of the other kernels and, in *us, what kv_pieces() gives their launch
+int prefill_unpacked_kv_splits(const PrefillArgs& a, double* us);
 
 }  // namespace rpa

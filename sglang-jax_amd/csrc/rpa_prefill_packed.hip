@@ -1,0 +1,547 @@
+// Flash kernel for prefill launches that the tiles of 128 query positions leave mostly idle on gfx950: one prompt on a
+// tensor-parallel share of the heads, a few short chunks, a verify step of speculative decoding.
+//
+// What bounds such a launch is a chain: a workgroup of rpa_prefill_pipe_kernel walks its 64-token K/V tiles one after the
+// other, 16 of them for a prompt of 1003 tokens, about 1 us each, on 64 of 256 CUs.  Here a workgroup owns 32 COLUMNS and
+// its eight waves walk DIFFERENT tiles:
+//   * a column is a (query position, query head) pair: the G query heads of a kv head times 32 / G positions, so that the
+//     32-column matrix instructions are full also for a chunk of a few tokens, and a kv head's rows are read once for all
+//     of its query heads (a verify step of 8 tokens on 2 heads per kv head has 16 columns; the 128-position tile ran it on
+//     8 rows of 128)
+//   * wave w takes the 32-token tiles w, w + 8, ...: a chain of 4 instead of 16 for 1003 tokens, and no barrier in it (every
+//     wave copies its own tiles into its own LDS).  The eight partial results meet in LDS at the end, in f32.
+// The price is that K/V rows are brought into LDS once per 32 columns instead of once per 128 (64 B per clock and CU from the
+// L2: 4 us for the 512 KB of the longest workgroup of that prompt), so launches that fill the GPU stay where they were:
+// see prefill_packed_pieces().
+//
+// A wave's tile, single buffers: K of the next tile is requested when this tile's scores have been taken, V when its second
+// product has; each copy then has the other half of the step to arrive.  bf16 rows: LDS layout and swizzles of
+// rpa_prefill_async_kernel.  e4m3 rows arrive as bytes; K operands are widened on their way from LDS to the matrix pipe, V
+// rows into a bf16 tile for the transposing reads.
+
+#include <cmath>
+
+#include "rpa_prefill_common.h"
+
+namespace rpa {
+
+using namespace pf;
+
+namespace {
+
+constexpr int kWaves = 8;
+constexpr int kTok = 32;                  // tokens per tile
+constexpr int kCols = 32;                 // (position, head) pairs per workgroup
+constexpr int kFeedB = 16384;             // LDS of a wave: bf16 K, V; e4m3 K bytes, V bytes, V widened
+constexpr int kMergePitch = 132;          // floats per column in the merge (16-byte writes of 16 columns meet every bank once)
+constexpr int kMergeB = kWaves * kCols * kMergePitch * 4;
+constexpr int kIdsAt = kWaves * kFeedB;   // 64 page ids per wave
+constexpr int kMaskAt = kIdsAt + kWaves * 256;
+constexpr int kMlAt = kMaskAt + kWaves * 256;
+constexpr int kLdsB = kMlAt + kWaves * kCols * 8;
+static_assert(kMergeB <= kMlAt, "the merge reuses the tiles, not the (maximum, sum) pairs");
+
+typedef __attribute__((address_space(3))) char* lds_t;
+typedef float f32x4v_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }  // lgkmcnt(0)
+
+// PG: pages of a tile.  1: the tile lies inside a page (page size a multiple of 32); 2: pages of 16 tokens; 0: any other
+// size, page ids through LDS (a load into a register would make the compiler drain the copies in flight).
+template <int PG, bool FP8>
+struct PackedFeed {
+  static constexpr int kPerRow = FP8 ? 8 : 16;        // 16-byte chunks of a row of 128 elements
+  static constexpr int kRowsPer = 64 / kPerRow;       // rows per copy instruction
+  static constexpr int N = kTok / kRowsPer;           // copy instructions for the K (or V) rows of a tile
+  static constexpr int kTileBytes = N * 1024;
+
+  uint32_t ofs_k[N], ofs_v[N];  // a lane's chunk from the first row of its page part (PG 2: 16 rows) of a whole tile
+  int64_t base[PG == 2 ? 2 : 1];  // byte offset of the tile's first row(s), the same in every lane
+  int64_t row[N];               // per-lane byte offsets of the rows (partial tiles, PG 0)
+  bool whole;
+
+  __device__ __forceinline__ static int row_of(int n, int lane) { return n * kRowsPer + lane / kPerRow; }
+  __device__ __forceinline__ static int chunk_k(int t, int cp) { return FP8 ? cp ^ ((t >> 1) & 7) : cp ^ (t & 15); }
+  __device__ __forceinline__ static int chunk_v(int t, int cp) { return FP8 ? cp : cp ^ ((t & 3) << 2); }
+
+  __device__ __forceinline__ void init(const KvAddr& kv, int lane) {
+    const int cp = lane % kPerRow;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int t = row_of(n, lane), in = PG == 2 ? (t & 15) : t;
+      ofs_k[n] = (uint32_t)(in * kv.tok_stride + (chunk_k(t, cp) << 4));
+      ofs_v[n] = (uint32_t)(in * kv.tok_stride + (chunk_v(t, cp) << 4));
+    }
+  }
+
+  __device__ __forceinline__ static void request_ids(uint32_t at, const TileSrc& s, int tb, int lane) {
+    tb = min(tb, s.last_tok);
+    const int32_t* src = s.pages + min(page_slot(s, tb) + lane, page_slot(s, s.last_tok));
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(at), "v"(src) : "memory", "m0");
+  }
+
+  // Where the rows of the tile at `tb` are (PG 0: its page ids have arrived at `ids`).
+  __device__ __forceinline__ void locate(const TileSrc& s, const KvAddr& kv, int tb, int lane, uint32_t ids) {
+    whole = PG != 0 && tb + kTok - 1 <= s.last_tok;
+    if constexpr (PG == 0) {
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const int tok = min(tb + row_of(n, lane), s.last_tok), ps = page_slot(s, tok);
+        const int id = *(__attribute__((address_space(3))) const int32_t*)(lds_t)(uintptr_t)(ids + 4u * (uint32_t)(ps - page_slot(s, tb)));
+        row[n] = (int64_t)id * kv.page_stride + (int64_t)((tok - ps * s.page_size) * kv.tok_stride);
+      }
+    } else {
+      const int ps = __builtin_amdgcn_readfirstlane(page_slot(s, tb));
+      const int pg0 = scalar_load_i32(s.pages + ps);
+      const int pg1 = PG == 2 ? scalar_load_i32(s.pages + min(ps + 1, page_slot(s, s.last_tok))) : pg0;
+      base[0] = (int64_t)pg0 * kv.page_stride + (PG == 1 ? (int64_t)(tb - ps * s.page_size) * kv.tok_stride : 0);
+      if constexpr (PG == 2) base[1] = (int64_t)pg1 * kv.page_stride;
+      if (!whole) {  // the sequence's last tile: rows clamped to the last token
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+          const int t = min(row_of(n, lane), s.last_tok - tb);
+          row[n] = PG == 2 ? (t >= 16 ? base[PG - 1] : base[0]) + (int64_t)((t & 15) * kv.tok_stride)
+                           : base[0] + (int64_t)(t * kv.tok_stride);
+        }
+      }
+    }
+  }
+
+  template <bool IS_V>
+  __device__ __forceinline__ void copy(uint32_t at, const char* head, int lane) const {
+    if (PG != 0 && whole) {
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const char* b = head + base[(PG == 2 && n >= N / 2) ? PG - 1 : 0];
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     :: "s"(at + n * 1024), "v"(IS_V ? ofs_v[n] : ofs_k[n]), "s"(b)
+                     : "memory", "m0");
+      }
+    } else {
+      const int cp = lane % kPerRow;
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const int t = row_of(n, lane);
+        const char* g = head + row[n] + ((IS_V ? chunk_v(t, cp) : chunk_k(t, cp)) << 4);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at + n * 1024), "v"(g) : "memory", "m0");
+      }
+    }
+  }
+};
+
+__device__ __forceinline__ u32x4_t at16(uint32_t at) {
+  return *(__attribute__((address_space(3))) const u32x4_t*)(lds_t)(uintptr_t)at;
+}
+__device__ __forceinline__ u32x2_t at8(uint32_t at) {
+  return *(__attribute__((address_space(3))) const u32x2_t*)(lds_t)(uintptr_t)at;
+}
+__device__ __forceinline__ u32x2_t at_tr(uint32_t at) {
+  typedef __attribute__((address_space(3))) s16x4_t* ptr_t;
+  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr_t)(uintptr_t)at));
+}
+
+// soft cap, temperature and rounding of 16 scores, to log2 units (as softmax_tile has them)
+template <class Smx>
+__device__ __forceinline__ void general_scores(f32x16_t& S, const Smx& sm) {
+  if (sm.cap != 0.f && !sm.round_mode) {
+    const float k1 = sm.scale * sm.inv_cap * (2.0f * kLog2e), k2 = sm.cap * sm.temp * kLog2e;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) S[v] = __builtin_fmaf(__builtin_amdgcn_rcpf(fast_exp2(S[v] * k1) + 1.0f), -2.0f * k2, k2);
+  } else {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      float x = S[v] * sm.scale;
+      if (sm.cap != 0.f) x = soft_cap_f(x, sm.cap, sm.inv_cap);
+      x = x * sm.temp;
+      if (sm.round_mode) x = round_logit(x, sm.round_mode);
+      S[v] = x * kLog2e;
+    }
+  }
+}
+
+// grid: (sequence, kv head) units x tiles of `per` = 32 / G positions, then the workgroups that write a prompt's rows;
+// blockIdx.y = piece of the K/V range.  CAP: soft cap or rounded logits; EXT: custom or no mask, temperature, q_scale.
+template <int PG, bool CAP, bool EXT, bool FP8>
+__global__ __launch_bounds__(512, 2) void rpa_prefill_packed_kernel(const PrefillArgs a_in, int tiles, int nseq, int per) {
+  PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
+  if (a.dist) {
+    a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
+    a.seq_end = min(a.seq_end, scalar_load_i32(a.dist + 2));
+  }
+  __shared__ __attribute__((aligned(1024))) char lds[kLdsB];
+  const Work w = decompose(a, tiles, nseq, false, per, a.G);
+  if (!w.valid) {
+    write_new_tokens(a_in);
+    return;
+  }
+  typedef PackedFeed<PG, FP8> Feed;
+  constexpr int N = Feed::N;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 31, h = lane >> 5;
+  const TileSrc src = make_src(a, w);
+  const char* kh = head_rows(a, w, a.kv.k_base);
+  const char* vh = head_rows(a, w, a.kv.v_base);
+
+  // columns: position c / G, head c % G; those behind the last whole position, and positions past the chunk, are not written
+  const int r_lo = w.q_start, r_hi = min(w.q_start + per, w.q_len) - 1;
+  const int pos = c / a.G;
+  const int row = r_lo + pos, qpos = w.prefix + row;
+  const int W_ = a.sm.window;
+  const bool causal = !EXT || a.sm.mask_mode == 0;
+  MaskCtx mc;
+  mc.mode = 0;
+  if constexpr (EXT) mc = make_mask_ctx(a, w, row);
+  int t_hi = causal ? min(w.kv_len, w.prefix + r_hi + 1) : w.kv_len;  // exclusive
+  int t_lo = 0;
+  if (W_ > 0) t_lo = max(0, w.prefix + r_lo - W_ + 1) & ~(kBN - 1);
+  int split = 0;
+  if (a.kv_splits > 1 && !kv_piece(a, t_lo, t_hi, split)) t_hi = t_lo;  // nothing left for this piece: rows that weigh nothing
+  t_lo = __builtin_amdgcn_readfirstlane(t_lo);
+  t_hi = __builtin_amdgcn_readfirstlane(t_hi);
+  const int nT = max(0, (t_hi - t_lo + kTok - 1) / kTok);
+
+  const uint32_t lds_at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_t)lds);
+  const uint32_t k_at = lds_at + wave * kFeedB, v_at = k_at + Feed::kTileBytes;
+  const uint32_t vt_at = FP8 ? k_at + 2 * Feed::kTileBytes : v_at;  // V rows as bf16
+  const uint32_t ids_at = lds_at + kIdsAt + wave * 256, mask_at = lds_at + kMaskAt + wave * 256;
+  const bool has_bits = EXT && mc.mode == 1 && mc.bits;  // (else the caller's words, one load per score)
+  auto request_mask = [&](int tb) __attribute__((always_inline)) {
+    const uint32_t* words = reinterpret_cast<const uint32_t*>(mc.bits) + min(tb >> 5, 2 * mc.bit_words - 1);
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(mask_at), "v"(words) : "memory", "m0");
+  };
+
+  Feed feed;
+  int j = wave;  // this wave's tile
+  if (j < nT) {
+    const int tb = t_lo + j * kTok;
+    if constexpr (PG == 0) {
+      Feed::request_ids(ids_at, src, tb, lane);
+      wait_all_loads();
+    }
+    feed.init(a.kv, lane);
+    feed.locate(src, a.kv, tb, lane, ids_at);
+    if constexpr (PG == 0) {
+      wait_lds();
+      Feed::request_ids(ids_at, src, tb + kWaves * kTok, lane);
+    }
+    if (has_bits) request_mask(tb);
+    feed.template copy<false>(k_at, kh, lane);
+    feed.template copy<true>(v_at, vh, lane);
+  }
+
+  u32x4_t qB[kSteps];
+  {
+    const int head = w.head + (c - pos * a.G);
+    const uint16_t* qp = a.q + ((int64_t)(w.qg0 + min(row, w.q_len - 1)) * a.Hq + head) * a.q_dim;
+    ld_query_row<kSteps, kHeadDim>(qB, qp, h, a.q_dim);
+    if (EXT && a.sm.q_scale > 0.f) {
+#pragma unroll
+      for (int ks = 0; ks < kSteps; ++ks) qB[ks] = requantise_q(qB[ks], a.sm.q_scale, FP8);
+    }
+  }
+  Softmax<CAP> sm;
+  sm.scale = a.sm.sm_scale * (a.k_scale ? scalar_load_f32(a.k_scale + w.hk) : 1.0f) *
+             ((EXT && a.sm.q_scale > 0.f) ? a.sm.q_scale : 1.0f);
+  // The maximum is taken over unscaled scores and masked ones are far below it: a scale has to be positive.  The sign of a
+  // negative one goes into the queries (exact), one of nothing makes every score zero.
+  if (!(sm.scale > 1e-25f)) {
+    const uint32_t flip = 0x80008000u, keep = sm.scale < -1e-25f ? 0xffffffffu : 0u;
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qB[ks][e] = (qB[ks][e] ^ flip) & keep;
+    sm.scale = keep ? -sm.scale : 1.0f;
+  }
+  sm.cap = a.sm.soft_cap;
+  sm.inv_cap = (sm.cap != 0.f) ? 1.0f / sm.cap : 0.f;
+  {
+    const float temp = EXT ? xai_factor(qpos, a.sm.xai_len) : 1.0f;  // per query position
+    sm.sc2 = CAP ? 1.0f : sm.scale * kLog2e * temp;
+    sm.temp = temp;
+    sm.round_mode = a.sm.round_logits;
+  }
+
+  f32x16_t O[kDimTiles];
+#pragma unroll
+  for (int d = 0; d < kDimTiles; ++d) O[d] = kZero16;
+  float m = kMaxFloor, l = 0.f;
+
+  // operand addresses inside a tile: see rpa_prefill_async_kernel
+  uint32_t koff[kSteps], voff[kDimTiles];
+  {
+    const int r16 = lane & 15, b16 = lane >> 4;
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks)
+      koff[ks] = FP8 ? k_at + c * 128 + ((ks ^ ((c >> 1) & 7)) << 4) + 8 * h : k_at + c * kRowB + ((ks * 32) ^ ((h ^ (c & 15)) << 4));
+#pragma unroll
+    for (int d = 0; d < kDimTiles; ++d)
+      voff[d] = vt_at + (4 * h + (r16 >> 2)) * kRowB + ((b16 & 1) << 5) + (((r16 & 3) >> 1) << 4) + ((r16 & 1) << 3) + ((d * 64) ^ ((r16 >> 2) << 6));
+  }
+  const bf16x2_t ones = {(__bf16)1.0f, (__bf16)1.0f};
+
+  while (j < nT) {
+    const int tb = t_lo + j * kTok;
+    const bool more = j + kWaves < nT;
+    __builtin_amdgcn_s_waitcnt(0x0F70 | N);  // K has landed (V's copies are younger)
+    asm volatile("" ::: "memory");
+    uint32_t mask_word = 0;
+    if (has_bits) mask_word = *(__attribute__((address_space(3))) const uint32_t*)(lds_t)(uintptr_t)(mask_at + 4u * lane);
+    f32x16_t S = kZero16;
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks) {
+      if constexpr (FP8) {
+        const u32x2_t x = at8(koff[ks]);
+        const u32x2_t lo = fp8x4_to_bf16x4(x[0]), hi = fp8x4_to_bf16x4(x[1]);
+        S = mfma32(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, qB[ks], S);
+      } else {
+        S = mfma32(at16(koff[ks]), qB[ks], S);
+      }
+    }
+    if (more) {
+      const int tn = tb + kWaves * kTok;
+      feed.locate(src, a.kv, tn, lane, ids_at);
+      wait_lds();  // the reads of K (and of the ids and the mask) have returned: their places may be filled again
+      if constexpr (PG == 0) Feed::request_ids(ids_at, src, tn + kWaves * kTok, lane);
+      if (has_bits) request_mask(tn);
+      feed.template copy<false>(k_at, kh, lane);
+    }
+
+    // ---- softmax of the 16 scores of this lane: tokens tb + 8 (v / 4) + 4 h + v % 4
+    if constexpr (CAP) general_scores(S, sm);
+    const bool need_mask = (causal ? (tb + kTok - 1 > w.prefix + r_lo) : (mc.mode == 1 || tb + kTok > w.kv_len)) ||
+                           (W_ > 0 && tb <= w.prefix + r_hi - W_);
+    if (need_mask) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int tok = tb + 8 * (v >> 2) + 4 * h + (v & 3);
+        bool masked;
+        if (!EXT || mc.mode == 0) masked = tok > qpos;
+        else masked = (tok >= mc.kv_len) || (mc.mode == 1 && (has_bits ? !((mask_word >> (8 * (v >> 2) + 4 * h + (v & 3))) & 1u) : mc.row[tok] < 1));
+        masked = masked || (W_ > 0 && tok <= qpos - W_);
+        S[v] = masked ? kMaskRaw : S[v];
+      }
+    }
+    float mx = __builtin_fmaxf(S[0], S[1]);
+#pragma unroll
+    for (int v = 2; v < 16; v += 2) mx = __builtin_fmaxf(__builtin_fmaxf(mx, S[v]), S[v + 1]);
+    update_running_max(swap_max(mx), m, l, O, sm.sc2);
+    const float neg_m = -m * sm.sc2;
+    u32x4_t pB[2];
+    float ps[2] = {0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t x = pack_bf16x2(fast_exp2(__builtin_fmaf(S[2 * i], sm.sc2, neg_m)), fast_exp2(__builtin_fmaf(S[2 * i + 1], sm.sc2, neg_m)));
+      ps[i & 1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, x), ones, ps[i & 1], false);
+      pB[i >> 2][i & 3] = x;
+    }
+    l += ps[0] + ps[1];
+
+    if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | N);  // V has landed (the next K's copies are younger)
+    else __builtin_amdgcn_s_waitcnt(0x0F70);
+    asm volatile("" ::: "memory");
+    if constexpr (FP8) {  // bytes -> bf16 rows, two chunks of 16 bytes each
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const int t = Feed::row_of(n, lane), cp = 2 * (lane & 7);
+        const u32x4_t x = at16(v_at + n * 1024 + lane * 16);
+        const u32x2_t p = fp8x4_to_bf16x4(x[0]), q = fp8x4_to_bf16x4(x[1]), r = fp8x4_to_bf16x4(x[2]), s = fp8x4_to_bf16x4(x[3]);
+        const uint32_t at = vt_at + t * kRowB;
+        *(__attribute__((address_space(3))) u32x4_t*)(lds_t)(uintptr_t)(at + ((cp ^ ((t & 3) << 2)) << 4)) = u32x4_t{p[0], p[1], q[0], q[1]};
+        *(__attribute__((address_space(3))) u32x4_t*)(lds_t)(uintptr_t)(at + (((cp + 1) ^ ((t & 3) << 2)) << 4)) = u32x4_t{r[0], r[1], s[0], s[1]};
+      }
+      wait_lds();
+      asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int d = 0; d < kDimTiles; ++d) {
+        const u32x2_t lo = at_tr(voff[d] + kk * 16 * kRowB), hi = at_tr(voff[d] + kk * 16 * kRowB + 8 * kRowB);
+        O[d] = mfma32(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pB[kk], O[d]);
+      }
+    if (more) {
+      wait_lds();
+      feed.template copy<true>(v_at, vh, lane);
+    }
+    j += kWaves;
+  }
+
+  // ---- merge of the waves' results, in f32: references and sums first, then the rows against the largest reference
+  typedef __attribute__((address_space(3))) f32x2_t* ml_t;
+  const uint32_t ml_at = lds_at + kMlAt;
+  l += __shfl_xor(l, 32);
+  const float m2 = wave < nT ? fmaxf(m * sm.sc2, kNoReference) : kNoReference;
+  if (h == 0) *(ml_t)(uintptr_t)(ml_at + (wave * kCols + c) * 8) = f32x2_t{m2, l};
+  __syncthreads();
+  const int n_waves = min(nT, kWaves);  // waves that had a tile
+  auto reference = [&](int col, float& den) __attribute__((always_inline)) {
+    f32x2_t x[kWaves];
+    float top = kNoReference;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) {
+      x[i] = *(ml_t)(uintptr_t)(ml_at + (i * kCols + col) * 8);
+      top = fmaxf(top, x[i][0]);
+    }
+    den = 0.f;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) den += x[i][1] * fast_exp2(x[i][0] - top);
+    return top;
+  };
+  float den;
+  if (wave < nT) {
+    const float f = fast_exp2(m2 - reference(c, den));
+    typedef __attribute__((address_space(3))) f32x4v_t* o_t;
+    const uint32_t at = lds_at + ((wave * kCols + c) * kMergePitch + 4 * h) * 4;
+#pragma unroll
+    for (int d = 0; d < kDimTiles; ++d)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *(o_t)(uintptr_t)(at + (d * 32 + q * 8) * 4) = f32x4v_t{O[d][4 * q] * f, O[d][4 * q + 1] * f, O[d][4 * q + 2] * f, O[d][4 * q + 3] * f};
+  }
+  __syncthreads();
+  const int col = threadIdx.x >> 4, dim = (threadIdx.x & 15) * 8;
+  const int out_pos = col / a.G, out_row = r_lo + out_pos, head = w.head + col - out_pos * a.G;
+  if (out_pos >= per || out_row >= w.q_len) return;
+  const float top = reference(col, den);
+  float o[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = 0.f;
+  for (int i = 0; i < n_waves; ++i) {
+    typedef __attribute__((address_space(3))) const f32x4v_t* o_t;
+    const uint32_t at = lds_at + ((i * kCols + col) * kMergePitch + dim) * 4;
+    const f32x4v_t x = *(o_t)(uintptr_t)at, y = *(o_t)(uintptr_t)(at + 16);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o[e] += x[e];
+      o[4 + e] += y[e];
+    }
+  }
+  const int64_t out_at = (int64_t)(w.qg0 + out_row) * a.Hq + head;
+  if (a.kv_splits > 1) {
+    const int64_t slot = out_at * a.kv_splits + split;
+    float* op = a.ws_o + slot * kHeadDim + dim;
+    *reinterpret_cast<f32x4v_t*>(op) = f32x4v_t{o[0], o[1], o[2], o[3]};
+    *reinterpret_cast<f32x4v_t*>(op + 4) = f32x4v_t{o[4], o[5], o[6], o[7]};
+    if (dim == 0) {
+      a.ws_ml[slot * 2] = top;
+      a.ws_ml[slot * 2 + 1] = den;
+    }
+    return;
+  }
+  if (dim >= a.q_dim) return;
+  const float vs = a.v_scale ? scalar_load_f32(a.v_scale + w.hk) : 1.0f;
+  const float inv = a.sm.sink ? vs * sink_inverse(top, den, sink_logit(a.sm.sink, a.sm.round_logits, head)) : vs / den;
+  st16(a.out + out_at * a.q_dim + dim, u32x4_t{pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv),
+                                               pack_bf16x2(o[4] * inv, o[5] * inv), pack_bf16x2(o[6] * inv, o[7] * inv)});
+}
+
+}  // namespace
+
+// Microseconds of a launch with every K/V range in n pieces, fitted to 60 prompts, chunks and verify steps of 8 .. 2048
+// tokens on prefixes of 0 .. 16384 (both kernels).  A workgroup has a CU to itself and pays 4.5 us (custom masks: 6.5) for its
+// start and its merge; eight tiles side by side take 1.25 us of a lone workgroup, up to 1.1 us more where few workgroups read the same
+// rows (they come from HBM), 1.45 us on a full chip; workgroups of the grid that find no tile 0.4 us a round; pieces the merge launch and the partial rows' way to memory and
+// back.
+static double packed_us(const PrefillArgs& a, int nseq, int n) {
+  const int per = kCols / a.G;
+  const int64_t tokens = std::max<int64_t>(1, (int64_t)a.num_tokens - a.seq_begin);
+  const int64_t grid = (int64_t)nseq * ((a.max_q_len + per - 1) / per) * a.Hkv;
+  const int64_t wgs = std::min(grid, (tokens / per + nseq) * a.Hkv);
+  double longest = a.max_kv_len, mean = std::max(1.0, a.max_kv_len - 0.5 * (a.max_q_len - 1));
+  if (a.sm.window > 0) {
+    longest = std::min(longest, (double)a.sm.window + per + kBN);
+    mean = std::min(mean, longest);
+  }
+  auto steps = [&](double range) { return std::ceil(std::ceil(range / n / kTok) / kWaves); };
+  const double step_us = 1.25 + 1.1 / ((a.max_q_len + per - 1) / per);
+  const double rounds = std::ceil((double)wgs * n / 256.0);
+  const double full = rounds * (a.sm.mask_mode == 1 ? 6.5 : 4.5) + 1.45 * (double)wgs * n * steps(mean) / 256.0 + 0.4 * (double)(grid - wgs) * n / 256.0;
+  return 2.5 + std::max(4.5 + step_us * steps(longest), full) + (n > 1 ? 3.5 + 0.29e-3 * (double)tokens * a.Hq * n : 0.0);
+}
+
+// The launches that the other kernels' tiles leave idle, by both models: those kernels take 8 us besides the chain that
+// kv_pieces() knows, and have to be behind by a tenth (a fifth for custom masks, a third behind decode rows).  Measured, other
+// kernels -> this one, us (8 / 2 heads unless said): prompts of 64 tokens 7.8 -> 7.4, 256 11.4 -> 8.7, 1003 21.9 -> 12.4, 2048
+// 34.6 -> 25.8; 1003 tokens on 32 / 8 heads stay (24.8 against 36.9), 500 too (16.6 / 17.4); 128 tokens on a prefix of 4000
+// 22.1 -> 18.0, of 16000 27.8 / 27.2; 16 verify steps of 8 tokens on 1000, 8 / 4 heads 32.7 -> 22.9, 32 / 8 heads on 4000
+// 99.2 -> 64.8.  60 drawn prefill calls with chunks of up to 4096 tokens: 1.26 times as fast on average.
+// Behind decode rows the bound on the lengths may be theirs: then it has to hold for chunks without a prefix too.
+// Not with the composition on the device: the grid is that of the bounds, and a workgroup without a tile holds a CU here.
+int prefill_packed_pieces(const PrefillArgs& a) {
+  const Tuning& tune = tuning();
+  const int nseq = a.seq_end - a.seq_begin, forced = tune.prefill_splits;
+  if (a.head_dim != 128 || a.G > kCols || tune.prefill_packed == 0 || nseq <= 0 || a.max_q_len <= 0 || a.num_tokens <= 0) return 0;
+  if (tune.prefill_packed == 1 && (forced >= 0 || a.max_kv_len <= 0)) return std::max(1, std::min(forced, 64));
+  double other = 1e9;
+  if (tune.prefill_packed != 1) {
+    if (a.dist || a.max_kv_len <= 0 || forced > 1 || tune.prefill_staged == 1 || tune.prefill_pipe == 0 || tune.prefill_pipe_nq == 2 ||
+        tune.prefill_pipe_tile == 128)
+      return 0;
+    // (RPA_PREFILL_SPLITS=0: what the model would cut runs whole on the other kernels, nothing else changes)
+    if (prefill_unpacked_kv_splits(a, &other) > 1 && forced >= 0) return 0;
+    // (a verify step of more than 32 columns whose heads come in fours: the short-chunk tile, 37.4 against 40.5 us for 12 x 16
+    // tokens on 40 / 8 heads)
+    const bool short_tile = a.max_q_len * a.G > kCols && a.G % 4 == 0;
+    const double margin = a.sm.mask_mode == 1 && short_tile ? 0.6 : a.seq_begin > 0 ? 0.65 : a.sm.mask_mode == 1 ? 0.8 : 0.9;
+    other = margin * (8.0 + other);
+    if (a.seq_begin > 0 && a.max_q_len < a.max_kv_len) {
+      PrefillArgs own = a;
+      own.max_kv_len = a.max_q_len;
+      double us = 0.0;
+      prefill_unpacked_kv_splits(own, &us);
+      if (packed_us(own, nseq, 1) >= margin * (8.0 + us)) return 0;
+      if (((int64_t)a.num_tokens - a.seq_begin) * a.Hq > 512 * kCols) return 0;  // more than two rounds of workgroups
+    }
+  }
+  // (no piece under eight tiles, the partial rows under 256 MB)
+  const int64_t row_bytes = (int64_t)a.num_tokens * a.Hq * (kHeadDim + 2) * 4;
+  const int64_t cap = forced >= 0 ? 1 : std::min<int64_t>({64, a.max_kv_len / (kWaves * kTok), ((int64_t)256 << 20) / row_bytes});
+  int best = 1;
+  double best_us = packed_us(a, nseq, 1);
+  for (int n : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+    if (n > cap) break;
+    const double us = packed_us(a, nseq, n);
+    if (us < best_us) {
+      best_us = us;
+      best = n;
+    }
+  }
+  return best_us < other ? best : 0;
+}
+
+hipError_t launch_prefill_packed(const PrefillArgs& a, int nseq, hipStream_t stream) {
+  const int per = kCols / a.G;
+  const int tiles = (a.max_q_len + per - 1) / per;
+  const int64_t units = (int64_t)nseq * a.Hkv;
+  const int64_t grid = (units >= 8 ? ((units + 7) / 8) * 8 : units) * tiles;
+  if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+  const bool cut = a.kv_splits > 1;
+  if (cut && (!a.ws_o || !a.ws_ml || a.kv_splits > 64)) return hipErrorInvalidValue;
+  const dim3 g((unsigned)(grid + a.write_blocks), cut ? (unsigned)a.kv_splits : 1u), blk(512);
+  const bool cap = a.sm.soft_cap != 0.f || a.sm.round_logits != 0;
+  const bool ext = a.sm.xai_len > 0.f || a.sm.mask_mode != 0 || a.sm.q_scale > 0.f;
+  const int pg = a.pt.page_size % kTok == 0 ? 1 : a.pt.page_size == 16 ? 2 : 0;
+#define RPA_PACKED(P, C, E, F) hipLaunchKernelGGL((rpa_prefill_packed_kernel<P, C, E, F>), g, blk, 0, stream, a, tiles, nseq, per)
+#define RPA_PACKED_OPTS(P, F)                            \
+  do {                                                   \
+    if (cap && ext) RPA_PACKED(P, true, true, F);        \
+    else if (cap) RPA_PACKED(P, true, false, F);         \
+    else if (ext) RPA_PACKED(P, false, true, F);         \
+    else RPA_PACKED(P, false, false, F);                 \
+  } while (0)
+#define RPA_PACKED_PAGES(F)                  \
+  do {                                       \
+    if (pg == 1) RPA_PACKED_OPTS(1, F);      \
+    else if (pg == 2) RPA_PACKED_OPTS(2, F); \
+    else RPA_PACKED_OPTS(0, F);              \
+  } while (0)
+  if (a.fp8) RPA_PACKED_PAGES(true);
+  else RPA_PACKED_PAGES(false);
+#undef RPA_PACKED_PAGES
+#undef RPA_PACKED_OPTS
+#undef RPA_PACKED
+  return cut ? launch_prefill_combine(a, stream) : hipGetLastError();
+}
+
+}  // namespace rpa

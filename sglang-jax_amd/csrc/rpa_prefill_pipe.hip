@@ -541,10 +541,10 @@ bool short_chunk_tile(const PrefillArgs& a, int nq) {
 }  // namespace
 
 // Pieces per K/V range for a launch of the pipelined kernel (1 = whole ranges).
-int prefill_pipe_kv_splits(const PrefillArgs& a, int nseq) {
+int prefill_pipe_kv_splits(const PrefillArgs& a, int nseq, double* us) {
   if (forced_nq() == 2) return 1;
   const bool heads4 = short_chunk_tile(a, 1);
-  return kv_pieces(a, nseq, heads4 ? 32 : 128, heads4 ? 4 : 1, 0.8);
+  return kv_pieces(a, nseq, heads4 ? 32 : 128, heads4 ? 4 : 1, 0.8, us);
 }
 
 hipError_t launch_prefill_pipe(const PrefillArgs& a, int nseq, bool level_order, hipStream_t stream) {

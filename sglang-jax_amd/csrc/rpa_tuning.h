@@ -29,6 +29,7 @@ struct Tuning {
   float prefill_pipe_limit = 0.f;   // RPA_PREFILL_PIPE_LIMIT     0: the kernel's own row-sum limit
   int prefill_pipe_masked = 1;      // RPA_PREFILL_PIPE_MASKED    0: the steps on the causal diagonal through compiled code
   int prefill_splits = -1;          // RPA_PREFILL_SPLITS         -1: cost model; 0 | 1 never; n forces n pieces
+  int prefill_packed = -1;          // RPA_PREFILL_PACKED         -1: cost model; 0 never; 1 wherever the 32-column kernel can
   // ---- absorbed MLA (rpa_mla.hip)
   int mla_min_chunk = 64;           // RPA_MLA_MIN_CHUNK          smallest piece of a row of more than 256 tokens (3 rows of 1479 x 128 heads 38.7 us at 256, 28.7 at 64)
   int mla_wg_capacity = 0;          // RPA_MLA_WG_CAPACITY        0: one workgroup per CU

@@ -1656,3 +1656,65 @@ def test_short_rows_in_one_workgroup(pkg, wl, gpu, monkeypatch, Hq, Hkv, P, kv_d
     assert_parity(got.float(), oracle_out(b, attention_sink=sink).float(), **tol)
     monkeypatch.setenv("RPA_DECODE_ROW_KB", "0")
     torch.testing.assert_close(gpu_out(pkg, b, gpu, attention_sink=sink).float(), got.float(), rtol=1e-2, atol=4e-3)
+
+
+# ------------------------------------------------------------------ 32 (position, head) columns per workgroup
+PACKED_CASES = {
+    # name: (Hq, Hkv, P, e4m3, window, soft cap, sink, sm_scale, mask)
+    "g4": (8, 2, 64, False, None, None, True, None, None),
+    "g1_window": (2, 2, 64, False, 70, None, False, None, None),
+    "g5_pages16": (10, 2, 16, False, None, None, False, None, None),
+    "g20_pages24_cap": (40, 2, 24, False, None, 30.0, True, None, None),
+    "g32_pages1": (32, 1, 1, False, None, None, False, None, None),
+    "g2_e4m3": (8, 4, 64, True, None, None, False, None, None),
+    "g8_e4m3_pages16_window_cap": (16, 2, 16, True, 200, 30.0, False, None, None),
+    "g3_e4m3_pages8": (6, 2, 8, True, None, None, True, None, None),
+    "negative_scale": (8, 2, 64, False, None, None, False, -0.09, None),
+    "no_scale": (8, 2, 16, False, 300, None, False, 0.0, None),
+    "mask": (8, 4, 64, False, None, None, False, None, "tree"),
+    "mask_e4m3_pages16": (16, 2, 16, True, None, None, False, None, "tree"),
+    "no_mask": (8, 2, 24, False, None, None, False, None, "none"),
+}
+
+
+@pytest.mark.parametrize("pieces", [None, "3"])
+@pytest.mark.parametrize("case", list(PACKED_CASES))
+def test_packed_columns(pkg, wl, gpu, monkeypatch, case, pieces):
+    """rpa_prefill_packed_kernel at the edges of its 32-token tiles, of its eight waves' share (256 tokens), of its positions
+    per workgroup and of the chunk, whole ranges and pieces, against the oracle and against the other kernels."""
+    Hq, Hkv, P, fp8, window, cap, sink, scale, mask = PACKED_CASES[case]
+    q_lens, kv_lens = [1, 2, 7, 16, 33, 64], [1, 257, 7, 32, 300, 1500]
+    b = wl.make_batch("packed", q_lens, kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=57,
+                      sliding_window=window, soft_cap=cap, sm_scale=scale, kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+    b.distribution = torch.tensor([0, 0, 6], dtype=torch.int32)  # the row of one token is a chunk here
+    if scale is None:
+        wl.plant_needles(b, seed=2)
+    okw, gkw = {}, {}
+    if sink:
+        okw = gkw = dict(attention_sink=torch.linspace(-1.0, 2.0, Hq))
+    if mask == "tree":
+        rng = np.random.default_rng(4)
+        masks = []
+        for ql, kv in zip(q_lens, kv_lens):
+            m = (rng.random((ql, kv)) < 0.5).astype(np.int32)
+            m[:, kv - 1] = 1
+            masks.append(m)
+        cm = flat_mask(masks)
+        okw, gkw = dict(causal=False, custom_mask=cm), dict(causal=0, custom_mask=cm.to(gpu))
+    elif mask == "none":
+        okw, gkw = dict(causal=False), dict(causal=0)
+    tol = FP8_TOL if fp8 else BF16_TOL
+    say(f"packed {case} pieces={pieces}")
+    want = oracle_out(b, **okw)
+    monkeypatch.setenv("RPA_PREFILL_PACKED", "1")
+    if pieces:
+        monkeypatch.setenv("RPA_PREFILL_SPLITS", pieces)
+    got = gpu_out(pkg, b, gpu, **gkw)
+    assert torch.isfinite(got.float()).all()
+    assert_parity(got.float(), want.float(), **tol)
+    if not scale and scale is not None:
+        return  # (the compiled kernels do not mask behind a scale of nothing)
+    monkeypatch.setenv("RPA_PREFILL_PACKED", "0")
+    if scale is None:
+        other = gpu_out(pkg, b, gpu, **gkw)
+        assert float(row_rel_error(got.float(), other.float()).max()) < (3e-2 if fp8 else 1e-2)
