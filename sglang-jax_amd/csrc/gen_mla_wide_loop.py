@@ -33,6 +33,10 @@ The loop runs EVERY tile of a segment, so no compiled code ever holds the accumu
     per-lane offsets whose rows are clamped to the last valid token, so no bytes from beyond the row ever
     reach LDS.
 
+A second loop is generated for pages of 16 tokens (``RPA_MLA_WIDE_P16_*``): the rows of a tile lie in two pages, so the copies
+of its first 16 rows and those of its last 16 have a scalar base each.  The row border falls inside copy block 18; the
+copies numbered 4 (blocks 16 .. 19 of the four waves) are issued once per page with the lanes of the other page switched off.
+
 Register use follows one table shared with the C++ side through the emitted constraint macros; waits for
 LDS data and the issue distances the hardware does not interlock come from the emitter of
 gen_prefill_pipe_loop.py.
@@ -96,6 +100,11 @@ PMASK, PSTR = 71, 72         # page_size - 1, bytes per page
 LASTK = 73                   # first tile, counted from the segment's first, of the masked tail (the row's last, or the one before)
 CPB = 74                     # LDS address of this wave's first copy block in slot 0 (see copy_group)
 SGPR_CLOBBERS = list(range(60, 75))
+# pages of 16 tokens
+PGN2 = 75                    # second page of tile t + 4
+SB2 = 76                     # s[76:77] global base of the second page of the tile being copied
+STRADDLE = 4                 # the copy that meets both pages
+P16 = False                  # which loop is being written
 
 NEG_BIG = "0xf149f2ca"       # -1e30
 
@@ -178,12 +187,20 @@ def copy_dest(n, fill_slot):
 
 
 def copy_load(n):
-    return Ins(f"global_load_lds_dwordx4 {vr(OFS + n)}, s[{SB}:{SB + 1}]", "vmem", [OFS + n], [])
+    def load(base):
+        return Ins(f"global_load_lds_dwordx4 {vr(OFS + n)}, s[{base}:{base + 1}]", "vmem", [OFS + n], [])
+
+    if not P16 or n < STRADDLE:
+        return [load(SB)]
+    if n > STRADDLE:
+        return [load(SB2)]
+    return [Ins("s_mov_b64 exec, %[mask_a]", "salu"), load(SB), Ins("s_mov_b64 exec, %[mask_b]", "salu"), load(SB2),
+            Ins("s_mov_b64 exec, -1", "salu")]
 
 
 def copy_group(n, fill_slot):
     """one copy as a self-contained group (a wait state between the write of m0 and its use)"""
-    return [copy_dest(n, fill_slot), Ins("s_nop 0", "nop"), copy_load(n)]
+    return [copy_dest(n, fill_slot), Ins("s_nop 0", "nop"), *copy_load(n)]
 
 
 def copy_bases(em):
@@ -202,8 +219,21 @@ def tile_scalars(em, k):
     em.raw(f"s_cbranch_scc1 L_lastofs_{k}_%=")
     em.label(f"L_ofs_back_{k}_%=")
     em.raw(f"s_add_u32 {t1}, {t0}, 32")                        # ... of tile t + 4
-    em.raw(f"s_min_i32 {t0}, {t0}, %[last_tile_tok]")          # past the end: the last tile again
+    if not P16:
+        em.raw(f"s_min_i32 {t0}, {t0}, %[last_tile_tok]")      # past the end: the last tile again
     em.raw(f"s_min_i32 {t1}, {t1}, %[last_tile_tok]")
+    if P16:
+        for page, base in (("pg", SB), ("pg2", SB2)):
+            em.raw(f"s_mul_hi_u32 {b}, %[{page}], s{PSTR}")
+            em.raw(f"s_mul_i32 s{base}, %[{page}], s{PSTR}")
+            em.raw(f"s_add_u32 s{base}, s{base}, %[cache_lo]")
+            em.raw(f"s_addc_u32 s{base + 1}, {b}, %[cache_hi]")
+        em.raw(f"s_lshr_b32 {t1}, {t1}, 2")                    # four bytes per page of 16
+        em.raw(f"s_load_dword s{PGN}, %[pages], {t1}")
+        em.raw(f"s_add_u32 {t1}, {t1}, 4")
+        em.raw(f"s_min_i32 {t1}, {t1}, %[last_page]")          # the row's last tile may have one page only
+        em.raw(f"s_load_dword s{PGN2}, %[pages], {t1}")
+        return
     em.raw(f"s_and_b32 {a}, {t0}, s{PMASK}")
     em.raw(f"s_mul_i32 {a}, {a}, %[row_bytes]")                # bytes inside the page (< 2^32)
     em.raw(f"s_mul_hi_u32 {b}, %[pg], s{PSTR}")
@@ -340,7 +370,7 @@ def qk_phase(em, sc, kaddr, copies, extra=None, into_pv=False):
         if f + AHEAD < (68 if into_pv else 36):
             emit_all(em, frag_read(f + AHEAD, kaddr))
         if cp:
-            em.emit(cp[1])
+            emit_all(em, cp[1])
     emit_all(em, extra)
 
 
@@ -359,9 +389,13 @@ def end_of_step(em):
     # newest copies -- tile t + 3's ten, plus tile t + 2's in the plain loop -- are outstanding.  Every LDS read of
     # tile t has returned, so its slot may be refilled after the barrier.
     assert not em.lds_queue
+    # (Pages of 16: the copy that meets both pages is two instructions, one of them without a lane in three of the waves.  The
+    # wait counts it once: whether or not the hardware does so for an instruction without lanes, tile t + 1 has landed.)
     ahead = COPIES if PIPELINED else 2 * COPIES
     em.raw("s_waitcnt lgkmcnt(0)" if "novmwait" in X else f"s_waitcnt vmcnt({ahead}) lgkmcnt(0)", "wait")
     em.raw(f"s_mov_b32 %[pg], s{PGN}")
+    if P16:
+        em.raw(f"s_mov_b32 %[pg2], s{PGN2}")
     if "nobarrier" not in X:
         em.raw("s_barrier")
     em.raw("s_add_u32 %[t], %[t], 1")
@@ -485,24 +519,26 @@ def generate():
     return em
 
 
-def emit_text():
+def emit_text(p16):
+    global P16
+    P16 = p16
     em = generate()
     n_mfma = sum(1 for i in em.out if i.kind == "mfma")
     n_valu = sum(1 for i in em.out if i.kind in ("valu", "trans", "swap", "dot"))
-    pre = "RPA_MLA_WIDE"
+    pre = "RPA_MLA_WIDE_P16" if p16 else "RPA_MLA_WIDE"
     text = (f"// {len(em.out)} lines, {n_mfma} matrix and {n_valu} vector instructions (four unrolled steps, their rare paths "
             f"and masking detours), {em.nops} padding wait states; {NUM_VGPR} vector + 256 accumulation registers\n")
     binds = {f"O{i}": (ACC + 32 * i, 32) for i in range(8)}
     binds.update({"Q0": (0, 32), "Q1": (32, 32), "Q2": (64, 32), "Q3": (96, 32), "Q4": (128, 16),
                   "ML": (ML, 8), "OFS": (OFS, 16), "OFSL": (OFSL, 16)})
-    for name, (lo, n) in binds.items():
+    for name, (lo, n) in ({} if p16 else binds).items():  # (the same registers in both loops)
         text += f'#define {pre}_C_{name} "{{{vr(lo, n)}}}"\n'
-    text += (f"#define {pre}_COPIES_AHEAD {COPIES if PIPELINED else 2 * COPIES}"
+    text += "" if p16 else (f"#define {pre}_COPIES_AHEAD {COPIES if PIPELINED else 2 * COPIES}"
              "  // copies that may be outstanding when a step starts\n")
     lines = ['    "%s\\n"' % ins.text for ins in em.out]
     text += f"#define {pre}_ASM \\\n" + " \\\n".join(lines) + "\n"
     clob = ['"v%d"' % r for r in list(range(SC[0][0], ML)) + list(range(OFSL + 16, NUM_VGPR))]
-    clob += ['"s%d"' % r for r in SGPR_CLOBBERS]
+    clob += ['"s%d"' % r for r in SGPR_CLOBBERS + ([PGN2, SB2, SB2 + 1] if p16 else [])]
     text += f"#define {pre}_CLOBBERS " + ", ".join(clob) + ', "vcc", "scc", "m0", "memory"\n'
     print(f"MLA wide: {len(em.out)} lines, {n_mfma} MFMAs, {n_valu} vector, {em.nops} padding wait states, {NUM_VGPR} VGPRs")
     return text
@@ -514,7 +550,9 @@ def main():
             "// Tile loop of the wide absorbed-MLA kernels: tiles t .. t_end-1 of one wave (two blocks of 16 heads).\n"
             "// The RPA_MLA_WIDE_C_* macros are the register constraints that bind the kernel's variables to the\n"
             "// registers the assembly uses.\n")
-    text += emit_text()
+    text += emit_text(False)
+    if not PIPELINED:
+        text += emit_text(True)
     with open(os.path.join(here, "rpa_mla_wide_loop.inc"), "w") as f:
         f.write(text)
 

@@ -1253,7 +1253,9 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const c
   a.forced_tiles_per_wg = 0;
   a.piece_pad = rpa::tuning().mla_piece_pad >= 0
                     ? rpa::tuning().mla_piece_pad
-                    : rpa::select_shape(rpa::mla_shape_key(a), rpa::mla_shape_skip(rpa::tuning())).piece_pad;
+                    : rpa::mla_takes_wide_p16(a, true)
+                          ? 12  // (the wide kernels' in the shape table)
+                          : rpa::select_shape(rpa::mla_shape_key(a), rpa::mla_shape_skip(rpa::tuning())).piece_pad;
   if (p->num_splits > 0) {
     const int64_t bound = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages,
                                        p->cu_kv_lens != nullptr);
@@ -1300,11 +1302,12 @@ int rpa_mla_describe_plan(const RpaMlaParams* p, int token_rows, char* buf, size
   a.balanced = bal ? 1 : 0;
   static const char* const kGroups[] = {"off", "eight_waves_compiled", "eight_waves", "wide"};
   const int tg = rpa::mla_token_group_mode(a, rpa::tuning(), r);
+  const bool p16 = !tg && rpa::mla_takes_wide_p16(a, true);
   return snprintf(buf, len, "mla: shape=%s rows=%lld waves_per_wg=%d heads_per_wg=%d share=%d token_groups=%s plan=%s "
-                  "pieces_per_row=%d workgroups=%d workspace=%zu\n",
-                  r.name, (long long)rows, tg == 3 ? 4 : r.waves_per_wg, tg ? 128 : r.tile_heads, tg ? 1 : r.share, kGroups[tg],
+                  "pieces_per_row=%d workgroups=%d workspace=%zu%s\n",
+                  r.name, (long long)rows, tg == 3 || p16 ? 4 : r.waves_per_wg, tg ? 128 : r.tile_heads, tg ? 1 : r.share, kGroups[tg],
                   bal ? "balanced" : "fixed", bal ? 0 : sp.splits, bal ? mla_wgs() : 0,
-                  mla_workspace(p, rows, token_rows != 0));
+                  mla_workspace(p, rows, token_rows != 0), p16 ? " (the wide loop of pages of 16 tokens)" : "");
 }
 
 int rpa_mla_decode(const RpaMlaParams* p, void* stream) {

@@ -246,6 +246,7 @@ ShapeKey mla_shape_key(const MlaDecodeArgs& a);
 unsigned mla_shape_skip(const Tuning& tune);
 // how query tokens of a chunk share a workgroup (0: they do not; 1, 2: eight waves; 3: wide workgroups)
 int mla_token_group_mode(const MlaDecodeArgs& a, const Tuning& tune, const ShapeRule& shape);
+bool mla_takes_wide_p16(const MlaDecodeArgs& a, bool heads_in_128s);
 hipError_t launch_sparse_table(const SparseMlaArgs& a, hipStream_t stream);
 hipError_t launch_mla_kv_write(const MlaWriteArgs& a, hipStream_t stream);
 

@@ -200,6 +200,20 @@ __device__ __forceinline__ void copy_tile(char* slot, const Src& s, const char* 
   }
 }
 
+// The wide kernels' prologue on pages of 16 tokens: rows 0 .. 15 of a tile in page `pg`, the others in `pg2`.
+template <int CPW>
+__device__ __forceinline__ void copy_tile_p16(char* slot, const Src& s, const char* cache, int tb, int wave, int lane, int pg, int pg2) {
+  tb = min(tb, s.last_tok & ~(kTok - 1));
+#pragma unroll
+  for (int n = 0; n < CPW; ++n) {
+    int row, inner;
+    chunk_of<CPW>(s, wave, lane, n, row, inner);
+    row = min(row, s.last_tok - tb);
+    async_copy16(cache + (int64_t)(row >= 16 ? pg2 : pg) * s.page_stride + (row & 15) * s.row_bytes + inner,
+                 slot + copy_block<CPW>(wave, n) * 1024);
+  }
+}
+
 // fp8 caches: the same copy, of a tile of bytes into a staging area.  Position p = 64 * block + lane
 // is chunk p % 36 of row p / 36; chunks 0..31 are kv_c, 32..35 k_pe.
 __device__ __forceinline__ int f8_copy_block(int wave, int n) {
@@ -802,11 +816,12 @@ constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 // is "head" 32 w + 16 hb .. of a 128-head row at mr.tq, i.e. token (32 w + 16 hb) / Hq of the group; mr.kv_len is what
 // the group's LAST token sees, a block's own token sees up to group_tokens - 1 fewer, so the loop masks the
 // tile before the last too and takes the second block's row end relative to the first's.
-template <bool M32, bool TG = false>
+// P16: pages of 16 tokens, on the loop that has a scalar base for each half of a tile.
+template <bool M32, bool TG = false, bool P16 = false>
 __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const MlaRow mr, int head_base, int t_lo,
                                                  int t_begin, int t_end, const MlaDest dest, char* ring,
                                                  int trace_piece = 0, int group_tokens = 1) {
-  static_assert(!(M32 && TG), "token groups run on the loop of two 16-head blocks");
+  static_assert(!(M32 && (TG || P16)), "token groups and pages of 16 tokens run on the loop of two 16-head blocks");
   (void)trace_piece;
   RPA_MLA_STAMP(0);
   constexpr int CPW = 2 * kCopiesPerWave;
@@ -851,6 +866,10 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
     tb = min(tb, src.last_tok & ~(kTok - 1));
     return scalar_load_i32(src.pages + __builtin_amdgcn_readfirstlane(page_slot(src, tb)));
   };
+  auto second_page_of = [&](int tb) -> int {  // P16: the page of the tile's last 16 rows (of its first ones where it ends there)
+    tb = min(tb, src.last_tok & ~(kTok - 1));
+    return scalar_load_i32(src.pages + __builtin_amdgcn_readfirstlane(min(page_slot(src, tb) + 1, page_slot(src, src.last_tok))));
+  };
 
   // ---- Q^T operands: column c of block hb = head head0 + 16 hb + c, k-step ks covers dims 32ks + 8g .. ----
   // 16x16x32: qB[hb][ks], k-step ks covers dims 32ks + 8g ..; 32x32x16: the same 36 registers of 4 as
@@ -877,9 +896,13 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
   const float scale2 = a.sm.sm_scale * kLog2e;
 
   int pg_next = page_of(t_begin + 3 * kTok);
-  copy_tile<true, CPW>(ring, src, a.cache, t_begin, wave, lane, page_of(t_begin));
-  copy_tile<true, CPW>(ring + kSlotB, src, a.cache, t_begin + kTok, wave, lane, page_of(t_begin + kTok));
-  copy_tile<true, CPW>(ring + 2 * kSlotB, src, a.cache, t_begin + 2 * kTok, wave, lane, page_of(t_begin + 2 * kTok));
+  int pg2_next = P16 ? second_page_of(t_begin + 3 * kTok) : 0;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int tb = t_begin + i * kTok;
+    if constexpr (P16) copy_tile_p16<CPW>(ring + i * kSlotB, src, a.cache, tb, wave, lane, page_of(tb), second_page_of(tb));
+    else copy_tile<true, CPW>(ring + i * kSlotB, src, a.cache, tb, wave, lane, page_of(tb));
+  }
 #pragma unroll
   for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
@@ -986,8 +1009,9 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
   for (int n = 0; n < CPW; ++n) {
     int row, inner;
     chunk_of<CPW>(src, wave, ln, n, row, inner);
-    ofs[n] = (uint32_t)(row * src.row_bytes + inner);
-    ofsl[n] = (uint32_t)(min(row, last_row) * src.row_bytes + inner);
+    // (P16: from the row's page; rows clamped below 16 are in the first page, which is the second one too then)
+    ofs[n] = (uint32_t)((P16 ? row & 15 : row) * src.row_bytes + inner);
+    ofsl[n] = (uint32_t)((P16 ? min(row, last_row) & 15 : min(row, last_row)) * src.row_bytes + inner);
   }
   const uint32_t cache_lo = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)a.cache);
   const uint32_t cache_hi = __builtin_amdgcn_readfirstlane((uint32_t)((uintptr_t)a.cache >> 32));
@@ -1009,6 +1033,20 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
     [wave_blk] "s"(wave_blk), [slot0] "s"(lds_base), [hi_step] "s"(hi_step), [mask_early] "s"(mask_early)
   if constexpr (M32) {
     asm volatile(RPA_MLA_WIDE32_ASM RPA_WIDE_OPERANDS : RPA_MLA_WIDE32_CLOBBERS);
+  } else if constexpr (P16) {
+    // lanes of this wave's copy 4 whose chunks belong to rows of the first page
+    const uint64_t mask_a = __builtin_amdgcn_ballot_w64((wave + 4 * 4) * 64 + ln < 16 * kChunks), mask_b = ~mask_a;
+    const int last_page = __builtin_amdgcn_readfirstlane(page_slot(src, src.last_tok) * 4);
+    asm volatile(RPA_MLA_WIDE_P16_ASM
+                 : "+" C(O0)(o[0]), "+" C(O1)(o[1]), "+" C(O2)(o[2]), "+" C(O3)(o[3]), "+" C(O4)(o[4]), "+" C(O5)(o[5]),
+                   "+" C(O6)(o[6]), "+" C(O7)(o[7]), "+" C(ML)(ml), "+" C(OFS)(ofs), [t] "+&s"(k), [pg] "+&s"(pg_next),
+                   [pg2] "+&s"(pg2_next)
+                 : C(Q0)(q0), C(Q1)(q1), C(Q2)(q2), C(Q3)(q3), C(Q4)(q4), C(OFSL)(ofsl), [t_end] "s"(nT), [t_begin] "s"(t_begin),
+                   [last_tile_tok] "s"(last_tile_tok), [row_bytes] "s"(src.row_bytes), [pshift] "s"(src.page_shift),
+                   [cache_lo] "s"(cache_lo), [cache_hi] "s"(cache_hi), [pages] "s"(src.pages), [scale2] "s"(scale2_bits),
+                   [wave_blk] "s"(wave_blk), [slot0] "s"(lds_base), [hi_step] "s"(hi_step), [mask_early] "s"(mask_early),
+                   [mask_a] "s"(mask_a), [mask_b] "s"(mask_b), [last_page] "s"(last_page)
+                 : RPA_MLA_WIDE_P16_CLOBBERS);
   } else {
     asm volatile(RPA_MLA_WIDE_ASM RPA_WIDE_OPERANDS : RPA_MLA_WIDE_CLOBBERS);
   }
@@ -1141,6 +1179,7 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_token_group_kernel(const MlaDe
 
 // ---- token groups on wide workgroups (see mla_segment_wide, TG): bf16 latents, no window.  Same grid and the same
 // walk over a window of 128 / Hq query tokens as rpa_mla_token_group_kernel.
+template <bool P16>
 __global__ __launch_bounds__(256, 1) void rpa_mla_token_group_wide_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char ring[4 * kSlotB];
   const int num_seqs = a.dist ? min(a.num_seqs, scalar_load_i32(a.dist + 2)) : a.num_seqs;
@@ -1169,7 +1208,7 @@ __global__ __launch_bounds__(256, 1) void rpa_mla_token_group_wide_kernel(const 
       MlaDest dest;
       dest.final_rows = true;
       dest.base = 0;
-      mla_segment_wide<false, true>(a, mr, 0, 0, 0, mr.kv_len, dest, ring, 0, n);
+      mla_segment_wide<false, true, P16>(a, mr, 0, 0, 0, mr.kv_len, dest, ring, 0, n);
     }
     t += n;
     if (t >= q1) ++seq;
@@ -1177,7 +1216,7 @@ __global__ __launch_bounds__(256, 1) void rpa_mla_token_group_wide_kernel(const 
 }
 
 // ---- fixed split plan, wide workgroups: grid = (max_splits * rows, 1, head groups of 128); block = 256 threads
-template <bool M32>
+template <bool M32, bool P16 = false>
 __global__ __launch_bounds__(256, 1) void rpa_mla_decode_wide_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char ring[4 * kSlotB];
   const int nsp = max(a.max_splits, 1);  // grid.x = max_splits * rows, splits fastest
@@ -1195,7 +1234,7 @@ __global__ __launch_bounds__(256, 1) void rpa_mla_decode_wide_kernel(const MlaDe
   MlaDest dest;
   dest.final_rows = a.max_splits == 1;
   dest.base = ((int64_t)row_id * a.max_splits + split) * a.Hq;
-  mla_segment_wide<M32>(a, mr, blockIdx.z * 128, t_lo, t_begin, t_end, dest, ring);
+  mla_segment_wide<M32, false, P16>(a, mr, blockIdx.z * 128, t_lo, t_begin, t_end, dest, ring);
 }
 
 // ---- balanced plan (one row per sequence): the 32-token tiles of the whole batch, sequence by
@@ -1346,12 +1385,12 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_balanced_kernel(const MlaDecod
 }
 
 // the same plan on wide workgroups (four waves of 32 heads)
-template <bool M32>
+template <bool M32, bool P16 = false>
 __global__ __launch_bounds__(256, 1) void rpa_mla_balanced_wide_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char ring[4 * kSlotB];
   mla_balanced_body(a, [&](const MlaRow& mr, int head_base, int t_lo, int t_begin, int t_end, const MlaDest& dest,
                            int piece) __attribute__((always_inline)) {
-    mla_segment_wide<M32>(a, mr, head_base, t_lo, t_begin, t_end, dest, ring, piece);
+    mla_segment_wide<M32, false, P16>(a, mr, head_base, t_lo, t_begin, t_end, dest, ring, piece);
   });
 }
 
@@ -1480,6 +1519,17 @@ hipError_t launch_mla_kv_write(const MlaWriteArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Pages of 16 tokens, two per tile: the wide loop has a variant for them (`heads_in_128s`: and the call's heads are for wide
+// workgroups without being grouped by tokens).  Its row of the shape table is that of small pages.
+// Other pages under a tile look every row's page up in LDS, and the compiled loop takes them.  Compiled -> wide: 64 rows of
+// 2048 .. 16384 tokens x 128 heads 282.4 -> 180.5 us (178.7 on pages of 64), chunks of 512 on 4096 3040 -> 1832 us, 7 prompts of
+// 16 .. 683 tokens 515 -> 354; 64 heads, 3 chunks of 74 .. 165 tokens on up to 1955 204 -> 105 us.
+bool mla_takes_wide_p16(const MlaDecodeArgs& a, bool heads_in_128s) {
+  const Tuning& tune = tuning();
+  return a.pt.page_size == 16 && !a.fp8 && !a.extra_rows && a.sm.soft_cap == 0.f && tune.mla_wide == 1 && tune.mla_pipe != 0 &&
+         (!heads_in_128s || a.Hq % 128 == 0);
+}
+
 ShapeKey mla_shape_key(const MlaDecodeArgs& a) {
   const int P = a.pt.page_size;
   ShapeKey k = {};
@@ -1509,6 +1559,7 @@ int mla_token_group_mode(const MlaDecodeArgs& a, const Tuning& tune, const Shape
     return 0;
   const int P = a.pt.page_size;
   const bool pipe_ok = tune.mla_pipe != 0 && (P & (P - 1)) == 0 && (P % kTok) == 0 && (int64_t)a.row_stride * 2 * P < (int64_t(1) << 32);
+  if (mla_takes_wide_p16(a, false) && a.sm.window <= 0) return 3;
   if (!pipe_ok) return 1;
   if (!a.fp8 && a.sm.window <= 0 && tune.mla_wide != 0 && tune.mla_wide != 32) return 3;
   return 2;
@@ -1535,7 +1586,8 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     const int per = 128 / a.Hq;
     const dim3 tg_grid((unsigned)((a.num_rows + per - 1) / per));
     if (tg == 3) {
-      hipLaunchKernelGGL(rpa_mla_token_group_wide_kernel, tg_grid, dim3(256), 0, stream, a);
+      if (a.pt.page_size == 16) hipLaunchKernelGGL(rpa_mla_token_group_wide_kernel<true>, tg_grid, dim3(256), 0, stream, a);
+      else hipLaunchKernelGGL(rpa_mla_token_group_wide_kernel<false>, tg_grid, dim3(256), 0, stream, a);
       return hipGetLastError();
     }
     if (a.fp8) {
@@ -1618,7 +1670,8 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   }
   // wide workgroups (four waves of 32 heads) wherever the assembly loop applies; RPA_MLA_WIDE=0 keeps the
   // eight-wave kernels
-  const bool wide = shape.kernel == kKernelMlaWide;
+  const bool p16 = mla_takes_wide_p16(a, true);
+  const bool wide = shape.kernel == kKernelMlaWide || p16;
   // RPA_MLA_WIDE=32: the wide loop on 32x32x16 matrix instructions (one head per lane and half).  Half the matrix
   // instructions, and 8 % faster than the default loop when neither reads its operands -- but its 32-row LDS
   // reads collide on the 1184-byte row pitch that suits the 16-row reads (7 % slower as a whole): opt-in until
@@ -1626,6 +1679,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   const bool m32 = tune.mla_wide == 32;
   if (wide && a.balanced) {
     if (m32) hipLaunchKernelGGL(rpa_mla_balanced_wide_kernel<true>, dim3(a.num_wgs), dim3(256), 0, stream, a);
+    else if (p16) hipLaunchKernelGGL((rpa_mla_balanced_wide_kernel<false, true>), dim3(a.num_wgs), dim3(256), 0, stream, a);
     else hipLaunchKernelGGL(rpa_mla_balanced_wide_kernel<false>, dim3(a.num_wgs), dim3(256), 0, stream, a);
     hipError_t eb = hipGetLastError();
     if (eb != hipSuccess) return eb;
@@ -1634,6 +1688,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   }
   if (wide) {
     if (m32) hipLaunchKernelGGL(rpa_mla_decode_wide_kernel<true>, grid, dim3(256), 0, stream, a);
+    else if (p16) hipLaunchKernelGGL((rpa_mla_decode_wide_kernel<false, true>), grid, dim3(256), 0, stream, a);
     else hipLaunchKernelGGL(rpa_mla_decode_wide_kernel<false>, grid, dim3(256), 0, stream, a);
     hipError_t ew = hipGetLastError();
     if (ew != hipSuccess) return ew;

@@ -775,3 +775,36 @@ def test_mla_token_groups_with_the_composition_on_the_device(pkg, wl, gpu):
     assert_parity(dev[:T].cpu().float(), want.float(), **TOL)
     assert torch.equal(dev[:T].view(torch.int16), host[:T].view(torch.int16))
 
+
+
+@pytest.mark.parametrize("kind,Hq,window", [("rows", 128, None), ("rows", 256, 40), ("long", 128, None), ("chunks", 128, None), ("chunks", 16, None),
+                                            ("chunks", 64, None), ("chunks", 32, 100)])
+def test_mla_pages_of_16_tokens_on_wide_workgroups(pkg, wl, gpu, kind, Hq, window):
+    """Two pages per tile, the row border inside a copy block: lengths around half and whole tiles, everything that no row
+    owns NaN, against the oracle and, bit for bit, against the same rows on pages of 64 tokens."""
+    edges = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 64, 96, 113, 129, 300]
+    q_lens, kv_lens = {"rows": ([1] * 15, edges), "long": ([1] * 3, [4001, 2064, 1]),
+                       "chunks": ([1, 16, 17, 5, 40], [1, 16, 49, 133, 700])}[kind]
+    b = wl.make_mla_batch("mla_p16", q_lens, kv_lens, num_q_heads=Hq, lkv_dim=512, rope_dim=64, page_size=16, seed=611,
+                          sm_scale=192 ** -0.5, sliding_window=window)
+    if window is None:
+        wl.plant_mla_needles(b, seed=3)
+    say(f"mla pages of 16: {kind} Hq={Hq} window={window}")
+    T, want = sum(q_lens), oracle(b)
+    table = b.padded_page_indices().reshape(len(kv_lens), -1)
+    used = torch.zeros(b.cache_kv.shape[:2], dtype=torch.bool)
+    n64 = [-(-kv // 64) for kv in kv_lens]
+    cache64 = torch.full((sum(n64), 64, 576), float("nan"), dtype=torch.bfloat16)
+    for i, kv in enumerate(kv_lens):
+        t = torch.arange(kv)
+        used[table[i][t // 16].long(), t % 16] = True
+        cache64[sum(n64[:i]) + t // 64, t % 64] = b.cache_kv[table[i][t // 16].long(), t % 16]
+    b.cache_kv[~used] = float("nan")
+    got = run_gpu(pkg, b, gpu)[:T]
+    assert_parity(got.float(), want[:T].float(), **TOL)
+    b.cache_kv, b.page_size = cache64, 64
+    b.page_indices = torch.arange(sum(n64), dtype=torch.int32)
+    b.cu_kv_lens = torch.tensor([0] + [64 * sum(n64[: i + 1]) for i in range(len(n64))], dtype=torch.int32)
+    same = run_gpu(pkg, b, gpu)[:T]
+    if Hq >= 128 or window is None:  # (groups of query tokens behind a window run on eight waves)
+        assert torch.equal(got.view(torch.int16), same.view(torch.int16))
