@@ -104,6 +104,10 @@ struct KvWriteArgs {
   int32_t skip_decode_rows;
 };
 
+struct FastDiv {
+  uint32_t mul, shift;
+};
+
 struct PrefillArgs {
   const uint16_t* q;
   uint16_t* out;
@@ -143,6 +147,9 @@ struct PrefillArgs {
   // never had that
   uint32_t page_options;
   int32_t packed;  // rpa_prefill_packed_kernel takes the call, K/V ranges in so many pieces where there is room for them; 0 = not
+  struct {
+    FastDiv groups, units, hkv, nseq;
+  } map;  // set by the launchers (prefill_grid)
 };
 
 struct GatherArgs {

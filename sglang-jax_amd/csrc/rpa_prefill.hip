@@ -938,7 +938,8 @@ size_t prefill_split_workspace_bytes(const PrefillArgs& a, int splits) {
   return splits > 1 ? (size_t)a.num_tokens * a.Hq * splits * (a.head_dim + 2) * sizeof(float) : 0;
 }
 
-hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
+hipError_t launch_prefill(const PrefillArgs& call, hipStream_t stream) {
+  PrefillArgs a = call;
   const int nseq = a.seq_end - a.seq_begin;
   if (nseq <= 0 || a.max_q_len <= 0) return hipSuccess;
   if (a.packed) {
@@ -960,8 +961,7 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) {
   const int levels = a.max_kv_len > 0 ? (a.max_kv_len + bm - 1) / bm + 1 : 0;
   const bool by_level = level_order && a.sm.mask_mode == 0 && levels > tiles && levels <= 2 * tiles + 2;
   if (by_level) tiles = levels;
-  const int64_t units = (int64_t)nseq * a.Hkv;
-  const int64_t grid = (units >= 8 ? ((units + 7) / 8) * 8 : units) * (heads4 ? a.G / 4 : a.G) * tiles;
+  const int64_t grid = prefill_grid(a, nseq, tiles, heads4 ? 4 : 1);
   if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   const bool uniform = (a.pt.page_size % kBN) == 0;
   // soft cap and logit rounding share the general score path

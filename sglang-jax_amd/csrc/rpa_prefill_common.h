@@ -70,18 +70,34 @@ __device__ __forceinline__ int64_t row_offset(const TileSrc& s, const KvAddr& kv
 }
 
 // ------------------------------------------------------------------ work decomposition
-// A unit is one (sequence, kv head): its G query heads and all their query tiles read the
-// same K/V, so a unit stays on one XCD (one L2).  Hardware deals workgroup n to XCD n % 8;
-// XCD x owns units x, x+8, ...: units of one sequence cost the same, so the XCDs stay
-// balanced whatever the ragged lengths are.  Inside an XCD the G heads of a unit sit next to
-// each other and the most expensive query tiles are issued first, so that the last workgroups
-// to start are short ones.  A causal tile costs what its last row sees: with a bound on kv_len
-// from the host, tiles are ordered by level = tile index + ceil(prefix / tile rows), i.e. by
-// that extent across sequences; without one, by position inside their own sequence.
+// A unit is one (sequence, kv head): its G query heads and all their query tiles read the same K/V.  Hardware deals
+// workgroup n to XCD n % 8, and inside an XCD to its four shader engines in turn, whatever they have left to do.  So
+//   * the G heads of a (unit, tile) pair sit next to each other on one XCD (one L2); pairs go round the XCDs, tile by tile;
+//   * the places of a sequence's pairs change with the tile.  A ragged sequence, which has
+//     workgroups for its own length only, then meets every shader engine, and with fewer than 8 kv heads other XCDs too (with
+//     8, 16, ... its kv heads stay on theirs).  Six chunks of 341 .. 1473 tokens x 16 / 8 heads of 256 dims, in the same places
+//     for every tile, had left 4 workgroups to each of 112 CUs and 1 to 48: 262.6 -> 203.5 us.  7 prompts of 264 .. 1643 tokens x 8 / 2 heads 46.6 -> 37.1, 4 prompts of 484 ..
+//     2368 x 16 / 8 heads 119 -> 87; odd numbers of sequences and 4 heads per kv head are where they were.
+// The most expensive query tiles are issued first, so that the last workgroups to start are short ones.  A causal tile costs
+// what its last row sees: with a bound on kv_len from the host, tiles are ordered by level = tile index + ceil(prefix / tile
+// rows), i.e. by that extent across sequences; without one, by position inside their own sequence.
 struct Work {
   int seq, hk, head, q_start, qg0, q_len, kv_len, prefix;
   bool valid;
 };
+
+// n / d by a multiplication, for n < 2^31: scalar instructions, where a division is some 40 of the vector pipe, one after the
+// other, in front of everything else that a workgroup does.
+__device__ __forceinline__ int by(int n, const FastDiv& d) {
+  return (int)((__umulhi((uint32_t)n, d.mul) + (uint32_t)n) >> d.shift);
+}
+inline FastDiv fast_div(int d) {
+  FastDiv f;
+  f.shift = 0;
+  while (((int64_t)1 << f.shift) < d) ++f.shift;
+  f.mul = (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << f.shift) - (uint64_t)d)) / (uint64_t)d + 1);
+  return f;
+}
 
 // `heads` query heads of a kv head per workgroup (1, or 4 when the waves of a workgroup take a head each):
 // Work.head is then the first of them.
@@ -91,25 +107,17 @@ __device__ __forceinline__ Work decompose(const PrefillArgs& a, int tiles, int n
   w.valid = false;
   const int units = nseq * a.Hkv;
   const int groups = a.G / heads;  // workgroups per (sequence, kv head, tile)
-  int tile_rev, u, gi;
-  if (units >= 8) {
-    const int xcd = blockIdx.x & 7, r = blockIdx.x >> 3;
-    const int units_per_xcd = (units + 7) >> 3;
-    const int per_tile = units_per_xcd * groups;
-    tile_rev = r / per_tile;
-    const int rest = r - tile_rev * per_tile;
-    u = xcd + 8 * (rest / groups);
-    gi = (rest % groups) * heads;
-  } else {
-    const int per_tile = units * groups;
-    tile_rev = blockIdx.x / per_tile;
-    const int rest = blockIdx.x - tile_rev * per_tile;
-    u = rest / groups;
-    gi = (rest % groups) * heads;
+  const int r = blockIdx.x >> 3, rg = by(r, a.map.groups), gi = (r - rg * groups) * heads;
+  const int pair = rg * 8 + (blockIdx.x & 7);
+  const int tile_rev = by(pair, a.map.units);
+  if (tile_rev >= tiles) return w;
+  const int place = pair - tile_rev * units;
+  int si = by(place, a.map.hkv);
+  w.hk = place - si * a.Hkv;
+  if ((nseq & 1) == 0) {  // (an odd number of them moves on by itself)
+    si += nseq == 2 ? tile_rev >> 1 : tile_rev;
+    si -= by(si, a.map.nseq) * nseq;
   }
-  if (u >= units || tile_rev >= tiles) return w;
-  const int si = u / a.Hkv;
-  w.hk = u - si * a.Hkv;
   w.head = w.hk * a.G + gi;
   w.seq = a.seq_begin + si;
   if (w.seq >= a.seq_end) return w;  // the grid was sized for a bound on the number of sequences
@@ -125,6 +133,15 @@ __device__ __forceinline__ Work decompose(const PrefillArgs& a, int tiles, int n
   if (tile < 0 || w.q_start >= w.q_len) return w;
   w.valid = true;
   return w;
+}
+
+// Workgroups of a launch of `tiles` tiles, and the divisors of their order (see decompose).
+inline int64_t prefill_grid(PrefillArgs& a, int nseq, int tiles, int heads) {
+  a.map.groups = fast_div(a.G / heads);
+  a.map.units = fast_div(nseq * a.Hkv);
+  a.map.hkv = fast_div(a.Hkv);
+  a.map.nseq = fast_div(nseq);
+  return ((int64_t)nseq * a.Hkv * tiles + 7) / 8 * 8 * (a.G / heads);
 }
 
 // K (or V) rows of the workgroup's kv head, token 0 of its sequence's first page.

@@ -510,11 +510,11 @@ int prefill_packed_pieces(const PrefillArgs& a) {
   return best_us < other ? best : 0;
 }
 
-hipError_t launch_prefill_packed(const PrefillArgs& a, int nseq, hipStream_t stream) {
+hipError_t launch_prefill_packed(const PrefillArgs& call, int nseq, hipStream_t stream) {
+  PrefillArgs a = call;
   const int per = kCols / a.G;
   const int tiles = (a.max_q_len + per - 1) / per;
-  const int64_t units = (int64_t)nseq * a.Hkv;
-  const int64_t grid = (units >= 8 ? ((units + 7) / 8) * 8 : units) * tiles;
+  const int64_t grid = prefill_grid(a, nseq, tiles, a.G);
   if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   const bool cut = a.kv_splits > 1;
   if (cut && (!a.ws_o || !a.ws_ml || a.kv_splits > 64)) return hipErrorInvalidValue;

@@ -547,7 +547,8 @@ int prefill_pipe_kv_splits(const PrefillArgs& a, int nseq, double* us) {
   return kv_pieces(a, nseq, heads4 ? 32 : 128, heads4 ? 4 : 1, 0.8, us);
 }
 
-hipError_t launch_prefill_pipe(const PrefillArgs& a, int nseq, bool level_order, hipStream_t stream) {
+hipError_t launch_prefill_pipe(const PrefillArgs& call, int nseq, bool level_order, hipStream_t stream) {
+  PrefillArgs a = call;
   const int force_nq = forced_nq();
   // a half's row sum above the limit sends a wave through the rescaling path (testing knob: -1 = always)
   const float limit = tuning().prefill_pipe_limit != 0.f ? tuning().prefill_pipe_limit : kRowSumLimit;
@@ -561,8 +562,7 @@ hipError_t launch_prefill_pipe(const PrefillArgs& a, int nseq, bool level_order,
   const int levels = a.max_kv_len > 0 ? (a.max_kv_len + bm - 1) / bm + 1 : 0;
   const bool by_level = level_order && levels > tiles && levels <= 2 * tiles + 2;
   if (by_level) tiles = levels;
-  const int64_t units = (int64_t)nseq * a.Hkv;
-  const int64_t grid = (units >= 8 ? ((units + 7) / 8) * 8 : units) * (heads4 ? a.G / 4 : a.G) * tiles;
+  const int64_t grid = prefill_grid(a, nseq, tiles, heads4 ? 4 : 1);
   if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   const dim3 g((unsigned)(grid + a.write_blocks)), blk(256);
   const bool win = a.sm.window > 0;
