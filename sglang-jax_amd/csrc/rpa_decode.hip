@@ -1243,6 +1243,8 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
 // (nearly always) everything is requested at once -- the (max, sum) pairs by lanes 0..n-1, the
 // partial rows by all lanes, the row's query token before either -- so the merge costs one round
 // trip to memory instead of three dependent ones.
+constexpr int kMergeWaves = 4;
+
 template <int N, int HD, typename SlotOf>
 __device__ __forceinline__ void merge_few(const DecodeArgs& a, int n, int lane, SlotOf slot_of, float& mstar,
                                           float& den, float (&acc)[HD / 64]) {
@@ -1277,56 +1279,89 @@ __device__ __forceinline__ void merge_few(const DecodeArgs& a, int n, int lane, 
   }
 }
 
+// More than 16 partials (a few rows cut over the whole chip): the waves of the workgroup take 16 partial rows each in turn, and
+// wave 0 adds what they have.  One wave with 32 rows at a time behind two passes over the references was a chain of up to
+// seven round trips: 7 rows of 221 .. 6024 tokens x 8 heads 11.1 -> 6.0 us, 2 rows of
+// 20000 .. 30000 x 8 heads 9.0 -> 4.8.  Returns whether this wave goes on to write.
+template <int HD, typename SlotOf>
+__device__ __forceinline__ bool merge_many(const DecodeArgs& a, int n, int lane, SlotOf slot_of, float& mstar, float& den,
+                                           float (&acc)[HD / 64]) {
+  constexpr int kDpl = HD / 64;
+  typedef float fvec_t __attribute__((ext_vector_type(kDpl)));
+  __shared__ float sums[kMergeWaves - 1][HD];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  for (int b0 = 0; b0 < n; b0 += 256) {  // references and sums of 256 partials in one round trip
+    float mj[4], lj[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = b0 + 64 * u + lane;
+      mj[u] = -INFINITY;
+      lj[u] = 0.f;
+      if (j < n) {
+        const int64_t slot = slot_of(j);
+        mj[u] = a.ws_ml[slot * 2];
+        lj[u] = a.ws_ml[slot * 2 + 1];
+      }
+    }
+    float top = fmaxf(fmaxf(mj[0], mj[1]), fmaxf(mj[2], mj[3]));
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off));
+    top = fmaxf(mstar, top);
+    const float keep = b0 > 0 ? fast_exp2(mstar - top) : 0.f;
+    mstar = top;
+    den *= keep;
+#pragma unroll
+    for (int e = 0; e < kDpl; ++e) acc[e] *= keep;
+    float wj[4], lsum = 0.f;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      wj[u] = b0 + 64 * u + lane < n ? fast_exp2(mj[u] - mstar) : 0.f;
+      lsum += lj[u] * wj[u];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
+    den += lsum;
+    for (int j0 = b0 + wave * 16; j0 < min(n, b0 + 256); j0 += waves * 16) {
+      const int part = (j0 - b0) >> 6, first = (j0 - b0) & 63;
+      const float wp = part == 0 ? wj[0] : part == 1 ? wj[1] : part == 2 ? wj[2] : wj[3];
+      fvec_t o[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) o[u] = *reinterpret_cast<const fvec_t*>(a.ws_o + slot_of(min(j0 + u, n - 1)) * HD + lane * kDpl);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const float wu = __shfl(wp, first + u);  // 0 beyond n: the repeated last row does not count
+#pragma unroll
+        for (int e = 0; e < kDpl; ++e) acc[e] += o[u][e] * wu;
+      }
+    }
+  }
+  if (waves == 1) return true;
+  if (wave > 0) {
+#pragma unroll
+    for (int e = 0; e < kDpl; ++e) sums[wave - 1][lane * kDpl + e] = acc[e];
+  }
+  __syncthreads();
+  if (wave > 0) return false;
+  for (int w = 0; w < waves - 1; ++w)
+#pragma unroll
+    for (int e = 0; e < kDpl; ++e) acc[e] += sums[w][lane * kDpl + e];
+  return true;
+}
+
 template <int HD = 128, typename SlotOf>
 __device__ __forceinline__ void merge_rows(const DecodeArgs& a, int tq, int head, int n, int lane, SlotOf slot_of) {
   constexpr int kDpl = HD / 64;  // dims per lane
-  typedef float fvec_t __attribute__((ext_vector_type(kDpl)));
   const int d = lane * kDpl;
   float mstar = -INFINITY, den = 0.f;
   float acc[kDpl];
 #pragma unroll
   for (int e = 0; e < kDpl; ++e) acc[e] = 0.f;
-  if (n <= 8) {
-    merge_few<8, HD>(a, n, lane, slot_of, mstar, den, acc);
-  } else if (n <= 16) {
-    merge_few<16, HD>(a, n, lane, slot_of, mstar, den, acc);
-  } else {
-    for (int j0 = 0; j0 < n; j0 += 64) {
-      const int j = j0 + lane;
-      float mj = (j < n) ? a.ws_ml[slot_of(j) * 2] : -INFINITY;
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) mj = fmaxf(mj, __shfl_xor(mj, off));
-      mstar = fmaxf(mstar, mj);
-    }
-    for (int j0 = 0; j0 < n; j0 += 64) {
-      const int j = j0 + lane;
-      float wj = 0.f, lj = 0.f;
-      if (j < n) {
-        const int64_t slot = slot_of(j);
-        wj = fast_exp2(a.ws_ml[slot * 2] - mstar);
-        lj = a.ws_ml[slot * 2 + 1] * wj;
-      }
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) lj += __shfl_xor(lj, off);
-      den += lj;
-      // 32 partial rows requested at a time: a row with hundreds of partials (one long
-      // sequence cut over the whole GPU) is a chain of such round trips
-      const int cnt = min(64, n - j0);
-      for (int jj = 0; jj < cnt; jj += 32) {
-        fvec_t o[32];
-        float wv[32];
-#pragma unroll
-        for (int u = 0; u < 32; ++u) {
-          const int js = min(jj + u, cnt - 1);
-          wv[u] = (jj + u < cnt) ? __shfl(wj, js) : 0.f;
-          o[u] = *reinterpret_cast<const fvec_t*>(a.ws_o + slot_of(j0 + js) * HD + d);
-        }
-#pragma unroll
-        for (int u = 0; u < 32; ++u)
-#pragma unroll
-          for (int e = 0; e < kDpl; ++e) acc[e] += o[u][e] * wv[u];
-      }
-    }
+  if (n <= 16) {
+    if (threadIdx.x >= 64) return;
+    if (n <= 8) merge_few<8, HD>(a, n, lane, slot_of, mstar, den, acc);
+    else merge_few<16, HD>(a, n, lane, slot_of, mstar, den, acc);
+  } else if (!merge_many<HD>(a, n, lane, slot_of, mstar, den, acc)) {
+    return;
   }
   const float inv = a.sm.sink ? sink_inverse(mstar, den, sink_logit(a.sm.sink, a.sm.round_logits, head)) : 1.0f / den;
   if (d >= a.q_dim) return;
@@ -1335,14 +1370,18 @@ __device__ __forceinline__ void merge_rows(const DecodeArgs& a, int tq, int head
   for (int e = 0; e < kDpl; e += 2) op[e / 2] = pack_bf16x2(acc[e] * inv, acc[e + 1] * inv);
 }
 
-// Merge the partial rows of the balanced plan.  grid = (Hq * decode rows); block = one wave.
-__global__ __launch_bounds__(64) void rpa_combine_balanced_kernel(const DecodeArgs a_in) {
+// Threads of a merge launch over `rows` rows whose units are cut into `pieces` on average: more than a wave where there are many
+// partials and few rows (idle waves of large launches cost more than they save).
+int merge_threads(const DecodeArgs& a, int64_t rows, int64_t pieces) { return pieces > 8 && rows * a.Hq <= 2048 ? 64 * kMergeWaves : 64; }
+
+// Merge the partial rows of the balanced plan.  grid = (Hq * decode rows); block = merge_threads().
+__global__ __launch_bounds__(64 * kMergeWaves) void rpa_combine_balanced_kernel(const DecodeArgs a_in) {
   DecodeArgs a = a_in;  // static-shape mode: the number of decode rows comes from the device
   if (a.dist) a.num_rows = min(a.num_rows, scalar_load_i32(a.dist));
   const int seq = (int)(blockIdx.x / (unsigned)a.Hq);  // grid.x = Hq * rows, heads fastest
   const int head = (int)blockIdx.x - seq * a.Hq;
   if (seq >= a.num_rows) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   const int nw = a.waves_per_wg;
   const int row_groups = (a.G + 15) / 16;
   const int units = ((a.Hkv + nw - 1) / nw) * row_groups;
@@ -1569,17 +1608,17 @@ __global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int
 }
 
 // Merge the split partials: out = sum_j o_j 2^(m_j - m*) / sum_j l_j 2^(m_j - m*).
-// grid = (Hq * decode rows); block = one wave, 2 dims per lane (D = 128).  Lane j
+// grid = (Hq * decode rows); block = merge_threads(), 2 dims per lane (D = 128).  Lane j
 // first fetches (m_j, l_j) of split j, the wave reduces m* and the denominator
 // with shuffles, then the weights are broadcast lane by lane while the partial
 // rows stream in with independent loads.
 template <int HD>
-__global__ __launch_bounds__(64) void rpa_combine_kernel(const DecodeArgs a) {
+__global__ __launch_bounds__(64 * kMergeWaves) void rpa_combine_kernel(const DecodeArgs a) {
   const int index = (int)(blockIdx.x / (unsigned)a.Hq);  // grid.x = Hq * rows, heads fastest
   const int head = (int)blockIdx.x - index * a.Hq;
   RowRef row;
   if (!fixed_row(a, index, row)) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   const int t0 = first_block_token(row.kv_len, a.sm.window);
   const int n = min(a.max_splits, (row.kv_len - t0 + a.chunk - 1) / a.chunk);
   if (n <= 0) return;
@@ -1710,7 +1749,8 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
     hipError_t e = launch_decode_mt(a, dim3(a.num_wgs), dim3(a.waves_per_wg * 64), uniform, stream);
     if (e != hipSuccess) return e;
     if (!a.merge_counters)
-      hipLaunchKernelGGL(rpa_combine_balanced_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(64), 0, stream, a);
+      hipLaunchKernelGGL(rpa_combine_balanced_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows),
+                         dim3(merge_threads(a, a.num_rows, a.num_wgs / std::max<int64_t>(1, (int64_t)a.num_rows * head_groups * row_groups))), 0, stream, a);
     return hipGetLastError();
   }
   if (a.whole_rows)
@@ -1722,7 +1762,8 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
   hipError_t e = launch_decode_mt(a, grid, block, uniform, stream);
   if (e != hipSuccess) return e;
   if (a.max_splits > 1) {
-    hipLaunchKernelGGL(rpa_combine_kernel<128>, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(64), 0, stream, a);
+    hipLaunchKernelGGL(rpa_combine_kernel<128>, dim3((unsigned)a.Hq * (unsigned)a.num_rows),
+                       dim3(merge_threads(a, a.num_rows, a.max_splits)), 0, stream, a);
     e = hipGetLastError();
   }
   return e;
@@ -1787,7 +1828,8 @@ hipError_t launch_rows256(const DecodeArgs& a, int seq_begin, int seq_end, int m
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nsplit == 1) return e;
   if ((int64_t)a.Hq * a.num_rows > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(rpa_combine_kernel<256>, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(64), 0, stream, a);
+  hipLaunchKernelGGL(rpa_combine_kernel<256>, dim3((unsigned)a.Hq * (unsigned)a.num_rows),
+                     dim3(merge_threads(a, a.num_rows, a.max_splits)), 0, stream, a);
   return hipGetLastError();
 }
 

@@ -76,7 +76,8 @@ __device__ __forceinline__ int64_t row_offset(const TileSrc& s, const KvAddr& kv
 //   * the places of a sequence's pairs change with the tile.  A ragged sequence, which has
 //     workgroups for its own length only, then meets every shader engine, and with fewer than 8 kv heads other XCDs too (with
 //     8, 16, ... its kv heads stay on theirs).  Six chunks of 341 .. 1473 tokens x 16 / 8 heads of 256 dims, in the same places
-//     for every tile, had left 4 workgroups to each of 112 CUs and 1 to 48: 262.6 -> 203.5 us.  7 prompts of 264 .. 1643 tokens x 8 / 2 heads 46.6 -> 37.1, 4 prompts of 484 ..
+//     for every tile, had left 4 workgroups to each of 112 CUs and 1 to 48: 262.6 -> 203.5 us.  7 prompts of 264 .. 1643
+//     tokens x 8 / 2 heads 46.6 -> 37.1, 4 prompts of 484 ..
 //     2368 x 16 / 8 heads 119 -> 87; odd numbers of sequences and 4 heads per kv head are where they were.
 // The most expensive query tiles are issued first, so that the last workgroups to start are short ones.  A causal tile costs
 // what its last row sees: with a bound on kv_len from the host, tiles are ordered by level = tile index + ceil(prefix / tile

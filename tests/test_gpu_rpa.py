@@ -1718,3 +1718,25 @@ def test_packed_columns(pkg, wl, gpu, monkeypatch, case, pieces):
     if scale is None:
         other = gpu_out(pkg, b, gpu, **gkw)
         assert float(row_rel_error(got.float(), other.float()).max()) < (3e-2 if fp8 else 1e-2)
+
+
+@pytest.mark.parametrize("rows,kv,window,P,kv_dtype", [
+    (1, 30000, None, 64, torch.bfloat16), (3, 9001, None, 16, torch.bfloat16), (2, 17 * 64, None, 64, torch.bfloat16),
+    (1, 16 * 64, None, 64, torch.float8_e4m3fn), (70, 5000, 1024, 64, torch.bfloat16), (70, 1023, None, 16, torch.float8_e4m3fn)])
+def test_rows_of_one_length_and_rows_cut_over_the_chip(pkg, wl, gpu, rows, kv, window, P, kv_dtype):
+    """Merges of more than 16 partials by four waves (at 16 and 17 of them, past 256, fewer rows than waves of a merge), and rows
+    of one length whose even pieces would leave most of a last round of the chip empty, on the balanced plan."""
+    say(f"merges {rows} x {kv} window={window} P={P} {kv_dtype}")
+    b = wl.make_batch("merges", [1] * rows, [kv] * rows, num_q_heads=16, num_kv_heads=8 if rows == 70 else 2, head_dim=128, page_size=P,
+                      seed=77, kv_dtype=kv_dtype, sliding_window=window)
+    wl.plant_needles(b, seed=6)
+    tol = BF16_TOL if kv_dtype == torch.bfloat16 else FP8_TOL
+    want = oracle_out(b)
+    g = b.to(gpu)
+    for ns in (0, 300 if rows == 1 else 20):  # the caller's 300 pieces: two groups of references
+        out, _ = pkg.ragged_paged_attention(
+            g.q, None, None, g.kv_cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, b.distribution.numpy(), sm_scale=b.sm_scale,
+            sliding_window=window, k_scale=g.k_scale, v_scale=g.v_scale, max_kv_len=kv, max_q_len=1,
+            host_kv_lens=np.full(rows, kv, dtype=np.int32), **({"num_splits": ns} if ns else {}))
+        torch.cuda.synchronize()
+        assert_parity(out.cpu().float(), want.float(), **tol)
