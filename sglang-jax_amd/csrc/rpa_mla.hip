@@ -291,6 +291,9 @@ __device__ __forceinline__ int owner_of_token(const int32_t* cu_q_lens, int num_
   return lo;
 }
 
+// Query tokens are taken last first: a chunk's last tokens see the most, and what starts last should be short.  1405 tokens x
+// 64 heads e4m3 124 -> 101 us, 6 prompts of 88 .. 307 tokens x 128 heads 137 -> 127, 900 tokens x 128 heads 164 -> 158.
+//
 // What a grid row attends to.  Sequence rows (decode batches): the one query of sequence `row`
 // sees all kv_len tokens.  Token rows: query token `row` of a sequence with q_len new tokens
 // sits at position kv_len - q_len + j and sees the tokens up to itself -- an absorbed-MLA
@@ -781,8 +784,9 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_decode_kernel(const MlaDecodeA
   __shared__ __attribute__((aligned(1024))) char slot2[kSlotB];
   __shared__ __attribute__((aligned(1024))) char slot3[kSlotB];
   const int nsp = max(a.max_splits, 1);  // grid.x = max_splits * rows, splits fastest
-  const int row_id = (int)(blockIdx.x / (unsigned)nsp);
+  int row_id = (int)(blockIdx.x / (unsigned)nsp);
   const int split = (int)blockIdx.x - row_id * nsp;
+  if (a.rows_are_tokens) row_id = a.num_rows - 1 - row_id;
   const MlaRow mr = mla_row(a, row_id);
   if (!mr.valid) return;
   const int kv_len = mr.kv_len;
@@ -1142,7 +1146,7 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_token_group_kernel(const MlaDe
   const int num_seqs = a.dist ? min(a.num_seqs, scalar_load_i32(a.dist + 2)) : a.num_seqs;
   const int total = min(a.num_rows, scalar_load_i32(a.pt.cu_q_lens + num_seqs));
   const int per = 128 / a.Hq;
-  int t = (int)blockIdx.x * per;
+  int t = (int)(gridDim.x - 1 - blockIdx.x) * per;
   if (t >= total) return;
   const int t_stop = min(t + per, total);
   int seq = owner_of_token(a.pt.cu_q_lens, num_seqs, t);
@@ -1185,7 +1189,7 @@ __global__ __launch_bounds__(256, 1) void rpa_mla_token_group_wide_kernel(const 
   const int num_seqs = a.dist ? min(a.num_seqs, scalar_load_i32(a.dist + 2)) : a.num_seqs;
   const int total = min(a.num_rows, scalar_load_i32(a.pt.cu_q_lens + num_seqs));
   const int per = 128 / a.Hq;
-  int t = (int)blockIdx.x * per;
+  int t = (int)(gridDim.x - 1 - blockIdx.x) * per;
   if (t >= total) return;
   const int t_stop = min(t + per, total);
   int seq = owner_of_token(a.pt.cu_q_lens, num_seqs, t);
@@ -1220,8 +1224,9 @@ template <bool M32, bool P16 = false>
 __global__ __launch_bounds__(256, 1) void rpa_mla_decode_wide_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char ring[4 * kSlotB];
   const int nsp = max(a.max_splits, 1);  // grid.x = max_splits * rows, splits fastest
-  const int row_id = (int)(blockIdx.x / (unsigned)nsp);
+  int row_id = (int)(blockIdx.x / (unsigned)nsp);
   const int split = (int)blockIdx.x - row_id * nsp;
+  if (a.rows_are_tokens) row_id = a.num_rows - 1 - row_id;
   const MlaRow mr = mla_row(a, row_id);
   if (!mr.valid) return;
   const int kv_len = mr.kv_len;
