@@ -148,7 +148,8 @@ struct PrefillArgs {
   uint32_t page_options;
   int32_t packed;  // rpa_prefill_packed_kernel takes the call, K/V ranges in so many pieces where there is room for them; 0 = not
   struct {
-    FastDiv groups, units, hkv, nseq;
+    FastDiv groups, units, hkv, per_kv, nseq;
+    int32_t apart;
   } map;  // set by the launchers (prefill_grid)
 };
 

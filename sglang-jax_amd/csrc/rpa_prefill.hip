@@ -26,6 +26,8 @@
 // evenly over the 8 XCDs: hardware deals workgroup n to XCD n % 8.
 
 #include <cstdlib>
+#include <type_traits>
+#include <utility>
 
 #include "rpa_prefill_common.h"
 
@@ -35,6 +37,47 @@ using namespace pf;
 
 namespace {
 
+// f(0), f(1), ... f(N - 1), each with its number as a compile-time constant
+template <class F, int... I>
+__device__ __forceinline__ void unroll_seq(F f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void unroll_n(F f) {
+  unroll_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// A 64-token tile of 128-wide heads: its 32 operand fragments in the order of their use -- K of the scores (f < 16: k-step f >> 1,
+// half f & 1), V^T of the second product (half, k-step, dim tile) -- AHEAD of them requested ahead of the matrix instruction
+// that takes them, across the softmax in between.  Left to itself the compiler requests a fragment or two and waits for it.
+// With the copies' scalar bases (RowFeed), 16-token pages, 32 / 8 heads: 4 chunks of 2048 on 2048 .. 4096 659 -> 553 us, 3639 tokens
+// x 64 heads on 5000 929 -> 755, 8 chunks of 64-wide heads 118 -> 94; soft cap, 64-token pages 750 -> 727; e4m3 677 -> 660.
+// `request(f, frag)` reads fragment f.  AHEAD = 1: no order of ours (kernels whose options leave no registers for it).
+template <int AHEAD, class Request>
+__device__ __forceinline__ void tile_scores(f32x16_t (&S)[2], u32x4_t (&frag)[AHEAD], const u32x4_t (&qB)[kSteps], Request request) {
+  if constexpr (AHEAD > 1) unroll_n<AHEAD>([&](auto i) __attribute__((always_inline)) { request(i, frag[decltype(i)::value % AHEAD]); });
+  unroll_n<16>([&](auto i) __attribute__((always_inline)) {
+    constexpr int f = decltype(i)::value;
+    if constexpr (AHEAD == 1) request(i, frag[0]);
+    S[f & 1] = mfma32(frag[f % AHEAD], qB[f >> 1], f < 2 ? kZero16 : S[f & 1]);
+    if constexpr (AHEAD > 1) {
+      request(std::integral_constant<int, f + AHEAD>{}, frag[(f + AHEAD) % AHEAD]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  });
+}
+template <int AHEAD, class Request>
+__device__ __forceinline__ void tile_product(f32x16_t (&O)[kDimTiles], u32x4_t (&frag)[AHEAD], const u32x4_t (&pB)[2][2], Request request) {
+  unroll_n<16>([&](auto i) __attribute__((always_inline)) {
+    constexpr int g = decltype(i)::value, f = 16 + g;
+    if constexpr (AHEAD == 1) request(std::integral_constant<int, f>{}, frag[0]);
+    O[g & 3] = mfma32(frag[f % AHEAD], pB[g >> 3][(g >> 2) & 1], O[g & 3]);
+    if constexpr (AHEAD > 1) {
+      if constexpr (f + AHEAD < 32) request(std::integral_constant<int, f + AHEAD>{}, frag[(f + AHEAD) % AHEAD]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  });
+}
 
 // EXT compiles in the rarely used options (temperature factor, custom mask / no mask); the
 // plain causal instantiation keeps its scale in a scalar register and its mask test to one compare.
@@ -149,11 +192,29 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
   }
 
   // ---- pipeline: page ids two tiles ahead, the asynchronous copy one tile ahead ----
-  const AsyncOffsets ofs = make_async_offsets(a.kv, wave, lane);
-  AsyncPages<UNIFORM> pg;
-  async_fetch_pages<UNIFORM>(pg, src, t_lo, wave, lane);
-  async_copy_tile<UNIFORM>(lds_k0, lds_v0, src, a.kv, kh, vh, t_lo, wave, lane, pg, ofs);
-  async_fetch_pages<UNIFORM>(pg, src, t_lo + kBN, wave, lane);
+  RowFeed<16, kCopies> feed;  // UNIFORM: a wave copies 16 rows of a tile
+  AsyncPages<false> pg;
+  auto feed_row = [&](int n) { return n * kRowsPerCopy + lane / kChunks; };
+  auto fetch_pages = [&](int tb) __attribute__((always_inline)) {
+    if constexpr (UNIFORM) feed.fetch_page(src, tb, wave);
+    else async_fetch_pages<false>(pg, src, tb, wave, lane);
+  };
+  auto copy_tile = [&](char* to_k, char* to_v, int tb) __attribute__((always_inline)) {
+    if constexpr (UNIFORM) {
+      typedef __attribute__((address_space(3))) char* at_t;
+      const int64_t base = feed.base(src, a.kv);
+      feed.template copy<false>((uint32_t)(uintptr_t)(at_t)to_k + wave * (kCopies * 1024), kh + base, src, a.kv, feed_row);
+      feed.template copy<true>((uint32_t)(uintptr_t)(at_t)to_v + wave * (kCopies * 1024), vh + base, src, a.kv, feed_row);
+    } else {
+      async_copy_tile(to_k, to_v, src, a.kv, kh, vh, tb, wave, lane, pg);
+    }
+  };
+  if constexpr (UNIFORM)
+    feed.init(a.kv, feed_row, [&](int n) { return (lane % kChunks) ^ (feed_row(n) & 15); },
+              [&](int n) { return (lane % kChunks) ^ ((feed_row(n) & 3) << 2); });
+  fetch_pages(t_lo);
+  copy_tile(lds_k0, lds_v0, t_lo);
+  fetch_pages(t_lo + kBN);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the copies have landed in LDS
   __syncthreads();
 
@@ -165,8 +226,8 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
     }
     if (tb + kBN < t_hi) {
       // the other slot was last read before the barrier that ended the previous tile
-      async_copy_tile<UNIFORM>(nxt_k, nxt_v, src, a.kv, kh, vh, tb + kBN, wave, lane, pg, ofs);
-      async_fetch_pages<UNIFORM>(pg, src, tb + 2 * kBN, wave, lane);
+      copy_tile(nxt_k, nxt_v, tb + kBN);
+      fetch_pages(tb + 2 * kBN);
     }
     // visible to this wave?  causal: some token <= last row's position; window: some token
     // newer than the first row's horizon
@@ -175,31 +236,22 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
     if (vis) {
       const bool need_mask = (causal ? (tb + kBN - 1 > w.prefix + wr.r_lo) : (mc.mode == 1 || tb + kBN > w.kv_len)) ||
                              (W_ > 0 && tb <= w.prefix + wr.r_hi - W_);
-      {
-        // the two 32-token halves form two independent accumulator chains, issued alternately
-        f32x16_t S[2];
-        S[0] = mfma32(lds_ld16(lds_k + koff[0]), qB[0], kZero16);  // zero accumulator as an inline constant
-        S[1] = mfma32(lds_ld16(lds_k + koff[0] + 32 * kRowB), qB[0], kZero16);
-#pragma unroll
-        for (int ks = 1; ks < kSteps; ++ks) {
-          S[0] = mfma32(lds_ld16(lds_k + koff[ks]), qB[ks], S[0]);
-          S[1] = mfma32(lds_ld16(lds_k + koff[ks] + 32 * kRowB), qB[ks], S[1]);
+      auto request = [&](auto tag, u32x4_t& to) __attribute__((always_inline)) {
+        constexpr int f = decltype(tag)::value;
+        if constexpr (f < 16) {
+          to = lds_ld16(lds_k + koff[f >> 1] + (f & 1) * (32 * kRowB));
+        } else {
+          const char* vt = lds_v + voff[f & 3] + (((f >> 3) & 1) * 32 + ((f >> 2) & 1) * 16) * kRowB;
+          const u32x2_t lo = lds_tr16(vt), hi = lds_tr16(vt + 8 * kRowB);
+          to = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
         }
-        u32x4_t pB[2][2];
-        softmax_tile<CAP, EXT>(S, O, m, l, sm, need_mask, tb, h, wr.qpos, W_, pB, mc, mask_word);
-        // independent accumulator chains (dim tiles), issued round-robin
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-          for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-            for (int d = 0; d < kDimTiles; ++d) {
-              const char* vt = lds_v + voff[d] + (mt * 32 + kk * 16) * kRowB;
-              const u32x2_t lo = lds_tr16(vt);
-              const u32x2_t hi = lds_tr16(vt + 8 * kRowB);
-              O[d] = mfma32(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pB[mt][kk], O[d]);
-            }
-      }
+      };
+      f32x16_t S[2];
+      u32x4_t frag[EXT ? 2 : UNIFORM ? 6 : 4];
+      tile_scores(S, frag, qB, request);
+      u32x4_t pB[2][2];
+      softmax_tile<CAP, EXT>(S, O, m, l, sm, need_mask, tb, h, wr.qpos, W_, pB, mc, mask_word);
+      tile_product(O, frag, pB, request);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the next tile has landed
     __syncthreads();
@@ -227,8 +279,8 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
 // through its phases together.
 // (Eight waves as pairs that share 32 positions, one set of scores each, and exchange their probabilities through LDS --
 // half the reads -- spilled 50 registers at 256: 423 us.)
-// Measured: 6 chunks of 300 .. 1500 tokens x 16 heads, e4m3, soft cap, window 1024 (89 GFLOP) 424 -> 262 us; 3 bf16 prompts of
-// 1490 .. 2883 tokens x 16 heads on 16-token pages 198 -> 152 us with the cache write.
+// Measured: 6 chunks of 300 .. 1500 tokens x 16 heads, e4m3, soft cap, window 1024 (89 GFLOP) 424 -> 191 us; 3 bf16 prompts of
+// 1490 .. 2883 tokens x 16 heads on 16-token pages 198 -> 137 us with the cache write.
 namespace {
 
 constexpr int kWRowB = 512;                // a K or V row in LDS
@@ -258,16 +310,24 @@ __device__ __forceinline__ int wide_v_swizzle(int t) { return ((t & 3) << 2) | (
 template <bool UNIFORM, bool FP8>
 struct WideFeed {
   static constexpr int N = FP8 ? 2 : 4;  // copy instructions per wave, for K and for V
-  int32_t id[UNIFORM ? 1 : N];           // pages of this lane's rows in the tile copied next
+  RowFeed<8, N> rows;                    // UNIFORM: a wave copies 8 rows of a tile
+  int32_t id[N];                         // else: pages of this lane's rows in the tile copied next
 
   __device__ __forceinline__ static int row(int n, int wave, int lane) {
     return FP8 ? wave * 8 + n * 4 + (lane >> 4) : wave * 8 + n * 2 + (lane >> 5);
   }
+  __device__ __forceinline__ static int own_row(int n, int lane) { return FP8 ? n * 4 + (lane >> 4) : n * 2 + (lane >> 5); }
+  __device__ __forceinline__ void init(const KvAddr& kv, int wave, int lane) {
+    if constexpr (UNIFORM)
+      rows.init(kv, [&](int n) { return own_row(n, lane); },
+                [&](int n) { return FP8 ? (lane & 15) : (lane & 31) ^ (row(n, wave, lane) & 15); },
+                [&](int n) { return FP8 ? (lane & 15) : (lane & 31) ^ wide_v_swizzle(row(n, wave, lane)); });
+  }
   __device__ __forceinline__ void fetch_pages(const TileSrc& s, int tb, int wave, int lane) {
-    tb = min(tb, s.last_tok & ~(kBN - 1));
     if constexpr (UNIFORM) {
-      id[0] = scalar_load_i32(s.pages + __builtin_amdgcn_readfirstlane(page_slot(s, tb)));
+      rows.fetch_page(s, tb, wave);
     } else {
+      tb = min(tb, s.last_tok & ~(kBN - 1));
 #pragma unroll
       for (int n = 0; n < N; ++n) id[n] = s.pages[page_slot(s, min(tb + row(n, wave, lane), s.last_tok))];
     }
@@ -275,11 +335,18 @@ struct WideFeed {
   // K (or V) rows to `at` (FP8: the bytes to the staging area at `at`)
   __device__ __forceinline__ void copy(bool is_v, uint32_t at, const TileSrc& s, const KvAddr& kv, const char* base, int tb, int wave,
                                        int lane) {
+    if constexpr (UNIFORM) {
+      const char* b = base + rows.base(s, kv);
+      auto own = [&](int n) { return own_row(n, lane); };
+      if (is_v) rows.template copy<true>(at + wave * (N * 1024), b, s, kv, own);
+      else rows.template copy<false>(at + wave * (N * 1024), b, s, kv, own);
+      return;
+    }
     tb = min(tb, s.last_tok & ~(kBN - 1));  // past the end: re-copy the last tile
 #pragma unroll
     for (int n = 0; n < N; ++n) {
       const int t = row(n, wave, lane);
-      const int64_t ro = row_offset<UNIFORM>(s, kv, tb, tb + t, id[UNIFORM ? 0 : n]);
+      const int64_t ro = row_offset<false>(s, kv, tb, tb + t, id[n]);
       const int j = FP8 ? (lane & 15) : (lane & 31) ^ (is_v ? wide_v_swizzle(t) : t & 15);
       async_copy16(base + ro + j * 16, ring_ptr(at + (wave * N + n) * 1024));
     }
@@ -461,11 +528,50 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_async_kernel_wide(const Pr
     }
   };
 
+  // ---- a step's 64 operand fragments in the order of their use -- K of the scores (f < 32), V^T of the two halves of the
+  // second product -- kAhead of them requested ahead of the matrix instruction that takes them, across the softmax in between.
+  // (Left to itself the compiler asks for two at a time and waits: 203.5 -> 191 us on the chunks above, 2 chunks of 1024 on 2048,
+  // bf16, 125.7 -> 113.1; 4, 8 or 10 ahead are the same.)
+  constexpr int kAhead = 6;
+  u32x4_t frag[kAhead];
+  auto request = [&](auto tag) __attribute__((always_inline)) {
+    constexpr int f = decltype(tag)::value;
+    if constexpr (f < 32) {
+      frag[f % kAhead] = ring_ld16(koff[(f >> 2) & 3] + (f >> 4) * 256 + (f & 3) * (16 * kWRowB));
+    } else if constexpr (f < 64) {
+      const uint32_t vt = voff[f & 7] + ((f & 15) >> 3) * 256 + ((f - 32) >> 4) * (32 * kWRowB);
+      const u32x2_t lo = ring_tr16(vt), hi = ring_tr16(vt + 16 * kWRowB);
+      frag[f % kAhead] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+    }
+  };
+  auto scores_of = [&](f32x4_t (&S)[4]) __attribute__((always_inline)) {
+    unroll_n<kAhead>([&](auto i) __attribute__((always_inline)) { request(i); });
+    unroll_n<32>([&](auto i) __attribute__((always_inline)) {
+      constexpr int f = decltype(i)::value;
+      S[f & 3] = mfma16(frag[f % kAhead], qB[f >> 2], f < 4 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : S[f & 3]);
+      request(std::integral_constant<int, f + kAhead>{});
+      __builtin_amdgcn_sched_barrier(0);
+    });
+#pragma unroll
+    for (int i = 0; i < 4; ++i) koff[i] ^= kWTileB;
+  };
+  auto product_half = [&](auto half) __attribute__((always_inline)) {
+    constexpr int kk = decltype(half)::value;
+    unroll_n<16>([&](auto i) __attribute__((always_inline)) {
+      constexpr int j = decltype(i)::value, f = 32 + 16 * kk + j;
+      O[j] = mfma16(frag[f % kAhead], pB[kk], O[j]);
+      request(std::integral_constant<int, f + kAhead>{});
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+
   // ---- K runs a tile ahead of V.  Step i: K of tile i + 2 and V of tile i + 1 are requested; scores of tile i + 1, whose
   // soft cap and exponentials run beside the two halves of the second product of tile i
   if (t_lo < t_hi) {
     const int n = __builtin_amdgcn_readfirstlane((t_hi - t_lo + kBN - 1) / kBN);
     WideFeed<UNIFORM, FP8> fk, fv;  // their page ids
+    fk.init(a.kv, wave, lane);
+    fv.init(a.kv, wave, lane);
     uint32_t k_fill = ring_at, v_fill = ring_at + 3 * kWTileB;
     fk.fetch_pages(src, t_lo, wave, lane);
     fv.fetch_pages(src, t_lo + kBN, wave, lane);
@@ -538,14 +644,14 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_async_kernel_wide(const Pr
         if (i == 0) __syncthreads();
         next(tb);
         f32x4_t S[4];
-        scores(S);
+        scores_of(S);
         cap_scores(S);
-        second_product(0);
+        product_half(std::integral_constant<int, 0>{});
         mask_scores(S, tb + kBN);
         const float alpha = raise_max(S);
         u32x4_t p_next[2];
         probabilities(S, p_next);
-        second_product(1);
+        product_half(std::integral_constant<int, 1>{});
         pB[0] = p_next[0];
         pB[1] = p_next[1];
 #pragma unroll
@@ -811,25 +917,17 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const Prefil
     if (vis) {
       const bool need_mask = (causal ? (tb + kBN - 1 > w.prefix + wr.r_lo) : (mc.mode == 1 || tb + kBN > w.kv_len)) ||
                              (W_ > 0 && tb <= w.prefix + wr.r_hi - W_);
+      auto request = [&](auto tag, u32x4_t& to) __attribute__((always_inline)) {
+        constexpr int f = decltype(tag)::value;
+        if constexpr (f < 16) to = lds_ld16(lds_k + ((f & 1) * 32 + c) * kKPitch + h * 16 + (f >> 1) * 32);
+        else to = lds_ld16(lds_v + ((f & 3) * 32 + c) * kVPitch + h * 16 + (((f >> 3) & 1) * 32 + ((f >> 2) & 1) * 16) * 2);
+      };
       f32x16_t S[2];
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        const char* kp = lds_k + (mt * 32 + c) * kKPitch + h * 16;
-        S[mt] = mfma32(lds_ld16(kp), qB[0], kZero16);
-#pragma unroll
-        for (int ks = 1; ks < 8; ++ks) S[mt] = mfma32(lds_ld16(kp + ks * 32), qB[ks], S[mt]);
-      }
+      u32x4_t frag[EXT || !FP8 ? 1 : CAP ? 2 : UNIFORM ? 6 : 4];
+      tile_scores(S, frag, qB, request);
       u32x4_t pB[2][2];
       softmax_tile<CAP, EXT>(S, O, m, l, sm, need_mask, tb, h, wr.qpos, W_, pB, mc, mask_word);
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const char* vp = lds_v + (d * 32 + c) * kVPitch + h * 16;
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-          for (int kk = 0; kk < 2; ++kk)
-            O[d] = mfma32(lds_ld16(vp + (mt * 32 + kk * 16) * 2), pB[mt][kk], O[d]);
-      }
+      tile_product(O, frag, pB, request);
     }
     __syncthreads();
   }
@@ -929,9 +1027,9 @@ int prefill_kv_splits(const PrefillArgs& a) {
 int prefill_unpacked_kv_splits(const PrefillArgs& a, double* us) {
   const int nseq = a.seq_end - a.seq_begin;
   if (takes_pipe_kernel(a)) return prefill_pipe_kv_splits(a, nseq, us);
-  // the compiled kernels: a tile takes about 1.1 us alone on its CU (2.2 us for 256-wide heads)
+  // the compiled kernels: a tile takes about 0.85 us alone on its CU (e4m3 1.05, 256-wide heads 2.0)
   const bool heads4 = compiled_short_chunk_tile(a);
-  return kv_pieces(a, nseq, heads4 ? 32 : kBM, heads4 ? 4 : 1, a.head_dim == 256 ? 2.2 : 1.1, us);
+  return kv_pieces(a, nseq, heads4 ? 32 : kBM, heads4 ? 4 : 1, a.head_dim == 256 ? 2.0 : a.fp8 ? 1.05 : 0.85, us);
 }
 
 size_t prefill_split_workspace_bytes(const PrefillArgs& a, int splits) {
@@ -963,7 +1061,9 @@ hipError_t launch_prefill(const PrefillArgs& call, hipStream_t stream) {
   if (by_level) tiles = levels;
   const int64_t grid = prefill_grid(a, nseq, tiles, heads4 ? 4 : 1);
   if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  const bool uniform = (a.pt.page_size % kBN) == 0;
+  // whether the rows that a wave brings in of a tile are one page's
+  const int wave_rows = a.head_dim == 256 ? 8 : (a.fp8 || tuning().prefill_staged == 1) ? kBN : 16;
+  const bool uniform = (a.pt.page_size % wave_rows) == 0;
   // soft cap and logit rounding share the general score path
   const bool cap = a.sm.soft_cap != 0.f || a.sm.round_logits != 0;
   const bool staged = a.fp8 || tuning().prefill_staged == 1;

@@ -108,13 +108,16 @@ __device__ __forceinline__ Work decompose(const PrefillArgs& a, int tiles, int n
   w.valid = false;
   const int units = nseq * a.Hkv;
   const int groups = a.G / heads;  // workgroups per (sequence, kv head, tile)
-  const int r = blockIdx.x >> 3, rg = by(r, a.map.groups), gi = (r - rg * groups) * heads;
+  const int span = a.map.apart ? 1 : groups, per_kv = a.map.apart ? groups : 1;  // workgroups of a kv head side by side; its places
+  const int r = blockIdx.x >> 3, rg = by(r, a.map.groups);
   const int pair = rg * 8 + (blockIdx.x & 7);
   const int tile_rev = by(pair, a.map.units);
   if (tile_rev >= tiles) return w;
-  const int place = pair - tile_rev * units;
+  const int place = pair - tile_rev * (units * per_kv);
   int si = by(place, a.map.hkv);
-  w.hk = place - si * a.Hkv;
+  const int in_seq = place - si * (a.Hkv * per_kv);
+  w.hk = by(in_seq, a.map.per_kv);
+  const int gi = ((r - rg * span) + (in_seq - w.hk * per_kv)) * heads;
   if ((nseq & 1) == 0) {  // (an odd number of them moves on by itself)
     si += nseq == 2 ? tile_rev >> 1 : tile_rev;
     si -= by(si, a.map.nseq) * nseq;
@@ -137,12 +140,18 @@ __device__ __forceinline__ Work decompose(const PrefillArgs& a, int tiles, int n
 }
 
 // Workgroups of a launch of `tiles` tiles, and the divisors of their order (see decompose).
+// With fewer than 8 units their heads go to XCDs of their own: what few pairs there are would leave XCDs without work (2 chunks of
+// 36 .. 171 tokens x 8 / 1 heads 42.8 -> 31.5 us).
 inline int64_t prefill_grid(PrefillArgs& a, int nseq, int tiles, int heads) {
-  a.map.groups = fast_div(a.G / heads);
-  a.map.units = fast_div(nseq * a.Hkv);
-  a.map.hkv = fast_div(a.Hkv);
+  const int groups = a.G / heads, units = nseq * a.Hkv;
+  a.map.apart = units < 8;
+  const int span = a.map.apart ? 1 : groups, per_kv = groups / span;
+  a.map.groups = fast_div(span);
+  a.map.units = fast_div(units * per_kv);
+  a.map.hkv = fast_div(a.Hkv * per_kv);
+  a.map.per_kv = fast_div(per_kv);
   a.map.nseq = fast_div(nseq);
-  return ((int64_t)nseq * a.Hkv * tiles + 7) / 8 * 8 * (a.G / heads);
+  return ((int64_t)units * per_kv * tiles + 7) / 8 * 8 * span;
 }
 
 // K (or V) rows of the workgroup's kv head, token 0 of its sequence's first page.
@@ -629,35 +638,63 @@ __device__ __forceinline__ AsyncOffsets make_async_offsets(const KvAddr& kv, int
   return o;
 }
 
-template <bool UNIFORM>
-__device__ __forceinline__ void async_copy_tile(char* lds_k, char* lds_v, const TileSrc& s, const KvAddr& kv,
-                                                const char* kh, const char* vh, int tb, int wave, int lane,
-                                                const AsyncPages<UNIFORM>& pg, const AsyncOffsets& ofs) {
+// Pages that hold whole groups of the ROWS consecutive rows that a wave copies of a tile (N copy instructions for K, N for V): one
+// page id per wave and tile, a scalar base, and per lane offsets that never change.  An address per lane and copy -- 64-bit
+// products, and ids through the vector memory pipe for pages under a tile -- was most of what a wave issued beside its matrix
+// instructions.  Issued as assembly: the caller waits for the copies (vmcnt) itself.
+template <int ROWS, int N>
+struct RowFeed {
+  uint32_t k[N], v[N];  // byte offset of this lane's chunk from the wave's first row
+  int first, id;        // of the tile asked for last: the first row that the wave copies, and its page
+
+  // `row(n)`: this lane's row of copy n, from the wave's first; chunk_k / chunk_v(n): the chunk that it moves
+  template <class Row, class ChunkK, class ChunkV>
+  __device__ __forceinline__ void init(const KvAddr& kv, Row row, ChunkK chunk_k, ChunkV chunk_v) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      k[n] = (uint32_t)(row(n) * kv.tok_stride + (chunk_k(n) << 4));
+      v[n] = (uint32_t)(row(n) * kv.tok_stride + (chunk_v(n) << 4));
+    }
+  }
+  // rows wave * ROWS .. of the tile at `tb`; past the end: the last rows again
+  __device__ __forceinline__ void fetch_page(const TileSrc& s, int tb, int wave) {
+    first = __builtin_amdgcn_readfirstlane(min(tb + wave * ROWS, s.last_tok & ~(ROWS - 1)));
+    id = scalar_load_i32(s.pages + __builtin_amdgcn_readfirstlane(page_slot(s, first)));
+  }
+  __device__ __forceinline__ int64_t base(const TileSrc& s, const KvAddr& kv) const {
+    return (int64_t)id * kv.page_stride + (int64_t)(first - page_slot(s, first) * s.page_size) * kv.tok_stride;
+  }
+  // `at`: LDS address of the wave's first KiB; `b`: the head's rows plus base()
+  template <bool IS_V, class Row>
+  __device__ __forceinline__ void copy(uint32_t at, const char* b, const TileSrc& s, const KvAddr& kv, Row row) const {
+    if (first + ROWS - 1 <= s.last_tok) {
+#pragma unroll
+      for (int n = 0; n < N; ++n)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     :: "s"(at + n * 1024), "v"(IS_V ? v[n] : k[n]), "s"(b) : "memory", "m0");
+    } else {  // the sequence's last rows: those past its end repeat the last one
+      const int last = s.last_tok - first;
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const uint32_t o = (IS_V ? v[n] : k[n]) - (uint32_t)(max(row(n) - last, 0) * kv.tok_stride);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(at + n * 1024), "v"(o), "s"(b) : "memory", "m0");
+      }
+    }
+  }
+};
+
+// Other page sizes: an address per lane and copy.
+__device__ __forceinline__ void async_copy_tile(char* lds_k, char* lds_v, const TileSrc& s, const KvAddr& kv, const char* kh,
+                                                const char* vh, int tb, int wave, int lane, const AsyncPages<false>& pg) {
   typedef const __attribute__((address_space(1))) void* gptr_t;
   typedef __attribute__((address_space(3))) void* lptr_t;
   tb = min(tb, s.last_tok & ~(kBN - 1));  // past the end: re-copy the last tile
-  if constexpr (UNIFORM) {
-    if (tb + kBN - 1 <= s.last_tok) {
-      const int64_t base = (int64_t)pg.id[0] * kv.page_stride +
-                           (int64_t)(tb - page_slot(s, tb) * s.page_size) * kv.tok_stride;  // scalar
-      const char* kb = kh + base;
-      const char* vb = vh + base;
-#pragma unroll
-      for (int n = 0; n < kCopies; ++n) {
-        const int blk = wave * kCopies + n;
-        __builtin_amdgcn_global_load_lds((gptr_t)(kb + ofs.k[n]), (lptr_t)(lds_k + blk * 1024), 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((gptr_t)(vb + ofs.v[n]), (lptr_t)(lds_v + blk * 1024), 16, 0, 0);
-      }
-      return;
-    }
-  }
-  // last, partial tile (rows clamped to the last valid token) or pages smaller than a tile
   const int cp = lane % kChunks;
 #pragma unroll
   for (int n = 0; n < kCopies; ++n) {
     const int blk = wave * kCopies + n;
     const int t = blk * kRowsPerCopy + lane / kChunks;
-    const int64_t ro = row_offset<UNIFORM>(s, kv, tb, tb + t, pg.id[UNIFORM ? 0 : n]);
+    const int64_t ro = row_offset<false>(s, kv, tb, tb + t, pg.id[n]);
     const int jk = cp ^ (t & 15);
     const int jv = cp ^ ((t & 3) << 2);
     __builtin_amdgcn_global_load_lds((gptr_t)(kh + ro + jk * 16), (lptr_t)(lds_k + blk * 1024), 16, 0, 0);

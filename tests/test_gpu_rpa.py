@@ -1740,3 +1740,28 @@ def test_rows_of_one_length_and_rows_cut_over_the_chip(pkg, wl, gpu, rows, kv, w
             host_kv_lens=np.full(rows, kv, dtype=np.int32), **({"num_splits": ns} if ns else {}))
         torch.cuda.synchronize()
         assert_parity(out.cpu().float(), want.float(), **tol)
+
+
+@pytest.mark.parametrize("P", [8, 16, 24, 48, 64])
+@pytest.mark.parametrize("D,fp8,cap", [(128, False, None), (128, False, 30.0), (256, False, None), (256, True, 30.0)])
+def test_prefill_rows_copied_by_page(pkg, wl, gpu, monkeypatch, P, D, fp8, cap):
+    """The compiled prefill kernels on pages that hold whole groups of a wave's rows (16 rows of 128 dims, 8 of 256: one page id per
+    wave and tile) and on pages that do not: lengths around those groups and around tiles, everything that no row owns NaN, and
+    every order of the workgroups (even and odd numbers of sequences, fewer units than XCDs)."""
+    for q_lens, kv_lens, Hq, Hkv in (([7, 130, 64, 1], [7, 137, 200, 129], 8, 4), ([33, 200], [47, 481], 4, 1), ([17, 129, 65], [63, 400, 65], 16, 8)):
+        say(f"rows by page P={P} D={D} fp8={fp8} cap={cap} q={q_lens}")
+        b = wl.make_batch("by_page", q_lens, kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=D, page_size=P, seed=61, soft_cap=cap,
+                          sliding_window=150 if P == 24 else None, kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+        b.distribution = torch.tensor([0, 0, len(q_lens)], dtype=torch.int32)
+        want = oracle_out(b)
+        table = b.padded_page_table()
+        used = torch.zeros(b.kv_cache.shape[:2], dtype=torch.bool)
+        for i, kv in enumerate(kv_lens):
+            t = torch.arange(kv)
+            used[table[i][t // P].long(), t % P] = True
+        b.kv_cache.view(torch.uint8 if fp8 else torch.int16)[~used] = 0x7F if fp8 else 0x7FC0
+        monkeypatch.setenv("RPA_PREFILL_PACKED", "0")
+        monkeypatch.setenv("RPA_PREFILL_PIPE", "0")
+        for splits in ("0", "2"):
+            monkeypatch.setenv("RPA_PREFILL_SPLITS", splits)
+            assert_parity(gpu_out(pkg, b, gpu).float(), want.float(), **(FP8_TOL if fp8 else BF16_TOL))
