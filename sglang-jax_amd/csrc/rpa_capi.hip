@@ -418,8 +418,19 @@ int check_hip(hipError_t e, const char* what) {
   return fail(RPA_EHIP, "%s: %s", what, hipGetErrorString(e));
 }
 
-// head_dim 256, decode rows: split like the fixed plan when there are too few rows to fill the GPU
-// (the row kernel keeps nothing in flight while it computes, so it wants every wave slot)
+size_t rows256_bytes(const RpaParams* p, const SplitPlan& sp) {
+  return (size_t)p->decode_end * sp.splits * p->num_q_heads * (p->head_dim + 2) * sizeof(float);
+}
+
+// head_dim 256, decode rows: split like the fixed plan when there are too few rows to fill the GPU.
+// Pieces of 256 tokens and more, for every wave slot at two waves per SIMD, except
+//   * 64 or 128 tokens while those are at most 512 pieces: such a batch is a chain of blocks and nothing else (one row of
+//     700 tokens x 8 heads 22.8 -> 13.4 us, 8 rows of 300..3000 x 2 heads 25.9 -> 18.6; 20000 tokens x 8 heads, 1250
+//     pieces of 128: 40.7 -> 51.7, the merge);
+//   * twice the slots where the rows alone take more than half of them and differ in length: a piece was longer than most
+//     rows there, and the long rows were waited for (180 rows of 500..3000 tokens x 8 heads 277 -> 238 us);
+// both only while their partial rows stay below 16 MiB (a few long rows among many short ones take a slot per piece of
+// the longest), far inside the array of rpa_attention_noalloc, so that no call needs more than it used to accept.
 SplitPlan rows256_plan(const RpaParams* p) {
   const int64_t bound = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages,
                                      p->cu_kv_lens != nullptr);
@@ -428,14 +439,22 @@ SplitPlan rows256_plan(const RpaParams* p) {
   const int64_t units = (int64_t)p->decode_end * per_row;
   int64_t work = p->sum_decode_kv_len > 0 ? p->sum_decode_kv_len * per_row : 0;
   if (p->sliding_window > 0) work = 0;
-  return plan_splits(bound, p->sliding_window, units, work, p->num_splits, 256, wave_capacity());
+  const int slots = wave_capacity();
+  const int64_t seen = p->sliding_window > 0 ? std::min<int64_t>(bound, (int64_t)p->sliding_window + 31) : bound;
+  const int64_t tokens = work > 0 ? std::min(work, units * seen) : units * seen;
+  const int min_chunk = tokens <= 64 * (slots / 4) ? 64 : tokens <= 128 * (slots / 4) ? 128 : 256;
+  const bool ragged = work > 0 && work < units * seen && units * 2 > slots;
+  if (min_chunk < 256 || ragged) {
+    const SplitPlan sp = plan_splits(bound, p->sliding_window, units, work, p->num_splits, min_chunk, ragged ? 2 * slots : slots);
+    if (rows256_bytes(p, sp) <= ((size_t)16 << 20)) return sp;
+  }
+  return plan_splits(bound, p->sliding_window, units, work, p->num_splits, 256, slots);
 }
 
 size_t rows256_workspace(const RpaParams* p) {
   if (p->decode_end <= 0) return 0;
   const SplitPlan sp = rows256_plan(p);
-  if (sp.splits <= 1) return 0;
-  return (size_t)p->decode_end * sp.splits * p->num_q_heads * (p->head_dim + 2) * sizeof(float);
+  return sp.splits <= 1 ? 0 : rows256_bytes(p, sp);
 }
 
 // head_dim 256: every query token of sequences [seq_begin, seq_end) is a row of the row kernel

@@ -100,7 +100,9 @@ __device__ __forceinline__ int page_slot_of(const SeqView& s, int tok) {
 // page-id load behind every block and drains the whole queue in front of each block's use.)
 // FRESH: the row's last tokens may come from the caller's new rows instead (SeqView.fresh_first).
 // HALF (bf16): heads of 64 dims in rows of 128 whose second half is zero: it is not read.
-template <bool FP8, bool UNIFORM_PAGE, bool WINDOW = false, bool FRESH = false, bool HALF = false>
+// PART: the K rows only, the V rows only, or both.
+enum BlockPart { kBoth, kOnlyK, kOnlyV };
+template <bool FP8, bool UNIFORM_PAGE, bool WINDOW = false, bool FRESH = false, bool HALF = false, BlockPart PART = kBoth>
 __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, int page, int c, int g,
                                            const int32_t* win = nullptr, int win_first = 0) {
   const KvAddr& kv = a.kv;
@@ -112,6 +114,7 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
     else if constexpr (FP8) return RPA_KV_LD8(p);
     else return RPA_KV_LD16(p);
   };
+  static_assert(!FRESH || PART == kBoth);
   // A block that reaches into the new tokens (the last one of a row): an address of its own per token row.  The
   // number of loads is that of the other branch, so the counted waits behind it stay the same.
   if (FRESH && rare(tb + kBlk > s.fresh_first)) {
@@ -143,48 +146,56 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
     const char* kp = kh + (int64_t)page * kv.page_stride;
     const char* vp = vh + (int64_t)page * kv.page_stride;
     const int t0 = slot * s.page_size;
+    if constexpr (PART != kOnlyV) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int tin = min(tb + b * 16 + c, s.last_tok) - t0;
-      const uint32_t off = (uint32_t)(tin * kv.tok_stride + g * kLaneK);
-      if constexpr (FP8) {
-        r.k[b][0] = RPA_KV_LD16(kp + off);
-        r.k[b][1] = RPA_KV_LD16(kp + off + 16);
-      } else {
+      for (int b = 0; b < 2; ++b) {
+        const int tin = min(tb + b * 16 + c, s.last_tok) - t0;
+        const uint32_t off = (uint32_t)(tin * kv.tok_stride + g * kLaneK);
+        if constexpr (FP8) {
+          r.k[b][0] = RPA_KV_LD16(kp + off);
+          r.k[b][1] = RPA_KV_LD16(kp + off + 16);
+        } else {
 #pragma unroll
-        for (int st = 0; st < kSteps; ++st) r.k[b][st] = RPA_KV_LD16(kp + off + st * 64);
+          for (int st = 0; st < kSteps; ++st) r.k[b][st] = RPA_KV_LD16(kp + off + st * 64);
+        }
       }
     }
+    if constexpr (PART != kOnlyK) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int tin = min(tb + tok_slot(g, i), s.last_tok) - t0;
-      const uint32_t off = (uint32_t)(tin * kv.tok_stride + c * kLaneV);
-      r.v[i] = ld_v(vp + off);
+      for (int i = 0; i < 8; ++i) {
+        const int tin = min(tb + tok_slot(g, i), s.last_tok) - t0;
+        const uint32_t off = (uint32_t)(tin * kv.tok_stride + c * kLaneV);
+        r.v[i] = ld_v(vp + off);
+      }
     }
   } else {
+    if constexpr (PART != kOnlyV) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int tok = min(tb + b * 16 + c, s.last_tok);
-      const int slot = page_slot_of(s, tok);
-      const int page = WINDOW ? win[slot - win_first] : s.pages[slot];
-      const char* kp = kh + (int64_t)page * kv.page_stride +
-                       (int64_t)((tok - slot * s.page_size) * kv.tok_stride + g * kLaneK);
-      if constexpr (FP8) {
-        r.k[b][0] = RPA_KV_LD16(kp);
-        r.k[b][1] = RPA_KV_LD16(kp + 16);
-      } else {
+      for (int b = 0; b < 2; ++b) {
+        const int tok = min(tb + b * 16 + c, s.last_tok);
+        const int slot = page_slot_of(s, tok);
+        const int page = WINDOW ? win[slot - win_first] : s.pages[slot];
+        const char* kp = kh + (int64_t)page * kv.page_stride +
+                         (int64_t)((tok - slot * s.page_size) * kv.tok_stride + g * kLaneK);
+        if constexpr (FP8) {
+          r.k[b][0] = RPA_KV_LD16(kp);
+          r.k[b][1] = RPA_KV_LD16(kp + 16);
+        } else {
 #pragma unroll
-        for (int st = 0; st < kSteps; ++st) r.k[b][st] = RPA_KV_LD16(kp + st * 64);
+          for (int st = 0; st < kSteps; ++st) r.k[b][st] = RPA_KV_LD16(kp + st * 64);
+        }
       }
     }
+    if constexpr (PART != kOnlyK) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int tok = min(tb + tok_slot(g, i), s.last_tok);
-      const int slot = page_slot_of(s, tok);
-      const int page = WINDOW ? win[slot - win_first] : s.pages[slot];
-      const char* vp = vh + (int64_t)page * kv.page_stride +
-                       (int64_t)((tok - slot * s.page_size) * kv.tok_stride + c * kLaneV);
-      r.v[i] = ld_v(vp);
+      for (int i = 0; i < 8; ++i) {
+        const int tok = min(tb + tok_slot(g, i), s.last_tok);
+        const int slot = page_slot_of(s, tok);
+        const int page = WINDOW ? win[slot - win_first] : s.pages[slot];
+        const char* vp = vh + (int64_t)page * kv.page_stride +
+                         (int64_t)((tok - slot * s.page_size) * kv.tok_stride + c * kLaneV);
+        r.v[i] = ld_v(vp);
+      }
     }
   }
 }
@@ -1425,14 +1436,13 @@ __global__ __launch_bounds__(64 * kMergeWaves) void rpa_combine_balanced_kernel(
 // decode row over the first kv_len - q_len + j + 1 tokens, so one kernel serves decode rows and
 // prefill chunks alike.  The two 128-dim halves of a head reuse the register layouts and the
 // loads of the 128-dim kernel (a half is 128 contiguous elements of the head's row); scores sum
-// over both halves, each half has its own accumulators.  No split over tokens, no prefetch
-// ahead of the block being consumed, and a chunk's tokens each stream the prefix again: this
-// path exists so that 256-dim heads work, it is not tuned.
+// over both halves, each half has its own accumulators.  A chunk's tokens each stream the prefix
+// again (chunks take the prefill kernel unless a switch sends them here).
 // grid = (token rows, Hkv, row groups of 16 query heads); block = one wave.
 // With the composition on the device (a.dist) seq_end is only a bound: dist_role 1 = the decode partition
 // [0, dist[0]), 2 = everything behind it [dist[0], dist[2]) (custom-mask calls: [0, dist[2])).
 template <bool FP8, bool UNIFORM_PAGE>
-__global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int seq_begin, int seq_end, int dist_role) {
+__global__ __launch_bounds__(64, FP8 ? 2 : 1) void rpa_rows256_kernel(const DecodeArgs a, int seq_begin, int seq_end, int dist_role) {
   if (a.dist && dist_role == 1) {
     seq_end = min(seq_end, scalar_load_i32(a.dist));
   } else if (a.dist && dist_role == 2) {
@@ -1446,8 +1456,11 @@ __global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int
   // decode rows may be cut into max_splits pieces of `chunk` tokens (one token per row then, and
   // row = sequence); partial rows go to the workspace in the fixed plan's layout
   const int nsplit = max(a.max_splits, 1);
-  const int split = blockIdx.x % nsplit;
-  const int tok_row = blockIdx.x / nsplit + a.pt.cu_q_lens[seq_begin];
+  // Pieces outermost, rows and heads turned against the workgroup's number: workgroups go to the XCDs by number, and with
+  // the pieces of a row next to one another an XCD got the same piece of every row, mostly an empty one where few rows
+  // are long (180 rows of 500..3000 e4m3 tokens x 8 heads, two pieces: 392 -> 277 us).
+  const int nrows = gridDim.x / nsplit, split = blockIdx.x / nrows;
+  const int tok_row = (blockIdx.x + split + hk) % nrows + a.pt.cu_q_lens[seq_begin];
   if (tok_row >= a.pt.cu_q_lens[seq_end]) return;
   const int seq = owner_of_token(a.pt.cu_q_lens, seq_end, tok_row);
   const int q0 = a.pt.cu_q_lens[seq];
@@ -1513,18 +1526,39 @@ __global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int
   __shared__ int32_t win_ids[UNIFORM_PAGE ? 1 : kWinSmallPages];
   const int32_t* win = nullptr;
   int win_first = 0;
-  for (int tb = tb_begin; tb < tb_end; tb += kBlk) {
-    int page = 0;
-    if constexpr (UNIFORM_PAGE) page = __builtin_amdgcn_readfirstlane(sv.pages[page_slot_of(sv, tb)]);
-    else if (!win || page_slot_of(sv, min(tb + kBlk - 1, sv.last_tok)) - win_first >= kWinSmallPages) {
+  // The registers of a block's K rows are free behind the first product, those of its V rows behind the second: the next
+  // block's rows are requested into them there, so that half a block is always on its way and no register is needed
+  // twice (two whole blocks do not fit beside the 64 accumulators at two waves per SIMD, which
+  // e4m3 keeps; bf16 needs one wave's registers).
+  // 32 rows of 8000..16000 tokens x 8 heads: bf16 642 -> 567 us, e4m3 on 16-token pages 431 -> 302 (e4m3 on 64-token pages
+  // was level at 300, bf16 on 16-token pages is 577 -> 589; 8 rows of 300..3000 there gain like the others); 100 rows, window 512, e4m3 46.2 -> 31; 8 rows of 300..3000 36.9 -> 26.
+  int page = 0, page_next = 0;
+  auto page_of = [&](int tb) __attribute__((always_inline)) { return scalar_load_i32(sv.pages + page_slot_of(sv, min(tb, sv.last_tok))); };
+  KvRegs<FP8> r0, r1;
+  auto request_k = [&](int tb) __attribute__((always_inline)) {
+    if constexpr (UNIFORM_PAGE) {
+      page = page_next;
+      page_next = page_of(tb + kBlk);
+    } else if (!win || page_slot_of(sv, min(tb + kBlk - 1, sv.last_tok)) - win_first >= kWinSmallPages) {
       win_first = __builtin_amdgcn_readfirstlane(page_slot_of(sv, tb));
       copy_page_window<kWinSmallPages>(sv.pages, page_slot_of(sv, sv.last_tok), win_ids, win_first, lane);
       wait_all_loads();
       win = win_ids;
     }
-    KvRegs<FP8> r0, r1;
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(r0, a, sv, kh, vh, tb, page, c, g, win, win_first);
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(r1, a, sv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, false, false, kOnlyK>(r0, a, sv, kh, vh, tb, page, c, g, win, win_first);
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, false, false, kOnlyK>(r1, a, sv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
+  };
+  auto request_v = [&](int tb) __attribute__((always_inline)) {
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, false, false, kOnlyV>(r0, a, sv, kh, vh, tb, page, c, g, win, win_first);
+    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, false, false, kOnlyV>(r1, a, sv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
+  };
+  if constexpr (UNIFORM_PAGE) page_next = page_of(tb_begin);
+  if (tb_begin < tb_end) {
+    request_k(tb_begin);
+    request_v(tb_begin);
+  }
+  for (int tb = tb_begin; tb < tb_end; tb += kBlk) {
+    const bool more = tb + kBlk < tb_end;
     f32x4_t s[2];
     {
       u32x4_t kA[2][4];
@@ -1541,6 +1575,7 @@ __global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int
 #pragma unroll
         for (int st = 0; st < 4; ++st) s[b] = mfma16(kA[b][st], qB[1][st], s[b]);
     }
+    if (more) request_k(tb + kBlk);
     float x[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = s[i >> 2][i & 3];
@@ -1567,15 +1602,22 @@ __global__ __launch_bounds__(64) void rpa_rows256_kernel(const DecodeArgs a, int
     m = m_new;
     const u32x4_t pB = u32x4_t{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
                                pack_bf16x2(p[6], p[7])};
+    if (!FP8 || __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {  // as in compute_block: a maximum seldom moves
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[hf][j] = acc[hf][j] * alpha;
+    }
     {
       u32x4_t vA[8];
       v_operands<FP8>(r0, vA);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[0][j] = mfma16(vA[j], pB, acc[0][j] * alpha);
+      for (int j = 0; j < 8; ++j) acc[0][j] = mfma16(vA[j], pB, acc[0][j]);
       v_operands<FP8>(r1, vA);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[1][j] = mfma16(vA[j], pB, acc[1][j] * alpha);
+      for (int j = 0; j < 8; ++j) acc[1][j] = mfma16(vA[j], pB, acc[1][j]);
     }
+    if (more) request_v(tb + kBlk);
   }
 
   // ---- epilogue: lane (c, g) holds q row c, dims 128 hf + 32g + 8r + j in acc[hf][j][r] ----

@@ -932,6 +932,19 @@ def test_head_dim_256_decode_and_prefill(pkg, wl, gpu, Hq, Hkv, P):
     assert_parity(got.float(), want.float(), **BF16_TOL)
 
 
+@pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("P,Hq,Hkv,kv_lens,window", [
+    (64, 16, 8, [700], None), (32, 2, 1, [1, 31, 32, 33, 64, 65, 2100], None),  # pieces of 64 and 128 tokens; ends of a block
+    (16, 4, 2, [5000, 40, 4097], None), (1, 2, 2, [300, 257], None),  # more page ids than the window in LDS holds
+    (64, 8, 4, [900] * 2 + [3] * 298, None),  # rows of unequal length on more than half of the wave slots
+    (64, 8, 4, [900, 20, 257], 200)])
+def test_head_dim_256_rows_requested_a_half_block_ahead(pkg, wl, gpu, kv_dtype, P, Hq, Hkv, kv_lens, window):
+    b = batch256(wl, "d256rows", [1] * len(kv_lens), kv_lens, 98, Hq=Hq, Hkv=Hkv, P=P, kv_dtype=kv_dtype, sliding_window=window)
+    say(f"case d256 rows P={P} rows={len(kv_lens)} window={window} {kv_dtype}")
+    got = gpu_out(pkg, b, gpu)
+    assert_parity(got.float(), oracle_out(b).float(), **(BF16_TOL if kv_dtype == torch.bfloat16 else FP8_TOL))
+
+
 @pytest.mark.parametrize("window,cap,kv_dtype", [(40, None, torch.bfloat16), (None, 20.0, torch.bfloat16),
                                                  (40, 20.0, torch.float8_e4m3fn), (None, None, torch.float8_e4m3fn)])
 def test_head_dim_256_options(pkg, wl, gpu, window, cap, kv_dtype):
