@@ -102,7 +102,7 @@ constexpr ShapeRule kShapeRules[] = {
   {"prefill_pipe", kStagePrefill, 16, 128, 0, 0, 0, 0, 0, kOptPlainOnly,
    kKernelPrefillPipe, 128, 1, 64, 4, 16, 1, 0, "assembly steady state: C2 295 -> 236 us"},
   {"prefill_256_fp8", kStagePrefill, 8, 256, 0, 0, 0, 0, 0, 0,
-   kKernelPrefillWide, 128, 1, 64, 8, 8, 1, 0, "e4m3 bytes staged in LDS and widened into the bf16 tiles; soft cap and window 424 -> 262 us"},
+   kKernelPrefillWide, 128, 1, 64, 8, 8, 1, 0, "e4m3 bytes staged in LDS and widened into the bf16 tiles; soft cap and window 262 -> 193 us with its operands requested ahead and its workgroups in another order"},
   {"prefill_256", kStagePrefill, 16, 256, 0, 0, 0, 0, 0, 0,
    kKernelPrefillWide, 128, 1, 64, 8, 8, 1, 0, "eight waves of 16 positions, one workgroup per CU: 3 prompts of up to 2883 tokens 198 -> 152 us"},
   {"prefill_fp8_short", kStagePrefill, 8, 128, 0, 0, 4, 64, 0, 0,
@@ -125,7 +125,7 @@ constexpr ShapeRule kShapeRules[] = {
   {"mla_shared_64", kStageMla, 0, 576, 33, 64, 0, 0, 0, kOptSoftCap,
    kKernelMlaShared, 1, 64, 32, 8, 8, 2, 8, "159 -> 147 us"},
   {"mla_compiled", kStageMla, 0, 576, 0, 0, 0, 0, 0, 0,
-   kKernelMlaCompiled, 1, 128, 32, 8, 8, 1, 5, "soft cap; more than 64 heads on pages under 32 tokens or in a count that is no multiple of 128"},
+   kKernelMlaCompiled, 1, 128, 32, 8, 8, 1, 5, "soft cap; more than 64 heads on pages under 32 tokens (bf16 pages of 16: the wide loop all the same) or in a count that is no multiple of 128"},
 };
 // clang-format on
 
