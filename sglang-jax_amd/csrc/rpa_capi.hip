@@ -284,11 +284,12 @@ SplitPlan decode_plan(const RpaParams* p) {
   // once, at two waves per CU for bf16 (a workgroup that finds its row ended still takes its turn at the dispatcher), or
   // where a row's partials outgrow the merge.  4 rows of 1000..4095 tokens x 8 heads 22.8 us at 64, 16.9 at 128, 14.6 at
   // 256; e4m3 8 rows of 500..2047 17.8 / 13.1 / 13.8; one row of 16000 x 1 head 21.3 -> 15.1.  From about 160 tokens on
-  // the pieces fill the chip and longer ones lose; bf16 on pages under a block, whose tokens cost more, gains by the merge only.
+  // the pieces fill the chip and longer ones lose; bf16 on pages that are
+  // no multiple of 16, whose tokens cost more, gains by the merge only.
   if (p->num_splits > 0 || sp.splits <= 1 || sp.chunk > 128) return sp;
   int64_t eff = std::max<int64_t>(bound, 1);
   if (p->sliding_window > 0) eff = std::min(eff, (int64_t)p->sliding_window + 31);
-  const bool fp8 = p->kv_dtype == RPA_KV_FP8_E4M3, small_pages = p->page_size % 32 != 0;
+  const bool fp8 = p->kv_dtype == RPA_KV_FP8_E4M3, small_pages = p->page_size % 16 != 0;
   const int64_t slots = decode_wave_capacity(p), most = fp8 || small_pages ? slots : slots / 2;
   auto splits = [&](int chunk) { return (eff + chunk - 1) / chunk; };
   auto crowded = [&](int chunk) {
@@ -359,7 +360,7 @@ bool use_balanced(const RpaParams* p, const SplitPlan& fixed) {
     // even pieces, unless most of a last round of them is empty: 67 rows behind a window of 4096 x 8 kv heads are 1072 pieces
     // on 1024 slots, two rounds for the work of one (e4m3 138.0 -> 93.1 us, bf16 261 -> 172; 140 rows of 1024 tokens 137 -> 104;
     // at 0.78 of the rounds the two plans are level).  Whole rows need no merge: 150 x 512 tokens e4m3 (167 MB) 41.6 against 43.3
-    // us, bf16 (333 MB) 76.0 against 67.1.  On pages under a block the balanced plan has a cache write in front, which it pays
+    // us, bf16 (333 MB) 76.0 against 67.1.  On pages that are no multiple of 16 the balanced plan has a cache write in front, which it pays
     // for many times over (pages of 16, tokens brought along: the 67 rows 311 -> 211 us, e4m3 243 -> 137; 140 x 1024 tokens
     // 160 -> 122, 36 x 4096 163 -> 119, 130 x 2048 x 4 heads 160 -> 111).  Without the room that the balanced plan needs the
     // rows stay on the fixed one, which needs less, or nothing.
@@ -1028,10 +1029,10 @@ static bool rows_take_new_tokens(const RpaParams* p) {
 }
 
 // Whether the decode kernels read their rows' new tokens from the caller's keys / values and write them into the cache
-// (not the 256-wide rows, nor the balanced plan on pages smaller than a block).
+// (not the 256-wide rows, nor the balanced plan on pages that are no multiple of 16 tokens).
 static bool decode_takes_new_tokens(const RpaParams* p_in) {
   if (p_in->head_dim != 128 || p_in->mask_mode == RPA_MASK_CUSTOM || !rows_take_new_tokens(p_in)) return false;
-  if (p_in->page_size % 32 == 0) return true;
+  if (p_in->page_size % 16 == 0) return true;
   const RpaParams p = planning_view(p_in);
   return !use_balanced(&p, decode_plan(&p));
 }

@@ -22,6 +22,7 @@
 
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include "rpa_common.h"
 #include "rpa_kernels.h"
@@ -45,6 +46,19 @@ namespace rpa {
 namespace {
 
 constexpr int kBlk = 32;
+constexpr int kCacheBits = RPA_DECODE_NT ? 2 : 0;  // of the buffer loads: nt
+
+// What a page holds of a 32-token block, by which the kernels find a block's rows.  kBlocks: whole blocks (a multiple of 32 tokens).
+// kHalves: whole halves (a multiple of 16).  Either way a block has one or two page ids, the same in every lane: they
+// come as scalars, a row's address is a scalar base and a 32-bit offset.  kLanes: anything else; every lane looks the page of each
+// of its ten rows up in LDS and multiplies it out in 64 bits, 0.7 us of arithmetic per block where one wave runs alone.  Pages of 16
+// tokens as kLanes and as kHalves: 64 rows of 1000..8000 tokens x 8 heads bf16 254 -> 214 us, e4m3 169 -> 137; 4 rows of
+// 1000..4095 25.3 -> 15.4; 5 rows of 64..512 in a bucket 10.2 -> 7.9.
+enum Pages { kLanes, kHalves, kBlocks };
+constexpr Pages pages_of(int page_size) { return page_size % 32 == 0 ? kBlocks : page_size % 16 == 0 ? kHalves : kLanes; }
+struct BlockPages {
+  int lo, hi;  // page ids of the block's first and second 16 tokens (kBlocks: lo is both)
+};
 constexpr int kRowWaves = 8;    // rpa_decode_row_kernel: waves of a workgroup
 constexpr int kRowPitch = 132;  // its partial rows in LDS: 128 floats and 16 bytes, so that neighbouring heads' banks differ
 
@@ -90,152 +104,195 @@ __device__ __forceinline__ int page_slot_of(const SeqView& s, int tok) {
   return s.page_shift >= 0 ? (tok >> s.page_shift) : (tok / s.page_size);
 }
 
-// Issue the global loads of one 32-token block.  Token indices are clamped to
-// the last valid token so that nothing past kv_len (and nothing past the
-// sequence's page list) is ever dereferenced; clamped rows are masked later.
-// WINDOW, win / win_first: for pages that do not hold whole blocks, the LDS window the caller keeps of this
-// row's page ids (entry 0 = page slot win_first); without it every lane fetches the ids of its tokens from
-// memory, a dependent round trip in front of the block's loads.
-// (A compile-time choice: with both lookups in the code the compiler's wait-count bookkeeping sees a possible
-// page-id load behind every block and drains the whole queue in front of each block's use.)
-// FRESH: the row's last tokens may come from the caller's new rows instead (SeqView.fresh_first).
+// Issue the global loads of one 32-token block, whatever it holds.  Token indices are clamped to the last valid token so that
+// nothing past kv_len (and nothing past the sequence's page list) is ever dereferenced; clamped rows are masked later.
+// kLanes, WINDOW, win / win_first: the LDS window the caller keeps of this row's page ids (entry 0 = page slot win_first);
+// without it every lane fetches the ids of its tokens from memory, a dependent round trip in front of the block's loads.
+// FRESH: the row's last tokens may come from the caller's new rows instead (SeqView.fresh_first).  Chosen by masks: a lane's
+// own branch around the choice costs a drained queue of loads behind it.
 // HALF (bf16): heads of 64 dims in rows of 128 whose second half is zero: it is not read.
 // PART: the K rows only, the V rows only, or both.
 enum BlockPart { kBoth, kOnlyK, kOnlyV };
-template <bool FP8, bool UNIFORM_PAGE, bool WINDOW = false, bool FRESH = false, bool HALF = false, BlockPart PART = kBoth>
-__device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, int page, int c, int g,
+template <bool FP8, Pages PG, bool WINDOW = false, bool FRESH = false, bool HALF = false, BlockPart PART = kBoth>
+__device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, BlockPages page, int c, int g,
                                            const int32_t* win = nullptr, int win_first = 0) {
   const KvAddr& kv = a.kv;
   constexpr int kLaneK = FP8 ? 32 : 16;  // byte offset step of lane group g inside a K row
   constexpr int kLaneV = FP8 ? 8 : 16;   // byte offset step of lane c inside a V row
-  constexpr int kSteps = HALF ? 2 : 4;   // k-steps of the first product
-  auto ld_v = [&](const char* p) __attribute__((always_inline)) {
-    if constexpr (HALF) return c < 8 ? RPA_KV_LD16(p) : u32x4_t{0u, 0u, 0u, 0u};
-    else if constexpr (FP8) return RPA_KV_LD8(p);
-    else return RPA_KV_LD16(p);
-  };
-  static_assert(!FRESH || PART == kBoth);
-  // A block that reaches into the new tokens (the last one of a row): an address of its own per token row.  The
-  // number of loads is that of the other branch, so the counted waits behind it stay the same.
-  if (FRESH && rare(tb + kBlk > s.fresh_first)) {
-    const int block_slot = UNIFORM_PAGE ? page_slot_of(s, tb) : 0;
-    auto row_of = [&](int tok, const char* cached, const char* fresh) __attribute__((always_inline)) -> const char* {
-      tok = min(tok, s.last_tok);
-      const int slot = UNIFORM_PAGE ? block_slot : page_slot_of(s, tok);
-      const int pg = UNIFORM_PAGE ? page : WINDOW ? win[slot - win_first] : s.pages[slot];
-      const char* old_at = cached + (int64_t)pg * kv.page_stride + (int64_t)((tok - slot * s.page_size) * kv.tok_stride);
+  // (HALF: the lanes of dims 64.. read those of dims 0.. once more; nothing that they compute is kept)
+  const int lane_v = (HALF ? c & 7 : c) * kLaneV;
+  int t0[2] = {0, 0};  // first token of each half's page
+  if constexpr (PG != kLanes) {
+    t0[0] = page_slot_of(s, tb) * s.page_size;
+    t0[1] = PG == kHalves ? page_slot_of(s, min(tb + 16, s.last_tok)) * s.page_size : t0[0];
+  }
+  auto row_of = [&](int tok, int half, const char* cached, const char* fresh) __attribute__((always_inline)) -> const char* {
+    tok = min(tok, s.last_tok);
+    const char* at;
+    if constexpr (PG != kLanes) {
+      at = cached + (int64_t)(PG == kHalves && half ? page.hi : page.lo) * kv.page_stride + (uint32_t)((tok - t0[half]) * kv.tok_stride);
+    } else {
+      const int slot = page_slot_of(s, tok);
+      const int pg = WINDOW ? win[slot - win_first] : s.pages[slot];
+      at = cached + (int64_t)pg * kv.page_stride + (int64_t)((tok - slot * s.page_size) * kv.tok_stride);
+    }
+    if constexpr (FRESH) {
       const char* new_at = fresh + (int64_t)(s.fresh_row + (tok - s.fresh_first) * a.Hkv) * (FP8 || HALF ? 128 : 256);
-      return tok >= s.fresh_first ? new_at : old_at;
-    };
+      at += (new_at - at) & -(int64_t)(tok >= s.fresh_first);
+    }
+    return at;
+  };
+  if constexpr (PART != kOnlyV) {
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const char* kp = row_of(tb + b * 16 + c, kh, a.new_k) + g * kLaneK;
+      const char* at = row_of(tb + b * 16 + c, b, kh, a.new_k) + g * kLaneK;
 #pragma unroll
-      for (int st = 0; st < (FP8 ? 2 : kSteps); ++st) r.k[b][st] = RPA_KV_LD16(kp + st * (FP8 ? 16 : 64));
+      for (int st = 0; st < (FP8 || HALF ? 2 : 4); ++st) r.k[b][st] = RPA_KV_LD16(at + st * (FP8 ? 16 : 64));
     }
+  }
+  if constexpr (PART != kOnlyK) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const char* vp = row_of(tb + tok_slot(g, i), vh, a.new_v) + c * kLaneV;
-      r.v[i] = ld_v(vp);
+      const char* at = row_of(tb + tok_slot(g, i), i >= 4, vh, a.new_v) + lane_v;
+      if constexpr (FP8) r.v[i] = RPA_KV_LD8(at);
+      else r.v[i] = RPA_KV_LD16(at);
     }
-    return;
   }
-  if constexpr (UNIFORM_PAGE) {
-    // the whole block lies in one page whose id the caller fetched a block ahead
-    const int slot = page_slot_of(s, tb);
-    const char* kp = kh + (int64_t)page * kv.page_stride;
-    const char* vp = vh + (int64_t)page * kv.page_stride;
-    const int t0 = slot * s.page_size;
-    if constexpr (PART != kOnlyV) {
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const int tin = min(tb + b * 16 + c, s.last_tok) - t0;
-        const uint32_t off = (uint32_t)(tin * kv.tok_stride + g * kLaneK);
-        if constexpr (FP8) {
-          r.k[b][0] = RPA_KV_LD16(kp + off);
-          r.k[b][1] = RPA_KV_LD16(kp + off + 16);
-        } else {
-#pragma unroll
-          for (int st = 0; st < kSteps; ++st) r.k[b][st] = RPA_KV_LD16(kp + off + st * 64);
-        }
-      }
-    }
-    if constexpr (PART != kOnlyK) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int tin = min(tb + tok_slot(g, i), s.last_tok) - t0;
-        const uint32_t off = (uint32_t)(tin * kv.tok_stride + c * kLaneV);
-        r.v[i] = ld_v(vp + off);
-      }
-    }
+}
+
+// The same of a block whose 32 tokens all lie in the cache.  Buffer loads: a half's first row as the base, one offset per lane
+// for all K rows and another for all V rows, what differs between the loads in a scalar: no vector instruction beside the
+// loads themselves.
+template <bool FP8, Pages PG, bool HALF>
+__device__ __forceinline__ void load_full_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, BlockPages page, int c, int g,
+                                                const int32_t* win = nullptr, int win_first = 0) {
+  if constexpr (PG == kLanes) {
+    load_block<FP8, PG, true, false, HALF>(r, a, s, kh, vh, tb, page, c, g, win, win_first);
   } else {
-    if constexpr (PART != kOnlyV) {
+    const KvAddr& kv = a.kv;
+    const int off_k = c * kv.tok_stride + g * (FP8 ? 32 : 16);
+    const int off_v = 4 * g * kv.tok_stride + (HALF ? c & 7 : c) * (FP8 ? 8 : 16);
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const int tok = min(tb + b * 16 + c, s.last_tok);
-        const int slot = page_slot_of(s, tok);
-        const int page = WINDOW ? win[slot - win_first] : s.pages[slot];
-        const char* kp = kh + (int64_t)page * kv.page_stride +
-                         (int64_t)((tok - slot * s.page_size) * kv.tok_stride + g * kLaneK);
-        if constexpr (FP8) {
-          r.k[b][0] = RPA_KV_LD16(kp);
-          r.k[b][1] = RPA_KV_LD16(kp + 16);
-        } else {
+    for (int h = 0; h < 2; ++h) {
+      // (a second half past the end of the row, which only a prefetch for nobody asks for, is the first one again)
+      const bool hi = PG == kHalves && h && tb + 16 <= s.last_tok;
+      const int tok = hi ? tb + 16 : tb;
+      const int64_t at = (int64_t)(hi ? page.hi : page.lo) * kv.page_stride + (int64_t)(tok - page_slot_of(s, tok) * s.page_size) * kv.tok_stride;
+      const int behind = PG == kBlocks ? h * 16 * kv.tok_stride : 0;
+      const auto k = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kh) + at, 0, 0x7fffffff, 0x00020000);
+      const auto v = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vh) + at, 0, 0x7fffffff, 0x00020000);
 #pragma unroll
-          for (int st = 0; st < kSteps; ++st) r.k[b][st] = RPA_KV_LD16(kp + st * 64);
-        }
-      }
-    }
-    if constexpr (PART != kOnlyK) {
+      for (int st = 0; st < (FP8 || HALF ? 2 : 4); ++st)
+        r.k[h][st] = __builtin_amdgcn_raw_buffer_load_b128(k, off_k + st * (FP8 ? 16 : 64), behind, kCacheBits);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int tok = min(tb + tok_slot(g, i), s.last_tok);
-        const int slot = page_slot_of(s, tok);
-        const int page = WINDOW ? win[slot - win_first] : s.pages[slot];
-        const char* vp = vh + (int64_t)page * kv.page_stride +
-                         (int64_t)((tok - slot * s.page_size) * kv.tok_stride + c * kLaneV);
-        r.v[i] = ld_v(vp);
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (FP8) r.v[h * 4 + i] = __builtin_amdgcn_raw_buffer_load_b64(v, off_v, i * kv.tok_stride + behind, kCacheBits);
+        else r.v[h * 4 + i] = __builtin_amdgcn_raw_buffer_load_b128(v, off_v, i * kv.tok_stride + behind, kCacheBits);
       }
     }
   }
 }
 
-// Leave a row's new token, its last one, in the cache: the registers of the block that ends the row hold it (token t of
-// the block), K dims of token 16b + c in lanes (c, g), V rows of slot i in lanes (., g).  kh / vh: this kv head's rows of
-// the page, tin: the token's place in it.
-template <bool FP8, bool HALF = false>
-__device__ __forceinline__ void store_new_token(const KvRegs<FP8>& r, const KvAddr& kv, const char* kh, const char* vh,
-                                                int page, int tin, int t, int c, int g) {
-  const int64_t at = (int64_t)page * kv.page_stride + (int64_t)(tin * kv.tok_stride);
-  char* kp = const_cast<char*>(kh) + at;
-  char* vp = const_cast<char*>(vh) + at;
-  // (branches on t, which is the same in every lane: selects between the registers would take their address)
-  constexpr int kN = FP8 || HALF ? 2 : 4, kStep = FP8 ? 16 : 64;
-  t = __builtin_amdgcn_readfirstlane(t);
-  if (c == (t & 15)) {
-    kp += g * (FP8 ? 32 : 16);
-    if (t < 16) {
+// Any block, out of the cache alone (a new token's slot is read for what stands there): rows past the row's last token are the
+// last token's again, by a bound on the lanes' offsets.
+template <bool FP8, Pages PG, bool HALF>
+__device__ __forceinline__ void load_cached_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, BlockPages page, int c, int g,
+                                                  const int32_t* win, int win_first) {
+  if constexpr (PG == kLanes) {
+    load_block<FP8, PG, true, false, HALF>(r, a, s, kh, vh, tb, page, c, g, win, win_first);
+  } else {
+    const KvAddr& kv = a.kv;
+    const int lane_k = g * (FP8 ? 32 : 16), lane_v = (HALF ? c & 7 : c) * (FP8 ? 8 : 16);
+    const int row_k = c * kv.tok_stride, row_v = 4 * g * kv.tok_stride;
 #pragma unroll
-      for (int st = 0; st < kN; ++st) st16(kp + st * kStep, r.k[0][st]);
-    } else {
+    for (int h = 0; h < 2; ++h) {
+      const bool hi = PG == kHalves && h && tb + 16 <= s.last_tok;
+      const int tok = hi ? tb + 16 : tb, first = PG == kBlocks ? h * 16 : 0;
+      const int64_t at = (int64_t)(hi ? page.hi : page.lo) * kv.page_stride + (int64_t)(tok - page_slot_of(s, tok) * s.page_size) * kv.tok_stride;
+      const int most = min(s.last_tok - tok, PG == kBlocks ? 31 : 15) * kv.tok_stride;  // offset of the last row that there is
+      const auto k = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kh) + at, 0, 0x7fffffff, 0x00020000);
+      const auto v = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vh) + at, 0, 0x7fffffff, 0x00020000);
+      const int off_k = min(row_k + first * kv.tok_stride, most) + lane_k;
 #pragma unroll
-      for (int st = 0; st < kN; ++st) st16(kp + st * kStep, r.k[1][st]);
-    }
-    if constexpr (HALF) {
-      st16(kp + 128, u32x4_t{0u, 0u, 0u, 0u});
-      st16(kp + 192, u32x4_t{0u, 0u, 0u, 0u});
-    }
-  }
-  if (g == ((t >> 2) & 3)) {
-    const int i = (t & 3) + (t < 16 ? 0 : 4);
+      for (int st = 0; st < (FP8 || HALF ? 2 : 4); ++st)
+        r.k[h][st] = __builtin_amdgcn_raw_buffer_load_b128(k, off_k + st * (FP8 ? 16 : 64), 0, kCacheBits);
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (i == k) {
-        if constexpr (FP8) *reinterpret_cast<u32x2_t*>(vp + c * 8) = r.v[k];
-        else st16(vp + c * 16, r.v[k]);
+      for (int i = 0; i < 4; ++i) {
+        const int off_v = min(row_v + (first + i) * kv.tok_stride, most) + lane_v;
+        if constexpr (FP8) r.v[h * 4 + i] = __builtin_amdgcn_raw_buffer_load_b64(v, off_v, 0, kCacheBits);
+        else r.v[h * 4 + i] = __builtin_amdgcn_raw_buffer_load_b128(v, off_v, 0, kCacheBits);
       }
+    }
   }
 }
+
+// A row's new token, its last one, in the registers of a block: asked for at the start of the piece that ends the row, put in the
+// place of what its cache slot held, and left in that slot.  (No lane's own branch in put(): see load_block.)
+template <bool FP8, bool HALF>
+struct NewTokenRegs {
+  static constexpr int kSteps = FP8 || HALF ? 2 : 4, kStep = FP8 ? 16 : 64, kSrc = FP8 || HALF ? 128 : 256;
+  u32x4_t k[kSteps];
+  std::conditional_t<FP8, u32x2_t, u32x4_t> v;
+  bool on = false;
+  __device__ __forceinline__ void load(const DecodeArgs& a, const SeqView& s, int c, int g) {
+    const int64_t row = (int64_t)(s.fresh_row + (s.last_tok - s.fresh_first) * a.Hkv) * kSrc;
+#pragma unroll
+    for (int st = 0; st < kSteps; ++st) k[st] = ld16(a.new_k + row + g * (FP8 ? 32 : 16) + st * kStep);
+    const char* vp = a.new_v + row + (HALF ? c & 7 : c) * (FP8 ? 8 : 16);
+    if constexpr (FP8) v = ld8(vp);
+    else v = ld16(vp);
+  }
+  __device__ __forceinline__ void put(KvRegs<FP8>& r, int t, int c, int g) const {
+    // token t of the block; the rows behind it were its slot's, too, and their values count 0 times something
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int st = 0; st < kSteps; ++st) r.k[b][st] = c + 16 * b >= t ? k[st] : r.k[b][st];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r.v[i] = tok_slot(g, i) >= t ? v : r.v[i];
+  }
+  // kh, vh: this kv head's rows of the cache; page: the id of the token's page, tin: its place there
+  __device__ __forceinline__ void store(const KvAddr& kv, const char* kh, const char* vh, int page, int tin, int c, int g) const {
+    const int64_t at = (int64_t)page * kv.page_stride + (int64_t)tin * kv.tok_stride;
+    char* kp = const_cast<char*>(kh) + at;
+    char* vp = const_cast<char*>(vh) + at;
+    const u32x4_t zero = {0u, 0u, 0u, 0u};
+    if (c == 0) {
+#pragma unroll
+      for (int st = 0; st < kSteps; ++st) st16(kp + g * (FP8 ? 32 : 16) + st * kStep, k[st]);
+      if constexpr (HALF) {
+        st16(kp + g * 16 + 128, zero);
+        st16(kp + g * 16 + 192, zero);
+      }
+    }
+    if (g == 0) {
+      if constexpr (FP8) *reinterpret_cast<u32x2_t*>(vp + c * 8) = v;
+      else st16(vp + c * 16, HALF && c >= 8 ? zero : v);
+    }
+  }
+};
+
+// A row's new token, its last one, on its way into the cache: the wave whose piece ends the row copies the K and V rows of its
+// kv head, 16 bytes per lane.  It is asked for in front of the piece's blocks and stored behind them.  (Nobody reads the slot
+// meanwhile: the blocks take new tokens from the caller's rows.  Taken out of the registers of the row's last block instead, it
+// was a dozen branches in the block loop, each lane its own way; see load_block.)
+template <bool FP8, bool HALF>
+struct NewToken {
+  static constexpr int kRow = FP8 ? 128 : 256, kSrc = HALF ? 128 : kRow;  // bytes of a row in the cache, in the caller's keys / values
+  u32x4_t data = {0u, 0u, 0u, 0u};
+  bool on = false;
+  __device__ __forceinline__ void load(const DecodeArgs& a, const SeqView& s, int lane) {
+    const int at = (lane & 15) * 16;
+    if (lane < 32 && at < kSrc)
+      data = ld16((lane < 16 ? a.new_k : a.new_v) + (int64_t)(s.fresh_row + (s.last_tok - s.fresh_first) * a.Hkv) * kSrc + at);
+  }
+  // kh, vh: this kv head's rows of the cache; page: the id of the token's page, tin: its place there
+  __device__ __forceinline__ void store(const KvAddr& kv, const char* kh, const char* vh, int page, int tin, int lane) const {
+    const int at = (lane & 15) * 16;
+    if (lane < 32 && at < kRow)
+      st16(const_cast<char*>(lane < 16 ? kh : vh) + (int64_t)page * kv.page_stride + (int64_t)(tin * kv.tok_stride) + at, data);
+  }
+};
 
 // The general path of a block's scores: soft cap (if any), temperature, the logit rounded (if asked), in log2 units.
 // The constants are folded once per row, cap tanh(s scale / cap) temp log2e = k2 - 2 k2 / (2^(s k1) + 1), and a choice
@@ -513,7 +570,7 @@ struct RowRef {
 };
 
 // One wave, one (row, kv head, group of 16 query heads), tokens [t_begin, t_end): unnormalised output rows, maxima, sums.
-template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool HALF, int WAVES>
+template <int MT, bool FP8, Pages PG, bool CAP, bool HALF, int WAVES>
 __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef& row, int hk, int rg, int t_lo,
                                                int t_begin, int t_end, f32x4_t (&acc)[MT][8], float (&m)[MT], float (&l)[MT],
                                                int lane) {
@@ -563,59 +620,83 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
     for (int j = 0; j < 8; ++j) acc[mt][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 
-  // ---- software pipeline: the loads of block i+1 are in flight while block i is consumed.
-  // The prefetch is unconditional (past the end it re-reads the last block) so that the
-  // number of outstanding loads is the same on every path and the waits stay partial; the
-  // page id of block i+2 is fetched while block i is consumed.
-  const int t_last = t_begin + (nblk - 1) * kBlk;
-  auto block_tok = [&](int b) { return min(t_begin + b * kBlk, t_last); };
-  auto page_of = [&](int tb) -> int {
-    if constexpr (UNIFORM_PAGE) return scalar_load_i32(sv.pages + __builtin_amdgcn_readfirstlane(page_slot_of(sv, tb)));
-    else return 0;
+  // ---- software pipeline: two blocks are in flight or in use.  The piece's last block goes first: it may end the row, or reach
+  // into its new tokens, and takes an address per lane and row; the blocks behind it are full ones of the cache, so the
+  // loop has one kind of loads, stands once in the code for it, and its waits stay counted: with a choice of loads in the
+  // loop the compiler closes it with a block that has a way past them and drains the queue in front of every use.  A piece of two
+  // blocks asks for those two and no more.  16 rows of 32 k tokens x 8 heads 316 -> 304 us (7.06 TB/s), 8 rows of 64..512 on
+  // pages of 64 8.4 -> 7.2.
+  const int full = nblk - 1;  // blocks but the last
+  const int t_last = t_begin + full * kBlk;
+  auto page_of = [&](int tb) -> BlockPages {
+    BlockPages p = {};
+    if constexpr (PG != kLanes) p.lo = scalar_load_i32(sv.pages + __builtin_amdgcn_readfirstlane(page_slot_of(sv, tb)));
+    if constexpr (PG == kHalves) p.hi = scalar_load_i32(sv.pages + __builtin_amdgcn_readfirstlane(page_slot_of(sv, min(tb + 16, sv.last_tok))));
+    return p;
   };
-  // Pages smaller than a block: the ids of the next kWinSmallPages pages wait in the wave's LDS window and
+  // Pages smaller than half a block: the ids of the next kWinSmallPages pages wait in the wave's LDS window and
   // every lane looks its token rows up there; fetched from memory per block they were a dependent round
   // trip in front of every block's loads, behind which the loads already in flight had to drain (page size
   // 16: 2.6 TB/s where pages of 64 stream 5.8).  The window moves on every kWinSmallPages pages, at the
   // price of one drained queue.
-  __shared__ int32_t seg_windows[UNIFORM_PAGE ? 1 : WAVES][UNIFORM_PAGE ? 1 : kWinSmallPages];  // [wave][entry]
+  __shared__ int32_t seg_windows[PG != kLanes ? 1 : WAVES][PG != kLanes ? 1 : kWinSmallPages];  // [wave][entry]
   const int32_t* win = nullptr;
   int win_first = 0;
   auto cover = [&](int tb) __attribute__((always_inline)) {  // make the window hold the pages of block tb
-    if constexpr (!UNIFORM_PAGE) {
-      const int last_slot = page_slot_of(sv, sv.last_tok);
-      if (!win || page_slot_of(sv, min(tb + kBlk - 1, sv.last_tok)) - win_first >= kWinSmallPages) {
+    if constexpr (PG == kLanes) {
+      const int lo = page_slot_of(sv, tb), hi = page_slot_of(sv, min(tb + kBlk - 1, sv.last_tok));
+      if (!win || lo < win_first || hi - win_first >= kWinSmallPages) {
         int32_t* mine = seg_windows[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
-        win_first = __builtin_amdgcn_readfirstlane(page_slot_of(sv, tb));
-        copy_page_window<kWinSmallPages>(sv.pages, last_slot, mine, win_first, lane);
+        // (from the piece's first page if the whole piece fits)
+        const int begin = page_slot_of(sv, t_begin);
+        win_first = __builtin_amdgcn_readfirstlane(page_slot_of(sv, t_end - 1) - begin < kWinSmallPages ? begin : lo);
+        copy_page_window<kWinSmallPages>(sv.pages, page_slot_of(sv, sv.last_tok), mine, win_first, lane);
         wait_all_loads();
         win = mine;
       }
     }
   };
-  auto leave_new_token = [&](const KvRegs<FP8>& r, int tb) __attribute__((always_inline)) {
-    if (rare(a.new_k && tb + kBlk > sv.last_tok)) {
-      const int slot = __builtin_amdgcn_readfirstlane(page_slot_of(sv, sv.last_tok));
-      store_new_token<FP8, HALF>(r, a.kv, kh, vh, scalar_load_i32(sv.pages + slot), sv.last_tok - slot * sv.page_size,
-                           sv.last_tok - tb, c, g);
-    }
-  };
+  NewToken<FP8, HALF> fresh;
+  fresh.on = a.new_k && t_end == kv_len;
+  if (fresh.on) fresh.load(a, sv, lane);
   KvRegs<FP8> ra, rb;
-  int pg_next = page_of(block_tok(1));
-  cover(t_begin);
-  load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true, HALF>(ra, a, sv, kh, vh, t_begin, page_of(t_begin), c, g, win, win_first);
-  for (int blk = 0; blk < nblk; blk += 2) {
-    cover(block_tok(blk + 1));
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true, HALF>(rb, a, sv, kh, vh, block_tok(blk + 1), pg_next, c, g, win, win_first);
-    pg_next = page_of(block_tok(blk + 2));
-    leave_new_token(ra, t_begin + blk * kBlk);
-    compute_block<MT, FP8, CAP, HALF>(ra, qB, acc, m, l, so, t_begin + blk * kBlk, g);
-    if (blk + 1 >= nblk) break;
-    cover(block_tok(blk + 2));
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, true, HALF>(ra, a, sv, kh, vh, block_tok(blk + 2), pg_next, c, g, win, win_first);
-    pg_next = page_of(block_tok(blk + 3));
-    leave_new_token(rb, t_begin + (blk + 1) * kBlk);
-    compute_block<MT, FP8, CAP, HALF>(rb, qB, acc, m, l, so, t_begin + (blk + 1) * kBlk, g);
+  // (a chunk's query tokens as rows: its new tokens may reach over several blocks, a few at most)
+  int first = 0;
+  if (a.token_rows) {
+    while (full - first > 0 && t_last - first * kBlk > sv.fresh_first) ++first;
+    for (int b = 1; b <= first; ++b) {
+      const int tb = t_last - b * kBlk;
+      cover(tb);
+      load_block<FP8, PG, PG == kLanes, true, HALF>(rb, a, sv, kh, vh, tb, page_of(tb), c, g, win, win_first);
+      compute_block<MT, FP8, CAP, HALF>(rb, qB, acc, m, l, so, tb, g);
+    }
+  }
+  const int n = full - first;  // full blocks of the cache
+  auto next_tok = [&](int b) { return t_begin + min(b, max(n - 1, 0)) * kBlk; };
+  BlockPages pg_next = page_of(next_tok(0));
+  cover(t_last);
+  load_block<FP8, PG, PG == kLanes, true, HALF>(ra, a, sv, kh, vh, t_last, page_of(t_last), c, g, win, win_first);
+  cover(next_tok(0));
+  load_full_block<FP8, PG, HALF>(rb, a, sv, kh, vh, next_tok(0), pg_next, c, g, win, win_first);
+  int in_a = t_last;  // first tokens of the blocks in ra, rb
+  int asked = 1;      // full blocks asked for; beyond n they are the last one again, for nobody
+  while (asked < n) {
+    pg_next = page_of(next_tok(asked));
+    compute_block<MT, FP8, CAP, HALF>(ra, qB, acc, m, l, so, in_a, g);
+    cover(next_tok(asked));
+    load_full_block<FP8, PG, HALF>(ra, a, sv, kh, vh, next_tok(asked), pg_next, c, g, win, win_first);
+    in_a = next_tok(asked);
+    pg_next = page_of(next_tok(asked + 1));
+    compute_block<MT, FP8, CAP, HALF>(rb, qB, acc, m, l, so, next_tok(asked - 1), g);
+    cover(next_tok(asked + 1));
+    load_full_block<FP8, PG, HALF>(rb, a, sv, kh, vh, next_tok(asked + 1), pg_next, c, g, win, win_first);
+    asked += 2;
+  }
+  compute_block<MT, FP8, CAP, HALF>(ra, qB, acc, m, l, so, in_a, g);
+  if (asked == n) compute_block<MT, FP8, CAP, HALF>(rb, qB, acc, m, l, so, next_tok(n - 1), g);
+  if (fresh.on) {
+    const int slot = __builtin_amdgcn_readfirstlane(page_slot_of(sv, sv.last_tok));
+    fresh.store(a.kv, kh, vh, scalar_load_i32(sv.pages + slot), sv.last_tok - slot * sv.page_size, lane);
   }
 }
 
@@ -652,7 +733,7 @@ __device__ __forceinline__ bool fixed_row(const DecodeArgs& a, int index, RowRef
 
 // ---- fixed split plan: grid = (max_splits * rows, 1, head groups * row groups), splits fastest (rows do
 // not sit on a grid dimension of their own: that one ends at 65535); block = NW waves
-template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool HALF = false>
+template <int MT, bool FP8, Pages PG, bool CAP, bool HALF = false>
 __global__ __launch_bounds__(256, 2) void rpa_decode_splitkv_kernel(const DecodeArgs a) {
   const int nsp = max(a.max_splits, 1);
   const int index = (int)(blockIdx.x / (unsigned)nsp);
@@ -679,7 +760,7 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_splitkv_kernel(const Decode
   dest.base = ((int64_t)index * a.max_splits + split) * a.Hq;
   f32x4_t acc[MT][8];
   float m[MT], l[MT];
-  decode_segment<MT, FP8, UNIFORM_PAGE, CAP, HALF, 4>(a, row, hk, rg, t_lo, t_begin, t_end, acc, m, l, lane);
+  decode_segment<MT, FP8, PG, CAP, HALF, 4>(a, row, hk, rg, t_lo, t_begin, t_end, acc, m, l, lane);
   write_rows<MT>(a, acc, m, l, row.tq, hk, rg * 16 * MT, dest, lane & 15, lane >> 4);
 }
 
@@ -688,7 +769,7 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_splitkv_kernel(const Decode
 // 4 us from its start to its first useful load; here the merge is two barriers and 8 KB of LDS per 2 query heads.  8 waves:
 // the registers allow two per SIMD, and a row of 255 tokens is then one 32-token block each.  A few rows of up to 255
 // tokens: 10.2 -> 7.5 us.
-template <bool FP8, bool UNIFORM_PAGE, bool CAP, bool HALF = false>
+template <bool FP8, Pages PG, bool CAP, bool HALF = false>
 __global__ __launch_bounds__(kRowWaves * 64, 2) void rpa_decode_row_kernel(const DecodeArgs a) {
   extern __shared__ float row_parts[];  // [wave][query head of the group][kRowPitch]
   __shared__ float row_ml[kRowWaves][16][2];
@@ -706,7 +787,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 2) void rpa_decode_row_kernel(const
   float m[1], l[1];
   if (wave < used) {
     const int t_begin = t0 + wave * piece;
-    decode_segment<1, FP8, UNIFORM_PAGE, CAP, HALF, kRowWaves>(a, row, hk, rg, t_lo, t_begin, min(row.kv_len, t_begin + piece),
+    decode_segment<1, FP8, PG, CAP, HALF, kRowWaves>(a, row, hk, rg, t_lo, t_begin, min(row.kv_len, t_begin + piece),
                                                                acc, m, l, lane);
     float lt = l[0];
     lt += __shfl_xor(lt, 16);
@@ -967,9 +1048,9 @@ __device__ __forceinline__ void merge_unit(const DecodeArgs& a, const PendingMer
 // are requested right behind that first block.  A piece border costs no round trip to memory,
 // and neither does a block: under load a small dependent load waits behind megabytes of queued
 // KV traffic (10 us and more), so there are none after the first block.
-// New tokens (a.new_k) are taken where pages hold whole blocks; with smaller pages there is no register left for it.
-template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool MERGE, bool HALF = false>
-__global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const DecodeArgs a_in) {
+// New tokens (a.new_k) are taken where pages hold whole blocks or halves.  (bf16: registers of one wave per SIMD, which is what is resident.)
+template <int MT, bool FP8, Pages PG, bool CAP, bool MERGE, bool HALF>
+__device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
   DecodeArgs a = a_in;  // static-shape mode: the number of decode rows comes from the device
   if (a.dist) a.num_rows = min(a.num_rows, scalar_load_i32(a.dist));
   if (a.num_rows <= 0) return;
@@ -1064,16 +1145,18 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
     sv.page_shift = page_shift;
     sv.last_tok = r.kv_len - 1;
     sv.pages = a.pt.page_indices + r.page0;
-    sv.fresh_first = (UNIFORM_PAGE && a.new_k) ? r.kv_len - 1 : kNoFresh;
+    sv.fresh_first = (PG != kLanes && a.new_k) ? r.kv_len - 1 : kNoFresh;
     sv.fresh_row = r.tq * a.Hkv + hk;
     return sv;
   };
   auto slot_of_tok = [&](int tok) { return page_shift >= 0 ? (tok >> page_shift) : (tok / page_size); };
-  auto page_in = [&](const PageWindow& pwn, int tok) -> int {
-    if constexpr (UNIFORM_PAGE) return uniform(pwn.lds[uniform(slot_of_tok(tok) - pwn.first)]);
-    else return 0;
+  // ids of the pages that hold block tb of a row
+  auto pages_in = [&](const PageWindow& pwn, const SeqView& v, int tb) -> BlockPages {
+    BlockPages p = {};
+    if constexpr (PG != kLanes) p.lo = uniform(pwn.lds[uniform(slot_of_tok(tb) - pwn.first)]);
+    if constexpr (PG == kHalves) p.hi = uniform(pwn.lds[uniform(slot_of_tok(min(tb + 16, v.last_tok)) - pwn.first)]);
+    return p;
   };
-
   Piece cur;
   {
     const int r = x - row_first;
@@ -1082,48 +1165,44 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
     cur = make_piece(row, unit, blk, min(row.nb - blk, x_end - x));
   }
   int cur_unit = (x - row_first) / row.nb;
-  constexpr int kWin = UNIFORM_PAGE ? 64 : kWinSmallPages;
+  constexpr int kWin = PG == kBlocks ? 64 : kWinSmallPages;
   __shared__ int32_t lds_windows[4][2][kWin];  // [wave][current / next piece][entry]
   PageWindow win = {lds_windows[wave][0], 0};
   PageWindow nwin = {lds_windows[wave][1], 0};
-  // what load_block takes besides the uniform page id: the window itself when pages are smaller than a block
-  auto lanes_win = [&](const PageWindow& pwn) -> const int32_t* { return UNIFORM_PAGE ? nullptr : pwn.lds; };
+  auto request = [&](KvRegs<FP8>& r, const SeqView& v, int of_head, const PageWindow& pwn, int tb) __attribute__((always_inline)) {
+    load_cached_block<FP8, PG, HALF>(r, a, v, a.kv.k_base + (int64_t)of_head * a.kv.head_stride, a.kv.v_base + (int64_t)of_head * a.kv.head_stride,
+                                     tb, pages_in(pwn, v, tb), c, g, pwn.lds, pwn.first);
+  };
   request_window<kWin>(a, cur.row, win, slot_of_tok(cur.t_first), page_shift, lane);
   u32x4_t qB[MT][4];
   load_queries<MT, FP8>(a, cur.row.tq, min(cur.hk, a.Hkv - 1), cur.rg * 16 * MT, c, g, qB);
   wait_all_loads();  // the window (and the queries behind it)
 
+  // ---- the piece at hand, and what is known of the one behind it: the next unit of the same row, or the first unit of the
+  // next row that has any block (has_next guarantees there is one)
   KvRegs<FP8> ra, rb;
-  bool in_b = false;  // which register set holds the block about to be consumed
-  {
-    const int hk = min(cur.hk, a.Hkv - 1);
-    const SeqView sv = view_of(cur.row, hk);
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE, HALF>(ra, a, sv, a.kv.k_base + (int64_t)hk * a.kv.head_stride,
-                                  a.kv.v_base + (int64_t)hk * a.kv.head_stride, cur.t_first,
-                                  page_in(win, cur.t_first), c, g, lanes_win(win), win.first);
-  }
-
-  PendingMerge pm_first = {}, pm_last = {};
-  for (;;) {
-    // ---- this piece
-    const int hk = min(cur.hk, a.Hkv - 1);
-    const SeqView sv = view_of(cur.row, hk);
-    const char* kh = a.kv.k_base + (int64_t)hk * a.kv.head_stride;
-    const char* vh = a.kv.v_base + (int64_t)hk * a.kv.head_stride;
+  int hk, i;  // its kv head, its next block
+  SeqView sv;
+  ScoreOpts so;
+  NewTokenRegs<FP8, HALF> fresh;
+  f32x4_t acc[MT][8];
+  float m[MT], l[MT];
+  bool has_next, next_row;
+  int nseq;
+  RowLoads nl;
+  Piece nxt;
+  auto begin_piece = [&]() __attribute__((always_inline)) {
+    hk = min(cur.hk, a.Hkv - 1);
+    sv = view_of(cur.row, hk);
     requantise_queries<MT, FP8>(a, qB);
-    ScoreOpts so;
-    {
-      const float ks = a.k_scale ? a.k_scale[hk] : 1.0f;
-      const float temp = xai_factor(cur.row.kv_len - 1, a.sm.xai_len);  // the one query sits at kv_len - 1
-      const float scale = a.sm.sm_scale * ks * (a.sm.q_scale > 0.f ? a.sm.q_scale : 1.0f);
-      so.scale2 = scale * kLog2e * temp;
-      so.general.set(a.sm, scale, temp);
-      so.mask2 = fmaxf(a.sm.mask_value * kLog2e, -3.0e38f);
-      so.t_lo = cur.t_lo;
-      so.kv_len = cur.row.kv_len;
-    }
-    f32x4_t acc[MT][8];
-    float m[MT], l[MT];
+    const float ks = a.k_scale ? a.k_scale[hk] : 1.0f;
+    const float temp = xai_factor(cur.row.kv_len - 1, a.sm.xai_len);  // the one query sits at kv_len - 1
+    const float scale = a.sm.sm_scale * ks * (a.sm.q_scale > 0.f ? a.sm.q_scale : 1.0f);
+    so.scale2 = scale * kLog2e * temp;
+    so.general.set(a.sm, scale, temp);
+    so.mask2 = fmaxf(a.sm.mask_value * kLog2e, -3.0e38f);
+    so.t_lo = cur.t_lo;
+    so.kv_len = cur.row.kv_len;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       m[mt] = -INFINITY;
@@ -1131,89 +1210,66 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[mt][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-
-    // ---- the piece after it: the next unit of the same row, or the first unit of the next row
-    // that has any block (has_next guarantees there is one)
-    const bool has_next = x + cur.nblk < x_end;
-    const bool next_row = has_next && (cur_unit == units - 1);
-    int nseq = cur.row.seq + 1;
-    RowLoads nl = {0, 0, 0};
+    has_next = x + cur.nblk < x_end;
+    next_row = has_next && (cur_unit == units - 1);
+    nseq = cur.row.seq + 1;
+    nl = RowLoads{0, 0, 0};
     if (next_row) nl = row_issue_scalar(a, nseq);
-    Piece nxt = cur;
-    SeqView nsv = sv;
-    const char* nkh = kh;
-    const char* nvh = vh;
+    nxt = cur;
+    fresh.on = PG != kLanes && a.new_k && cur.t_first + cur.nblk * kBlk > sv.last_tok;
+    if (fresh.on) fresh.load(a, sv, c, g);
+    i = 0;
+  };
+  PendingMerge pm_first = {}, pm_last = {};
+
+  // One block: the one behind it is requested, then it is worked on; a piece's rows are written behind its last one.
+  // false: nothing is left.
+  auto step = [&](KvRegs<FP8>& use, KvRegs<FP8>& fill) __attribute__((always_inline)) -> bool {
+    const int tb = cur.t_first + i * kBlk;
+    const bool last = (i + 1 == cur.nblk);
     // resolved one block into the piece when it has more than one block, at once otherwise
     const int resolve_at = (cur.nblk > 1) ? 1 : 0;
-
-    auto step = [&](int i, const KvRegs<FP8>& use, KvRegs<FP8>& fill) __attribute__((always_inline)) {
-      if (has_next && i == resolve_at) {
-        RowMeta nrow = cur.row;
-        int nunit = cur_unit + 1;
-        if (next_row) {
-          nrow = row_resolve(a, nseq, nl);
-          while (nrow.nb == 0) {  // rows without tokens (padding)
-            ++nseq;
-            nrow = row_resolve(a, nseq, row_issue_scalar(a, nseq));
-          }
-          nunit = 0;
+    if (has_next && i == resolve_at) {
+      RowMeta nrow = cur.row;
+      int nunit = cur_unit + 1;
+      if (next_row) {
+        nrow = row_resolve(a, nseq, nl);
+        while (nrow.nb == 0) {  // rows without tokens (padding)
+          ++nseq;
+          nrow = row_resolve(a, nseq, row_issue_scalar(a, nseq));
         }
-        const int x_next = x + cur.nblk;
-        nxt = make_piece(nrow, nunit, 0, min(nrow.nb, x_end - x_next));
-        request_window<kWin>(a, nrow, nwin, slot_of_tok(nxt.t_first), page_shift, lane);
-        const int nhk = min(nxt.hk, a.Hkv - 1);
-        nsv = view_of(nrow, nhk);
-        nkh = a.kv.k_base + (int64_t)nhk * a.kv.head_stride;
-        nvh = a.kv.v_base + (int64_t)nhk * a.kv.head_stride;
+        nunit = 0;
       }
-      const int tb = cur.t_first + i * kBlk;
-      const bool last = (i + 1 == cur.nblk);
-      // the block to request now: the next one of this piece, the first one of the next piece,
-      // or (nothing left) this block again, so that every path has the same loads in flight
-      // the window moves on when the next block's last page lies beyond it
-      if (!last && slot_of_tok(tb + kBlk + (UNIFORM_PAGE ? 0 : kBlk - 1)) - win.first >= kWin) {
-        request_window<kWin>(a, cur.row, win, slot_of_tok(tb + kBlk), page_shift, lane);
-        wait_all_loads();
-      }
-      // real branches, not selects: looking a page up in the next piece's window must not make
-      // every block wait for that window
-      if (last && has_next) {
-        // The next piece's window was requested at block resolve_at, in front of that block's
-        // prefetch.  Two blocks later a wait for younger loads has passed; earlier it has not.
-        if (i <= resolve_at + 1) wait_all_loads();
-        load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE, HALF>(fill, a, nsv, nkh, nvh, nxt.t_first, page_in(nwin, nxt.t_first), c, g,
-                                      lanes_win(nwin), nwin.first);
-      } else {
-        const int ptb = last ? tb : tb + kBlk;
-        load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, UNIFORM_PAGE, HALF>(fill, a, sv, kh, vh, ptb, page_in(win, ptb), c, g, lanes_win(win), win.first);
-      }
-      if (UNIFORM_PAGE && rare(a.new_k && tb + kBlk > sv.last_tok)) {  // the block that ends the row
-        const int slot = slot_of_tok(sv.last_tok);
-        store_new_token<FP8, HALF>(use, a.kv, kh, vh, page_in(win, sv.last_tok), sv.last_tok - slot * page_size, sv.last_tok - tb, c, g);
-      }
-      compute_block<MT, FP8, CAP, HALF, UNIFORM_PAGE>(use, qB, acc, m, l, so, tb, g);
-    };
-    // the piece's first block sits in ra or in rb, wherever the piece before it ended
-    {
-      int i = 0;
-      bool skip_a = in_b;
-      for (;;) {
-        if (!skip_a) {
-          step(i, ra, rb);
-          if (++i == cur.nblk) {
-            in_b = true;
-            break;
-          }
-        }
-        skip_a = false;
-        step(i, rb, ra);
-        if (++i == cur.nblk) {
-          in_b = false;
-          break;
-        }
-      }
+      const int x_next = x + cur.nblk;
+      nxt = make_piece(nrow, nunit, 0, min(nrow.nb, x_end - x_next));
+      request_window<kWin>(a, nrow, nwin, slot_of_tok(nxt.t_first), page_shift, lane);
     }
+    // the window moves on when the next block's last page lies beyond it
+    if (!last && slot_of_tok(tb + kBlk + (PG == kBlocks ? 0 : kBlk - 1)) - win.first >= kWin) {
+      request_window<kWin>(a, cur.row, win, slot_of_tok(tb + kBlk), page_shift, lane);
+      wait_all_loads();
+    }
+    // The next piece's window was requested at block resolve_at, in front of that block's
+    // prefetch.  Two blocks later a wait for younger loads has passed; earlier it has not.
+    if (last && has_next && i <= resolve_at + 1) wait_all_loads();
+    // The block to request now: the next one of this piece, the first one of the next piece, or (nothing left) this block
+    // again.  What differs is chosen in scalars and the loads stand once, in no branch: with a way around them in the code the
+    // compiler waits for all loads where it should wait for the block in use alone.
+    {
+      const bool ahead = last && has_next;
+      const int fhk = ahead ? min(nxt.hk, a.Hkv - 1) : hk;
+      request(fill, view_of(ahead ? nxt.row : cur.row, fhk), fhk, ahead ? nwin : win, ahead ? nxt.t_first : last ? tb : tb + kBlk);
+    }
+    if (PG != kLanes && rare(fresh.on && last)) fresh.put(use, sv.last_tok - tb, c, g);
+    compute_block<MT, FP8, CAP, HALF, PG == kBlocks>(use, qB, acc, m, l, so, tb, g);
+    ++i;
+    if (!last) return true;
 
+    if (PG != kLanes && fresh.on) {
+      const int slot = slot_of_tok(sv.last_tok);
+      fresh.store(a.kv, a.kv.k_base + (int64_t)hk * a.kv.head_stride, a.kv.v_base + (int64_t)hk * a.kv.head_stride,
+                  uniform(win.lds[uniform(slot - win.first)]), sv.last_tok - slot * page_size, c, g);
+    }
     if (cur.hk < a.Hkv) {
       PartDest dest;
       dest.final_rows = cur.final_rows;
@@ -1254,7 +1310,7 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
         }
       }
     }
-    if (!has_next) break;
+    if (!has_next) return false;
     x += cur.nblk;
     cur_unit = next_row ? 0 : cur_unit + 1;
     cur = nxt;
@@ -1265,11 +1321,27 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_balanced_kernel(const Decod
     }
     // the queries queue up right behind the piece's first block, which is already on its way
     load_queries<MT, FP8>(a, cur.row.tq, min(cur.hk, a.Hkv - 1), cur.rg * 16 * MT, c, g, qB);
+    begin_piece();
+    return true;
+  };
+  begin_piece();
+  request(ra, sv, hk, win, cur.t_first);
+  while (step(ra, rb) && step(rb, ra)) {
   }
   if (MERGE && (pm_first.n | pm_last.n)) {
     if (pm_first.n) merge_unit(a, pm_first, pw, wave, nw, a.generation, lane);
     if (pm_last.n) merge_unit(a, pm_last, pw, wave, nw, a.generation, lane);
   }
+}
+
+template <int MT, bool FP8, bool UNIFORM_PAGE, bool CAP, bool MERGE, bool HALF = false>
+__global__ __launch_bounds__(256, FP8 ? 2 : 1) void rpa_decode_balanced_kernel(const DecodeArgs a) {
+  decode_balanced<MT, FP8, UNIFORM_PAGE ? kBlocks : kLanes, CAP, MERGE, HALF>(a);
+}
+
+template <int MT, bool FP8, bool CAP, bool HALF = false>
+__global__ __launch_bounds__(256, FP8 ? 2 : 1) void rpa_decode_balanced_halves_kernel(const DecodeArgs a) {
+  decode_balanced<MT, FP8, kHalves, CAP, false, HALF>(a);
 }
 
 // Merge the n partial rows of one (decode row, query head) and write the finished row.
@@ -1466,7 +1538,7 @@ __global__ __launch_bounds__(merge_threads(SIZE)) void rpa_combine_balanced_kern
 // grid = (token rows, Hkv, row groups of 16 query heads); block = one wave.
 // With the composition on the device (a.dist) seq_end is only a bound: dist_role 1 = the decode partition
 // [0, dist[0]), 2 = everything behind it [dist[0], dist[2]) (custom-mask calls: [0, dist[2])).
-template <bool FP8, bool UNIFORM_PAGE>
+template <bool FP8, Pages PG>
 __global__ __launch_bounds__(64, FP8 ? 2 : 1) void rpa_rows256_kernel(const DecodeArgs a, int seq_begin, int seq_end, int dist_role) {
   if (a.dist && dist_role == 1) {
     seq_end = min(seq_end, scalar_load_i32(a.dist));
@@ -1547,9 +1619,9 @@ __global__ __launch_bounds__(64, FP8 ? 2 : 1) void rpa_rows256_kernel(const Deco
     if (tb_begin >= t_hi) return;  // the merge pass knows how many pieces a row has
     if (split < nsplit - 1) tb_end = min(t_hi, tb_begin + a.chunk);
   }
-  // pages smaller than a block: the lanes look their token rows' pages up in an LDS window of the row's page
+  // kLanes: the lanes look their token rows' pages up in an LDS window of the row's page
   // ids (see decode_segment) instead of fetching them from memory in front of every block
-  __shared__ int32_t win_ids[UNIFORM_PAGE ? 1 : kWinSmallPages];
+  __shared__ int32_t win_ids[PG != kLanes ? 1 : kWinSmallPages];
   const int32_t* win = nullptr;
   int win_first = 0;
   // The registers of a block's K rows are free behind the first product, those of its V rows behind the second: the next
@@ -1558,15 +1630,20 @@ __global__ __launch_bounds__(64, FP8 ? 2 : 1) void rpa_rows256_kernel(const Deco
   // e4m3 keeps; bf16 needs one wave's registers).
   // 32 rows of 8000..16000 tokens x 8 heads: bf16 642 -> 567 us, e4m3 on 16-token pages 431 -> 302 (e4m3 on 64-token pages
   // was level at 300); 100 rows, window 512, e4m3 46.2 -> 31; 8 rows of 300..3000 36.9 -> 26.
-  // Not bf16 on pages under a block, where every half would begin with ids from LDS and an address per lane and load: the loop
+  // Not bf16 on kLanes pages, where every half would begin with ids from LDS and an address per lane and load: the loop
   // there is the plain one, options asked per score (32 rows 575 us, 589 with half a block ahead; 64 rows of 1000 .. 8000 521
   // and 534).
-  constexpr bool kAhead = FP8 || UNIFORM_PAGE;
-  int page = 0, page_next = 0;
-  auto page_of = [&](int tb) __attribute__((always_inline)) { return scalar_load_i32(sv.pages + page_slot_of(sv, min(tb, sv.last_tok))); };
+  constexpr bool kAhead = FP8 || PG != kLanes;
+  BlockPages page = {}, page_next = {};
+  auto page_of = [&](int tb) __attribute__((always_inline)) {
+    BlockPages p = {};
+    p.lo = scalar_load_i32(sv.pages + page_slot_of(sv, min(tb, sv.last_tok)));
+    if constexpr (PG == kHalves) p.hi = scalar_load_i32(sv.pages + page_slot_of(sv, min(tb + 16, sv.last_tok)));
+    return p;
+  };
   KvRegs<FP8> r0, r1;
   auto locate = [&](int tb) __attribute__((always_inline)) {
-    if constexpr (UNIFORM_PAGE) {
+    if constexpr (PG != kLanes) {
       page = page_next;
       page_next = page_of(tb + kBlk);
     } else if (!win || page_slot_of(sv, min(tb + kBlk - 1, sv.last_tok)) - win_first >= kWinSmallPages) {
@@ -1578,14 +1655,14 @@ __global__ __launch_bounds__(64, FP8 ? 2 : 1) void rpa_rows256_kernel(const Deco
   };
   auto request_k = [&](int tb) __attribute__((always_inline)) {
     locate(tb);
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, false, false, kOnlyK>(r0, a, sv, kh, vh, tb, page, c, g, win, win_first);
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, false, false, kOnlyK>(r1, a, sv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
+    load_block<FP8, PG, PG == kLanes, false, false, kOnlyK>(r0, a, sv, kh, vh, tb, page, c, g, win, win_first);
+    load_block<FP8, PG, PG == kLanes, false, false, kOnlyK>(r1, a, sv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
   };
   auto request_v = [&](int tb) __attribute__((always_inline)) {
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, false, false, kOnlyV>(r0, a, sv, kh, vh, tb, page, c, g, win, win_first);
-    load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE, false, false, kOnlyV>(r1, a, sv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
+    load_block<FP8, PG, PG == kLanes, false, false, kOnlyV>(r0, a, sv, kh, vh, tb, page, c, g, win, win_first);
+    load_block<FP8, PG, PG == kLanes, false, false, kOnlyV>(r1, a, sv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
   };
-  if constexpr (UNIFORM_PAGE) page_next = page_of(tb_begin);
+  if constexpr (PG != kLanes) page_next = page_of(tb_begin);
   if (kAhead && tb_begin < tb_end) {
     request_k(tb_begin);
     request_v(tb_begin);
@@ -1594,8 +1671,8 @@ __global__ __launch_bounds__(64, FP8 ? 2 : 1) void rpa_rows256_kernel(const Deco
     const bool more = kAhead && tb + kBlk < tb_end;
     if constexpr (!kAhead) {
       locate(tb);
-      load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(r0, a, sv, kh, vh, tb, page, c, g, win, win_first);
-      load_block<FP8, UNIFORM_PAGE, !UNIFORM_PAGE>(r1, a, sv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
+      load_block<FP8, PG, PG == kLanes>(r0, a, sv, kh, vh, tb, page, c, g, win, win_first);
+      load_block<FP8, PG, PG == kLanes>(r1, a, sv, kh + kHalfB, vh + kHalfB, tb, page, c, g, win, win_first);
     }
     f32x4_t s[2];
     {
@@ -1797,7 +1874,7 @@ void launch_combine(const DecodeArgs& a, hipStream_t st) {
 #undef RPA_COMBINE
 }
 
-template <bool FP8, bool UNIFORM, bool CAP>
+template <bool FP8, Pages PG, bool CAP>
 void launch_decode_variant(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t st) {
   // LDS nobody uses keeps four waves on a CU, one per SIMD: without it the dispatcher doubles workgroups up on some CUs
   // while others stand idle, and a CU draws about 39 bytes per ns at most (fixed plan, 128 rows of 256..2048 tokens x 2
@@ -1811,41 +1888,48 @@ void launch_decode_variant(const DecodeArgs& a, dim3 grid, dim3 block, hipStream
     const unsigned parts = std::max(84u << 10, (unsigned)(kRowWaves * min(a.G, 16) * kRowPitch * sizeof(float)));
     if constexpr (!FP8) {
       if (a.q_dim == 64) {
-        hipLaunchKernelGGL((rpa_decode_row_kernel<false, UNIFORM, CAP, true>), grid, block, parts, st, a);
+        hipLaunchKernelGGL((rpa_decode_row_kernel<false, PG, CAP, true>), grid, block, parts, st, a);
         return;
       }
     }
-    hipLaunchKernelGGL((rpa_decode_row_kernel<FP8, UNIFORM, CAP>), grid, block, parts, st, a);
+    hipLaunchKernelGGL((rpa_decode_row_kernel<FP8, PG, CAP>), grid, block, parts, st, a);
     return;
   }
   // heads of 64 dims (rows of 128, the second half zero): half the bytes.  (Not with the opt-in merge inside the kernel.)
   if constexpr (!FP8) {
     if (a.q_dim == 64 && !(a.balanced && a.merge_counters)) {
-      if (a.balanced) hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, false, UNIFORM, CAP, false, true>), grid, block, lds, st, a);
-      else hipLaunchKernelGGL((rpa_decode_splitkv_kernel<1, false, UNIFORM, CAP, true>), grid, block, lds, st, a);
+      if (!a.balanced) hipLaunchKernelGGL((rpa_decode_splitkv_kernel<1, false, PG, CAP, true>), grid, block, lds, st, a);
+      else if constexpr (PG == kHalves) hipLaunchKernelGGL((rpa_decode_balanced_halves_kernel<1, false, CAP, true>), grid, block, lds, st, a);
+      else hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, false, PG == kBlocks, CAP, false, true>), grid, block, lds, st, a);
       return;
     }
   }
-  if (a.balanced && a.merge_counters)
-    hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, FP8, UNIFORM, CAP, true>), grid, block, lds, st, a);
-  else if (a.balanced)
-    hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, FP8, UNIFORM, CAP, false>), grid, block, lds, st, a);
-  else hipLaunchKernelGGL((rpa_decode_splitkv_kernel<1, FP8, UNIFORM, CAP>), grid, block, lds, st, a);
+  if (!a.balanced) {
+    hipLaunchKernelGGL((rpa_decode_splitkv_kernel<1, FP8, PG, CAP>), grid, block, lds, st, a);
+  } else if constexpr (PG == kHalves) {
+    hipLaunchKernelGGL((rpa_decode_balanced_halves_kernel<1, FP8, CAP>), grid, block, lds, st, a);
+  } else if (a.merge_counters) {
+    hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, FP8, PG == kBlocks, CAP, true>), grid, block, lds, st, a);
+  } else {
+    hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, FP8, PG == kBlocks, CAP, false>), grid, block, lds, st, a);
+  }
 }
 
-hipError_t launch_decode_mt(const DecodeArgs& a, dim3 grid, dim3 block, bool uniform, hipStream_t st) {
+template <bool FP8, Pages PG>
+void launch_decode_pages(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t st) {
   // soft cap and logit rounding share the general score path
-  const bool cap = a.sm.soft_cap != 0.f || a.sm.round_logits != 0;
-  const int key = (a.fp8 ? 4 : 0) | (uniform ? 2 : 0) | (cap ? 1 : 0);
-  switch (key) {
-    case 0: launch_decode_variant<false, false, false>(a, grid, block, st); break;
-    case 1: launch_decode_variant<false, false, true>(a, grid, block, st); break;
-    case 2: launch_decode_variant<false, true, false>(a, grid, block, st); break;
-    case 3: launch_decode_variant<false, true, true>(a, grid, block, st); break;
-    case 4: launch_decode_variant<true, false, false>(a, grid, block, st); break;
-    case 5: launch_decode_variant<true, false, true>(a, grid, block, st); break;
-    case 6: launch_decode_variant<true, true, false>(a, grid, block, st); break;
-    default: launch_decode_variant<true, true, true>(a, grid, block, st); break;
+  if (a.sm.soft_cap != 0.f || a.sm.round_logits != 0) launch_decode_variant<FP8, PG, true>(a, grid, block, st);
+  else launch_decode_variant<FP8, PG, false>(a, grid, block, st);
+}
+
+hipError_t launch_decode_mt(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t st) {
+  switch (pages_of(a.pt.page_size) * 2 + (a.fp8 ? 1 : 0)) {
+    case kLanes * 2: launch_decode_pages<false, kLanes>(a, grid, block, st); break;
+    case kLanes * 2 + 1: launch_decode_pages<true, kLanes>(a, grid, block, st); break;
+    case kHalves * 2: launch_decode_pages<false, kHalves>(a, grid, block, st); break;
+    case kHalves * 2 + 1: launch_decode_pages<true, kHalves>(a, grid, block, st); break;
+    case kBlocks * 2: launch_decode_pages<false, kBlocks>(a, grid, block, st); break;
+    default: launch_decode_pages<true, kBlocks>(a, grid, block, st); break;
   }
   return hipGetLastError();
 }
@@ -1858,9 +1942,8 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
   const int head_groups = (a.Hkv + nw - 1) / nw;
   // more than 16 query heads per kv head: further groups of 16 re-walk the KV (rare: MQA-like shapes)
   const int row_groups = (a.G + 15) / 16;
-  const bool uniform = (a.pt.page_size % kBlk) == 0;
   if (a.balanced) {
-    hipError_t e = launch_decode_mt(a, dim3(a.num_wgs), dim3(a.waves_per_wg * 64), uniform, stream);
+    hipError_t e = launch_decode_mt(a, dim3(a.num_wgs), dim3(a.waves_per_wg * 64), stream);
     if (e != hipSuccess) return e;
     if (!a.merge_counters) {
       const dim3 grid((unsigned)a.Hq * (unsigned)a.num_rows);
@@ -1873,12 +1956,12 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
     return hipGetLastError();
   }
   if (a.whole_rows)
-    return launch_decode_mt(a, dim3((unsigned)a.num_rows, 1, (unsigned)(a.Hkv * row_groups)), dim3(kRowWaves * 64), uniform, stream);
+    return launch_decode_mt(a, dim3((unsigned)a.num_rows, 1, (unsigned)(a.Hkv * row_groups)), dim3(kRowWaves * 64), stream);
   if ((int64_t)a.max_splits * a.num_rows > 0x7fffffffLL || (int64_t)a.Hq * a.num_rows > 0x7fffffffLL)
     return hipErrorInvalidValue;
   dim3 grid((unsigned)max(a.max_splits, 1) * (unsigned)a.num_rows, 1, head_groups * row_groups);
   dim3 block(nw * 64);
-  hipError_t e = launch_decode_mt(a, grid, block, uniform, stream);
+  hipError_t e = launch_decode_mt(a, grid, block, stream);
   if (e != hipSuccess) return e;
   if (a.max_splits > 1) {
     launch_combine<128>(a, stream);
@@ -1935,14 +2018,16 @@ hipError_t launch_rows256(const DecodeArgs& a, int seq_begin, int seq_end, int m
   const int nsplit = a.max_splits > 1 ? a.max_splits : 1;
   if ((int64_t)max_token_rows * nsplit > 0x7fffffffLL) return hipErrorInvalidValue;
   const dim3 grid(max_token_rows * nsplit, a.Hkv, (a.G + 15) / 16), block(64);
-  const bool uniform = (a.pt.page_size % kBlk) == 0;
-  if (a.fp8) {
-    if (uniform) hipLaunchKernelGGL((rpa_rows256_kernel<true, true>), grid, block, 0, stream, a, seq_begin, seq_end, dist_role);
-    else hipLaunchKernelGGL((rpa_rows256_kernel<true, false>), grid, block, 0, stream, a, seq_begin, seq_end, dist_role);
-  } else {
-    if (uniform) hipLaunchKernelGGL((rpa_rows256_kernel<false, true>), grid, block, 0, stream, a, seq_begin, seq_end, dist_role);
-    else hipLaunchKernelGGL((rpa_rows256_kernel<false, false>), grid, block, 0, stream, a, seq_begin, seq_end, dist_role);
+#define RPA_ROWS256(FP8, PG) hipLaunchKernelGGL((rpa_rows256_kernel<FP8, PG>), grid, block, 0, stream, a, seq_begin, seq_end, dist_role)
+  switch (pages_of(a.pt.page_size) * 2 + (a.fp8 ? 1 : 0)) {
+    case kLanes * 2: RPA_ROWS256(false, kLanes); break;
+    case kLanes * 2 + 1: RPA_ROWS256(true, kLanes); break;
+    case kHalves * 2: RPA_ROWS256(false, kHalves); break;
+    case kHalves * 2 + 1: RPA_ROWS256(true, kHalves); break;
+    case kBlocks * 2: RPA_ROWS256(false, kBlocks); break;
+    default: RPA_ROWS256(true, kBlocks); break;
   }
+#undef RPA_ROWS256
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nsplit == 1) return e;
   if ((int64_t)a.Hq * a.num_rows > 0x7fffffffLL) return hipErrorInvalidValue;

@@ -1947,3 +1947,42 @@ def test_prefill_rows_copied_by_page(pkg, wl, gpu, monkeypatch, P, D, fp8, cap):
         for splits in ("0", "2"):
             monkeypatch.setenv("RPA_PREFILL_SPLITS", splits)
             assert_parity(gpu_out(pkg, b, gpu).float(), want.float(), **(FP8_TOL if fp8 else BF16_TOL))
+
+
+@pytest.mark.parametrize("P", [16, 48, 24])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("rows,Hkv,head_dim", [(5, 2, 128), (40, 8, 128), (40, 8, 64), (7, 2, 256)])
+def test_decode_rows_by_halves_of_a_block(pkg, wl, gpu, monkeypatch, P, fp8, rows, Hkv, head_dim):
+    """Pages of whole 16-token halves (16, 48) against pages that are looked up row by row (24): lengths around halves, blocks and
+    pieces, in pieces and on the balanced plan, the new token brought along (its slot and all unused ones hold NaN), a
+    window whose first block is cut.  The new tokens' bytes arrive in their slots."""
+    if fp8 and head_dim == 64:
+        pytest.skip("heads of 64 dims in rows of 128 are bf16")
+    edges = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 79, 80, 81]
+    kv_lens = [edges[i % 16] + (0 if i < 16 else 32 * (37 * i % 90)) for i in range(rows - 1)] + [2905]
+    say(f"halves P={P} fp8={fp8} rows={rows} D={head_dim}")
+    wide = max(head_dim, 128)
+    for window in (None, 50):
+        b = wl.make_batch("halves", [1] * rows, kv_lens, num_q_heads=2 * Hkv, num_kv_heads=Hkv, head_dim=wide, page_size=P, seed=5,
+                          kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16, sliding_window=window)
+        if head_dim < wide:
+            b.kv_cache[..., head_dim:] = 0
+            b.q[..., head_dim:] = 0
+        want = oracle_out(b)
+        keys, values, cache = with_new_tokens(b)
+        g, cache = b.to(gpu), cache.to(gpu)
+        if head_dim < wide:
+            keys, values = keys[..., :head_dim].contiguous(), values[..., :head_dim].contiguous()
+        q = g.q[..., :head_dim].contiguous()
+        out, after = pkg.ragged_paged_attention(
+            q, keys.to(gpu), values.to(gpu), cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, b.distribution.numpy(),
+            sm_scale=b.sm_scale, sliding_window=window, k_scale=g.k_scale, v_scale=g.v_scale, max_kv_len=max(kv_lens), max_q_len=1,
+            host_kv_lens=b.kv_lens.numpy())
+        torch.cuda.synchronize()
+        assert_parity(out.cpu().float(), want[..., :head_dim].float(), **(FP8_TOL if fp8 else BF16_TOL))
+        bits = torch.uint8 if fp8 else torch.int16
+        got, full, expect = after.cpu().view(bits), b.kv_cache.view(bits), with_new_tokens(b)[2].view(bits).clone()
+        for i, kv in enumerate(kv_lens):
+            page = int(b.page_indices[int(b.cu_kv_lens[i]) // P + (kv - 1) // P])
+            expect[page, (kv - 1) % P] = full[page, (kv - 1) % P]
+        assert torch.equal(got, expect)
