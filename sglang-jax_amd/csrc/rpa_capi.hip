@@ -52,6 +52,7 @@ const Tuning& tuning() {
   geti("RPA_DECODE_WAVES_PER_WG", t.decode_waves_per_wg);
   geti("RPA_DECODE_WAVE_CAPACITY", t.decode_wave_capacity);
   geti("RPA_DECODE_ROW_KB", t.decode_row_kb);
+  geti("RPA_DECODE_ROW_PIECES", t.decode_row_pieces);
   geti("RPA_DECODE_MERGE_IN_KERNEL", t.decode_merge_in_kernel);
   geti("RPA_DECODE_LDS_KB", t.decode_lds_kb);
   geti("RPA_MASK_BITS", t.mask_bits);
@@ -373,18 +374,68 @@ bool use_balanced(const RpaParams* p, const SplitPlan& fixed) {
   return true;
 }
 
-// Whether rpa_decode_row_kernel takes the rows: what a workgroup cannot read in the time that a merge pass costs loses (a CU
-// draws about 39 bytes per ns), and a second round of them does.  Up to 255 tokens or a window of 224 in bf16, twice that in
-// e4m3: 10.2 -> 7.5 us for a few rows (the second launch is the host's time too), 64 rows of 64..255 x 4 heads 15.7 -> 12.1;
-// 511 tokens: 9.8 against 11.0.
-bool rows_in_one_workgroup(const RpaParams* p, const SplitPlan& fixed) {
-  if (fixed.splits <= 1 || p->num_splits > 0) return false;
-  int64_t longest = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages, p->cu_kv_lens != nullptr);
+// The pieces of rpa_decode_row_kernel, a workgroup of eight waves for each (row, kv head, piece), one to a CU; splits == 0: it does
+// not take the rows.
+//   * Rows of up to 128 KiB per kv head (255 bf16 tokens, twice that in e4m3, or a short window), as many as there are CUs: whole, in
+//     one launch.  10.2 -> 7.5 us for a few rows (the second launch is the host's time too), 64 rows of 64..255 x 4 heads
+//     15.7 -> 12.1; a few rows of 511 tokens: 7.8 against 9.6, a CU draws about 40 bytes per ns from beyond its L1.
+//   * Even rows whose pieces are one round of the CUs, nearly all of them, where those of single waves are more than a workgroup per
+//     CU: a piece of 224 bf16 tokens and more is a
+//     stream of eight waves that start together and are merged in LDS, against single waves on 64 to 256 tokens or on a share of the
+//     balanced plan, each with a start and a partial row of its own.  32 rows of 800..1000 tokens x 8 heads 31.5 -> 24.1 us, 8 of
+//     800..1000 (4 pieces) 14.0 -> 12.0, 2 of 8000 (16 pieces) 21.5 -> 17.9, e4m3 32 x 1600..2000 34.7 -> 26.6.  Not below that
+//     (8 x 500 in 4 pieces 9.1 -> 9.8; e4m3, whose blocks cost more, 16 x 1000 in 2 13.5 -> 14.3), nor beyond 640 KiB (whole rows 1 MiB) a piece, where every plan streams at the memory's rate
+//     (16 x 8000 e4m3 46.8 -> 49.2), nor for uneven rows (mean under 0.75 of the longest, 0.85 in more than two
+//     pieces: 16 x 500..2000 x 8 heads, 0.78 and 2 pieces, 26.3 -> 24.8, x 2 heads, 8 pieces, 12.2 -> 13.6)
+//     or a quarter of the CUs idle (48 rows x 2 heads x 800..1000 16.5 -> 18.0), unless the rows are whole and of up to 512 KiB
+//     (24 x 800..1000 x 8 heads 25.2 -> 23.2).
+SplitPlan row_plan(const RpaParams* p, const SplitPlan& fixed) {
+  const SplitPlan none = {0, 0};
+  const rpa::Tuning& tune = rpa::tuning();
+  if (p->num_splits > 0 || tune.decode_row_kb == 0) return none;
+  int64_t longest = std::max<int64_t>(1, kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages, p->cu_kv_lens != nullptr));
   if (p->sliding_window > 0) longest = std::min(longest, (int64_t)p->sliding_window + 31);
-  const int64_t bytes = longest * 2 * (q_dim_of(p) == 64 && p->kv_dtype == RPA_KV_BF16 ? 64 : p->head_dim) * esize_of(p->kv_dtype);
+  const int64_t token = 2 * (q_dim_of(p) == 64 && p->kv_dtype == RPA_KV_BF16 ? 64 : p->head_dim) * esize_of(p->kv_dtype);
   const int64_t units = (int64_t)p->decode_end * p->num_kv_heads * ((p->num_q_heads / p->num_kv_heads + 15) / 16);
-  const int kb = rpa::tuning().decode_row_kb >= 0 ? rpa::tuning().decode_row_kb : 128;
-  return bytes <= ((int64_t)kb << 10) && units <= rpa::compute_units();
+  const int64_t cus = rpa::compute_units(), kb = tune.decode_row_kb >= 0 ? tune.decode_row_kb : 128;
+  auto pieces = [&](int64_t n) {
+    SplitPlan sp;
+    sp.chunk = (int)(((longest + n - 1) / n + 31) / 32 * 32);
+    sp.splits = (int)((longest + sp.chunk - 1) / sp.chunk);
+    return sp;
+  };
+  if (tune.decode_row_pieces > 0) return pieces(tune.decode_row_pieces);
+  if (units > cus || units < 1) return none;
+  if (longest * token <= (kb << 10)) return fixed.splits > 1 ? pieces(1) : none;
+  const SplitPlan sp = pieces(cus / units);
+  const bool even = p->sum_decode_kv_len > 0 && p->max_kv_len > 0 &&
+                    (p->sliding_window > 0 && p->max_kv_len > p->sliding_window
+                         ? p->sum_decode_kv_len >= (int64_t)p->decode_end * p->sliding_window
+                         : p->sum_decode_kv_len * 20 >= (int64_t)p->decode_end * p->max_kv_len * (sp.splits <= 2 ? 15 : 17));
+  if (!even || fixed.splits * units <= 2 * cus) return none;
+  const bool fp8 = p->kv_dtype == RPA_KV_FP8_E4M3;
+  const int64_t bytes = sp.chunk * token, least = (fp8 ? 160 : 112) << 10, most = sp.splits > 1 ? 640 << 10 : 1 << 20;
+  const int64_t busy = cus / units * units;
+  if (busy * 8 < cus * 7 && !(busy * 4 >= cus * 3 && sp.splits == 1 && bytes <= (512 << 10))) return none;
+  // (a call that brings less workspace than this needs stays on the plan that stood here before)
+  const size_t need = sp.splits > 1 ? (size_t)p->decode_end * sp.splits * p->num_q_heads * (p->head_dim + 2) * sizeof(float) : 0;
+  return bytes >= least && bytes <= most && need <= workspace_of(p) ? sp : none;
+}
+
+struct DecodeChoice {
+  bool balanced, rows;  // neither: pieces of single waves
+  SplitPlan sp;         // (not balanced)
+};
+DecodeChoice decode_choice(const RpaParams* p, bool token_rows = false) {
+  DecodeChoice c = {false, false, decode_plan(p)};
+  const SplitPlan r = row_plan(p, c.sp);
+  if (r.splits > 0) {
+    c.rows = true;
+    c.sp = r;
+    return c;
+  }
+  c.balanced = !token_rows && use_balanced(p, c.sp);
+  return c;
 }
 
 // Bytes of KV the decode rows will read, as far as the host knows (its sum of lengths, or rows
@@ -705,11 +756,9 @@ static size_t required_workspace_bytes(const RpaParams* p_in) {
   const RpaParams* p = &pv;
   if (p->decode_end <= 0) return 0;
   if (p->head_dim == 256) return rows256_workspace(p);
-  const SplitPlan sp = decode_plan(p);
-  if (use_balanced(p, sp))
-    return balanced_layout(p).total;
-  if (sp.splits <= 1 || rows_in_one_workgroup(p, sp)) return 0;
-  return (size_t)p->decode_end * sp.splits * p->num_q_heads * (p->head_dim + 2) * sizeof(float);
+  const DecodeChoice c = decode_choice(p);
+  if (c.balanced) return balanced_layout(p).total;
+  return c.sp.splits <= 1 ? 0 : (size_t)p->decode_end * c.sp.splits * p->num_q_heads * (p->head_dim + 2) * sizeof(float);
 }
 
 size_t rpa_workspace_bytes(const RpaParams* given) {
@@ -763,8 +812,8 @@ static bool takes_token_rows(const RpaParams* p) {
 }
 static size_t token_row_workspace(const RpaParams* p) {
   const RpaParams v = token_row_view(p);
-  const SplitPlan sp = decode_plan(&v);
-  return sp.splits <= 1 || rows_in_one_workgroup(&v, sp) ? 0 : (size_t)v.decode_end * sp.splits * v.num_q_heads * (v.head_dim + 2) * sizeof(float);
+  const SplitPlan sp = decode_choice(&v, true).sp;
+  return sp.splits <= 1 ? 0 : (size_t)v.decode_end * sp.splits * v.num_q_heads * (v.head_dim + 2) * sizeof(float);
 }
 
 // Decode rows; with keys / values the rows' own tokens are not in the cache yet and are written by these kernels.
@@ -775,7 +824,8 @@ static int decode_rows(const RpaParams* p_in, const void* keys, const void* valu
   if (p->decode_end <= 0) return RPA_OK;
   if (p->mask_mode == RPA_MASK_CUSTOM) return RPA_OK;  // masked rows all go through the prefill kernel
   if (p->head_dim == 256) return rows256(p, 0, p->decode_end, stream, p->distribution ? 1 : 0);
-  const SplitPlan sp = decode_plan(p);
+  const DecodeChoice choice = decode_choice(p, token_rows);
+  const SplitPlan& sp = choice.sp;
   rpa::DecodeArgs a;
   a.new_k = static_cast<const char*>(keys);
   a.new_v = static_cast<const char*>(values);
@@ -802,9 +852,9 @@ static int decode_rows(const RpaParams* p_in, const void* keys, const void* valu
   a.merge_counters = nullptr;
   a.generation = 0;
   a.dist = p->distribution;
-  a.balanced = (!token_rows && use_balanced(p, sp)) ? 1 : 0;
+  a.balanced = choice.balanced ? 1 : 0;
   a.num_wgs = decode_wgs(p);
-  a.whole_rows = (!a.balanced && rows_in_one_workgroup(p, sp)) ? 1 : 0;
+  a.group_rows = choice.rows ? 1 : 0;
   a.waves_per_wg = a.balanced ? decode_waves_per_wg(p) : decode_fixed_waves(p);
   a.min_blocks_per_wave = std::max(1, rpa::tuning().decode_min_chunk / 32);
   a.forced_blocks_per_wave = 0;
@@ -832,7 +882,7 @@ static int decode_rows(const RpaParams* p_in, const void* keys, const void* valu
       // look like this call's
       a.generation = (g_decode_generation.fetch_add(1, std::memory_order_relaxed) % ((1ull << 48) - 1)) + 1;
     }
-  } else if (sp.splits > 1 && !a.whole_rows) {
+  } else if (sp.splits > 1) {
     const size_t need = token_rows ? token_row_workspace(p_in) : required_workspace_bytes(p);
     if (!p->workspace || p->workspace_bytes < need)
       return fail(RPA_EINVAL_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, p->workspace_bytes);
@@ -1034,7 +1084,7 @@ static bool decode_takes_new_tokens(const RpaParams* p_in) {
   if (p_in->head_dim != 128 || p_in->mask_mode == RPA_MASK_CUSTOM || !rows_take_new_tokens(p_in)) return false;
   if (p_in->page_size % 16 == 0) return true;
   const RpaParams p = planning_view(p_in);
-  return !use_balanced(&p, decode_plan(&p));
+  return !decode_choice(&p).balanced;
 }
 
 static int write_new_tokens(const RpaParams* p, const void* keys, const void* values, bool skip_decode_rows, void* stream) {
@@ -1097,13 +1147,14 @@ int rpa_describe_plan(const RpaParams* given, char* buf, size_t len) {
   buf[0] = 0;
   auto put_rows = [&](const char* what, const RpaParams* v, bool token_rows, size_t workspace) {
     const rpa::ShapeRule& r = decode_shape(v);
-    const SplitPlan sp = decode_plan(v);
-    const bool bal = !token_rows && use_balanced(v, sp), whole = !bal && rows_in_one_workgroup(v, sp);
+    const DecodeChoice c = decode_choice(v, token_rows);
+    const SplitPlan& sp = c.sp;
+    const bool bal = c.balanced, whole = c.rows;
     put("%s: shape=%s kernel=%s rows=%d", what, r.name,
         whole ? "rpa_decode_row_kernel" : bal ? "rpa_decode_balanced_kernel" : "rpa_decode_splitkv_kernel", v->decode_end);
     if (!whole) put(" waves_per_wg=%d", bal ? decode_waves_per_wg(v) : decode_fixed_waves(v));
     if (bal) put(" resident_waves=%d merge=rpa_combine_balanced_kernel", decode_wave_capacity(v));
-    else if (!whole) put(" pieces_per_row=%d chunk=%d merge=%s", sp.splits, sp.chunk, sp.splits > 1 ? "rpa_combine_kernel" : "none");
+    else if (!whole || sp.splits > 1) put(" pieces_per_row=%d chunk=%d merge=%s", sp.splits, sp.chunk, sp.splits > 1 ? "rpa_combine_kernel" : "none");
     put(" workspace=%zu\n", workspace);
   };
   if (takes_token_rows(p_in)) {

@@ -162,9 +162,10 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
 
 // The same of a block whose 32 tokens all lie in the cache.  Buffer loads: a half's first row as the base, one offset per lane
 // for all K rows and another for all V rows, what differs between the loads in a scalar: no vector instruction beside the
-// loads themselves.
+// loads themselves.  wanted == false: a block that nobody needs, asked for so that the waits behind it count the same on every
+// path; its buffers have no bytes, and nothing is fetched.
 template <bool FP8, Pages PG, bool HALF>
-__device__ __forceinline__ void load_full_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, BlockPages page, int c, int g,
+__device__ __forceinline__ void load_full_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, BlockPages page, bool wanted, int c, int g,
                                                 const int32_t* win = nullptr, int win_first = 0) {
   if constexpr (PG == kLanes) {
     load_block<FP8, PG, true, false, HALF>(r, a, s, kh, vh, tb, page, c, g, win, win_first);
@@ -174,13 +175,11 @@ __device__ __forceinline__ void load_full_block(KvRegs<FP8>& r, const DecodeArgs
     const int off_v = 4 * g * kv.tok_stride + (HALF ? c & 7 : c) * (FP8 ? 8 : 16);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      // (a second half past the end of the row, which only a prefetch for nobody asks for, is the first one again)
-      const bool hi = PG == kHalves && h && tb + 16 <= s.last_tok;
-      const int tok = hi ? tb + 16 : tb;
-      const int64_t at = (int64_t)(hi ? page.hi : page.lo) * kv.page_stride + (int64_t)(tok - page_slot_of(s, tok) * s.page_size) * kv.tok_stride;
-      const int behind = PG == kBlocks ? h * 16 * kv.tok_stride : 0;
-      const auto k = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kh) + at, 0, 0x7fffffff, 0x00020000);
-      const auto v = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vh) + at, 0, 0x7fffffff, 0x00020000);
+      const int tok = PG == kHalves && h ? tb + 16 : tb;
+      const int64_t at = (int64_t)(PG == kHalves && h ? page.hi : page.lo) * kv.page_stride + (int64_t)(tok - page_slot_of(s, tok) * s.page_size) * kv.tok_stride;
+      const int behind = PG == kBlocks ? h * 16 * kv.tok_stride : 0, bytes = wanted ? 0x7fffffff : 0;
+      const auto k = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kh) + at, 0, bytes, 0x00020000);
+      const auto v = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vh) + at, 0, bytes, 0x00020000);
 #pragma unroll
       for (int st = 0; st < (FP8 || HALF ? 2 : 4); ++st)
         r.k[h][st] = __builtin_amdgcn_raw_buffer_load_b128(k, off_k + st * (FP8 ? 16 : 64), behind, kCacheBits);
@@ -196,22 +195,22 @@ __device__ __forceinline__ void load_full_block(KvRegs<FP8>& r, const DecodeArgs
 // Any block, out of the cache alone (a new token's slot is read for what stands there): rows past the row's last token are the
 // last token's again, by a bound on the lanes' offsets.
 template <bool FP8, Pages PG, bool HALF>
-__device__ __forceinline__ void load_cached_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, BlockPages page, int c, int g,
+__device__ __forceinline__ void load_cached_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, BlockPages page, bool wanted, int c, int g,
                                                   const int32_t* win, int win_first) {
   if constexpr (PG == kLanes) {
     load_block<FP8, PG, true, false, HALF>(r, a, s, kh, vh, tb, page, c, g, win, win_first);
   } else {
     const KvAddr& kv = a.kv;
     const int lane_k = g * (FP8 ? 32 : 16), lane_v = (HALF ? c & 7 : c) * (FP8 ? 8 : 16);
-    const int row_k = c * kv.tok_stride, row_v = 4 * g * kv.tok_stride;
+    const int row_k = c * kv.tok_stride, row_v = 4 * g * kv.tok_stride, bytes = wanted ? 0x7fffffff : 0;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const bool hi = PG == kHalves && h && tb + 16 <= s.last_tok;
       const int tok = hi ? tb + 16 : tb, first = PG == kBlocks ? h * 16 : 0;
       const int64_t at = (int64_t)(hi ? page.hi : page.lo) * kv.page_stride + (int64_t)(tok - page_slot_of(s, tok) * s.page_size) * kv.tok_stride;
       const int most = min(s.last_tok - tok, PG == kBlocks ? 31 : 15) * kv.tok_stride;  // offset of the last row that there is
-      const auto k = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kh) + at, 0, 0x7fffffff, 0x00020000);
-      const auto v = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vh) + at, 0, 0x7fffffff, 0x00020000);
+      const auto k = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kh) + at, 0, bytes, 0x00020000);
+      const auto v = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vh) + at, 0, bytes, 0x00020000);
       const int off_k = min(row_k + first * kv.tok_stride, most) + lane_k;
 #pragma unroll
       for (int st = 0; st < (FP8 || HALF ? 2 : 4); ++st)
@@ -509,8 +508,7 @@ __device__ __forceinline__ void requantise_queries(const DecodeArgs& a, u32x4_t 
 template <int MT, bool THROUGH = false>
 __device__ __forceinline__ void write_rows(const DecodeArgs& a, const f32x4_t (&acc)[MT][8], const float (&m)[MT],
                                            const float (&l)[MT], int tq, int hk, int row0, const PartDest dest,
-                                           int c, int g) {
-  const float vs = a.v_scale ? a.v_scale[hk] : 1.0f;
+                                           float vs, int c, int g) {
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     float lt = l[mt];
@@ -564,10 +562,70 @@ __device__ __forceinline__ void write_rows(const DecodeArgs& a, const f32x4_t (&
 }
 
 // One row: query token tq of sequence seq, which sees kv_len tokens; new tokens start at position fresh_first, whose
-// query token is fresh_tq.
+// query token is fresh_tq; its page ids start at page_indices[page0].
 struct RowRef {
   int seq, tq, kv_len, fresh_first, fresh_tq;
+  int64_t page0;
 };
+
+__device__ __forceinline__ int owner_of_token(const int32_t* cu_q_lens, int num_seqs, int tok) {
+  int lo = 0, hi = num_seqs;  // last i with cu_q_lens[i] <= tok (zero-length sequences are skipped)
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (cu_q_lens[mid] <= tok) lo = mid; else hi = mid;
+  }
+  return lo;
+}
+
+__device__ __forceinline__ int64_t first_page(const DecodeArgs& a, int seq, int cu_kv) {
+  if (!a.pt.cu_kv_lens) return (int64_t)seq * a.pt.pages_per_seq;
+  const int P = a.pt.page_size;
+  return (P & (P - 1)) == 0 ? cu_kv >> (31 - __builtin_clz(P)) : cu_kv / P;
+}
+
+// Row `index` of the fixed plan: decode row `index`, or (token_rows) query token `index` of whatever sequence owns it.
+// false: nothing there.
+// Everything that the batch holds about the row is asked for at once.  With each answer asking the next question (composition, owner by a
+// binary search, lengths, page offset) it was 1.9 us of a launch of 8, for a bucket of 5 rows.
+__device__ __forceinline__ bool fixed_row(const DecodeArgs& a, int index, RowRef& row) {
+  const int32_t* cu_kv_lens = a.pt.cu_kv_lens ? a.pt.cu_kv_lens : a.pt.kv_lens;  // (any words that are there)
+  if (a.token_rows) {
+    int cu_kv;
+    if (a.num_seqs < 64) {  // a sequence per lane
+      const int lane = threadIdx.x & 63, own = min(lane, a.num_seqs - 1);
+      const int seqs_now = scalar_load_i32(a.dist ? a.dist + 2 : a.pt.kv_lens);
+      const int q0 = a.pt.cu_q_lens[min(lane, a.num_seqs)], kv = a.pt.kv_lens[own], at = cu_kv_lens[own];
+      const int seqs = a.dist ? max(min(a.num_seqs, seqs_now), 0) : a.num_seqs;
+      if (index >= __builtin_amdgcn_readlane(q0, seqs)) return false;
+      row.tq = index;
+      row.seq = max(__builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < seqs && q0 <= index)) - 1, 0);
+      row.fresh_tq = __builtin_amdgcn_readlane(q0, row.seq);
+      row.fresh_first = __builtin_amdgcn_readlane(kv, row.seq) - (__builtin_amdgcn_readlane(q0, row.seq + 1) - row.fresh_tq);
+      cu_kv = __builtin_amdgcn_readlane(at, row.seq);
+    } else {
+      const int seqs = a.dist ? min(a.num_seqs, scalar_load_i32(a.dist + 2)) : a.num_seqs;
+      if (index >= scalar_load_i32(a.pt.cu_q_lens + seqs)) return false;
+      row.tq = index;
+      row.seq = __builtin_amdgcn_readfirstlane(owner_of_token(a.pt.cu_q_lens, seqs, index));
+      row.fresh_tq = scalar_load_i32(a.pt.cu_q_lens + row.seq);
+      row.fresh_first = scalar_load_i32(a.pt.kv_lens + row.seq) - (scalar_load_i32(a.pt.cu_q_lens + row.seq + 1) - row.fresh_tq);
+      cu_kv = scalar_load_i32(cu_kv_lens + row.seq);
+    }
+    row.kv_len = row.fresh_first + (index - row.fresh_tq) + 1;
+    row.page0 = first_page(a, row.seq, cu_kv);
+    return row.fresh_first >= 0;
+  }
+  // (static-shape mode: the number of decode rows comes from the device; the grid's rows are all sequences of the call)
+  const int rows_now = scalar_load_i32(a.dist ? a.dist : a.pt.kv_lens);
+  row.seq = index;
+  row.kv_len = scalar_load_i32(a.pt.kv_lens + index);
+  row.tq = row.fresh_tq = scalar_load_i32(a.pt.cu_q_lens + index);
+  const int cu_kv = scalar_load_i32(cu_kv_lens + index);
+  if (index >= (a.dist ? min(a.num_rows, rows_now) : a.num_rows)) return false;
+  row.fresh_first = row.kv_len - 1;
+  row.page0 = first_page(a, index, cu_kv);
+  return row.kv_len > 0;
+}
 
 // One wave, one (row, kv head, group of 16 query heads), tokens [t_begin, t_end): unnormalised output rows, maxima, sums.
 template <int MT, bool FP8, Pages PG, bool CAP, bool HALF, int WAVES>
@@ -575,7 +633,6 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
                                                int t_begin, int t_end, f32x4_t (&acc)[MT][8], float (&m)[MT], float (&l)[MT],
                                                int lane) {
   const int kv_len = row.kv_len;
-  const int seq = __builtin_amdgcn_readfirstlane(row.seq);
   const int c = lane & 15, g = lane >> 4;
   const int nblk = (t_end - t_begin + kBlk - 1) / kBlk;
 
@@ -586,13 +643,38 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
   // Sequence metadata and page ids go through the scalar cache: nothing writes them while the
   // kernel runs, and a scalar load is not counted by vmcnt, so waiting for a page id never
   // drains the block prefetch issued just before it.
-  sv.pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (scalar_load_i32(a.pt.cu_kv_lens + seq) / a.pt.page_size)
-                                                  : (int64_t)seq * a.pt.pages_per_seq);
+  sv.pages = a.pt.page_indices + row.page0;
 
   const char* kh = a.kv.k_base + (int64_t)hk * a.kv.head_stride;
   const char* vh = a.kv.v_base + (int64_t)hk * a.kv.head_stride;
   sv.fresh_first = a.new_k ? row.fresh_first : kNoFresh;
   sv.fresh_row = row.fresh_tq * a.Hkv + hk;
+
+  // ---- software pipeline: two blocks are in flight or in use.  The piece's last block goes first: it may end the row, or reach
+  // into its new tokens, and takes an address per lane and row; the blocks behind it are full ones of the cache, so the
+  // loop has one kind of loads, stands once in the code for it, and its waits stay counted: with a choice of loads in the
+  // loop the compiler closes it with a block that has a way past them and drains the queue in front of every use.  A piece of two
+  // blocks asks for those two and no more.  16 rows of 32 k tokens x 8 heads 316 -> 304 us (7.06 TB/s), 8 rows of 64..512 on
+  // pages of 64 8.4 -> 7.2.
+  const int full = nblk - 1;  // blocks but the last
+  const int t_last = t_begin + full * kBlk;
+  auto page_of = [&](int tb) -> BlockPages {
+    BlockPages p = {};
+    if constexpr (PG != kLanes) p.lo = scalar_load_i32(sv.pages + __builtin_amdgcn_readfirstlane(page_slot_of(sv, tb)));
+    if constexpr (PG == kHalves) p.hi = scalar_load_i32(sv.pages + __builtin_amdgcn_readfirstlane(page_slot_of(sv, min(tb + 16, sv.last_tok))));
+    return p;
+  };
+  // (a chunk's query tokens as rows: its new tokens may reach over several blocks, a few at most)
+  int first = 0;
+  if (a.token_rows)
+    while (full - first > 0 && t_last - first * kBlk > sv.fresh_first) ++first;
+  const int n = full - first;  // full blocks of the cache
+  auto next_tok = [&](int b) { return t_begin + min(b, max(n - 1, 0)) * kBlk; };
+  const BlockPages pg_last = page_of(t_last);
+  BlockPages pg_next = page_of(next_tok(0));
+  NewToken<FP8, HALF> fresh;
+  fresh.on = a.new_k && t_end == kv_len;
+  if (fresh.on) fresh.load(a, sv, lane);
 
   // ---- Q^T operands: column c = query head (row0 + 16*mt + c) of this kv head ----
   const int tq = row.tq;
@@ -602,7 +684,7 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
   requantise_queries<MT, FP8>(a, qB);
 
   ScoreOpts so;
-  const float ks = a.k_scale ? a.k_scale[hk] : 1.0f;
+  const float ks = a.k_scale ? scalar_load_f32(a.k_scale + hk) : 1.0f;
   // the one query of a decode row sits at position kv_len - 1
   const float temp = xai_factor(kv_len - 1, a.sm.xai_len);
   const float scale = a.sm.sm_scale * ks * (a.sm.q_scale > 0.f ? a.sm.q_scale : 1.0f);
@@ -620,20 +702,6 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
     for (int j = 0; j < 8; ++j) acc[mt][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 
-  // ---- software pipeline: two blocks are in flight or in use.  The piece's last block goes first: it may end the row, or reach
-  // into its new tokens, and takes an address per lane and row; the blocks behind it are full ones of the cache, so the
-  // loop has one kind of loads, stands once in the code for it, and its waits stay counted: with a choice of loads in the
-  // loop the compiler closes it with a block that has a way past them and drains the queue in front of every use.  A piece of two
-  // blocks asks for those two and no more.  16 rows of 32 k tokens x 8 heads 316 -> 304 us (7.06 TB/s), 8 rows of 64..512 on
-  // pages of 64 8.4 -> 7.2.
-  const int full = nblk - 1;  // blocks but the last
-  const int t_last = t_begin + full * kBlk;
-  auto page_of = [&](int tb) -> BlockPages {
-    BlockPages p = {};
-    if constexpr (PG != kLanes) p.lo = scalar_load_i32(sv.pages + __builtin_amdgcn_readfirstlane(page_slot_of(sv, tb)));
-    if constexpr (PG == kHalves) p.hi = scalar_load_i32(sv.pages + __builtin_amdgcn_readfirstlane(page_slot_of(sv, min(tb + 16, sv.last_tok))));
-    return p;
-  };
   // Pages smaller than half a block: the ids of the next kWinSmallPages pages wait in the wave's LDS window and
   // every lane looks its token rows up there; fetched from memory per block they were a dependent round
   // trip in front of every block's loads, behind which the loads already in flight had to drain (page size
@@ -656,40 +724,29 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
       }
     }
   };
-  NewToken<FP8, HALF> fresh;
-  fresh.on = a.new_k && t_end == kv_len;
-  if (fresh.on) fresh.load(a, sv, lane);
   KvRegs<FP8> ra, rb;
-  // (a chunk's query tokens as rows: its new tokens may reach over several blocks, a few at most)
-  int first = 0;
-  if (a.token_rows) {
-    while (full - first > 0 && t_last - first * kBlk > sv.fresh_first) ++first;
-    for (int b = 1; b <= first; ++b) {
-      const int tb = t_last - b * kBlk;
-      cover(tb);
-      load_block<FP8, PG, PG == kLanes, true, HALF>(rb, a, sv, kh, vh, tb, page_of(tb), c, g, win, win_first);
-      compute_block<MT, FP8, CAP, HALF>(rb, qB, acc, m, l, so, tb, g);
-    }
+  for (int b = 1; b <= first; ++b) {
+    const int tb = t_last - b * kBlk;
+    cover(tb);
+    load_block<FP8, PG, PG == kLanes, true, HALF>(rb, a, sv, kh, vh, tb, page_of(tb), c, g, win, win_first);
+    compute_block<MT, FP8, CAP, HALF>(rb, qB, acc, m, l, so, tb, g);
   }
-  const int n = full - first;  // full blocks of the cache
-  auto next_tok = [&](int b) { return t_begin + min(b, max(n - 1, 0)) * kBlk; };
-  BlockPages pg_next = page_of(next_tok(0));
   cover(t_last);
-  load_block<FP8, PG, PG == kLanes, true, HALF>(ra, a, sv, kh, vh, t_last, page_of(t_last), c, g, win, win_first);
-  cover(next_tok(0));
-  load_full_block<FP8, PG, HALF>(rb, a, sv, kh, vh, next_tok(0), pg_next, c, g, win, win_first);
+  load_block<FP8, PG, PG == kLanes, true, HALF>(ra, a, sv, kh, vh, t_last, pg_last, c, g, win, win_first);
   int in_a = t_last;  // first tokens of the blocks in ra, rb
-  int asked = 1;      // full blocks asked for; beyond n they are the last one again, for nobody
+  int asked = 1;      // full blocks asked for; beyond n they are the last one again and not wanted
+  cover(next_tok(0));
+  load_full_block<FP8, PG, HALF>(rb, a, sv, kh, vh, next_tok(0), pg_next, n > 0, c, g, win, win_first);
   while (asked < n) {
     pg_next = page_of(next_tok(asked));
     compute_block<MT, FP8, CAP, HALF>(ra, qB, acc, m, l, so, in_a, g);
     cover(next_tok(asked));
-    load_full_block<FP8, PG, HALF>(ra, a, sv, kh, vh, next_tok(asked), pg_next, c, g, win, win_first);
+    load_full_block<FP8, PG, HALF>(ra, a, sv, kh, vh, next_tok(asked), pg_next, true, c, g, win, win_first);
     in_a = next_tok(asked);
     pg_next = page_of(next_tok(asked + 1));
     compute_block<MT, FP8, CAP, HALF>(rb, qB, acc, m, l, so, next_tok(asked - 1), g);
     cover(next_tok(asked + 1));
-    load_full_block<FP8, PG, HALF>(rb, a, sv, kh, vh, next_tok(asked + 1), pg_next, c, g, win, win_first);
+    load_full_block<FP8, PG, HALF>(rb, a, sv, kh, vh, next_tok(asked + 1), pg_next, asked + 1 < n, c, g, win, win_first);
     asked += 2;
   }
   compute_block<MT, FP8, CAP, HALF>(ra, qB, acc, m, l, so, in_a, g);
@@ -698,37 +755,6 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const RowRef
     const int slot = __builtin_amdgcn_readfirstlane(page_slot_of(sv, sv.last_tok));
     fresh.store(a.kv, kh, vh, scalar_load_i32(sv.pages + slot), sv.last_tok - slot * sv.page_size, lane);
   }
-}
-
-__device__ __forceinline__ int owner_of_token(const int32_t* cu_q_lens, int num_seqs, int tok) {
-  int lo = 0, hi = num_seqs;  // last i with cu_q_lens[i] <= tok (zero-length sequences are skipped)
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (cu_q_lens[mid] <= tok) lo = mid; else hi = mid;
-  }
-  return lo;
-}
-
-// Row `index` of the fixed plan: decode row `index`, or (token_rows) query token `index` of whatever sequence owns it.
-// false: nothing there.
-__device__ __forceinline__ bool fixed_row(const DecodeArgs& a, int index, RowRef& row) {
-  if (a.token_rows) {
-    const int seqs = a.dist ? min(a.num_seqs, scalar_load_i32(a.dist + 2)) : a.num_seqs;
-    if (index >= scalar_load_i32(a.pt.cu_q_lens + seqs)) return false;
-    row.tq = index;
-    row.seq = __builtin_amdgcn_readfirstlane(owner_of_token(a.pt.cu_q_lens, seqs, index));
-    row.fresh_tq = scalar_load_i32(a.pt.cu_q_lens + row.seq);
-    row.fresh_first = scalar_load_i32(a.pt.kv_lens + row.seq) - (scalar_load_i32(a.pt.cu_q_lens + row.seq + 1) - row.fresh_tq);
-    row.kv_len = row.fresh_first + (index - row.fresh_tq) + 1;
-    return row.fresh_first >= 0;
-  }
-  // (static-shape mode: the number of decode rows comes from the device)
-  if (index >= (a.dist ? min(a.num_rows, scalar_load_i32(a.dist)) : a.num_rows)) return false;
-  row.seq = index;
-  row.kv_len = scalar_load_i32(a.pt.kv_lens + index);
-  row.tq = row.fresh_tq = scalar_load_i32(a.pt.cu_q_lens + index);
-  row.fresh_first = row.kv_len - 1;
-  return row.kv_len > 0;
 }
 
 // ---- fixed split plan: grid = (max_splits * rows, 1, head groups * row groups), splits fastest (rows do
@@ -760,15 +786,16 @@ __global__ __launch_bounds__(256, 2) void rpa_decode_splitkv_kernel(const Decode
   dest.base = ((int64_t)index * a.max_splits + split) * a.Hq;
   f32x4_t acc[MT][8];
   float m[MT], l[MT];
+  const float vs = a.v_scale ? scalar_load_f32(a.v_scale + hk) : 1.0f;
   decode_segment<MT, FP8, PG, CAP, HALF, 4>(a, row, hk, rg, t_lo, t_begin, t_end, acc, m, l, lane);
-  write_rows<MT>(a, acc, m, l, row.tq, hk, rg * 16 * MT, dest, lane & 15, lane >> 4);
+  write_rows<MT>(a, acc, m, l, row.tq, hk, rg * 16 * MT, dest, vs, lane & 15, lane >> 4);
 }
 
-// ---- short rows: grid = (rows, 1, kv heads * row groups); one workgroup of kRowWaves waves deals a row's blocks out among
-// them and merges their partial rows in LDS.  Bound by latency: the split kernel and its merge are two launches, each about
-// 4 us from its start to its first useful load; here the merge is two barriers and 8 KB of LDS per 2 query heads.  8 waves:
-// the registers allow two per SIMD, and a row of 255 tokens is then one 32-token block each.  A few rows of up to 255
-// tokens: 10.2 -> 7.5 us.
+// ---- rows by workgroups: grid = (pieces * rows, 1, kv heads * row groups); one workgroup of kRowWaves waves deals the blocks of a
+// row, or of one of max_splits pieces of it, out among them and merges their partial rows in LDS: two barriers and 8 KB per 2 query
+// heads.  8 waves: the registers allow two per SIMD.  Whole short rows are bound by latency (the split kernel and its merge are
+// two launches; a few rows of up to 255 tokens 10.2 -> 7.5 us), pieces that fill the chip by what a CU draws:
+// 32 rows of 800..1000 tokens x 8 heads, whole, 31.5 -> 24.1 us.  Which rows come here: row_plan().
 template <bool FP8, Pages PG, bool CAP, bool HALF = false>
 __global__ __launch_bounds__(kRowWaves * 64, 2) void rpa_decode_row_kernel(const DecodeArgs a) {
   extern __shared__ float row_parts[];  // [wave][query head of the group][kRowPitch]
@@ -776,18 +803,23 @@ __global__ __launch_bounds__(kRowWaves * 64, 2) void rpa_decode_row_kernel(const
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hk = (int)blockIdx.z % a.Hkv, rg = (int)blockIdx.z / a.Hkv;
+  const int nsp = max(a.max_splits, 1), index = (int)(blockIdx.x / (unsigned)nsp), split = (int)blockIdx.x - index * nsp;
   RowRef row;
-  if (!fixed_row(a, (int)blockIdx.x, row)) return;
+  if (!fixed_row(a, index, row)) return;
   const int t_lo = (a.sm.window > 0) ? max(0, row.kv_len - a.sm.window) : 0;
-  const int t0 = t_lo & ~(kBlk - 1);
-  const int piece = ((row.kv_len - t0 + kBlk - 1) / kBlk + kRowWaves - 1) / kRowWaves * kBlk;
-  const int used = (row.kv_len - t0 + piece - 1) / piece;  // waves with work
+  const int t0 = (t_lo & ~(kBlk - 1)) + split * a.chunk;
+  // (the last split runs to kv_len even if the host's length bound was too small)
+  const int t1 = split == nsp - 1 ? row.kv_len : min(row.kv_len, t0 + a.chunk);
+  if (t0 >= t1) return;
+  const int piece = ((t1 - t0 + kBlk - 1) / kBlk + kRowWaves - 1) / kRowWaves * kBlk;
+  const int used = (t1 - t0 + piece - 1) / piece;  // waves with work
   const int heads = min(16, a.G - rg * 16);
+  const float vs = a.v_scale ? scalar_load_f32(a.v_scale + hk) : 1.0f;
   f32x4_t acc[1][8];
   float m[1], l[1];
   if (wave < used) {
     const int t_begin = t0 + wave * piece;
-    decode_segment<1, FP8, PG, CAP, HALF, kRowWaves>(a, row, hk, rg, t_lo, t_begin, min(row.kv_len, t_begin + piece),
+    decode_segment<1, FP8, PG, CAP, HALF, kRowWaves>(a, row, hk, rg, t_lo, t_begin, min(t1, t_begin + piece),
                                                                acc, m, l, lane);
     float lt = l[0];
     lt += __shfl_xor(lt, 16);
@@ -812,7 +844,6 @@ __global__ __launch_bounds__(kRowWaves * 64, 2) void rpa_decode_row_kernel(const
     }
   }
   __syncthreads();
-  const float vs = a.v_scale ? a.v_scale[hk] : 1.0f;
   for (int at = (int)threadIdx.x; at < heads * 64; at += kRowWaves * 64) {
     const int h = at >> 6, d = (at & 63) * 2;  // two dims of one query head
     const int head = hk * a.G + rg * 16 + h;
@@ -824,6 +855,12 @@ __global__ __launch_bounds__(kRowWaves * 64, 2) void rpa_decode_row_kernel(const
       const float* from = row_parts + (w * heads + h) * kRowPitch + d;
       x += from[0];
       y += from[1];
+    }
+    if (nsp > 1) {
+      const int64_t slot = ((int64_t)index * nsp + split) * a.Hq + head;
+      *reinterpret_cast<f32x2_t*>(a.ws_o + slot * 128 + d) = f32x2_t{x * vs, y * vs};
+      if (d == 0) *reinterpret_cast<f32x2_t*>(a.ws_ml + slot * 2) = f32x2_t{top, den};
+      continue;
     }
     const float inv = a.sm.sink ? vs * sink_inverse(top, den, sink_logit(a.sm.sink, a.sm.round_logits, head)) : vs / den;
     if (d < a.q_dim)
@@ -955,6 +992,7 @@ struct Piece {
   int t_first;  // first token of the piece (a multiple of 32 past the window's first block)
   int nblk;     // its 32-token blocks
   bool final_rows;
+  float ks, vs;  // scales of the kv head's keys and values (asked for with the piece, a block before it begins)
 };
 
 // The wave that arrives last at a cut unit merges it.  A unit (row, kv head, group of 16 query
@@ -1137,6 +1175,9 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
     p.t_first = (p.t_lo & ~(kBlk - 1)) + blk * kBlk;
     p.nblk = take;
     p.final_rows = (blk == 0) && (take == r.nb);
+    const int hk = min(p.hk, a.Hkv - 1);
+    p.ks = a.k_scale ? scalar_load_f32(a.k_scale + hk) : 1.0f;
+    p.vs = a.v_scale ? scalar_load_f32(a.v_scale + hk) : 1.0f;
     return p;
   };
   auto view_of = [&](const RowMeta& r, int hk) {
@@ -1169,9 +1210,9 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
   __shared__ int32_t lds_windows[4][2][kWin];  // [wave][current / next piece][entry]
   PageWindow win = {lds_windows[wave][0], 0};
   PageWindow nwin = {lds_windows[wave][1], 0};
-  auto request = [&](KvRegs<FP8>& r, const SeqView& v, int of_head, const PageWindow& pwn, int tb) __attribute__((always_inline)) {
+  auto request = [&](KvRegs<FP8>& r, const SeqView& v, int of_head, const PageWindow& pwn, int tb, bool wanted) __attribute__((always_inline)) {
     load_cached_block<FP8, PG, HALF>(r, a, v, a.kv.k_base + (int64_t)of_head * a.kv.head_stride, a.kv.v_base + (int64_t)of_head * a.kv.head_stride,
-                                     tb, pages_in(pwn, v, tb), c, g, pwn.lds, pwn.first);
+                                     tb, pages_in(pwn, v, tb), wanted, c, g, pwn.lds, pwn.first);
   };
   request_window<kWin>(a, cur.row, win, slot_of_tok(cur.t_first), page_shift, lane);
   u32x4_t qB[MT][4];
@@ -1195,9 +1236,8 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
     hk = min(cur.hk, a.Hkv - 1);
     sv = view_of(cur.row, hk);
     requantise_queries<MT, FP8>(a, qB);
-    const float ks = a.k_scale ? a.k_scale[hk] : 1.0f;
     const float temp = xai_factor(cur.row.kv_len - 1, a.sm.xai_len);  // the one query sits at kv_len - 1
-    const float scale = a.sm.sm_scale * ks * (a.sm.q_scale > 0.f ? a.sm.q_scale : 1.0f);
+    const float scale = a.sm.sm_scale * cur.ks * (a.sm.q_scale > 0.f ? a.sm.q_scale : 1.0f);
     so.scale2 = scale * kLog2e * temp;
     so.general.set(a.sm, scale, temp);
     so.mask2 = fmaxf(a.sm.mask_value * kLog2e, -3.0e38f);
@@ -1252,13 +1292,13 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
     // The next piece's window was requested at block resolve_at, in front of that block's
     // prefetch.  Two blocks later a wait for younger loads has passed; earlier it has not.
     if (last && has_next && i <= resolve_at + 1) wait_all_loads();
-    // The block to request now: the next one of this piece, the first one of the next piece, or (nothing left) this block
-    // again.  What differs is chosen in scalars and the loads stand once, in no branch: with a way around them in the code the
+    // The block to request now: the next one of this piece, the first one of the next piece, or (nothing left) one that is not
+    // wanted.  What differs is chosen in scalars and the loads stand once, in no branch: with a way around them in the code the
     // compiler waits for all loads where it should wait for the block in use alone.
     {
       const bool ahead = last && has_next;
       const int fhk = ahead ? min(nxt.hk, a.Hkv - 1) : hk;
-      request(fill, view_of(ahead ? nxt.row : cur.row, fhk), fhk, ahead ? nwin : win, ahead ? nxt.t_first : last ? tb : tb + kBlk);
+      request(fill, view_of(ahead ? nxt.row : cur.row, fhk), fhk, ahead ? nwin : win, ahead ? nxt.t_first : last ? tb : tb + kBlk, ahead || !last);
     }
     if (PG != kLanes && rare(fresh.on && last)) fresh.put(use, sv.last_tok - tb, c, g);
     compute_block<MT, FP8, CAP, HALF, PG == kBlocks>(use, qB, acc, m, l, so, tb, g);
@@ -1275,7 +1315,7 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
       dest.final_rows = cur.final_rows;
       dest.by_head = false;
       dest.base = ((int64_t)w * 2 + (x == x_first ? 0 : 1)) * 16;
-      write_rows<MT, MERGE>(a, acc, m, l, cur.row.tq, hk, cur.rg * 16 * MT, dest, c, g);
+      write_rows<MT, MERGE>(a, acc, m, l, cur.row.tq, hk, cur.rg * 16 * MT, dest, cur.vs, c, g);
       if (MERGE && !cur.final_rows) {
         // the unit's first block in the linear order, and the workgroups that share the unit
         const int64_t first_block = (int64_t)x - (cur.t_first - (cur.t_lo & ~(kBlk - 1))) / kBlk;
@@ -1325,7 +1365,7 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
     return true;
   };
   begin_piece();
-  request(ra, sv, hk, win, cur.t_first);
+  request(ra, sv, hk, win, cur.t_first, true);
   while (step(ra, rb) && step(rb, ra)) {
   }
   if (MERGE && (pm_first.n | pm_last.n)) {
@@ -1506,10 +1546,11 @@ __global__ __launch_bounds__(merge_threads(SIZE)) void rpa_combine_balanced_kern
   const int nw = a.waves_per_wg;
   const int row_groups = (a.G + 15) / 16;
   const int units = ((a.Hkv + nw - 1) / nw) * row_groups;
-  const int nb = seq_blocks(a.pt.kv_lens[seq], a.sm.window);
+  // (what the merge has to know in one round trip)
+  const int kv_len = scalar_load_i32(a.pt.kv_lens + seq), before = scalar_load_i32(a.cu_blocks + seq);
+  const int total = scalar_load_i32(a.cu_blocks + a.num_rows) * units, tq = scalar_load_i32(a.pt.cu_q_lens + seq);
+  const int nb = seq_blocks(kv_len, a.sm.window);
   if (nb == 0) return;
-  const int before = scalar_load_i32(a.cu_blocks + seq);
-  const int total = scalar_load_i32(a.cu_blocks + a.num_rows) * units;
   const int pw = blocks_per_wave(a, total);
   const int hk = head / a.G, row = head - hk * a.G;
   const int unit = (hk / nw) * row_groups + row / 16;
@@ -1525,7 +1566,7 @@ __global__ __launch_bounds__(merge_threads(SIZE)) void rpa_combine_balanced_kern
     const int part = ((int64_t)wj * pw >= first_block) ? 0 : 1;
     return (((int64_t)wj * nw + wv) * 2 + part) * 16 + r16;
   };
-  merge_rows<128, SIZE>(a, scalar_load_i32(a.pt.cu_q_lens + seq), head, n, lane, slot_of);
+  merge_rows<128, SIZE>(a, tq, head, n, lane, slot_of);
 }
 
 // ---- head_dim 256 ---------------------------------------------------------------------------
@@ -1883,7 +1924,7 @@ void launch_decode_variant(const DecodeArgs& a, dim3 grid, dim3 block, hipStream
   const bool one_round = (int64_t)grid.x * grid.z * (block.x / 64) <= 2048;
   const int forced = tuning().decode_lds_kb;
   const unsigned lds = forced >= 0 ? (unsigned)forced << 10 : !one_round ? 0u : block.x >= 256 ? 84u << 10 : block.x >= 128 ? 54u << 10 : 34u << 10;
-  if (a.whole_rows) {
+  if (a.group_rows) {
     // (one workgroup per CU, too)
     const unsigned parts = std::max(84u << 10, (unsigned)(kRowWaves * min(a.G, 16) * kRowPitch * sizeof(float)));
     if constexpr (!FP8) {
@@ -1955,12 +1996,10 @@ hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream) {
     }
     return hipGetLastError();
   }
-  if (a.whole_rows)
-    return launch_decode_mt(a, dim3((unsigned)a.num_rows, 1, (unsigned)(a.Hkv * row_groups)), dim3(kRowWaves * 64), stream);
   if ((int64_t)a.max_splits * a.num_rows > 0x7fffffffLL || (int64_t)a.Hq * a.num_rows > 0x7fffffffLL)
     return hipErrorInvalidValue;
-  dim3 grid((unsigned)max(a.max_splits, 1) * (unsigned)a.num_rows, 1, head_groups * row_groups);
-  dim3 block(nw * 64);
+  dim3 grid((unsigned)max(a.max_splits, 1) * (unsigned)a.num_rows, 1, (a.group_rows ? a.Hkv : head_groups) * row_groups);
+  dim3 block(a.group_rows ? kRowWaves * 64 : nw * 64);
   hipError_t e = launch_decode_mt(a, grid, block, stream);
   if (e != hipSuccess) return e;
   if (a.max_splits > 1) {

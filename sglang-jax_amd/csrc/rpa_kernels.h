@@ -83,7 +83,7 @@ struct DecodeArgs {
   const char* new_v;
   int32_t token_rows;    // fixed plan: rows are the query tokens of sequences [0, num_seqs), of any length
   int32_t num_seqs;      // token_rows: sequences (with dist: a bound on dist[2])
-  int32_t whole_rows;    // fixed plan: one workgroup per (row, kv head), merged in LDS (rpa_decode_row_kernel)
+  int32_t group_rows;    // fixed plan: one workgroup per (row, kv head, piece), merged in LDS (rpa_decode_row_kernel)
 };
 
 // New tokens on their way into the cache.

@@ -18,6 +18,7 @@ struct Tuning {
   int decode_merge_in_kernel = 0;   // RPA_DECODE_MERGE_IN_KERNEL 1: one launch, merge behind arrival counters
   int decode_lds_kb = -1;           // RPA_DECODE_LDS_KB          -1: by the workgroup's waves; n: unused LDS per workgroup, KiB
   int decode_row_kb = -1;           // RPA_DECODE_ROW_KB          -1: 128; KiB of a row's kv head up to which one workgroup takes it
+  int decode_row_pieces = -1;       // RPA_DECODE_ROW_PIECES      -1: by the launch; n: workgroups that share a row's kv head
   // ---- prefill (rpa_prefill.hip, rpa_prefill_pipe.hip)
   int mask_bits = 1;                // RPA_MASK_BITS              0: kernels read the caller's i32 mask words
   int prefill_rows256 = 0;          // RPA_PREFILL_ROWS256        1: 256-wide chunks through the row kernel

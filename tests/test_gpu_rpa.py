@@ -1986,3 +1986,56 @@ def test_decode_rows_by_halves_of_a_block(pkg, wl, gpu, monkeypatch, P, fp8, row
             page = int(b.page_indices[int(b.cu_kv_lens[i]) // P + (kv - 1) // P])
             expect[page, (kv - 1) % P] = full[page, (kv - 1) % P]
         assert torch.equal(got, expect)
+
+
+@pytest.mark.parametrize("Hq,Hkv,P,fp8,window", [(16, 8, 64, False, None), (40, 2, 16, False, 150), (12, 1, 24, True, None), (16, 2, 64, True, 333)])
+def test_rows_by_workgroups_in_pieces(pkg, wl, gpu, monkeypatch, Hq, Hkv, P, fp8, window):
+    """Pieces of a row by workgroups of eight waves, any number of them: rows shorter than a piece, pieces of fewer blocks than waves, ends
+    inside a block, a sink; the new token brought along.  Against the oracle and against pieces of single waves."""
+    kv_lens = [1, 31, 33, 256, 257, 300, 511, 513, 1000]
+    say(f"row pieces {Hq}/{Hkv} P={P} fp8={fp8} window={window}")
+    b = wl.make_batch("row_pieces", [1] * len(kv_lens), kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=17,
+                      kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16, sliding_window=window)
+    sink = torch.from_numpy(np.random.RandomState(5).randn(Hq).astype(np.float32))
+    want, tol = oracle_out(b, attention_sink=sink).float(), FP8_TOL if fp8 else BF16_TOL
+    monkeypatch.setenv("RPA_DECODE_ROW_KB", "0")
+    single = gpu_out(pkg, b, gpu, attention_sink=sink).float()
+    assert_parity(single, want, **tol)
+    monkeypatch.delenv("RPA_DECODE_ROW_KB")
+    for pieces in ("1", "2", "5", "32"):
+        monkeypatch.setenv("RPA_DECODE_ROW_PIECES", pieces)
+        got = gpu_out(pkg, b, gpu, attention_sink=sink).float()
+        assert_parity(got, want, **tol)
+        torch.testing.assert_close(got, single, rtol=1e-2, atol=4e-3)
+
+
+@pytest.mark.parametrize("rows,Hkv,lo,hi,fp8", [(4, 8, 1800, 2000, False), (32, 8, 900, 1000, False), (8, 8, 3600, 4000, True)])
+def test_even_rows_fill_the_chip(pkg, wl, gpu, monkeypatch, rows, Hkv, lo, hi, fp8):
+    """Even rows in pieces that are one round of the CUs run by workgroups, in the workspace that rpa_workspace_bytes() names, and in
+    less of it, where the plan that stood there before still runs; a call that brings too little for that one is refused."""
+    kv_lens = [lo + (i * 37) % (hi - lo) for i in range(rows - 1)] + [hi]
+    say(f"even rows {rows} x {Hkv} x {lo}..{hi} fp8={fp8}")
+    b = wl.make_batch("even", [1] * rows, kv_lens, num_q_heads=2 * Hkv, num_kv_heads=Hkv, head_dim=128, page_size=64, seed=18,
+                      kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+    want, tol = oracle_out(b).float(), FP8_TOL if fp8 else BF16_TOL
+    g = b.to(gpu)
+    def make():
+        return sys.modules["sglang_jax_amd.ragged_paged_attention"].RpaCall(
+            g.q, g.kv_cache, None, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, num_seqs=rows, decode_end=rows, sm_scale=b.sm_scale,
+            max_kv_len=hi, max_q_len=1, sum_decode_kv_len=sum(kv_lens), own_workspace=True, k_scale=g.k_scale, v_scale=g.v_scale)
+    call = make()
+    assert "rpa_decode_row_kernel" in sys.modules["sglang_jax_amd._lib"].describe_plan(call.params)
+    monkeypatch.setenv("RPA_DECODE_ROW_KB", "0")
+    other = make()
+    monkeypatch.delenv("RPA_DECODE_ROW_KB")
+    least = min(call.params.workspace_bytes, other.params.workspace_bytes)
+    for c, given in ((call, call.params.workspace_bytes), (other, other.params.workspace_bytes), (other, least)):
+        c.params.workspace_bytes = given
+        c.out.fill_(math.nan)
+        c.attention()
+        torch.cuda.synchronize()
+        assert_parity(c.out.cpu().float(), want, **tol)
+    if least:
+        other.params.workspace_bytes = least - 1
+        with pytest.raises(ValueError, match="workspace"):
+            other.attention()
