@@ -48,6 +48,17 @@ __device__ __forceinline__ f32x16_t mfma32(u32x4_t a, u32x4_t b, f32x16_t c) {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// The maximum over a pair of lanes 32 (16) apart, through a lane swap: no round trip through LDS.
+__device__ __forceinline__ float swap_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+__device__ __forceinline__ float swap16_max(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // cap * tanh(x / cap) = cap - 2 cap / (e^(2x/cap) + 1), written so that +-inf arguments give +-cap: one
 // multiply, v_exp_f32, one add, v_rcp_f32 (1 ulp; an IEEE division here is ten instructions per score), one fma.
 __device__ __forceinline__ float soft_cap_f(float x, float cap, float inv_cap) {

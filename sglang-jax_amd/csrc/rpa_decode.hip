@@ -397,39 +397,63 @@ __device__ __forceinline__ void v_operands(const KvRegs<FP8>& r, u32x4_t (&vA)[8
   }
 }
 
-template <int MT, bool FP8, bool CAP, bool HALF = false, bool LOOPS = false>
+__device__ __forceinline__ float max8(const float (&x)[8]) {
+  return fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+}
+
+struct Nothing {
+  __device__ __forceinline__ void operator()() const {}
+};
+
+// `taken` runs when the block's registers have been read (FP8: its operands are in registers of their own): the place to ask for
+// another block in the same registers.
+template <int MT, bool FP8, bool CAP, bool HALF = false, bool LOOPS = false, class Taken = Nothing>
 __device__ __forceinline__ void compute_block(const KvRegs<FP8>& r, const u32x4_t (&qB)[MT][4],
                                               f32x4_t (&acc)[MT][8], float (&m)[MT], float (&l)[MT],
-                                              const ScoreOpts& so, int tb, int g) {
+                                              const ScoreOpts& so, int tb, int g, const Taken& taken = Taken()) {
+  constexpr bool kEarly = !std::is_same_v<Taken, Nothing>;
   u32x4_t kA[2][4];
   k_operands<FP8, HALF>(r, kA);
-  u32x4_t vA[8];
-  v_operands<FP8>(r, vA);
-  const bool need_mask = (tb + kBlk > so.kv_len) || (tb < so.t_lo);
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    f32x4_t s[2];
+  f32x4_t s_of[kEarly ? MT : 1][2];
+  auto scores = [&](int mt, f32x4_t (&s)[2]) __attribute__((always_inline)) {
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       s[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int st = 0; st < (HALF ? 2 : 4); ++st) s[b] = mfma16(kA[b][st], qB[mt][st], s[b]);
     }
+  };
+  if constexpr (kEarly) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) scores(mt, s_of[mt]);
+  }
+  u32x4_t vA[8];
+  v_operands<FP8>(r, vA);
+  if constexpr (kEarly) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(vA[j]));  // made here, not where they are used
+    taken();
+  }
+  const bool need_mask = (tb + kBlk > so.kv_len) || (tb < so.t_lo);
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    f32x4_t(&s)[2] = s_of[kEarly ? mt : 0];
+    if constexpr (!kEarly) scores(mt, s);
     float x[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = CAP ? s[i >> 2][i & 3] : s[i >> 2][i & 3] * so.scale2;
     if constexpr (CAP) so.general.apply<LOOPS>(x);
+    // (the maximum of unmasked scores in front of the branch: behind it every one of them would be canonicalised first)
+    float mx = max8(x);
     if (need_mask) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int tok = tb + tok_slot(g, i);
         if (tok >= so.kv_len || tok < so.t_lo) x[i] = so.mask2;
       }
+      mx = max8(x);
     }
-    float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
-                     fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    mx = swap_max(swap16_max(mx));
     const float m_new = fmaxf(m[mt], mx);
     const float alpha = fast_exp2(m[mt] - m_new);
     float p[8];
@@ -487,7 +511,7 @@ __device__ __forceinline__ void load_queries(const DecodeArgs& a, int tq, int hk
     const uint16_t* qp = a.q + ((int64_t)tq * a.Hq + (int64_t)hk * a.G + row) * a.q_dim;
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
-      const int d0 = FP8 ? (g * 32 + st * 8) : (st * 32 + g * 8);
+      const int d0 = FP8 ? g * 32 + st * 8 : st * 32 + g * 8;
       qB[mt][st] = ld_query(qp, row < a.G ? d0 : a.q_dim, a.q_dim);
     }
   }
@@ -1086,6 +1110,11 @@ __device__ __forceinline__ void merge_unit(const DecodeArgs& a, const PendingMer
 // are requested right behind that first block.  A piece border costs no round trip to memory,
 // and neither does a block: under load a small dependent load waits behind megabytes of queued
 // KV traffic (10 us and more), so there are none after the first block.
+// e4m3: a block is half the bytes of a bf16 one and takes as long to work on, so one block ahead leaves the queue short (a block
+// per 1.36 us and wave where the compute alone takes 1.0).  Its operands are converted into registers of their own first thing, and
+// the block after next goes into the registers that this empties, across the borders of pieces: 64 rows of 1000..8000 tokens x 8
+// heads on 16-token pages 124 -> 114 us, 128 rows of 1024..8192 x 8 heads on 64-token pages 204.7 -> 202.3 (the same without its compute: 2 % less).
+// bf16 is bound by memory either way, and so has one block ahead.
 // New tokens (a.new_k) are taken where pages hold whole blocks or halves.  (bf16: registers of one wave per SIMD, which is what is resident.)
 template <int MT, bool FP8, Pages PG, bool CAP, bool MERGE, bool HALF>
 __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
@@ -1215,7 +1244,8 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
                                      tb, pages_in(pwn, v, tb), wanted, c, g, pwn.lds, pwn.first);
   };
   request_window<kWin>(a, cur.row, win, slot_of_tok(cur.t_first), page_shift, lane);
-  u32x4_t qB[MT][4];
+  constexpr bool kTwo = FP8 && PG != kLanes;  // two blocks ahead
+  u32x4_t qB[MT][4], q_next[MT][4];
   load_queries<MT, FP8>(a, cur.row.tq, min(cur.hk, a.Hkv - 1), cur.rg * 16 * MT, c, g, qB);
   wait_all_loads();  // the window (and the queries behind it)
 
@@ -1261,6 +1291,8 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
     i = 0;
   };
   PendingMerge pm_first = {}, pm_last = {};
+  bool done = false;
+  bool late = false;  // (two ahead) the piece's first block has not been asked for: the piece before was one block
 
   // One block: the one behind it is requested, then it is worked on; a piece's rows are written behind its last one.
   // false: nothing is left.
@@ -1268,7 +1300,7 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
     const int tb = cur.t_first + i * kBlk;
     const bool last = (i + 1 == cur.nblk);
     // resolved one block into the piece when it has more than one block, at once otherwise
-    const int resolve_at = (cur.nblk > 1) ? 1 : 0;
+    const int resolve_at = cur.nblk > (kTwo ? 2 : 1) ? 1 : 0;
     if (has_next && i == resolve_at) {
       RowMeta nrow = cur.row;
       int nunit = cur_unit + 1;
@@ -1283,25 +1315,48 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
       const int x_next = x + cur.nblk;
       nxt = make_piece(nrow, nunit, 0, min(nrow.nb, x_end - x_next));
       request_window<kWin>(a, nrow, nwin, slot_of_tok(nxt.t_first), page_shift, lane);
+      if constexpr (kTwo) load_queries<MT, FP8>(a, nxt.row.tq, min(nxt.hk, a.Hkv - 1), nxt.rg * 16 * MT, c, g, q_next);
     }
-    // the window moves on when the next block's last page lies beyond it
-    if (!last && slot_of_tok(tb + kBlk + (PG == kBlocks ? 0 : kBlk - 1)) - win.first >= kWin) {
-      request_window<kWin>(a, cur.row, win, slot_of_tok(tb + kBlk), page_shift, lane);
-      wait_all_loads();
+    if constexpr (kTwo) {
+      if (rare(late)) {
+        wait_all_loads();
+        request(use, sv, hk, win, tb, true);
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), by a name that the compiler counts by
+        late = false;
+      }
+      if (rare(fresh.on && last)) fresh.put(use, sv.last_tok - tb, c, g);
+      compute_block<MT, FP8, CAP, HALF, PG == kBlocks>(use, qB, acc, m, l, so, tb, g, [&]() __attribute__((always_inline)) {
+        const int beyond = i + 2 - cur.nblk;  // block of the next piece, when not negative
+        const bool here = beyond < 0, there = has_next && beyond >= 0 && beyond < nxt.nblk;
+        const int t_ask = min(tb + 2 * kBlk, cur.t_first + (cur.nblk - 1) * kBlk);
+        if (here && slot_of_tok(t_ask + (PG == kBlocks ? 0 : kBlk - 1)) - win.first >= kWin) {
+          request_window<kWin>(a, cur.row, win, slot_of_tok(t_ask), page_shift, lane);
+          wait_all_loads();
+        }
+        if (there && i <= resolve_at + 1) wait_all_loads();
+        const int fhk = there ? min(nxt.hk, a.Hkv - 1) : hk;
+        request(use, view_of(there ? nxt.row : cur.row, fhk), fhk, there ? nwin : win, there ? nxt.t_first + beyond * kBlk : t_ask, here || there);
+      });
+    } else {
+      // the window moves on when the next block's last page lies beyond it
+      if (!last && slot_of_tok(tb + kBlk + (PG == kBlocks ? 0 : kBlk - 1)) - win.first >= kWin) {
+        request_window<kWin>(a, cur.row, win, slot_of_tok(tb + kBlk), page_shift, lane);
+        wait_all_loads();
+      }
+      // The next piece's window was requested at block resolve_at, in front of that block's
+      // prefetch.  Two blocks later a wait for younger loads has passed; earlier it has not.
+      if (last && has_next && i <= resolve_at + 1) wait_all_loads();
+      // The block to request now: the next one of this piece, the first one of the next piece, or (nothing left) one that is not
+      // wanted.  What differs is chosen in scalars and the loads stand once, in no branch: with a way around them in the code the
+      // compiler waits for all loads where it should wait for the block in use alone.
+      {
+        const bool ahead = last && has_next;
+        const int fhk = ahead ? min(nxt.hk, a.Hkv - 1) : hk;
+        request(fill, view_of(ahead ? nxt.row : cur.row, fhk), fhk, ahead ? nwin : win, ahead ? nxt.t_first : last ? tb : tb + kBlk, ahead || !last);
+      }
+      if (PG != kLanes && rare(fresh.on && last)) fresh.put(use, sv.last_tok - tb, c, g);
+      compute_block<MT, FP8, CAP, HALF, PG == kBlocks>(use, qB, acc, m, l, so, tb, g);
     }
-    // The next piece's window was requested at block resolve_at, in front of that block's
-    // prefetch.  Two blocks later a wait for younger loads has passed; earlier it has not.
-    if (last && has_next && i <= resolve_at + 1) wait_all_loads();
-    // The block to request now: the next one of this piece, the first one of the next piece, or (nothing left) one that is not
-    // wanted.  What differs is chosen in scalars and the loads stand once, in no branch: with a way around them in the code the
-    // compiler waits for all loads where it should wait for the block in use alone.
-    {
-      const bool ahead = last && has_next;
-      const int fhk = ahead ? min(nxt.hk, a.Hkv - 1) : hk;
-      request(fill, view_of(ahead ? nxt.row : cur.row, fhk), fhk, ahead ? nwin : win, ahead ? nxt.t_first : last ? tb : tb + kBlk, ahead || !last);
-    }
-    if (PG != kLanes && rare(fresh.on && last)) fresh.put(use, sv.last_tok - tb, c, g);
-    compute_block<MT, FP8, CAP, HALF, PG == kBlocks>(use, qB, acc, m, l, so, tb, g);
     ++i;
     if (!last) return true;
 
@@ -1350,9 +1405,13 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
         }
       }
     }
-    if (!has_next) return false;
+    if (!has_next) {
+      done = true;
+      return false;
+    }
     x += cur.nblk;
     cur_unit = next_row ? 0 : cur_unit + 1;
+    late = cur.nblk == 1;
     cur = nxt;
     {  // the two LDS windows trade places
       const PageWindow t = win;
@@ -1360,13 +1419,31 @@ __device__ __forceinline__ void decode_balanced(const DecodeArgs& a_in) {
       nwin = t;
     }
     // the queries queue up right behind the piece's first block, which is already on its way
-    load_queries<MT, FP8>(a, cur.row.tq, min(cur.hk, a.Hkv - 1), cur.rg * 16 * MT, c, g, qB);
+    if constexpr (kTwo) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int st = 0; st < 4; ++st) qB[mt][st] = q_next[mt][st];
+    } else {
+      load_queries<MT, FP8>(a, cur.row.tq, min(cur.hk, a.Hkv - 1), cur.rg * 16 * MT, c, g, qB);
+    }
     begin_piece();
     return true;
   };
   begin_piece();
   request(ra, sv, hk, win, cur.t_first, true);
-  while (step(ra, rb) && step(rb, ra)) {
+  if constexpr (kTwo) __builtin_amdgcn_sched_barrier(0);  // (the waits in the loop count on this order)
+  if constexpr (kTwo) request(rb, sv, hk, win, min(cur.t_first + kBlk, cur.t_first + (cur.nblk - 1) * kBlk), cur.nblk > 1);
+  if constexpr (kTwo) {
+    // no way out between the two: the compiler would see one from there back to the top, with the first step's loads as the
+    // youngest in flight, and wait for all of them.  A step behind the last block works on one that is not wanted.
+    do {
+      step(ra, rb);
+      step(rb, ra);
+    } while (!done);
+  } else {
+    while (step(ra, rb) && step(rb, ra)) {
+    }
   }
   if (MERGE && (pm_first.n | pm_last.n)) {
     if (pm_first.n) merge_unit(a, pm_first, pw, wave, nw, a.generation, lane);
@@ -1636,7 +1713,7 @@ __global__ __launch_bounds__(64, FP8 ? 2 : 1) void rpa_rows256_kernel(const Deco
     for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
       for (int st = 0; st < 4; ++st) {
-        const int d0 = hf * 128 + (FP8 ? (g * 32 + st * 8) : (st * 32 + g * 8));
+        const int d0 = hf * 128 + (FP8 ? g * 32 + st * 8 : st * 32 + g * 8);
         qB[hf][st] = ld_query(qp, d0, a.q_dim);
         if (a.sm.q_scale > 0.f) qB[hf][st] = requantise_q(qB[hf][st], a.sm.q_scale, FP8);
       }
@@ -1754,9 +1831,7 @@ __global__ __launch_bounds__(64, FP8 ? 2 : 1) void rpa_rows256_kernel(const Deco
       if (mask_row && !dead) dead = mask_row[tok] < 1;
       if (dead) x[i] = mask2;
     }
-    float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float mx = swap_max(swap16_max(max8(x)));
     const float m_new = fmaxf(m, mx);
     const float alpha = fast_exp2(m - m_new);
     float p[8], ps = 0.f;

@@ -264,18 +264,6 @@ __device__ __forceinline__ void update_running_max(float mx, float& m, float& l,
   }
 }
 
-// xor-32 lane exchange of a maximum through v_permlane32_swap (no LDS round trip)
-__device__ __forceinline__ float swap_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
-// the same over lanes 16 apart
-__device__ __forceinline__ float swap16_max(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
 // Which tokens a query row may see.  mode 0: causal (token <= row position); mode 1: the
 // caller's mask row (>= 1 keeps), mode 2: everything; modes 1 and 2 still hide the tokens of a
 // partial last tile beyond kv_len.  The sliding window applies on top in every mode.

@@ -1988,6 +1988,37 @@ def test_decode_rows_by_halves_of_a_block(pkg, wl, gpu, monkeypatch, P, fp8, row
         assert torch.equal(got, expect)
 
 
+@pytest.mark.parametrize("P", [16, 64])
+@pytest.mark.parametrize("window", [None, 40])
+def test_e4m3_shares_of_short_pieces(pkg, wl, gpu, monkeypatch, P, window):
+    """e4m3 rows on the balanced plan ask for their blocks two ahead, over the borders of pieces: pieces of one to six blocks in every
+    order, runs of one-block rows (whose next block is asked for late), rows without tokens among them, few waves and many; the
+    new tokens brought along."""
+    Hkv = 2
+    sizes = [1, 5, 2, 4, 3, 1, 1, 2, 2, 1, 6, 3, 1, 3, 1, 4, 1, 1, 1, 5, 5, 2, 1, 2, 4, 1, 3, 3, 1, 6, 6, 1, 4, 4, 130, 2]
+    kv_lens = [32 * n - 7 * i % 31 for i, n in enumerate(sizes)]
+    empty = [11, 24, 25]
+    keep = torch.tensor([i for i in range(len(sizes)) if i not in empty])
+    b = wl.make_batch("short_pieces", [1] * len(sizes), kv_lens, num_q_heads=4 * Hkv, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=11,
+                      kv_dtype=torch.float8_e4m3fn, sliding_window=window)
+    want = oracle_out(b)
+    keys, values, cache = with_new_tokens(b)
+    g = b.to(gpu)
+    lens = g.kv_lens.clone()
+    lens[torch.tensor(empty, device=gpu)] = 0
+    for waves in ("2", "6", "16", "1024"):
+        monkeypatch.setenv("RPA_DECODE_WAVE_CAPACITY", waves)
+        say(f"short pieces P={P} window={window} waves={waves}")
+        for new, kv in ((True, g.kv_lens), (False, lens)):
+            out, _ = pkg.ragged_paged_attention(
+                g.q, keys.to(gpu) if new else None, values.to(gpu) if new else None, cache.to(gpu) if new else g.kv_cache, kv,
+                g.page_indices, g.cu_q_lens, g.cu_kv_lens, b.distribution.numpy(), sm_scale=b.sm_scale, sliding_window=window,
+                k_scale=g.k_scale, v_scale=g.v_scale, max_kv_len=max(kv_lens), max_q_len=1, num_splits=2)
+            torch.cuda.synchronize()
+            rows = torch.arange(len(sizes)) if new else keep
+            assert_parity(out.cpu()[rows].float(), want[rows].float(), **FP8_TOL)
+
+
 @pytest.mark.parametrize("Hq,Hkv,P,fp8,window", [(16, 8, 64, False, None), (40, 2, 16, False, 150), (12, 1, 24, True, None), (16, 2, 64, True, 333)])
 def test_rows_by_workgroups_in_pieces(pkg, wl, gpu, monkeypatch, Hq, Hkv, P, fp8, window):
     """Pieces of a row by workgroups of eight waves, any number of them: rows shorter than a piece, pieces of fewer blocks than waves, ends
