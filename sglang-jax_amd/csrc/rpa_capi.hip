@@ -1327,7 +1327,9 @@ static float mla_logit_scale(const RpaMlaParams* p) {
   return p->sm_scale * (p->k_scale > 0.f ? p->k_scale : 1.0f) * (p->q_scale > 0.f ? p->q_scale : 1.0f);
 }
 
-static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const char* extra_rows = nullptr) {
+// new_kv_c, new_k_pe: the sequences' new tokens where the kernels are to put them into the cache (not with token_rows).
+static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const char* extra_rows = nullptr, const void* new_kv_c = nullptr,
+                   const void* new_k_pe = nullptr) {
   const rpa::TuningOfCall tuning;
   int rc = mla_validate(p);
   if (rc != RPA_OK) return rc;
@@ -1339,6 +1341,8 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const c
   const SplitPlan sp = mla_plan(p, rows);
   rpa::MlaDecodeArgs a;
   a.extra_rows = extra_rows;
+  a.new_kv_c = static_cast<const char*>(new_kv_c);
+  a.new_k_pe = static_cast<const char*>(new_k_pe);
   a.ql_nope = static_cast<const uint16_t*>(p->ql_nope);
   a.q_pe = static_cast<const uint16_t*>(p->q_pe);
   a.out = static_cast<uint16_t*>(p->out);
@@ -1467,11 +1471,10 @@ int rpa_mla_kv_write(const RpaMlaParams* p, const void* new_kv_c, const void* ne
 int rpa_mla_attention_update(const RpaMlaParams* p, const void* new_kv_c, const void* new_k_pe, int token_rows,
                              void* stream) {
   const WorkspaceTurn turn(p ? p->workspace : nullptr);
-  if (new_kv_c || new_k_pe) {
-    const int rc = rpa_mla_kv_write(p, new_kv_c, new_k_pe, stream);
-    if (rc != RPA_OK) return rc;
-  }
-  return mla_run(p, stream, token_rows != 0);
+  if (!new_kv_c && !new_k_pe) return mla_run(p, stream, token_rows != 0);
+  if (!token_rows && new_kv_c && new_k_pe) return mla_run(p, stream, false, nullptr, new_kv_c, new_k_pe);
+  const int rc = rpa_mla_kv_write(p, new_kv_c, new_k_pe, stream);
+  return rc != RPA_OK ? rc : mla_run(p, stream, token_rows != 0);
 }
 
 // ---- sparse attention: the dense kernels over a page table per query token ----

@@ -195,6 +195,9 @@ struct MlaDecodeArgs {
   int32_t fp8;          // cache rows are e4m3 bytes (row_stride / rope_offset stay in elements)
   // pages -1, -2, ... of the page table are pages 0, 1, ... of this buffer (pages under 32 tokens only), or nullptr
   const char* extra_rows;
+  // sequence rows: the new tokens' latents, [T, 512] and [T, 64] in the cache's type, which the kernels put into the cache; or nullptr
+  const char* new_kv_c;
+  const char* new_k_pe;
 };
 
 struct MlaWriteArgs {

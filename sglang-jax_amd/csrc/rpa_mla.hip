@@ -335,6 +335,42 @@ struct MlaDest {
   int64_t base;
 };
 
+// A sequence row's new token, from the caller's rows into the cache (a.new_kv_c), by every workgroup whose share holds the row's last
+// tile, in front of everything else that it does.  A launch of its own for 1152 bytes a row took 5.4 us of the GPU and 2.7 of the
+// host; here it is a round trip to memory at the start of those workgroups: 64 ragged rows x 128 heads 179.8 -> 177.4 us, 25 rows of
+// 125..1062 38.0 -> 35.8, 2 of 4516..9525 x 16 heads 32.3 -> 30.2, 6 of 351..927 e4m3 33.7 -> 30.7.
+// Every wave writes the whole row (the same bytes, 2 stores), so the copies that it makes of it afterwards follow its own stores
+// and no barrier is needed.  Tiles behind a piece's first three are asked for behind a wait for the first one, which is younger than
+// the stores; where the row's last tile may be among the first three the caller of this waits for the stores.  (Registers that
+// wait for the token beside the first copies are live into the tile loops, which spill then and drain their copies to
+// reload: 22 rows on token-level selections x 128 heads, which bring no token here, 50.3 -> 52.3 us.)
+template <bool FP8>
+__device__ __forceinline__ void put_new_row(const MlaDecodeArgs& a, int seq, int kv_len) {
+  const int lane = threadIdx.x & 63;
+  const int P = a.pt.page_size;
+  const int q0 = scalar_load_i32(a.pt.cu_q_lens + seq), n = scalar_load_i32(a.pt.cu_q_lens + seq + 1) - q0;
+  const int32_t* pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (int64_t)(scalar_load_i32(a.pt.cu_kv_lens + seq) / P)
+                                                            : (int64_t)seq * a.pt.pages_per_seq);
+  for (int j = 0; j < n; ++j) {  // (one: a decode row brings one token)
+    const int64_t tok = q0 + j;
+    const int pos = kv_len - n + j;
+    if (pos < 0) continue;
+    const int slot = __builtin_amdgcn_readfirstlane((P & (P - 1)) == 0 ? pos >> (31 - __builtin_clz(P)) : pos / P);
+    char* page = const_cast<char*>(a.cache);
+    if constexpr (FP8) {
+      const int t = min(lane, 35);
+      const u32x4_t x = ld16(t < 32 ? a.new_kv_c + tok * 512 + t * 16 : a.new_k_pe + tok * 64 + (t - 32) * 16);
+      char* row = page + ((int64_t)scalar_load_i32(pages + slot) * P + (pos - slot * P)) * a.row_stride;
+      if (lane < 36) st16(row + (lane < 32 ? lane * 16 : a.rope_offset + (lane - 32) * 16), x);
+    } else {
+      const u32x4_t x = ld16(a.new_kv_c + tok * 1024 + lane * 16), y = ld16(a.new_k_pe + tok * 128 + (lane & 7) * 16);
+      char* row = page + ((int64_t)scalar_load_i32(pages + slot) * P + (pos - slot * P)) * a.row_stride * 2;
+      st16(row + lane * 16, x);
+      if (lane < 8) st16(row + a.rope_offset * 2 + lane * 16, y);
+    }
+  }
+}
+
 // One workgroup, one row, one group of 128 heads, tokens [t_begin, t_end).  Every wave of the
 // workgroup calls it with the same arguments; all LDS reads of an earlier call are behind a
 // barrier when it returns.
@@ -799,6 +835,10 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_decode_kernel(const MlaDecodeA
   MlaDest dest;
   dest.final_rows = a.max_splits == 1;
   dest.base = ((int64_t)row_id * a.max_splits + split) * a.Hq;
+  if (a.new_kv_c && t_end == kv_len) {
+    put_new_row<FP8>(a, mr.seq, kv_len);
+    if (kv_len - t_begin <= 3 * kTok) wait_all_loads();  // (and stores)
+  }
   mla_segment<UNIFORM, CAP, PIPE, FP8, DS>(a, mr, blockIdx.z * 128, t_lo, t_begin, t_end, dest, slot0, slot1, slot2, slot3);
 }
 
@@ -1248,6 +1288,10 @@ __global__ __launch_bounds__(256, 1) void rpa_mla_decode_wide_kernel(const MlaDe
   MlaDest dest;
   dest.final_rows = a.max_splits == 1;
   dest.base = ((int64_t)row_id * a.max_splits + split) * a.Hq;
+  if (a.new_kv_c && t_end == kv_len) {
+    put_new_row<false>(a, mr.seq, kv_len);
+    if (kv_len - t_begin <= 3 * kTok) wait_all_loads();  // (and stores)
+  }
   mla_segment_wide<M32, false, P16>(a, mr, blockIdx.z * 128, t_lo, t_begin, t_end, dest, ring);
 }
 
@@ -1282,7 +1326,7 @@ __device__ __forceinline__ int mla_tiles_per_wg(const MlaDecodeArgs& a, int tota
 }
 
 // `segment(mr, head_base, t_lo, t_begin, t_end, dest)` runs one piece on the workgroup's LDS ring.
-template <class Segment>
+template <bool FP8, class Segment>
 __device__ __forceinline__ void mla_balanced_body(const MlaDecodeArgs& a, Segment segment) {
   const int lane = threadIdx.x & 63;
   const int wg = blockIdx.x;
@@ -1348,6 +1392,22 @@ __device__ __forceinline__ void mla_balanced_body(const MlaDecodeArgs& a, Segmen
   int kv_len = scalar_load_i32(a.pt.kv_lens + seq);
   int nt = mla_tiles(kv_len, a.sm.window);
   const int pad = a.piece_pad;
+  if (a.new_kv_c) {  // the new tokens of the rows that end in this share, all of them in front of its first piece
+    int s = seq, len = kv_len, from = seq_first, tiles = nt;
+    for (;;) {
+      const int unit_end = from + (max(x - from, 0) / (tiles + pad) + 1) * (tiles + pad);
+      if (unit_end > x_end) break;
+      put_new_row<FP8>(a, s, len);
+      from += (tiles + pad) * units;
+      if (from >= x_end) break;
+      do {
+        ++s;
+        len = scalar_load_i32(a.pt.kv_lens + s);
+        tiles = mla_tiles(len, a.sm.window);
+      } while (tiles == 0);
+    }
+    wait_all_loads();  // (and stores)
+  }
   bool first_piece = true;
   int piece_no = 0;  // (only the optional timestamps use it)
   while (x < x_end) {
@@ -1392,7 +1452,7 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_balanced_kernel(const MlaDecod
   __shared__ __attribute__((aligned(1024))) char slot1[kSlotB];
   __shared__ __attribute__((aligned(1024))) char slot2[kSlotB];
   __shared__ __attribute__((aligned(1024))) char slot3[kSlotB];
-  mla_balanced_body(a, [&](const MlaRow& mr, int head_base, int t_lo, int t_begin, int t_end, const MlaDest& dest, int)
+  mla_balanced_body<FP8>(a, [&](const MlaRow& mr, int head_base, int t_lo, int t_begin, int t_end, const MlaDest& dest, int)
                         __attribute__((always_inline)) {
     mla_segment<UNIFORM, CAP, PIPE, FP8, DS>(a, mr, head_base, t_lo, t_begin, t_end, dest, slot0, slot1, slot2, slot3);
   });
@@ -1402,7 +1462,7 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_balanced_kernel(const MlaDecod
 template <bool M32, bool P16 = false>
 __global__ __launch_bounds__(256, 1) void rpa_mla_balanced_wide_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char ring[4 * kSlotB];
-  mla_balanced_body(a, [&](const MlaRow& mr, int head_base, int t_lo, int t_begin, int t_end, const MlaDest& dest,
+  mla_balanced_body<false>(a, [&](const MlaRow& mr, int head_base, int t_lo, int t_begin, int t_end, const MlaDest& dest,
                            int piece) __attribute__((always_inline)) {
     mla_segment_wide<M32, false, P16>(a, mr, head_base, t_lo, t_begin, t_end, dest, ring, piece);
   });
