@@ -165,19 +165,24 @@ __device__ __forceinline__ void chunk_of(const Src& s, int wave, int lane, int n
   inner = j < 64 ? j * 16 : s.rope_byte + (j - 64) * 16;
 }
 
-template <bool UNIFORM, int CPW = kCopiesPerWave>
+// Rows past the row's last token are that token's again.  Pages of whole tiles: a tile lies in one page, so that is a bound on the
+// lane's row; with a page looked up for each row of a partial tile (what was here before, for every copy of the last tile, and a piece
+// copies that one up to four times) 2 rows of 100..200 tokens x 16 heads took 18.6 us instead of 17.4.
+// KEEP: registers to spare for the lanes' offsets (tiles shared among waves).
+template <bool UNIFORM, int CPW = kCopiesPerWave, bool KEEP = false>
 __device__ __forceinline__ void copy_tile(char* slot, const Src& s, const char* cache, int tb, int wave, int lane,
                                           int page) {
   tb = min(tb, s.last_tok & ~(kTok - 1));  // past the end: re-copy the last tile
+  // chunk offsets are recomputed per tile (a dozen integer ops) rather than kept in
+  // registers: the accumulators and Q^T leave no room, and a spill reload would be a
+  // vector-memory load that drains the copy queue
+  int ln = lane;
+  if constexpr (UNIFORM && !KEEP) asm volatile("" : "+v"(ln));  // opaque: keeps the offset arithmetic inside the loop
   if constexpr (UNIFORM) {
-    if (tb + kTok - 1 <= s.last_tok) {
-      const char* base = cache + (int64_t)page * s.page_stride +
-                         (int64_t)(tb - page_slot(s, tb) * s.page_size) * s.row_bytes;  // scalar
-      // chunk offsets are recomputed per tile (a dozen integer ops) rather than kept in
-      // registers: the accumulators and Q^T leave no room, and a spill reload would be a
-      // vector-memory load that drains the copy queue
-      int ln = lane;
-      asm volatile("" : "+v"(ln));  // opaque: keeps the offset arithmetic inside the loop
+    const char* base = cache + (int64_t)page * s.page_stride +
+                       (int64_t)(tb - page_slot(s, tb) * s.page_size) * s.row_bytes;  // scalar
+    const int most = s.last_tok - tb;
+    if (CPW > kCopiesPerWave && most >= kTok - 1) {  // (the wide kernels' prologue: three tiles on the same offsets)
 #pragma unroll
       for (int n = 0; n < CPW; ++n) {
         int row, inner;
@@ -186,17 +191,26 @@ __device__ __forceinline__ void copy_tile(char* slot, const Src& s, const char* 
       }
       return;
     }
-  }
-  // last, partial tile (rows clamped to the last valid token) or pages smaller than a tile
 #pragma unroll
-  for (int n = 0; n < CPW; ++n) {
-    int row, inner;
-    chunk_of<CPW>(s, wave, lane, n, row, inner);
-    const int tok = min(tb + row, s.last_tok);
-    const int ps = page_slot(s, tok);
-    const int pg = UNIFORM ? page : page_in_ring(s, tb, ps);
-    const char* src = page_base<UNIFORM>(s, cache, pg) + (int64_t)(tok - ps * s.page_size) * s.row_bytes + inner;
-    async_copy16(src, slot + copy_block<CPW>(wave, n) * 1024);
+    for (int n = 0; n < CPW; ++n) {
+      int row, inner;
+      chunk_of<CPW>(s, wave, ln, n, row, inner);
+      async_copy16(base + (uint32_t)(min(row, most) * s.row_bytes + inner), slot + copy_block<CPW>(wave, n) * 1024);
+    }
+  } else {
+    // pages smaller than a tile: all the ids first, one round trip to LDS
+    int64_t at[CPW];
+    int pg[CPW];
+#pragma unroll
+    for (int n = 0; n < CPW; ++n) {
+      int row, inner;
+      chunk_of<CPW>(s, wave, ln, n, row, inner);
+      const int tok = min(tb + row, s.last_tok), ps = page_slot(s, tok);
+      pg[n] = page_in_ring(s, tb, ps);
+      at[n] = (int64_t)(tok - ps * s.page_size) * s.row_bytes + inner;
+    }
+#pragma unroll
+    for (int n = 0; n < CPW; ++n) async_copy16(page_base<false>(s, cache, pg[n]) + at[n], slot + copy_block<CPW>(wave, n) * 1024);
   }
 }
 
@@ -229,29 +243,31 @@ __device__ __forceinline__ void f8_chunk_of(const Src& s, int wave, int lane, in
   inner = j < 32 ? j * 16 : s.rope_byte + (j - 32) * 16;
 }
 
-template <bool UNIFORM>
+template <bool UNIFORM, bool KEEP = false>
 __device__ __forceinline__ void copy_tile_f8(char* stage, const Src& s, const char* cache, int tb, int wave, int lane,
                                              int page) {
   tb = min(tb, s.last_tok & ~(kTok - 1));
-  const bool whole = UNIFORM && (tb + kTok - 1 <= s.last_tok);
   const char* base = cache + (int64_t)page * s.page_stride + (int64_t)(tb - page_slot(s, tb) * s.page_size) * s.row_bytes;
+  const int most = s.last_tok - tb;
   int ln = lane;
-  asm volatile("" : "+v"(ln));
+  if constexpr (UNIFORM && !KEEP) asm volatile("" : "+v"(ln));
+  std::conditional_t<UNIFORM, uint32_t, int64_t> at[kF8CopiesPerWave];
+  int pg[kF8CopiesPerWave];
 #pragma unroll
   for (int n = 0; n < kF8CopiesPerWave; ++n) {
-    const int blk = f8_copy_block(wave, n);
     int row, inner;
     f8_chunk_of(s, wave, ln, n, row, inner);
-    if (whole) {
-      async_copy16(base + (uint32_t)(row * s.row_bytes + inner), stage + blk * 1024);
-    } else {  // last, partial tile (rows clamped to the last valid token) or pages smaller than a tile
-      const int tok = min(tb + row, s.last_tok);
-      const int ps = page_slot(s, tok);
-      const int pg = UNIFORM ? page : page_in_ring(s, tb, ps);
-      async_copy16(page_base<UNIFORM>(s, cache, pg) + (int64_t)(tok - ps * s.page_size) * s.row_bytes + inner,
-                   stage + blk * 1024);
+    pg[n] = 0;
+    at[n] = min(row, most) * s.row_bytes + inner;
+    if constexpr (!UNIFORM) {  // pages smaller than a tile
+      const int tok = min(tb + row, s.last_tok), ps = page_slot(s, tok);
+      pg[n] = page_in_ring(s, tb, ps);
+      at[n] = (int64_t)(tok - ps * s.page_size) * s.row_bytes + inner;
     }
   }
+#pragma unroll
+  for (int n = 0; n < kF8CopiesPerWave; ++n)
+    async_copy16((UNIFORM ? base : page_base<false>(s, cache, pg[n])) + at[n], stage + f8_copy_block(wave, n) * 1024);
 }
 
 // e4m3 bytes of a staged tile -> bf16 rows of a ring slot (exact).  512 threads, 1152 chunks of 16
@@ -387,6 +403,12 @@ __device__ __forceinline__ void put_new_row(const MlaDecodeArgs& a, int seq, int
 // block of 16 heads share its tile instead: wave `sub` of the block takes token half sub & 1 and k-step group
 // sub >> 1 of the first product, leaves its partial scores in LDS, every wave of the block sums them and takes
 // the (same) probabilities, and the second product's 32 output chunks are dealt out 32 / DS per wave.
+// What bounds a shared tile's step is its chain: K operands from LDS, products, partial scores to LDS and back, softmax, second product.
+// So a wave keeps its own k-steps' queries alone, asks for its K operands before it works out the copies' addresses, and for the partial
+// scores and the V^T operands together behind the barrier; page ids come from a register and the lanes' offsets stay in some.  With
+// the reads two at a time, each waited for, and a scalar load among them: 32 rows of 1000..4000 tokens x 32 heads 40.1 -> 32.1 us,
+// 64 of 2048..16384 x 64 heads 192 -> 170, x 16 heads 146 -> 134, 2 of 100..200 x 16 heads 17.4 -> 14.4, 32 selections of whole
+// pages x 16 heads 46.7 -> 44.6 (the call).
 // TG (token group): with 16 / 32 / 64 heads, the eight waves hold 8 / 4 / 2 CONSECUTIVE QUERY TOKENS of one
 // sequence instead of one token's heads, `group_tokens` of them real (a chunk's tail may leave fewer): wave w
 // owns token (16 w) / Hq of the group and the block of 16 heads (16 w) % Hq.  mr.tq is the group's first token,
@@ -433,26 +455,48 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   src.ids = (lds_i32_t)id_ring;
   src.extra = a.extra_rows;
   src.t_begin = t_begin;
+  // (Shared tiles: the ids of 64 pages wait in a register, a lane each.  A scalar load in the step is waited for with the step's LDS
+  // reads, whichever comes first, and from the next cache line of ids it is a round trip to memory.)
+  int page_ids = 0, page_ids_first = 0;
+  auto fetch_page_ids = [&](int slot) {
+    page_ids_first = slot;
+    const int32_t* at = src.pages + min(slot + lane, page_slot(src, src.last_tok));
+    // (by name, wait included: the compiler would wait for every load in flight at each use)
+    asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=v"(page_ids) : "v"(at) : "memory");
+  };
+  if constexpr (UNIFORM && DS > 1) fetch_page_ids(page_slot(src, t_begin));
   auto page_of = [&](int tb) -> int {
     if constexpr (UNIFORM) {
       tb = min(tb, src.last_tok & ~(kTok - 1));
-      return scalar_load_i32(src.pages + __builtin_amdgcn_readfirstlane(page_slot(src, tb)));
+      const int slot = __builtin_amdgcn_readfirstlane(page_slot(src, tb));
+      if constexpr (DS > 1) {
+        if (slot - page_ids_first >= 64) fetch_page_ids(slot);
+        return __builtin_amdgcn_readlane(page_ids, slot - page_ids_first);
+      } else {
+        return scalar_load_i32(src.pages + slot);
+      }
     } else {
       return 0;
     }
   };
 
   // ---- Q^T operands of this wave: column c = head head0 + c, k-step ks covers dims 32ks + 8g .. ----
+  // (shared tiles: the k-steps of this wave's group alone)
   const int tq = mr.tq;
-  u32x4_t qB[18];
+  constexpr int kGroups = DS == 1 ? 1 : DS / 2;  // of k-steps: 4 groups of 5, 5, 4, 4; 2 of 9; 1 of 18
+  constexpr int kQ = kGroups == 4 ? 5 : 18 / kGroups;
+  const int kg = DS == 1 ? 0 : sub >> 1;
+  const int ks0 = kGroups == 4 && kg == 3 ? 14 : kg * kQ;
+  u32x4_t qB[kQ];
   {
     const int head = TG ? head0 + c : min(head0 + c, a.Hq - 1);
     const uint16_t* qn = a.ql_nope + ((int64_t)tq * a.Hq + head) * 512 + g * 8;
     const uint16_t* qr = a.q_pe + ((int64_t)tq * a.Hq + head) * 64 + g * 8;
 #pragma unroll
-    for (int ks = 0; ks < 16; ++ks) qB[ks] = ld16(qn + ks * 32);
-    qB[16] = ld16(qr);
-    qB[17] = ld16(qr + 32);
+    for (int i = 0; i < kQ; ++i) {
+      const int ks = min(ks0 + i, 17);
+      qB[i] = ld16(ks < 16 ? qn + ks * 32 : qr + (ks - 16) * 32);
+    }
   }
 
   const float scale = a.sm.sm_scale;
@@ -497,7 +541,7 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   // re-checking them with s_waitcnt vmcnt(0..4) inside the loop, where such a wait would also
   // drain the copy queue.
 #pragma unroll
-  for (int ks = 0; ks < 18; ++ks) asm volatile("" ::"v"(qB[ks]));
+  for (int ks = 0; ks < kQ; ++ks) asm volatile("" ::"v"(qB[ks]));
   // wait for the first tile (all but the 10 newest copies), then meet
   constexpr int kAhead = 2 * (FP8 ? kF8CopiesPerWave : kCopiesPerWave);  // copies of the two tiles behind the next one
   // in the loop a step's id request precedes its copies: the ids it has to wait for are older than both tiles' copies
@@ -527,36 +571,42 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
     const int v_off_t = PIPE ? ((4 * g_t + (c_t >> 2)) * kRowB + (c_t & 3) * 8) : v_off;
     // `fill` held tile tb - 32, which every wave finished before the last barrier
     if constexpr (!UNIFORM) copy_tile_ids(src, tb + 5 * kTok, lane_t);
-    if constexpr (FP8) copy_tile_f8<UNIFORM>(fill, src, a.cache, tb + 3 * kTok, wave, lane_t, pg_next);
-    else copy_tile<UNIFORM>(fill, src, a.cache, tb + 3 * kTok, wave, lane_t, pg_next);
+    constexpr int kKx = kQ < 9 ? kQ : 9, kVx = kChunksPerWave < 8 ? kChunksPerWave : 8;  // (what the registers hold)
+    u32x4_t kx[DS > 1 ? kKx : 1];
+    const char* kp = cur + k_off_t + (DS > 1 ? (sub & 1) * 16 * kRowB + ks0 * 64 : 0);
+    if constexpr (DS > 1) {  // this wave's K operands are on their way before the copies' addresses are worked out
+#pragma unroll
+      for (int i = 0; i < kKx; ++i) kx[i] = lds_ld16(kp + (kGroups == 4 && i == 4 && kg >= 2 ? 3 : i) * 64);
+    }
+    if constexpr (FP8) copy_tile_f8<UNIFORM, (DS > 1)>(fill, src, a.cache, tb + 3 * kTok, wave, lane_t, pg_next);
+    else copy_tile<UNIFORM, kCopiesPerWave, (DS > 1)>(fill, src, a.cache, tb + 3 * kTok, wave, lane_t, pg_next);
     pg_next = page_of(tb + 4 * kTok);
+    f32x4_t part[DS > 1 ? DS : 1];
+    u32x2_t vx[DS > 1 ? kVx : 1][2];
+    // (shared tiles: this wave's chunks are sub * kChunksPerWave .. of the 32)
+    const char* vp = cur + v_off_t + (DS > 1 ? sub * kChunksPerWave * 32 : 0);
     if constexpr (DS > 1) {
       // this wave's share of the first product: one token half, one group of k-steps
       f32x4_t sp = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      if (wave_on) {
-        const char* kp = cur + k_off_t + (sub & 1) * 16 * kRowB;
-        constexpr int kGroups = DS / 2;  // 4 groups of 5, 5, 4, 4 k-steps; 2 of 9; 1 of 18
-        auto chain = [&](auto lo, auto hi) __attribute__((always_inline)) {
 #pragma unroll
-          for (int ks = decltype(lo)::value; ks < decltype(hi)::value; ++ks) sp = mfma16(lds_ld16(kp + ks * 64), qB[ks], sp);
-        };
-        using std::integral_constant;
-        const int kg = sub >> 1;
-        if constexpr (kGroups == 4) {
-          if (kg == 0) chain(integral_constant<int, 0>{}, integral_constant<int, 5>{});
-          else if (kg == 1) chain(integral_constant<int, 5>{}, integral_constant<int, 10>{});
-          else if (kg == 2) chain(integral_constant<int, 10>{}, integral_constant<int, 14>{});
-          else chain(integral_constant<int, 14>{}, integral_constant<int, 18>{});
-        } else if constexpr (kGroups == 2) {
-          if (kg == 0) chain(integral_constant<int, 0>{}, integral_constant<int, 9>{});
-          else chain(integral_constant<int, 9>{}, integral_constant<int, 18>{});
-        } else {
-          chain(integral_constant<int, 0>{}, integral_constant<int, 18>{});
-        }
+      for (int i = 0; i < kQ; ++i) {
+        if (!(kGroups == 4 && i == 4) || kg < 2) sp = mfma16(kx[i % kKx], qB[i], sp);
+        if (i + kKx < kQ) kx[i] = lds_ld16(kp + (i + kKx) * 64);
       }
       *reinterpret_cast<f32x4_t*>(&partial_scores[wave][lane_t * 4]) = sp;
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the partial scores are written
       bare_barrier();
+      // everything else that the step reads from LDS, at once: the partial sums of the block's DS waves (wave sub' holds half
+      // sub' & 1, group sub' >> 1) and the V^T operands
+      const int w0 = (wave / DS) * DS;
+#pragma unroll
+      for (int u = 0; u < DS; ++u) part[u] = *reinterpret_cast<const f32x4_t*>(&partial_scores[w0 + u][lane_t * 4]);
+#pragma unroll
+      for (int j = 0; j < kVx; ++j) {
+        vx[j][0] = lds_tr16(vp + j * 32);
+        vx[j][1] = lds_tr16(vp + j * 32 + 16 * kRowB);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
     if (wave_on) {
       // two independent accumulator chains (token halves), issued alternately
@@ -564,15 +614,9 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
       s[0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       s[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       if constexpr (DS > 1) {
-        // the block's scores: the partial sums of its DS waves (wave sub' holds half sub' & 1, group sub' >> 1)
-        const int w0 = (wave / DS) * DS;
 #pragma unroll
-        for (int u = 0; u < DS; ++u) {
-          const f32x4_t part = *reinterpret_cast<const f32x4_t*>(&partial_scores[w0 + u][lane_t * 4]);
-          s[u & 1] += part;
-        }
+        for (int u = 0; u < DS; ++u) s[u & 1] += part[u];
       } else {
-      const char* kp = cur + k_off_t;
 #pragma unroll
       for (int ks = 0; ks < 18; ++ks) {
         s[0] = mfma16(lds_ld16(kp + ks * 64), qB[ks], s[0]);
@@ -598,8 +642,7 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
         }
       }
       float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      mx = swap_max(swap16_max(mx));
       const float m_new = fmaxf(m, mx);
       const float alpha = fast_exp2(m - m_new);
       float p[8], ps = 0.f;
@@ -616,15 +659,17 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
 #pragma unroll
         for (int j = 0; j < kChunksPerWave; ++j) acc[j] = acc[j] * alpha;
       }
-      // (shared tiles: this wave's chunks are sub * kChunksPerWave .. of the 32)
-      const char* vp = cur + v_off_t + (DS > 1 ? sub * kChunksPerWave * 32 : 0);
 #pragma unroll
       for (int j = 0; j < kChunksPerWave; ++j) {
-        const char* vt = vp + j * 32;
-        const u32x2_t lo = lds_tr16(vt);
-        const u32x2_t hi = lds_tr16(vt + 16 * kRowB);
-        acc[j] = mfma16(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pB, acc[j]);
-        if (j % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+        if (DS > 1 && j < kVx) {
+          acc[j] = mfma16(u32x4_t{vx[j][0][0], vx[j][0][1], vx[j][1][0], vx[j][1][1]}, pB, acc[j]);
+        } else {
+          const char* vt = vp + j * 32;
+          const u32x2_t lo = lds_tr16(vt);
+          const u32x2_t hi = lds_tr16(vt + 16 * kRowB);
+          acc[j] = mfma16(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pB, acc[j]);
+          if (DS == 1 && j % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
     // Tile tb + 32 has landed once at most the 10 copies of tiles tb + 64 and tb + 96 are outstanding.  A bare
@@ -945,7 +990,7 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
   for (int i = 0; i < 3; ++i) {
     const int tb = t_begin + i * kTok;
     if constexpr (P16) copy_tile_p16<CPW>(ring + i * kSlotB, src, a.cache, tb, wave, lane, page_of(tb), second_page_of(tb));
-    else copy_tile<true, CPW>(ring + i * kSlotB, src, a.cache, tb, wave, lane, page_of(tb));
+    else copy_tile<true, CPW, true>(ring + i * kSlotB, src, a.cache, tb, wave, lane, page_of(tb));
   }
 #pragma unroll
   for (int hb = 0; hb < 2; ++hb)
@@ -971,7 +1016,7 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
       const int tok = t_begin + 8 * (i >> 2) + 4 * g + (i & 3);
       if (tok < kv_len && tok >= t_lo) mx = fmaxf(mx, s[i] * scale2);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    mx = swap_max(mx);
     m_init[0] = m_init[1] = mx;
   } else {
     f32x4_t s[2][2];
@@ -996,8 +1041,7 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
         const int tok = t_begin + tok_of(g, i);
         if (tok < blk_len[hb] && tok >= t_lo) mx = fmaxf(mx, s[hb][i >> 2][i & 3] * scale2);
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      mx = swap_max(swap16_max(mx));
       m_init[hb] = mx;
     }
   }
