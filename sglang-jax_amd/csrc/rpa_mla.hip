@@ -1512,19 +1512,21 @@ __global__ __launch_bounds__(256, 1) void rpa_mla_balanced_wide_kernel(const Mla
   });
 }
 
-// Merge the n partial rows of one (row, head): one wave, 8 dims (16 bytes) per lane.  Partials are taken eight at
+// Merge the n partial rows of one (row, head): 8 dims (16 bytes) per lane.  Partials are taken eight at
 // a time with every load of a group (references, sums, rows) requested before any is used -- one
 // round trip to memory per group instead of one per partial -- and groups are chained like tiles of
 // an online softmax.  Places of a group past the last partial load nothing.
-constexpr int kMergeThreads = 64;
-template <typename SlotOf>
+// WAVES: the groups are dealt out to that many waves, whose results meet in LDS.  For few (row, head)s in many pieces (merge_waves()):
+// one wave's chain of round trips was all that the launch did.
+template <int WAVES, typename SlotOf>
 __device__ __forceinline__ void mla_merge(const MlaDecodeArgs& a, int n, SlotOf slot_of, int head, int tq) {
-  const int d = threadIdx.x * 8;
+  const int wave = WAVES > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, lane = threadIdx.x & 63;
+  const int d = lane * 8;
   float mstar = -INFINITY, den = 0.f;
   float o[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = 0.f;
-  for (int j0 = 0; j0 < n; j0 += 8) {
+  for (int j0 = wave * 8; j0 < n; j0 += 8 * WAVES) {
     float mj[8], lj[8];
     u32x4_t pr[8];
 #pragma unroll
@@ -1558,14 +1560,44 @@ __device__ __forceinline__ void mla_merge(const MlaDecodeArgs& a, int n, SlotOf 
       }
     }
   }
+  if constexpr (WAVES > 1) {
+    __shared__ float parts[WAVES][512], refs[WAVES][2];
+    if (wave * 8 < n) {
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) *reinterpret_cast<f32x4_t*>(&parts[wave][d + e]) = f32x4_t{o[e], o[e + 1], o[e + 2], o[e + 3]};
+      if (lane == 0) {
+        refs[wave][0] = mstar;
+        refs[wave][1] = den;
+      }
+    }
+    __syncthreads();
+    const int used = min((n + 7) / 8, WAVES);
+    mstar = refs[0][0];
+    for (int u = 1; u < used; ++u) mstar = fmaxf(mstar, refs[u][0]);
+    constexpr int kDims = 512 / (64 * WAVES);  // dims per thread
+    float x[kDims] = {};
+    den = 0.f;
+    for (int u = 0; u < used; ++u) {
+      const float w = fast_exp2(refs[u][0] - mstar);
+      den += refs[u][1] * w;
+#pragma unroll
+      for (int e = 0; e < kDims; ++e) x[e] += parts[u][threadIdx.x * kDims + e] * w;
+    }
+    const float inv = a.out_scale / den;
+    uint16_t* op = a.out + ((int64_t)tq * a.Hq + head) * 512 + threadIdx.x * kDims;
+    if constexpr (kDims == 2) *reinterpret_cast<uint32_t*>(op) = pack_bf16x2(x[0] * inv, x[1] * inv);
+    else *op = (uint16_t)pack_bf16x2(x[0] * inv, 0.f);
+    return;
+  }
   const float inv = a.out_scale / den;
   const u32x4_t w = {pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv),
                      pack_bf16x2(o[4] * inv, o[5] * inv), pack_bf16x2(o[6] * inv, o[7] * inv)};
   st16(a.out + ((int64_t)tq * a.Hq + head) * 512 + d, w);
 }
 
-// Merge of the balanced plan.  grid = (Hq * rows); block = kMergeThreads.
-__global__ __launch_bounds__(kMergeThreads) void rpa_mla_combine_balanced_kernel(const MlaDecodeArgs a) {
+// Merge of the balanced plan.  grid = (Hq * rows); block = WAVES waves.
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void rpa_mla_combine_balanced_kernel(const MlaDecodeArgs a) {
   const int seq = (int)(blockIdx.x / (unsigned)a.Hq);  // grid.x = Hq * rows, heads fastest
   const int head = (int)blockIdx.x - seq * a.Hq;
   const int nt = mla_tiles(a.pt.kv_lens[seq], a.sm.window);
@@ -1586,11 +1618,12 @@ __global__ __launch_bounds__(kMergeThreads) void rpa_mla_combine_balanced_kernel
     return ((int64_t)wj * 2 + part) * 128 + (head & 127);
   };
   const int tq = scalar_load_i32(a.pt.cu_q_lens + seq);
-  mla_merge(a, w_last - w_first + 1, [&](int j) { return slot_of(w_first + j); }, head, tq);
+  mla_merge<WAVES>(a, w_last - w_first + 1, [&](int j) { return slot_of(w_first + j); }, head, tq);
 }
 
-// grid = (Hq * rows); block = kMergeThreads.
-__global__ __launch_bounds__(kMergeThreads) void rpa_mla_combine_kernel(const MlaDecodeArgs a) {
+// grid = (Hq * rows); block = WAVES waves.
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void rpa_mla_combine_kernel(const MlaDecodeArgs a) {
   const int row_id = (int)(blockIdx.x / (unsigned)a.Hq);  // grid.x = Hq * rows, heads fastest
   const int head = (int)blockIdx.x - row_id * a.Hq;
   const MlaRow mr = mla_row(a, row_id);
@@ -1601,7 +1634,7 @@ __global__ __launch_bounds__(kMergeThreads) void rpa_mla_combine_kernel(const Ml
   const int n = min(a.max_splits, (kv_len - t0 + a.chunk - 1) / a.chunk);
   if (n <= 0) return;
   const int64_t base = ((int64_t)row_id * a.max_splits) * a.Hq + head;
-  mla_merge(a, n, [&](int jj) { return base + (int64_t)jj * a.Hq; }, head, mr.tq);
+  mla_merge<WAVES>(a, n, [&](int jj) { return base + (int64_t)jj * a.Hq; }, head, mr.tq);
 }
 
 // New latent rows into the paged cache (mla/v1/ref.py:56-105): token j of sequence i goes to
@@ -1691,6 +1724,31 @@ int mla_token_group_mode(const MlaDecodeArgs& a, const Tuning& tune, const Shape
   return 2;
 }
 
+// Waves that merge the pieces of a (row, head).  One wave takes eight pieces per round trip; where there are more pieces and the
+// launch is few waves, four or eight of them take them at once: one row of 16000 tokens x 128 heads 55.8 -> 34.5 us, 2 rows of
+// 4000..9000 x 16 heads 26.4 -> 17.7, 4 sparse rows x 16 heads 26.8 -> 21.4, 4 of 300..3000 x 128 heads 32.2 -> 30.2.  Not from some
+// thousand waves on, which hide each other's round trips: 9 rows of 500..800 x 128 heads 28.1 -> 28.7, 16 of 1000..2000 37.9 -> 38.9.
+static int merge_waves(int64_t rows_and_heads, int64_t pieces) {
+  return rows_and_heads > 768 || pieces <= 8 ? 1 : pieces <= 32 ? 4 : 8;
+}
+
+static void launch_mla_combine(const MlaDecodeArgs& a, hipStream_t stream) {
+  const int units = (a.Hq + 127) / 128;
+  const int64_t grid = (int64_t)a.Hq * a.num_rows;
+  const int64_t pieces = a.balanced ? a.num_wgs / std::max<int64_t>(1, (int64_t)a.num_rows * units) : a.max_splits;
+#define RPA_MLA_COMBINE(W)                                                                                                          \
+  do {                                                                                                                              \
+    if (a.balanced) hipLaunchKernelGGL(rpa_mla_combine_balanced_kernel<W>, dim3((unsigned)grid), dim3(64 * W), 0, stream, a);       \
+    else hipLaunchKernelGGL(rpa_mla_combine_kernel<W>, dim3((unsigned)grid), dim3(64 * W), 0, stream, a);                           \
+  } while (0)
+  switch (merge_waves(grid, pieces)) {
+    case 1: RPA_MLA_COMBINE(1); break;
+    case 4: RPA_MLA_COMBINE(4); break;
+    default: RPA_MLA_COMBINE(8); break;
+  }
+#undef RPA_MLA_COMBINE
+}
+
 hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   if (a.num_rows <= 0) return hipSuccess;
   const int head_groups = (a.Hq + 127) / 128;
@@ -1745,7 +1803,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
       else RPA_MLA_DS(rpa_mla_balanced_kernel, bgrid, false);
       hipError_t eb = hipGetLastError();
       if (eb != hipSuccess) return eb;
-      hipLaunchKernelGGL(rpa_mla_combine_balanced_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(kMergeThreads), 0, stream, a);
+      launch_mla_combine(a, stream);
       return hipGetLastError();
     }
     if (a.fp8) RPA_MLA_DS(rpa_mla_decode_kernel, grid, true);
@@ -1755,7 +1813,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     hipError_t es = hipGetLastError();
     if (es != hipSuccess) return es;
     if (a.max_splits > 1) {
-      hipLaunchKernelGGL(rpa_mla_combine_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(kMergeThreads), 0, stream, a);
+      launch_mla_combine(a, stream);
       es = hipGetLastError();
     }
     return es;
@@ -1774,7 +1832,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
       }
       hipError_t eb = hipGetLastError();
       if (eb != hipSuccess) return eb;
-      hipLaunchKernelGGL(rpa_mla_combine_balanced_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(kMergeThreads), 0, stream, a);
+      launch_mla_combine(a, stream);
       return hipGetLastError();
     }
     if (pipe) {
@@ -1789,7 +1847,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     hipError_t ef = hipGetLastError();
     if (ef != hipSuccess) return ef;
     if (a.max_splits > 1) {
-      hipLaunchKernelGGL(rpa_mla_combine_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(kMergeThreads), 0, stream, a);
+      launch_mla_combine(a, stream);
       ef = hipGetLastError();
     }
     return ef;
@@ -1809,7 +1867,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     else hipLaunchKernelGGL(rpa_mla_balanced_wide_kernel<false>, dim3(a.num_wgs), dim3(256), 0, stream, a);
     hipError_t eb = hipGetLastError();
     if (eb != hipSuccess) return eb;
-    hipLaunchKernelGGL(rpa_mla_combine_balanced_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(kMergeThreads), 0, stream, a);
+    launch_mla_combine(a, stream);
     return hipGetLastError();
   }
   if (wide) {
@@ -1819,7 +1877,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     hipError_t ew = hipGetLastError();
     if (ew != hipSuccess) return ew;
     if (a.max_splits > 1) {
-      hipLaunchKernelGGL(rpa_mla_combine_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(kMergeThreads), 0, stream, a);
+      launch_mla_combine(a, stream);
       ew = hipGetLastError();
     }
     return ew;
@@ -1837,7 +1895,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     }
     hipError_t eb = hipGetLastError();
     if (eb != hipSuccess) return eb;
-    hipLaunchKernelGGL(rpa_mla_combine_balanced_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(kMergeThreads), 0, stream, a);
+    launch_mla_combine(a, stream);
     return hipGetLastError();
   }
   if (pipe) {
@@ -1852,7 +1910,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (a.max_splits > 1) {
-    hipLaunchKernelGGL(rpa_mla_combine_kernel, dim3((unsigned)a.Hq * (unsigned)a.num_rows), dim3(kMergeThreads), 0, stream, a);
+    launch_mla_combine(a, stream);
     e = hipGetLastError();
   }
   return e;
