@@ -126,18 +126,19 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
     t0[0] = page_slot_of(s, tb) * s.page_size;
     t0[1] = PG == kHalves ? page_slot_of(s, min(tb + 16, s.last_tok)) * s.page_size : t0[0];
   }
-  auto row_of = [&](int tok, int half, const char* cached, const char* fresh) __attribute__((always_inline)) -> const char* {
+  // (the lane's bytes in the 32-bit offset: a scalar base and one offset per load)
+  auto row_of = [&](int tok, int half, const char* cached, const char* fresh, int lane_bytes) __attribute__((always_inline)) -> const char* {
     tok = min(tok, s.last_tok);
     const char* at;
     if constexpr (PG != kLanes) {
-      at = cached + (int64_t)(PG == kHalves && half ? page.hi : page.lo) * kv.page_stride + (uint32_t)((tok - t0[half]) * kv.tok_stride);
+      at = cached + (int64_t)(PG == kHalves && half ? page.hi : page.lo) * kv.page_stride + (uint32_t)((tok - t0[half]) * kv.tok_stride + lane_bytes);
     } else {
       const int slot = page_slot_of(s, tok);
       const int pg = WINDOW ? win[slot - win_first] : s.pages[slot];
-      at = cached + (int64_t)pg * kv.page_stride + (int64_t)((tok - slot * s.page_size) * kv.tok_stride);
+      at = cached + (int64_t)pg * kv.page_stride + (int64_t)((tok - slot * s.page_size) * kv.tok_stride + lane_bytes);
     }
     if constexpr (FRESH) {
-      const char* new_at = fresh + (int64_t)(s.fresh_row + (tok - s.fresh_first) * a.Hkv) * (FP8 || HALF ? 128 : 256);
+      const char* new_at = fresh + (int64_t)(s.fresh_row + (tok - s.fresh_first) * a.Hkv) * (FP8 || HALF ? 128 : 256) + lane_bytes;
       at += (new_at - at) & -(int64_t)(tok >= s.fresh_first);
     }
     return at;
@@ -145,7 +146,7 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
   if constexpr (PART != kOnlyV) {
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const char* at = row_of(tb + b * 16 + c, b, kh, a.new_k) + g * kLaneK;
+      const char* at = row_of(tb + b * 16 + c, b, kh, a.new_k, g * kLaneK);
 #pragma unroll
       for (int st = 0; st < (FP8 || HALF ? 2 : 4); ++st) r.k[b][st] = RPA_KV_LD16(at + st * (FP8 ? 16 : 64));
     }
@@ -153,7 +154,7 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
   if constexpr (PART != kOnlyK) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const char* at = row_of(tb + tok_slot(g, i), i >= 4, vh, a.new_v) + lane_v;
+      const char* at = row_of(tb + tok_slot(g, i), i >= 4, vh, a.new_v, lane_v);
       if constexpr (FP8) r.v[i] = RPA_KV_LD8(at);
       else r.v[i] = RPA_KV_LD16(at);
     }
