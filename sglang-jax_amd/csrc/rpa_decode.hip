@@ -1457,9 +1457,9 @@ __global__ __launch_bounds__(256, FP8 ? 2 : 1) void rpa_decode_balanced_kernel(c
   decode_balanced<MT, FP8, UNIFORM_PAGE ? kBlocks : kLanes, CAP, MERGE, HALF>(a);
 }
 
-template <int MT, bool FP8, bool CAP, bool HALF = false>
+template <int MT, bool FP8, bool CAP, bool MERGE, bool HALF = false>
 __global__ __launch_bounds__(256, FP8 ? 2 : 1) void rpa_decode_balanced_halves_kernel(const DecodeArgs a) {
-  decode_balanced<MT, FP8, kHalves, CAP, false, HALF>(a);
+  decode_balanced<MT, FP8, kHalves, CAP, MERGE, HALF>(a);
 }
 
 // Merge the n partial rows of one (decode row, query head) and write the finished row.
@@ -2016,15 +2016,17 @@ void launch_decode_variant(const DecodeArgs& a, dim3 grid, dim3 block, hipStream
   if constexpr (!FP8) {
     if (a.q_dim == 64 && !(a.balanced && a.merge_counters)) {
       if (!a.balanced) hipLaunchKernelGGL((rpa_decode_splitkv_kernel<1, false, PG, CAP, true>), grid, block, lds, st, a);
-      else if constexpr (PG == kHalves) hipLaunchKernelGGL((rpa_decode_balanced_halves_kernel<1, false, CAP, true>), grid, block, lds, st, a);
+      else if constexpr (PG == kHalves) hipLaunchKernelGGL((rpa_decode_balanced_halves_kernel<1, false, CAP, false, true>), grid, block, lds, st, a);
       else hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, false, PG == kBlocks, CAP, false, true>), grid, block, lds, st, a);
       return;
     }
   }
+  // (with merge_counters set launch_decode() leaves the merge launch out: the kernel has to merge)
   if (!a.balanced) {
     hipLaunchKernelGGL((rpa_decode_splitkv_kernel<1, FP8, PG, CAP>), grid, block, lds, st, a);
   } else if constexpr (PG == kHalves) {
-    hipLaunchKernelGGL((rpa_decode_balanced_halves_kernel<1, FP8, CAP>), grid, block, lds, st, a);
+    if (a.merge_counters) hipLaunchKernelGGL((rpa_decode_balanced_halves_kernel<1, FP8, CAP, true>), grid, block, lds, st, a);
+    else hipLaunchKernelGGL((rpa_decode_balanced_halves_kernel<1, FP8, CAP, false>), grid, block, lds, st, a);
   } else if (a.merge_counters) {
     hipLaunchKernelGGL((rpa_decode_balanced_kernel<1, FP8, PG == kBlocks, CAP, true>), grid, block, lds, st, a);
   } else {

@@ -891,6 +891,48 @@ def test_balanced_plan_merge_inside_the_kernel(pkg, wl, gpu, monkeypatch):
     assert torch.equal(got, gpu_out(pkg, b, gpu))
 
 
+@pytest.mark.parametrize("P", [16, 48, 24])
+@pytest.mark.parametrize("fp8,head_dim,cap", [(False, 128, None), (False, 128, 30.0), (True, 128, None), (True, 128, 30.0), (False, 64, None)])
+def test_merge_inside_the_kernel_on_pages_under_a_block(pkg, wl, gpu, monkeypatch, P, fp8, head_dim, cap):
+    """RPA_DECODE_MERGE_IN_KERNEL=1 on pages of whole halves of a block (16, 48) and on others (24), and on heads of 64 dims, which take the
+    same kernels as wide ones there: cut rows are merged.  The new tokens brought along, into slots that hold NaN; the result is
+    the two-launch form's but for the order of its sums."""
+    kv_lens = [1 + (911 * i) % 4000 for i in range(40)]
+    say(f"merge in kernel P={P} fp8={fp8} D={head_dim} cap={cap}")
+    b = wl.make_batch("merge_in_kernel_pages", [1] * 40, kv_lens, num_q_heads=32, num_kv_heads=8, head_dim=128, page_size=P, seed=196,
+                      kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16, soft_cap=cap)
+    b.kv_cache[..., head_dim:] = 0
+    b.q[..., head_dim:] = 0
+    want, tol = oracle_out(b)[..., :head_dim].float(), FP8_TOL if fp8 else BF16_TOL
+    keys, values, holed = with_new_tokens(b)
+    keys, values = keys[..., :head_dim].contiguous().to(gpu), values[..., :head_dim].contiguous().to(gpu)
+    g = b.to(gpu)
+    q = g.q[..., :head_dim].contiguous()
+
+    def call(splits):
+        cache = holed.to(gpu)
+        # every free block of the output's size holds NaN: rows that no kernel writes are not an earlier call's
+        poison = [torch.full_like(q, math.nan) for _ in range(8)]
+        del poison
+        out, _ = pkg.ragged_paged_attention(
+            q, keys, values, cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, b.distribution.numpy(), sm_scale=b.sm_scale,
+            soft_cap=cap, k_scale=g.k_scale, v_scale=g.v_scale, max_kv_len=max(kv_lens), max_q_len=1, host_kv_lens=b.kv_lens.numpy(),
+            num_splits=splits)
+        torch.cuda.synchronize()
+        return out.cpu().float()
+
+    for splits in (0, 3, 50):
+        monkeypatch.delenv("RPA_DECODE_MERGE_IN_KERNEL", raising=False)
+        two = call(splits)
+        assert_parity(two, want, **tol)
+        monkeypatch.setenv("RPA_DECODE_MERGE_IN_KERNEL", "1")
+        for _ in range(2):
+            got = call(splits)
+            assert_parity(got, want, **tol)
+            # (both round f32 sums to bf16: 2^-8 where they fall on either side of a rounding border)
+            assert float(row_rel_error(got, two).max()) < 4e-3
+
+
 def test_balanced_plan_when_rows_outnumber_wave_slots(pkg, wl, gpu):
     """More (row, kv head) jobs than resident waves and far more than 64 MB of KV: the fixed plan
     would leave every row whole (one job each, as different in length as the rows are), so the
