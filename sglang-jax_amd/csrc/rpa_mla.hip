@@ -250,7 +250,21 @@ __device__ __forceinline__ void copy_tile_f8(char* stage, const Src& s, const ch
   const char* base = cache + (int64_t)page * s.page_stride + (int64_t)(tb - page_slot(s, tb) * s.page_size) * s.row_bytes;
   const int most = s.last_tok - tb;
   int ln = lane;
-  if constexpr (UNIFORM && !KEEP) asm volatile("" : "+v"(ln));
+  if constexpr (!KEEP) asm volatile("" : "+v"(ln));
+  if constexpr (!UNIFORM && !KEEP) {
+    // Pages smaller than a tile where each wave has heads of its own: a copy at a time.  With the ids of all three copies asked for
+    // first, as shared tiles have them below, the token-group kernel spilled four registers and every chunk lost 4 to 6 %: 4 chunks
+    // of 512 on up to 2000 tokens, pages of 16, 16 heads 239 -> 251 us, 64 heads 499 -> 520, 128 heads 976 -> 1024; so 235, 492 and 971.
+#pragma unroll
+    for (int n = 0; n < kF8CopiesPerWave; ++n) {
+      int row, inner;
+      f8_chunk_of(s, wave, ln, n, row, inner);
+      const int tok = min(tb + row, s.last_tok), ps = page_slot(s, tok);
+      async_copy16(page_base<false>(s, cache, page_in_ring(s, tb, ps)) + (int64_t)(tok - ps * s.page_size) * s.row_bytes + inner,
+                   stage + f8_copy_block(wave, n) * 1024);
+    }
+    return;
+  }
   std::conditional_t<UNIFORM, uint32_t, int64_t> at[kF8CopiesPerWave];
   int pg[kF8CopiesPerWave];
 #pragma unroll
@@ -259,7 +273,7 @@ __device__ __forceinline__ void copy_tile_f8(char* stage, const Src& s, const ch
     f8_chunk_of(s, wave, ln, n, row, inner);
     pg[n] = 0;
     at[n] = min(row, most) * s.row_bytes + inner;
-    if constexpr (!UNIFORM) {  // pages smaller than a tile
+    if constexpr (!UNIFORM) {  // pages smaller than a tile: all the ids first, one round trip to LDS
       const int tok = min(tb + row, s.last_tok), ps = page_slot(s, tok);
       pg[n] = page_in_ring(s, tb, ps);
       at[n] = (int64_t)(tok - ps * s.page_size) * s.row_bytes + inner;
