@@ -803,8 +803,9 @@ static RpaParams token_row_view(const RpaParams* p) {
 // Whether a call that may hold chunks runs with a row per query token on the decode kernels: a few tokens on short
 // contexts, where what counts is launches (cache write, decode rows, their merge, chunks, their merge: 5 x 3 us of host
 // time against 2) and not that a chunk's prefix is read once per token.  (RPA_PREFILL_SPLITS asks for the prefill kernels.)
+// Not a bucket of no sequences: the row kernels ask for the first one's lengths before they know how many there are.
 static bool takes_token_rows(const RpaParams* p) {
-  if (p->head_dim != 128 || p->mask_mode != RPA_MASK_CAUSAL || p->num_splits > 0 || p->num_tokens <= 0 ||
+  if (p->num_seqs <= 0 || p->head_dim != 128 || p->mask_mode != RPA_MASK_CAUSAL || p->num_splits > 0 || p->num_tokens <= 0 ||
       p->num_tokens > kTokenRows || rpa::tuning().prefill_splits >= 0 || (!p->distribution && p->num_seqs <= p->decode_end))
     return false;
   const RpaParams v = token_row_view(p);

@@ -162,6 +162,26 @@ def test_a_caller_of_the_earlier_struct_is_read_no_further_than_it_reaches(pkg):
         assert status(pkg, lib.rpa_validate(ctypes.byref(p))) == "RPA_EINVAL_SHAPE"
 
 
+@pytest.mark.parametrize("D,tokens", [(128, 1), (128, 64), (128, 65), (256, 4)])
+def test_a_call_without_sequences_launches_nothing(pkg, D, tokens):
+    """A bucket of no sequences, composition on the device: its arrays may have no element, so nothing may be launched that reads the
+    first one's lengths.  (Without a GPU a launch is an error; with one the addresses below would be read.)"""
+    import torch
+
+    if torch.cuda.device_count() > 0:
+        pytest.skip("a launch is seen by its failing without a GPU")
+    lib = pkg._lib.load()
+    for lens in (0x1000, None):
+        p = base_params(pkg)
+        p.num_seqs, p.num_tokens, p.decode_end, p.head_dim = 0, tokens, 0, D
+        p.distribution, p.kv_lens, p.page_indices, p.max_kv_len = 0x1000, lens, lens, 100
+        assert lib.rpa_workspace_bytes(ctypes.byref(p)) == 0
+        for new in (None, 0x1000):
+            assert lib.rpa_attention_update(ctypes.byref(p), new, new, None) == 0
+        assert lib.rpa_decode(ctypes.byref(p), None) == 0
+        assert lib.rpa_prefill(ctypes.byref(p), None) == 0
+
+
 def status(pkg, code):
     return pkg._lib.STATUS_NAMES[code]
 
