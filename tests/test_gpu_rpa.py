@@ -2064,22 +2064,39 @@ def test_e4m3_shares_of_short_pieces(pkg, wl, gpu, monkeypatch, P, window):
 @pytest.mark.parametrize("Hq,Hkv,P,fp8,window", [(16, 8, 64, False, None), (40, 2, 16, False, 150), (12, 1, 24, True, None), (16, 2, 64, True, 333)])
 def test_rows_by_workgroups_in_pieces(pkg, wl, gpu, monkeypatch, Hq, Hkv, P, fp8, window):
     """Pieces of a row by workgroups of eight waves, any number of them: rows shorter than a piece, pieces of fewer blocks than waves, ends
-    inside a block, a sink; the new token brought along.  Against the oracle and against pieces of single waves."""
+    inside a block, a sink; the new token in the cache, and brought along.  Against the oracle and against pieces of single waves."""
     kv_lens = [1, 31, 33, 256, 257, 300, 511, 513, 1000]
     say(f"row pieces {Hq}/{Hkv} P={P} fp8={fp8} window={window}")
     b = wl.make_batch("row_pieces", [1] * len(kv_lens), kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=17,
                       kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16, sliding_window=window)
     sink = torch.from_numpy(np.random.RandomState(5).randn(Hq).astype(np.float32))
     want, tol = oracle_out(b, attention_sink=sink).float(), FP8_TOL if fp8 else BF16_TOL
+    keys, values, holed = with_new_tokens(b)
+    bits = torch.uint8 if fp8 else torch.int16
+    full, expect = b.kv_cache.view(bits), holed.view(bits).clone()
+    for i, kv in enumerate(kv_lens):
+        page = int(b.page_indices[int(b.cu_kv_lens[i]) // P + (kv - 1) // P])
+        expect[page, (kv - 1) % P] = full[page, (kv - 1) % P]
+    keys, values, g = keys.to(gpu), values.to(gpu), b.to(gpu)
+
+    def bringing():
+        """The new tokens with the call, into slots that hold NaN like all unused ones: they arrive, and nothing beside them."""
+        out, after = pkg.ragged_paged_attention(
+            g.q, keys, values, holed.to(gpu), g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, b.distribution.numpy(), None, sink.to(gpu),
+            sm_scale=b.sm_scale, sliding_window=window, k_scale=g.k_scale, v_scale=g.v_scale, max_kv_len=max(kv_lens), max_q_len=1)
+        torch.cuda.synchronize()
+        assert torch.equal(after.cpu().view(bits), expect)
+        return out.cpu().float()
+
     monkeypatch.setenv("RPA_DECODE_ROW_KB", "0")
     single = gpu_out(pkg, b, gpu, attention_sink=sink).float()
     assert_parity(single, want, **tol)
     monkeypatch.delenv("RPA_DECODE_ROW_KB")
     for pieces in ("1", "2", "5", "32"):
         monkeypatch.setenv("RPA_DECODE_ROW_PIECES", pieces)
-        got = gpu_out(pkg, b, gpu, attention_sink=sink).float()
-        assert_parity(got, want, **tol)
-        torch.testing.assert_close(got, single, rtol=1e-2, atol=4e-3)
+        for got in (gpu_out(pkg, b, gpu, attention_sink=sink).float(), bringing()):
+            assert_parity(got, want, **tol)
+            torch.testing.assert_close(got, single, rtol=1e-2, atol=4e-3)
 
 
 @pytest.mark.parametrize("rows,Hkv,lo,hi,fp8", [(4, 8, 1800, 2000, False), (32, 8, 900, 1000, False), (8, 8, 3600, 4000, True)])
