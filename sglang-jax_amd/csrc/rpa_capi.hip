@@ -389,6 +389,9 @@ bool use_balanced(const RpaParams* p, const SplitPlan& fixed) {
 //     pieces: 16 x 500..2000 x 8 heads, 0.78 and 2 pieces, 26.3 -> 24.8, x 2 heads, 8 pieces, 12.2 -> 13.6)
 //     or a quarter of the CUs idle (48 rows x 2 heads x 800..1000 16.5 -> 18.0), unless the rows are whole and of up to 512 KiB
 //     (24 x 800..1000 x 8 heads 25.2 -> 23.2).
+//   Most of these borders stand on one or two shapes.  194 drawn decode batches (1 to 400 rows of 20 to 32000 tokens, head counts, page
+//   sizes and options at random) and 78 buckets, against the kernels and plans that took them before there were pieces by workgroups:
+//   0.86 of the time in the geometric mean, none slower by more than 0.5 %.
 SplitPlan row_plan(const RpaParams* p, const SplitPlan& fixed) {
   const SplitPlan none = {0, 0};
   const rpa::Tuning& tune = rpa::tuning();

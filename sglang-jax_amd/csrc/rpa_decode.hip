@@ -53,7 +53,8 @@ constexpr int kCacheBits = RPA_DECODE_NT ? 2 : 0;  // of the buffer loads: nt
 // come as scalars, a row's address is a scalar base and a 32-bit offset.  kLanes: anything else; every lane looks the page of each
 // of its ten rows up in LDS and multiplies it out in 64 bits, 0.7 us of arithmetic per block where one wave runs alone.  Pages of 16
 // tokens as kLanes and as kHalves: 64 rows of 1000..8000 tokens x 8 heads bf16 254 -> 214 us, e4m3 169 -> 137; 4 rows of
-// 1000..4095 25.3 -> 15.4; 5 rows of 64..512 in a bucket 10.2 -> 7.9.
+// 1000..4095 25.3 -> 15.4; 5 rows of 64..512 in a bucket 10.2 -> 7.9.  32 rows of 16384 tokens x 8 heads, bf16 / e4m3: 318 / 167 us on
+// pages of 64, 319 / 170 on 16 (kHalves), 336 / 231 on 24, 339 / 188 on 4, 337..351 / 204 on 1 (kLanes).
 enum Pages { kLanes, kHalves, kBlocks };
 constexpr Pages pages_of(int page_size) { return page_size % 32 == 0 ? kBlocks : page_size % 16 == 0 ? kHalves : kLanes; }
 struct BlockPages {
@@ -164,7 +165,7 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
 // The same of a block whose 32 tokens all lie in the cache.  Buffer loads: a half's first row as the base, one offset per lane
 // for all K rows and another for all V rows, what differs between the loads in a scalar: no vector instruction beside the
 // loads themselves.  wanted == false: a block that nobody needs, asked for so that the waits behind it count the same on every
-// path; its buffers have no bytes, and nothing is fetched.
+// path; its buffers have no bytes, and nothing is fetched.  (kLanes: a block that the piece reads anyway is fetched once more.)
 template <bool FP8, Pages PG, bool HALF>
 __device__ __forceinline__ void load_full_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, BlockPages page, bool wanted, int c, int g,
                                                 const int32_t* win = nullptr, int win_first = 0) {
@@ -194,7 +195,7 @@ __device__ __forceinline__ void load_full_block(KvRegs<FP8>& r, const DecodeArgs
 }
 
 // Any block, out of the cache alone (a new token's slot is read for what stands there): rows past the row's last token are the
-// last token's again, by a bound on the lanes' offsets.
+// last token's again, by a bound on the lanes' offsets.  (wanted: as above.)
 template <bool FP8, Pages PG, bool HALF>
 __device__ __forceinline__ void load_cached_block(KvRegs<FP8>& r, const DecodeArgs& a, const SeqView& s, const char* kh, const char* vh, int tb, BlockPages page, bool wanted, int c, int g,
                                                   const int32_t* win, int win_first) {
@@ -299,10 +300,10 @@ struct NewToken {
 // that is the same for the whole call is asked once per block: asked per score, as it was first, each score's chain of
 // v_exp_f32 and v_rcp_f32 ran alone between two branches, with one wave per SIMD to wait for it.
 // 32 rows of 8000..16000 tokens, soft cap, 8 kv heads: e4m3 158 -> 140 us, on 256-wide heads 350.6 -> 299.6.
-// The bf16 kernels have no register to spare beside the blocks in flight: the constants stand in scalar registers, and
-// LOOPS, a loop for either rounding, is for the balanced kernel on whole pages, which is the faster for it (bf16 rows as
-// above 269 us asked per score, 273 without LOOPS, 260 with them) though it spills four registers; the other kernels spilled up to 19 in their block loops
-// (128 rows of 128 tokens on 16-token pages, soft cap: 20.6 us asked per score, 22.7 with LOOPS, 19.3 without).
+// The bf16 kernels have no register to spare beside the blocks in flight: the constants stand in scalar registers.
+// LOOPS, a loop for either rounding, is for the balanced kernels on whole pages: rounded e4m3 logits are the faster for it (rows as
+// above, rounded to bf16 with the cap 149 -> 136 us, without 150 -> 140), everything else is level.  On other pages e4m3 loses by it
+// (capped rows as above on 16-token pages 138 -> 143 us, on 24-token pages 210 -> 213).
 struct LogitOpts {
   float k1, k2;
   bool capped;

@@ -198,7 +198,8 @@ __device__ __forceinline__ void copy_tile(char* slot, const Src& s, const char* 
       async_copy16(base + (uint32_t)(min(row, most) * s.row_bytes + inner), slot + copy_block<CPW>(wave, n) * 1024);
     }
   } else {
-    // pages smaller than a tile: all the ids first, one round trip to LDS
+    // pages smaller than a tile: all the ids first, one round trip to LDS (chunks of 512 on up to 2000 tokens, pages of 48: 128 heads
+    // 1043 -> 972 us, 16 heads 257 -> 249; with a soft cap 64 rows of 2000..8000 x 128 heads, pages of 24, 210 -> 195)
     int64_t at[CPW];
     int pg[CPW];
 #pragma unroll
@@ -368,7 +369,8 @@ struct MlaDest {
 // A sequence row's new token, from the caller's rows into the cache (a.new_kv_c), by every workgroup whose share holds the row's last
 // tile, in front of everything else that it does.  A launch of its own for 1152 bytes a row took 5.4 us of the GPU and 2.7 of the
 // host; here it is a round trip to memory at the start of those workgroups: 64 ragged rows x 128 heads 179.8 -> 177.4 us, 25 rows of
-// 125..1062 38.0 -> 35.8, 2 of 4516..9525 x 16 heads 32.3 -> 30.2, 6 of 351..927 e4m3 33.7 -> 30.7.
+// 125..1062 38.0 -> 35.8, 2 of 4516..9525 x 16 heads 32.3 -> 30.2, 6 of 351..927 e4m3 33.7 -> 30.7.  Many short rows, each of which
+// pays that round trip, are no slower: 600 rows of 100..200 x 128 heads 95.5 -> 94.2, 1000 of 30..100 118.6 -> 117.8, e4m3 121.4 -> 116.0.
 // Every wave writes the whole row (the same bytes, 2 stores), so the copies that it makes of it afterwards follow its own stores
 // and no barrier is needed.  Tiles behind a piece's first three are asked for behind a wait for the first one, which is younger than
 // the stores; where the row's last tile may be among the first three the caller of this waits for the stores.  (Registers that
