@@ -567,8 +567,11 @@ __device__ __forceinline__ void write_rows(const DecodeArgs& a, const f32x4_t (&
         f32x4_t w0 = {acc[mt][0][r] * vs, acc[mt][1][r] * vs, acc[mt][2][r] * vs, acc[mt][3][r] * vs};
         f32x4_t w1 = {acc[mt][4][r] * vs, acc[mt][5][r] * vs, acc[mt][6][r] * vs, acc[mt][7][r] * vs};
         if (through) {
-          asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(wo + r * 8), "v"(w0) : "memory");
-          asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(wo + r * 8 + 4), "v"(w1) : "memory");
+          // s_nop: a store of more than 8 bytes needs a wait state in front of a vector instruction that overwrites its data.  The
+          // compiler sees to that behind its own stores, not behind these: in one build the next row's address went straight into
+          // the registers of a store (bf16, whole pages, soft cap), and 3 of 2250 random batches came out wrong.
+          asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(wo + r * 8), "v"(w0) : "memory");
+          asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(wo + r * 8 + 4), "v"(w1) : "memory");
         } else {
           *reinterpret_cast<f32x4_t*>(wo + r * 8) = w0;
           *reinterpret_cast<f32x4_t*>(wo + r * 8 + 4) = w1;

@@ -407,17 +407,14 @@ def test_generated_assembly_is_up_to_date(tmp_path):
             assert f.read() == g.read(), f"{inc} is stale: run {gen}"
 
 
-def _device_kernels():
-    """{demangled kernel name: (spilled vector registers, scratch bytes per lane)} of the built library, from the metadata
-    notes of its device code."""
+def _device_code():
+    """The device code objects of the built library, as files."""
     import struct
-    import subprocess
     import tempfile
 
     with open(os.path.join(ROOT, "sglang-jax_amd", "lib", "librpa_mi355.so"), "rb") as f:
         blob = f.read()
-    llvm = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin")
-    found, at = {}, blob.find(b"__CLANG_OFFLOAD_BUNDLE__")
+    at = blob.find(b"__CLANG_OFFLOAD_BUNDLE__")
     while at >= 0:
         (n,), pos = struct.unpack_from("<Q", blob, at + 24), at + 32
         for _ in range(n):
@@ -429,11 +426,27 @@ def _device_kernels():
             with tempfile.NamedTemporaryFile(suffix=".co") as co:
                 co.write(blob[at + offset : at + offset + size])
                 co.flush()
-                notes = subprocess.run([os.path.join(llvm, "llvm-readelf"), "--notes", co.name], check=True, capture_output=True, text=True).stdout
-            for entry in notes.split(".agpr_count")[1:]:
-                value = {k: re.search(rf"\.{k}:\s+(\S+)", entry).group(1) for k in ("symbol", "vgpr_spill_count", "private_segment_fixed_size")}
-                found[value["symbol"]] = (int(value["vgpr_spill_count"]), int(value["private_segment_fixed_size"]))
+                yield co.name
         at = blob.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 1)
+
+
+def _llvm(tool, *args):
+    import subprocess
+
+    path = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", tool)
+    return subprocess.run([path, *args], check=True, capture_output=True, text=True).stdout
+
+
+def _device_kernels():
+    """{demangled kernel name: (spilled vector registers, scratch bytes per lane)} of the built library, from the metadata
+    notes of its device code."""
+    import subprocess
+
+    found = {}
+    for co in _device_code():
+        for entry in _llvm("llvm-readelf", "--notes", co).split(".agpr_count")[1:]:
+            value = {k: re.search(rf"\.{k}:\s+(\S+)", entry).group(1) for k in ("symbol", "vgpr_spill_count", "private_segment_fixed_size")}
+            found[value["symbol"]] = (int(value["vgpr_spill_count"]), int(value["private_segment_fixed_size"]))
     names = subprocess.run(["c++filt"], input="\n".join(n.removesuffix(".kd") for n in found), capture_output=True, text=True, check=True).stdout.split("\n")
     return dict(zip(names, found.values()))
 
@@ -452,6 +465,48 @@ def test_decode_kernels_keep_their_block_loops_in_registers(pkg):
                "rpa_decode_balanced_kernel<1, false, true, true, true, false>": 9,
                "rpa_decode_balanced_kernel<1, false, true, true, false, false>": 4}
     assert all(n <= allowed.get(k, 0) for k, n in spilled.items()), spilled
+
+
+def _instructions():
+    """(kernel, [(operation, operands), ...]) of the built library's device code, in program order."""
+    for co in _device_code():
+        kernel, ins = None, []
+        for line in _llvm("llvm-objdump", "-d", "--no-show-raw-insn", "--no-leading-addr", co).split("\n"):
+            if line.startswith("<") and line.endswith(">:"):
+                if ins:
+                    yield kernel, ins
+                kernel, ins = line[1:-2], []
+            elif line.startswith("\t"):
+                operation, _, operands = line.split("//")[0].strip().partition(" ")
+                ins.append((operation, operands))
+        if ins:
+            yield kernel, ins
+
+
+def _vector_registers(operand):
+    m = re.match(r"v\[(\d+):(\d+)\]|v(\d+)", operand.strip())
+    return set() if not m else {int(m.group(3))} if m.group(3) else set(range(int(m.group(1)), int(m.group(2)) + 1))
+
+
+def test_a_wide_store_keeps_its_data(pkg):
+    """A store of more than 8 bytes reads its registers after it has issued: one wait state before a vector instruction writes them.
+    The compiler keeps it behind its own stores; those of inline assembly (written through, sc1) bring it along."""
+    written_through, overwritten, bare = 0, [], []
+    for kernel, ins in _instructions():
+        for (op, operands), (then, target) in zip(ins, ins[1:]):
+            if not re.match(r"(global|flat|scratch|buffer)_store_dwordx[34]$", op):
+                continue
+            fields = re.split(r",\s*(?![^\[]*\])", operands)
+            data = _vector_registers(fields[0 if op.startswith("buffer") else 1])
+            by_scalar = op.startswith("buffer") and re.match(r"s\d", fields[3])  # a scalar offset is that wait state
+            if then.startswith("v_") and not by_scalar and data & _vector_registers(target):
+                overwritten.append((kernel, operands, then, target))
+            if op.startswith("global") and "sc1" in operands:
+                written_through += 1
+                if then != "s_nop":
+                    bare.append((kernel, operands, then))
+    assert written_through > 0
+    assert not overwritten and not bare, (overwritten[:3], bare[:3])
 
 
 # ------------------------------------------------------------------ the shape table (csrc/rpa_shapes.h)
