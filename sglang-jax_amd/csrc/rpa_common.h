@@ -139,10 +139,12 @@ __device__ __forceinline__ float scalar_load_f32(const float* p) {
 // inline assembly so that the compiler does not model it as an LDS store: it would otherwise
 // wait for ALL outstanding copies (vmcnt(0)) in front of every LDS read it cannot disambiguate,
 // which destroys a multi-tile prefetch.  The caller waits with s_waitcnt vmcnt(n) itself.
+// s_nop, here and at every other copy into LDS: its address is taken from m0, which a scalar instruction has to have written one wait
+// state before; the compiler does not look into inline assembly for that.
 __device__ __forceinline__ void async_copy16(const void* gsrc, const void* lds_base_uniform) {
   typedef const __attribute__((address_space(3))) char* lds_ptr_t;
   const uint32_t m0v = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)lds_base_uniform));
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0v), "v"(gsrc) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0v), "v"(gsrc) : "memory", "m0");
 }
 
 // Eight query elements from dim d of a row of q_dim (a multiple of 8); dims past it are zero.
@@ -202,7 +204,7 @@ __device__ __forceinline__ void copy_page_window(const int32_t* row_pages, int l
 #pragma unroll
   for (int k = 0; k < ENTRIES / 64; ++k) {
     const int32_t* src = row_pages + min(first_slot + 64 * k + lane, last_slot);
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(base + 256u * k), "v"(src) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(base + 256u * k), "v"(src) : "memory", "m0");
   }
 }
 

@@ -138,7 +138,7 @@ __device__ __forceinline__ void copy_tile_ids(const Src& s, int tb, int lane) {
   tb = min(tb, s.last_tok & ~(kTok - 1));
   const uint32_t dst = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s.ids + id_slot(s, tb) * kIdEntries));
   const int32_t* src = s.pages + min(page_slot(s, tb) + lane, page_slot(s, s.last_tok));
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(src) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(src) : "memory", "m0");
 }
 
 // A lane's 5 chunks of a tile: position p = 64*(5*wave + n) + lane; row p / 74, chunk

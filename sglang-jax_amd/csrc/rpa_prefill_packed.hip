@@ -77,7 +77,7 @@ struct PackedFeed {
   __device__ __forceinline__ static void request_ids(uint32_t at, const TileSrc& s, int tb, int lane) {
     tb = min(tb, s.last_tok);
     const int32_t* src = s.pages + min(page_slot(s, tb) + lane, page_slot(s, s.last_tok));
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(at), "v"(src) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(at), "v"(src) : "memory", "m0");
   }
 
   // Where the rows of the tile at `tb` are (PG 0: its page ids have arrived at `ids`).
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_packed_kernel(const Prefil
   const bool has_bits = EXT && mc.mode == 1 && mc.bits;  // (else the caller's words, one load per score)
   auto request_mask = [&](int tb) __attribute__((always_inline)) {
     const uint32_t* words = reinterpret_cast<const uint32_t*>(mc.bits) + min(tb >> 5, 2 * mc.bit_words - 1);
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(mask_at), "v"(words) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(mask_at), "v"(words) : "memory", "m0");
   };
 
   Feed feed;

@@ -509,6 +509,20 @@ def test_a_wide_store_keeps_its_data(pkg):
     assert not overwritten and not bare, (overwritten[:3], bare[:3])
 
 
+def test_a_copy_into_lds_finds_its_address(pkg):
+    """A copy into LDS takes its address from m0, which a scalar instruction has to have written one wait state before: another
+    instruction, or s_nop, stands in between.  (All of these copies are inline assembly, which the compiler does not look into.)"""
+    copies, short = 0, []
+    for kernel, ins in _instructions():
+        for (op, operands), (then, target) in zip(ins, ins[1:]):
+            if "_load_lds_" in then:
+                copies += 1
+                if op.startswith("s_") and operands.split(",")[0] == "m0":
+                    short.append((kernel, op, operands, then, target))
+    assert copies > 1000
+    assert not short, (len(short), short[:3])
+
+
 # ------------------------------------------------------------------ the shape table (csrc/rpa_shapes.h)
 def _shape_params(pkg, *, S, decode_end, T, Hq, Hkv, D=128, P=64, fp8=False, max_q=0, max_kv=0, sum_dec=0, **opts):
     p = base_params(pkg)
