@@ -38,3 +38,10 @@ def assert_parity(got, want, *, rtol, atol, rel=None):
     assert float(err.max()) <= rel, (
         f"row-relative error {float(err.max()):.3e} > {rel:g} at row {worst} of {err.numel()} "
         f"(|want| = {float(want.reshape(-1, want.shape[-1])[worst].norm()):.3e})")
+
+
+def poison_free_blocks(like):
+    """NaN in the free blocks of the size of `like`, one of which the next call's output will be: rows that no kernel writes must not
+    pass as an earlier call's."""
+    blocks = [torch.full_like(like, float("nan")) for _ in range(8)]
+    del blocks

@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 import torch
 
-from parity import assert_parity, row_rel_error
+from parity import assert_parity, poison_free_blocks, row_rel_error
 
 from oracle.ref_rpa import gather_pages as oracle_gather
 from oracle.ref_rpa import ref_ragged_paged_attention, ref_ragged_paged_attention_fused, split_fused_cache
@@ -43,6 +43,7 @@ def gpu_out(pkg, b, dev, **kw):
     q_lens = b.q_lens()
     dist = b.distribution.cpu().numpy()
     n = int(dist[2])
+    poison_free_blocks(g.q)
     out, _ = pkg.ragged_paged_attention(
         g.q, None, None, g.kv_cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, dist,
         kw.pop("custom_mask", None), sm_scale=b.sm_scale, sliding_window=b.sliding_window, soft_cap=b.soft_cap, k_scale=g.k_scale,
@@ -911,9 +912,7 @@ def test_merge_inside_the_kernel_on_pages_under_a_block(pkg, wl, gpu, monkeypatc
 
     def call(splits):
         cache = holed.to(gpu)
-        # every free block of the output's size holds NaN: rows that no kernel writes are not an earlier call's
-        poison = [torch.full_like(q, math.nan) for _ in range(8)]
-        del poison
+        poison_free_blocks(q)
         out, _ = pkg.ragged_paged_attention(
             q, keys, values, cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, b.distribution.numpy(), sm_scale=b.sm_scale,
             soft_cap=cap, k_scale=g.k_scale, v_scale=g.v_scale, max_kv_len=max(kv_lens), max_q_len=1, host_kv_lens=b.kv_lens.numpy(),
