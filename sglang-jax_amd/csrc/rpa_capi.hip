@@ -1332,8 +1332,9 @@ static float mla_logit_scale(const RpaMlaParams* p) {
 }
 
 // new_kv_c, new_k_pe: the sequences' new tokens where the kernels are to put them into the cache (not with token_rows).
-static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const char* extra_rows = nullptr, const void* new_kv_c = nullptr,
-                   const void* new_k_pe = nullptr) {
+// sparse: the rows' tables and lengths, which the kernels write first.
+static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const void* new_kv_c = nullptr, const void* new_k_pe = nullptr,
+                   const rpa::SparseMlaArgs* sparse = nullptr) {
   const rpa::TuningOfCall tuning;
   int rc = mla_validate(p);
   if (rc != RPA_OK) return rc;
@@ -1344,7 +1345,9 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const c
   if (rows <= 0) return RPA_OK;
   const SplitPlan sp = mla_plan(p, rows);
   rpa::MlaDecodeArgs a;
-  a.extra_rows = extra_rows;
+  a.sparse = {};
+  if (sparse) a.sparse = *sparse;
+  a.extra_rows = a.sparse.extra;
   a.new_kv_c = static_cast<const char*>(new_kv_c);
   a.new_k_pe = static_cast<const char*>(new_k_pe);
   a.ql_nope = static_cast<const uint16_t*>(p->ql_nope);
@@ -1374,7 +1377,7 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const c
   a.ws_o = nullptr;
   a.ws_ml = nullptr;
   a.cu_tiles = nullptr;
-  a.balanced = mla_use_balanced(p, sp, token_rows) ? 1 : 0;
+  a.balanced = !sparse && mla_use_balanced(p, sp, token_rows) ? 1 : 0;
   a.num_wgs = mla_wgs();
   a.min_tiles_per_wg = std::max(1, mla_min_piece(p) / 32);
   a.forced_tiles_per_wg = 0;
@@ -1476,7 +1479,7 @@ int rpa_mla_attention_update(const RpaMlaParams* p, const void* new_kv_c, const 
                              void* stream) {
   const WorkspaceTurn turn(p ? p->workspace : nullptr);
   if (!new_kv_c && !new_k_pe) return mla_run(p, stream, token_rows != 0);
-  if (!token_rows && new_kv_c && new_k_pe) return mla_run(p, stream, false, nullptr, new_kv_c, new_k_pe);
+  if (!token_rows && new_kv_c && new_k_pe) return mla_run(p, stream, false, new_kv_c, new_k_pe);
   const int rc = rpa_mla_kv_write(p, new_kv_c, new_k_pe, stream);
   return rc != RPA_OK ? rc : mla_run(p, stream, token_rows != 0);
 }
@@ -1490,10 +1493,11 @@ RpaMlaParams sparse_view(const RpaMlaParams* p, const RpaMlaSparse* s) {
   v.num_seqs = p->num_tokens;
   v.cu_kv_lens = nullptr;
   if (rows) v.page_size = 1;
-  v.pages_per_seq = rows ? s->topk_count : s->k_pages_max;
+  const int entries = rows ? s->topk_count : s->k_pages_max;
+  v.pages_per_seq = (entries + 31) & ~31;  // (rows of the table share no cache line)
   // a selection is as long as it can be, or as its sequence is: rows of one length, as far as the host knows (the fixed plan's
   // even pieces, 32 rows x 4096 tokens 52.5 -> 46 us against the balanced plan)
-  int64_t bound = (int64_t)v.pages_per_seq * v.page_size;
+  int64_t bound = (int64_t)entries * v.page_size;
   if (s->pages_per_seq > 0) bound = std::min(bound, (int64_t)s->pages_per_seq * p->page_size);
   v.max_kv_len = (int32_t)bound;
   v.sum_kv_len = p->num_tokens * bound;
@@ -1502,18 +1506,19 @@ RpaMlaParams sparse_view(const RpaMlaParams* p, const RpaMlaSparse* s) {
   return v;
 }
 
-// Workspace: what the view's plan needs, then the tables.
+// Workspace: what the view's plan needs, then the lengths and the tables (on a cache line of its own from wherever the workspace
+// begins, see rpa_dsa.h).
+constexpr size_t kLine = 128;
 struct SparseLayout {
-  size_t kv_lens, cu_q, table, extra, total;
+  size_t kv_lens, table, extra, total;
 };
 SparseLayout sparse_layout(const RpaMlaParams* p, const RpaMlaSparse* s, const RpaMlaParams& view) {
   auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
   const size_t T = (size_t)p->num_tokens;
   SparseLayout l;
   l.kv_lens = up(rpa_mla_workspace_bytes(&view));
-  l.cu_q = l.kv_lens + up(T * sizeof(int32_t));
-  l.table = l.cu_q + up((T + 1) * sizeof(int32_t));
-  l.extra = l.table + up(T * view.pages_per_seq * sizeof(int32_t));
+  l.table = l.kv_lens + up(T * sizeof(int32_t));
+  l.extra = l.table + up(T * view.pages_per_seq * sizeof(int32_t) + kLine);
   l.total = l.extra + (s->k_pages_max > 0 ? 0 : (T + 1) * p->row_stride * (p->cache_dtype == RPA_KV_FP8_E4M3 ? 1 : 2));
   return l;
 }
@@ -1544,7 +1549,7 @@ int rpa_mla_sparse_attention(const RpaMlaParams* p, const RpaMlaSparse* s, const
     return fail(RPA_EINVAL_WORKSPACE, "workspace of %zu bytes needed (aligned to 16), %zu given", l.total, p->workspace_bytes);
   const WorkspaceTurn turn(p->workspace);
   char* ws = static_cast<char*>(p->workspace);
-  rpa::SparseMlaArgs a;
+  rpa::SparseMlaArgs a = {};
   a.pt.kv_lens = p->kv_lens;
   a.pt.page_indices = p->page_indices;
   a.pt.cu_q_lens = p->cu_q_lens;
@@ -1567,16 +1572,14 @@ int rpa_mla_sparse_attention(const RpaMlaParams* p, const RpaMlaSparse* s, const
   a.fp8 = p->cache_dtype == RPA_KV_FP8_E4M3 ? 1 : 0;
   a.new_kv_c = static_cast<const char*>(new_kv_c);
   a.new_k_pe = static_cast<const char*>(new_k_pe);
-  a.table = reinterpret_cast<int32_t*>(ws + l.table);
+  a.table = reinterpret_cast<int32_t*>((reinterpret_cast<uintptr_t>(ws + l.table) + kLine - 1) & ~(uintptr_t)(kLine - 1));
+  a.table_stride = v.pages_per_seq;
   a.kv_len_out = reinterpret_cast<int32_t*>(ws + l.kv_lens);
-  a.cu_q_out = reinterpret_cast<int32_t*>(ws + l.cu_q);
-  a.extra = ws + l.extra;
-  if ((rc = check_hip(rpa::launch_sparse_table(a, static_cast<hipStream_t>(stream)), "rpa sparse table")) != RPA_OK) return rc;
+  a.extra = rows ? ws + l.extra : nullptr;
   v.kv_lens = a.kv_len_out;
-  v.cu_q_lens = a.cu_q_out;
   v.page_indices = a.table;
   v.workspace_bytes = l.kv_lens;
-  return mla_run(&v, stream, false, rows ? a.extra : nullptr);
+  return mla_run(&v, stream, false, nullptr, nullptr, &a);
 }
 
 }  // extern "C"

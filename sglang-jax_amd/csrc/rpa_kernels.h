@@ -165,6 +165,28 @@ struct GatherArgs {
   int32_t max_tokens;
 };
 
+// Sparse MLA: every query token is a decode row over a page table of its own, which the attention kernels write (rpa_dsa.h).
+struct SparseMlaArgs {
+  PageTable pt;              // of the batch: ragged table (cu_kv_lens)
+  int32_t num_page_indices;  // entries of pt.page_indices
+  int32_t num_tokens;
+  int32_t num_seqs;
+  const int32_t* topk;       // [T, topk_stride], the first topk_count of a row are read; -1 = unused
+  int32_t topk_count, topk_stride;
+  int32_t topk_is_pages;     // entries are pages of the sequence, not tokens
+  int32_t pages_per_seq;
+  int32_t k_pages_max;       // > 0: tables of whole pages; 0: tables of single rows
+  int32_t total_pages;
+  char* cache;               // whole pages: the new rows are written here
+  int32_t row_stride, rope_offset, fp8;
+  const char* new_kv_c;      // [T, 512] in the cache's element type, or nullptr: the cache holds them already
+  const char* new_k_pe;      // [T, 64]
+  int32_t* table;            // [T, table_stride], k_pages_max or topk_count entries of each row
+  int32_t table_stride;      // a multiple of 32: no two rows share a cache line
+  int32_t* kv_len_out;       // [T]
+  char* extra;               // single rows: [T + 1] rows, the new ones and one of zeros
+};
+
 struct MlaDecodeArgs {
   const uint16_t* ql_nope;  // [T, Hq, lkv]
   const uint16_t* q_pe;     // [T, Hq, rope]
@@ -198,6 +220,7 @@ struct MlaDecodeArgs {
   // sequence rows: the new tokens' latents, [T, 512] and [T, 64] in the cache's type, which the kernels put into the cache; or nullptr
   const char* new_kv_c;
   const char* new_k_pe;
+  SparseMlaArgs sparse;  // sparse.topk: the rows' page tables and lengths (pt) are still to be written, new rows are sparse.new_kv_c
 };
 
 struct MlaWriteArgs {
@@ -211,27 +234,6 @@ struct MlaWriteArgs {
   int32_t row_stride;
   int32_t rope_offset;
   const int32_t* dist;  // device i32[3] or nullptr: when given, num_seqs is only a bound on dist[2]
-};
-
-struct SparseMlaArgs {
-  PageTable pt;              // of the batch: ragged table (cu_kv_lens)
-  int32_t num_page_indices;  // entries of pt.page_indices
-  int32_t num_tokens;
-  int32_t num_seqs;
-  const int32_t* topk;       // [T, topk_stride], the first topk_count of a row are read; -1 = unused
-  int32_t topk_count, topk_stride;
-  int32_t topk_is_pages;     // entries are pages of the sequence, not tokens
-  int32_t pages_per_seq;
-  int32_t k_pages_max;       // > 0: tables of whole pages; 0: tables of single rows
-  int32_t total_pages;
-  char* cache;               // whole pages: the new rows are written here
-  int32_t row_stride, rope_offset, fp8;
-  const char* new_kv_c;      // [T, 512] in the cache's element type, or nullptr: the cache holds them already
-  const char* new_k_pe;      // [T, 64]
-  int32_t* table;            // [T, k_pages_max or topk_count]
-  int32_t* kv_len_out;       // [T]
-  int32_t* cu_q_out;         // [T + 1]
-  char* extra;               // single rows: [T + 1] rows, the new ones and one of zeros
 };
 
 hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream);
@@ -259,7 +261,6 @@ unsigned mla_shape_skip(const MlaDecodeArgs& a, const Tuning& tune);
 // how query tokens of a chunk share a workgroup (0: they do not; 1, 2: eight waves; 3: wide workgroups)
 int mla_token_group_mode(const MlaDecodeArgs& a, const Tuning& tune, const ShapeRule& shape);
 bool mla_takes_wide_p16(const MlaDecodeArgs& a, bool heads_in_128s);
-hipError_t launch_sparse_table(const SparseMlaArgs& a, hipStream_t stream);
 hipError_t launch_mla_kv_write(const MlaWriteArgs& a, hipStream_t stream);
 
 }  // namespace rpa

@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "rpa_common.h"
+#include "rpa_dsa.h"
 #include "rpa_kernels.h"
 #include "rpa_shapes.h"
 #include "rpa_tuning.h"
@@ -353,7 +354,7 @@ __device__ __forceinline__ MlaRow mla_row(const MlaDecodeArgs& a, int row) {
   } else {
     r.seq = row;
     r.kv_len = (row < num_seqs) ? a.pt.kv_lens[row] : 0;
-    r.tq = a.pt.cu_q_lens[row];
+    r.tq = a.sparse.topk ? row : a.pt.cu_q_lens[row];
     r.valid = row < num_seqs;
   }
   return r;
@@ -432,10 +433,11 @@ __device__ __forceinline__ void put_new_row(const MlaDecodeArgs& a, int seq, int
 // masks with that.  Tokens of one sequence follow each other in q and out, so (token, head) of the group is
 // "head" 16 w + c of a 128-head row at mr.tq: every address below stays what it was.  The reference's
 // kernel shares each latent tile among 16 query tokens the same way (kernels/mla/v2/kernel.py:1448-1459).
-template <bool UNIFORM, bool CAP, bool PIPE = false, bool FP8 = false, int DS = 1, bool TG = false>
+// IDS: the first 64 pages' ids are in first_ids already, a lane each.
+template <bool UNIFORM, bool CAP, bool PIPE = false, bool FP8 = false, int DS = 1, bool TG = false, bool IDS = false>
 __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow mr, int head_base, int t_lo,
                                             int t_begin, int t_end, const MlaDest dest, char* slot0, char* slot1,
-                                            char* slot2, char* slot3, int group_tokens = 1) {
+                                            char* slot2, char* slot3, int group_tokens = 1, int first_ids = 0) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -480,7 +482,12 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
     // (by name, wait included: the compiler would wait for every load in flight at each use)
     asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=v"(page_ids) : "v"(at) : "memory");
   };
-  if constexpr (UNIFORM && DS > 1) fetch_page_ids(page_slot(src, t_begin));
+  if constexpr (IDS) {
+    page_ids = first_ids;
+    page_ids_first = page_slot(src, t_begin);
+  } else if constexpr (UNIFORM && DS > 1) {
+    fetch_page_ids(page_slot(src, t_begin));
+  }
   auto page_of = [&](int tb) -> int {
     if constexpr (UNIFORM) {
       tb = min(tb, src.last_tok & ~(kTok - 1));
@@ -872,7 +879,8 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
 }
 
 // ---- fixed split plan: grid = (max_splits * rows, 1, head groups of 128); block = 512 threads
-template <bool UNIFORM, bool CAP, bool PIPE = false, bool FP8 = false, int DS = 1>
+// SPARSE: the rows' page tables are written here first (rpa_dsa.h).
+template <bool UNIFORM, bool CAP, bool PIPE = false, bool FP8 = false, int DS = 1, bool SPARSE = false>
 __global__ __launch_bounds__(512, 2) void rpa_mla_decode_kernel(const MlaDecodeArgs a) {
   // three separate arrays: lets the compiler see that a copy into one slot does not alias the
   // reads of another, so it does not drain the vector-memory queue before LDS reads
@@ -883,6 +891,20 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_decode_kernel(const MlaDecodeA
   const int nsp = max(a.max_splits, 1);  // grid.x = max_splits * rows, splits fastest
   int row_id = (int)(blockIdx.x / (unsigned)nsp);
   const int split = (int)blockIdx.x - row_id * nsp;
+  MlaDest dest;
+  dest.final_rows = a.max_splits == 1;
+  if constexpr (SPARSE) {
+    sparse::Piece p = {};
+    constexpr bool kIds = UNIFORM && DS > 1;
+    if (!sparse::begin_piece<512, kIds>(a, row_id, split, slot0, p)) return;
+    const MlaRow mr = {row_id, p.kv_len, row_id, true};
+    dest.base = ((int64_t)row_id * a.max_splits + split) * a.Hq;
+    MlaDecodeArgs b = a;
+    // (behind the table's barrier: page ids are read as what nobody writes, and could be asked for in front of it)
+    asm volatile("" : "+s"(b.pt.page_indices)::"memory");
+    mla_segment<UNIFORM, CAP, PIPE, FP8, DS, false, kIds>(b, mr, blockIdx.z * 128, 0, p.t_begin, p.t_end, dest, slot0, slot1, slot2, slot3, 1, p.page_ids);
+    return;
+  }
   if (a.rows_are_tokens) row_id = a.num_rows - 1 - row_id;
   const MlaRow mr = mla_row(a, row_id);
   if (!mr.valid) return;
@@ -893,8 +915,6 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_decode_kernel(const MlaDecodeA
   const int t_begin = t0 + split * a.chunk;
   if (t_begin >= kv_len) return;
   const int t_end = (split == a.max_splits - 1) ? kv_len : min(kv_len, t_begin + a.chunk);
-  MlaDest dest;
-  dest.final_rows = a.max_splits == 1;
   dest.base = ((int64_t)row_id * a.max_splits + split) * a.Hq;
   if (a.new_kv_c && t_end == kv_len) {
     put_new_row<FP8>(a, mr.seq, kv_len);
@@ -1329,12 +1349,24 @@ __global__ __launch_bounds__(256, 1) void rpa_mla_token_group_wide_kernel(const 
 }
 
 // ---- fixed split plan, wide workgroups: grid = (max_splits * rows, 1, head groups of 128); block = 256 threads
-template <bool M32, bool P16 = false>
+template <bool M32, bool P16 = false, bool SPARSE = false>
 __global__ __launch_bounds__(256, 1) void rpa_mla_decode_wide_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char ring[4 * kSlotB];
   const int nsp = max(a.max_splits, 1);  // grid.x = max_splits * rows, splits fastest
   int row_id = (int)(blockIdx.x / (unsigned)nsp);
   const int split = (int)blockIdx.x - row_id * nsp;
+  MlaDest dest;
+  dest.final_rows = a.max_splits == 1;
+  if constexpr (SPARSE) {
+    sparse::Piece p = {};
+    if (!sparse::begin_piece<256>(a, row_id, split, ring, p)) return;
+    const MlaRow mr = {row_id, p.kv_len, row_id, true};
+    dest.base = ((int64_t)row_id * a.max_splits + split) * a.Hq;
+    MlaDecodeArgs b = a;
+    asm volatile("" : "+s"(b.pt.page_indices)::"memory");  // (as above)
+    mla_segment_wide<M32, false, P16>(b, mr, blockIdx.z * 128, 0, p.t_begin, p.t_end, dest, ring);
+    return;
+  }
   if (a.rows_are_tokens) row_id = a.num_rows - 1 - row_id;
   const MlaRow mr = mla_row(a, row_id);
   if (!mr.valid) return;
@@ -1345,8 +1377,6 @@ __global__ __launch_bounds__(256, 1) void rpa_mla_decode_wide_kernel(const MlaDe
   const int t_begin = t0 + split * a.chunk;
   if (t_begin >= kv_len) return;
   const int t_end = (split == a.max_splits - 1) ? kv_len : min(kv_len, t_begin + a.chunk);
-  MlaDest dest;
-  dest.final_rows = a.max_splits == 1;
   dest.base = ((int64_t)row_id * a.max_splits + split) * a.Hq;
   if (a.new_kv_c && t_end == kv_len) {
     put_new_row<false>(a, mr.seq, kv_len);
@@ -1765,12 +1795,30 @@ static void launch_mla_combine(const MlaDecodeArgs& a, hipStream_t stream) {
 #undef RPA_MLA_COMBINE
 }
 
+// The kernels of the fixed plan, of the same with the rows' tables still to be written, and of the balanced plan.
+static dim3 rows_grid(const MlaDecodeArgs& a) {
+  return dim3((unsigned)max(a.max_splits, 1) * (unsigned)a.num_rows, 1, (a.Hq + 127) / 128);
+}
+template <bool UNIFORM, bool CAP, bool PIPE = false, bool FP8 = false, int DS = 1>
+static void launch_rows(const MlaDecodeArgs& a, hipStream_t stream) {
+  if (a.sparse.topk) hipLaunchKernelGGL((rpa_mla_decode_kernel<UNIFORM, CAP, PIPE, FP8, DS, true>), rows_grid(a), dim3(512), 0, stream, a);
+  else hipLaunchKernelGGL((rpa_mla_decode_kernel<UNIFORM, CAP, PIPE, FP8, DS>), rows_grid(a), dim3(512), 0, stream, a);
+}
+template <bool M32, bool P16>
+static void launch_wide_rows(const MlaDecodeArgs& a, hipStream_t stream) {
+  if (a.sparse.topk) hipLaunchKernelGGL((rpa_mla_decode_wide_kernel<M32, P16, true>), rows_grid(a), dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((rpa_mla_decode_wide_kernel<M32, P16>), rows_grid(a), dim3(256), 0, stream, a);
+}
+template <bool UNIFORM, bool CAP, bool PIPE = false, bool FP8 = false, int DS = 1>
+static void launch_shares(const MlaDecodeArgs& a, hipStream_t stream) {
+  hipLaunchKernelGGL((rpa_mla_balanced_kernel<UNIFORM, CAP, PIPE, FP8, DS>), dim3(a.num_wgs), dim3(512), 0, stream, a);
+}
+
 hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   if (a.num_rows <= 0) return hipSuccess;
-  const int head_groups = (a.Hq + 127) / 128;
   if ((int64_t)a.max_splits * a.num_rows > 0x7fffffffLL || (int64_t)a.Hq * a.num_rows > 0x7fffffffLL)
     return hipErrorInvalidValue;
-  const dim3 grid((unsigned)max(a.max_splits, 1) * (unsigned)a.num_rows, 1, head_groups), block(512);
+  const dim3 block(512);
   const bool uniform = (a.pt.page_size % kTok) == 0;
   const bool cap = a.sm.soft_cap != 0.f;
   // the kernel family by shape (rpa_shapes.h): wide workgroups and the assembly tile loops need whole tiles inside
@@ -1802,28 +1850,27 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     return hipGetLastError();
   }
   if (ds != 1) {
-#define RPA_MLA_DS_U(KERNEL, GRID, U, F8)                                                                            \
-  do {                                                                                                                \
-    if (ds == 8) hipLaunchKernelGGL((KERNEL<U, false, false, F8, 8>), GRID, block, 0, stream, a);                    \
-    else if (ds == 4) hipLaunchKernelGGL((KERNEL<U, false, false, F8, 4>), GRID, block, 0, stream, a);               \
-    else hipLaunchKernelGGL((KERNEL<U, false, false, F8, 2>), GRID, block, 0, stream, a);                            \
+#define RPA_MLA_DS_U(LAUNCH, U, F8)                              \
+  do {                                                           \
+    if (ds == 8) LAUNCH<U, false, false, F8, 8>(a, stream);      \
+    else if (ds == 4) LAUNCH<U, false, false, F8, 4>(a, stream); \
+    else LAUNCH<U, false, false, F8, 2>(a, stream);              \
   } while (0)
-#define RPA_MLA_DS(KERNEL, GRID, F8)                                                                                 \
-  do {                                                                                                                \
-    if (uniform) RPA_MLA_DS_U(KERNEL, GRID, true, F8);                                                                \
-    else RPA_MLA_DS_U(KERNEL, GRID, false, F8);                                                                       \
+#define RPA_MLA_DS(LAUNCH, F8)                    \
+  do {                                            \
+    if (uniform) RPA_MLA_DS_U(LAUNCH, true, F8);  \
+    else RPA_MLA_DS_U(LAUNCH, false, F8);         \
   } while (0)
     if (a.balanced) {
-      const dim3 bgrid(a.num_wgs);
-      if (a.fp8) RPA_MLA_DS(rpa_mla_balanced_kernel, bgrid, true);
-      else RPA_MLA_DS(rpa_mla_balanced_kernel, bgrid, false);
+      if (a.fp8) RPA_MLA_DS(launch_shares, true);
+      else RPA_MLA_DS(launch_shares, false);
       hipError_t eb = hipGetLastError();
       if (eb != hipSuccess) return eb;
       launch_mla_combine(a, stream);
       return hipGetLastError();
     }
-    if (a.fp8) RPA_MLA_DS(rpa_mla_decode_kernel, grid, true);
-    else RPA_MLA_DS(rpa_mla_decode_kernel, grid, false);
+    if (a.fp8) RPA_MLA_DS(launch_rows, true);
+    else RPA_MLA_DS(launch_rows, false);
 #undef RPA_MLA_DS
 #undef RPA_MLA_DS_U
     hipError_t es = hipGetLastError();
@@ -1836,15 +1883,14 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   }
   if (a.fp8) {  // e4m3 caches
     if (a.balanced) {
-      const dim3 bgrid(a.num_wgs);
-      if (pipe) {
-        hipLaunchKernelGGL((rpa_mla_balanced_kernel<true, false, true, true>), bgrid, block, 0, stream, a);
+        if (pipe) {
+        launch_shares<true, false, true, true>(a, stream);
       } else if (uniform) {
-        if (cap) hipLaunchKernelGGL((rpa_mla_balanced_kernel<true, true, false, true>), bgrid, block, 0, stream, a);
-        else hipLaunchKernelGGL((rpa_mla_balanced_kernel<true, false, false, true>), bgrid, block, 0, stream, a);
+        if (cap) launch_shares<true, true, false, true>(a, stream);
+        else launch_shares<true, false, false, true>(a, stream);
       } else {
-        if (cap) hipLaunchKernelGGL((rpa_mla_balanced_kernel<false, true, false, true>), bgrid, block, 0, stream, a);
-        else hipLaunchKernelGGL((rpa_mla_balanced_kernel<false, false, false, true>), bgrid, block, 0, stream, a);
+        if (cap) launch_shares<false, true, false, true>(a, stream);
+        else launch_shares<false, false, false, true>(a, stream);
       }
       hipError_t eb = hipGetLastError();
       if (eb != hipSuccess) return eb;
@@ -1852,13 +1898,13 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
       return hipGetLastError();
     }
     if (pipe) {
-      hipLaunchKernelGGL((rpa_mla_decode_kernel<true, false, true, true>), grid, block, 0, stream, a);
+      launch_rows<true, false, true, true>(a, stream);
     } else if (uniform) {
-      if (cap) hipLaunchKernelGGL((rpa_mla_decode_kernel<true, true, false, true>), grid, block, 0, stream, a);
-      else hipLaunchKernelGGL((rpa_mla_decode_kernel<true, false, false, true>), grid, block, 0, stream, a);
+      if (cap) launch_rows<true, true, false, true>(a, stream);
+      else launch_rows<true, false, false, true>(a, stream);
     } else {
-      if (cap) hipLaunchKernelGGL((rpa_mla_decode_kernel<false, true, false, true>), grid, block, 0, stream, a);
-      else hipLaunchKernelGGL((rpa_mla_decode_kernel<false, false, false, true>), grid, block, 0, stream, a);
+      if (cap) launch_rows<false, true, false, true>(a, stream);
+      else launch_rows<false, false, false, true>(a, stream);
     }
     hipError_t ef = hipGetLastError();
     if (ef != hipSuccess) return ef;
@@ -1887,9 +1933,9 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     return hipGetLastError();
   }
   if (wide) {
-    if (m32) hipLaunchKernelGGL(rpa_mla_decode_wide_kernel<true>, grid, dim3(256), 0, stream, a);
-    else if (p16) hipLaunchKernelGGL((rpa_mla_decode_wide_kernel<false, true>), grid, dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL(rpa_mla_decode_wide_kernel<false>, grid, dim3(256), 0, stream, a);
+    if (m32) launch_wide_rows<true, false>(a, stream);
+    else if (p16) launch_wide_rows<false, true>(a, stream);
+    else launch_wide_rows<false, false>(a, stream);
     hipError_t ew = hipGetLastError();
     if (ew != hipSuccess) return ew;
     if (a.max_splits > 1) {
@@ -1899,15 +1945,14 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     return ew;
   }
   if (a.balanced) {
-    const dim3 bgrid(a.num_wgs);
     if (pipe) {
-      hipLaunchKernelGGL((rpa_mla_balanced_kernel<true, false, true>), bgrid, block, 0, stream, a);
+      launch_shares<true, false, true>(a, stream);
     } else if (uniform) {
-      if (cap) hipLaunchKernelGGL((rpa_mla_balanced_kernel<true, true>), bgrid, block, 0, stream, a);
-      else hipLaunchKernelGGL((rpa_mla_balanced_kernel<true, false>), bgrid, block, 0, stream, a);
+      if (cap) launch_shares<true, true>(a, stream);
+      else launch_shares<true, false>(a, stream);
     } else {
-      if (cap) hipLaunchKernelGGL((rpa_mla_balanced_kernel<false, true>), bgrid, block, 0, stream, a);
-      else hipLaunchKernelGGL((rpa_mla_balanced_kernel<false, false>), bgrid, block, 0, stream, a);
+      if (cap) launch_shares<false, true>(a, stream);
+      else launch_shares<false, false>(a, stream);
     }
     hipError_t eb = hipGetLastError();
     if (eb != hipSuccess) return eb;
@@ -1915,13 +1960,13 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     return hipGetLastError();
   }
   if (pipe) {
-    hipLaunchKernelGGL((rpa_mla_decode_kernel<true, false, true>), grid, block, 0, stream, a);
+    launch_rows<true, false, true>(a, stream);
   } else if (uniform) {
-    if (cap) hipLaunchKernelGGL((rpa_mla_decode_kernel<true, true>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((rpa_mla_decode_kernel<true, false>), grid, block, 0, stream, a);
+    if (cap) launch_rows<true, true>(a, stream);
+    else launch_rows<true, false>(a, stream);
   } else {
-    if (cap) hipLaunchKernelGGL((rpa_mla_decode_kernel<false, true>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((rpa_mla_decode_kernel<false, false>), grid, block, 0, stream, a);
+    if (cap) launch_rows<false, true>(a, stream);
+    else launch_rows<false, false>(a, stream);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

@@ -129,7 +129,24 @@ def test_page_level_selection(pkg, wl, gpu, precomputed):
 def test_selections_of_every_shape(pkg, wl, gpu, level, P, Hq, k, dtype):
     """Head counts of every workgroup shape, pages below and above a tile, selections that end inside one, rows cut in pieces;
     lengths from one token to far more than the selection."""
-    kv_lens, kp = [1, 2, 31, P, P + 1, 700, 5003], 40
+    check_selections(pkg, wl, gpu, level, P, Hq, k, dtype, [1, 2, 31, P, P + 1, 700, 5003], 40)
+
+
+@pytest.mark.parametrize("level,P,Hq,k,dtype,kv_lens,kp", [
+    # sequences of 2048 pages (whose ids wait in LDS) and of more, and more of them than a wave has lanes
+    ("page", 16, 16, 300, "bf16", [32768, 5, 900], 40), ("page", 16, 16, 300, "bf16", [32769, 40000, 5, 900], 40),
+    ("page", 32, 64, 2048, "e4m3", [70000, 33, 3000], 70), ("page", 64, 16, 64, "bf16", list(range(1, 140)), 4),
+    # pieces of more than 64 pages, and a last one that ends in its 64th
+    ("page", 32, 16, 2048, "bf16", [4500 + i for i in range(150)], 130), ("page", 32, 32, 2048, "bf16", [2048] * 256, 64),
+    # selections of more than one batch, unused entries between valid ones aside
+    ("page", 64, 128, 2600, "bf16", [2600, 6000, 1], 64), ("token", 16, 64, 2600, "bf16", [2600, 2599, 6000, 1], 0),
+    ("token", 16, 16, 40, "e4m3", list(range(1, 140)), 0),
+])
+def test_tables_of_every_size(pkg, wl, gpu, level, P, Hq, k, dtype, kv_lens, kp):
+    check_selections(pkg, wl, gpu, level, P, Hq, k, dtype, kv_lens, kp)
+
+
+def check_selections(pkg, wl, gpu, level, P, Hq, k, dtype, kv_lens, kp):
     b = batch(wl, kv_lens, P, 83, Hq=Hq)
     topk_np = draw_topk(kv_lens, k, 8)
     S, pps = len(kv_lens), -(-max(kv_lens) // P)
