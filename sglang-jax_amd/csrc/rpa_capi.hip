@@ -534,7 +534,9 @@ size_t rows256_workspace(const RpaParams* p) {
 }
 
 // head_dim 256: every query token of sequences [seq_begin, seq_end) is a row of the row kernel
-int rows256(const RpaParams* p, int seq_begin, int seq_end, void* stream, int dist_role = 0) {
+// (keys / values: of decode rows whose tokens the kernel is to write)
+int rows256(const RpaParams* p, int seq_begin, int seq_end, void* stream, int dist_role = 0, const void* keys = nullptr,
+            const void* values = nullptr) {
   if (seq_end <= seq_begin) return RPA_OK;
   rpa::DecodeArgs a = {};
   a.q = static_cast<const uint16_t*>(p->q);
@@ -551,6 +553,8 @@ int rows256(const RpaParams* p, int seq_begin, int seq_end, void* stream, int di
   a.q_dim = q_dim_of(p);
   a.fp8 = p->kv_dtype == RPA_KV_FP8_E4M3;
   a.dist = dist_role ? p->distribution : nullptr;
+  a.new_k = static_cast<const char*>(keys);
+  a.new_v = static_cast<const char*>(values);
   // decode rows are one token each; other sequences are bounded by the tokens of the call
   const int rows = (dist_role != 2 && seq_end <= p->decode_end) ? (seq_end - seq_begin) : p->num_tokens;
   if (seq_begin == 0 && seq_end == p->decode_end && p->mask_mode != RPA_MASK_CUSTOM) {
@@ -827,7 +831,7 @@ static int decode_rows(const RpaParams* p_in, const void* keys, const void* valu
   const RpaParams* p = &pv;
   if (p->decode_end <= 0) return RPA_OK;
   if (p->mask_mode == RPA_MASK_CUSTOM) return RPA_OK;  // masked rows all go through the prefill kernel
-  if (p->head_dim == 256) return rows256(p, 0, p->decode_end, stream, p->distribution ? 1 : 0);
+  if (p->head_dim == 256) return rows256(p, 0, p->decode_end, stream, p->distribution ? 1 : 0, keys, values);
   const DecodeChoice choice = decode_choice(p, token_rows);
   const SplitPlan& sp = choice.sp;
   rpa::DecodeArgs a;
@@ -1082,9 +1086,16 @@ static bool rows_take_new_tokens(const RpaParams* p) {
   return d == p->head_dim || (d == 64 && p->kv_dtype == RPA_KV_BF16 && rpa::tuning().decode_merge_in_kernel == 0);
 }
 
-// Whether the decode kernels read their rows' new tokens from the caller's keys / values and write them into the cache
-// (not the 256-wide rows, nor the balanced plan on pages that are no multiple of 16 tokens).
+// Whether the decode kernels take their rows' new tokens from the caller's keys / values and write them into the cache
+// (not the balanced plan on pages that are no multiple of 16 tokens).  256-wide rows: up to 768 MB of cache, where a launch in front is a
+// part of the call that one notices (5 rows of 1396..8992 e4m3 tokens x 2 heads 22.2 -> 17.6 us, one of 700 bf16 x 8 heads 11.9 -> 9.7,
+// 32 of 300..3000 x 4 heads 50.6 -> 47.6, 64 of 300..3000 e4m3 x 8 heads, 0.4 GB, 95.6 -> 89.4, 180 of 500..3000, 0.6 GB, 244 -> 239); the
+// same on bf16, 1.3 GB, 447 -> 447.5.
 static bool decode_takes_new_tokens(const RpaParams* p_in) {
+  if (p_in->head_dim == 256) {
+    const RpaParams p = planning_view(p_in);
+    return p_in->mask_mode != RPA_MASK_CUSTOM && decode_kv_bytes(&p) <= (768ll << 20);
+  }
   if (p_in->head_dim != 128 || p_in->mask_mode == RPA_MASK_CUSTOM || !rows_take_new_tokens(p_in)) return false;
   if (p_in->page_size % 16 == 0) return true;
   const RpaParams p = planning_view(p_in);

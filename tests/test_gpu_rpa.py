@@ -2128,3 +2128,36 @@ def test_even_rows_fill_the_chip(pkg, wl, gpu, monkeypatch, rows, Hkv, lo, hi, f
         other.params.workspace_bytes = least - 1
         with pytest.raises(ValueError, match="workspace"):
             other.attention()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,P,D,on_device,kv_lens", [
+    (40, 2, 64, 256, False, [1, 31, 64, 65, 700]),        # 20 query heads per kv head: two waves read each row
+    (16, 2, 64, 192, False, [1, 33, 128, 129, 2500]),     # narrow rows: their slots end in zeros
+    (8, 8, 1, 256, True, [5, 32, 64, 97]), (4, 4, 128, 256, True, [1, 128, 129, 5000]),
+])
+def test_head_dim_256_rows_bring_their_tokens(pkg, wl, gpu, Hq, Hkv, P, D, on_device, kv_lens, fp8):
+    """256-wide decode rows put their new tokens into the cache themselves: rows that end at the edges of blocks and pages, whole and in
+    pieces; the slots held NaN before."""
+    say(f"256 new tokens {Hq}/{Hkv} P={P} D={D} fp8={fp8}")
+    b = wl.make_batch("new256", [1] * len(kv_lens), kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=256, page_size=P, seed=17,
+                      kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+    if D < 256:
+        b.kv_cache.view(torch.uint8 if fp8 else torch.int16)[..., D:] = 0
+        b.q[..., D:] = 0
+    want = oracle_out(b)[..., :D]
+    keys, values, cache = with_new_tokens(b)
+    g, cache = b.to(gpu), cache.to(gpu)
+    bounds = {} if on_device else dict(max_kv_len=max(kv_lens), max_q_len=1, host_kv_lens=b.kv_lens.numpy())
+    out, after = pkg.ragged_paged_attention(
+        g.q[..., :D].contiguous(), keys[..., :D].contiguous().to(gpu), values[..., :D].contiguous().to(gpu), cache, g.kv_lens, g.page_indices,
+        g.cu_q_lens, g.cu_kv_lens, g.distribution if on_device else b.distribution.numpy(), sm_scale=b.sm_scale, k_scale=g.k_scale,
+        v_scale=g.v_scale, **bounds)
+    torch.cuda.synchronize()
+    assert_parity(out.cpu().float(), want.float(), **(FP8_TOL if fp8 else BF16_TOL))
+    bits = torch.uint8 if fp8 else torch.int16
+    got, full, expect = after.cpu().view(bits), b.kv_cache.view(bits), with_new_tokens(b)[2].view(bits).clone()
+    for i, kv in enumerate(kv_lens):
+        page = int(b.page_indices[int(b.cu_kv_lens[i]) // P + (kv - 1) // P])
+        expect[page, (kv - 1) % P] = full[page, (kv - 1) % P]
+    assert torch.equal(got, expect)
