@@ -956,34 +956,65 @@ __device__ __forceinline__ int mask_owner_of_token(const int32_t* cu_q_lens, int
   return lo;
 }
 
+// grid = (query tokens, workgroups of a row, kMaskWords words at a time each); a wave has eight words, requested together.
+// What bounds it: round trips to memory, so a workgroup has one for its words (all of a row in one workgroup, as it was first,
+// were up to eight in a chain), and up to 63 sequences are searched, and where the row's words begin is worked out, in one.
+// 6 verify steps of 4 tokens on 4421..15445 x 32 / 8 heads 112.4 -> 89.6 us (the call), 21 of 4 on 591..8700 122.3 -> 111.2, one of 8 on
+// 16000 x 8 / 1 heads 50.5 -> 34.3.  Some 2048 workgroups at most: the bound on the lengths may be far above them, and those that find
+// nothing are not free.
+constexpr int kMaskWords = 32;
 __global__ __launch_bounds__(256) void rpa_mask_bits_kernel(const PrefillArgs a) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // (masked calls run every sequence through the prefill kernels; with the composition on the device the number
   // of sequences is only a bound)
-  const int seq_end = a.dist ? min(a.seq_end, a.dist[2]) : a.seq_end;
-  const int token = a.pt.cu_q_lens[a.seq_begin] + (int)blockIdx.x;
-  if (token >= a.pt.cu_q_lens[seq_end]) return;
-  const int seq = mask_owner_of_token(a.pt.cu_q_lens, seq_end, token);
-  const int kv_len = a.pt.kv_lens[seq];
-  const int width = a.sm.mask_rows_page_aligned ? (a.pt.cu_kv_lens[seq + 1] - a.pt.cu_kv_lens[seq]) : kv_len;
+  int seq_end = a.seq_end, token, kv_len, width;
   // where the sequence's rows start: given, or the sum over the sequences before it (cheap beside the rows themselves, and
   // the caller is spared a scan of its own)
   int64_t first = 0;
-  if (a.sm.cu_mask_lens) {
-    first = a.sm.cu_mask_lens[seq];
-  } else {
-    for (int s = (int)(threadIdx.x & 63); s < seq; s += 64) {
-      const int n = a.pt.cu_q_lens[s + 1] - a.pt.cu_q_lens[s];
-      first += (int64_t)n * (a.sm.mask_rows_page_aligned ? a.pt.cu_kv_lens[s + 1] - a.pt.cu_kv_lens[s] : a.pt.kv_lens[s]);
-    }
+  if (seq_end < 64) {  // a sequence per lane
+    const int s = min(lane, a.seq_end), own = min(lane, a.seq_end - 1);
+    const int seqs_now = a.dist ? scalar_load_i32(a.dist + 2) : seq_end;
+    const int q = a.pt.cu_q_lens[s], kv = a.pt.kv_lens[own];
+    const int pages = a.sm.mask_rows_page_aligned ? a.pt.cu_kv_lens[s] : 0;
+    const int given = a.sm.cu_mask_lens ? a.sm.cu_mask_lens[own] : 0;
+    seq_end = max(min(seq_end, seqs_now), 0);
+    token = __builtin_amdgcn_readlane(q, a.seq_begin) + (int)blockIdx.x;
+    if (token >= __builtin_amdgcn_readlane(q, seq_end)) return;
+    const int seq = max(__builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < seq_end && q <= token)) - 1, 0);
+    const int tokens = __shfl_down(q, 1) - q, row_width = a.sm.mask_rows_page_aligned ? __shfl_down(pages, 1) - pages : kv;
+    kv_len = __builtin_amdgcn_readlane(kv, seq);
+    width = __builtin_amdgcn_readlane(row_width, seq);
+    if (a.sm.cu_mask_lens) {
+      first = __builtin_amdgcn_readlane(given, seq);
+    } else {
+      first = lane < seq ? (int64_t)tokens * row_width : 0;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off);
+      for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off);
+    }
+    first += (int64_t)(token - __builtin_amdgcn_readlane(q, seq)) * width;
+  } else {
+    if (a.dist) seq_end = min(seq_end, a.dist[2]);
+    token = a.pt.cu_q_lens[a.seq_begin] + (int)blockIdx.x;
+    if (token >= a.pt.cu_q_lens[seq_end]) return;
+    const int seq = mask_owner_of_token(a.pt.cu_q_lens, seq_end, token);
+    kv_len = a.pt.kv_lens[seq];
+    width = a.sm.mask_rows_page_aligned ? (a.pt.cu_kv_lens[seq + 1] - a.pt.cu_kv_lens[seq]) : kv_len;
+    if (a.sm.cu_mask_lens) {
+      first = a.sm.cu_mask_lens[seq];
+    } else {
+      for (int s = lane; s < seq; s += 64) {
+        const int n = a.pt.cu_q_lens[s + 1] - a.pt.cu_q_lens[s];
+        first += (int64_t)n * (a.sm.mask_rows_page_aligned ? a.pt.cu_kv_lens[s + 1] - a.pt.cu_kv_lens[s] : a.pt.kv_lens[s]);
+      }
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off);
+    }
+    first += (int64_t)(token - a.pt.cu_q_lens[seq]) * width;
   }
-  const int32_t* row = a.sm.custom_mask + first + (int64_t)(token - a.pt.cu_q_lens[seq]) * width;
+  const int32_t* row = a.sm.custom_mask + first;
   uint64_t* out = a.mask_bits + (int64_t)token * a.mask_pitch;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int words = min((kv_len + 63) >> 6, a.mask_pitch);
-  // eight words of a wave requested at a time: one after the other, a row of 16000 was 60 round trips to memory
-  for (int k0 = wave; k0 < words; k0 += 32) {
+  for (int k0 = (int)blockIdx.y * kMaskWords + wave; k0 < words; k0 += (int)gridDim.y * kMaskWords) {
     int v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -1000,7 +1031,9 @@ __global__ __launch_bounds__(256) void rpa_mask_bits_kernel(const PrefillArgs a)
 
 hipError_t launch_mask_bits(const PrefillArgs& a, hipStream_t stream) {
   if (!a.mask_bits || a.num_tokens <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rpa_mask_bits_kernel, dim3((unsigned)a.num_tokens), dim3(256), 0, stream, a);
+  const int most = std::max(1, 2048 / a.num_tokens);
+  const dim3 grid((unsigned)a.num_tokens, (unsigned)std::min((a.mask_pitch + kMaskWords - 1) / kMaskWords, most));
+  hipLaunchKernelGGL(rpa_mask_bits_kernel, grid, dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

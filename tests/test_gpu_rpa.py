@@ -1572,6 +1572,33 @@ def test_custom_mask_as_bits_equals_the_callers_words(pkg, wl, gpu, monkeypatch,
         monkeypatch.delenv("RPA_PREFILL_SPLITS")
 
 
+@pytest.mark.parametrize("seqs", [1, 62, 63, 64, 130])
+@pytest.mark.parametrize("bound", [5000, 400000])
+def test_mask_bits_of_many_sequences_and_long_rows(pkg, wl, gpu, monkeypatch, seqs, bound):
+    """The pre-pass against the caller's words on both sides of the sequences that a wave searches at once, on rows around the words of
+    a workgroup, and with more words in the bound than workgroups."""
+    kv_lens = [5000, 2047, 2048, 2049, 64, 65][:seqs] + [3 + i for i in range(seqs - 6)]
+    q_lens = [3, 1, 2, 1, 4, 1][:seqs] + [1 + i % 3 for i in range(seqs - 6)]
+    rng = np.random.default_rng(seqs)
+    masks = [(rng.random((ql, kv)) < 0.5).astype(np.int32) for ql, kv in zip(q_lens, kv_lens)]
+    for m in masks:
+        m[:, -1] = 1
+    say(f"mask bits of {seqs} sequences, bound {bound}")
+    b = wl.make_batch("mask_many", q_lens, kv_lens, num_q_heads=4, num_kv_heads=2, head_dim=128, page_size=64, seed=94)
+    g, mask = b.to(gpu), flat_mask(masks).to(gpu)
+
+    def run():
+        out, _ = pkg.ragged_paged_attention(g.q, None, None, g.kv_cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens,
+                                            b.distribution.numpy(), mask, sm_scale=b.sm_scale, causal=0, max_kv_len=bound, max_q_len=4)
+        torch.cuda.synchronize()
+        return out[: sum(q_lens)].cpu()
+
+    monkeypatch.setenv("RPA_MASK_BITS", "0")
+    words = run()
+    monkeypatch.delenv("RPA_MASK_BITS")
+    assert torch.equal(run(), words)
+
+
 @pytest.mark.parametrize("kind", ["soft_cap", "xai_temperature", "custom_mask", "no_mask", "softmax_bf16", "fp8", "fp8_custom_mask"])
 def test_short_chunks_take_the_four_head_tile_in_the_compiled_kernel(pkg, wl, gpu, monkeypatch, kind):
     """The compiled flash kernel (every option the pipelined one does not take) with the same short-chunk tile:
