@@ -15,10 +15,13 @@ The 256 accumulators live in the accumulation registers and are touched by nothi
 instructions (and the rare path); Q^T takes 144 vector registers; one wave per SIMD.
 
 A step runs scores, softmax, second product of one tile in that order, LDS operands requested six fragments
-(twelve matrix instructions) ahead into a ring of eight buffers.  `RPA_MLA_WIDE_X=pipe` generates a loop that
-is software-pipelined across tiles instead (step t issues the scores of tile t + 1 into a second set of score
-registers, interleaved one for one with the softmax of tile t; four operand buffers): measured 4 % slower --
-what bounds a lone wave is the number of instructions it has to issue, not the softmax's place in the step.
+(twelve matrix instructions) ahead into a ring of eight buffers.  The requests run on across the border of two steps: in front of
+the last three fragments of a tile the waves meet, and the next tile's first operands and its scalars travel under what is
+left.  With the meeting at the very end, and the scalars and the first requests behind it, as it was first, the border was a gap in the
+matrix pipe: 4 chunks of 512 tokens on 4096 x 128 heads 1819 -> 1796 us, 7 chunks of 25 .. 235 x 32 heads 353 -> 342, 64 decode rows
+180.6 -> 179.6.  (It gives less than the gap was long: these launches run at 2.0 of 2.4 GHz, the power that they draw decides, and
+what fills the pipe lowers the clock; the matrix instructions alone run at 1.85 GHz.)  A loop that was software-pipelined across tiles,
+scores of tile t + 1 interleaved with the softmax of tile t into registers of their own, was 4 % slower.
 
 The loop runs EVERY tile of a segment, so no compiled code ever holds the accumulators:
   * the reference the probabilities are taken against comes in from the caller (the maximum of the first
@@ -58,10 +61,12 @@ sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
 from gen_prefill_pipe_loop import ACC, Emitter, Ins, rng, valu, vr  # noqa: E402
 
 X = set(os.environ.get("RPA_MLA_WIDE_X", "").split(","))   # timing probes (nocopy, nolds, novalu, norare: wrong results)
-PIPELINED = "pipe" in X      # scores of tile t + 1 under the softmax of tile t (measured slower: off)
-NBUF = 4 if PIPELINED else 8  # operand fragment buffers (the second set of score registers of the pipelined loop pays for four)
-AHEAD = int(os.environ.get("RPA_MLA_WIDE_AHEAD", 3 if PIPELINED else 6))
+NBUF = 8                     # operand fragment buffers
+AHEAD = int(os.environ.get("RPA_MLA_WIDE_AHEAD", 6))
 assert AHEAD < NBUF
+MEET = int(os.environ.get("RPA_MLA_WIDE_MEET", 65))           # the fragment in front of which the waves meet
+COPY_FIRST = int(os.environ.get("RPA_MLA_WIDE_COPY_FIRST", 6))  # the fragment of a step's first copy
+BETWEEN = int(os.environ.get("RPA_MLA_WIDE_BETWEEN", 2))
 WAITGROUP = int(os.environ.get("RPA_MLA_WIDE_WAITGROUP", 4))  # fragments whose data one wait instruction covers
 assert 1 <= WAITGROUP <= AHEAD
 
@@ -75,16 +80,9 @@ O = [ACC, ACC + 128]
 # ---- vector registers
 Q = [0, 72]                  # 18 Q^T operands of 4 per block of heads
 SC = [[144, 148], [152, 156]]            # scores [hb][token block]
-if PIPELINED:
-    SC2 = [[160, 164], [168, 172]]       # the other set (sets alternate per step)
-    P = [176, 180]           # packed probabilities per block of heads
-    E = 184                  # 8 exponent temporaries
-    RING = 192               # NBUF operand buffers of 4
-else:
-    SC2 = SC
-    P = [160, 164]
-    E = 168
-    RING = 176
+P = [160, 164]               # packed probabilities per block of heads
+E = 168                      # 8 exponent temporaries
+RING = 176                   # NBUF operand buffers of 4
 ML = 208                     # one operand of 8: M0, L0, M1, L1, KBASE, VBASE, LO, HI
 M = [208, 210]
 L = [209, 211]
@@ -128,13 +126,14 @@ def mfma(dst, a, b, c):
     return Ins(f"v_mfma_f32_16x16x32_bf16 {vr(dst, 4)}, {vr(a, 4)}, {vr(b, 4)}, {ctext}", "mfma", reads, rng(dst, 4))
 
 
-def ring(f):
-    return RING + 4 * (f % NBUF)
+def ring(f, k=0):
+    """buffer of fragment f of a tile in slot k: a tile has 68, so those of the next one go on where they end"""
+    return RING + 4 * ((68 * k + f) % NBUF)
 
 
-def frag_read(f, kaddr=None):
+def frag_read(f, kaddr=None, k=0):
     """operand fragment f of a tile: 0..35 K of (k-step f >> 1, token block f & 1), 36..67 V^T of dim chunk f - 36"""
-    dst = ring(f)
+    dst = ring(f, k)
     if "nolds" in X:
         return []
     if f < 36:
@@ -152,7 +151,7 @@ def frag_tags(f):
     return [("k", f)] if f < 36 else [("vlo", f), ("vhi", f)]
 
 
-def frag_mfmas(f, sc, p=P):
+def frag_mfmas(f, sc, p=P, k=0):
     """the two matrix instructions (one per block of heads) that consume fragment f; scores go to `sc`.  The first
     instruction of every WAITGROUP-th fragment also waits for the fragments behind it in its group (requested long
     before): one wait instruction per group -- a lone wave pays for every instruction it issues."""
@@ -160,10 +159,10 @@ def frag_mfmas(f, sc, p=P):
     for hb in range(2):
         if f < 36:
             ks, b = f >> 1, f & 1
-            ins = mfma(sc[hb][b], ring(f), Q[hb] + 4 * ks, None if ks == 0 else sc[hb][b])
+            ins = mfma(sc[hb][b], ring(f, k), Q[hb] + 4 * ks, None if ks == 0 else sc[hb][b])
         else:
             j = f - 36
-            ins = mfma(O[hb] + 4 * j, ring(f), p[hb], O[hb] + 4 * j)
+            ins = mfma(O[hb] + 4 * j, ring(f, k), p[hb], O[hb] + 4 * j)
         ins.lds_need = None if "nolds" in X else list(frag_tags(f))
         if hb == 0 and f % WAITGROUP == 0 and ins.lds_need is not None:
             for g in range(f + 1, min(f + WAITGROUP, 68)):
@@ -401,75 +400,76 @@ def again_block(em, k, queue):
     em.raw(f"s_mov_b32 s{AGAIN}, 0")
     em.raw("s_nop 7", "nop")
     em.lds_queue = list(queue)
-    for f in range(36, 68):
-        emit_all(em, frag_mfmas(f, None))
-        if f > 36:
-            emit_all(em, frag_mfmas(f - 1, None, PL))
-        if f + AHEAD < 68:
-            emit_all(em, frag_read(f + AHEAD))
-    emit_all(em, frag_mfmas(67, None, PL))
+    pv_phase(em, k, again=True)
     em.raw(f"s_branch L_again_back_{k}_%=")
 
 
-def qk_phase(em, sc, kaddr, copies, extra=None, into_pv=False):
-    """the 72 matrix instructions of a tile's scores; copy groups and (pipelined loop) vector work in between.
-    `into_pv`: the operand requests run on into the second product's first fragments, which then travel under the
-    softmax"""
-    extra = list(extra or [])
-    copy_at = {2 + 3 * n: n for n in range(COPIES)}
-    for f in range(AHEAD):
-        emit_all(em, frag_read(f, kaddr))
+def qk_phase(em, k, copies, between):
+    """the 72 matrix instructions of a tile's scores, its first AHEAD operands on their way already; `between`: instructions for the
+    places behind the first ones, the copies follow; the operand requests run on into the second product's, which travel under the softmax"""
+    between = list(between)
+    copy_at = {COPY_FIRST + 3 * n: n for n in range(COPIES)}
     for f in range(36):
         cp = copies[copy_at[f]] if (f in copy_at and copies) else None
+        assert not (cp and between)
         if cp:
             em.emit(cp[0])       # m0; the matrix instructions behind it are the wait state its use needs
-        for ins in frag_mfmas(f, sc):
+        for ins in frag_mfmas(f, SC, k=k):
             em.emit(ins)
-            if extra:
-                em.emit(extra.pop(0))
-        if f + AHEAD < (68 if into_pv else 36):
-            emit_all(em, frag_read(f + AHEAD, kaddr))
+            for _ in range(BETWEEN):
+                if between:
+                    em.emit(between.pop(0))
+                    while between and between[0].kind == "label":   # (where a detour comes back to)
+                        em.emit(between.pop(0))
+        emit_all(em, frag_read(f + AHEAD, KADDR, k))
         if cp:
             emit_all(em, cp[1])
-    emit_all(em, extra)
 
 
-def pv_phase(em, prefetched=False):
-    if not prefetched:
-        for f in range(36, 36 + AHEAD):
-            emit_all(em, frag_read(f))
+def pv_phase(em, k, again=False):
+    """the second product.  Before its last fragments the waves meet (meet()), and the next tile's first operands are requested."""
+    asked = 36 + AHEAD
     for f in range(36, 68):
-        emit_all(em, frag_mfmas(f, None))
-        if f + AHEAD < 68:
-            emit_all(em, frag_read(f + AHEAD))
+        if f == 60:
+            em.emit(valu(f"v_add_u32 {vr(KADDR)}, {((k + 1) & 3) * SLOT_B}, {vr(KBASE)}", [KBASE], [KADDR]))
+        if f == MEET:
+            meet(em)
+        want = min(f + AHEAD, 68) if f < MEET else f + AHEAD
+        while asked < want:
+            emit_all(em, frag_read(asked, None, k) if asked < 68 else frag_read(asked - 68, KADDR, k + 1))
+            asked += 1
+        emit_all(em, frag_mfmas(f, None, k=k))
+        if again and f > 36:
+            emit_all(em, frag_mfmas(f - 1, None, PL, k))
+    if again:
+        emit_all(em, frag_mfmas(67, None, PL, k))
+    while asked < 68 + AHEAD:
+        emit_all(em, frag_read(asked - 68, KADDR, k + 1))
+        asked += 1
 
 
-def end_of_step(em):
-    # The next step reads tile t + 1 and (pipelined loop) the K rows of tile t + 2: they have landed once only the
-    # newest copies -- tile t + 3's ten, plus tile t + 2's in the plain loop -- are outstanding.  Every LDS read of
-    # tile t has returned, so its slot may be refilled after the barrier.
-    assert not em.lds_queue
+def meet(em):
+    # Behind the barrier the next tile may be read: it has landed once only the newest copies, those of the two tiles behind it, are
+    # outstanding.  And every LDS read of this tile has returned, so the next step's copies may fill its slot.
     # (Pages of 16: the copy that meets both pages is two instructions, one of them without a lane in three of the waves.  The
     # wait counts it once: whether or not the hardware does so for an instruction without lanes, tile t + 1 has landed.)
-    ahead = COPIES if PIPELINED else 2 * COPIES
-    em.raw("s_waitcnt lgkmcnt(0)" if "novmwait" in X else f"s_waitcnt vmcnt({ahead}) lgkmcnt(0)", "wait")
+    em.raw("s_waitcnt lgkmcnt(0)" if "novmwait" in X else f"s_waitcnt vmcnt({2 * COPIES}) lgkmcnt(0)", "wait")
+    em.lds_queue = []
+    if "nobarrier" not in X:
+        em.raw("s_barrier")
     em.raw(f"s_mov_b32 %[pg], s{PGN}")
     if P16:
         em.raw(f"s_mov_b32 %[pg2], s{PGN2}")
-    if "nobarrier" not in X:
-        em.raw("s_barrier")
-    em.raw("s_add_u32 %[t], %[t], 1")
-    em.raw("s_cmp_lt_i32 %[t], %[t_end]")
 
 
-def step_plain(em, k):
+def step(em, k):
     """tile t in slot k: scores, softmax, second product; tile t + 3 goes to slot (k + 3) & 3"""
     fill = (k + 3) & 3
-    tile_scalars(em, k)
-    em.emit(valu(f"v_add_u32 {vr(KADDR)}, {k * SLOT_B}, {vr(KBASE)}", [KBASE], [KADDR]))
-    em.emit(valu(f"v_add_u32 {vr(VADDR)}, {k * SLOT_B}, {vr(VBASE)}", [VBASE], [VADDR]))
+    scalars = Emitter()
+    tile_scalars(scalars, k)
+    v = valu(f"v_add_u32 {vr(VADDR)}, {k * SLOT_B}, {vr(VBASE)}", [VBASE], [VADDR])
     copies = [] if "nocopy" in X else [(copy_dest(n, fill), copy_load(n)) for n in range(COPIES)]
-    qk_phase(em, SC, KADDR, copies, into_pv=True)
+    qk_phase(em, k, copies, [v] + scalars.out)
     mask_check(em, f"{k}")
     for hb in range(2):
         softmax_and_check(em, k, hb, SC)
@@ -477,62 +477,12 @@ def step_plain(em, k):
     if P16 and "noagain" not in X:
         em.raw(f"s_cmp_lg_u32 s{AGAIN}, 0")
         em.raw(f"s_cbranch_scc1 L_again_{k}_%=")
-    pv_phase(em, prefetched=True)
+    pv_phase(em, k)
     if P16 and "noagain" not in X:
         em.label(f"L_again_back_{k}_%=")
-    end_of_step(em)
+    em.raw("s_add_u32 %[t], %[t], 1")
+    em.raw("s_cmp_lt_i32 %[t], %[t_end]")
     return queue
-
-
-def step_pipelined(em, k):
-    """tile t in slot k (scores in set k & 1): scores of tile t + 1 (slot (k + 1) & 3) into the other set,
-    interleaved with the softmax of tile t; then the second product of tile t"""
-    fill = (k + 3) & 3
-    cur, nxt = (SC, SC2) if k % 2 == 0 else (SC2, SC)
-    tile_scalars(em, k)
-    em.emit(valu(f"v_add_u32 {vr(KADDR2)}, {((k + 1) & 3) * SLOT_B}, {vr(KBASE)}", [KBASE], [KADDR2]))
-    em.emit(valu(f"v_add_u32 {vr(VADDR)}, {k * SLOT_B}, {vr(VBASE)}", [VBASE], [VADDR]))
-    copies = [] if "nocopy" in X else [copy_group(n, fill) for n in range(COPIES)]
-    mask_check(em, f"{k}")
-    # the softmax of block 0, its check and the softmax of block 1 ride on the matrix instructions of the next
-    # tile's scores; a rare path taken in between leaves and re-enters the instruction stream at its label
-    sm0 = [] if "novalu" in X else softmax(0, cur)
-    qk_first = 40   # matrix instructions the first softmax is spread over
-    copy_at = {2 + 3 * n: n for n in range(COPIES)}
-    for f in range(AHEAD):
-        emit_all(em, frag_read(f, KADDR2))
-    issued = 0
-    pending = list(sm0)
-    stage = 0
-    sm1 = None
-    for f in range(36):
-        for ins in frag_mfmas(f, nxt):
-            em.emit(ins)
-            issued += 1
-            if pending:
-                em.emit(pending.pop(0))
-            if stage == 0 and not pending and issued >= len(sm0):
-                # the first block's probabilities are complete: check, row sum, then the second block's softmax
-                if "novalu" not in X and "norare" not in X:
-                    em.raw(f"s_cbranch_vccnz L_rare_{k}_0_%=")
-                em.label(f"L_back_{k}_0_%=")
-                if "novalu" not in X:
-                    em.emit(valu(f"v_add_f32 {vr(L[0])}, {vr(L[0])}, {vr(PS)}", [L[0], PS], [L[0]]))
-                    pending = softmax(1, cur)
-                stage = 1
-        if f + AHEAD < 36:
-            emit_all(em, frag_read(f + AHEAD, KADDR2))
-        if f in copy_at and copies:
-            emit_all(em, copies[copy_at[f]])
-    emit_all(em, pending)
-    assert stage == 1
-    if "novalu" not in X and "norare" not in X:
-        em.raw(f"s_cbranch_vccnz L_rare_{k}_1_%=")
-    em.label(f"L_back_{k}_1_%=")
-    if "novalu" not in X:
-        em.emit(valu(f"v_add_f32 {vr(L[1])}, {vr(L[1])}, {vr(PS)}", [L[1], PS], [L[1]]))
-    pv_phase(em)
-    end_of_step(em)
 
 
 def generate():
@@ -555,41 +505,32 @@ def generate():
         em.raw(f"s_mov_b32 s{AGAIN}, 0")
         for hb in range(2):
             em.emit(valu(f"v_mov_b32 {vr(PM[hb])}, 0", [], [PM[hb]]))
-    if PIPELINED:
-        # scores of the first tile (slot t & 3) into the set step t reads
-        for k in range(4):
-            em.raw(f"s_and_b32 {a}, %[t], 3")
-            em.raw(f"s_cmp_eq_u32 {a}, {k}")
-            em.raw(f"s_cbranch_scc0 L_pre_skip_{k}_%=")
-            em.emit(valu(f"v_add_u32 {vr(KADDR2)}, {k * SLOT_B}, {vr(KBASE)}", [KBASE], [KADDR2]))
-            qk_phase(em, SC if k % 2 == 0 else SC2, KADDR2, None)
-            em.raw("s_waitcnt lgkmcnt(0)", "wait")
-            em.lds_queue = []
-            em.label(f"L_pre_skip_{k}_%=")
-    em.raw(f"s_and_b32 {a}, %[t], 3")
-    for k in range(1, 4):
-        em.raw(f"s_cmp_eq_u32 {a}, {k}")
-        em.raw(f"s_cbranch_scc1 L_step_{k}_%=")
+    # (the loop is entered with t = 0)
+    em.emit(valu(f"v_mov_b32 {vr(KADDR)}, {vr(KBASE)}", [KBASE], [KADDR]))
+    for f in range(AHEAD):
+        emit_all(em, frag_read(f, KADDR))
+    asked = list(em.lds_queue)
     queues = []
     for k in range(4):
         em.label(f"L_step_{k}_%=")
-        queues.append((step_pipelined if PIPELINED else step_plain)(em, k))
+        queues.append(step(em, k))
+        assert em.lds_queue == asked
         if k < 3:
             em.raw("s_cbranch_scc0 L_exit_%=")
         else:
             em.raw("s_cbranch_scc1 L_step_0_%=")
             em.raw("s_branch L_exit_%=")
     for k in range(4):
-        cur = SC if (k % 2 == 0 or not PIPELINED) else SC2
         for hb in range(2):
-            rare_block(em, f"{k}_{hb}", hb, cur)
+            rare_block(em, f"{k}_{hb}", hb, SC)
             if P16 and "noagain" not in X:
                 heavy_block(em, k, hb)
         if P16 and "noagain" not in X:
             again_block(em, k, queues[k])
-        mask_block(em, k, cur, f"{k}")
+        mask_block(em, k, SC, f"{k}")
         lastofs_block(em, k)
     em.label("L_exit_%=")
+    em.raw("s_waitcnt lgkmcnt(0)", "wait")                      # operands requested for a tile that does not come
     em.raw("s_nop 15", "nop")
     em.raw("s_nop 3", "nop")
     if P16:
@@ -612,7 +553,7 @@ def emit_text(p16):
                   "ML": (ML, 8), "OFS": (OFS, 16), "OFSL": (OFSL, 16)})
     for name, (lo, n) in ({} if p16 else binds).items():  # (the same registers in both loops)
         text += f'#define {pre}_C_{name} "{{{vr(lo, n)}}}"\n'
-    text += "" if p16 else (f"#define {pre}_COPIES_AHEAD {COPIES if PIPELINED else 2 * COPIES}"
+    text += "" if p16 else (f"#define {pre}_COPIES_AHEAD {2 * COPIES}"
              "  // copies that may be outstanding when a step starts\n")
     lines = ['    "%s\\n"' % ins.text for ins in em.out]
     text += f"#define {pre}_ASM \\\n" + " \\\n".join(lines) + "\n"
@@ -630,8 +571,7 @@ def main():
             "// The RPA_MLA_WIDE_C_* macros are the register constraints that bind the kernel's variables to the\n"
             "// registers the assembly uses.\n")
     text += emit_text(False)
-    if not PIPELINED:
-        text += emit_text(True)
+    text += emit_text(True)
     with open(os.path.join(here, "rpa_mla_wide_loop.inc"), "w") as f:
         f.write(text)
 
