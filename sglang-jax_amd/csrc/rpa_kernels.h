@@ -150,6 +150,8 @@ struct PrefillArgs {
   struct {
     FastDiv groups, units, hkv, per_kv, nseq;
     int32_t apart;
+    int32_t block;  // > 0: so many tiles of a sequence one after the other (the order by streams)
+    FastDiv round, seq_round, run;
   } map;  // set by the launchers (prefill_grid)
 };
 

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
   __shared__ __attribute__((aligned(1024))) char lds_v1[kTileB];
 
   constexpr int BM = HEADS4 ? 32 : kBM;  // query positions per workgroup
-  Work w = decompose(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
+  Work w = decompose<true>(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
   if (!w.valid) {
     write_new_tokens(a_in);
     return;
@@ -825,7 +825,7 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const Prefil
   __shared__ __attribute__((aligned(16))) char lds_v_buf[2][128 * kVPitch];
 
   constexpr int BM = HEADS4 ? 32 : kBM;  // the short-chunk tile: 32 positions x 4 heads, one head per wave
-  Work w = decompose(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
+  Work w = decompose<true>(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
   if (!w.valid) {
     write_new_tokens(a_in);
     return;
@@ -1095,7 +1095,7 @@ hipError_t launch_prefill(const PrefillArgs& call, hipStream_t stream) {
   const int levels = a.max_kv_len > 0 ? (a.max_kv_len + bm - 1) / bm + 1 : 0;
   const bool by_level = level_order && a.sm.mask_mode == 0 && levels > tiles && levels <= 2 * tiles + 2;
   if (by_level) tiles = levels;
-  const int64_t grid = prefill_grid(a, nseq, tiles, heads4 ? 4 : 1);
+  const int64_t grid = prefill_grid(a, nseq, tiles, heads4 ? 4 : 1, a.head_dim == 256 ? 0 : 64);
   if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   // whether the rows that a wave brings in of a tile are one page's
   const int wave_rows = a.head_dim == 256 ? 8 : (a.fp8 || tuning().prefill_staged == 1) ? kBN : 16;

@@ -79,6 +79,10 @@ __device__ __forceinline__ int64_t row_offset(const TileSrc& s, const KvAddr& kv
 //     for every tile, had left 4 workgroups to each of 112 CUs and 1 to 48: 262.6 -> 203.5 us.  7 prompts of 264 .. 1643
 //     tokens x 8 / 2 heads 46.6 -> 37.1, 4 prompts of 484 ..
 //     2368 x 16 / 8 heads 119 -> 87; odd numbers of sequences and 4 heads per kv head are where they were.
+// Sequences with much to read take the order by streams instead (STREAMS, a.map.block; streams_in_turn()): a.map.block tiles of one
+// sequence and kv head, as many as an XCD has places for with their heads, come one after the other, then those of the next sequence.
+// They walk the same K/V side by side, which their XCD's L2 then fetches once; in the order of pairs four sequences share it, and
+// once workgroups of different lengths have ended, four heads are all that still walk together.
 // The most expensive query tiles are issued first, so that the last workgroups to start are short ones.  A causal tile costs
 // what its last row sees: with a bound on kv_len from the host, tiles are ordered by level = tile index + ceil(prefix / tile
 // rows), i.e. by that extent across sequences; without one, by position inside their own sequence.
@@ -102,6 +106,7 @@ inline FastDiv fast_div(int d) {
 
 // `heads` query heads of a kv head per workgroup (1, or 4 when the waves of a workgroup take a head each):
 // Work.head is then the first of them.
+template <bool STREAMS = false>
 __device__ __forceinline__ Work decompose(const PrefillArgs& a, int tiles, int nseq, bool by_level, int bm = kBM,
                                           int heads = 1) {
   Work w;
@@ -110,17 +115,29 @@ __device__ __forceinline__ Work decompose(const PrefillArgs& a, int tiles, int n
   const int groups = a.G / heads;  // workgroups per (sequence, kv head, tile)
   const int span = a.map.apart ? 1 : groups, per_kv = a.map.apart ? groups : 1;  // workgroups of a kv head side by side; its places
   const int r = blockIdx.x >> 3, rg = by(r, a.map.groups);
-  const int pair = rg * 8 + (blockIdx.x & 7);
-  const int tile_rev = by(pair, a.map.units);
-  if (tile_rev >= tiles) return w;
-  const int place = pair - tile_rev * (units * per_kv);
-  int si = by(place, a.map.hkv);
-  const int in_seq = place - si * (a.Hkv * per_kv);
-  w.hk = by(in_seq, a.map.per_kv);
-  const int gi = ((r - rg * span) + (in_seq - w.hk * per_kv)) * heads;
-  if ((nseq & 1) == 0) {  // (an odd number of them moves on by itself)
-    si += tile_rev;
-    si -= by(si, a.map.nseq) * nseq;
+  int tile_rev, si, gi;
+  if (STREAMS && a.map.block > 0) {
+    const int run = a.map.block, of_seq = (a.Hkv >> 3) * run;  // pairs of one kv head and round; of a sequence, on one XCD
+    const int round = by(rg, a.map.round), in_round = rg - round * of_seq * nseq;
+    si = by(in_round, a.map.seq_round);
+    const int in_seq = in_round - si * of_seq, turn = by(in_seq, a.map.run);
+    tile_rev = (round * run) + in_seq - turn * run;
+    if (tile_rev >= tiles) return w;
+    w.hk = turn * 8 + (blockIdx.x & 7);
+    gi = (r - rg * span) * heads;
+  } else {
+    const int pair = rg * 8 + (blockIdx.x & 7);
+    tile_rev = by(pair, a.map.units);
+    if (tile_rev >= tiles) return w;
+    const int place = pair - tile_rev * (units * per_kv);
+    si = by(place, a.map.hkv);
+    const int in_seq = place - si * (a.Hkv * per_kv);
+    w.hk = by(in_seq, a.map.per_kv);
+    gi = ((r - rg * span) + (in_seq - w.hk * per_kv)) * heads;
+    if ((nseq & 1) == 0) {  // (an odd number of them moves on by itself)
+      si += tile_rev;
+      si -= by(si, a.map.nseq) * nseq;
+    }
   }
   w.head = w.hk * a.G + gi;
   w.seq = a.seq_begin + si;
@@ -139,10 +156,26 @@ __device__ __forceinline__ Work decompose(const PrefillArgs& a, int tiles, int n
   return w;
 }
 
+// Whether a launch takes the order by streams (decompose): several sequences on a multiple of 8 kv heads, each XCD with more workgroups
+// than it has places for, and so much to read for one of them that four side by side do not stay in an XCD's 4 MB.  Known on the host
+// and of the chunks themselves (behind decode rows the bound on the lengths may be theirs).  In order of pairs -> by streams:
+//   4 chunks of 1900 .. 2048 tokens on 4096 .. 16384 x 32 / 8 heads 1500 -> 1382 us (4.2 GB past the L2s for 0.2 GB of cache, now 0.35),
+//   4 of 1024 on 4000 .. 12000 e4m3 605 -> 545, 2 of 2223 .. 2599 on 3471 .. 13887 x 16 / 8 heads 405 -> 369, 5 of 1000 .. 3000 on up to 8000
+//   394 -> 378, 2 of 1161 .. 1305 on 4260 x 32 / 8 237 -> 219, 8 of 512 on 8192 510 -> 500.
+// What it costs are the short tiles at the end of the launch: chunks of 1905 and 321 on 5811 e4m3 368 -> 380.  On up to 4600 tokens
+// the two orders are level or the order of pairs ahead (chunks of 29 .. 1946 on 276 58 against 61), and with 256-wide heads, one
+// workgroup to a CU, 0.95 .. 1.0.  Fewer kv heads would spread a sequence over the XCDs by its tiles: 0.72 .. 1.28 times as fast, by how
+// the tiles come out.
+inline bool streams_in_turn(const PrefillArgs& a, int nseq, int64_t grid, int slots) {
+  const int64_t seen = a.sm.window > 0 ? std::min<int64_t>(a.max_kv_len, (int64_t)a.sm.window + kBM) : a.max_kv_len;
+  return nseq > 1 && a.Hkv % 8 == 0 && !a.dist && a.seq_begin == 0 && seen >= 4608 && grid > 8ll * slots;
+}
+
 // Workgroups of a launch of `tiles` tiles, and the divisors of their order (see decompose).
+// slots: workgroups that an XCD has places for, of a kernel that knows the order by streams (0: it does not).
 // With fewer than 8 units their heads go to XCDs of their own: what few pairs there are would leave XCDs without work (2 chunks of
 // 36 .. 171 tokens x 8 / 1 heads 42.8 -> 31.5 us).
-inline int64_t prefill_grid(PrefillArgs& a, int nseq, int tiles, int heads) {
+inline int64_t prefill_grid(PrefillArgs& a, int nseq, int tiles, int heads, int slots = 0) {
   const int groups = a.G / heads, units = nseq * a.Hkv;
   a.map.apart = units < 8;
   const int span = a.map.apart ? 1 : groups, per_kv = groups / span;
@@ -151,7 +184,17 @@ inline int64_t prefill_grid(PrefillArgs& a, int nseq, int tiles, int heads) {
   a.map.hkv = fast_div(a.Hkv * per_kv);
   a.map.per_kv = fast_div(per_kv);
   a.map.nseq = fast_div(nseq);
-  return ((int64_t)units * per_kv * tiles + 7) / 8 * 8 * span;
+  a.map.block = 0;
+  const int64_t grid = ((int64_t)units * per_kv * tiles + 7) / 8 * 8 * span;
+  if (slots > 0 && streams_in_turn(a, nseq, grid, slots)) {
+    const int most = std::max(1, slots / groups), rounds = (tiles + most - 1) / most, m = a.Hkv / 8;
+    a.map.block = (tiles + rounds - 1) / rounds;
+    a.map.run = fast_div(a.map.block);
+    a.map.seq_round = fast_div(a.map.block * m);
+    a.map.round = fast_div(a.map.block * m * nseq);
+    return (int64_t)8 * m * nseq * rounds * a.map.block * groups;
+  }
+  return grid;
 }
 
 // K (or V) rows of the workgroup's kv head, token 0 of its sequence's first page.

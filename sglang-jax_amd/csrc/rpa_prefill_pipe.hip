@@ -321,7 +321,7 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
   constexpr int BM = HEADS4 ? 32 : 128 * NQ;  // query positions per workgroup
   __shared__ __attribute__((aligned(1024))) char lds[4 * kTileB];
 
-  Work w = decompose(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
+  Work w = decompose<true>(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
   if (!w.valid) {
     write_new_tokens(a_in);
     return;
@@ -580,7 +580,7 @@ hipError_t launch_prefill_pipe(const PrefillArgs& call, int nseq, bool level_ord
   const int levels = a.max_kv_len > 0 ? (a.max_kv_len + bm - 1) / bm + 1 : 0;
   const bool by_level = level_order && levels > tiles && levels <= 2 * tiles + 2;
   if (by_level) tiles = levels;
-  const int64_t grid = prefill_grid(a, nseq, tiles, heads4 ? 4 : 1);
+  const int64_t grid = prefill_grid(a, nseq, tiles, heads4 ? 4 : 1, 64);
   if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   const dim3 g((unsigned)(grid + a.write_blocks)), blk(256);
   const bool win = a.sm.window > 0;

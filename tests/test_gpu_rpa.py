@@ -2188,3 +2188,32 @@ def test_head_dim_256_rows_bring_their_tokens(pkg, wl, gpu, Hq, Hkv, P, D, on_de
         page = int(b.page_indices[int(b.cu_kv_lens[i]) // P + (kv - 1) // P])
         expect[page, (kv - 1) % P] = full[page, (kv - 1) % P]
     assert torch.equal(got, expect)
+
+
+@pytest.mark.parametrize("Hq,Hkv,q_lens,kv_lens,fp8", [
+    (32, 8, [1300, 1299, 1], [5000, 1299, 4700], False), (64, 16, [600, 129, 640, 640], [5300, 4800, 640, 4609], False),
+    (40, 8, [2200, 130, 1], [2200, 4700, 1], False), (32, 8, [900, 1000, 128], [4700, 1000, 4900], True),
+])
+def test_sequences_one_after_the_other(pkg, wl, gpu, monkeypatch, Hq, Hkv, q_lens, kv_lens, fp8):
+    """Long sequences take the launch's workgroups in turn: the same rows, bit for bit, as each sequence in a call of its own (one
+    sequence keeps the order of pairs), tiles that some of them do not have among them."""
+    say(f"streams {Hq}/{Hkv} {q_lens} {kv_lens} fp8={fp8}")
+    monkeypatch.setenv("RPA_PREFILL_SPLITS", "0")
+    monkeypatch.setenv("RPA_PREFILL_PACKED", "0")
+    b = wl.make_batch("streams", q_lens, kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=128, page_size=64, seed=23,
+                      kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+    g = b.to(gpu)
+
+    def run(first, last):
+        q0, q1 = int(b.cu_q_lens[first]), int(b.cu_q_lens[last])
+        p0, p1 = int(b.cu_kv_lens[first]) // 64, int(b.cu_kv_lens[last]) // 64
+        poison_free_blocks(g.q)
+        out, _ = pkg.ragged_paged_attention(
+            g.q[q0:q1].contiguous(), None, None, g.kv_cache, g.kv_lens[first:last].contiguous(), g.page_indices[p0:p1].contiguous(),
+            g.cu_q_lens[first : last + 1] - q0, g.cu_kv_lens[first : last + 1] - p0 * 64, (0, 0, last - first), sm_scale=b.sm_scale,
+            k_scale=g.k_scale, v_scale=g.v_scale, max_kv_len=max(kv_lens), max_q_len=max(q_lens))
+        torch.cuda.synchronize()
+        return out.cpu()
+
+    n = len(q_lens)
+    assert torch.equal(run(0, n), torch.cat([run(i, i + 1) for i in range(n)]))
