@@ -1015,6 +1015,9 @@ static size_t prefill_optional_workspace(const RpaParams* p) {
   return prefill_workspace(p, a).total;
 }
 
+static int write_new_tokens(const RpaParams* p, const void* keys, const void* values, bool skip_decode_rows, void* stream);
+
+// keys / values: new tokens that the launch itself puts into the cache (prompts without a prefix, custom masks).
 static int prefill_run(const RpaParams* p, const void* keys, const void* values, void* stream) {
   int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
@@ -1049,6 +1052,10 @@ static int prefill_run(const RpaParams* p, const void* keys, const void* values,
       a.mask_bits = reinterpret_cast<uint64_t*>(ws + bits_at);
       a.mask_pitch = w.pitch;
     }
+  }
+  if (keys && p->mask_mode == RPA_MASK_CUSTOM) {  // by the launch that makes the bits, if there is one
+    if (a.mask_bits) a.write = kv_write_args(p, keys, values);
+    else if ((rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
   }
   if (p->mask_mode == RPA_MASK_CUSTOM && !p->cu_mask_lens && !a.mask_bits)
     return fail(RPA_EINVAL_WORKSPACE, "a mask without cu_mask_lens needs rpa_workspace_bytes() of workspace");
@@ -1130,7 +1137,7 @@ int rpa_attention_update(const RpaParams* given, const void* keys, const void* v
     if (keys && !with_rows && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
     return decode_rows(p, with_rows ? keys : nullptr, with_rows ? values : nullptr, true, stream);
   }
-  if (keys && takes_fresh_prompts(p)) return prefill_run(p, keys, values, stream);
+  if (keys && (takes_fresh_prompts(p) || mask_as_bits(p))) return prefill_run(p, keys, values, stream);
   const bool fused = keys && decode_rows_write(p);
   if (keys && !fused && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
   if ((rc = decode_rows(p, fused ? keys : nullptr, fused ? values : nullptr, false, stream)) != RPA_OK) return rc;
@@ -1201,7 +1208,8 @@ int rpa_describe_plan(const RpaParams* given, char* buf, size_t len) {
   }
   const bool rows = takes_token_rows(p_in), prompts = !rows && takes_fresh_prompts(p_in);
   const bool by_rows = rows ? rows_take_new_tokens(p_in) : !prompts && decode_rows_write(p_in);
-  put("new tokens: written by %s\n", prompts                            ? "workgroups of the prefill launch, which reads the caller's rows"
+  put("new tokens: written by %s\n", !rows && mask_as_bits(p_in)        ? "the launch that makes bits of the mask"
+                                     : prompts                           ? "workgroups of the prefill launch, which reads the caller's rows"
                                      : !by_rows                         ? "rpa_kv_write_kernel, in front"
                                      : p_in->distribution && !rows      ? "the decode kernels, those of chunks by rpa_kv_write_kernel"
                                                                         : "the decode kernels");

@@ -134,7 +134,8 @@ struct PrefillArgs {
   float* ws_o;
   float* ws_ml;
   // Custom masks: one bit per (query token, kv token), mask_pitch 64-bit words per token row, written by
-  // rpa_mask_bits_kernel in front of the attention kernels; nullptr: the kernels read the caller's i32 words
+  // rpa_mask_bits_kernel in front of the attention kernels (with write.keys it also puts the new tokens into the
+  // cache); nullptr: the kernels read the caller's i32 words
   uint64_t* mask_bits;
   int32_t mask_pitch;
   // Prompts without a prefix: kv addresses the caller's new rows (a sequence's start at its first query token, one huge

@@ -1599,6 +1599,47 @@ def test_mask_bits_of_many_sequences_and_long_rows(pkg, wl, gpu, monkeypatch, se
     assert torch.equal(run(), words)
 
 
+@pytest.mark.parametrize("seqs", [1, 63, 64])
+@pytest.mark.parametrize("D,Hkv,P,fp8", [(128, 2, 16, False), (128, 20, 64, True), (64, 3, 48, False)])
+@pytest.mark.parametrize("on_device", [False, True])
+def test_masked_calls_bring_their_tokens(pkg, wl, gpu, monkeypatch, seqs, D, Hkv, P, fp8, on_device):
+    """The launch that makes bits of a mask puts the new tokens into the cache as well: same rows and the same cache, byte for byte, as
+    the launch in front of it leaves where the mask stays words.  Both searches, rows shorter and longer than a workgroup,
+    narrow heads, and a padded batch whose size is on the device."""
+    q_lens = [[3, 1, 17, 4][i % 4] for i in range(seqs)]
+    kv_lens = [q + [0, 61, 300][i % 3] for i, q in enumerate(q_lens)]
+    rng = np.random.default_rng(seqs)
+    masks = [(rng.random((ql, kv)) < 0.5).astype(np.int32) for ql, kv in zip(q_lens, kv_lens)]
+    for m in masks:
+        m[:, -1] = 1
+    say(f"masked, own tokens: {seqs} sequences D={D} Hkv={Hkv} P={P} fp8={fp8} on_device={on_device}")
+    b = wl.make_batch("mask_new", q_lens, kv_lens, num_q_heads=2 * Hkv, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=95,
+                      kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+    g, mask = b.to(gpu), flat_mask(masks).to(gpu)
+    T, pad = sum(q_lens), 5 if on_device else 0
+    gen = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(T + pad, h, D, generator=gen).to(torch.bfloat16).to(gpu) for h in (2 * Hkv, Hkv, Hkv))
+    k, v = k.to(g.kv_cache.dtype), v.to(g.kv_cache.dtype)
+    lens, cu_q, cu_kv, pages, dist = g.kv_lens, g.cu_q_lens, g.cu_kv_lens, g.page_indices, b.distribution.numpy()
+    if on_device:  # two sequences of the bucket are not there
+        lens, cu_q, cu_kv = (torch.cat([x, x[-1:].repeat(2)]) for x in (lens, cu_q, cu_kv))
+        dist = b.distribution.to(torch.int32).to(gpu)
+
+    def run():
+        cache = g.kv_cache.clone()
+        out, cache = pkg.ragged_paged_attention(q, k, v, cache, lens, pages, cu_q, cu_kv, dist, mask, sm_scale=D ** -0.5, causal=0,
+                                                k_scale=g.k_scale, v_scale=g.v_scale, max_kv_len=max(kv_lens), max_q_len=17)
+        torch.cuda.synchronize()
+        return out[:T].cpu(), cache.cpu().view(torch.uint8)
+
+    monkeypatch.setenv("RPA_MASK_BITS", "0")
+    words = run()
+    monkeypatch.delenv("RPA_MASK_BITS")
+    bits = run()
+    assert torch.equal(bits[1], words[1]) and not torch.equal(bits[1], g.kv_cache.cpu().view(torch.uint8))
+    assert torch.equal(bits[0], words[0])
+
+
 @pytest.mark.parametrize("kind", ["soft_cap", "xai_temperature", "custom_mask", "no_mask", "softmax_bf16", "fp8", "fp8_custom_mask"])
 def test_short_chunks_take_the_four_head_tile_in_the_compiled_kernel(pkg, wl, gpu, monkeypatch, kind):
     """The compiled flash kernel (every option the pipelined one does not take) with the same short-chunk tile:
