@@ -59,6 +59,33 @@ __device__ __forceinline__ float swap16_max(float x) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+// Rows on their way out.  Stretches of 32 bytes cost a store as much as stretches of 64: 128 KB from the four waves of every CU take
+// 4.4 us against 2.5 (1.9 and 1.2 from one CU alone), longer ones no less.  What the matrix units leave in a lane is 8 bytes here and 8
+// there, so it changes places between the lanes first.
+// 16 columns, lane (c, g = lane / 16) holding bytes 8g .. of two 32-byte chunks of row c: then bytes 16g .. of the 64.
+__device__ __forceinline__ u32x4_t row_of_16(u32x2_t a, u32x2_t b) {
+  u32x4_t w;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a[i], b[i], false, false);
+    const auto s = __builtin_amdgcn_permlane16_swap(r[0], r[1], false, false);
+    w[i] = s[0];
+    w[2 + i] = s[1];
+  }
+  return w;
+}
+
+// x + the pair lane's x, likewise.
+__device__ __forceinline__ float swap_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+__device__ __forceinline__ float swap16_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // cap * tanh(x / cap) = cap - 2 cap / (e^(2x/cap) + 1), written so that +-inf arguments give +-cap: one
 // multiply, v_exp_f32, one add, v_rcp_f32 (1 ulp; an IEEE division here is ten instructions per score), one fma.
 __device__ __forceinline__ float soft_cap_f(float x, float cap, float inv_cap) {
@@ -145,6 +172,16 @@ __device__ __forceinline__ void async_copy16(const void* gsrc, const void* lds_b
   typedef const __attribute__((address_space(3))) char* lds_ptr_t;
   const uint32_t m0v = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)lds_base_uniform));
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0v), "v"(gsrc) : "memory", "m0");
+}
+
+// The same from a wave-uniform address and the lane's offset from it.
+__device__ __forceinline__ void async_copy16_from(const char* base_uniform, uint32_t offset, const void* lds_base_uniform) {
+  typedef const __attribute__((address_space(3))) char* lds_ptr_t;
+  const uint32_t m0v = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)lds_base_uniform));
+  const uint64_t a = reinterpret_cast<uint64_t>(base_uniform);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a >> 32));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0v), "v"(offset), "s"((static_cast<uint64_t>(hi) << 32) | lo) : "memory", "m0");
 }
 
 // Eight query elements from dim d of a row of q_dim (a multiple of 8); dims past it are zero.

@@ -188,7 +188,7 @@ __device__ __forceinline__ void copy_tile(char* slot, const Src& s, const char* 
       for (int n = 0; n < CPW; ++n) {
         int row, inner;
         chunk_of<CPW>(s, wave, ln, n, row, inner);
-        async_copy16(base + (uint32_t)(row * s.row_bytes + inner), slot + copy_block<CPW>(wave, n) * 1024);
+        async_copy16_from(base, (uint32_t)(row * s.row_bytes + inner), slot + copy_block<CPW>(wave, n) * 1024);
       }
       return;
     }
@@ -196,7 +196,7 @@ __device__ __forceinline__ void copy_tile(char* slot, const Src& s, const char* 
     for (int n = 0; n < CPW; ++n) {
       int row, inner;
       chunk_of<CPW>(s, wave, ln, n, row, inner);
-      async_copy16(base + (uint32_t)(min(row, most) * s.row_bytes + inner), slot + copy_block<CPW>(wave, n) * 1024);
+      async_copy16_from(base, (uint32_t)(min(row, most) * s.row_bytes + inner), slot + copy_block<CPW>(wave, n) * 1024);
     }
   } else {
     // pages smaller than a tile: all the ids first, one round trip to LDS (chunks of 512 on up to 2000 tokens, pages of 48: 128 heads
@@ -838,8 +838,7 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   if constexpr (!UNIFORM) bare_barrier();
 
   // ---- epilogue: lane (c, g) holds head head0+c, dims 16j + 4g + r in acc[j][r] ----
-  l += __shfl_xor(l, 16);
-  l += __shfl_xor(l, 32);
+  l = swap_sum(swap16_sum(l));
   // The lane parts of the output addresses are worked out here, from values the compiler cannot
   // trace back across the tile loop: hoisted out of it they would sit in registers the loop has
   // none to spare for (they were spilled to scratch memory).
@@ -851,27 +850,27 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   }
   asm volatile("" : "+v"(c_out), "+v"(g_out));
   const int head = head0 + c_out;
-  if (TG ? !tg_real : (!wave_on || head >= a.Hq)) return;
+  if (TG ? !tg_real : !wave_on) return;
+  const bool real = TG || head < a.Hq;  // (every lane takes part in the exchange)
   const int chunk0 = DS > 1 ? sub * kChunksPerWave : 0;  // shared tiles: this wave's output chunks
-  if (dest.final_rows) {
-    const float inv = a.out_scale / l;
-    uint16_t* op = a.out + ((int64_t)tq * a.Hq + head) * 512 + g_out * 4 + chunk0 * 16;
+  auto put = [&](uint16_t* row, float inv) __attribute__((always_inline)) {
+    u32x4_t w[kChunksPerWave / 2];
 #pragma unroll
-    for (int j = 0; j < kChunksPerWave; ++j) {
-      u32x2_t w = {pack_bf16x2(acc[j][0] * inv, acc[j][1] * inv), pack_bf16x2(acc[j][2] * inv, acc[j][3] * inv)};
-      *reinterpret_cast<u32x2_t*>(op + j * 16) = w;
-    }
+    for (int j = 0; j < kChunksPerWave; j += 2)
+      w[j / 2] = row_of_16(u32x2_t{pack_bf16x2(acc[j][0] * inv, acc[j][1] * inv), pack_bf16x2(acc[j][2] * inv, acc[j][3] * inv)},
+                           u32x2_t{pack_bf16x2(acc[j + 1][0] * inv, acc[j + 1][1] * inv), pack_bf16x2(acc[j + 1][2] * inv, acc[j + 1][3] * inv)});
+    if (!real) return;
+#pragma unroll
+    for (int j = 0; j < kChunksPerWave; j += 2) st16(row + (chunk0 + j) * 16 + g_out * 8, w[j / 2]);
+  };
+  if (dest.final_rows) {
+    put(a.out + ((int64_t)tq * a.Hq + head) * 512, a.out_scale / l);
   } else {
     const int64_t slot = dest.base + head;
     // partial rows are left as bf16: the merge reads half the bytes, and the result is rounded to
     // bf16 anyway
-    uint16_t* wo = a.ws_o + slot * 512 + g_out * 4 + chunk0 * 16;
-#pragma unroll
-    for (int j = 0; j < kChunksPerWave; ++j) {
-      u32x2_t w = {pack_bf16x2(acc[j][0], acc[j][1]), pack_bf16x2(acc[j][2], acc[j][3])};
-      *reinterpret_cast<u32x2_t*>(wo + j * 16) = w;
-    }
-    if (g_out == 0 && (DS == 1 || sub == 0)) {
+    put(a.ws_o + slot * 512, 1.0f);
+    if (g_out == 0 && real && (DS == 1 || sub == 0)) {
       a.ws_ml[slot * 2 + 0] = m;
       a.ws_ml[slot * 2 + 1] = l;
     }
@@ -942,6 +941,15 @@ constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 // the group's LAST token sees, a block's own token sees up to group_tokens - 1 fewer, so the loop masks the
 // tile before the last too and takes the second block's row end relative to the first's.
 // P16: pages of 16 tokens, on the loop that has a scalar base for each half of a tile.
+//
+// What a piece costs besides its tiles: 20 rows of 1000..9000 tokens, 15 tiles of 1.7 us each, us from a workgroup's clock: page ids, queries
+// and first tile 8.5 -> 6, reference 1.3, rows written 6.7 -> 3.5.  The loop takes 251 of a wave's 256 registers, and whatever the compiler
+// keeps from piece to piece -- lane offsets, a constant of zero, the scale -- goes to scratch memory, whose reloads wait for everything in
+// flight: half of the queries, each tile's copies, the rows of the first 16 heads.  So all of it is worked out in the piece, behind
+// values that the compiler cannot trace; copies take a scalar base; no kernel of the wide loop spills.
+// The call: 20 rows of 1000..9000 tokens 60.5 -> 55.0 us, 67 of 179..2380 58.9 -> 52.0, 300 of 300..1500 138.5 -> 122.0, one of 4000 27.9 -> 25.3,
+// 64 of 2047..16383 1.01 .. 1.04 times as fast; chunks of 200..400 tokens x 64 heads 118.5 -> 104, of 1000 x 16 heads 131 -> 122;
+// sparse token selections of 20 rows x 128 heads 49.2 -> 45.7.
 template <bool M32, bool TG = false, bool P16 = false>
 __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const MlaRow mr, int head_base, int t_lo,
                                                  int t_begin, int t_end, const MlaDest dest, char* ring,
@@ -951,7 +959,7 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
   RPA_MLA_STAMP(0);
   constexpr int CPW = 2 * kCopiesPerWave;
   const int tid = threadIdx.x;
-  const int lane = tid & 63;
+  const int lane = fresh_lane();  // (nothing of it is kept from piece to piece: it would be in scratch memory)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = M32 ? (lane & 31) : (lane & 15), g = M32 ? (lane >> 5) : (lane >> 4);
   const int head0 = head_base + wave * 32;
@@ -982,7 +990,7 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
   src.page_size = a.pt.page_size;
   src.page_shift = 31 - __builtin_clz(src.page_size);
   src.last_tok = kv_len - 1;
-  src.pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (a.pt.cu_kv_lens[seq] / a.pt.page_size)
+  src.pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (scalar_load_i32(a.pt.cu_kv_lens + seq) >> src.page_shift)
                                                   : (int64_t)seq * a.pt.pages_per_seq);
   src.row_bytes = a.row_stride * 2;
   src.page_stride = (int64_t)src.row_bytes * a.pt.page_size;
@@ -995,6 +1003,14 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
     tb = min(tb, src.last_tok & ~(kTok - 1));
     return scalar_load_i32(src.pages + __builtin_amdgcn_readfirstlane(min(page_slot(src, tb) + 1, page_slot(src, src.last_tok))));
   };
+
+  // page ids of the first tiles, in one round trip
+  int pg[4], pg2[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    pg[i] = page_of(t_begin + i * kTok);
+    if constexpr (P16) pg2[i] = second_page_of(t_begin + i * kTok);
+  }
 
   // ---- Q^T operands: column c of block hb = head head0 + 16 hb + c, k-step ks covers dims 32ks + 8g .. ----
   // 16x16x32: qB[hb][ks], k-step ks covers dims 32ks + 8g ..; 32x32x16: the same 36 registers of 4 as
@@ -1018,24 +1034,26 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
       qB[hb][17] = ld16(qr + 32);
     }
   }
-  const float scale2 = a.sm.sm_scale * kLog2e;
+  float sm_scale = a.sm.sm_scale;
+  asm volatile("" : "+s"(sm_scale));  // (worked out anew in every piece, as the lane)
+  const float scale2 = sm_scale * kLog2e;
 
-  int pg_next = page_of(t_begin + 3 * kTok);
-  int pg2_next = P16 ? second_page_of(t_begin + 3 * kTok) : 0;
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const int tb = t_begin + i * kTok;
-    if constexpr (P16) copy_tile_p16<CPW>(ring + i * kSlotB, src, a.cache, tb, wave, lane, page_of(tb), second_page_of(tb));
-    else copy_tile<true, CPW, true>(ring + i * kSlotB, src, a.cache, tb, wave, lane, page_of(tb));
-  }
+  // Queries and the first tile are waited for, all of them: the next two tiles, which nothing needs before the first step's end,
+  // are asked for behind that, and travel under the reference below and the first step.
+  auto copy = [&](int i) __attribute__((always_inline)) {
+    if constexpr (P16) copy_tile_p16<CPW>(ring + i * kSlotB, src, a.cache, t_begin + i * kTok, wave, lane, pg[i], pg2[i]);
+    else copy_tile<true, CPW, true>(ring + i * kSlotB, src, a.cache, t_begin + i * kTok, wave, lane, pg[i]);
+  };
+  copy(0);
 #pragma unroll
   for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
     for (int ks = 0; ks < 18; ++ks) asm volatile("" ::"v"(qB[hb][ks]));
-  // the tiles the first step reads have landed once only the newest copies are outstanding (the generated
-  // loop says how many: the same count its own end-of-step wait uses)
-  static_assert(RPA_MLA_WIDE_COPIES_AHEAD == RPA_MLA_WIDE32_COPIES_AHEAD, "one prologue for both loops");
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(RPA_MLA_WIDE_COPIES_AHEAD));
+  wait_all_loads();
+  copy(1);
+  copy(2);
+  int pg_next = pg[3], pg2_next = pg2[3];
+  static_assert(RPA_MLA_WIDE_COPIES_AHEAD == 2 * CPW && RPA_MLA_WIDE32_COPIES_AHEAD == 2 * CPW, "the loops wait for all but the newest two tiles");
   __syncthreads();
   RPA_MLA_STAMP(1);
 
@@ -1107,18 +1125,20 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
   for (int e = 0; e < 16; ++e) q4[e] = qB[1][14 + (e >> 2)][e & 3];                // registers 128 .. 143
   const int ln = fresh_lane();  // lane parts are worked out here, not carried from the top
   u32x8_t ml;
+  uint32_t none;  // (a constant would be kept from piece to piece, through scratch memory)
+  asm volatile("v_mov_b32 %0, 0" : "=v"(none));
   if constexpr (M32) {
     // K operand: row c, bytes 32ks + 16g.  V^T operand of (dim block d, k-step kk): the lane points at token
     // 16kk + 4g + (r >> 2) (+ 8 for the second read), dims 32d + 16 (b & 1) + 8 ((r & 3) >> 1) + 4 (r & 1), with
     // r = lane & 15, b = lane >> 4 (what the transposing read hands to lane dim = lane % 32)
     const int cc = ln & 31, gg = ln >> 5, r16 = ln & 15, b16 = ln >> 4;
     const int v_in = ((b16 & 1) << 5) + (((r16 & 3) >> 1) << 4) + ((r16 & 1) << 3);
-    ml = u32x8_t{__float_as_uint(m_init[0]), 0u, lds_base + (uint32_t)(cc * kRowB + gg * 16),
+    ml = u32x8_t{__float_as_uint(m_init[0]), none, lds_base + (uint32_t)(cc * kRowB + gg * 16),
                  lds_base + (uint32_t)((4 * gg + (r16 >> 2)) * kRowB + v_in), (uint32_t)(t_lo - t_begin - 4 * gg),
-                 (uint32_t)(kv_len - t_begin - 4 * gg), 0u, 0u};
+                 (uint32_t)(kv_len - t_begin - 4 * gg), none, none};
   } else {
     const int cc = ln & 15, gg = ln >> 4;
-    ml = u32x8_t{__float_as_uint(m_init[0]), 0u, __float_as_uint(m_init[1]), 0u,
+    ml = u32x8_t{__float_as_uint(m_init[0]), none, __float_as_uint(m_init[1]), none,
                  lds_base + (uint32_t)(cc * kRowB + gg * 16),
                  lds_base + (uint32_t)((4 * gg + (cc >> 2)) * kRowB + (cc & 3) * 8),
                  (uint32_t)(t_lo - t_begin - 4 * gg), (uint32_t)(blk_len[0] - t_begin - 4 * gg)};
@@ -1185,8 +1205,7 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
     // lane (c, h) holds head head0 + c, dims 32d + 8q + 4h + r in accumulator 16d + 4q + r
     const int c_out = lo_ & 31, h_out = lo_ >> 5;
     const float m = __uint_as_float(ml[0]);
-    float l = __uint_as_float(ml[1]);
-    l += __shfl_xor(l, 32);
+    const float l = swap_sum(__uint_as_float(ml[1]));
     const int head = head0 + c_out;
     if (head < a.Hq) {
       const float inv = dest.final_rows ? a.out_scale / l : 1.0f;
@@ -1208,44 +1227,40 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
   } else {
   // lane (c, g) holds head head0 + 16 hb + c, dims 16j + 4g + r in accumulator 128 hb + 4 j + r
   const int c_out = lo_ & 15, g_out = lo_ >> 4;
+  const float m_out[2] = {__uint_as_float(ml[0]), __uint_as_float(ml[2])};
+  const float l_out[2] = {swap_sum(swap16_sum(__uint_as_float(ml[1]))), swap_sum(swap16_sum(__uint_as_float(ml[3])))};
+  // P16: against the piece's largest probability.  A piece of which one token is nearly all is that token's row then and has
+  // no rounding, as on eight waves, where that probability is 1.
+  float top[2] = {1.0f, 1.0f};
+  if constexpr (P16) {
+#pragma unroll
+    for (int hb = 0; hb < 2; ++hb) {
+      top[hb] = swap_max(swap16_max(__uint_as_float(ml[4 + 2 * hb])));
+      if (!(top[hb] > 0.f)) top[hb] = 1.0f;
+    }
+  }
 #pragma unroll
   for (int hb = 0; hb < 2; ++hb) {
-    const float m = __uint_as_float(ml[2 * hb]);
-    float l = __uint_as_float(ml[2 * hb + 1]);
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
-    const int head = blk_head[hb] + c_out;
-    if (TG ? !blk_real[hb] : head >= a.Hq) continue;
-    if (dest.final_rows) {
-      const float inv = a.out_scale / l;
-      uint16_t* op = a.out + ((int64_t)tq * a.Hq + head) * 512 + g_out * 4;
+    if (TG && !blk_real[hb]) continue;
+    const int head = blk_head[hb] + c_out;  // (< Hq: the heads come in 128s)
+    auto put = [&](uint16_t* row, float inv) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < 32; ++j) {
+      for (int j = 0; j < 32; j += 2) {
         const int e = (4 * j) & 31, i = 4 * hb + (j >> 3);
-        u32x2_t w = {pack_bf16x2(o[i][e] * inv, o[i][e + 1] * inv), pack_bf16x2(o[i][e + 2] * inv, o[i][e + 3] * inv)};
-        *reinterpret_cast<u32x2_t*>(op + j * 16) = w;
+        st16(row + j * 16 + g_out * 8,
+             row_of_16(u32x2_t{pack_bf16x2(o[i][e] * inv, o[i][e + 1] * inv), pack_bf16x2(o[i][e + 2] * inv, o[i][e + 3] * inv)},
+                       u32x2_t{pack_bf16x2(o[i][e + 4] * inv, o[i][e + 5] * inv), pack_bf16x2(o[i][e + 6] * inv, o[i][e + 7] * inv)}));
       }
+    };
+    if (dest.final_rows) {
+      put(a.out + ((int64_t)tq * a.Hq + head) * 512, a.out_scale / l_out[hb]);
     } else {
       const int64_t slot = dest.base + head;
-      uint16_t* wo = a.ws_o + slot * 512 + g_out * 4;
-      // P16: against the piece's largest probability.  A piece of which one token is nearly all is that token's row then and has
-      // no rounding, as on eight waves, where that probability is 1.
-      float top = P16 ? __uint_as_float(ml[4 + 2 * hb]) : 1.0f;
-      if constexpr (P16) {
-        top = fmaxf(top, __shfl_xor(top, 16));
-        top = fmaxf(top, __shfl_xor(top, 32));
-        if (!(top > 0.f)) top = 1.0f;
-      }
-      const float inv = P16 ? 1.0f / top : 1.0f;
-#pragma unroll
-      for (int j = 0; j < 32; ++j) {
-        const int e = (4 * j) & 31, i = 4 * hb + (j >> 3);
-        u32x2_t w = {pack_bf16x2(o[i][e] * inv, o[i][e + 1] * inv), pack_bf16x2(o[i][e + 2] * inv, o[i][e + 3] * inv)};
-        *reinterpret_cast<u32x2_t*>(wo + j * 16) = w;
-      }
+      const float inv = P16 ? 1.0f / top[hb] : 1.0f;
+      put(a.ws_o + slot * 512, inv);
       if (g_out == 0) {
-        a.ws_ml[slot * 2 + 0] = P16 ? m + __builtin_amdgcn_logf(top) : m;
-        a.ws_ml[slot * 2 + 1] = l * inv;
+        a.ws_ml[slot * 2 + 0] = P16 ? m_out[hb] + __builtin_amdgcn_logf(top[hb]) : m_out[hb];
+        a.ws_ml[slot * 2 + 1] = l_out[hb] * inv;
       }
     }
   }
