@@ -82,10 +82,11 @@ __device__ __forceinline__ u32x2_t lds_tr16(const char* p) {
 // subexpressions of anything earlier, so they are worked out again where they are used instead of being
 // kept in registers across code that has none to spare (the assembly loop pins 251 of a wave's 256; with
 // them carried over it, 23-37 registers went to scratch memory per segment, 100 MB a launch on a
-// prefill batch).  Taken from threadIdx: the same helper on v_mbcnt made the allocator spill 140.
+// prefill batch).  Counted by two instructions of its own, not taken from threadIdx, which would itself be kept in scratch memory across
+// the loops.
 __device__ __forceinline__ int fresh_lane() {
-  int ln = (int)(threadIdx.x & 63);
-  asm volatile("" : "+v"(ln));
+  int ln;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
   return ln;
 }
 
@@ -283,7 +284,8 @@ __device__ __forceinline__ void copy_tile_f8(char* stage, const Src& s, const ch
   }
 #pragma unroll
   for (int n = 0; n < kF8CopiesPerWave; ++n)
-    async_copy16((UNIFORM ? base : page_base<false>(s, cache, pg[n])) + at[n], stage + f8_copy_block(wave, n) * 1024);
+    if constexpr (UNIFORM) async_copy16_from(base, at[n], stage + f8_copy_block(wave, n) * 1024);
+    else async_copy16(page_base<false>(s, cache, pg[n]) + at[n], stage + f8_copy_block(wave, n) * 1024);
 }
 
 // e4m3 bytes of a staged tile -> bf16 rows of a ring slot (exact).  512 threads, 1152 chunks of 16
@@ -439,7 +441,7 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
                                             int t_begin, int t_end, const MlaDest dest, char* slot0, char* slot1,
                                             char* slot2, char* slot3, int group_tokens = 1, int first_ids = 0) {
   const int tid = threadIdx.x;
-  const int lane = tid & 63;
+  const int lane = PIPE ? fresh_lane() : tid & 63;  // (assembly loop: nothing is kept from piece to piece, see mla_segment_wide)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   static_assert(DS == 1 || !PIPE, "shared tiles: compiled loop (LDS for the partial scores)");
@@ -464,7 +466,7 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   src.page_size = a.pt.page_size;
   src.page_shift = ((src.page_size & (src.page_size - 1)) == 0) ? (31 - __builtin_clz(src.page_size)) : -1;
   src.last_tok = kv_len - 1;
-  src.pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (a.pt.cu_kv_lens[seq] / a.pt.page_size)
+  src.pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (scalar_load_i32(a.pt.cu_kv_lens + seq) / a.pt.page_size)
                                                   : (int64_t)seq * a.pt.pages_per_seq);
   src.row_bytes = a.row_stride * (FP8 ? 1 : 2);
   src.page_stride = (int64_t)src.row_bytes * a.pt.page_size;
@@ -503,6 +505,12 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
     }
   };
 
+  int pg[4];  // page ids of the first tiles, in one round trip in front of the queries
+  if constexpr (DS == 1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pg[i] = page_of(t_begin + i * kTok);
+  }
+
   // ---- Q^T operands of this wave: column c = head head0 + c, k-step ks covers dims 32ks + 8g .. ----
   // (shared tiles: the k-steps of this wave's group alone)
   const int tq = mr.tq;
@@ -522,7 +530,8 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
     }
   }
 
-  const float scale = a.sm.sm_scale;
+  float scale = a.sm.sm_scale;
+  if constexpr (PIPE) asm volatile("" : "+s"(scale));
   const float scale2 = scale * kLog2e;
   const float cap = a.sm.soft_cap;
   const float inv_cap = (cap != 0.f) ? 1.0f / cap : 0.f;
@@ -536,8 +545,10 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   const int v_off = (4 * g + (c >> 2)) * kRowB + (c & 3) * 8;
 
   f32x4_t acc[32];
+  float nothing = 0.f;
+  if constexpr (PIPE) asm volatile("v_mov_b32 %0, 0" : "=v"(nothing));
 #pragma unroll
-  for (int j = 0; j < 32; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < 32; ++j) acc[j] = f32x4_t{nothing, nothing, nothing, nothing};
   float m = -INFINITY, l = 0.f;
 
   // ---- pipeline: copies run three tiles ahead of the MFMAs (4-slot ring, 148 of the CU's 160 KiB:
@@ -549,27 +560,35 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
     for (int k = 0; k < 5; ++k) copy_tile_ids(src, t_begin + k * kTok, lane);
     wait_all_loads();
   }
-  int pg_next = page_of(t_begin + 3 * kTok);
   auto stage_of = [&](int i) -> char* { return i == 0 ? slot2 : (i == 1 ? slot2 + kF8StageB : slot3); };
-  if constexpr (FP8) {
-    copy_tile_f8<UNIFORM>(stage_of(0), src, a.cache, t_begin, wave, lane, page_of(t_begin));
-    copy_tile_f8<UNIFORM>(stage_of(1), src, a.cache, t_begin + kTok, wave, lane, page_of(t_begin + kTok));
-    copy_tile_f8<UNIFORM>(stage_of(2), src, a.cache, t_begin + 2 * kTok, wave, lane, page_of(t_begin + 2 * kTok));
-  } else {
-    copy_tile<UNIFORM>(slot0, src, a.cache, t_begin, wave, lane, page_of(t_begin));
-    copy_tile<UNIFORM>(slot1, src, a.cache, t_begin + kTok, wave, lane, page_of(t_begin + kTok));
-    copy_tile<UNIFORM>(slot2, src, a.cache, t_begin + 2 * kTok, wave, lane, page_of(t_begin + 2 * kTok));
+  auto copy = [&](int i) __attribute__((always_inline)) {
+    if constexpr (FP8) copy_tile_f8<UNIFORM>(stage_of(i), src, a.cache, t_begin + i * kTok, wave, lane, pg[i]);
+    else copy_tile<UNIFORM>(i == 0 ? slot0 : i == 1 ? slot1 : slot2, src, a.cache, t_begin + i * kTok, wave, lane, pg[i]);
+  };
+  // Queries and the first tile are waited for, all of them (the compiler knows nothing of the copies: its own wait for the queries is one
+  // for everything in flight); the next two tiles, which nothing needs before the first step's end, are asked for behind that: 100 rows of
+  // 200..1000 e4m3 tokens x 128 heads 66.7 -> 65.0 us, 40 of 500..9000 x 16 heads 52.9 -> 51.7, 64 of 2047..16383 x 128 221 -> 217.  (Shared tiles: a
+  // wave's queries are few, and the three tiles are asked for at once; the other way 2 rows x 16 heads lose 2 %.)
+  if constexpr (DS > 1) {  // (from registers)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pg[i] = page_of(t_begin + i * kTok);
   }
-  // Touch every Q^T register here: the compiler then waits for the Q loads now, instead of
-  // re-checking them with s_waitcnt vmcnt(0..4) inside the loop, where such a wait would also
-  // drain the copy queue.
+  copy(0);
+  if constexpr (DS > 1) {
+    copy(1);
+    copy(2);
+  }
 #pragma unroll
   for (int ks = 0; ks < kQ; ++ks) asm volatile("" ::"v"(qB[ks]));
-  // wait for the first tile (all but the 10 newest copies), then meet
+  wait_all_loads();
+  if constexpr (DS == 1) {
+    copy(1);
+    copy(2);
+  }
+  int pg_next = pg[3];
   constexpr int kAhead = 2 * (FP8 ? kF8CopiesPerWave : kCopiesPerWave);  // copies of the two tiles behind the next one
   // in the loop a step's id request precedes its copies: the ids it has to wait for are older than both tiles' copies
   constexpr int kAheadLoop = kAhead + (UNIFORM ? 0 : 1);
-  __builtin_amdgcn_s_waitcnt(0x0F70 | kAhead);
   __syncthreads();
   auto bare_barrier = [&]() {
     asm volatile("" ::: "memory");
@@ -764,7 +783,9 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
       const int cc = ln & 15, gg = ln >> 4;
       u32x4_t ml = {__float_as_uint(m), __float_as_uint(l), (uint32_t)(cc * kRowB + gg * 16),
                     (uint32_t)((4 * gg + (cc >> 2)) * kRowB + (cc & 3) * 8)};
-      u32x8_t ofs = {0, 0, 0, 0, 0, 0, 0, 0};
+      uint32_t none;
+      asm volatile("v_mov_b32 %0, 0" : "=v"(none));
+      u32x8_t ofs = {none, none, none, none, none, none, none, none};
       if constexpr (FP8) {
 #pragma unroll
         for (int n = 0; n < kF8CopiesPerWave; ++n) {
