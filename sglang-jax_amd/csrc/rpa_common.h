@@ -75,6 +75,24 @@ __device__ __forceinline__ u32x4_t row_of_16(u32x2_t a, u32x2_t b) {
   return w;
 }
 
+// 32 columns, lane (c = lane % 32, h = lane / 32) holding bytes 8 h .. of four 16-byte chunks of row c: then bytes row_of_32_at(lane) .. of
+// the 64, of row lane % 16 in `lower`, of row 16 + lane % 16 in `upper`.
+__device__ __forceinline__ int row_of_32_at(int lane) { return 16 * (lane >> 5) + 32 * ((lane >> 4) & 1); }
+
+__device__ __forceinline__ void row_of_32(const u32x2_t (&p)[4], u32x4_t& lower, u32x4_t& upper) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto x = __builtin_amdgcn_permlane32_swap(p[0][i], p[1][i], false, false);
+    const auto y = __builtin_amdgcn_permlane32_swap(p[2][i], p[3][i], false, false);
+    const auto lo = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
+    lower[i] = lo[0];
+    upper[i] = lo[1];
+    lower[2 + i] = hi[0];
+    upper[2 + i] = hi[1];
+  }
+}
+
 // x + the pair lane's x, likewise.
 __device__ __forceinline__ float swap_sum(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);

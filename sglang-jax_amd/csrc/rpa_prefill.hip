@@ -672,11 +672,12 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_async_kernel_wide(const Pr
   }
 
   // ---- lane (c, g) holds position r_lo + c, dims 16 j + 4 g + r
-  l += __shfl_xor(l, 16);
-  l += __shfl_xor(l, 32);
-  if (!active || row >= w.q_len) return;
+  l = swap_sum(swap16_sum(l));
+  if (!active) return;
+  const bool real = row < w.q_len;
   const int64_t out_row = (int64_t)(w.qg0 + row) * a.Hq + w.head;
   if (a.kv_splits > 1) {
+    if (!real) return;
     const int64_t slot = out_row * a.kv_splits + split;
     float* op = a.ws_o + slot * 256 + 4 * g;
 #pragma unroll
@@ -689,11 +690,13 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_async_kernel_wide(const Pr
   }
   const float vs = a.v_scale ? scalar_load_f32(a.v_scale + w.hk) : 1.0f;
   const float inv = a.sm.sink ? vs * sink_inverse(m * sc2, l, sink_logit(a.sm.sink, a.sm.round_logits, w.head)) : vs / l;
-  uint16_t* op = a.out + out_row * a.q_dim + 4 * g;
+  uint16_t* op = a.out + out_row * a.q_dim + 8 * g;
 #pragma unroll
-  for (int j = 0; j < 16; ++j)
-    if (16 * j + 4 * g < a.q_dim)
-      *reinterpret_cast<u32x2_t*>(op + 16 * j) = u32x2_t{pack_bf16x2(O[j][0] * inv, O[j][1] * inv), pack_bf16x2(O[j][2] * inv, O[j][3] * inv)};
+  for (int j = 0; j < 16; j += 2) {
+    const u32x4_t o = row_of_16(u32x2_t{pack_bf16x2(O[j][0] * inv, O[j][1] * inv), pack_bf16x2(O[j][2] * inv, O[j][3] * inv)},
+                                u32x2_t{pack_bf16x2(O[j + 1][0] * inv, O[j + 1][1] * inv), pack_bf16x2(O[j + 1][2] * inv, O[j + 1][3] * inv)});
+    if (real && 16 * j + 8 * g < a.q_dim) st16(op + 16 * j, o);
+  }
 }
 
 }  // namespace
