@@ -1455,7 +1455,7 @@ __device__ __forceinline__ int mla_tiles_per_wg(const MlaDecodeArgs& a, int tota
 template <bool FP8, class Segment>
 __device__ __forceinline__ void mla_balanced_body(const MlaDecodeArgs& a, Segment segment) {
   const int lane = threadIdx.x & 63;
-  const int wg = blockIdx.x;
+  int wg = blockIdx.x;  // this workgroup's share of the line
   const int units = (a.Hq + 127) / 128;
 #ifdef RPA_MLA_TRACE
   if (threadIdx.x == 0) rpa_mla_trace_buf[blockIdx.x & 1023][0][7] = wall_clock64();  // kernel entry
@@ -1474,6 +1474,14 @@ __device__ __forceinline__ void mla_balanced_body(const MlaDecodeArgs& a, Segmen
     total = __builtin_amdgcn_readfirstlane(total) * units;
   }
   const int pw = mla_tiles_per_wg(a, total);
+  // The shares of an XCD's workgroups (every eighth) one after the other on the line: a row's pieces then find its queries, 147 KB at 128 heads,
+  // in one L2.  10 rows of 500..5000 tokens x 16 heads 20.5 -> 19.7 us, 64 of 2000..16000 127.5 -> 126.2, 20 of 1000..9000 x 128 heads 55.8 -> 54.7; 3
+  // rows of 8000..16000 x 128 heads, 27 shares each, 38.1 against 38.9: not with fewer rows than XCDs.
+  const int per_xcd = ((total + pw - 1) / pw + 7) >> 3;  // (at most gridDim.x / 8: the shares are at most gridDim.x)
+  if (a.num_rows >= 8 && (gridDim.x & 7) == 0) {
+    if ((int)(blockIdx.x >> 3) >= per_xcd && blockIdx.x != 0) return;  // (the first one also writes the prefix sums of no work)
+    wg = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+  }
   if (wg == 0 && threadIdx.x < 64) {
     int base = 0;
     for (int s0 = 0; s0 < a.num_rows; s0 += 64) {
