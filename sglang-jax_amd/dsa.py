@@ -1,7 +1,7 @@
 """Sparse absorbed-MLA (DeepSeek sparse attention) on the dense MLA kernels: the reference's
 ``python/sgl_jax/srt/kernels/dsa/sparse_mla.py`` re-indexes the page table (or gathers rows) and
 hands the result to its dense kernel; here ``rpa_mla_sparse_attention`` writes one page table per query
-token and runs the dense kernel over it, three launches in all.  All index work stays
+token and runs the dense kernel over it, two launches in all.  All index work stays
 on the device (no host reads), so a call can sit inside a captured step.
 
 * ``compute_topk_pages``     sparse_mla.py:35-60   unique pages a top-k list touches
@@ -48,7 +48,7 @@ def compute_topk_pages(topk_indices, *, page_size: int, pages_per_seq: int, k_pa
 
 def _sparse(ql_nope, q_pe, new_kv_c, new_k_pe, cache_kv, kv_lens, topk, topk_is_pages, page_indices, cu_q_lens,
             cu_kv_lens, sm_scale, page_size, pages_per_seq, k_pages_max):
-    """The table of every query token's selection and the dense kernel over it (csrc/rpa_dsa.hip, rpa_mla.hip)."""
+    """The table of every query token's selection and the dense kernel over it (csrc/rpa_dsa.h, rpa_mla.hip)."""
     native = _lib.load_torch().sparse_mla
     rest = (sm_scale, page_size, pages_per_seq, k_pages_max)
     o = native(ql_nope, q_pe, new_kv_c, new_k_pe, cache_kv, kv_lens, topk, topk_is_pages, page_indices, cu_q_lens,
