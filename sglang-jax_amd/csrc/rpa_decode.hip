@@ -291,7 +291,7 @@ struct NewToken {
   __device__ __forceinline__ void store(const KvAddr& kv, const char* kh, const char* vh, int page, int tin, int lane) const {
     const int at = (lane & 15) * 16;
     if (lane < 32 && at < kRow)
-      st16(const_cast<char*>(lane < 16 ? kh : vh) + (int64_t)page * kv.page_stride + (int64_t)(tin * kv.tok_stride) + at, data);
+      st16(const_cast<char*>(lane < 16 ? kh : vh) + (int64_t)page * kv.page_stride + (int64_t)tin * kv.tok_stride + at, data);
   }
 };
 
@@ -1750,7 +1750,8 @@ __global__ __launch_bounds__(64, FP8 ? 2 : 1) void rpa_rows256_kernel(const Deco
     const int src_row = a.q_dim * (FP8 ? 1 : 2);  // the rest of a cached row is zero
     const int at = (lane & 31) * 16;
     const int slot = page_slot_of(sv, sv.last_tok);
-    const int64_t to = (int64_t)scalar_load_i32(sv.pages + __builtin_amdgcn_readfirstlane(slot)) * a.kv.page_stride + (int64_t)((sv.last_tok - slot * sv.page_size) * a.kv.tok_stride) + at;
+    const int64_t to = (int64_t)scalar_load_i32(sv.pages + __builtin_amdgcn_readfirstlane(slot)) * a.kv.page_stride +
+                       (int64_t)(sv.last_tok - slot * sv.page_size) * a.kv.tok_stride + at;
     const int64_t from = ((int64_t)tok_row * a.Hkv + hk) * src_row + at;
     u32x4_t x = {0u, 0u, 0u, 0u};
     if (at < src_row) x = ld16((lane < 32 ? a.new_k : a.new_v) + from);

@@ -2258,3 +2258,41 @@ def test_sequences_one_after_the_other(pkg, wl, gpu, monkeypatch, Hq, Hkv, q_len
 
     n = len(q_lens)
     assert torch.equal(run(0, n), torch.cat([run(i, i + 1) for i in range(n)]))
+
+
+@pytest.mark.parametrize("D,Hkv,P", [(256, 16, 131200), (128, 32, 131200), (128, 32, 131184)])
+def test_new_tokens_beyond_2_gib_of_a_page(pkg, gpu, D, Hkv, P):
+    """Pages of more than 2 GiB, rows behind a window that end beyond that: the byte offset of a token within its page takes more than 31
+    bits, for the new token's store as for the window's loads.  Nothing but the two slots changes."""
+    say(f"page of {P * Hkv * D * 4 / 2**30:.4f} GiB D={D} Hkv={Hkv}")
+    window, G, rows = 300, 2, 2
+    kv = [131130, 131079]
+    tok_bytes = Hkv * D * 4
+    assert all((n - 1) * tok_bytes >= 2**31 for n in kv) and P * tok_bytes < 2**32
+    gen = torch.Generator(device=gpu).manual_seed(5)
+
+    def draw(*shape):
+        return torch.randn(*shape, generator=gen, device=gpu).to(torch.bfloat16)
+
+    cache = torch.zeros(rows, P, 2 * Hkv, D, dtype=torch.bfloat16, device=gpu)
+    cache[:, P - 600 :] = draw(rows, 600, 2 * Hkv, D)
+    q, keys, values = draw(rows, G * Hkv, D), draw(rows, Hkv, D), draw(rows, Hkv, D)
+    expect = cache.clone()
+    table = [1, 0]
+    for i, n in enumerate(kv):
+        expect[table[i], n - 1, 0::2], expect[table[i], n - 1, 1::2] = keys[i], values[i]
+
+    def i32(x):
+        return torch.tensor(x, dtype=torch.int32, device=gpu)
+
+    poison_free_blocks(q)
+    out, after = pkg.ragged_paged_attention(
+        q, keys, values, cache, i32(kv), i32(table), i32([0, 1, 2]), i32([0, P, 2 * P]), (rows, rows, rows), sm_scale=D**-0.5,
+        sliding_window=window, max_kv_len=max(kv), max_q_len=1, host_kv_lens=np.array(kv, dtype=np.int32))
+    torch.cuda.synchronize()
+    for i, n in enumerate(kv):
+        seen = expect[table[i], n - window : n].float()
+        logits = torch.einsum("hgd,thd->hgt", q[i].float().view(Hkv, G, D), seen[:, 0::2]) * D**-0.5
+        want = torch.einsum("hgt,thd->hgd", torch.softmax(logits, -1), seen[:, 1::2])
+        assert_parity(out[i].float(), want.reshape(G * Hkv, D), **BF16_TOL)
+    assert torch.equal(after, expect)
