@@ -192,14 +192,16 @@ __device__ __forceinline__ void async_copy16(const void* gsrc, const void* lds_b
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0v), "v"(gsrc) : "memory", "m0");
 }
 
-// The same from a wave-uniform address and the lane's offset from it.
+// The same from a wave-uniform address and the lane's offset from it.  The address may come straight out of v_readfirstlane, and a
+// memory instruction may read what a vector instruction wrote to a scalar register five wait states later: s_mov is the first,
+// s_nop 3 the other four (and m0's).
 __device__ __forceinline__ void async_copy16_from(const char* base_uniform, uint32_t offset, const void* lds_base_uniform) {
   typedef const __attribute__((address_space(3))) char* lds_ptr_t;
   const uint32_t m0v = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)lds_base_uniform));
   const uint64_t a = reinterpret_cast<uint64_t>(base_uniform);
   const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a));
   const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a >> 32));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0v), "v"(offset), "s"((static_cast<uint64_t>(hi) << 32) | lo) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0v), "v"(offset), "s"((static_cast<uint64_t>(hi) << 32) | lo) : "memory", "m0");
 }
 
 // Eight query elements from dim d of a row of q_dim (a multiple of 8); dims past it are zero.

@@ -523,6 +523,41 @@ def test_a_copy_into_lds_finds_its_address(pkg):
     assert not short, (len(short), short[:3])
 
 
+def _scalar_registers(operands):
+    found = set()
+    for lo, hi, one in re.findall(r"\bs\[(\d+):(\d+)\]|\bs(\d+)\b", operands):
+        found |= {int(one)} if one else set(range(int(lo), int(hi) + 1))
+    return found | ({"vcc"} if "vcc" in operands else set())
+
+
+def test_a_memory_instruction_finds_its_scalars(pkg):
+    """A scalar register that a vector instruction wrote (v_readfirstlane) is read by a memory instruction no sooner than five wait states
+    later: what stands between counts one each, s_nop n counts n + 1.  The compiler keeps that for its own instructions, inline assembly
+    has to keep it by itself, whatever the compiler puts in front."""
+    readers, short = 0, []
+    for kernel, ins in _instructions():
+        written = {}  # scalar register -> wait states since a vector instruction wrote it
+        for op, operands in ins:
+            if re.match(r"(global|buffer|flat|scratch)_", op):
+                read = _scalar_registers(operands)
+                readers += bool(read)
+                if any(written.get(r, 5) < 5 for r in read):
+                    short.append((kernel, op, operands))
+            states = int(operands.split()[0], 0) + 1 if op == "s_nop" else 1
+            written = {r: n + states for r, n in written.items() if n + states < 5}
+            fields = re.split(r",\s*(?![^\[]*\])", operands)
+            if op.startswith("v_"):  # (carries and comparisons: the second operand, or the first)
+                wrote = _scalar_registers(fields[0])
+                if re.match(r"v_(add|sub|subrev|addc|subb|subbrev)_co|v_div_scale|v_mad_[iu]64", op) and len(fields) > 1:
+                    wrote |= _scalar_registers(fields[1])
+                written.update({r: 0 for r in wrote})
+            elif op.startswith("s_") and not re.match(r"s_(cmp|bitcmp|set|nop|wait)", op):
+                for r in _scalar_registers(fields[0]):  # (written anew by a scalar instruction)
+                    written.pop(r, None)
+    assert readers > 1000
+    assert not short, (len(short), short[:3])
+
+
 # ------------------------------------------------------------------ the shape table (csrc/rpa_shapes.h)
 def _shape_params(pkg, *, S, decode_end, T, Hq, Hkv, D=128, P=64, fp8=False, max_q=0, max_kv=0, sum_dec=0, **opts):
     p = base_params(pkg)
