@@ -392,7 +392,8 @@ RPA_API int rpa_mla_attention_update(const RpaMlaParams* p, const void* new_kv_c
  *   k_pages_max == 0  single tokens (sparse_mla.py:206-297): the valid entries of the selection, which come first; the
  *                     new row stands for the last of them and the cache is not written.
  * `p` is the batch as rpa_mla_decode takes it (ragged page table; kv_lens, cu_q_lens of num_seqs sequences; max_kv_len
- * and sum_kv_len are not read).  The new rows may both be NULL when the cache already holds every token.
+ * and sum_kv_len are not read; sliding_window counts tokens of the selection).  The new rows may both be NULL when the
+ * cache already holds every token.
  */
 typedef struct RpaMlaSparse {
   const int32_t* topk;       /* i32[T, topk_stride]: positions in the sequence, -1 = unused */

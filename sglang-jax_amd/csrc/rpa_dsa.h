@@ -33,13 +33,14 @@ struct Row {
   char* fresh;
 };
 
-// A piece of a row: tokens [t_begin, t_end) of kv_len.
+// A piece of a row: tokens [t_begin, t_end) of kv_len, those below t_lo behind the window.
 struct Piece {
-  int kv_len, t_begin, t_end;
+  int kv_len, t_lo, t_begin, t_end;
   int page_ids;  // lane's: of page t_begin / page size + lane, where the kernel keeps them in a register
 };
 __device__ __forceinline__ void cut(Piece& p, const MlaDecodeArgs& a, int split) {
-  p.t_begin = split * a.chunk;
+  p.t_lo = a.sm.window > 0 ? max(0, p.kv_len - a.sm.window) : 0;
+  p.t_begin = (p.t_lo & ~31) + split * a.chunk;  // (as the ordinary rows' pieces, and as the merge counts them)
   p.t_end = split == a.max_splits - 1 ? p.kv_len : min(p.kv_len, p.t_begin + a.chunk);
 }
 

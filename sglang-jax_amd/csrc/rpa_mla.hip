@@ -922,7 +922,7 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_decode_kernel(const MlaDecodeA
     MlaDecodeArgs b = a;
     // (behind the table's barrier: page ids are read as what nobody writes, and could be asked for in front of it)
     asm volatile("" : "+s"(b.pt.page_indices)::"memory");
-    mla_segment<UNIFORM, CAP, PIPE, FP8, DS, false, kIds>(b, mr, blockIdx.z * 128, 0, p.t_begin, p.t_end, dest, slot0, slot1, slot2, slot3, 1, p.page_ids);
+    mla_segment<UNIFORM, CAP, PIPE, FP8, DS, false, kIds>(b, mr, blockIdx.z * 128, p.t_lo, p.t_begin, p.t_end, dest, slot0, slot1, slot2, slot3, 1, p.page_ids);
     return;
   }
   if (a.rows_are_tokens) row_id = a.num_rows - 1 - row_id;
@@ -1400,7 +1400,7 @@ __global__ __launch_bounds__(256, 1) void rpa_mla_decode_wide_kernel(const MlaDe
     dest.base = ((int64_t)row_id * a.max_splits + split) * a.Hq;
     MlaDecodeArgs b = a;
     asm volatile("" : "+s"(b.pt.page_indices)::"memory");  // (as above)
-    mla_segment_wide<M32, false, P16>(b, mr, blockIdx.z * 128, 0, p.t_begin, p.t_end, dest, ring);
+    mla_segment_wide<M32, false, P16>(b, mr, blockIdx.z * 128, p.t_lo, p.t_begin, p.t_end, dest, ring);
     return;
   }
   if (a.rows_are_tokens) row_id = a.num_rows - 1 - row_id;

@@ -3,6 +3,7 @@ token-level selection against the restated sparse reference (dsa/ref.py:272-337)
 selection against the dense MLA oracle over the page lists worked out in plain loops
 (dsa/sparse_mla.py:107-175).  rtol = atol = 2e-2 (bf16)."""
 
+import ctypes
 import sys
 
 import numpy as np
@@ -186,3 +187,58 @@ def check_selections(pkg, wl, gpu, level, P, Hq, k, dtype, kv_lens, kp):
         assert torch.equal(cache_out.cpu().view(torch.uint8), stored.view(torch.uint8))
     torch.cuda.synchronize()
     assert_parity(got.cpu().float(), want.float(), **TOL)
+
+
+class SparseParams(ctypes.Structure):  # RpaMlaSparse of include/rpa.h
+    _fields_ = [("topk", ctypes.c_void_p)] + [(n, ctypes.c_int32) for n in (
+        "topk_count", "topk_stride", "topk_is_pages", "pages_per_seq", "k_pages_max", "num_page_indices")]
+
+
+@pytest.mark.parametrize("window", [1, 33, 700])
+@pytest.mark.parametrize("level,P,Hq,dtype", [
+    ("page", 64, 16, "bf16"), ("page", 64, 128, "bf16"), ("page", 16, 128, "bf16"), ("page", 24, 96, "bf16"), ("page", 32, 64, "e4m3"),
+    ("token", 64, 32, "bf16"), ("token", 16, 128, "e4m3"),
+])
+def test_a_window_over_a_selection(pkg, wl, gpu, level, P, Hq, dtype, window):
+    """The C entry takes the batch as rpa_mla_decode does, its window too: the last `window` tokens of a selection, in rows that stay
+    whole and in rows cut into pieces."""
+    kv_lens, k, kp = [1, 31, P + 1, 900, 5003], 2048, 40
+    b = batch(wl, kv_lens, P, 84, Hq=Hq)
+    S, pps = len(kv_lens), -(-max(kv_lens) // P)
+    topk_np = draw_topk(kv_lens, k, 9)
+    stored = b.cache_kv.to(torch.float8_e4m3fn if dtype == "e4m3" else torch.bfloat16)
+    say(f"dsa window {level} P={P} Hq={Hq} {dtype} window={window}")
+    if level == "token":
+        seen = np.full_like(topk_np, -1)
+        for i, n in enumerate(kv_lens):
+            valid = topk_np[i, : min(k, n)][-window:]
+            seen[i, : len(valid)] = valid
+        pages = torch.cat([b.page_indices, torch.zeros(pps, dtype=torch.int32)])
+        want = sparse_mla_ref(torch.cat([b.ql_nope, b.q_pe], dim=-1), stored.to(torch.bfloat16), b.kv_lens, torch.from_numpy(seen), pages,
+                              b.cu_q_lens, b.cu_kv_lens, [S, S, S], sm_scale=b.sm_scale, pages_per_seq=pps, v_dim=512)
+    else:
+        sp_len, sp_pages = page_level_metadata_ref(b.kv_lens.numpy(), topk_np, b.page_indices.numpy(), b.cu_q_lens.numpy(),
+                                                   b.cu_kv_lens.numpy(), page_size=P, pages_per_seq=pps, k_pages_max=kp,
+                                                   sentinel_page=stored.shape[0] - 1)
+        want, _ = ref_mla_ragged_paged_attention(
+            b.ql_nope, b.q_pe, None, None, stored.to(torch.bfloat16), torch.from_numpy(sp_len), torch.from_numpy(sp_pages).reshape(-1),
+            torch.arange(S + 1, dtype=torch.int32), [S, S, S], sm_scale=b.sm_scale, sliding_window=window)
+    g, cache, topk = b.to(gpu), stored.to(gpu), torch.from_numpy(topk_np).to(gpu)
+    out = torch.full_like(g.ql_nope, float("nan"))
+    p = pkg._lib.RpaMlaParams(
+        ql_nope=g.ql_nope.data_ptr(), q_pe=g.q_pe.data_ptr(), out=out.data_ptr(), cache_kv=cache.data_ptr(), kv_lens=g.kv_lens.data_ptr(),
+        page_indices=g.page_indices.data_ptr(), cu_q_lens=g.cu_q_lens.data_ptr(), cu_kv_lens=g.cu_kv_lens.data_ptr(), num_tokens=S,
+        num_seqs=S, num_q_heads=Hq, lkv_dim=512, rope_dim=64, row_stride=cache.shape[-1], rope_offset=512, page_size=P,
+        total_pages=cache.shape[0], sliding_window=window, sm_scale=b.sm_scale,
+        cache_dtype=pkg._lib.RPA_KV_FP8_E4M3 if dtype == "e4m3" else pkg._lib.RPA_KV_BF16)
+    s = SparseParams(topk=topk.data_ptr(), topk_count=k, topk_stride=k, pages_per_seq=pps, k_pages_max=kp if level == "page" else 0,
+                     num_page_indices=g.page_indices.numel())
+    lib = pkg._lib.load()
+    size, run = lib.rpa_mla_sparse_workspace_bytes, lib.rpa_mla_sparse_attention
+    size.restype, size.argtypes = ctypes.c_size_t, [ctypes.c_void_p] * 2
+    run.restype, run.argtypes = ctypes.c_int, [ctypes.c_void_p] * 5
+    ws = torch.full((size(ctypes.byref(p), ctypes.byref(s)),), 0xFF, dtype=torch.uint8, device=gpu)
+    p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
+    assert run(ctypes.byref(p), ctypes.byref(s), None, None, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert_parity(out.cpu().float(), want.float(), **TOL)
