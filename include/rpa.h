@@ -302,7 +302,8 @@ RPA_API int rpa_attention(const RpaParams* p, void* stream);
 /*
  * Which launch shape a call would take, as text: the row of the library's shape table (kernel family, query
  * positions x query heads x K/V tokens per workgroup, waves walked together, resident waves), the split plan
- * of the decode rows and the workspace behind it, and who leaves the new tokens of rpa_attention_update in the cache.
+ * of the decode rows and the workspace behind it, whether a prefill launch takes its sequences one after the other, and
+ * who leaves the new tokens of rpa_attention_update in the cache.
  * "whole call" stands in front where rpa_attention and rpa_attention_update run every query token as a row of the decode
  * kernels (few tokens on short contexts, workspace of rpa_workspace_bytes()); "decode" and "prefill" are then what
  * rpa_decode and rpa_prefill take.  The counterpart of the reference's get_tuned_block_sizes /

@@ -1202,6 +1202,7 @@ int rpa_describe_plan(const RpaParams* given, char* buf, size_t len) {
       const PrefillWorkspace w = prefill_workspace(p_in, a);
       put("prefill: shape=%s kernel=%s tile=%dx%dx%d kv_pieces_with_workspace=%d mask_bits=%s optional_workspace=%zu\n",
           r.name, kernel, r.tile_q, r.tile_heads, r.tile_kv, w.splits, w.bits_bytes ? "yes" : "no", w.total);
+      if (rpa::prefill_by_streams(a)) put("prefill, long sequences: one after the other\n");
       if (a.packed)
         put("prefill, small launch: kernel=rpa_prefill_packed_kernel instead, columns=%d tile=%dx%dx32\n", 32, 32 / a.G, a.G);
     }

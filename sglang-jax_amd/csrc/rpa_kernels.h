@@ -259,6 +259,8 @@ hipError_t launch_kv_write(const KvWriteArgs& a, hipStream_t stream);
 hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream);
 // The rows of the shape table (rpa_shapes.h) these launchers select for a call, RPA_* overrides applied.
 const ShapeRule& prefill_shape_of(const PrefillArgs& a);
+// Whether launch_prefill would take long sequences one after the other (streams_in_turn, rpa_prefill_common.h).
+bool prefill_by_streams(const PrefillArgs& a);
 ShapeKey mla_shape_key(const MlaDecodeArgs& a);
 unsigned mla_shape_skip(const MlaDecodeArgs& a, const Tuning& tune);
 // how query tokens of a chunk share a workgroup (0: they do not; 1, 2: eight waves; 3: wide workgroups)

@@ -1111,6 +1111,29 @@ size_t prefill_split_workspace_bytes(const PrefillArgs& a, int splits) {
   return splits > 1 ? (size_t)a.num_tokens * a.Hq * splits * (a.head_dim + 2) * sizeof(float) : 0;
 }
 
+static int64_t compiled_grid(PrefillArgs& a, int nseq, bool heads4, int& tiles, bool& by_level) {
+  const int bm = heads4 ? 32 : kBM;
+  tiles = (a.max_q_len + bm - 1) / bm;
+  // levels 0 .. ceil(max_kv_len / rows): only worth their empty workgroups when prefixes are
+  // not much longer than the chunks (else every tile of a sequence costs about the same anyway)
+  const bool level_order = tuning().prefill_level_order != 0;
+  const int levels = a.max_kv_len > 0 ? (a.max_kv_len + bm - 1) / bm + 1 : 0;
+  by_level = level_order && a.sm.mask_mode == 0 && levels > tiles && levels <= 2 * tiles + 2;
+  if (by_level) tiles = levels;
+  return prefill_grid(a, nseq, tiles, GridShape{bm, heads4 ? 4 : 1, a.head_dim == 256 ? 0 : 64, false});
+}
+
+bool prefill_by_streams(const PrefillArgs& call) {
+  PrefillArgs a = call;
+  const int nseq = a.seq_end - a.seq_begin;
+  if (nseq <= 0 || a.max_q_len <= 0 || a.packed) return false;
+  int tiles;
+  bool by_level;
+  if (takes_pipe_kernel(a)) prefill_pipe_grid(a, nseq, tuning().prefill_level_order != 0);
+  else compiled_grid(a, nseq, compiled_short_chunk_tile(a), tiles, by_level);
+  return a.map.block > 0;
+}
+
 hipError_t launch_prefill(const PrefillArgs& call, hipStream_t stream) {
   PrefillArgs a = call;
   const int nseq = a.seq_end - a.seq_begin;
@@ -1126,15 +1149,9 @@ hipError_t launch_prefill(const PrefillArgs& call, hipStream_t stream) {
     return launch_prefill_pipe(a, nseq, tuning().prefill_level_order != 0, stream);
   }
   const bool heads4 = compiled_short_chunk_tile(a);
-  const int bm = heads4 ? 32 : kBM;
-  int tiles = (a.max_q_len + bm - 1) / bm;
-  // levels 0 .. ceil(max_kv_len / rows): only worth their empty workgroups when prefixes are
-  // not much longer than the chunks (else every tile of a sequence costs about the same anyway)
-  const bool level_order = tuning().prefill_level_order != 0;
-  const int levels = a.max_kv_len > 0 ? (a.max_kv_len + bm - 1) / bm + 1 : 0;
-  const bool by_level = level_order && a.sm.mask_mode == 0 && levels > tiles && levels <= 2 * tiles + 2;
-  if (by_level) tiles = levels;
-  const int64_t grid = prefill_grid(a, nseq, tiles, heads4 ? 4 : 1, a.head_dim == 256 ? 0 : 64);
+  int tiles;
+  bool by_level;
+  const int64_t grid = compiled_grid(a, nseq, heads4, tiles, by_level);
   if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   // whether the rows that a wave brings in of a tile are one page's
   const int wave_rows = a.head_dim == 256 ? 8 : (a.fp8 || tuning().prefill_staged == 1) ? kBN : 16;

@@ -156,27 +156,45 @@ __device__ __forceinline__ Work decompose(const PrefillArgs& a, int tiles, int n
   return w;
 }
 
-// Whether a launch takes the order by streams (decompose): several sequences on a multiple of 8 kv heads, each XCD with more workgroups
-// than it has places for, and so much to read for one of them that four side by side do not stay in an XCD's 4 MB.  Known on the host
-// and of the chunks themselves (behind decode rows the bound on the lengths may be theirs).  In order of pairs -> by streams:
-//   4 chunks of 1900 .. 2048 tokens on 4096 .. 16384 x 32 / 8 heads 1500 -> 1382 us (4.2 GB past the L2s for 0.2 GB of cache, now 0.35),
-//   4 of 1024 on 4000 .. 12000 e4m3 605 -> 545, 2 of 2223 .. 2599 on 3471 .. 13887 x 16 / 8 heads 405 -> 369, 5 of 1000 .. 3000 on up to 8000
-//   394 -> 378, 2 of 1161 .. 1305 on 4260 x 32 / 8 237 -> 219, 8 of 512 on 8192 510 -> 500.
-// What it costs are the short tiles at the end of the launch: chunks of 1905 and 321 on 5811 e4m3 368 -> 380.  On up to 4600 tokens
-// the two orders are level or the order of pairs ahead (chunks of 29 .. 1946 on 276 58 against 61), and with 256-wide heads, one
-// workgroup to a CU, 0.95 .. 1.0.  Fewer kv heads would spread a sequence over the XCDs by its tiles: 0.72 .. 1.28 times as fast, by how
-// the tiles come out.
-inline bool streams_in_turn(const PrefillArgs& a, int nseq, int64_t grid, int slots) {
+// Whether a launch takes the order by streams (decompose): several sequences on a multiple of 8 kv heads with 4608 tokens or more to
+// read for one of them, and the workgroups that have a tile, `work`, fit into the places at once or are 5/3 of them and more.  Known on
+// the host and of the chunks themselves (behind decode rows the bound on the lengths may be theirs).
+// What it gives is one K/V on its way to an XCD at a time, where four side by side do not stay in 4 MB, and long sequences that start first
+// although they are few tiles.  What it costs is the end: the last sequence's workgroups start last, whatever they have to read, and
+// where they are the few of a second round they are waited for.  In order of pairs -> by streams, us, prefixes ragged / all 5000 .. 6000:
+//   fits         32 / 8 heads, 1905 + 60 tokens e4m3 323 -> 312, 40 / 8 heads, 1400 + 100 e4m3 371 -> 266 and bf16 283 -> 208
+//   more         4 chunks of 1900 .. 2048 x 32 / 8 1500 -> 1382 (4.2 GB past the L2s for 0.2 GB of cache, now 0.35), 4 of 1000 bf16
+//                571 -> 514 and e4m3 777 -> 680, with a cap 864 -> 750, 2 of 2400 x 24 / 8 648 -> 519 and e4m3 871 -> 698, 6 of 1500 x 16 / 8
+//                446 -> 406 and e4m3 590 -> 495, 5 of 500 .. 3000 x 64 / 16 1318 -> 1249;
+//                even prefixes are level, 0.97 .. 1.06; at worst 2400 on 3400 and 2300 on 13800 x 32 / 16 771 -> 816 (the longer first
+//                781 -> 747), 1900 + 300 + 200 x 64 / 16 e4m3 648 -> 685
+//   between      e4m3 1905 + 321 on 5811 375 -> 386, 1905 + 700 400 -> 439, 1500 + 900 386 -> 432, bf16 with a cap 394 -> 405, 3 of 2000 x 16 / 8
+//                e4m3 382 -> 410; others gain (1905, 321, 400 e4m3 501 -> 474), and nothing that the host knows tells them apart.
+//                The assembly kernel on four heads or more per kv head waits for the L2s most and does gain: 1905 + 321 bf16 309 -> 286,
+//                1500 + 900 314 -> 286, 900 + 1905 328 -> 309, 64 / 8 900 + 100 297 -> 272, at worst 1905 + 1200 347 -> 351.
+// On up to 4600 tokens the two orders are level or the order of pairs ahead (chunks of 29 .. 1946 on 276 58 against 61), and with 256-wide
+// heads, one workgroup to a CU, 0.95 .. 1.0.  Fewer kv heads would spread a sequence over the XCDs by its tiles: 0.72 .. 1.28 times as
+// fast, by how the tiles come out.  (The bound is one of tokens for both element types: e4m3 on 4000 .. 6000, 4 of 1000, 464 -> 448.)
+struct GridShape {
+  int bm, heads;  // query positions and heads of a workgroup
+  int slots;      // workgroups that an XCD has places for, of a kernel that knows the order by streams (0: it does not)
+  bool assembly;
+};
+inline bool streams_in_turn(const PrefillArgs& a, int nseq, int64_t grid, const GridShape& s) {
+  if (s.slots <= 0 || nseq <= 1 || a.Hkv % 8 != 0 || a.dist || a.seq_begin != 0) return false;
   const int64_t seen = a.sm.window > 0 ? std::min<int64_t>(a.max_kv_len, (int64_t)a.sm.window + kBM) : a.max_kv_len;
-  return nseq > 1 && a.Hkv % 8 == 0 && !a.dist && a.seq_begin == 0 && seen >= 4608 && grid > 8ll * slots;
+  const int64_t places = 8ll * s.slots;
+  if (seen < 4608 || grid <= places) return false;
+  const int groups = a.G / s.heads;
+  const int64_t work = ((int64_t)a.num_tokens + nseq * (s.bm / 2)) / s.bm * groups * a.Hkv;  // (a sequence's last tile is half full on average)
+  return (s.assembly && groups >= 4) || work <= places || 3 * work >= 5 * places;
 }
 
 // Workgroups of a launch of `tiles` tiles, and the divisors of their order (see decompose).
-// slots: workgroups that an XCD has places for, of a kernel that knows the order by streams (0: it does not).
 // With fewer than 8 units their heads go to XCDs of their own: what few pairs there are would leave XCDs without work (2 chunks of
 // 36 .. 171 tokens x 8 / 1 heads 42.8 -> 31.5 us).
-inline int64_t prefill_grid(PrefillArgs& a, int nseq, int tiles, int heads, int slots = 0) {
-  const int groups = a.G / heads, units = nseq * a.Hkv;
+inline int64_t prefill_grid(PrefillArgs& a, int nseq, int tiles, const GridShape& s) {
+  const int groups = a.G / s.heads, units = nseq * a.Hkv;
   a.map.apart = units < 8;
   const int span = a.map.apart ? 1 : groups, per_kv = groups / span;
   a.map.groups = fast_div(span);
@@ -186,8 +204,8 @@ inline int64_t prefill_grid(PrefillArgs& a, int nseq, int tiles, int heads, int 
   a.map.nseq = fast_div(nseq);
   a.map.block = 0;
   const int64_t grid = ((int64_t)units * per_kv * tiles + 7) / 8 * 8 * span;
-  if (slots > 0 && streams_in_turn(a, nseq, grid, slots)) {
-    const int most = std::max(1, slots / groups), rounds = (tiles + most - 1) / most, m = a.Hkv / 8;
+  if (streams_in_turn(a, nseq, grid, s)) {
+    const int most = std::max(1, s.slots / groups), rounds = (tiles + most - 1) / most, m = a.Hkv / 8;
     a.map.block = (tiles + rounds - 1) / rounds;
     a.map.run = fast_div(a.map.block);
     a.map.seq_round = fast_div(a.map.block * m);
@@ -740,6 +758,13 @@ __device__ __forceinline__ void async_copy_tile(char* lds_k, char* lds_v, const 
 // rpa_prefill_pipe.hip: the software-pipelined kernel for the plain causal bf16 case
 bool prefill_pipe_applies(const PrefillArgs& a);
 hipError_t launch_prefill_pipe(const PrefillArgs& a, int nseq, bool level_order, hipStream_t stream);
+// What the pipelined kernel is launched as; sets a.map.
+struct PipeGrid {
+  int nq, tiles;
+  bool heads4, by_level;
+  int64_t grid;
+};
+PipeGrid prefill_pipe_grid(PrefillArgs& a, int nseq, bool level_order);
 int prefill_pipe_kv_splits(const PrefillArgs& a, int nseq, double* us = nullptr);
 
 // rpa_prefill_packed.hip: 32 (position, head) columns per workgroup, whose waves walk different tiles

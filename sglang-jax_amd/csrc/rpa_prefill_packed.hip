@@ -509,7 +509,7 @@ hipError_t launch_prefill_packed(const PrefillArgs& call, int nseq, hipStream_t 
   PrefillArgs a = call;
   const int per = kCols / a.G;
   const int tiles = (a.max_q_len + per - 1) / per;
-  const int64_t grid = prefill_grid(a, nseq, tiles, a.G);
+  const int64_t grid = prefill_grid(a, nseq, tiles, GridShape{per, a.G, 0, false});
   if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   const bool cut = a.kv_splits > 1;
   if (cut && (!a.ws_o || !a.ws_ml || a.kv_splits > 64)) return hipErrorInvalidValue;

@@ -565,22 +565,31 @@ int prefill_pipe_kv_splits(const PrefillArgs& a, int nseq, double* us) {
   return kv_pieces(a, nseq, heads4 ? 32 : 128, heads4 ? 4 : 1, 0.8, us);
 }
 
+PipeGrid prefill_pipe_grid(PrefillArgs& a, int nseq, bool level_order) {
+  PipeGrid g;
+  const int force_nq = forced_nq();
+  g.nq = force_nq ? force_nq : 1;
+  // Tile by shape (the reference's per-shape block sizes, tuned_block_sizes.py, have this one counterpart
+  // here): chunks of at most 64 tokens take 32 positions x 4 heads per workgroup when the heads come in fours
+  g.heads4 = short_chunk_tile(a, g.nq);
+  const int bm = g.heads4 ? 32 : 128 * g.nq;
+  g.tiles = (a.max_q_len + bm - 1) / bm;
+  const int levels = a.max_kv_len > 0 ? (a.max_kv_len + bm - 1) / bm + 1 : 0;
+  g.by_level = level_order && levels > g.tiles && levels <= 2 * g.tiles + 2;
+  if (g.by_level) g.tiles = levels;
+  g.grid = prefill_grid(a, nseq, g.tiles, GridShape{bm, g.heads4 ? 4 : 1, 64, true});
+  return g;
+}
+
 hipError_t launch_prefill_pipe(const PrefillArgs& call, int nseq, bool level_order, hipStream_t stream) {
   PrefillArgs a = call;
-  const int force_nq = forced_nq();
   // a half's row sum above the limit sends a wave through the rescaling path (testing knob: -1 = always)
   const float limit = tuning().prefill_pipe_limit != 0.f ? tuning().prefill_pipe_limit : kRowSumLimit;
   const bool masked = tuning().prefill_pipe_masked != 0;  // the steps on the causal diagonal in assembly too
-  const int nq = force_nq ? force_nq : 1;
-  // Tile by shape (the reference's per-shape block sizes, tuned_block_sizes.py, have this one counterpart
-  // here): chunks of at most 64 tokens take 32 positions x 4 heads per workgroup when the heads come in fours
-  const bool heads4 = short_chunk_tile(a, nq);
-  const int bm = heads4 ? 32 : 128 * nq;
-  int tiles = (a.max_q_len + bm - 1) / bm;
-  const int levels = a.max_kv_len > 0 ? (a.max_kv_len + bm - 1) / bm + 1 : 0;
-  const bool by_level = level_order && levels > tiles && levels <= 2 * tiles + 2;
-  if (by_level) tiles = levels;
-  const int64_t grid = prefill_grid(a, nseq, tiles, heads4 ? 4 : 1, 64);
+  const PipeGrid shape = prefill_pipe_grid(a, nseq, level_order);
+  const int nq = shape.nq, tiles = shape.tiles;
+  const bool heads4 = shape.heads4, by_level = shape.by_level;
+  const int64_t grid = shape.grid;
   if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   const dim3 g((unsigned)(grid + a.write_blocks)), blk(256);
   const bool win = a.sm.window > 0;

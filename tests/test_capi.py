@@ -628,6 +628,28 @@ def test_described_plan_names_what_runs(pkg):
         assert kernel in text and "written by rpa_kv_write_kernel, in front" in text
 
 
+@pytest.mark.parametrize("chunks,longest,Hq,Hkv,opts,streams", [
+    ([1900, 1980, 2020, 2048], 18432, 32, 8, {}, True), ([1024, 1000, 1020, 1010], 13000, 32, 8, dict(fp8=True), True),
+    # a round and a bit of the compiled kernels: the last sequence's workgroups would be waited for
+    ([1905, 321], 7716, 32, 8, dict(fp8=True), False), ([1905, 700], 7716, 32, 8, dict(fp8=True), False), ([1905, 321], 7716, 32, 8, dict(soft_cap=30.0), False),
+    ([1905, 321], 7716, 32, 8, {}, True),  # the assembly kernel
+    ([1905, 60], 7716, 32, 8, dict(fp8=True), True),  # all at once
+    ([1905, 1200], 7716, 32, 8, dict(fp8=True), False), ([1905, 1600], 7716, 32, 8, dict(fp8=True), True),  # 1.56 and 1.75 rounds
+    # fewer heads per kv head
+    ([2000] * 3, 7000, 16, 8, {}, False), ([2400, 2300], 16100, 24, 8, {}, True), ([1500] * 6, 7500, 16, 8, {}, True),
+    # 4608 tokens, behind a window too; one sequence; kv heads that are not in eights; 256-wide heads
+    ([2000] * 4, 4607, 32, 8, {}, False), ([2000] * 4, 4608, 32, 8, {}, True), ([2000] * 4, 9000, 32, 8, dict(sliding_window=4479), False),
+    ([2000] * 4, 9000, 32, 8, dict(sliding_window=4480), True), ([4000], 9000, 32, 8, {}, False), ([2000] * 4, 9000, 16, 4, {}, False),
+    ([2000] * 4, 9000, 32, 8, dict(D=256), False),
+])
+def test_sequences_one_after_the_other_by_their_work(pkg, chunks, longest, Hq, Hkv, opts, streams):
+    """The order by streams: as many workgroups as fit at once, or 5/3 of them and more; on the assembly kernel with four heads or
+    more per kv head in between too."""
+    text = pkg._lib.describe_plan(_shape_params(pkg, S=len(chunks), decode_end=0, T=sum(chunks), Hq=Hq, Hkv=Hkv, max_q=max(chunks),
+                                                max_kv=longest, **opts))
+    assert ("\nprefill, long sequences: one after the other\n" in text) == streams, text
+
+
 def test_plans_on_both_sides_of_their_rules(pkg, monkeypatch):
     """Prefill launches that the tiles of 128 positions leave idle, rows of one length in a mostly empty last round, and the
     pieces of 256-wide rows with what they need of a workspace."""
