@@ -577,7 +577,7 @@ PipeGrid prefill_pipe_grid(PrefillArgs& a, int nseq, bool level_order) {
   const int levels = a.max_kv_len > 0 ? (a.max_kv_len + bm - 1) / bm + 1 : 0;
   g.by_level = level_order && levels > g.tiles && levels <= 2 * g.tiles + 2;
   if (g.by_level) g.tiles = levels;
-  g.grid = prefill_grid(a, nseq, g.tiles, GridShape{bm, g.heads4 ? 4 : 1, 64, true});
+  g.grid = prefill_grid(a, nseq, g.tiles, GridShape{bm, g.heads4 ? 4 : 1, g.nq == 2 ? 32 : 64, true});  // (one or two workgroups per CU: the launch bounds)
   return g;
 }
 

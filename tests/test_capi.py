@@ -650,6 +650,14 @@ def test_sequences_one_after_the_other_by_their_work(pkg, chunks, longest, Hq, H
     assert ("\nprefill, long sequences: one after the other\n" in text) == streams, text
 
 
+def test_sequences_one_after_the_other_on_workgroups_of_256_rows(pkg, monkeypatch):
+    """A kernel with one workgroup per CU has half the places: 384 workgroups of 256 rows are more than fit."""
+    p = _shape_params(pkg, S=3, decode_end=0, T=3072, Hq=32, Hkv=8, max_q=1024, max_kv=6024)
+    for rows_in_128s in ("1", "2"):
+        monkeypatch.setenv("RPA_PREFILL_PIPE_NQ", rows_in_128s)
+        assert "one after the other" in pkg._lib.describe_plan(p)
+
+
 def test_plans_on_both_sides_of_their_rules(pkg, monkeypatch):
     """Prefill launches that the tiles of 128 positions leave idle, rows of one length in a mostly empty last round, and the
     pieces of 256-wide rows with what they need of a workspace."""

@@ -2233,7 +2233,7 @@ def test_head_dim_256_rows_bring_their_tokens(pkg, wl, gpu, Hq, Hkv, P, D, on_de
 
 @pytest.mark.parametrize("Hq,Hkv,q_lens,kv_lens,fp8", [
     (32, 8, [1300, 1299, 1], [5000, 1299, 4700], False), (64, 16, [600, 129, 640, 640], [5300, 4800, 640, 4609], False),
-    (40, 8, [2200, 130, 1], [2200, 4700, 1], False), (32, 8, [900, 1000, 128], [4700, 1000, 4900], True),
+    (40, 8, [2200, 130, 1], [2200, 4700, 1], False), (64, 16, [900, 1000, 128], [4700, 1000, 4900], True),
 ])
 def test_sequences_one_after_the_other(pkg, wl, gpu, monkeypatch, Hq, Hkv, q_lens, kv_lens, fp8):
     """Long sequences take the launch's workgroups in turn: the same rows, bit for bit, as each sequence in a call of its own (one
@@ -2296,3 +2296,54 @@ def test_new_tokens_beyond_2_gib_of_a_page(pkg, gpu, D, Hkv, P):
         want = torch.einsum("hgt,thd->hgd", torch.softmax(logits, -1), seen[:, 1::2])
         assert_parity(out[i].float(), want.reshape(G * Hkv, D), **BF16_TOL)
     assert torch.equal(after, expect)
+
+
+SHORT = [64 if i % 3 else 33 for i in range(56)]
+
+
+@pytest.mark.parametrize("kernel,P,Hq,Hkv,q_lens,kv_lens,opts", [
+    ("pipe", 64, 32, 8, [700, 300, 513, 900], [5000, 5300, 513, 1700], dict(nq="2")),
+    ("pipe", 64, 32, 8, [1300, 640, 129], [6000, 5200, 129], dict(window=4700)),
+    ("pipe", 64, 32, 8, SHORT, [4700 if i == 9 else 70 + i for i in range(56)], {}),
+    ("async", 64, 64, 16, [600, 129, 640, 640], [5300, 4800, 640, 4609], dict(cap=30.0)),
+    ("async", 24, 64, 8, [1000, 129, 640, 640], [6100, 5800, 640, 4609], dict(window=4650, cap=30.0)),
+    ("async", 64, 32, 8, SHORT, [4700 if i == 40 else 70 + i for i in range(56)], dict(cap=30.0)),
+    ("staged", 64, 64, 16, [600, 129, 640, 640], [5300, 4800, 640, 4609], dict(fp8=True)),
+    ("staged", 16, 64, 8, [1000, 129, 640, 640], [6100, 5800, 640, 4609], dict(fp8=True, window=4650, cap=30.0)),
+    ("staged", 64, 32, 8, SHORT, [4700 if i == 0 else 70 + i for i in range(56)], dict(fp8=True)),
+])
+def test_sequences_one_after_the_other_in_every_kernel(pkg, wl, gpu, monkeypatch, kernel, P, Hq, Hkv, q_lens, kv_lens, opts):
+    """The order by streams on every kernel that knows it and on its options: workgroups of 256 rows, tiles of 32 positions x 4 heads, windows,
+    the soft cap, pages of any size.  The rows are those of each sequence in a call of its own, bit for bit."""
+    from test_capi import _shape_params
+
+    fp8, window, cap = opts.get("fp8", False), opts.get("window"), opts.get("cap")
+    say(f"streams {kernel} {Hq}/{Hkv} P={P} {opts}")
+    monkeypatch.setenv("RPA_PREFILL_SPLITS", "0")
+    monkeypatch.setenv("RPA_PREFILL_PACKED", "0")
+    if "nq" in opts:
+        monkeypatch.setenv("RPA_PREFILL_PIPE_NQ", opts["nq"])
+    n = len(q_lens)
+    plan = pkg._lib.describe_plan(_shape_params(pkg, S=n, decode_end=0, T=sum(q_lens), Hq=Hq, Hkv=Hkv, P=P, fp8=fp8, max_q=max(q_lens),
+                                                max_kv=max(kv_lens), sliding_window=window or 0, soft_cap=cap or 0.0))
+    assert f"kernel=rpa_prefill_{kernel}_kernel " in plan and "one after the other" in plan, plan
+    b = wl.make_batch("streams", q_lens, kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=29,
+                      kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+    g = b.to(gpu)
+
+    def run(first, last):
+        q0, q1 = int(b.cu_q_lens[first]), int(b.cu_q_lens[last])
+        p0, p1 = int(b.cu_kv_lens[first]) // P, int(b.cu_kv_lens[last]) // P
+        poison_free_blocks(g.q)
+        out, _ = pkg.ragged_paged_attention(
+            g.q[q0:q1].contiguous(), None, None, g.kv_cache, g.kv_lens[first:last].contiguous(), g.page_indices[p0:p1].contiguous(),
+            g.cu_q_lens[first : last + 1] - q0, g.cu_kv_lens[first : last + 1] - p0 * P, (0, 0, last - first), sm_scale=b.sm_scale,
+            k_scale=g.k_scale, v_scale=g.v_scale, max_kv_len=max(kv_lens), max_q_len=max(q_lens), sliding_window=window, soft_cap=cap)
+        torch.cuda.synchronize()
+        return out.cpu()
+
+    together, alone = run(0, n), torch.cat([run(i, i + 1) for i in range(n)])
+    assert torch.equal(together, alone)
+    assert_parity(together.float(), ref_ragged_paged_attention_fused(
+        b.q, b.kv_cache, b.kv_lens, b.padded_page_table(), b.cu_q_lens, [n], sm_scale=b.sm_scale, sliding_window=window, soft_cap=cap,
+        k_scale=b.k_scale, v_scale=b.v_scale).float(), **(FP8_TOL if fp8 else BF16_TOL))
