@@ -104,7 +104,7 @@ __device__ __forceinline__ int block_scan(int x, int& total, int* wave_sums) {
     if (w < wave) before += wave_sums[w];
     all += wave_sums[w];
   }
-  total = all;
+  total = __builtin_amdgcn_readfirstlane(all);  // (out of LDS: the compiler would take it, and every length and address after it, for the lane's own)
   return before + incl - x;
 }
 

@@ -558,6 +558,26 @@ def test_a_memory_instruction_finds_its_scalars(pkg):
     assert not short, (len(short), short[:3])
 
 
+def test_bases_of_latent_tiles_are_worked_out_by_scalar_instructions(pkg):
+    """Where a tile begins is the same for all lanes, and the MLA kernels keep it known to the compiler: no copy's scalar base comes back
+    from vector registers (a row length read from LDS made every address of the sparse kernels the lane's own)."""
+    copies, returned = 0, []
+    for kernel, ins in _instructions():
+        from_lanes = set()
+        for op, operands in ins if "mla" in kernel else ():
+            if "_load_lds_" in op and (base := _scalar_registers(operands)):
+                copies += 1
+                if base & from_lanes:
+                    returned.append((kernel, operands))
+            first = _scalar_registers(operands.split(",")[0])
+            if op.startswith(("v_readfirstlane", "v_readlane")):
+                from_lanes |= first
+            elif op.startswith("s_") and not re.match(r"s_(cmp|bitcmp|set|nop|wait)", op):
+                from_lanes -= first
+    assert copies > 1000
+    assert not returned, (len(returned), returned[:3])
+
+
 # ------------------------------------------------------------------ the shape table (csrc/rpa_shapes.h)
 def _shape_params(pkg, *, S, decode_end, T, Hq, Hkv, D=128, P=64, fp8=False, max_q=0, max_kv=0, sum_dec=0, **opts):
     p = base_params(pkg)
