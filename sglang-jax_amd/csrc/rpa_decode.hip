@@ -136,7 +136,7 @@ __device__ __forceinline__ void load_block(KvRegs<FP8>& r, const DecodeArgs& a, 
     } else {
       const int slot = page_slot_of(s, tok);
       const int pg = WINDOW ? win[slot - win_first] : s.pages[slot];
-      at = cached + (int64_t)pg * kv.page_stride + (int64_t)((tok - slot * s.page_size) * kv.tok_stride + lane_bytes);
+      at = cached + (int64_t)pg * kv.page_stride + (int64_t)(tok - slot * s.page_size) * kv.tok_stride + lane_bytes;
     }
     if constexpr (FRESH) {
       const char* new_at = fresh + (int64_t)(s.fresh_row + (tok - s.fresh_first) * a.Hkv) * (FP8 || HALF ? 128 : 256) + lane_bytes;

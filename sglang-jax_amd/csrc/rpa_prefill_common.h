@@ -63,7 +63,7 @@ __device__ __forceinline__ int64_t row_offset(const TileSrc& s, const KvAddr& kv
   tok = min(tok, s.last_tok);
   if constexpr (UNIFORM) {
     const int page_tok0 = page_slot(s, tb) * s.page_size;  // wave-uniform
-    return (int64_t)page * kv.page_stride + (int64_t)((tok - page_tok0) * kv.tok_stride);
+    return (int64_t)page * kv.page_stride + (int64_t)(tok - page_tok0) * kv.tok_stride;
   } else {
     return (int64_t)page * kv.page_stride + (int64_t)(tok - page_slot(s, tok) * s.page_size) * kv.tok_stride;
   }

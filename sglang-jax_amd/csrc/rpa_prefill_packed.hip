@@ -88,7 +88,7 @@ struct PackedFeed {
       for (int n = 0; n < N; ++n) {
         const int tok = min(tb + row_of(n, lane), s.last_tok), ps = page_slot(s, tok);
         const int id = *(__attribute__((address_space(3))) const int32_t*)(lds_t)(uintptr_t)(ids + 4u * (uint32_t)(ps - page_slot(s, tb)));
-        row[n] = (int64_t)id * kv.page_stride + (int64_t)((tok - ps * s.page_size) * kv.tok_stride);
+        row[n] = (int64_t)id * kv.page_stride + (int64_t)(tok - ps * s.page_size) * kv.tok_stride;
       }
     } else {
       const int ps = __builtin_amdgcn_readfirstlane(page_slot(s, tb));

@@ -2260,7 +2260,7 @@ def test_sequences_one_after_the_other(pkg, wl, gpu, monkeypatch, Hq, Hkv, q_len
     assert torch.equal(run(0, n), torch.cat([run(i, i + 1) for i in range(n)]))
 
 
-@pytest.mark.parametrize("D,Hkv,P", [(256, 16, 131200), (128, 32, 131200), (128, 32, 131184)])
+@pytest.mark.parametrize("D,Hkv,P", [(256, 16, 131200), (128, 32, 131200), (128, 32, 131184), (128, 32, 131201), (256, 16, 131201)])
 def test_new_tokens_beyond_2_gib_of_a_page(pkg, gpu, D, Hkv, P):
     """Pages of more than 2 GiB, rows behind a window that end beyond that: the byte offset of a token within its page takes more than 31
     bits, for the new token's store as for the window's loads.  Nothing but the two slots changes."""
@@ -2347,3 +2347,50 @@ def test_sequences_one_after_the_other_in_every_kernel(pkg, wl, gpu, monkeypatch
     assert_parity(together.float(), ref_ragged_paged_attention_fused(
         b.q, b.kv_cache, b.kv_lens, b.padded_page_table(), b.cu_q_lens, [n], sm_scale=b.sm_scale, sliding_window=window, soft_cap=cap,
         k_scale=b.k_scale, v_scale=b.v_scale).float(), **(FP8_TOL if fp8 else BF16_TOL))
+
+
+@pytest.mark.parametrize("kernel,P,fp8,D,opts", [
+    ("packed", 131201, False, 128, {}), ("packed", 131200, True, 128, {}), ("async", 131200, False, 128, {}),
+    ("async", 131201, False, 128, {}), ("staged", 131200, True, 128, {}), ("staged", 131201, True, 128, dict(cap=30.0)),
+    ("async", 131200, False, 256, {}), ("async", 131201, True, 256, dict(cap=30.0)),
+])
+def test_chunks_beyond_2_gib_of_a_page(pkg, gpu, monkeypatch, kernel, P, fp8, D, opts):
+    """Chunks behind a window on pages of more than 2 GiB that end beyond that: where a tile's rows begin takes more than 31 bits."""
+    Hkv, G, window, cap = (2 if fp8 else 1) * 32 * 128 // D, 2, 300, opts.get("cap")
+    tok_bytes = Hkv * D * 2 * (1 if fp8 else 2)
+    kv, new = [131190, 131111], [60, 33]
+    assert min(n - window - 60 for n in kv) * tok_bytes < 2**31 <= (min(kv) - 33) * tok_bytes and P * tok_bytes < 2**32
+    say(f"chunk on a page of {P * tok_bytes / 2**30:.4f} GiB {kernel} fp8={fp8} D={D} {opts}")
+    if kernel != "packed":
+        monkeypatch.setenv("RPA_PREFILL_PACKED", "0")
+    gen = torch.Generator(device=gpu).manual_seed(6)
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    first = 130700
+    part = torch.randn(2, P - first, 2 * Hkv, D, generator=gen, device=gpu).to(dt)
+    cache = torch.zeros(2, P, 2 * Hkv, D, dtype=torch.uint8 if fp8 else torch.int16, device=gpu)
+    cache[:, first:] = part.view(cache.dtype)
+    cache = cache.view(dt)
+    q = torch.randn(sum(new), G * Hkv, D, generator=gen, device=gpu).to(torch.bfloat16)
+    table = [1, 0]
+
+    def i32(x):
+        return torch.tensor(x, dtype=torch.int32, device=gpu)
+
+    poison_free_blocks(q)
+    out, _ = pkg.ragged_paged_attention(
+        q, None, None, cache, i32(kv), i32(table), i32([0, new[0], sum(new)]), i32([0, P, 2 * P]), (0, 0, 2), sm_scale=D**-0.5,
+        sliding_window=window, soft_cap=cap, max_kv_len=max(kv), max_q_len=max(new))
+    torch.cuda.synchronize()
+    t = 0
+    for i, n in enumerate(kv):
+        rows = part[table[i], : n - first].float()
+        at = torch.arange(first, n, device=gpu)
+        for j in range(new[i]):
+            pos = n - new[i] + j
+            logits = torch.einsum("hgd,thd->hgt", q[t].float().view(Hkv, G, D), rows[:, 0::2]) * D**-0.5
+            if cap:
+                logits = cap * torch.tanh(logits / cap)
+            logits = logits.masked_fill((at > pos) | (at <= pos - window), float("-inf"))
+            want = torch.einsum("hgt,thd->hgd", torch.softmax(logits, -1), rows[:, 1::2])
+            assert_parity(out[t].float(), want.reshape(G * Hkv, D), **(FP8_TOL if fp8 else BF16_TOL))
+            t += 1
