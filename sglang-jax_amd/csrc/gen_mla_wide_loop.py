@@ -91,7 +91,7 @@ OFS = 216                    # one operand of 16: 10 per-lane copy offsets, scra
 NEGM = [226, 227]
 PS, KADDR, VADDR, D = 228, 229, 230, 231
 OFSL = 232                   # one operand of 16: the 10 offsets with rows clamped to the row's last token, scratch behind
-A, T0, T1, KADDR2 = 242, 243, 244, 245
+A, T0, T1 = 242, 243, 244
 TR = [246, 247]              # temporaries of the accumulator rescale
 NUM_VGPR = 248
 

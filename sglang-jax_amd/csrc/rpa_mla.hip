@@ -1927,7 +1927,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   }
   if (a.fp8) {  // e4m3 caches
     if (a.balanced) {
-        if (pipe) {
+      if (pipe) {
         launch_shares<true, false, true, true>(a, stream);
       } else if (uniform) {
         if (cap) launch_shares<true, true, false, true>(a, stream);
