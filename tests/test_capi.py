@@ -626,10 +626,12 @@ def test_described_plan_names_what_runs(pkg):
     d, tail = pkg._lib.describe_plan, pkg._lib.RPA_PARAMS_TAIL
     wide = d(_shape_params(pkg, S=6, decode_end=4, T=304, Hq=16, Hkv=4, D=256, max_q=200, max_kv=900, sum_dec=3000))
     assert "kernel=rpa_prefill_async_kernel_wide " in wide and "whole call" not in wide
-    # decode rows only: their kernels write the tokens; with chunks behind them, or 256-wide heads, a launch in front does
+    # decode rows only: their kernels write the tokens; with chunks behind them, or 256-wide heads and more than 768 MB, a launch in front does
     rows = dict(S=64, decode_end=64, T=64, Hq=32, Hkv=8, max_kv=4000, sum_dec=130000)
     assert d(_shape_params(pkg, **rows)).endswith("new tokens: written by the decode kernels\n")
     assert "written by rpa_kv_write_kernel, in front" in d(_shape_params(pkg, D=256, **rows))
+    assert d(_shape_params(pkg, D=256, **{**rows, "sum_dec": 90000})).endswith("new tokens: written by the decode kernels\n")
+    assert d(_shape_params(pkg, D=256, sliding_window=1024, **rows)).endswith("new tokens: written by the decode kernels\n")
     mixed = dict(S=64, decode_end=56, T=8760, Hq=32, Hkv=8, max_q=2048, max_kv=4096, sum_dec=130000)
     assert "written by rpa_kv_write_kernel, in front" in d(_shape_params(pkg, **mixed))
     bucket = d(_shape_params(pkg, distribution=0x1000, **mixed))
