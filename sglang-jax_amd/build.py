@@ -17,7 +17,7 @@ OUT_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(OUT_DIR, "librpa_mi355.so")
 HASH_PATH = os.path.join(OUT_DIR, "librpa_mi355.srchash")
 
-SOURCES = ["rpa_capi.hip", "rpa_decode.hip", "rpa_prefill.hip", "rpa_prefill_pipe.hip", "rpa_prefill_packed.hip", "rpa_mla.hip"]
+SOURCES = ["rpa_capi.hip", "rpa_decode.hip", "rpa_prefill.hip", "rpa_prefill_pipe.hip", "rpa_prefill_packed.hip", "rpa_mla.hip", "rpa_mla_waves.hip"]
 # bench.py's measurement kernels (a streaming read, a matrix-instruction issue loop): a library of their own,
 # so that the attention library carries nothing but the attention path
 CEILINGS_SOURCE = "rpa_ceilings.hip"

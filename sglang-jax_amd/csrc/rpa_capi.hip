@@ -73,6 +73,7 @@ const Tuning& tuning() {
   geti("RPA_MLA_SHARED_TILES", t.mla_shared_tiles);
   geti("RPA_MLA_WIDE", t.mla_wide);
   geti("RPA_MLA_TOKEN_GROUPS", t.mla_token_groups);
+  geti("RPA_MLA_WAVES", t.mla_waves);
   if (const char* v = getenv("RPA_PREFILL_PIPE_LIMIT")) {
     if (*v) t.prefill_pipe_limit = (float)atof(v);
   }
@@ -1257,29 +1258,114 @@ int rpa_kv_write(const RpaParams* given, const void* keys, const void* values, v
 // ---------------------------------------------------------------- MLA ----
 
 static int mla_wgs();
+static float mla_logit_scale(const RpaMlaParams* p);
 
 // The smallest piece of a row.  Partial rows are bf16, so a row that is cut is rounded once more than a whole one: batches of
 // rows up to 256 tokens are left whole (their result is 2.3e-3 from the 64-bit one, in pieces of 64 it was 2.8e-3).  That is
 // also the faster plan from 16 rows on (128 heads, rows of 100..255 tokens: 64 rows 36.0 -> 32.4 us, 200 rows 64.1 -> 36.5),
 // but not for a few (4 rows 25.3 -> 29.1; 16 heads 16.3 -> 20.6).
 constexpr int kMlaWholeRow = 256;
+static int64_t mla_longest(const RpaMlaParams* p) {
+  const int64_t longest = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages, p->cu_kv_lens != nullptr);
+  return std::max<int64_t>(1, p->sliding_window > 0 ? std::min(longest, (int64_t)p->sliding_window + 31) : longest);
+}
 static int mla_min_piece(const RpaMlaParams* p) {
-  int64_t longest = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages, p->cu_kv_lens != nullptr);
-  if (p->sliding_window > 0) longest = std::min(longest, (int64_t)p->sliding_window + 31);
-  return longest <= kMlaWholeRow ? kMlaWholeRow : std::max(1, rpa::tuning().mla_min_chunk);
+  return mla_longest(p) <= kMlaWholeRow ? kMlaWholeRow : std::max(1, rpa::tuning().mla_min_chunk);
 }
 
-static SplitPlan mla_plan(const RpaMlaParams* p, int64_t rows) {
+// What the choice of an MLA kernel depends on.
+static rpa::MlaDecodeArgs mla_key_args(const RpaMlaParams* p, int64_t rows, bool token_rows) {
+  rpa::MlaDecodeArgs a = {};
+  a.pt.page_size = p->page_size;
+  a.sm.soft_cap = p->soft_cap;
+  a.sm.sm_scale = mla_logit_scale(p);
+  a.sm.window = p->sliding_window;
+  a.fp8 = p->cache_dtype == RPA_KV_FP8_E4M3 ? 1 : 0;
+  a.Hq = p->num_q_heads;
+  a.row_stride = p->row_stride;
+  a.num_rows = (int32_t)rows;
+  a.num_seqs = p->num_seqs;
+  a.rows_are_tokens = token_rows ? 1 : 0;
+  return a;
+}
+
+// How a call is cut.  wgs: pieces or shares that run at once; head_blocks > 0: the kernels of a wave per tile (rpa_mla_waves.hip), so many
+// blocks of 16 heads per workgroup and `siblings` workgroups per piece.
+struct MlaPlan {
+  SplitPlan sp;
+  const rpa::ShapeRule* rule;
+  int wgs, head_blocks, siblings, token_groups;
+  bool balanced;
+};
+
+// Whether a call runs on a wave per tile, with 16 heads a workgroup.  What a piece costs besides its tiles is half of the other kernels', what
+// a tile costs grows with every 16 heads: so by the work, in rounds of 64 tokens x 16 heads per CU.  us, other kernels -> these, and the rounds:
+//   16 heads           64 rows of 2047..16383 bf16 128 -> 113, e4m3 119 -> 76, on pages of 16 130 -> 114 and 137 -> 78; small ones level to 1.2 x
+//   32 heads, e4m3     the same rows 125 -> 105 (72), 128 of 500 28.2 -> 18.5 (8); bf16 133 -> 141 (72), 30.5 -> 32.0 (9.8), 128 of 500 26.9 -> 21.4 (7.8), on
+//                      pages of 16 35.3 -> 31.9 (9.8), 141 -> 145 (72); selections of 32 rows x 64 pages 39.6 -> 37.8 (16), of 50 rows 47.9 -> 54.4 (25)
+//   64 heads, bf16     20 rows of 300..1500 28.0 -> 24.5 (4.4), 54 of 300..800 31.0 -> 31.8 (7.3), on pages of 16 33.4 -> 31.7; 32 of 1000..4000 41.9 -> 45.0 (20);
+//                      e4m3 44.3 -> 42.6 (20), 157 -> 165 (144); selections of 12 rows x 64 pages 35.3 -> 33.8 (12), of 32 52.2 -> 57.2 (32)
+//   128 heads          one row of 4000 25.1 -> 15.8 (2), 8 of 300..1500 26.7 -> 22.8 (3.5), 20 33.1 -> 34.1 (8.8), on pages of 16 36.9 -> 34.1, e4m3 39.7 -> 33.1;
+//                      54 of 300..800 37.6 -> 45.8 (14.5); selections of 4 rows x 64 pages 33.3 -> 26.3 (8), 12 of 2048 tokens 39.9 -> 39.4 (12)
+static bool mla_takes_waves(const RpaMlaParams* p, int64_t rows, bool sparse) {
+  const int blocks = (p->num_q_heads + 15) / 16;
+  if (blocks == 1) return true;
+  if (blocks > 8) return false;
+  const int64_t longest = mla_longest(p);
+  const int64_t tokens = p->sum_kv_len > 0 ? std::min(p->sum_kv_len, rows * longest) : rows * longest;
+  const bool fp8 = p->cache_dtype == RPA_KV_FP8_E4M3, whole = p->page_size % 32 == 0;  // (pages of whole tiles: where the other kernels are at their best)
+  const int64_t rounds = tokens * blocks / (64 * (int64_t)mla_wgs());
+  if (blocks <= 2) return fp8 || rounds < (sparse ? 20 : whole ? 8 : 24);
+  if (blocks <= 4) return rounds < (fp8 ? whole ? 32 : 200 : sparse || !whole ? 14 : 6);
+  return rounds < (fp8 || sparse || !whole ? 10 : 6);
+}
+
+static bool mla_use_balanced(const RpaMlaParams* p, const MlaPlan& plan, bool token_rows);
+static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bool sparse = false, bool waves = true) {
   const int64_t bound = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages,
                                      p->cu_kv_lens != nullptr);
-  // one 8-wave workgroup per (row, split, 128 heads) and per CU; every split costs a 256 KiB
+  rpa::MlaDecodeArgs a = mla_key_args(p, rows, token_rows);
+  const rpa::Tuning& tune = rpa::tuning();
+  MlaPlan m;
+  m.rule = &rpa::select_shape(rpa::mla_shape_key(a), rpa::mla_shape_skip(a, tune));
+  m.wgs = mla_wgs();
+  m.head_blocks = 0;
+  m.siblings = 1;
+  // one workgroup per (row, split, 128 heads) and per CU; every split costs a 256 KiB
   // partial write per 128 heads, so splits are kept as few as fill the CUs once
-  const int64_t groups = (p->num_q_heads + 127) / 128;
-  const int64_t units = rows * groups;
-  int64_t work = p->sum_kv_len > 0 ? p->sum_kv_len * groups : 0;
-  if (p->sliding_window > 0) work = 0;
-  return plan_splits(bound, p->sliding_window, units, work, p->num_splits,
-                     mla_min_piece(p), mla_wgs(), true);
+  auto cut = [&](int64_t groups) {
+    int64_t work = p->sum_kv_len > 0 ? p->sum_kv_len * groups : 0;
+    if (p->sliding_window > 0) work = 0;
+    return plan_splits(bound, p->sliding_window, rows * groups, work, p->num_splits, mla_min_piece(p), m.wgs, true);
+  };
+  m.sp = cut((p->num_q_heads + 127) / 128);
+  a.max_splits = m.sp.splits;
+  m.token_groups = rpa::mla_token_group_mode(a, tune, *m.rule);
+  const int blocks = (p->num_q_heads + 15) / 16;
+  if (waves && tune.mla_waves != 0 && !m.token_groups && p->soft_cap == 0.f && tune.mla_shared_tiles != 0 && (tune.mla_waves > 0 || mla_takes_waves(p, rows, sparse))) {
+    m.head_blocks = 1;
+    m.siblings = blocks;
+    m.wgs = std::max(1, m.wgs / m.siblings);
+    if (m.siblings > 1 && m.wgs > 8) m.wgs &= ~7;  // (whole eights of workgroups, see Sibling)
+    m.sp = cut(1);
+    // Rows of several lengths: the shortest pieces, counted by the longest row, that are one round of workgroups, if any of up to 512 tokens are.  The
+    // balanced plan evens them out, but its start (prefix sums, a search) is 2 us later: 20 rows of 300..1500 x 16 heads 17.9 -> 16.1 us in pieces
+    // of 128, 8 of 1000..8000 22.5 -> 20.0 of 256, 100 of 200..1000 e4m3 25.9 -> 22.7 of 512, 20 of 300..1500 x 32 heads 19.2 -> 17.4; beyond, 100 of
+    // 200..1000 in pieces of 256 26.3 -> 33.4.
+    const int64_t longest = mla_longest(p);
+    if (p->num_splits == 0 && !(p->sum_kv_len > 0 && p->sum_kv_len == rows * longest)) {
+      for (int64_t chunk = mla_min_piece(p); chunk <= 512; chunk *= 2) {
+        const int64_t pieces = (longest + chunk - 1) / chunk;
+        if (rows * pieces > m.wgs) continue;
+        m.sp.splits = (int)pieces;
+        m.sp.chunk = (int)((longest + pieces - 1) / pieces + 31) / 32 * 32;
+        m.balanced = false;
+        return m;
+      }
+    }
+  }
+  m.balanced = !sparse && mla_use_balanced(p, m, token_rows);
+  return m;
 }
 
 static int mla_validate(const RpaMlaParams* p) {
@@ -1310,34 +1396,38 @@ static int mla_wgs() {
 }
 
 // same criteria as the MHA decode path: ragged sequence rows that need splitting
-static bool mla_use_balanced(const RpaMlaParams* p, const SplitPlan& fixed, bool token_rows) {
+static bool mla_use_balanced(const RpaMlaParams* p, const MlaPlan& plan, bool token_rows) {
+  const SplitPlan& fixed = plan.sp;
   const bool on = rpa::tuning().mla_balanced != 0;
   if (!on || token_rows || p->num_splits == 1) return false;
+  if (plan.head_blocks > 0 && mla_min_piece(p) >= kMlaWholeRow) return false;  // (rows of up to 256 tokens stay whole: see there)
   // Rows the fixed plan leaves whole: one workgroup job per row.  With many more jobs than
   // workgroup slots the dispatcher evens them out by itself; with up to two per slot the kernel
   // ends with the longest rows, and dealing the tiles out evenly pays (300 rows of 1000..8000
   // tokens: 832 -> 673 us; 256 rows of 2048..16384: 1214 -> 1013 us; 1000 rows of 200..2000:
   // 617 -> 659 us, so not there).
-  if (fixed.splits <= 1 && (int64_t)p->num_seqs * ((p->num_q_heads + 127) / 128) > 2 * (int64_t)mla_wgs()) return false;
+  if (fixed.splits <= 1 && (int64_t)p->num_seqs * ((p->num_q_heads + 127) / 128) > 2 * (int64_t)plan.wgs) return false;
   if (p->num_splits > 0) return true;
   const int64_t bound = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages,
                                      p->cu_kv_lens != nullptr);
   const int64_t units = (p->num_q_heads + 127) / 128;
   const int64_t min_tiles = std::max(1, mla_min_piece(p) / 32);
-  if ((int64_t)p->num_seqs * ((bound + 31) / 32) * units <= (int64_t)mla_wgs() * min_tiles) return false;
+  if ((int64_t)p->num_seqs * ((bound + 31) / 32) * units <= (int64_t)plan.wgs * min_tiles) return false;
   const bool equal_lengths = p->sum_kv_len > 0 && p->max_kv_len > 0 &&
                              p->sum_kv_len == (int64_t)p->num_seqs * p->max_kv_len;
   return !equal_lengths;
 }
 
-static size_t mla_workspace(const RpaMlaParams* p, int64_t rows, bool token_rows) {
+static size_t mla_workspace(const RpaMlaParams* p, int64_t rows, const MlaPlan& plan) {
+  if (plan.balanced) return (size_t)plan.wgs * 2 * 128 * (p->lkv_dim + 2) * sizeof(float) + ((size_t)p->num_seqs + 1) * sizeof(int32_t);
+  if (plan.sp.splits <= 1) return 0;
+  return (size_t)rows * plan.sp.splits * p->num_q_heads * (p->lkv_dim + 2) * sizeof(float);
+}
+
+static size_t mla_workspace(const RpaMlaParams* p, int64_t rows, bool token_rows, bool sparse = false) {
   const rpa::TuningOfCall tuning;
   if (!p || p->num_seqs <= 0 || rows <= 0) return 0;
-  const SplitPlan sp = mla_plan(p, rows);
-  if (mla_use_balanced(p, sp, token_rows))
-    return (size_t)mla_wgs() * 2 * 128 * (p->lkv_dim + 2) * sizeof(float) + ((size_t)p->num_seqs + 1) * sizeof(int32_t);
-  if (sp.splits <= 1) return 0;
-  return (size_t)rows * sp.splits * p->num_q_heads * (p->lkv_dim + 2) * sizeof(float);
+  return mla_workspace(p, rows, mla_plan(p, rows, token_rows, sparse));
 }
 
 size_t rpa_mla_workspace_bytes(const RpaMlaParams* p) { return mla_workspace(p, p ? p->num_seqs : 0, false); }
@@ -1363,7 +1453,10 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const v
     return fail(RPA_EINVAL_SHAPE, "decode rows=%d exceed tokens=%d", p->num_seqs, p->num_tokens);
   const int64_t rows = token_rows ? p->num_tokens : p->num_seqs;
   if (rows <= 0) return RPA_OK;
-  const SplitPlan sp = mla_plan(p, rows);
+  MlaPlan plan = mla_plan(p, rows, token_rows, sparse != nullptr);
+  // (a call that brings the room of the plan that stood here before stays on it)
+  if (plan.head_blocks > 0 && mla_workspace(p, rows, plan) > (p->workspace ? p->workspace_bytes : 0)) plan = mla_plan(p, rows, token_rows, sparse != nullptr, false);
+  const SplitPlan& sp = plan.sp;
   rpa::MlaDecodeArgs a;
   a.sparse = {};
   if (sparse) a.sparse = *sparse;
@@ -1397,22 +1490,26 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const v
   a.ws_o = nullptr;
   a.ws_ml = nullptr;
   a.cu_tiles = nullptr;
-  a.balanced = !sparse && mla_use_balanced(p, sp, token_rows) ? 1 : 0;
-  a.num_wgs = mla_wgs();
+  a.balanced = plan.balanced ? 1 : 0;
+  a.num_wgs = plan.wgs;
+  a.head_blocks = plan.head_blocks;
+  a.siblings = plan.siblings;
   a.min_tiles_per_wg = std::max(1, mla_min_piece(p) / 32);
   a.forced_tiles_per_wg = 0;
   a.piece_pad = rpa::tuning().mla_piece_pad >= 0
                     ? rpa::tuning().mla_piece_pad
+                    : plan.head_blocks > 0
+                          ? 8  // (a wave per tile: 6 .. 14 within 1 %; 3 loses 3 % on 64 rows of 2047..16383 e4m3 tokens, 10 % on short rows)
                     : rpa::mla_takes_wide_p16(a, true)
                           ? 12  // (the wide kernels' in the shape table)
-                          : rpa::select_shape(rpa::mla_shape_key(a), rpa::mla_shape_skip(a, rpa::tuning())).piece_pad;
+                          : plan.rule->piece_pad;
   if (p->num_splits > 0) {
     const int64_t bound = kv_len_bound(p->max_kv_len, p->pages_per_seq, p->page_size, p->total_pages,
                                        p->cu_kv_lens != nullptr);
     a.forced_tiles_per_wg = (int32_t)std::max<int64_t>(1, ((bound + 31) / 32 + p->num_splits - 1) / p->num_splits);
   }
   if (a.balanced) {
-    const size_t need = mla_workspace(p, rows, token_rows);
+    const size_t need = mla_workspace(p, rows, plan);
     if (!p->workspace || p->workspace_bytes < need)
       return fail(RPA_EINVAL_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, p->workspace_bytes);
     // partial rows are bf16 (the workspace is sized for f32 rows: room to spare)
@@ -1420,7 +1517,7 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const v
     a.ws_ml = reinterpret_cast<float*>(a.ws_o + (size_t)a.num_wgs * 2 * 128 * p->lkv_dim);
     a.cu_tiles = reinterpret_cast<int32_t*>(a.ws_ml + (size_t)a.num_wgs * 2 * 128 * 2);
   } else if (sp.splits > 1) {
-    const size_t need = mla_workspace(p, rows, token_rows);
+    const size_t need = mla_workspace(p, rows, plan);
     if (!p->workspace || p->workspace_bytes < need)
       return fail(RPA_EINVAL_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, p->workspace_bytes);
     a.ws_o = static_cast<uint16_t*>(p->workspace);
@@ -1435,30 +1532,17 @@ int rpa_mla_describe_plan(const RpaMlaParams* p, int token_rows, char* buf, size
   if (rc != RPA_OK) return rc;
   if (!buf || len == 0) return fail(RPA_EINVAL_NULL, "buf is NULL or empty");
   const int64_t rows = token_rows ? p->num_tokens : p->num_seqs;
-  rpa::MlaDecodeArgs a = {};
-  a.pt.page_size = p->page_size;
-  a.sm.soft_cap = p->soft_cap;
-  a.sm.sm_scale = mla_logit_scale(p);
-  a.fp8 = p->cache_dtype == RPA_KV_FP8_E4M3 ? 1 : 0;
-  a.Hq = p->num_q_heads;
-  a.row_stride = p->row_stride;
-  const rpa::ShapeRule& r = rpa::select_shape(rpa::mla_shape_key(a), rpa::mla_shape_skip(a, rpa::tuning()));
-  const SplitPlan sp = mla_plan(p, std::max<int64_t>(rows, 1));
-  const bool bal = rows > 0 && mla_use_balanced(p, sp, token_rows != 0);
-  a.sm.window = p->sliding_window;
-  a.num_rows = (int32_t)rows;
-  a.num_seqs = p->num_seqs;
-  a.rows_are_tokens = token_rows ? 1 : 0;
-  a.max_splits = sp.splits;
-  a.balanced = bal ? 1 : 0;
+  const MlaPlan plan = mla_plan(p, std::max<int64_t>(rows, 1), token_rows != 0);
+  const rpa::ShapeRule& r = *plan.rule;
+  const bool bal = rows > 0 && plan.balanced;
   static const char* const kGroups[] = {"off", "eight_waves_compiled", "eight_waves", "wide"};
-  const int tg = rpa::mla_token_group_mode(a, rpa::tuning(), r);
-  const bool p16 = !tg && rpa::mla_takes_wide_p16(a, true);
+  const int tg = plan.token_groups;
+  const bool p16 = !tg && plan.head_blocks == 0 && rpa::mla_takes_wide_p16(mla_key_args(p, rows, token_rows != 0), true);
   return snprintf(buf, len, "mla: shape=%s rows=%lld waves_per_wg=%d heads_per_wg=%d share=%d token_groups=%s plan=%s "
                   "pieces_per_row=%d workgroups=%d workspace=%zu%s\n",
                   r.name, (long long)rows, tg == 3 || p16 ? 4 : r.waves_per_wg, tg ? 128 : r.tile_heads, tg ? 1 : r.share, kGroups[tg],
-                  bal ? "balanced" : "fixed", bal ? 0 : sp.splits, bal ? mla_wgs() : 0,
-                  mla_workspace(p, rows, token_rows != 0), p16 ? " (the wide loop of pages of 16 tokens)" : "");
+                  bal ? "balanced" : "fixed", bal ? 0 : plan.sp.splits, bal ? plan.wgs * plan.siblings : 0,
+                  mla_workspace(p, rows, token_rows != 0), plan.head_blocks > 0 ? " (a wave per tile, 16 heads per workgroup)" : p16 ? " (the wide loop of pages of 16 tokens)" : "");
 }
 
 int rpa_mla_decode(const RpaMlaParams* p, void* stream) {
@@ -1536,7 +1620,7 @@ SparseLayout sparse_layout(const RpaMlaParams* p, const RpaMlaSparse* s, const R
   auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
   const size_t T = (size_t)p->num_tokens;
   SparseLayout l;
-  l.kv_lens = up(rpa_mla_workspace_bytes(&view));
+  l.kv_lens = up(mla_workspace(&view, view.num_seqs, false, true));
   l.table = l.kv_lens + up(T * sizeof(int32_t));
   l.extra = l.table + up(T * view.pages_per_seq * sizeof(int32_t) + kLine);
   l.total = l.extra + (s->k_pages_max > 0 ? 0 : (T + 1) * p->row_stride * (p->cache_dtype == RPA_KV_FP8_E4M3 ? 1 : 2));

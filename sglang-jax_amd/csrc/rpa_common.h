@@ -179,6 +179,23 @@ __device__ __forceinline__ float scalar_load_f32(const float* p) {
   return __int_as_float(scalar_load_i32(reinterpret_cast<const int32_t*>(p)));
 }
 
+// All cache lines of a kernel's arguments in one round trip, first thing: read where they are first needed, a line here and a line there, they
+// are one each.
+template <class Args>
+__device__ __forceinline__ void fetch_arguments() {
+  constexpr int kLast = (int)sizeof(Args) - 4;
+  static_assert(kLast >= 0 && kLast <= 7 * 64, "eight lines");
+  const uint64_t at = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
+  uint32_t x[8];
+#define RPA_LINE(i) (64 * i < kLast ? 64 * i : kLast)
+  asm volatile(
+      "s_load_dword %0, %8, %9\n\ts_load_dword %1, %8, %10\n\ts_load_dword %2, %8, %11\n\ts_load_dword %3, %8, %12\n\t"
+      "s_load_dword %4, %8, %13\n\ts_load_dword %5, %8, %14\n\ts_load_dword %6, %8, %15\n\ts_load_dword %7, %8, %16\n\ts_waitcnt lgkmcnt(0)"
+      : "=&s"(x[0]), "=&s"(x[1]), "=&s"(x[2]), "=&s"(x[3]), "=&s"(x[4]), "=&s"(x[5]), "=&s"(x[6]), "=&s"(x[7])
+      : "s"(at), "i"(RPA_LINE(0)), "i"(RPA_LINE(1)), "i"(RPA_LINE(2)), "i"(RPA_LINE(3)), "i"(RPA_LINE(4)), "i"(RPA_LINE(5)), "i"(RPA_LINE(6)), "i"(RPA_LINE(7)));
+#undef RPA_LINE
+}
+
 // Asynchronous 16-byte copy global -> LDS (global_load_lds_dwordx4): lane l's 16 bytes land at
 // lds_base + 16*l; the data never touches a VGPR and completion is counted by vmcnt.  Issued as
 // inline assembly so that the compiler does not model it as an LDS store: it would otherwise

@@ -213,6 +213,8 @@ struct MlaDecodeArgs {
   int32_t num_wgs;
   int32_t min_tiles_per_wg;
   int32_t forced_tiles_per_wg;
+  int32_t head_blocks;  // > 0: the kernels of a wave per tile (rpa_mla_waves.hip), so many blocks of 16 heads per workgroup
+  int32_t siblings;   // workgroups that take the same share or piece, each for heads of its own (rpa_mla_waves.hip); 1 elsewhere
   int32_t piece_pad;  // balanced plan: what starting one more (row, head group) costs a workgroup, in tiles
   int32_t* cu_tiles;  // [num_rows + 1] prefix sum of tiles, written by the kernel
   float out_scale;    // finished rows are multiplied by it (v_scale; 1 when off)
@@ -257,6 +259,7 @@ hipError_t launch_rows256(const DecodeArgs& a, int seq_begin, int seq_end, int m
                           hipStream_t stream);
 hipError_t launch_kv_write(const KvWriteArgs& a, hipStream_t stream);
 hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream);
+hipError_t launch_mla_waves(const MlaDecodeArgs& a, hipStream_t stream);
 // The rows of the shape table (rpa_shapes.h) these launchers select for a call, RPA_* overrides applied.
 const ShapeRule& prefill_shape_of(const PrefillArgs& a);
 // Whether launch_prefill would take long sequences one after the other (streams_in_turn, rpa_prefill_common.h).

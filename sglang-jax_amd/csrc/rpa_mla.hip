@@ -29,6 +29,7 @@
 #include "rpa_common.h"
 #include "rpa_dsa.h"
 #include "rpa_kernels.h"
+#include "rpa_mla_common.h"
 #include "rpa_shapes.h"
 #include "rpa_tuning.h"
 #include "rpa_mla_pipe_loop.inc"
@@ -37,22 +38,8 @@
 
 namespace rpa {
 
-// Per-workgroup timestamps of the wide balanced kernel, compiled in with -DRPA_MLA_TRACE only (build.py passes
-// extra flags through): for up to four pieces per workgroup the 100 MHz clock at piece entry, first tiles and
-// queries landed, tile loop entered, tile loop left, rows written.  rpa_debug_mla_trace() copies them out.
-#ifdef RPA_MLA_TRACE
-__device__ unsigned long long rpa_mla_trace_buf[1024][4][8];
-#define RPA_MLA_STAMP(slot)                                                                              \
-  do {                                                                                                   \
-    if (threadIdx.x == 0 && trace_piece < 4) rpa_mla_trace_buf[blockIdx.x & 1023][trace_piece][slot] = wall_clock64(); \
-  } while (0)
-#else
-#define RPA_MLA_STAMP(slot) do { } while (0)
-#endif
-
 namespace {
 
-constexpr int kTok = 32;                 // tokens per tile
 constexpr int kRowB = 1184;              // latent row in LDS: 576 bf16 + 32 bytes of padding
 constexpr int kChunks = 74;              // 16-byte chunks per row (72 data + 2 pad)
 constexpr int kUsedBlocks = 37;          // copy blocks of 64 chunks that hold a tile (32 rows x 74 chunks)
@@ -64,36 +51,6 @@ constexpr int kF8Chunks = 36;            // 16-byte chunks per staged row
 constexpr int kF8Blocks = 18;            // copy blocks per staged tile (32 rows x 36 chunks)
 constexpr int kF8StageB = kF8Blocks * 1024;
 constexpr int kF8CopiesPerWave = 3;      // 8 x 3 = 24 copy instructions cover 18 blocks (the rest repeat block 0)
-
-__device__ __forceinline__ u32x4_t lds_ld16(const char* p) { return *reinterpret_cast<const u32x4_t*>(p); }
-
-typedef uint32_t u32x32_t __attribute__((ext_vector_type(32)));
-typedef uint32_t u32x8_t __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x16_t __attribute__((ext_vector_type(16)));
-typedef float f32x32_t __attribute__((ext_vector_type(32)));
-typedef short s16x4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x2_t lds_tr16(const char* p) {
-  typedef __attribute__((address_space(3))) s16x4_t* lds_ptr_t;
-  const s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr_t)(p));
-  return __builtin_bit_cast(u32x2_t, v);
-}
-
-// The lane id behind a fence the compiler cannot see through: values derived from it are not common
-// subexpressions of anything earlier, so they are worked out again where they are used instead of being
-// kept in registers across code that has none to spare (the assembly loop pins 251 of a wave's 256; with
-// them carried over it, 23-37 registers went to scratch memory per segment, 100 MB a launch on a
-// prefill batch).  Counted by two instructions of its own, not taken from threadIdx, which would itself be kept in scratch memory across
-// the loops.
-__device__ __forceinline__ int fresh_lane() {
-  int ln;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-  return ln;
-}
-
-// token (inside a tile) behind slot i = 4b + r of lane group g in the S^T result registers
-__device__ __forceinline__ int tok_of(int g, int i) {
-  return 16 * (i >> 2) + 4 * g + (i & 3);
-}
 
 // Pages that are no whole number of tiles: the ids of a tile's pages arrive in LDS by a copy of their own
 // (global_load_lds_dword, entry i = page slot of the tile's first token + i), two tiles ahead of the tile's rows, in
@@ -313,99 +270,6 @@ __device__ __forceinline__ void expand_f8_tile(const char* stage, char* slot, in
   }
 }
 
-// Sequence that owns query token `row`: the last one whose first token is <= row
-// (zero-length sequences are skipped).  cu_q_lens[0 .. num_seqs] is non-decreasing.
-__device__ __forceinline__ int owner_of_token(const int32_t* cu_q_lens, int num_seqs, int row) {
-  int lo = 0, hi = num_seqs;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (scalar_load_i32(cu_q_lens + mid) <= row) lo = mid;
-    else hi = mid;
-  }
-  return lo;
-}
-
-// Query tokens are taken last first: a chunk's last tokens see the most, and what starts last should be short.  1405 tokens x
-// 64 heads e4m3 124 -> 101 us, 6 prompts of 88 .. 307 tokens x 128 heads 137 -> 127, 900 tokens x 128 heads 164 -> 158.
-//
-// What a grid row attends to.  Sequence rows (decode batches): the one query of sequence `row`
-// sees all kv_len tokens.  Token rows: query token `row` of a sequence with q_len new tokens
-// sits at position kv_len - q_len + j and sees the tokens up to itself -- an absorbed-MLA
-// prefill row is a decode row over a shorter prefix (mla/v1/ref.py:229-233).
-struct MlaRow {
-  int seq, kv_len, tq;
-  bool valid;
-};
-
-__device__ __forceinline__ MlaRow mla_row(const MlaDecodeArgs& a, int row) {
-  MlaRow r;
-  r.valid = true;
-  // static-shape mode: num_seqs is a bound, the number of sequences comes from the device
-  const int num_seqs = a.dist ? min(a.num_seqs, scalar_load_i32(a.dist + 2)) : a.num_seqs;
-  if (a.rows_are_tokens) {
-    if (row >= scalar_load_i32(a.pt.cu_q_lens + num_seqs)) {
-      r.valid = false;
-      r.seq = r.kv_len = r.tq = 0;
-      return r;
-    }
-    r.seq = owner_of_token(a.pt.cu_q_lens, num_seqs, row);
-    const int q0 = scalar_load_i32(a.pt.cu_q_lens + r.seq);
-    const int q_len = scalar_load_i32(a.pt.cu_q_lens + r.seq + 1) - q0;
-    r.kv_len = scalar_load_i32(a.pt.kv_lens + r.seq) - q_len + (row - q0) + 1;
-    r.tq = row;
-  } else {
-    r.seq = row;
-    r.kv_len = (row < num_seqs) ? a.pt.kv_lens[row] : 0;
-    r.tq = a.sparse.topk ? row : a.pt.cu_q_lens[row];
-    r.valid = row < num_seqs;
-  }
-  return r;
-}
-
-// Where a workgroup leaves the result of one piece of work: finished bf16 rows in `out`, or
-// unnormalised partial rows plus (max, sum) in workspace slot `base` + head.
-struct MlaDest {
-  bool final_rows;
-  int64_t base;
-};
-
-// A sequence row's new token, from the caller's rows into the cache (a.new_kv_c), by every workgroup whose share holds the row's last
-// tile, in front of everything else that it does.  A launch of its own for 1152 bytes a row took 5.4 us of the GPU and 2.7 of the
-// host; here it is a round trip to memory at the start of those workgroups: 64 ragged rows x 128 heads 179.8 -> 177.4 us, 25 rows of
-// 125..1062 38.0 -> 35.8, 2 of 4516..9525 x 16 heads 32.3 -> 30.2, 6 of 351..927 e4m3 33.7 -> 30.7.  Many short rows, each of which
-// pays that round trip, are no slower: 600 rows of 100..200 x 128 heads 95.5 -> 94.2, 1000 of 30..100 118.6 -> 117.8, e4m3 121.4 -> 116.0.
-// Every wave writes the whole row (the same bytes, 2 stores), so the copies that it makes of it afterwards follow its own stores
-// and no barrier is needed.  Tiles behind a piece's first three are asked for behind a wait for the first one, which is younger than
-// the stores; where the row's last tile may be among the first three the caller of this waits for the stores.  (Registers that
-// wait for the token beside the first copies are live into the tile loops, which spill then and drain their copies to
-// reload: 22 rows on token-level selections x 128 heads, which bring no token here, 50.3 -> 52.3 us.)
-template <bool FP8>
-__device__ __forceinline__ void put_new_row(const MlaDecodeArgs& a, int seq, int kv_len) {
-  const int lane = threadIdx.x & 63;
-  const int P = a.pt.page_size;
-  const int q0 = scalar_load_i32(a.pt.cu_q_lens + seq), n = scalar_load_i32(a.pt.cu_q_lens + seq + 1) - q0;
-  const int32_t* pages = a.pt.page_indices + (a.pt.cu_kv_lens ? (int64_t)(scalar_load_i32(a.pt.cu_kv_lens + seq) / P)
-                                                            : (int64_t)seq * a.pt.pages_per_seq);
-  for (int j = 0; j < n; ++j) {  // (one: a decode row brings one token)
-    const int64_t tok = q0 + j;
-    const int pos = kv_len - n + j;
-    if (pos < 0) continue;
-    const int slot = __builtin_amdgcn_readfirstlane((P & (P - 1)) == 0 ? pos >> (31 - __builtin_clz(P)) : pos / P);
-    char* page = const_cast<char*>(a.cache);
-    if constexpr (FP8) {
-      const int t = min(lane, 35);
-      const u32x4_t x = ld16(t < 32 ? a.new_kv_c + tok * 512 + t * 16 : a.new_k_pe + tok * 64 + (t - 32) * 16);
-      char* row = page + ((int64_t)scalar_load_i32(pages + slot) * P + (pos - slot * P)) * a.row_stride;
-      if (lane < 36) st16(row + (lane < 32 ? lane * 16 : a.rope_offset + (lane - 32) * 16), x);
-    } else {
-      const u32x4_t x = ld16(a.new_kv_c + tok * 1024 + lane * 16), y = ld16(a.new_k_pe + tok * 128 + (lane & 7) * 16);
-      char* row = page + ((int64_t)scalar_load_i32(pages + slot) * P + (pos - slot * P)) * a.row_stride * 2;
-      st16(row + lane * 16, x);
-      if (lane < 8) st16(row + a.rope_offset * 2 + lane * 16, y);
-    }
-  }
-}
-
 // One workgroup, one row, one group of 128 heads, tokens [t_begin, t_end).  Every wave of the
 // workgroup calls it with the same arguments; all LDS reads of an earlier call are behind a
 // barrier when it returns.
@@ -418,7 +282,7 @@ __device__ __forceinline__ void put_new_row(const MlaDecodeArgs& a, int seq, int
 // k + 1 between two barriers.
 // DS: with at most 64 heads (a tensor-parallel share) most waves of the workgroup would have no heads, and a step
 // would last as long as one wave's serial chain through the tile (36 + 32 dependent matrix instructions with
-// their LDS reads) while the others only copy.  With DS = 8 / 4 / 2 (at most 16 / 32 / 64 heads) the DS waves of a
+// their LDS reads) while the others only copy.  With DS = 4 / 2 (at most 32 / 64 heads) the DS waves of a
 // block of 16 heads share its tile instead: wave `sub` of the block takes token half sub & 1 and k-step group
 // sub >> 1 of the first product, leaves its partial scores in LDS, every wave of the block sums them and takes
 // the (same) probabilities, and the second product's 32 output chunks are dealt out 32 / DS per wave.
@@ -426,8 +290,7 @@ __device__ __forceinline__ void put_new_row(const MlaDecodeArgs& a, int seq, int
 // So a wave keeps its own k-steps' queries alone, asks for its K operands before it works out the copies' addresses, and for the partial
 // scores and the V^T operands together behind the barrier; page ids come from a register and the lanes' offsets stay in some.  With
 // the reads two at a time, each waited for, and a scalar load among them: 32 rows of 1000..4000 tokens x 32 heads 40.1 -> 32.1 us,
-// 64 of 2048..16384 x 64 heads 192 -> 170, x 16 heads 146 -> 134, 2 of 100..200 x 16 heads 17.4 -> 14.4, 32 selections of whole
-// pages x 16 heads 46.7 -> 44.6 (the call).
+// 64 of 2048..16384 x 64 heads 192 -> 170.  16 heads, and little work of more, run a wave per tile (rpa_mla_waves.hip).
 // TG (token group): with 16 / 32 / 64 heads, the eight waves hold 8 / 4 / 2 CONSECUTIVE QUERY TOKENS of one
 // sequence instead of one token's heads, `group_tokens` of them real (a chunk's tail may leave fewer): wave w
 // owns token (16 w) / Hq of the group and the block of 16 heads (16 w) % Hq.  mr.tq is the group's first token,
@@ -514,10 +377,9 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
   // ---- Q^T operands of this wave: column c = head head0 + c, k-step ks covers dims 32ks + 8g .. ----
   // (shared tiles: the k-steps of this wave's group alone)
   const int tq = mr.tq;
-  constexpr int kGroups = DS == 1 ? 1 : DS / 2;  // of k-steps: 4 groups of 5, 5, 4, 4; 2 of 9; 1 of 18
-  constexpr int kQ = kGroups == 4 ? 5 : 18 / kGroups;
-  const int kg = DS == 1 ? 0 : sub >> 1;
-  const int ks0 = kGroups == 4 && kg == 3 ? 14 : kg * kQ;
+  constexpr int kGroups = DS == 1 ? 1 : DS / 2;  // of k-steps: 2 of 9; 1 of 18
+  constexpr int kQ = 18 / kGroups;
+  const int ks0 = DS == 1 ? 0 : (sub >> 1) * kQ;
   u32x4_t qB[kQ];
   {
     const int head = TG ? head0 + c : min(head0 + c, a.Hq - 1);
@@ -618,7 +480,7 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
     const char* kp = cur + k_off_t + (DS > 1 ? (sub & 1) * 16 * kRowB + ks0 * 64 : 0);
     if constexpr (DS > 1) {  // this wave's K operands are on their way before the copies' addresses are worked out
 #pragma unroll
-      for (int i = 0; i < kKx; ++i) kx[i] = lds_ld16(kp + (kGroups == 4 && i == 4 && kg >= 2 ? 3 : i) * 64);
+      for (int i = 0; i < kKx; ++i) kx[i] = lds_ld16(kp + i * 64);
     }
     if constexpr (FP8) copy_tile_f8<UNIFORM, (DS > 1)>(fill, src, a.cache, tb + 3 * kTok, wave, lane_t, pg_next);
     else copy_tile<UNIFORM, kCopiesPerWave, (DS > 1)>(fill, src, a.cache, tb + 3 * kTok, wave, lane_t, pg_next);
@@ -632,7 +494,7 @@ __device__ __forceinline__ void mla_segment(const MlaDecodeArgs& a, const MlaRow
       f32x4_t sp = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < kQ; ++i) {
-        if (!(kGroups == 4 && i == 4) || kg < 2) sp = mfma16(kx[i % kKx], qB[i], sp);
+        sp = mfma16(kx[i % kKx], qB[i], sp);
         if (i + kKx < kQ) kx[i] = lds_ld16(kp + (i + kKx) * 64);
       }
       *reinterpret_cast<f32x4_t*>(&partial_scores[wave][lane_t * 4]) = sp;
@@ -1421,172 +1283,13 @@ __global__ __launch_bounds__(256, 1) void rpa_mla_decode_wide_kernel(const MlaDe
   mla_segment_wide<M32, false, P16>(a, mr, blockIdx.z * 128, t_lo, t_begin, t_end, dest, ring);
 }
 
-// ---- balanced plan (one row per sequence): the 32-token tiles of the whole batch, sequence by
-// sequence and inside a sequence head group by head group, are dealt evenly to the workgroups;
-// workgroup j takes tiles [j * pw, (j + 1) * pw).  Pieces that are whole rows are finished in
-// place, cut ones (at most the first and the last of a workgroup) leave partial rows in the
-// workspace slots 2j and 2j + 1 (128 heads each).
-//
-// Starting a piece is not free: 147 KB of queries and the first tiles have to arrive and the
-// piece before it has to be written out -- 17 us on the DeepSeek-V3 batch, five tiles' worth, and
-// a workgroup with three pieces finished 37 us after one with a single piece.  So the line the
-// workgroups share is padded: every (row, head group) is preceded by `piece_pad` tiles that hold
-// no work.  A workgroup that runs into a new row spends that much of its share on the way, which
-// is what the switch costs it; one that starts in the middle of a row, like most, pays nothing
-// extra -- every workgroup has one start of its own anyway.
-__device__ __forceinline__ int mla_tiles(int kv_len, int window) {
-  if (kv_len <= 0) return 0;
-  const int t_lo = (window > 0) ? max(0, kv_len - window) : 0;
-  return (kv_len - (t_lo & ~(kTok - 1)) + kTok - 1) / kTok;
-}
-
-// extent of a (row, head group) on the padded line
-__device__ __forceinline__ int mla_extent(const MlaDecodeArgs& a, int kv_len) {
-  const int nt = mla_tiles(kv_len, a.sm.window);
-  return nt > 0 ? nt + a.piece_pad : 0;
-}
-
-__device__ __forceinline__ int mla_tiles_per_wg(const MlaDecodeArgs& a, int total) {
-  const int even = (total + a.num_wgs - 1) / a.num_wgs;  // the grid has exactly num_wgs workgroups
-  return max(a.forced_tiles_per_wg > 0 ? a.forced_tiles_per_wg : a.min_tiles_per_wg, even);
-}
-
-// `segment(mr, head_base, t_lo, t_begin, t_end, dest)` runs one piece on the workgroup's LDS ring.
-template <bool FP8, class Segment>
-__device__ __forceinline__ void mla_balanced_body(const MlaDecodeArgs& a, Segment segment) {
-  const int lane = threadIdx.x & 63;
-  int wg = blockIdx.x;  // this workgroup's share of the line
-  const int units = (a.Hq + 127) / 128;
-#ifdef RPA_MLA_TRACE
-  if (threadIdx.x == 0) rpa_mla_trace_buf[blockIdx.x & 1023][0][7] = wall_clock64();  // kernel entry
-#endif
-  // prefix sums of tiles over the sequences: every wave scans (the result is wave-uniform)
-  int total = 0, seq = -1, seq_first = 0;
-  {
-    // first pass: total; second pass (below) locates this workgroup's first tile
-    for (int s0 = 0; s0 < a.num_rows; s0 += 64) {
-      const int s = s0 + lane;
-      int nt = (s < a.num_rows) ? mla_extent(a, a.pt.kv_lens[s]) : 0;
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) nt += __shfl_xor(nt, off);
-      total += nt;
-    }
-    total = __builtin_amdgcn_readfirstlane(total) * units;
-  }
-  const int pw = mla_tiles_per_wg(a, total);
-  // The shares of an XCD's workgroups (every eighth) one after the other on the line: a row's pieces then find its queries, 147 KB at 128 heads,
-  // in one L2.  10 rows of 500..5000 tokens x 16 heads 20.5 -> 19.7 us, 64 of 2000..16000 127.5 -> 126.2, 20 of 1000..9000 x 128 heads 55.8 -> 54.7; 3
-  // rows of 8000..16000 x 128 heads, 27 shares each, 38.1 against 38.9: not with fewer rows than XCDs.
-  const int per_xcd = ((total + pw - 1) / pw + 7) >> 3;  // (at most gridDim.x / 8: the shares are at most gridDim.x)
-  if (a.num_rows >= 8 && (gridDim.x & 7) == 0) {
-    if ((int)(blockIdx.x >> 3) >= per_xcd && blockIdx.x != 0) return;  // (the first one also writes the prefix sums of no work)
-    wg = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-  }
-  if (wg == 0 && threadIdx.x < 64) {
-    int base = 0;
-    for (int s0 = 0; s0 < a.num_rows; s0 += 64) {
-      const int s = s0 + lane;
-      const int nt = (s < a.num_rows) ? mla_extent(a, a.pt.kv_lens[s]) : 0;
-      int incl = nt;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const int n = __shfl_up(incl, off);
-        if (lane >= off) incl += n;
-      }
-      if (s < a.num_rows) a.cu_tiles[s + 1] = base + incl;
-      base += __builtin_amdgcn_readfirstlane(__shfl(incl, 63));
-    }
-    if (lane == 0) a.cu_tiles[0] = 0;
-  }
-  if ((int64_t)wg * pw >= total) return;
-  int x = wg * pw;
-  const int x_end = min(total, x + pw);
-  {
-    int base = 0;
-    for (int s0 = 0; s0 < a.num_rows && seq < 0; s0 += 64) {
-      const int s = s0 + lane;
-      const int nt = (s < a.num_rows) ? mla_extent(a, a.pt.kv_lens[s]) : 0;
-      int incl = nt;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const int n = __shfl_up(incl, off);
-        if (lane >= off) incl += n;
-      }
-      const uint64_t hit = __builtin_amdgcn_ballot_w64((base + incl) * units > x);
-      if (hit != 0) {
-        const int first = __builtin_ctzll(hit);
-        seq = s0 + first;
-        seq_first = __builtin_amdgcn_readfirstlane((base + __shfl(incl - nt, first)) * units);
-      } else {
-        base += __builtin_amdgcn_readfirstlane(__shfl(incl, 63));
-      }
-    }
-    seq = __builtin_amdgcn_readfirstlane(seq);
-  }
-  int kv_len = scalar_load_i32(a.pt.kv_lens + seq);
-  int nt = mla_tiles(kv_len, a.sm.window);
-  const int pad = a.piece_pad;
-  if (a.new_kv_c) {  // the new tokens of the rows that end in this share, all of them in front of its first piece
-    int s = seq, len = kv_len, from = seq_first, tiles = nt;
-    for (;;) {
-      const int unit_end = from + (max(x - from, 0) / (tiles + pad) + 1) * (tiles + pad);
-      if (unit_end > x_end) break;
-      put_new_row<FP8>(a, s, len);
-      from += (tiles + pad) * units;
-      if (from >= x_end) break;
-      do {
-        ++s;
-        len = scalar_load_i32(a.pt.kv_lens + s);
-        tiles = mla_tiles(len, a.sm.window);
-      } while (tiles == 0);
-    }
-    wait_all_loads();  // (and stores)
-  }
-  bool first_piece = true;
-  int piece_no = 0;  // (only the optional timestamps use it)
-  while (x < x_end) {
-    const int r = x - seq_first;  // position inside the row's padded extents
-    const int unit = r / (nt + pad);
-    int off = r - unit * (nt + pad);
-    if (off < pad) {  // the padding in front of this (row, head group): no work there
-      x += pad - off;
-      off = pad;
-      if (x >= x_end) break;
-    }
-    const int tile = off - pad;
-    const int take = min(nt - tile, x_end - x);
-    const int t_lo = (a.sm.window > 0) ? max(0, kv_len - a.sm.window) : 0;
-    const int t0 = t_lo & ~(kTok - 1);
-    MlaRow mr;
-    mr.seq = seq;
-    mr.kv_len = kv_len;
-    mr.tq = scalar_load_i32(a.pt.cu_q_lens + seq);
-    mr.valid = true;
-    MlaDest dest;
-    dest.final_rows = (tile == 0) && (take == nt);
-    dest.base = ((int64_t)wg * 2 + (first_piece ? 0 : 1)) * 128 - unit * 128;  // + head
-    first_piece = false;
-    segment(mr, unit * 128, t_lo, t0 + tile * kTok, min(kv_len, t0 + (tile + take) * kTok), dest, piece_no++);
-    x += take;
-    if (x < x_end && tile + take == nt && unit == units - 1) {
-      seq_first += (nt + pad) * units;
-      do {
-        ++seq;
-        kv_len = scalar_load_i32(a.pt.kv_lens + seq);
-        nt = mla_tiles(kv_len, a.sm.window);
-      } while (nt == 0);
-    }
-  }
-}
-
-
 template <bool UNIFORM, bool CAP, bool PIPE = false, bool FP8 = false, int DS = 1>
 __global__ __launch_bounds__(512, 2) void rpa_mla_balanced_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char slot0[kSlotB];
   __shared__ __attribute__((aligned(1024))) char slot1[kSlotB];
   __shared__ __attribute__((aligned(1024))) char slot2[kSlotB];
   __shared__ __attribute__((aligned(1024))) char slot3[kSlotB];
-  mla_balanced_body<FP8>(a, [&](const MlaRow& mr, int head_base, int t_lo, int t_begin, int t_end, const MlaDest& dest, int)
+  mla_balanced_body<FP8, true>(a, [&](const MlaRow& mr, int head_base, int t_lo, int t_begin, int t_end, const MlaDest& dest, int)
                         __attribute__((always_inline)) {
     mla_segment<UNIFORM, CAP, PIPE, FP8, DS>(a, mr, head_base, t_lo, t_begin, t_end, dest, slot0, slot1, slot2, slot3);
   });
@@ -1596,7 +1299,7 @@ __global__ __launch_bounds__(512, 2) void rpa_mla_balanced_kernel(const MlaDecod
 template <bool M32, bool P16 = false>
 __global__ __launch_bounds__(256, 1) void rpa_mla_balanced_wide_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char ring[4 * kSlotB];
-  mla_balanced_body<false>(a, [&](const MlaRow& mr, int head_base, int t_lo, int t_begin, int t_end, const MlaDest& dest,
+  mla_balanced_body<false, true>(a, [&](const MlaRow& mr, int head_base, int t_lo, int t_begin, int t_end, const MlaDest& dest,
                            int piece) __attribute__((always_inline)) {
     mla_segment_wide<M32, false, P16>(a, mr, head_base, t_lo, t_begin, t_end, dest, ring, piece);
   });
@@ -1893,12 +1596,17 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
     }
     return hipGetLastError();
   }
+  if (a.head_blocks > 0) {
+    hipError_t ew = launch_mla_waves(a, stream);
+    if (ew != hipSuccess) return ew;
+    if (a.balanced || a.max_splits > 1) launch_mla_combine(a, stream);
+    return hipGetLastError();
+  }
   if (ds != 1) {
-#define RPA_MLA_DS_U(LAUNCH, U, F8)                              \
-  do {                                                           \
-    if (ds == 8) LAUNCH<U, false, false, F8, 8>(a, stream);      \
-    else if (ds == 4) LAUNCH<U, false, false, F8, 4>(a, stream); \
-    else LAUNCH<U, false, false, F8, 2>(a, stream);              \
+#define RPA_MLA_DS_U(LAUNCH, U, F8)                         \
+  do {                                                      \
+    if (ds >= 4) LAUNCH<U, false, false, F8, 4>(a, stream); \
+    else LAUNCH<U, false, false, F8, 2>(a, stream);         \
   } while (0)
 #define RPA_MLA_DS(LAUNCH, F8)                    \
   do {                                            \

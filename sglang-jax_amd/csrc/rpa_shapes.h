@@ -119,7 +119,7 @@ constexpr ShapeRule kShapeRules[] = {
   {"mla_pipe", kStageMla, 0, 576, 128, 0, 128, 0, 0, kOptSoftCap | kOptAsmPages,
    kKernelMlaPipe, 1, 128, 32, 8, 8, 1, 12, "e4m3 latents (bytes staged and expanded once per tile) and RPA_MLA_WIDE=0"},
   {"mla_shared_16", kStageMla, 0, 576, 1, 16, 0, 0, 0, kOptSoftCap,
-   kKernelMlaShared, 1, 16, 32, 8, 8, 8, 8, "a tensor-parallel share of the heads: 64 rows x 8192 tokens 146 -> 120 us"},
+   kKernelMlaShared, 1, 16, 32, 8, 8, 8, 8, "a tensor-parallel share of the heads; a wave per tile unless RPA_MLA_WAVES=0: 64 rows of 2047..16383 tokens 128 -> 113 us"},
   {"mla_shared_32", kStageMla, 0, 576, 17, 32, 0, 0, 0, kOptSoftCap,
    kKernelMlaShared, 1, 32, 32, 8, 8, 4, 8, "144 -> 126 us"},
   {"mla_shared_64", kStageMla, 0, 576, 33, 64, 0, 0, 0, kOptSoftCap,

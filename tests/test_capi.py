@@ -756,6 +756,21 @@ def test_mla_rows_of_up_to_256_tokens_are_left_whole(pkg, S, Hq, fp8):
             assert whole != cut, (longest, window, total, d)
 
 
+def test_mla_little_work_runs_a_wave_per_tile(pkg, monkeypatch):
+    """16 heads always; more heads, a workgroup per 16 of them, where the rounds of 64 tokens per CU are few.  A call that brings the room of the
+    plan that stood there before keeps it, and the switch turns it off."""
+    takes = lambda Hq, S, longest, **kw: "a wave per tile" in pkg._lib.describe_mla_plan(
+        _mla_params(pkg, Hq, S=S, T=S, max_kv=longest, sum_kv=S * longest * 3 // 4, **kw), False)
+    assert takes(16, 64, 16384) and takes(16, 1, 40, P=1, fp8=True) and takes(5, 300, 3000) and not takes(16, 64, 16384, soft_cap=30.0)
+    assert takes(32, 64, 16384, fp8=True) and not takes(32, 64, 16384) and takes(24, 8, 1500)
+    assert takes(64, 20, 1000) and not takes(64, 40, 4000) and takes(64, 40, 4000, fp8=True) and takes(64, 30, 2000, P=16)
+    assert takes(128, 3, 4000) and takes(128, 16, 1000, fp8=True) and not takes(128, 64, 1000) and not takes(160, 1, 100)
+    p = _mla_params(pkg, 16, S=20, T=20, max_kv=1500, sum_kv=18000)
+    assert "plan=fixed pieces_per_row=12" in pkg._lib.describe_mla_plan(p, False)  # one round of pieces of 128 tokens
+    monkeypatch.setenv("RPA_MLA_WAVES", "0")
+    assert not takes(16, 64, 16384)
+
+
 def test_mla_pages_that_the_wide_loops_do_not_take(pkg):
     """The wide loops: bytes inside a page in 32 bits, masks in front of a scale that has to be positive."""
     d = pkg._lib.describe_mla_plan
