@@ -1,7 +1,8 @@
 #!/usr/bin/env python3
 """Generator of ``rpa_prefill_pipe_loop.inc``: the steady-state loop of the pipelined prefill
 kernel (rpa_prefill_pipe.hip) as hand-scheduled gfx950 assembly, for NQ = 1 and NQ = 2 blocks of
-32 query rows per wave.
+32 query rows per wave, and for heads of 64 dims (hd = 64, NQ = 1): the second half of their cached rows is
+zero, so the step copies half the bytes and runs half the matrix instructions.
 
     python gen_prefill_pipe_loop.py            # rewrites rpa_prefill_pipe_loop.inc next to it
 
@@ -48,9 +49,14 @@ import sys
 ACC = 1000                                # register ids >= ACC name accumulation registers a[id - ACC]
 # Experiment switches (timing probes only: results are wrong with any of them set)
 X = set(os.environ.get("RPA_PIPE_X", "").split(","))
-AHEAD = int(os.environ.get("RPA_PIPE_AHEAD", 3))   # fragments requested ahead of the MFMAs that use them
 STAGGER = int(os.environ.get("RPA_PIPE_STAGGER", 4))  # matrix slots a wave spreads its copies over (with X = stagger)
-NBUF = 4                                  # operand fragment buffers per matrix
+
+
+def ahead(hd):
+    """Operand fragments of each matrix requested ahead of the MFMAs that use them (one buffer more): heads of 64 dims have to fit
+    the 168 registers of a wave at three waves per SIMD."""
+    return int(os.environ.get("RPA_PIPE_AHEAD", 3 if hd == 128 else 2))
+
 
 # scalar registers used inside the block (all listed as clobbers)
 KB, VB = 60, 62                           # s[60:61], s[62:63]: global base of the K / V tile being copied
@@ -61,11 +67,6 @@ MASK_SGPR = [70, 72, 74, 76]              # s[70:71] .. s[76:77]: lane masks of 
 SGPR_BASE = 5000                          # register ids >= SGPR_BASE name scalar registers in the hazard bookkeeping
 SGPR_CLOBBERS = list(range(60, 70 if "stagger" in X else 69))
 
-K_SLOT = [0, 16384]                       # byte offsets of the ring slots from the LDS array's start
-V_SLOT = [32768, 49152]
-V_READ = [0, 16384]                       # ... of the V slots from the addresses in VOFF (which point into V slot 0)
-HALF = 8192
-
 MFMA_TO_VALU = 12
 VALU_TO_MFMA = 2
 TRANS_TO_VALU = 1
@@ -75,11 +76,14 @@ VALU_SGPR_TO_VALU = 2                     # a vector instruction's scalar result
 
 
 class Table:
-    """Register table of one NQ variant."""
+    """Register table of one NQ / head-width variant."""
 
-    def __init__(self, nq, masked=False):
+    def __init__(self, nq, masked=False, hd=128):
         self.nq = nq
         self.masked = masked
+        self.hd = hd
+        self.nbuf = ahead(hd) + 1
+        dims, steps = hd // 32, hd // 16                           # dim tiles of the output; k-steps of the scores
         self._v, self._a = 0, ACC
 
         def v(n):
@@ -96,19 +100,19 @@ class Table:
             self._a += n
             return lo
 
-        self.O = [[a(16) for d in range(4)] for q in range(nq)]    # accumulators: only matrix instructions touch them
-        self.Q = [a(32) for q in range(nq)]                        # Q^T operands, 8 x 4 registers
-        self.KF = a(4 * NBUF)                                      # K fragments, 4 registers each
-        self.VF = a(4 * NBUF)                                      # V^T fragments
+        self.O = [[a(16) for d in range(dims)] for q in range(nq)] # accumulators: only matrix instructions touch them
+        self.Q = [a(4 * steps) for q in range(nq)]                 # Q^T operands, 4 registers per k-step
+        self.KF = a(4 * self.nbuf)                                      # K fragments, 4 registers each
+        self.VF = a(4 * self.nbuf)                                      # V^T fragments
         self.S = [[v(16), v(16)] for q in range(nq)]               # scores of the even / odd half in flight
         self.P = [[v(8), v(8)] for q in range(nq)]                 # probabilities of the even / odd half
         self.NM = [v(16) for q in range(nq)]                       # minus the running maximum, 16 times
         self.M = [v(1) for q in range(nq)]                         # running maximum (log2 units)
         self.L = [v(1) for q in range(nq)]                         # running sum
-        self.KOFF = v(8)                                           # LDS byte addresses of the K operand reads
-        self.VOFF = v(4)                                           # ... of the V^T operand reads
-        self.OFSK = v(4)                                           # per-lane global byte offsets of this wave's K copies
-        self.OFSV = v(4)
+        self.KOFF = v(steps)                                       # LDS byte addresses of the K operand reads
+        self.VOFF = v(dims)                                        # ... of the V^T operand reads
+        self.OFSK = v(dims)                                        # per-lane global byte offsets of this wave's K copies
+        self.OFSV = v(dims)                                        # (as many copies of K and of V as dim tiles)
         if masked:
             self.THR = v(1)                                        # query position - first token of the half - 4 * lane half
             self.NINF = v(1)                                       # -1e30
@@ -208,11 +212,20 @@ def valu(text, reads, writes, kind="valu"):
 
 
 class Gen:
-    def __init__(self, nq, masked=False):
-        assert not (masked and nq != 1)
+    def __init__(self, nq, masked=False, hd=128):
+        assert not ((masked or hd != 128) and nq != 1)
         self.nq = nq
         self.masked = masked
-        self.t = Table(nq, masked)
+        self.hd = hd
+        self.dims = hd // 32                  # dim tiles of the output, and copy instructions of a wave for K and for V
+        self.frags = hd // 16                 # operand fragments of a half, of K (k-steps) and of V^T (dim tiles x 2)
+        self.row = 2 * hd                     # bytes of a K or V row in LDS
+        self.half = 32 * self.row
+        tile = 2 * self.half
+        self.k_slot = [0, tile]               # byte offsets of the ring slots from the LDS array's start
+        self.v_slot = [2 * tile, 3 * tile]
+        self.v_read = [0, tile]               # ... of the V slots from the addresses in VOFF (which point into V slot 0)
+        self.t = Table(nq, masked, hd)
 
     # ---------------------------------------------------------------- instruction builders
     def mfma(self, dst, a, b, c):
@@ -222,36 +235,36 @@ class Gen:
         return Ins(f"v_mfma_f32_32x32x16_bf16 {vr(dst, 16)}, {vr(a, 4)}, {vr(b, 4)}, {vr(c, 16)}", "mfma", reads, rng(dst, 16))
 
     def lds_k(self, f, slot):
-        """K fragment f (0..15: half f // 8, k-step f % 8) -> KF[f % NBUF]"""
+        """K fragment f (half f // frags, k-step f % frags) -> KF[f % nbuf]"""
         t = self.t
-        k, half = f % 8, f // 8
-        dst = t.KF + 4 * (f % NBUF)
-        off = K_SLOT[slot] + half * HALF
+        k, half = f % self.frags, f // self.frags
+        dst = t.KF + 4 * (f % t.nbuf)
+        off = self.k_slot[slot] + half * self.half
         return [Ins(f"ds_read_b128 {vr(dst, 4)}, {vr(t.KOFF + k)} offset:{off}", "lds", [t.KOFF + k], rng(dst, 4), lds_tag=("k", f))]
 
     def lds_v(self, f, slot):
-        """two transposing reads: V^T fragment f (half f // 8, k-step (f % 8) >> 2, dim tile f & 3) -> VF[f % NBUF]"""
+        """two transposing reads: V^T fragment f (half f // frags, in it k-step by k-step the dim tiles) -> VF[f % nbuf]"""
         t = self.t
-        k, half = f % 8, f // 8
-        dst = t.VF + 4 * (f % NBUF)
-        d, kk = k & 3, k >> 2
-        off = V_READ[slot] + half * HALF + kk * 4096
+        k, half = f % self.frags, f // self.frags
+        dst = t.VF + 4 * (f % t.nbuf)
+        d, kk = k % self.dims, k // self.dims
+        off = self.v_read[slot] + half * self.half + kk * 16 * self.row
         return [Ins(f"ds_read_b64_tr_b16 {vr(dst, 2)}, {vr(t.VOFF + d)} offset:{off}", "lds", [t.VOFF + d], rng(dst, 2), lds_tag=("vlo", f)),
-                Ins(f"ds_read_b64_tr_b16 {vr(dst + 2, 2)}, {vr(t.VOFF + d)} offset:{off + 2048}", "lds", [t.VOFF + d],
+                Ins(f"ds_read_b64_tr_b16 {vr(dst + 2, 2)}, {vr(t.VOFF + d)} offset:{off + 8 * self.row}", "lds", [t.VOFF + d],
                     rng(dst + 2, 2), lds_tag=("vhi", f))]
 
     def mfma_qk(self, f, q, sn):
         t = self.t
-        k = f % 8
-        ins = self.mfma(t.S[q][sn], t.KF + 4 * (f % NBUF), t.Q[q] + 4 * k, t.NM[q] if k == 0 else t.S[q][sn])
+        k = f % self.frags
+        ins = self.mfma(t.S[q][sn], t.KF + 4 * (f % t.nbuf), t.Q[q] + 4 * k, t.NM[q] if k == 0 else t.S[q][sn])
         ins.lds_need = None if "nolds" in X else [("k", f)]
         return ins
 
     def mfma_pv(self, f, q, pp):
         t = self.t
-        k = f % 8
-        d, kk = k & 3, k >> 2
-        ins = self.mfma(t.O[q][d], t.VF + 4 * (f % NBUF), t.P[q][pp] + 4 * kk, t.O[q][d])
+        k = f % self.frags
+        d, kk = k % self.dims, k // self.dims
+        ins = self.mfma(t.O[q][d], t.VF + 4 * (f % t.nbuf), t.P[q][pp] + 4 * kk, t.O[q][d])
         ins.lds_need = None if "nolds" in X else [("vlo", f), ("vhi", f)]
         return ins
 
@@ -346,9 +359,9 @@ class Gen:
         return out
 
     def copy_ins(self, n, is_v, fill_slot):
-        """global -> LDS copy n (0..3) of this wave: 1 KiB block 4*wave + n of the slot"""
+        """global -> LDS copy n of this wave: 1 KiB block dims * wave + n of the slot"""
         t = self.t
-        base = (V_SLOT if is_v else K_SLOT)[fill_slot] + n * 1024
+        base = (self.v_slot if is_v else self.k_slot)[fill_slot] + n * 1024
         ofs = (t.OFSV if is_v else t.OFSK) + n
         sb = VB if is_v else KB
         if "copyexec0" in X:  # probe: the instruction is issued, no lane moves data
@@ -380,7 +393,7 @@ class Gen:
                     pos += 1
 
         def frag_reads(which, f):
-            if f >= 16 or "nolds" in X:
+            if f >= 2 * self.frags or "nolds" in X:
                 return
             for x in (self.lds_k(f, ks) if which == "k" else self.lds_v(f, vs)):
                 em.emit(x)
@@ -389,25 +402,25 @@ class Gen:
         # runs while the step's first fragments travel; the rest is dealt out behind the matrix instructions
         lead = (12 if self.masked else 6) if it == 0 else 0
         deal(lead)
-        slots = 16 * nq
+        slots = 2 * self.frags * nq
         rest = len(stream) - lead
         per = [rest // slots] * slots
         rem = rest - sum(per)
         for i in range(rem):
             per[(i * slots) // rem] += 1
         s = 0
-        for k in range(8):
-            f = 8 * it + k
+        for k in range(self.frags):
+            f = self.frags * it + k
             for q in range(nq):
                 em.emit(self.mfma_qk(f, q, sn))
                 if q == nq - 1:
-                    frag_reads("k", f + AHEAD)
+                    frag_reads("k", f + ahead(self.hd))
                 deal(per[s])
                 s += 1
             for q in range(nq):
                 em.emit(self.mfma_pv(f, q, pp))
                 if q == nq - 1:
-                    frag_reads("v", f + AHEAD)
+                    frag_reads("v", f + ahead(self.hd))
                     if copies and "stagger" in X:
                         # wave w of the workgroup issues its eight copies at matrix slots 4w .. 4w+3 of the
                         # step (two per slot): the four waves never queue for the texture path together
@@ -492,10 +505,10 @@ class Gen:
         em.raw(f"s_lshl_b32 {t1}, {t1}, 2")
         em.raw(f"s_load_dword s{PGC}, %[pages], {t1}")
         if "nolds" not in X:
-            for f in range(AHEAD):
+            for f in range(ahead(self.hd)):
                 for x in self.lds_k(f, ks) + self.lds_v(f, vs):
                     em.emit(x)
-        copies = [self.copy_ins(n, False, 1 - ks) for n in range(4)] + [self.copy_ins(n, True, 1 - vs) for n in range(4)]
+        copies = [self.copy_ins(n, False, 1 - ks) for n in range(self.dims)] + [self.copy_ins(n, True, 1 - vs) for n in range(self.dims)]
         if "nocopy" in X:
             copies = []
         if "halfcopy" in X:  # probe: half of the tile bytes (what a tile shared by 256 rows would move per wave)
@@ -553,21 +566,21 @@ class Gen:
         em = self.generate()
         n_mfma = sum(1 for i in em.out if i.kind == "mfma")
         n_valu = sum(1 for i in em.out if i.kind in ("valu", "trans", "swap", "dot"))
-        sfx = f"_NQ{nq}" + ("M" if self.masked else "")
+        sfx = (f"_NQ{nq}" if self.hd == 128 else f"_D{self.hd}") + ("M" if self.masked else "")
         text = (
-            f"// ---- NQ = {nq}{' with the causal mask' if self.masked else ''}: {len(em.out)} lines, {n_mfma} matrix and {n_valu} vector instructions (rare paths "
+            f"// ---- NQ = {nq}{'' if self.hd == 128 else f', heads of {self.hd} dims'}{' with the causal mask' if self.masked else ''}: {len(em.out)} lines, {n_mfma} matrix and {n_valu} vector instructions (rare paths "
             f"included), {em.nops} padding wait states; {t.num_vgpr} vector + {t.num_agpr} accumulation registers\n"
         )
         binds = {}
         for q in range(nq):
-            for d in range(4):
+            for d in range(self.dims):
                 binds[f"O{q}{d}"] = (t.O[q][d], 16)
-            binds[f"Q{q}"] = (t.Q[q], 32)
+            binds[f"Q{q}"] = (t.Q[q], 4 * self.frags)
             binds[f"S{q}0"], binds[f"S{q}1"] = (t.S[q][0], 16), (t.S[q][1], 16)
             binds[f"P{q}0"], binds[f"P{q}1"] = (t.P[q][0], 8), (t.P[q][1], 8)
             binds[f"NM{q}"] = (t.NM[q], 16)
             binds[f"M{q}"], binds[f"L{q}"] = (t.M[q], 1), (t.L[q], 1)
-        binds.update({"KOFF": (t.KOFF, 8), "VOFF": (t.VOFF, 4), "OFSK": (t.OFSK, 4), "OFSV": (t.OFSV, 4)})
+        binds.update({"KOFF": (t.KOFF, self.frags), "VOFF": (t.VOFF, self.dims), "OFSK": (t.OFSK, self.dims), "OFSV": (t.OFSV, self.dims)})
         if self.masked:
             binds.update({"THR": (t.THR, 1), "NINF": (t.NINF, 1)})
         for name, (lo, n) in binds.items():
@@ -575,12 +588,12 @@ class Gen:
         lines = ['    "%s\\n"' % ins.text for ins in em.out]
         text += f"#define RPA_PIPE{sfx}_ASM \\\n" + " \\\n".join(lines) + "\n"
         clob = ['"v%d"' % r for r in range(t.first_scratch, t.num_vgpr)]
-        clob += ['"%s"' % vr(r) for r in list(rng(t.KF, 4 * NBUF)) + list(rng(t.VF, 4 * NBUF))]
+        clob += ['"%s"' % vr(r) for r in list(rng(t.KF, 4 * t.nbuf)) + list(rng(t.VF, 4 * t.nbuf))]
         clob += ['"s%d"' % r for r in SGPR_CLOBBERS]
         if self.masked:
             clob += ['"s%d"' % r for sg in MASK_SGPR for r in (sg, sg + 1)]
         text += f"#define RPA_PIPE{sfx}_CLOBBERS " + ", ".join(clob) + ', "vcc", "scc", "m0", "memory"\n'
-        print(f"NQ={nq}{'M' if self.masked else ''}: {len(em.out)} lines, {n_mfma} MFMAs, {n_valu} vector, {em.nops} padding wait states, "
+        print(f"{sfx[1:]}: {len(em.out)} lines, {n_mfma} MFMAs, {n_valu} vector, {em.nops} padding wait states, "
               f"{t.num_vgpr} VGPRs + {t.num_agpr} AGPRs")
         return text
 
@@ -589,11 +602,13 @@ def main():
     here = os.path.dirname(os.path.abspath(__file__))
     text = ("// GENERATED by gen_prefill_pipe_loop.py -- do not edit; edit the generator and run it.\n"
             "// Steady-state loop of rpa_prefill_pipe_kernel: steps t .. t_end-1 of one wave, for one and two\n"
-            "// blocks of 32 query rows per wave.  The RPA_PIPE_NQn_C_* macros are the register constraints\n"
-            "// that bind the kernel's variables to the registers the assembly uses.\n")
+            "// blocks of 32 query rows per wave and for heads of 64 dims.  The RPA_PIPE_*_C_* macros are the register\n"
+            "// constraints that bind the kernel's variables to the registers the assembly uses.\n")
     for nq in (1, 2):
         text += Gen(nq).emit_text()
     text += Gen(1, masked=True).emit_text()
+    text += Gen(1, hd=64).emit_text()
+    text += Gen(1, masked=True, hd=64).emit_text()
     with open(os.path.join(here, "rpa_prefill_pipe_loop.inc"), "w") as f:
         f.write(text)
 

@@ -457,8 +457,8 @@ __device__ __forceinline__ void softmax_tile(f32x16_t (&S)[2], f32x16_t (&O)[kDi
 // has no row of its own takes part in the exchange (row_of_32).  8 prompts of 500..1500 tokens x 32 / 8 heads 108.7 -> 102.0 us, 30 of
 // 100..300 65.5 -> 60.9, 20 of 200..600 x 16 / 8 with a window and sinks 56.5 -> 52.2, 6 chunks of 200..900 e4m3 64.7 -> 61.9, the mixed batch of 56
 // rows and 8 chunks 332 -> 325, 256-wide prompts 105 -> 101.  (Partial rows, 32 bytes at a time, lost 1 % by the exchange.)
-__device__ __forceinline__ void write_rows(const PrefillArgs& a, const Work& w, const WaveRows& wr,
-                                           const f32x16_t (&O)[kDimTiles], float l, int h, float m2) {
+template <int N = kDimTiles>
+__device__ __forceinline__ void write_rows(const PrefillArgs& a, const Work& w, const WaveRows& wr, const f32x16_t (&O)[N], float l, int h, float m2) {
   l = swap_sum(l);
   if (!wr.active) return;
   const float vs = a.v_scale ? scalar_load_f32(a.v_scale + w.hk) : 1.0f;
@@ -468,7 +468,7 @@ __device__ __forceinline__ void write_rows(const PrefillArgs& a, const Work& w, 
   const int64_t upper_rows = (int64_t)16 * a.Hq * a.q_dim;
   const bool has_lower = row < w.q_len, has_upper = row + 16 < w.q_len;
 #pragma unroll
-  for (int d = 0; d < kDimTiles; ++d) {
+  for (int d = 0; d < N; ++d) {
     u32x2_t p[4];
 #pragma unroll
     for (int vq = 0; vq < 4; ++vq)
@@ -532,15 +532,16 @@ __device__ __forceinline__ bool kv_piece(const PrefillArgs& a, int& t_lo, int& t
 }
 
 // lane (c, h) holds query row c, dims 32d + 8*(v/4) + 4h + v%4 in O[d][v]
-__device__ __forceinline__ void write_partial_rows(const PrefillArgs& a, const Work& w, const WaveRows& wr,
-                                                   const f32x16_t (&O)[kDimTiles], float l, int h, float m2, int split) {
+// (of narrow heads the first N tiles of 32; the merge's sums of the others are not used)
+template <int N = kDimTiles>
+__device__ __forceinline__ void write_partial_rows(const PrefillArgs& a, const Work& w, const WaveRows& wr, const f32x16_t (&O)[N], float l, int h, float m2, int split) {
   typedef float f32x4_t __attribute__((ext_vector_type(4)));
   l += __shfl_xor(l, 32);
   if (!wr.active || wr.row >= w.q_len) return;
   const int64_t slot = ((int64_t)(w.qg0 + wr.row) * a.Hq + w.head) * a.kv_splits + split;
   float* op = a.ws_o + slot * kHeadDim + 4 * h;
 #pragma unroll
-  for (int d = 0; d < kDimTiles; ++d)
+  for (int d = 0; d < N; ++d)
 #pragma unroll
     for (int vq = 0; vq < 4; ++vq)
       *reinterpret_cast<f32x4_t*>(op + d * 32 + vq * 8) =
@@ -551,11 +552,12 @@ __device__ __forceinline__ void write_partial_rows(const PrefillArgs& a, const W
   }
 }
 
+template <int N = kDimTiles>
 __device__ __forceinline__ void write_empty_partial_rows(const PrefillArgs& a, const Work& w, const WaveRows& wr, int h,
                                                          int split) {
-  f32x16_t zero[kDimTiles];
+  f32x16_t zero[N];
 #pragma unroll
-  for (int d = 0; d < kDimTiles; ++d) zero[d] = kZero16;
+  for (int d = 0; d < N; ++d) zero[d] = kZero16;
   write_partial_rows(a, w, wr, zero, 0.f, h, kNoReference, split);
 }
 

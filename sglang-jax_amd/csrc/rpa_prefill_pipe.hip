@@ -46,34 +46,34 @@ using namespace pf;
 
 namespace {
 
-// For a full tile inside one page the byte offset of a lane's chunk from the tile's first row never changes: it is computed
-// once, and a copy costs no vector ALU work, only a scalar tile base.
-struct AsyncOffsets {
-  uint32_t k[kCopies], v[kCopies];
+// Heads of HD dims (128, or 64: the second half of a cached row is zero, and is neither copied nor multiplied).  A K or V row
+// takes 2 * HD bytes of LDS; 16-byte chunk j of row t sits at chunk position j ^ swizzle(t):
+//   K: 16 consecutive rows in 16 distinct 16-byte columns of the 256 bytes that one clock reads (ds_read_b128)
+//   V: 4 consecutive rows in its 4 distinct 64-byte windows (transposing read)
+// with two rows of 64 dims side by side in those 256 bytes.
+template <int HD>
+struct Head {
+  static_assert(HD == 128 || HD == 64, "");
+  static constexpr int kSteps = HD / 16;        // k-steps of the first product
+  static constexpr int kDims = HD / 32;         // dim tiles of the output; copy instructions per wave for K and for V
+  static constexpr int kChunksPerRow = HD / 8;
+  static constexpr int kRow = 2 * HD;
+  static constexpr int kHalfB = 32 * kRow;      // byte distance between the halves of a tile
+  static constexpr int kTile = 2 * kHalfB;
+  static constexpr int kKSlot = 0;              // ring slots inside the LDS array: K0 K1 V0 V1
+  static constexpr int kVSlot = 2 * kTile;
+  __device__ static __forceinline__ int k_swizzle(int t) { return HD == 128 ? (t & 15) : ((t >> 1) & 7); }
+  __device__ static __forceinline__ int v_swizzle(int t) { return HD == 128 ? ((t & 3) << 2) : ((t & 2) << 1); }
+  // copy n of a wave moves chunk position lane % kChunksPerRow of this row of the tile
+  __device__ static __forceinline__ int copy_row(int wave, int n, int lane) {
+    return (wave * kDims + n) * (64 / kChunksPerRow) + lane / kChunksPerRow;
+  }
 };
 
-__device__ __forceinline__ AsyncOffsets make_async_offsets(const KvAddr& kv, int wave, int lane) {
-  AsyncOffsets o;
-  const int cp = lane % kChunks;
-#pragma unroll
-  for (int n = 0; n < kCopies; ++n) {
-    const int t = (wave * kCopies + n) * kRowsPerCopy + lane / kChunks;
-    o.k[n] = (uint32_t)(t * kv.tok_stride + ((cp ^ (t & 15)) << 4));
-    o.v[n] = (uint32_t)(t * kv.tok_stride + ((cp ^ ((t & 3) << 2)) << 4));
-  }
-  return o;
-}
-
-constexpr int kHalfB = 32 * kRowB;       // byte distance between the halves of a tile
-constexpr int kKSlot = 0;                // ring slots inside the LDS array: K0 K1 V0 V1
-constexpr int kVSlot = 2 * kTileB;
 constexpr float kRowSumLimit = 256.0f;   // a half's row sum above it: the stale maximum is too stale
 constexpr float kSeenFloor = -1.0e30f;   // a row maximum below it: every token so far was masked
 
-typedef uint32_t u32x32_t __attribute__((ext_vector_type(32)));
 typedef uint32_t u32x8_t __attribute__((ext_vector_type(8)));
-typedef int32_t i32x8_t __attribute__((ext_vector_type(8)));
-typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x4v_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ u32x4_t lds_ld16_at(int addr) {
@@ -87,9 +87,11 @@ __device__ __forceinline__ u32x2_t lds_tr16_at(int addr) {
 
 // The registers of one block of 32 query rows.  The assembly loop expects them in the registers the
 // RPA_PIPE_NQn_C_* constraints of rpa_prefill_pipe_loop.inc name.
+template <int HD>
 struct RowBlock {
-  f32x16_t O[4];    // accumulators, lane (c, h): row c, dims 32d + 8*(v/4) + 4h + v%4
-  u32x32_t Q;       // Q^T operands of the 8 k-steps, scaled to log2 units
+  typedef uint32_t q_t __attribute__((ext_vector_type(4 * Head<HD>::kSteps)));
+  f32x16_t O[Head<HD>::kDims];  // accumulators, lane (c, h): row c, dims 32d + 8*(v/4) + 4h + v%4
+  q_t Q;            // Q^T operands of the k-steps, scaled to log2 units
   f32x16_t S[2];    // scores of the even / odd half in flight, minus the running maximum
   u32x8_t P[2];     // probabilities of the even / odd half (two B operands of the second product each)
   f32x16_t NM;      // minus the running maximum in all 16 registers (C operand of a score chain's first MFMA)
@@ -98,28 +100,32 @@ struct RowBlock {
   int qpos;         // position of this lane's row
 };
 
+template <int HD>
 struct Shared {   // what the row blocks of a wave share
-  i32x8_t koff;   // LDS addresses of the K operand reads (slot 0, first half)
-  i32x4_t voff;   // LDS addresses of the V^T operand reads (slot 0, first half, first k-step)
-  u32x4_t ofs_k, ofs_v;  // per-lane byte offsets of this wave's four K / V copy instructions
+  typedef int32_t koff_t __attribute__((ext_vector_type(Head<HD>::kSteps)));
+  typedef int32_t voff_t __attribute__((ext_vector_type(Head<HD>::kDims)));
+  typedef uint32_t ofs_t __attribute__((ext_vector_type(Head<HD>::kDims)));
+  koff_t koff;    // LDS addresses of the K operand reads (slot 0, first half)
+  voff_t voff;    // LDS addresses of the V^T operand reads (slot 0, first half, first k-step)
+  ofs_t ofs_k, ofs_v;  // per-lane byte offsets of this wave's K / V copy instructions
 };
 
-template <int KS>
-__device__ __forceinline__ u32x4_t q_frag(const u32x32_t& q) {
-  return u32x4_t{q[4 * KS], q[4 * KS + 1], q[4 * KS + 2], q[4 * KS + 3]};
+template <int HD>
+__device__ __forceinline__ u32x4_t q_frag(const RowBlock<HD>& b, int ks) {
+  return u32x4_t{b.Q[4 * ks], b.Q[4 * ks + 1], b.Q[4 * ks + 2], b.Q[4 * ks + 3]};
 }
 
-// K or V rows of one tile, global -> LDS: 4 instructions per wave.  `lds_wave` is the LDS address
+// K or V rows of one tile, global -> LDS: HD / 32 instructions per wave.  `lds_wave` is the LDS address
 // of this wave's first 1 KiB block of the slot.
-template <bool IS_V>
+template <bool IS_V, int HD>
 __device__ __forceinline__ void copy_rows(uint32_t lds_wave, const TileSrc& s, const KvAddr& kv, const char* head, int tb,
-                                          int wave, int lane, int page, const Shared& sh) {
+                                          int wave, int lane, int page, const Shared<HD>& sh) {
   tb = min(tb, s.last_tok & ~(kBN - 1));
   if (tb + kBN - 1 <= s.last_tok) {
     const int64_t base = (int64_t)page * kv.page_stride + (int64_t)(tb - page_slot(s, tb) * s.page_size) * kv.tok_stride;
     const char* b = head + base;  // wave-uniform
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
+    for (int n = 0; n < Head<HD>::kDims; ++n) {
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                    :: "s"(lds_wave + n * 1024), "v"(IS_V ? sh.ofs_v[n] : sh.ofs_k[n]), "s"(b)
                    : "memory", "m0");
@@ -127,12 +133,12 @@ __device__ __forceinline__ void copy_rows(uint32_t lds_wave, const TileSrc& s, c
     return;
   }
   // last, partial tile: rows clamped to the last valid token
-  const int cp = lane & 15;
+  const int cp = lane % Head<HD>::kChunksPerRow;
 #pragma unroll
-  for (int n = 0; n < 4; ++n) {
-    const int t = (wave * 4 + n) * 4 + (lane >> 4);
+  for (int n = 0; n < Head<HD>::kDims; ++n) {
+    const int t = Head<HD>::copy_row(wave, n, lane);
     const int64_t ro = row_offset<true>(s, kv, tb, tb + t, page);
-    const int j = IS_V ? (cp ^ ((t & 3) << 2)) : (cp ^ (t & 15));
+    const int j = cp ^ (IS_V ? Head<HD>::v_swizzle(t) : Head<HD>::k_swizzle(t));
     const char* g = head + ro + j * 16;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                  :: "s"(lds_wave + n * 1024), "v"(g)
@@ -145,29 +151,26 @@ __device__ __forceinline__ int scalar_page(const TileSrc& s, int tb) {
   return scalar_load_i32(s.pages + __builtin_amdgcn_readfirstlane(page_slot(s, tb)));
 }
 
-// first product of one 32-token half: one chain of 8 MFMAs starting from minus the running
+// first product of one 32-token half: one chain of MFMAs starting from minus the running
 // maximum; `off` = slot and half offset
-__device__ __forceinline__ f32x16_t qk_half(const RowBlock& b, const Shared& sh, int off) {
-  f32x16_t S = mfma32(lds_ld16_at(sh.koff[0] + off), q_frag<0>(b.Q), b.NM);
-  S = mfma32(lds_ld16_at(sh.koff[1] + off), q_frag<1>(b.Q), S);
-  S = mfma32(lds_ld16_at(sh.koff[2] + off), q_frag<2>(b.Q), S);
-  S = mfma32(lds_ld16_at(sh.koff[3] + off), q_frag<3>(b.Q), S);
-  S = mfma32(lds_ld16_at(sh.koff[4] + off), q_frag<4>(b.Q), S);
-  S = mfma32(lds_ld16_at(sh.koff[5] + off), q_frag<5>(b.Q), S);
-  S = mfma32(lds_ld16_at(sh.koff[6] + off), q_frag<6>(b.Q), S);
-  S = mfma32(lds_ld16_at(sh.koff[7] + off), q_frag<7>(b.Q), S);
+template <int HD>
+__device__ __forceinline__ f32x16_t qk_half(const RowBlock<HD>& b, const Shared<HD>& sh, int off) {
+  f32x16_t S = mfma32(lds_ld16_at(sh.koff[0] + off), q_frag(b, 0), b.NM);
+#pragma unroll
+  for (int ks = 1; ks < Head<HD>::kSteps; ++ks) S = mfma32(lds_ld16_at(sh.koff[ks] + off), q_frag(b, ks), S);
   return S;
 }
 
-// second product of one 32-token half: four chains of 2 MFMAs
-__device__ __forceinline__ void pv_half(RowBlock& b, const Shared& sh, int off, const u32x8_t& P) {
+// second product of one 32-token half: a chain of 2 MFMAs per dim tile
+template <int HD>
+__device__ __forceinline__ void pv_half(RowBlock<HD>& b, const Shared<HD>& sh, int off, const u32x8_t& P) {
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const int vt = sh.voff[d] + off + kk * 16 * kRowB;
+    for (int d = 0; d < Head<HD>::kDims; ++d) {
+      const int vt = sh.voff[d] + off + kk * 16 * Head<HD>::kRow;
       const u32x2_t lo = lds_tr16_at(vt);
-      const u32x2_t hi = lds_tr16_at(vt + 8 * kRowB);
+      const u32x2_t hi = lds_tr16_at(vt + 8 * Head<HD>::kRow);
       b.O[d] = mfma32(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, u32x4_t{P[4 * kk], P[4 * kk + 1], P[4 * kk + 2], P[4 * kk + 3]},
                       b.O[d]);
     }
@@ -198,7 +201,8 @@ __device__ __forceinline__ float row_max16(const f32x16_t& S) {
 // Softmax of a half with the maximum taken first (first halves of a row, masked halves).  Sc: the
 // half's scores relative to the running maximum; Sn: the scores of the next half, already computed
 // against the same maximum, which move with it.
-__device__ __forceinline__ void softmax_half_general(f32x16_t& Sc, f32x16_t& Sn, RowBlock& b, bool need_mask, int tb, int h,
+template <int HD>
+__device__ __forceinline__ void softmax_half_general(f32x16_t& Sc, f32x16_t& Sn, RowBlock<HD>& b, bool need_mask, int tb, int h,
                                                      int window, u32x8_t& P) {
   if (need_mask) {
 #pragma unroll
@@ -218,7 +222,7 @@ __device__ __forceinline__ void softmax_half_general(f32x16_t& Sc, f32x16_t& Sn,
     b.m += d;
     b.l *= alpha;
 #pragma unroll
-    for (int dd = 0; dd < 4; ++dd)
+    for (int dd = 0; dd < Head<HD>::kDims; ++dd)
 #pragma unroll
       for (int v = 0; v < 16; ++v) b.O[dd][v] *= alpha;
 #pragma unroll
@@ -248,7 +252,7 @@ struct LoopScalars {
       [pstr] "s"(sc.pstr), [kh_lo] "s"(sc.kh_lo), [kh_hi] "s"(sc.kh_hi), [vh_lo] "s"(sc.vh_lo),                    \
       [vh_hi] "s"(sc.vh_hi), [lds_wave] "s"(sc.lds_wave), [pages] "s"(sc.pages)
 
-__device__ __forceinline__ void pipe_loop(RowBlock (&b)[1], const Shared& sh, int& t, int& pg_a, int& pg_b,
+__device__ __forceinline__ void pipe_loop(RowBlock<128> (&b)[1], const Shared<128>& sh, int& t, int& pg_a, int& pg_b,
                                           const LoopScalars& sc) {
 #define C(n) RPA_PIPE_NQ1_C_##n
   // t and the page ids change inside the block while inputs are still being read: early-clobber, so that no
@@ -267,7 +271,7 @@ __device__ __forceinline__ void pipe_loop(RowBlock (&b)[1], const Shared& sh, in
 // The same steps with the causal mask applied to every half before its exponentials (the steps on the
 // diagonal).  thr: query position - first token of the half whose probabilities the block's first iteration
 // takes (half 2t - 1) - 4 * (lane / 32); the block moves it on by 32 per half.
-__device__ __forceinline__ void pipe_loop_masked(RowBlock (&b)[1], const Shared& sh, int& t, int& pg_a, int& pg_b,
+__device__ __forceinline__ void pipe_loop_masked(RowBlock<128> (&b)[1], const Shared<128>& sh, int& t, int& pg_a, int& pg_b,
                                                  const LoopScalars& sc, int thr) {
 #define C(n) RPA_PIPE_NQ1M_C_##n
   const float ninf = -1.0e30f;
@@ -281,9 +285,9 @@ __device__ __forceinline__ void pipe_loop_masked(RowBlock (&b)[1], const Shared&
                : RPA_PIPE_NQ1M_CLOBBERS);
 #undef C
 }
-__device__ __forceinline__ void pipe_loop_masked(RowBlock (&)[2], const Shared&, int&, int&, int&, const LoopScalars&, int) {}
+__device__ __forceinline__ void pipe_loop_masked(RowBlock<128> (&)[2], const Shared<128>&, int&, int&, int&, const LoopScalars&, int) {}
 
-__device__ __forceinline__ void pipe_loop(RowBlock (&b)[2], const Shared& sh, int& t, int& pg_a, int& pg_b,
+__device__ __forceinline__ void pipe_loop(RowBlock<128> (&b)[2], const Shared<128>& sh, int& t, int& pg_a, int& pg_b,
                                           const LoopScalars& sc) {
 #define C(n) RPA_PIPE_NQ2_C_##n
   asm volatile(RPA_PIPE_NQ2_ASM
@@ -300,6 +304,42 @@ __device__ __forceinline__ void pipe_loop(RowBlock (&b)[2], const Shared& sh, in
 #undef C
 }
 
+// The same two blocks for heads of 64 dims.
+__device__ __forceinline__ void pipe_loop(RowBlock<64> (&b)[1], const Shared<64>& sh, int& t, int& pg_a, int& pg_b,
+                                          const LoopScalars& sc) {
+#define C(n) RPA_PIPE_D64_C_##n
+  asm volatile(RPA_PIPE_D64_ASM
+               : "+" C(O00)(b[0].O[0]), "+" C(O01)(b[0].O[1]),
+                 "+" C(S00)(b[0].S[0]), "+" C(S01)(b[0].S[1]), "+" C(P00)(b[0].P[0]), "+" C(P01)(b[0].P[1]),
+                 "+" C(NM0)(b[0].NM), "+" C(M0)(b[0].m), "+" C(L0)(b[0].l),
+                 [t] "+&s"(t), [pg_a] "+&s"(pg_a), [pg_b] "+&s"(pg_b)
+               : C(Q0)(b[0].Q), C(KOFF)(sh.koff), C(VOFF)(sh.voff), C(OFSK)(sh.ofs_k), C(OFSV)(sh.ofs_v),
+                 RPA_PIPE_SCALARS(sc)
+               : RPA_PIPE_D64_CLOBBERS);
+#undef C
+}
+
+__device__ __forceinline__ void pipe_loop_masked(RowBlock<64> (&b)[1], const Shared<64>& sh, int& t, int& pg_a, int& pg_b,
+                                                 const LoopScalars& sc, int thr) {
+#define C(n) RPA_PIPE_D64M_C_##n
+  const float ninf = -1.0e30f;
+  asm volatile(RPA_PIPE_D64M_ASM
+               : "+" C(O00)(b[0].O[0]), "+" C(O01)(b[0].O[1]),
+                 "+" C(S00)(b[0].S[0]), "+" C(S01)(b[0].S[1]), "+" C(P00)(b[0].P[0]), "+" C(P01)(b[0].P[1]),
+                 "+" C(NM0)(b[0].NM), "+" C(M0)(b[0].m), "+" C(L0)(b[0].l), "+" C(THR)(thr),
+                 [t] "+&s"(t), [pg_a] "+&s"(pg_a), [pg_b] "+&s"(pg_b)
+               : C(Q0)(b[0].Q), C(KOFF)(sh.koff), C(VOFF)(sh.voff), C(OFSK)(sh.ofs_k), C(OFSV)(sh.ofs_v), C(NINF)(ninf),
+                 RPA_PIPE_SCALARS(sc)
+               : RPA_PIPE_D64M_CLOBBERS);
+#undef C
+}
+
+// HD = 64: narrow heads.  With the zeros of their rows copied and multiplied, 4 chunks of 1500..2048 tokens on prefixes of up to
+// 4096, 32 / 8 heads, took 391 us, as long as heads of 128 dims but for the writes.  Half the copies and matrix instructions at two
+// workgroups per CU: 268 us; 166 registers and 32 KiB of LDS leave room for a third, whose wavefronts fill what the others wait for
+// (operands two instead of three fragments ahead): 253, 2 x 2000 tokens on 16000 832 -> 539, 3 prompts of 200..1400 34.6 -> 25.9.  What
+// bounds it now is the rate at which a CU's copies land (32 bytes per ns) and the exponentials, which are as many as of wide heads.
+//
 // HEADS4: the short-chunk tile.  A workgroup owns 32 query positions of FOUR query heads of a kv head, one
 // head per wave, instead of 128 positions of one head: chunks of a few dozen tokens (a verify step, a short
 // prompt, the tail of a long one) then fill their tiles, and the four waves still share every K/V tile.
@@ -308,8 +348,8 @@ __device__ __forceinline__ void pipe_loop(RowBlock (&b)[2], const Shared& sh, in
 // long context) cut every workgroup's run of K/V tiles into a.kv_splits pieces, blockIdx.y picks the piece,
 // and the workgroup leaves unnormalised rows with their (reference, sum) in the workspace for
 // rpa_prefill_combine_kernel instead of finished rows.
-template <bool WIN, int NQ, bool HEADS4 = false, bool SPLIT = false>
-__global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kernel(const PrefillArgs a_in, int tiles, int nseq,
+template <bool WIN, int NQ, bool HEADS4 = false, bool SPLIT = false, int HD = 128>
+__global__ __launch_bounds__(256, (HD == 64 ? 3 : NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kernel(const PrefillArgs a_in, int tiles, int nseq,
                                                                                  bool by_level, float row_sum_limit,
                                                                                  bool masked_steps) {
   PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
@@ -317,9 +357,10 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
     a.seq_end = min(a.seq_end, scalar_load_i32(a.dist + 2));
   }
-  static_assert(!HEADS4 || NQ == 1, "the short-chunk tile has one block of rows per wave");
+  static_assert((!HEADS4 && HD == 128) || NQ == 1, "the short-chunk tile and narrow heads have one block of rows per wave");
+  typedef Head<HD> HL;
   constexpr int BM = HEADS4 ? 32 : 128 * NQ;  // query positions per workgroup
-  __shared__ __attribute__((aligned(1024))) char lds[4 * kTileB];
+  __shared__ __attribute__((aligned(1024))) char lds[4 * HL::kTile];
 
   Work w = decompose<true>(a, tiles, nseq, by_level, BM, HEADS4 ? 4 : 1);
   if (!w.valid) {
@@ -359,7 +400,7 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
         wr.active = wr.r_lo < w.q_len;
         wr.row = wr.r_lo + c;
         wr.qpos = w.prefix + wr.row;
-        write_empty_partial_rows(a, w, wr, h, split);
+        write_empty_partial_rows<HL::kDims>(a, w, wr, h, split);
       }
       return;
     }
@@ -369,22 +410,22 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
   }
   const int nT = (t_hi - t_lo + kBN - 1) / kBN;  // K/V tiles of the workgroup (of its piece)
 
-  RowBlock b[NQ];
+  RowBlock<HD> b[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
     const int row = r_lo + 32 * q + c;
     b[q].qpos = w.prefix + row;
     const int rr = min(row, w.q_len - 1);
     const uint16_t* qp = a.q + ((int64_t)(w.qg0 + rr) * a.Hq + w.head) * a.q_dim;
-    u32x4_t x[8];
-    ld_query_row<8, 128>(x, qp, h, a.q_dim);
+    u32x4_t x[HL::kSteps];
+    ld_query_row<HL::kSteps, HD>(x, qp, h, a.q_dim);
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks)
+    for (int ks = 0; ks < HL::kSteps; ++ks)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         b[q].Q[4 * ks + e] = pack_bf16x2(bf16_lo_to_f32(x[ks][e]) * sc2, bf16_hi_to_f32(x[ks][e]) * sc2);
 #pragma unroll
-    for (int d = 0; d < 4; ++d) b[q].O[d] = kZero16;
+    for (int d = 0; d < HL::kDims; ++d) b[q].O[d] = kZero16;
     b[q].S[0] = b[q].S[1] = b[q].NM = kZero16;
     b[q].P[0] = b[q].P[1] = u32x8_t{0, 0, 0, 0, 0, 0, 0, 0};
     b[q].m = 0.f;
@@ -408,29 +449,32 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
   i_f1 = __builtin_amdgcn_readfirstlane(i_f1);
 
   // operand addresses inside the LDS array (see rpa_prefill_async_kernel for the swizzles)
-  Shared sh;
+  Shared<HD> sh;
   {
-    const int k_row = c * kRowB;
-    const int k_swz = (h ^ (c & 15)) << 4;
+    const int k_row = c * HL::kRow;
+    const int k_swz = (h ^ HL::k_swizzle(c)) << 4;
     const int r16 = lane & 15, b16 = lane >> 4;
-    const int v_row = (4 * h + (r16 >> 2)) * kRowB;
+    const int v_row = (4 * h + (r16 >> 2)) * HL::kRow;
     const int v_in = ((b16 & 1) << 5) + (((r16 & 3) >> 1) << 4) + ((r16 & 1) << 3);
-    const int v_swz = (r16 >> 2) << 6;
+    const int v_swz = HL::v_swizzle(r16 >> 2) << 4;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) sh.koff[ks] = (int)lds_base + kKSlot + k_row + ((ks * 32) ^ k_swz);
+    for (int ks = 0; ks < HL::kSteps; ++ks) sh.koff[ks] = (int)lds_base + HL::kKSlot + k_row + ((ks * 32) ^ k_swz);
 #pragma unroll
-    for (int d = 0; d < 4; ++d) sh.voff[d] = (int)lds_base + kVSlot + v_row + v_in + ((d * 64) ^ v_swz);
-    const AsyncOffsets ofs = make_async_offsets(a.kv, wave, lane);
+    for (int d = 0; d < HL::kDims; ++d) sh.voff[d] = (int)lds_base + HL::kVSlot + v_row + v_in + ((d * 64) ^ v_swz);
+    // For a full tile inside one page the byte offset of a lane's chunk from the tile's first row never changes: it is
+    // computed once, and a copy costs no vector ALU work, only a scalar tile base.
+    const int cp = lane % HL::kChunksPerRow;
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      sh.ofs_k[n] = ofs.k[n];
-      sh.ofs_v[n] = ofs.v[n];
+    for (int n = 0; n < HL::kDims; ++n) {
+      const int t = HL::copy_row(wave, n, lane);
+      sh.ofs_k[n] = (uint32_t)(t * a.kv.tok_stride + ((cp ^ HL::k_swizzle(t)) << 4));
+      sh.ofs_v[n] = (uint32_t)(t * a.kv.tok_stride + ((cp ^ HL::v_swizzle(t)) << 4));
     }
   }
 
-  const uint32_t lds_wave = lds_base + wave * 4096;  // this wave's four 1 KiB blocks of slot K0
+  const uint32_t lds_wave = lds_base + wave * (HL::kDims * 1024);  // this wave's 1 KiB blocks of slot K0
   int pg_a = scalar_page(src, t_lo);         // page of tile t
-  copy_rows<false>(lds_wave + kKSlot, src, a.kv, kh, t_lo, wave, lane, pg_a, sh);
+  copy_rows<false>(lds_wave + HL::kKSlot, src, a.kv, kh, t_lo, wave, lane, pg_a, sh);
   int pg_b = scalar_page(src, t_lo + kBN);   // page of tile t + 1
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
@@ -456,8 +500,8 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
   // t - 1 from V slot 1 - par, fills K slot 1 - par with tile t + 1 and V slot par with tile t
   auto copies = [&](int t, int par) __attribute__((always_inline)) {
     if (t + 1 < nT)
-      copy_rows<false>(lds_wave + kKSlot + (1 - par) * kTileB, src, a.kv, kh, t_lo + (t + 1) * kBN, wave, lane, pg_b, sh);
-    if (t < nT) copy_rows<true>(lds_wave + kVSlot + par * kTileB, src, a.kv, vh, t_lo + t * kBN, wave, lane, pg_a, sh);
+      copy_rows<false>(lds_wave + HL::kKSlot + (1 - par) * HL::kTile, src, a.kv, kh, t_lo + (t + 1) * kBN, wave, lane, pg_b, sh);
+    if (t < nT) copy_rows<true>(lds_wave + HL::kVSlot + par * HL::kTile, src, a.kv, vh, t_lo + t * kBN, wave, lane, pg_a, sh);
     pg_a = pg_b;
     if (t + 2 < nT) pg_b = scalar_page(src, t_lo + (t + 2) * kBN);
   };
@@ -485,9 +529,9 @@ __global__ __launch_bounds__(256, (NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kerne
   auto general_step = [&](int t) __attribute__((always_inline)) {
     const int par = t & 1;
     copies(t, par);
-    const int k_off = par * kTileB, v_off = (1 - par) * kTileB;
+    const int k_off = par * HL::kTile, v_off = (1 - par) * HL::kTile;
     general_iter(std::integral_constant<int, 1>{}, 2 * t - 1, k_off, v_off);
-    general_iter(std::integral_constant<int, 0>{}, 2 * t, k_off + kHalfB, v_off + kHalfB);
+    general_iter(std::integral_constant<int, 0>{}, 2 * t, k_off + HL::kHalfB, v_off + HL::kHalfB);
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
   };
@@ -552,6 +596,8 @@ bool prefill_pipe_applies(const PrefillArgs& a) {
 
 namespace {
 int forced_nq() { return tuning().prefill_pipe_nq; }
+// queries and outputs of at most 64 dims, zero behind them in the cache
+bool narrow_heads(const PrefillArgs& a, int nq) { return nq == 1 && a.q_dim <= 64; }
 // 32 positions x 4 heads per workgroup instead of 128 x 1: row "prefill_pipe_short" of the shape table
 bool short_chunk_tile(const PrefillArgs& a, int nq) {
   return nq == 1 && select_shape(prefill_shape_key(a)).tile_q == 32;
@@ -593,33 +639,36 @@ hipError_t launch_prefill_pipe(const PrefillArgs& call, int nseq, bool level_ord
   if (grid + a.write_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   const dim3 g((unsigned)(grid + a.write_blocks)), blk(256);
   const bool win = a.sm.window > 0;
+  const bool narrow = narrow_heads(a, nq);
+#define RPA_LAUNCH(GRID, W, H4, SPLIT, HD) \
+  hipLaunchKernelGGL((rpa_prefill_pipe_kernel<W, 1, H4, SPLIT, HD>), GRID, blk, 0, stream, a, tiles, nseq, by_level, limit, masked)
+#define RPA_LAUNCH_W(GRID, H4, SPLIT, HD)             \
+  do {                                                \
+    if (win) RPA_LAUNCH(GRID, true, H4, SPLIT, HD);   \
+    else RPA_LAUNCH(GRID, false, H4, SPLIT, HD);      \
+  } while (0)
+#define RPA_LAUNCH_D(GRID, H4, SPLIT)                 \
+  do {                                                \
+    if (narrow) RPA_LAUNCH_W(GRID, H4, SPLIT, 64);    \
+    else RPA_LAUNCH_W(GRID, H4, SPLIT, 128);          \
+  } while (0)
   if (a.kv_splits > 1 && nq == 1) {  // pieces of the K/V ranges, then the merge
     if (!a.ws_o || !a.ws_ml || a.kv_splits > 64) return hipErrorInvalidValue;
     const dim3 gs((unsigned)(grid + a.write_blocks), (unsigned)a.kv_splits);
-#define RPA_LAUNCH_SPLIT(W, H4) \
-  hipLaunchKernelGGL((rpa_prefill_pipe_kernel<W, 1, H4, true>), gs, blk, 0, stream, a, tiles, nseq, by_level, limit, masked)
-    if (heads4) {
-      if (win) RPA_LAUNCH_SPLIT(true, true);
-      else RPA_LAUNCH_SPLIT(false, true);
-    } else {
-      if (win) RPA_LAUNCH_SPLIT(true, false);
-      else RPA_LAUNCH_SPLIT(false, false);
-    }
-#undef RPA_LAUNCH_SPLIT
+    if (heads4) RPA_LAUNCH_D(gs, true, true);
+    else RPA_LAUNCH_D(gs, false, true);
     return launch_prefill_combine(a, stream);
   }
-#define RPA_LAUNCH(W, N) \
-  hipLaunchKernelGGL((rpa_prefill_pipe_kernel<W, N>), g, blk, 0, stream, a, tiles, nseq, by_level, limit, masked)
   if (heads4) {
-    if (win) hipLaunchKernelGGL((rpa_prefill_pipe_kernel<true, 1, true>), g, blk, 0, stream, a, tiles, nseq, by_level, limit, masked);
-    else hipLaunchKernelGGL((rpa_prefill_pipe_kernel<false, 1, true>), g, blk, 0, stream, a, tiles, nseq, by_level, limit, masked);
+    RPA_LAUNCH_D(g, true, false);
   } else if (nq == 1) {
-    if (win) RPA_LAUNCH(true, 1);
-    else RPA_LAUNCH(false, 1);
+    RPA_LAUNCH_D(g, false, false);
   } else {
-    if (win) RPA_LAUNCH(true, 2);
-    else RPA_LAUNCH(false, 2);
+    if (win) hipLaunchKernelGGL((rpa_prefill_pipe_kernel<true, 2>), g, blk, 0, stream, a, tiles, nseq, by_level, limit, masked);
+    else hipLaunchKernelGGL((rpa_prefill_pipe_kernel<false, 2>), g, blk, 0, stream, a, tiles, nseq, by_level, limit, masked);
   }
+#undef RPA_LAUNCH_D
+#undef RPA_LAUNCH_W
 #undef RPA_LAUNCH
   return hipGetLastError();
 }

@@ -400,6 +400,29 @@ def test_narrow_heads_decode_rows(pkg, wl, gpu, head_dim, P, kv_lens, window, ca
     assert_parity(out.cpu().float(), want.float(), **BF16_TOL)
 
 
+@pytest.mark.parametrize("head_dim,Hq,Hkv,P,q_lens,kv_lens,window,splits", [
+    (64, 8, 2, 64, [1003, 130, 1, 64, 257], [1003, 700, 90, 64, 2049], None, 0), (64, 8, 4, 128, [300, 129], [4200, 129], 200, 0),
+    (48, 4, 1, 64, [33, 500], [33, 1100], None, 0), (64, 16, 4, 64, [16, 64, 3], [700, 64, 2500], None, 0),
+    (64, 8, 1, 64, [200, 31], [3000, 31], None, 3), (40, 8, 2, 64, [20, 7], [3000, 40], 1000, 4)])
+def test_narrow_heads_chunks(pkg, wl, gpu, monkeypatch, head_dim, Hq, Hkv, P, q_lens, kv_lens, window, splits):
+    """Chunks of heads of up to 64 dims on pages of whole tiles: tiles, halves and rows that end early, a window, the tile of 32
+    positions x 4 heads, K/V ranges in pieces.  Whatever stands behind the first 64 dims of a cached row is not read.  The same bf16
+    probabilities and the same sums as 128-wide heads with zeros: the tolerance is theirs."""
+    monkeypatch.setenv("RPA_PREFILL_PACKED", "0")
+    monkeypatch.setenv("RPA_PREFILL_SPLITS", str(splits))
+    b = wl.make_batch("narrow_chunks", q_lens, kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=head_dim, page_size=P, seed=79,
+                      sliding_window=window)
+    want = oracle_out(b)
+    cache = torch.nn.functional.pad(b.kv_cache, (0, 128 - head_dim))
+    cache[..., 64:] = float("nan")
+    say(f"case narrow chunks D={head_dim} Hq={Hq} Hkv={Hkv} P={P} q={q_lens} kv={kv_lens} window={window} splits={splits}")
+    g = b.to(gpu)
+    out, _ = pkg.ragged_paged_attention(g.q, None, None, cache.to(gpu), g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, (0, 0, len(q_lens)),
+                                        None, sm_scale=b.sm_scale, sliding_window=window, max_kv_len=max(kv_lens), max_q_len=max(q_lens))
+    torch.cuda.synchronize()
+    assert_parity(out[: sum(q_lens)].cpu().float(), want.float(), **BF16_TOL)
+
+
 @pytest.mark.parametrize("head_dim,aligned_pool", [(64, True), (64, False), (96, True), (80, False), (192, True), (192, False)])
 def test_head_dims_that_are_not_a_multiple_of_128(pkg, wl, gpu, head_dim, aligned_pool):
     """rpa_v3:1187-1241, 1270-1296: queries, new tokens and narrow caches run zero-padded to the next
