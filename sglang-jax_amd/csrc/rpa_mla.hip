@@ -1161,89 +1161,67 @@ __device__ __forceinline__ void mla_segment_wide(const MlaDecodeArgs& a, const M
 }
 
 // ---- token groups (see mla_segment, TG): 16 / 32 / 64 heads, every query token a row, whole rows (no pieces).
-// grid = windows of 128 / Hq consecutive query tokens of the call.  A window that lies inside one sequence is one
-// group; one that spans a border between sequences (the end of a chunk, decode rows of one token each) runs one
-// group per sequence, one after the other.
+// Windows of 128 / Hq consecutive query tokens of the call; a group is what a window holds of one sequence.  grid = num_seqs + windows: a
+// window's workgroup takes the sequence of its first token, the workgroup of a sequence that begins inside a window what the window holds of it.
+// (One workgroup ran a window's groups one after the other: a launch of few workgroups ended with two groups' times, start and end included:
+// 7 chunks of 22..80 tokens on up to 460 x 16 heads 53 -> 38 us, 3 of 80..191 on 7958 x 64 heads 245 -> 146, 6 e4m3 of 125..1556 x 16 heads 544 -> 451.)
+struct TokenGroup {
+  MlaRow row;  // the group's first token; kv_len: what its last token sees
+  int tokens;
+};
+
+__device__ __forceinline__ bool token_group(const MlaDecodeArgs& a, TokenGroup& g) {
+  const int num_seqs = a.dist ? min(a.num_seqs, scalar_load_i32(a.dist + 2)) : a.num_seqs;
+  const int per = 128 / a.Hq, id = (int)blockIdx.x - a.num_seqs;
+  if (id < 0 && (int)blockIdx.x >= num_seqs) return false;
+  const int total = min(a.num_rows, scalar_load_i32(a.pt.cu_q_lens + num_seqs));
+  int t = ((int)gridDim.x - 1 - (int)blockIdx.x) * per;  // (the longest rows first)
+  if (id >= 0 && t >= total) return false;
+  // (everything here is the same in every lane; said so explicitly, the assembly loop takes scalars)
+  const int seq = __builtin_amdgcn_readfirstlane(id < 0 ? (int)blockIdx.x : owner_of_token(a.pt.cu_q_lens, num_seqs, t));
+  const int q0 = scalar_load_i32(a.pt.cu_q_lens + seq);
+  const int q1 = scalar_load_i32(a.pt.cu_q_lens + seq + 1);
+  if (id < 0) {
+    if ((q0 & (per - 1)) == 0) return false;
+    t = q0;
+  }
+  t = __builtin_amdgcn_readfirstlane(t);
+  const int n = __builtin_amdgcn_readfirstlane(min(min((t & -per) + per, q1), total) - t);
+  if (n <= 0) return false;
+  g.row.seq = seq;
+  g.row.tq = t;
+  g.row.valid = true;
+  g.row.kv_len = __builtin_amdgcn_readfirstlane(scalar_load_i32(a.pt.kv_lens + seq) - (q1 - q0) + (t + n - 1 - q0) + 1);
+  g.tokens = n;
+  return g.row.kv_len > 0 && g.row.kv_len - (n - 1) > 0;
+}
+
 template <bool UNIFORM, bool PIPE, bool FP8>
 __global__ __launch_bounds__(512, 2) void rpa_mla_token_group_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char slot0[kSlotB];
   __shared__ __attribute__((aligned(1024))) char slot1[kSlotB];
   __shared__ __attribute__((aligned(1024))) char slot2[kSlotB];
   __shared__ __attribute__((aligned(1024))) char slot3[kSlotB];
-  const int num_seqs = a.dist ? min(a.num_seqs, scalar_load_i32(a.dist + 2)) : a.num_seqs;
-  const int total = min(a.num_rows, scalar_load_i32(a.pt.cu_q_lens + num_seqs));
-  const int per = 128 / a.Hq;
-  int t = (int)(gridDim.x - 1 - blockIdx.x) * per;
-  if (t >= total) return;
-  const int t_stop = min(t + per, total);
-  int seq = owner_of_token(a.pt.cu_q_lens, num_seqs, t);
-  while (t < t_stop) {
-    // (everything here is the same in every lane; said so explicitly, the assembly loop takes scalars)
-    seq = __builtin_amdgcn_readfirstlane(seq);
-    t = __builtin_amdgcn_readfirstlane(t);
-    const int q0 = scalar_load_i32(a.pt.cu_q_lens + seq);
-    const int q1 = scalar_load_i32(a.pt.cu_q_lens + seq + 1);
-    if (q1 <= t) {  // (a sequence without tokens)
-      ++seq;
-      continue;
-    }
-    const int n = __builtin_amdgcn_readfirstlane(min(t_stop, q1) - t);  // tokens of this sequence in the window
-    MlaRow mr;
-    mr.seq = seq;
-    mr.tq = t;
-    mr.valid = true;
-    // what the group's last token sees
-    mr.kv_len = __builtin_amdgcn_readfirstlane(scalar_load_i32(a.pt.kv_lens + seq) - (q1 - q0) + (t + n - 1 - q0) + 1);
-    const int first_len = mr.kv_len - (n - 1);
-    if (mr.kv_len > 0 && first_len > 0) {
-      const int t_lo = (a.sm.window > 0) ? max(0, first_len - a.sm.window) : 0;
-      MlaDest dest;
-      dest.final_rows = true;
-      dest.base = 0;
-      mla_segment<UNIFORM, false, PIPE, FP8, 1, true>(a, mr, 0, t_lo, t_lo & ~(kTok - 1), mr.kv_len, dest, slot0, slot1, slot2,
-                                                   slot3, n);
-    }
-    t += n;
-    if (t >= q1) ++seq;
-  }
+  TokenGroup g;
+  if (!token_group(a, g)) return;
+  const int first_len = g.row.kv_len - (g.tokens - 1);
+  const int t_lo = (a.sm.window > 0) ? max(0, first_len - a.sm.window) : 0;
+  MlaDest dest;
+  dest.final_rows = true;
+  dest.base = 0;
+  mla_segment<UNIFORM, false, PIPE, FP8, 1, true>(a, g.row, 0, t_lo, t_lo & ~(kTok - 1), g.row.kv_len, dest, slot0, slot1, slot2, slot3, g.tokens);
 }
 
-// ---- token groups on wide workgroups (see mla_segment_wide, TG): bf16 latents, no window.  Same grid and the same
-// walk over a window of 128 / Hq query tokens as rpa_mla_token_group_kernel.
+// ---- token groups on wide workgroups (see mla_segment_wide, TG): bf16 latents, no window.  Same grid.
 template <bool P16>
 __global__ __launch_bounds__(256, 1) void rpa_mla_token_group_wide_kernel(const MlaDecodeArgs a) {
   __shared__ __attribute__((aligned(1024))) char ring[4 * kSlotB];
-  const int num_seqs = a.dist ? min(a.num_seqs, scalar_load_i32(a.dist + 2)) : a.num_seqs;
-  const int total = min(a.num_rows, scalar_load_i32(a.pt.cu_q_lens + num_seqs));
-  const int per = 128 / a.Hq;
-  int t = (int)(gridDim.x - 1 - blockIdx.x) * per;
-  if (t >= total) return;
-  const int t_stop = min(t + per, total);
-  int seq = owner_of_token(a.pt.cu_q_lens, num_seqs, t);
-  while (t < t_stop) {
-    seq = __builtin_amdgcn_readfirstlane(seq);
-    t = __builtin_amdgcn_readfirstlane(t);
-    const int q0 = scalar_load_i32(a.pt.cu_q_lens + seq);
-    const int q1 = scalar_load_i32(a.pt.cu_q_lens + seq + 1);
-    if (q1 <= t) {  // (a sequence without tokens)
-      ++seq;
-      continue;
-    }
-    const int n = __builtin_amdgcn_readfirstlane(min(t_stop, q1) - t);  // tokens of this sequence in the window
-    MlaRow mr;
-    mr.seq = seq;
-    mr.tq = t;
-    mr.valid = true;
-    mr.kv_len = __builtin_amdgcn_readfirstlane(scalar_load_i32(a.pt.kv_lens + seq) - (q1 - q0) + (t + n - 1 - q0) + 1);
-    if (mr.kv_len > 0 && mr.kv_len - (n - 1) > 0) {
-      MlaDest dest;
-      dest.final_rows = true;
-      dest.base = 0;
-      mla_segment_wide<false, true, P16>(a, mr, 0, 0, 0, mr.kv_len, dest, ring, 0, n);
-    }
-    t += n;
-    if (t >= q1) ++seq;
-  }
+  TokenGroup g;
+  if (!token_group(a, g)) return;
+  MlaDest dest;
+  dest.final_rows = true;
+  dest.base = 0;
+  mla_segment_wide<false, true, P16>(a, g.row, 0, 0, 0, g.row.kv_len, dest, ring, 0, g.tokens);
 }
 
 // ---- fixed split plan, wide workgroups: grid = (max_splits * rows, 1, head groups of 128); block = 256 threads
@@ -1579,7 +1557,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   if (const int tg = mla_token_group_mode(a, tune, shape)) {
     const bool pipe_ok = tg >= 2;
     const int per = 128 / a.Hq;
-    const dim3 tg_grid((unsigned)((a.num_rows + per - 1) / per));
+    const dim3 tg_grid((unsigned)(a.num_seqs + (a.num_rows + per - 1) / per));
     if (tg == 3) {
       if (a.pt.page_size == 16) hipLaunchKernelGGL(rpa_mla_token_group_wide_kernel<true>, tg_grid, dim3(256), 0, stream, a);
       else hipLaunchKernelGGL(rpa_mla_token_group_wide_kernel<false>, tg_grid, dim3(256), 0, stream, a);
