@@ -1307,6 +1307,10 @@ struct MlaPlan {
 //                      e4m3 44.3 -> 42.6 (20), 157 -> 165 (144); selections of 12 rows x 64 pages 35.3 -> 33.8 (12), of 32 52.2 -> 57.2 (32)
 //   128 heads          one row of 4000 25.1 -> 15.8 (2), 8 of 300..1500 26.7 -> 22.8 (3.5), 20 33.1 -> 34.1 (8.8), on pages of 16 36.9 -> 34.1, e4m3 39.7 -> 33.1;
 //                      54 of 300..800 37.6 -> 45.8 (14.5); selections of 4 rows x 64 pages 33.3 -> 26.3 (8), 12 of 2048 tokens 39.9 -> 39.4 (12)
+// Rows that stay whole (up to 256 tokens) are short beside what a workgroup costs anyway: there by the workgroups, in rounds of the CUs.  351 drawn
+// batches of rows and chunk tokens, best limit 0.75 .. 0.9 rounds for 32 heads, 0.6 .. 0.75 (pages under a tile 1.25 .. 1.75) for 64, 1.4 .. 1.7 (e4m3 2.0 .. 2.1)
+// for 128: 128 heads, 78 rows of 67 tokens 20.7 -> 27.2 (2.4 rounds), 130 of 75 21.1 -> 44.3 (4.1), 32 heads 162 of 89 13.9 -> 20.1 (1.3).  So too for e4m3 rows of
+// a few hundred tokens on whole tiles: 82 of 777 x 64 heads 42.8 -> 47.4 (1.3 rounds), 192 of 242 x 32 heads 33.1 -> 37.4 (1.5).
 static bool mla_takes_waves(const RpaMlaParams* p, int64_t rows, bool sparse) {
   const int blocks = (p->num_q_heads + 15) / 16;
   if (blocks == 1) return true;
@@ -1314,10 +1318,30 @@ static bool mla_takes_waves(const RpaMlaParams* p, int64_t rows, bool sparse) {
   const int64_t longest = mla_longest(p);
   const int64_t tokens = p->sum_kv_len > 0 ? std::min(p->sum_kv_len, rows * longest) : rows * longest;
   const bool fp8 = p->cache_dtype == RPA_KV_FP8_E4M3, whole = p->page_size % 32 == 0;  // (pages of whole tiles: where the other kernels are at their best)
+  if (longest <= kMlaWholeRow && !sparse) {
+    const int eighths = blocks > 4 ? (fp8 ? 16 : 12) : blocks > 2 ? (whole ? 6 : 10) : (fp8 ? 7 : 6);
+    return 8 * rows * blocks <= (int64_t)eighths * mla_wgs();
+  }
   const int64_t rounds = tokens * blocks / (64 * (int64_t)mla_wgs());
-  if (blocks <= 2) return fp8 || rounds < (sparse ? 20 : whole ? 8 : 24);
-  if (blocks <= 4) return rounds < (fp8 ? whole ? 32 : 200 : sparse || !whole ? 14 : 6);
+  const bool one_round = sparse || rows * blocks <= mla_wgs();
+  if (blocks <= 2) return fp8 ? one_round || !whole || tokens >= 512 * rows : rounds < (sparse ? 20 : whole ? 6 : 24);
+  if (blocks <= 4) return rounds < (fp8 ? whole ? (one_round ? 32 : 0) : 200 : sparse || !whole ? 14 : 6);
   return rounds < (fp8 || sparse || !whole ? 10 : 6);
+}
+
+// Whether a call whose query tokens could share workgroups (rpa_mla.hip, token groups) runs each of them on a wave per tile instead, its rows whole as the
+// groups' are.  A group's tile costs a CU twice what four waves' tiles of one token do and its start and end (147 KB of queries, 128 KB of
+// results) three times as much, but it is 8 / 4 / 2 tokens: groups win as soon as the tokens x blocks of 16 heads are some rounds of the CUs, however
+// long the rows.  997 drawn calls of 16..900 new tokens on up to 8192, best limit in rounds: bf16 2.0 .. 2.25 (of 16-token pages and 16 heads 3), e4m3
+// 2.75 .. 3.25, on pages under a tile, where a group's copies are slow, 2.75 .. 4.5; with the limits here 1.27 x in the geometric mean (the better
+// of the two everywhere would be 1.274), none more than 4 % slower.  us, groups -> these: 16 heads, bf16, 46 tokens 29 -> 14, 163 on 512 47 -> 28, 351 on 2500 125 -> 100
+// (1.4 rounds), 580 on 400 56 -> 65 (2.3); e4m3 220 on 300 47 -> 22, 735 on 2300 180 -> 141 (2.9), 1056 on 320 61 -> 84 (4.1); 32 heads e4m3 on
+// pages of 16 238 on 150 54 -> 32.
+static bool mla_groups_as_waves(const RpaMlaParams* p, int64_t rows) {
+  const int blocks = p->num_q_heads / 16;
+  const bool fp8 = p->cache_dtype == RPA_KV_FP8_E4M3, whole = p->page_size % 32 == 0;
+  const int half_rounds = !fp8 ? 4 : whole ? 5 : blocks == 1 ? 8 : 6;
+  return p->sliding_window <= 0 && 2 * rows * blocks <= (int64_t)half_rounds * mla_wgs();
 }
 
 static bool mla_use_balanced(const RpaMlaParams* p, const MlaPlan& plan, bool token_rows);
@@ -1336,18 +1360,36 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
   auto cut = [&](int64_t groups) {
     int64_t work = p->sum_kv_len > 0 ? p->sum_kv_len * groups : 0;
     if (p->sliding_window > 0) work = 0;
+    // The tokens of a chunk see nearly the same: rows of one length, or pieces of the mean length leave a tail of each row for a second round of
+    // workgroups (137 tokens on 4473 x 16 heads in pieces of 4192 180 us, whole 102; x 32 heads 279 and 175).
+    if (token_rows && 8 * work >= 7 * rows * groups * bound) work = 0;
     return plan_splits(bound, p->sliding_window, rows * groups, work, p->num_splits, mla_min_piece(p), m.wgs, true);
   };
   m.sp = cut((p->num_q_heads + 127) / 128);
   a.max_splits = m.sp.splits;
   m.token_groups = rpa::mla_token_group_mode(a, tune, *m.rule);
   const int blocks = (p->num_q_heads + 15) / 16;
+  if (m.token_groups && waves && tune.mla_waves != 0 && tune.mla_shared_tiles != 0 && (tune.mla_waves > 0 || mla_groups_as_waves(p, rows))) {
+    m.token_groups = 0;
+    m.head_blocks = 1;
+    m.siblings = blocks;
+    m.balanced = false;
+    return m;
+  }
   if (waves && tune.mla_waves != 0 && !m.token_groups && p->soft_cap == 0.f && tune.mla_shared_tiles != 0 && (tune.mla_waves > 0 || mla_takes_waves(p, rows, sparse))) {
+    const MlaPlan other = m;
     m.head_blocks = 1;
     m.siblings = blocks;
     m.wgs = std::max(1, m.wgs / m.siblings);
     if (m.siblings > 1 && m.wgs > 8) m.wgs &= ~7;  // (whole eights of workgroups, see Sibling)
     m.sp = cut(1);
+    // Whole long rows that are a little more than a round of workgroups, where the other kernels have pieces of them: 66 tokens on 4700 x 64 heads,
+    // e4m3 on pages of 16, 170 us and 138 in three pieces, 136 of 1205 and less x 32 heads 47 and 36.
+    if (token_rows && m.sp.splits <= 1 && other.sp.splits > 1 && rows * blocks > mla_wgs()) {
+      m = other;
+      m.balanced = false;
+      return m;
+    }
     // Rows of several lengths: the shortest pieces, counted by the longest row, that are one round of workgroups, if any of up to 512 tokens are.  The
     // balanced plan evens them out, but its start (prefix sums, a search) is 2 us later: 20 rows of 300..1500 x 16 heads 17.9 -> 16.1 us in pieces
     // of 128, 8 of 1000..8000 22.5 -> 20.0 of 256, 100 of 200..1000 e4m3 25.9 -> 22.7 of 512, 20 of 300..1500 x 32 heads 19.2 -> 17.4; beyond, 100 of

@@ -1554,6 +1554,12 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   const ShapeRule& shape = select_shape(mla_shape_key(a), mla_shape_skip(a, tune));
   const bool pipe = shape.kernel == kKernelMlaWide || shape.kernel == kKernelMlaPipe;
   const int ds = shape.kernel == kKernelMlaShared ? shape.share : 1;
+  if (a.head_blocks > 0) {
+    hipError_t ew = launch_mla_waves(a, stream);
+    if (ew != hipSuccess) return ew;
+    if (a.balanced || a.max_splits > 1) launch_mla_combine(a, stream);
+    return hipGetLastError();
+  }
   if (const int tg = mla_token_group_mode(a, tune, shape)) {
     const bool pipe_ok = tg >= 2;
     const int per = 128 / a.Hq;
@@ -1572,12 +1578,6 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
       else if (uniform) hipLaunchKernelGGL((rpa_mla_token_group_kernel<true, false, false>), tg_grid, block, 0, stream, a);
       else hipLaunchKernelGGL((rpa_mla_token_group_kernel<false, false, false>), tg_grid, block, 0, stream, a);
     }
-    return hipGetLastError();
-  }
-  if (a.head_blocks > 0) {
-    hipError_t ew = launch_mla_waves(a, stream);
-    if (ew != hipSuccess) return ew;
-    if (a.balanced || a.max_splits > 1) launch_mla_combine(a, stream);
     return hipGetLastError();
   }
   if (ds != 1) {

@@ -771,6 +771,27 @@ def test_mla_little_work_runs_a_wave_per_tile(pkg, monkeypatch):
     assert not takes(16, 64, 16384)
 
 
+def test_mla_chunks_of_few_tokens_run_a_wave_per_tile(pkg, monkeypatch):
+    """Chunk tokens that could share workgroups: a wave per tile and whole rows up to some rounds of the CUs, groups beyond, with windows and where the
+    switch says so.  Short whole rows of more heads: by the workgroups too."""
+    def plan(Hq, T, longest, S=2, rows=True, **kw):
+        return pkg._lib.describe_mla_plan(_mla_params(pkg, Hq, S=S, T=T, max_kv=longest, sum_kv=T * longest * 3 // 4, **kw), rows)
+
+    for Hq, most, kw in ((16, 512, {}), (32, 256, {}), (64, 128, {}), (16, 640, dict(fp8=True)), (32, 320, dict(fp8=True)), (16, 1024, dict(fp8=True, P=16)),
+                         (32, 384, dict(fp8=True, P=16))):
+        for T, waves in ((most, True), (most + 1, False)):
+            d = plan(Hq, T, 250, **kw)
+            assert ("a wave per tile" in d) == waves and ("token_groups=off" in d) == waves and "pieces_per_row=1 " in d and " workspace=0" in d, (Hq, T, kw, d)
+    assert "token_groups=off" not in plan(16, 300, 4000, window=1000) and "a wave per tile" in plan(16, 300, 4000)
+    p = _mla_params(pkg, 16, S=1, T=137, max_kv=4610, sum_kv=137 * 4542)  # rows of nearly one length: no tail in a round of its own
+    assert "pieces_per_row=1 " in pkg._lib.describe_mla_plan(p, True)
+    for Hq, S, longest, waves, kw in ((128, 48, 100, True, {}), (128, 49, 100, False, {}), (128, 64, 100, True, dict(fp8=True)), (128, 65, 100, False, dict(fp8=True)),
+                                      (64, 48, 200, True, {}), (64, 49, 200, False, {}), (32, 96, 200, True, {}), (32, 97, 200, False, {}), (16, 256, 200, True, {})):
+        assert ("a wave per tile" in plan(Hq, S, longest, S=S, rows=False, **kw)) == waves, (Hq, S, kw)
+    monkeypatch.setenv("RPA_MLA_WAVES", "0")
+    assert "token_groups=wide" in plan(16, 100, 250)
+
+
 def test_mla_pages_that_the_wide_loops_do_not_take(pkg):
     """The wide loops: bytes inside a page in 32 bits, masks in front of a scale that has to be positive."""
     d = pkg._lib.describe_mla_plan
