@@ -70,6 +70,26 @@ struct Head {
   }
 };
 
+// For a full tile inside one page the byte offset of a lane's chunk from the tile's first row never changes: it is computed
+// once, and a copy costs no vector ALU work, only a scalar tile base.  (Worked out in place, 12 registers more and spills.)
+template <int HD>
+struct AsyncOffsets {
+  uint32_t k[Head<HD>::kDims], v[Head<HD>::kDims];
+};
+
+template <int HD>
+__device__ __forceinline__ AsyncOffsets<HD> make_async_offsets(const KvAddr& kv, int wave, int lane) {
+  AsyncOffsets<HD> o;
+  const int cp = lane % Head<HD>::kChunksPerRow;
+#pragma unroll
+  for (int n = 0; n < Head<HD>::kDims; ++n) {
+    const int t = Head<HD>::copy_row(wave, n, lane);
+    o.k[n] = (uint32_t)(t * kv.tok_stride + ((cp ^ Head<HD>::k_swizzle(t)) << 4));
+    o.v[n] = (uint32_t)(t * kv.tok_stride + ((cp ^ Head<HD>::v_swizzle(t)) << 4));
+  }
+  return o;
+}
+
 constexpr float kRowSumLimit = 256.0f;   // a half's row sum above it: the stale maximum is too stale
 constexpr float kSeenFloor = -1.0e30f;   // a row maximum below it: every token so far was masked
 
@@ -110,9 +130,9 @@ struct Shared {   // what the row blocks of a wave share
   ofs_t ofs_k, ofs_v;  // per-lane byte offsets of this wave's K / V copy instructions
 };
 
-template <int HD>
-__device__ __forceinline__ u32x4_t q_frag(const RowBlock<HD>& b, int ks) {
-  return u32x4_t{b.Q[4 * ks], b.Q[4 * ks + 1], b.Q[4 * ks + 2], b.Q[4 * ks + 3]};
+template <int KS, class Q>
+__device__ __forceinline__ u32x4_t q_frag(const Q& q) {
+  return u32x4_t{q[4 * KS], q[4 * KS + 1], q[4 * KS + 2], q[4 * KS + 3]};
 }
 
 // K or V rows of one tile, global -> LDS: HD / 32 instructions per wave.  `lds_wave` is the LDS address
@@ -155,9 +175,16 @@ __device__ __forceinline__ int scalar_page(const TileSrc& s, int tb) {
 // maximum; `off` = slot and half offset
 template <int HD>
 __device__ __forceinline__ f32x16_t qk_half(const RowBlock<HD>& b, const Shared<HD>& sh, int off) {
-  f32x16_t S = mfma32(lds_ld16_at(sh.koff[0] + off), q_frag(b, 0), b.NM);
-#pragma unroll
-  for (int ks = 1; ks < Head<HD>::kSteps; ++ks) S = mfma32(lds_ld16_at(sh.koff[ks] + off), q_frag(b, ks), S);
+  f32x16_t S = mfma32(lds_ld16_at(sh.koff[0] + off), q_frag<0>(b.Q), b.NM);
+  S = mfma32(lds_ld16_at(sh.koff[1] + off), q_frag<1>(b.Q), S);
+  S = mfma32(lds_ld16_at(sh.koff[2] + off), q_frag<2>(b.Q), S);
+  S = mfma32(lds_ld16_at(sh.koff[3] + off), q_frag<3>(b.Q), S);
+  if constexpr (HD == 128) {
+    S = mfma32(lds_ld16_at(sh.koff[4] + off), q_frag<4>(b.Q), S);
+    S = mfma32(lds_ld16_at(sh.koff[5] + off), q_frag<5>(b.Q), S);
+    S = mfma32(lds_ld16_at(sh.koff[6] + off), q_frag<6>(b.Q), S);
+    S = mfma32(lds_ld16_at(sh.koff[7] + off), q_frag<7>(b.Q), S);
+  }
   return S;
 }
 
@@ -461,14 +488,11 @@ __global__ __launch_bounds__(256, (HD == 64 ? 3 : NQ == 1 ? 2 : 1)) void rpa_pre
     for (int ks = 0; ks < HL::kSteps; ++ks) sh.koff[ks] = (int)lds_base + HL::kKSlot + k_row + ((ks * 32) ^ k_swz);
 #pragma unroll
     for (int d = 0; d < HL::kDims; ++d) sh.voff[d] = (int)lds_base + HL::kVSlot + v_row + v_in + ((d * 64) ^ v_swz);
-    // For a full tile inside one page the byte offset of a lane's chunk from the tile's first row never changes: it is
-    // computed once, and a copy costs no vector ALU work, only a scalar tile base.
-    const int cp = lane % HL::kChunksPerRow;
+    const AsyncOffsets<HD> ofs = make_async_offsets<HD>(a.kv, wave, lane);
 #pragma unroll
     for (int n = 0; n < HL::kDims; ++n) {
-      const int t = HL::copy_row(wave, n, lane);
-      sh.ofs_k[n] = (uint32_t)(t * a.kv.tok_stride + ((cp ^ HL::k_swizzle(t)) << 4));
-      sh.ofs_v[n] = (uint32_t)(t * a.kv.tok_stride + ((cp ^ HL::v_swizzle(t)) << 4));
+      sh.ofs_k[n] = ofs.k[n];
+      sh.ofs_v[n] = ofs.v[n];
     }
   }
 
