@@ -934,6 +934,15 @@ static bool takes_fresh_prompts(const RpaParams* p) {
          (int64_t)p->num_tokens * p->num_kv_heads * p->head_dim * esize_of(p->kv_dtype) < (int64_t(1) << 31);
 }
 
+// Whether the launch of small chunks behind prefixes (rpa_prefill_packed_kernel) may take the new tokens from the caller's rows and write them into
+// the cache beside the attention.  Not with decode rows in the call, whose launch in front writes the chunks' tokens too.  A call that says
+// nothing of a prefix may be all new, an address per lane and row: up to 512 tokens.
+static bool chunks_bring_tokens(const RpaParams* p, const void* keys, const void* values) {
+  return !p->distribution && (p->decode_end == 0 || p->mask_mode == RPA_MASK_CUSTOM) && p->head_dim == 128 && q_dim_of(p) == p->head_dim &&
+         (p->max_kv_len > p->max_q_len || p->num_tokens <= 512) && ((reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(values)) & 15) == 0 &&
+         (int64_t)p->num_tokens * p->num_kv_heads * p->head_dim * esize_of(p->kv_dtype) < (int64_t(1) << 31);
+}
+
 // The prefill kernels' view of a call; false when the call has no chunk for them.
 // fresh: a prompt's keys / values, which the kernels read in place of the cache (takes_fresh_prompts).
 static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a, const void* keys = nullptr, const void* values = nullptr) {
@@ -968,11 +977,15 @@ static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a, const void* ke
   a.page_options = rpa::page_options(p->page_size, a.kv.page_stride, 64);
   a.write_blocks = a.write_tokens = 0;
   a.write = {};
-  if (takes_fresh_prompts(p)) {
+  a.tail_is_new = a.mask_words = a.saves_launch = 0;
+  auto write_beside = [&]() {
     a.write = kv_write_args(p, keys, values);
     // two tokens per wave on a small launch, where the attention's own workgroups leave CUs idle
     a.write_tokens = p->num_tokens <= 2048 ? 8 : 32;
     a.write_blocks = (p->num_tokens + a.write_tokens - 1) / a.write_tokens;
+  };
+  if (takes_fresh_prompts(p)) {
+    write_beside();
     a.rows_are_new = 1;
     a.kv.k_base = static_cast<const char*>(keys);
     a.kv.v_base = static_cast<const char*>(values);
@@ -982,7 +995,17 @@ static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a, const void* ke
     a.pt.page_size = 1 << 30;  // (a.page_options stay the cache's)
   }
   // (not where the caller pins the partition: such a call agrees bit for bit with one whose composition is on the device)
+  // (the mask rows of a workgroup in its LDS: two query heads per kv head and more; RPA_MASK_BITS=0 keeps a load per score, on the same kernel)
+  a.mask_words = p->mask_mode == RPA_MASK_CUSTOM && !dyn && a.G >= 2 && p->max_kv_len <= (1 << 24) && p->page_size <= (1 << 24) && p->soft_cap == 0.f &&
+                 a.sm.round_logits == 0 && a.sm.xai_len <= 0.f && a.sm.q_scale <= 0.f;
+  // (of the call's shape alone, whether or not it brings tokens: the workspace is asked for before that is known)
+  a.saves_launch = !a.rows_are_new && chunks_bring_tokens(p, keys, values);
   a.packed = p->num_splits == 0 ? rpa::prefill_packed_pieces(a) : 0;
+  if (!a.packed || rpa::tuning().mask_bits == 0) a.mask_words = 0;
+  if (a.packed && keys && !a.rows_are_new && chunks_bring_tokens(p, keys, values)) {
+    write_beside();
+    a.tail_is_new = 1;
+  }
   return true;
 }
 
@@ -1018,12 +1041,18 @@ static size_t prefill_optional_workspace(const RpaParams* p) {
 
 static int write_new_tokens(const RpaParams* p, const void* keys, const void* values, bool skip_decode_rows, void* stream);
 
+static int prefill_launch(const RpaParams* p, rpa::PrefillArgs& a, const void* keys, const void* values, void* stream);
+
 // keys / values: new tokens that the launch itself puts into the cache (prompts without a prefix, custom masks).
 static int prefill_run(const RpaParams* p, const void* keys, const void* values, void* stream) {
-  int rc = rpa_validate(p);
+  const int rc = rpa_validate(p);
   if (rc != RPA_OK) return rc;
   rpa::PrefillArgs a;
-  if (!prefill_args(p, a, keys, values)) return RPA_OK;
+  return prefill_args(p, a, keys, values) ? prefill_launch(p, a, keys, values, stream) : RPA_OK;
+}
+
+static int prefill_launch(const RpaParams* p, rpa::PrefillArgs& a, const void* keys, const void* values, void* stream) {
+  int rc;
   // 256-wide heads take the flash kernel (two 128-dim halves per row, one workgroup per CU; e4m3
   // caches staged through registers); RPA_PREFILL_ROWS256=1 sends them through the row kernel
   if (p->head_dim == 256 && rpa::tuning().prefill_rows256 != 0)
@@ -1054,11 +1083,12 @@ static int prefill_run(const RpaParams* p, const void* keys, const void* values,
       a.mask_pitch = w.pitch;
     }
   }
-  if (keys && p->mask_mode == RPA_MASK_CUSTOM) {  // by the launch that makes the bits, if there is one
+  if (a.mask_words) a.mask_bits = nullptr;
+  if (keys && p->mask_mode == RPA_MASK_CUSTOM && !a.tail_is_new) {  // by the launch that makes the bits, if there is one
     if (a.mask_bits) a.write = kv_write_args(p, keys, values);
     else if ((rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
   }
-  if (p->mask_mode == RPA_MASK_CUSTOM && !p->cu_mask_lens && !a.mask_bits)
+  if (p->mask_mode == RPA_MASK_CUSTOM && !p->cu_mask_lens && !a.mask_bits && !a.mask_words)
     return fail(RPA_EINVAL_WORKSPACE, "a mask without cu_mask_lens needs rpa_workspace_bytes() of workspace");
   return check_hip(rpa::launch_prefill(a, static_cast<hipStream_t>(stream)), "rpa_prefill");
 }
@@ -1139,6 +1169,14 @@ int rpa_attention_update(const RpaParams* given, const void* keys, const void* v
     return decode_rows(p, with_rows ? keys : nullptr, with_rows ? values : nullptr, true, stream);
   }
   if (keys && (takes_fresh_prompts(p) || mask_as_bits(p))) return prefill_run(p, keys, values, stream);
+  // chunks alone: their plan is made once, and says who writes their tokens
+  rpa::PrefillArgs a;
+  const bool chunks = keys && chunks_bring_tokens(p, keys, values);
+  if (chunks) {
+    if (!prefill_args(p, a, keys, values)) return RPA_OK;
+    if (!a.tail_is_new && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
+    return prefill_launch(p, a, a.tail_is_new ? keys : nullptr, values, stream);
+  }
   const bool fused = keys && decode_rows_write(p);
   if (keys && !fused && (rc = write_new_tokens(p, keys, values, false, stream)) != RPA_OK) return rc;
   if ((rc = decode_rows(p, fused ? keys : nullptr, fused ? values : nullptr, false, stream)) != RPA_OK) return rc;
@@ -1147,6 +1185,11 @@ int rpa_attention_update(const RpaParams* given, const void* keys, const void* v
 }
 
 int rpa_attention(const RpaParams* p, void* stream) { return rpa_attention_update(p, nullptr, nullptr, stream); }
+
+static bool prefill_brings_tokens(const RpaParams* p, const void* keys, const void* values) {
+  rpa::PrefillArgs a;
+  return chunks_bring_tokens(p, keys, values) && prefill_args(p, a, keys, values) && a.tail_is_new;
+}
 
 int rpa_describe_plan(const RpaParams* given, char* buf, size_t len) {
   const OwnParams in(given);
@@ -1210,8 +1253,10 @@ int rpa_describe_plan(const RpaParams* given, char* buf, size_t len) {
   }
   const bool rows = takes_token_rows(p_in), prompts = !rows && takes_fresh_prompts(p_in);
   const bool by_rows = rows ? rows_take_new_tokens(p_in) : !prompts && decode_rows_write(p_in);
-  put("new tokens: written by %s\n", !rows && mask_as_bits(p_in)        ? "the launch that makes bits of the mask"
-                                     : prompts                           ? "workgroups of the prefill launch, which reads the caller's rows"
+  alignas(16) static const char some_rows[16] = {};  // (aligned ones)
+  const bool beside = !rows && (prompts || prefill_brings_tokens(p_in, some_rows, some_rows));
+  put("new tokens: written by %s\n", !rows && !beside && mask_as_bits(p_in) ? "the launch that makes bits of the mask"
+                                     : beside                           ? "workgroups of the prefill launch, which reads the caller's rows"
                                      : !by_rows                         ? "rpa_kv_write_kernel, in front"
                                      : p_in->distribution && !rows      ? "the decode kernels, those of chunks by rpa_kv_write_kernel"
                                                                         : "the decode kernels");

@@ -147,6 +147,11 @@ struct PrefillArgs {
   // rows, which would suit any: the assembly kernel rounds the scaled queries to bf16, and pages that it does not take
   // never had that
   uint32_t page_options;
+  // The new tokens are not in the cache yet: rpa_prefill_packed_kernel reads those behind a sequence's prefix from write.keys /
+  // write.values, and the last write_blocks workgroups put them into the cache.
+  int32_t tail_is_new;
+  int32_t mask_words;  // custom masks: rpa_prefill_packed_kernel reads the caller's words itself, no bits are made
+  int32_t saves_launch;  // (for the choice) rpa_prefill_packed_kernel would spare the launch that writes the new tokens
   int32_t packed;  // rpa_prefill_packed_kernel takes the call, K/V ranges in so many pieces where there is room for them; 0 = not
   struct {
     FastDiv groups, units, hkv, per_kv, nseq;

@@ -1139,7 +1139,7 @@ hipError_t launch_prefill(const PrefillArgs& call, hipStream_t stream) {
   const int nseq = a.seq_end - a.seq_begin;
   if (nseq <= 0 || a.max_q_len <= 0) return hipSuccess;
   if (a.packed) {
-    if (a.sm.mask_mode == 1) {
+    if (a.sm.mask_mode == 1 && !a.mask_words) {
       hipError_t e = launch_mask_bits(a, stream);
       if (e != hipSuccess) return e;
     }

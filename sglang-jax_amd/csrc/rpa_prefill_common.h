@@ -255,6 +255,68 @@ __device__ __forceinline__ void write_new_tokens(const PrefillArgs& a) {
   }
 }
 
+// The same for sequences with a prefix, in front of which nothing wrote (a.tail_is_new).
+__device__ __forceinline__ void write_tail_tokens(const PrefillArgs& a) {
+  const int first = (int)gridDim.x - a.write_blocks;
+  if ((int)blockIdx.x < first || blockIdx.y != 0) return;
+  const KvWriteArgs& wr = a.write;
+  const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+  // A sequence per lane: whose a token is, and where its pages begin, in one trip to memory for up to 63 of them (looked up one after the
+  // other, as before, these workgroups, the last to start, ended the launch: 0.5 us per trip and token).
+  const bool few = wr.num_seqs < 64;
+  int q = 0, kv = 0, first_page = 0;
+  if (few) {
+    const int s = min(lane, wr.num_seqs), own = min(lane, wr.num_seqs - 1);
+    q = wr.pt.cu_q_lens[s];
+    kv = wr.pt.kv_lens[own];
+    first_page = wr.pt.cu_kv_lens ? wr.pt.cu_kv_lens[own] : 0;
+  }
+  const int t0 = ((int)blockIdx.x - first) * a.write_tokens;
+  const int t1 = min(t0 + a.write_tokens, min(wr.num_tokens, few ? __builtin_amdgcn_readlane(q, wr.num_seqs) : scalar_load_i32(wr.pt.cu_q_lens + wr.num_seqs)));
+  const int row_bytes = wr.Hkv * wr.head_bytes;
+  for (int t = t0 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); t < t1; t += waves) {
+    const int64_t from = (int64_t)t * row_bytes;
+    u32x4_t k = {}, v = {};  // the row's first KiB: asked for before its place is known
+    if (lane * 16 < row_bytes) {
+      k = ld16(wr.keys + from + lane * 16);
+      v = ld16(wr.values + from + lane * 16);
+    }
+    int seq, next, kv_len, page0;
+    if (few) {
+      seq = max(__builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < wr.num_seqs && q <= t)) - 1, 0);
+      next = __builtin_amdgcn_readlane(q, seq + 1);
+      kv_len = __builtin_amdgcn_readlane(kv, seq);
+      page0 = __builtin_amdgcn_readlane(first_page, seq);
+    } else {
+      int lo = 0, hi = wr.num_seqs;  // last i with cu_q_lens[i] <= t
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (scalar_load_i32(wr.pt.cu_q_lens + mid) <= t) lo = mid; else hi = mid;
+      }
+      seq = lo;
+      next = scalar_load_i32(wr.pt.cu_q_lens + lo + 1);
+      kv_len = scalar_load_i32(wr.pt.kv_lens + lo);
+      page0 = wr.pt.cu_kv_lens ? scalar_load_i32(wr.pt.cu_kv_lens + lo) : 0;
+    }
+    const int pos = kv_len - (next - t);
+    if (pos < 0) continue;
+    const int slot = __builtin_amdgcn_readfirstlane(pos / wr.pt.page_size);
+    const int page = scalar_load_i32(wr.pt.page_indices + slot + (wr.pt.cu_kv_lens ? (int64_t)__builtin_amdgcn_readfirstlane(page0 / wr.pt.page_size)
+                                                                                   : (int64_t)seq * wr.pt.pages_per_seq));
+    const int64_t off = (int64_t)page * wr.kv.page_stride + (int64_t)(pos - slot * wr.pt.page_size) * wr.kv.tok_stride;
+    for (int b = lane * 16; b < row_bytes; b += 1024) {
+      if (b >= 1024) {
+        k = ld16(wr.keys + from + b);
+        v = ld16(wr.values + from + b);
+      }
+      const int head = b / wr.head_bytes;
+      const int64_t at = off + (int64_t)head * wr.kv.head_stride + (b - head * wr.head_bytes);
+      st16(const_cast<char*>(wr.kv.k_base) + at, k);
+      st16(const_cast<char*>(wr.kv.v_base) + at, v);
+    }
+  }
+}
+
 __device__ __forceinline__ TileSrc make_src(const PrefillArgs& a, const Work& w) {
   TileSrc src;
   src.page_size = a.pt.page_size;

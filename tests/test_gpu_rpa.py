@@ -1663,6 +1663,70 @@ def test_masked_calls_bring_their_tokens(pkg, wl, gpu, monkeypatch, seqs, D, Hkv
     assert torch.equal(bits[0], words[0])
 
 
+@pytest.mark.parametrize("Hq,Hkv,P,fp8,seqs,aligned,window", [
+    (8, 4, 64, False, 3, False, None), (16, 4, 16, True, 70, False, None), (10, 2, 48, False, 5, True, None), (8, 1, 128, True, 4, True, 100),
+    (8, 1, 16, False, 130, False, 40), (16, 2, 64, False, 1, False, None)])
+def test_masks_are_read_as_words(pkg, wl, gpu, monkeypatch, Hq, Hkv, P, fp8, seqs, aligned, window):
+    """Verify steps on the kernel that makes bits of a tile's mask words itself: 2 to 8 query heads per kv head, odd numbers of rows, rows as long as the
+    pages, a window, sequences beyond a wavefront's lanes.  The same bits as with a load per score (RPA_MASK_BITS=0)."""
+    q_lens = [[4, 1, 7, 3, 16][i % 5] for i in range(seqs)]
+    kv_lens = [q + [0, 61, 300, 31, 700][i % 5] for i, q in enumerate(q_lens)]
+    rng = np.random.default_rng(seqs)
+    masks = [(rng.random((ql, -(-kv // P) * P if aligned else kv)) < 0.6).astype(np.int32) for ql, kv in zip(q_lens, kv_lens)]
+    for m, kv in zip(masks, kv_lens):
+        m[:, kv - 1] = 1
+    say(f"masks as words Hq={Hq} Hkv={Hkv} P={P} fp8={fp8} seqs={seqs} aligned={aligned} window={window}")
+    b = wl.make_batch("mask_words", q_lens, kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=96, sliding_window=window,
+                      kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+    g, mask = b.to(gpu), flat_mask(masks).to(gpu)
+    monkeypatch.setenv("RPA_PREFILL_PACKED", "1")
+
+    def run():
+        out, _ = pkg.ragged_paged_attention(g.q, None, None, g.kv_cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, b.distribution.numpy(), mask,
+                                            sm_scale=b.sm_scale, causal=0, sliding_window=window, k_scale=g.k_scale, v_scale=g.v_scale,
+                                            mask_aligned_to_cu_kv=aligned, max_kv_len=max(kv_lens), max_q_len=16)
+        torch.cuda.synchronize()
+        return out[: sum(q_lens)].cpu()
+
+    words = run()
+    monkeypatch.setenv("RPA_MASK_BITS", "0")
+    assert torch.equal(run(), words)
+
+
+@pytest.mark.parametrize("Hkv,P,fp8,q_lens,old,window,splits", [
+    (2, 64, False, [33, 1, 20], [100, 64, 0], None, 0), (2, 16, False, [40, 5], [17, 400], 50, 0), (4, 48, True, [9, 31], [95, 200], None, 0),
+    (1, 128, True, [64, 64], [31, 1], None, 0), (2, 64, False, [20], [3000], None, 3), (2, 16, True, [3] * 70, [5 * i for i in range(70)], None, 0)])
+def test_small_chunks_bring_their_tokens(pkg, wl, gpu, monkeypatch, Hkv, P, fp8, q_lens, old, window, splits):
+    """Chunks behind prefixes whose new tokens are not in the cache: tiles with old and new rows, new ones alone, the last one short; pages of a tile,
+    of half a one and odd ones; a window; pieces; sequences beyond a wavefront's lanes.  The same bits as with the tokens in the cache,
+    and the same cache."""
+    monkeypatch.setenv("RPA_PREFILL_PACKED", "1")
+    monkeypatch.setenv("RPA_PREFILL_SPLITS", str(splits))
+    kv_lens = [q + n for q, n in zip(q_lens, old)]
+    say(f"small chunks, own tokens Hkv={Hkv} P={P} fp8={fp8} q={q_lens[:4]} old={old[:4]} window={window} splits={splits}")
+    b = wl.make_batch("chunk_new", q_lens, kv_lens, num_q_heads=4 * Hkv, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=97, sliding_window=window,
+                      kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+    rows, table = b.kv_cache.view(torch.uint8), b.padded_page_table()
+    holed, at = rows.clone(), [(int(table[s, t // P]), t % P) for s, n in enumerate(kv_lens) for t in range(n - q_lens[s], n)]
+    new = torch.stack([rows[page, slot] for page, slot in at])
+    for page, slot in at:
+        holed[page, slot] = 0x7f  # (no number)
+    g, dt = b.to(gpu), b.kv_cache.dtype
+    keys, vals = (new[:, i::2].contiguous().view(dt).to(gpu) for i in (0, 1))
+
+    def run(cache, k, v):
+        out, _ = pkg.ragged_paged_attention(g.q, k, v, cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, (0, 0, len(q_lens)), None,
+                                            sm_scale=b.sm_scale, sliding_window=window, k_scale=g.k_scale, v_scale=g.v_scale,
+                                            max_kv_len=max(kv_lens), max_q_len=max(q_lens))
+        torch.cuda.synchronize()
+        return out[: sum(q_lens)].cpu()
+
+    want = run(g.kv_cache, None, None)
+    cache = holed.view(dt).to(gpu)
+    assert torch.equal(run(cache, keys, vals), want)
+    assert torch.equal(cache.cpu().view(torch.uint8), rows)
+
+
 @pytest.mark.parametrize("kind", ["soft_cap", "xai_temperature", "custom_mask", "no_mask", "softmax_bf16", "fp8", "fp8_custom_mask"])
 def test_short_chunks_take_the_four_head_tile_in_the_compiled_kernel(pkg, wl, gpu, monkeypatch, kind):
     """The compiled flash kernel (every option the pipelined one does not take) with the same short-chunk tile:
