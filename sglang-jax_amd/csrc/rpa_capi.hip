@@ -1405,10 +1405,18 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
   auto cut = [&](int64_t groups) {
     int64_t work = p->sum_kv_len > 0 ? p->sum_kv_len * groups : 0;
     if (p->sliding_window > 0) work = 0;
-    // The tokens of a chunk see nearly the same: rows of one length, or pieces of the mean length leave a tail of each row for a second round of
-    // workgroups (137 tokens on 4473 x 16 heads in pieces of 4192 180 us, whole 102; x 32 heads 279 and 175).
-    if (token_rows && 8 * work >= 7 * rows * groups * bound) work = 0;
-    return plan_splits(bound, p->sliding_window, rows * groups, work, p->num_splits, mla_min_piece(p), m.wgs, true);
+    // The tokens of a chunk see nearly the same, and pieces of the mean length leave a tail of the longer rows for a second round of workgroups: rows
+    // that are 70 % full are cut by the longest, into what one round holds (137 tokens on 4473 x 16 heads 180 us, whole 102; 167 on 593 x 128 heads
+    // 83 and 45; 34 on 3295 x 64, e4m3, 105 and 66), those of more than 3/5 of a round from 65 % on (174 on 2074 x 32, e4m3, 68 % full, 158 and 72).
+    // Emptier ones stay with the mean: 88 on 3116 x 64 heads, 68 % full, 80 us and in two pieces 97, 129 on 4453 x 128, e4m3, 67 %, 208 and whole 259.
+    const bool full = 20 * work >= (5 * rows * groups > 3 * m.wgs ? 13 : 14) * rows * groups * bound;
+    // Of more rows than a quarter of the CUs the short ones stay whole, a merge costs more than their pieces give (101 of 259 x 128 heads 38 us, whole 29;
+    // 65 of 308 x 64 27 and 18; 92 of 466 x 128 39 and 37; but e4m3 74 of 401 x 128 44, whole 54).
+    const int64_t kept = p->cache_dtype == RPA_KV_FP8_E4M3 && p->num_q_heads > 64 ? 384 : 512;
+    const bool keep = token_rows && 4 * rows > mla_wgs() && bound <= kept && tune.mla_min_chunk >= rpa::Tuning().mla_min_chunk;
+    if (keep || (token_rows && full)) work = 0;
+    const int piece = keep ? (int)kept : mla_min_piece(p);
+    return plan_splits(bound, p->sliding_window, rows * groups, work, p->num_splits, piece, m.wgs, true);
   };
   m.sp = cut((p->num_q_heads + 127) / 128);
   a.max_splits = m.sp.splits;

@@ -792,6 +792,22 @@ def test_mla_chunks_of_few_tokens_run_a_wave_per_tile(pkg, monkeypatch):
     assert "token_groups=wide" in plan(16, 100, 250)
 
 
+def test_mla_chunk_tokens_are_cut_by_the_longest(pkg, monkeypatch):
+    """Tokens of chunks, mostly as long as the longest: pieces that one round of workgroups holds, none of short rows of many; emptier ones by the mean."""
+    def pieces(Hq, T, longest, percent, **kw):
+        d = pkg._lib.describe_mla_plan(_mla_params(pkg, Hq, S=2, T=T, max_kv=longest, sum_kv=-(-T * longest * percent // 100), **kw), True)
+        return int(d.split("pieces_per_row=")[1].split()[0])
+
+    for T in (40, 100, 127, 128, 129, 200):
+        assert pieces(128, T, 4000, 70) == max(1, 256 // T), T
+    assert pieces(128, 160, 4000, 65) == 1 and pieces(128, 160, 4000, 64) > 1 and pieces(128, 90, 4000, 69) > 2
+    for longest, f8, cut in ((512, False, False), (513, False, True), (384, True, False), (385, True, True)):
+        assert (pieces(128, 65, longest, 50, fp8=f8) > 1) == cut, (longest, f8)
+    assert pieces(64, 65, 512, 50, fp8=True) == 1 and pieces(128, 64, 512, 70) > 1
+    monkeypatch.setenv("RPA_MLA_MIN_CHUNK", "32")  # shorter pieces asked for
+    assert pieces(128, 65, 512, 70) > 1
+
+
 def test_mla_pages_that_the_wide_loops_do_not_take(pkg):
     """The wide loops: bytes inside a page in 32 bits, masks in front of a scale that has to be positive."""
     d = pkg._lib.describe_mla_plan
