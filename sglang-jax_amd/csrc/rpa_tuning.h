@@ -20,7 +20,7 @@ struct Tuning {
   int decode_row_kb = -1;           // RPA_DECODE_ROW_KB          -1: 128; KiB of a row's kv head up to which one workgroup takes it
   int decode_row_pieces = -1;       // RPA_DECODE_ROW_PIECES      -1: by the launch; n: workgroups that share a row's kv head
   // ---- prefill (rpa_prefill.hip, rpa_prefill_pipe.hip)
-  int mask_bits = 1;                // RPA_MASK_BITS              0: kernels read the caller's i32 mask words
+  int mask_bits = 1;                // RPA_MASK_BITS              0: a load per score of the caller's i32 mask words
   int prefill_rows256 = 0;          // RPA_PREFILL_ROWS256        1: 256-wide chunks through the row kernel
   int prefill_staged = 0;           // RPA_PREFILL_STAGED         1: bf16 caches through the register-staged kernel
   int prefill_pipe = 1;             // RPA_PREFILL_PIPE           0: no assembly loop, compiled flash kernel
