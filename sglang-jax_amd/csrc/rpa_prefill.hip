@@ -90,6 +90,7 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_async_kernel(const Prefill
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
     a.seq_end = min(a.seq_end, scalar_load_i32(a.dist + 2));
+    if (a.seq_begin >= a.seq_end) return;
   }
   // Four separate arrays (not one indexed array): the compiler can then prove that the
   // asynchronous copy into one ring slot does not alias the LDS reads of the other slot and
@@ -371,6 +372,7 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_async_kernel_wide(const Pr
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
     a.seq_end = min(a.seq_end, scalar_load_i32(a.dist + 2));
+    if (a.seq_begin >= a.seq_end) return;
   }
   __shared__ __attribute__((aligned(65536))) char ring[4 * kWTileB];  // K, K, V, V
   __shared__ __attribute__((aligned(1024))) char stage[FP8 ? kWTileB : 16];  // K bytes, V bytes
@@ -828,6 +830,7 @@ __global__ __launch_bounds__(256, 2) void rpa_prefill_staged_kernel(const Prefil
   if (a.dist) {
     a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
     a.seq_end = min(a.seq_end, scalar_load_i32(a.dist + 2));
+    if (a.seq_begin >= a.seq_end) return;
   }
   __shared__ __attribute__((aligned(16))) char lds_k_buf[2][kBN * kKPitch];
   __shared__ __attribute__((aligned(16))) char lds_v_buf[2][128 * kVPitch];
