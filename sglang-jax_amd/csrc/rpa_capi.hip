@@ -1371,7 +1371,8 @@ static bool mla_takes_waves(const RpaMlaParams* p, int64_t rows, bool sparse) {
   const bool one_round = sparse || rows * blocks <= mla_wgs();
   if (blocks <= 2) return fp8 ? one_round || !whole || tokens >= 512 * rows : rounds < (sparse ? 20 : whole ? 6 : 24);
   if (blocks <= 4) return rounds < (fp8 ? whole ? (one_round ? 32 : 0) : 200 : sparse || !whole ? 14 : 6);
-  return rounds < (fp8 || sparse || !whole ? 10 : 6);
+  // (selections, one workgroup more than the CUs: 33 rows of 512 tokens 34.5 -> 42)
+  return rounds < (fp8 || sparse || !whole ? 10 : 6) && (!sparse || rows * blocks <= mla_wgs());
 }
 
 // Whether a call whose query tokens could share workgroups (rpa_mla.hip, token groups) runs each of them on a wave per tile instead, its rows whole as the
@@ -1457,6 +1458,13 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
         m.balanced = false;
         return m;
       }
+      // Longer pieces of bf16 rows on pages of whole tiles: shared tiles have less of a start than the waves' 16-token tiles and keep it up to 15 rounds
+      // of 64 tokens per CU (113 drawn batches x 16 heads, shared -> waves: 12 of 5800..23203 37.4 -> 40.0, 41 of 472..7560 40.6 -> 43.6, 13.2 rounds 48.3 ->
+      // 50.6; 16.3 rounds 60.3 -> 59.3, 17.2 and more 1.11 .. 1.14 x; pages of 16 1.03 .. 1.14 x, e4m3 1.11 .. 1.64 x throughout; selections level).
+      const int64_t tokens = p->sum_kv_len > 0 ? std::min(p->sum_kv_len, rows * longest) : rows * longest;
+      if (blocks == 1 && !sparse && !token_rows && tune.mla_waves < 0 && p->cache_dtype == RPA_KV_BF16 && p->page_size % 32 == 0 &&
+          tokens < 15 * 64 * (int64_t)mla_wgs())
+        m = other;
     }
   }
   m.balanced = !sparse && mla_use_balanced(p, m, token_rows);

@@ -788,6 +788,9 @@ def test_mla_chunks_of_few_tokens_run_a_wave_per_tile(pkg, monkeypatch):
     for Hq, S, longest, waves, kw in ((128, 48, 100, True, {}), (128, 49, 100, False, {}), (128, 64, 100, True, dict(fp8=True)), (128, 65, 100, False, dict(fp8=True)),
                                       (64, 48, 200, True, {}), (64, 49, 200, False, {}), (32, 96, 200, True, {}), (32, 97, 200, False, {}), (16, 256, 200, True, {})):
         assert ("a wave per tile" in plan(Hq, S, longest, S=S, rows=False, **kw)) == waves, (Hq, S, kw)
+    for tokens, kw, waves in ((245759, {}, False), (245760, {}, True), (200000, dict(fp8=True), True), (200000, dict(P=16), True)):  # long ragged rows
+        p = _mla_params(pkg, 16, S=20, T=20, max_kv=16000, sum_kv=tokens, **kw)
+        assert ("a wave per tile" in pkg._lib.describe_mla_plan(p, False)) == waves, (tokens, kw)
     monkeypatch.setenv("RPA_MLA_WAVES", "0")
     assert "token_groups=wide" in plan(16, 100, 250)
 
