@@ -64,7 +64,7 @@ DECODE_KERNEL = {
     "c4swa": "rpa_decode_splitkv_kernel",
     "c5": "rpa_mla_balanced_wide_kernel",
     "c5fp8": "rpa_mla_balanced_kernel",
-    "c5tp8": "rpa_mla_balanced_kernel (shared tiles)",
+    "c5tp8": "rpa_mla_waves_balanced_kernel (a wave per tile)",
 }
 
 PREFILL_KERNEL = "rpa_prefill_pipe_kernel"
