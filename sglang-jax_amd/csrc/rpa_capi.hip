@@ -1359,7 +1359,6 @@ struct MlaPlan {
 static bool mla_takes_waves(const RpaMlaParams* p, int64_t rows, bool sparse) {
   const int blocks = (p->num_q_heads + 15) / 16;
   if (blocks == 1) return true;
-  if (blocks > 8) return false;
   const int64_t longest = mla_longest(p);
   const int64_t tokens = p->sum_kv_len > 0 ? std::min(p->sum_kv_len, rows * longest) : rows * longest;
   const bool fp8 = p->cache_dtype == RPA_KV_FP8_E4M3, whole = p->page_size % 32 == 0;  // (pages of whole tiles: where the other kernels are at their best)
@@ -1430,7 +1429,9 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
     m.balanced = false;
     return m;
   }
-  if (waves && tune.mla_waves != 0 && !m.token_groups && p->soft_cap == 0.f && tune.mla_shared_tiles != 0 && (tune.mla_waves > 0 || mla_takes_waves(p, rows, sparse))) {
+  // (at most 128 heads, whatever the switch says: a share's slots in the workspace hold so many, and its line has one unit per row)
+  if (waves && blocks <= 8 && tune.mla_waves != 0 && !m.token_groups && p->soft_cap == 0.f && tune.mla_shared_tiles != 0 &&
+      (tune.mla_waves > 0 || mla_takes_waves(p, rows, sparse))) {
     const MlaPlan other = m;
     m.head_blocks = 1;
     m.siblings = blocks;

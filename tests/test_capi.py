@@ -771,6 +771,17 @@ def test_mla_little_work_runs_a_wave_per_tile(pkg, monkeypatch):
     assert not takes(16, 64, 16384)
 
 
+@pytest.mark.parametrize("Hq", [112, 128, 129, 144, 160, 256])
+def test_mla_more_than_128_heads_never_run_a_wave_per_tile(pkg, monkeypatch, Hq):
+    """A share of the balanced plan has room for partial rows of 128 heads: the switch sends no more than that to the kernel of a wave per tile, on
+    either plan, for rows of sequences and of tokens."""
+    monkeypatch.setenv("RPA_MLA_WAVES", "1")
+    for S, longest, fp8 in ((20, 16000, False), (1, 100, False), (300, 3000, True)):
+        for token_rows in (False, True):
+            d = pkg._lib.describe_mla_plan(_mla_params(pkg, Hq, S=S, T=S, max_kv=longest, sum_kv=S * longest * 3 // 4, fp8=fp8), token_rows)
+            assert ("a wave per tile" in d) == (Hq <= 128), d
+
+
 def test_mla_chunks_of_few_tokens_run_a_wave_per_tile(pkg, monkeypatch):
     """Chunk tokens that could share workgroups: a wave per tile and whole rows up to some rounds of the CUs, groups beyond, with windows and where the
     switch says so.  Short whole rows of more heads: by the workgroups too."""
