@@ -217,7 +217,8 @@ typedef struct RpaMlaParams {
   float sm_scale;
   float soft_cap;             /* 0 => off */
   float mask_value;           /* 0 => default */
-  int64_t sum_kv_len;         /* sum of kv_lens (host-side, balances the split plan); 0 => unknown */
+  int64_t sum_kv_len;         /* what the call's rows see, added up (host-side, the plans go by it); 0 => unknown: the kv_lens of
+                                 decode rows, of chunks what every query token sees */
   /* Scalar scales of kernels/mla/v2/kernel.py:1354-1356 (used at :372-375, :408-409; oracle
    * kernels/mla/v1/ref.py:223-226, 241-242): logits are multiplied by k_scale and q_scale next to
    * sm_scale, the output by v_scale.  0 => off. */

@@ -21,6 +21,19 @@ from ._lib import RpaMlaParams
 from .ragged_paged_attention import DEFAULT_MASK_VALUE, _host_decode_sum, _host_max, _i32, _require_gpu, _workspace
 
 
+def _host_visible_sum(kv_lens, cu_q_lens, num_seqs, decode_only):
+    """What the rows of a call see, added up, from HOST copies only (0 when one is missing).  A decode row sees its sequence, token j
+    of a chunk's q new ones kv_len - q + j + 1."""
+    if decode_only:
+        return _host_decode_sum(kv_lens, num_seqs)
+    for t in (kv_lens, cu_q_lens):
+        if not isinstance(t, np.ndarray) and not (isinstance(t, torch.Tensor) and t.device.type == "cpu"):
+            return 0
+    kv = np.asarray(kv_lens[:num_seqs]).astype(np.int64)
+    q = np.diff(np.asarray(cu_q_lens[: num_seqs + 1]).astype(np.int64))
+    return int((q * kv - q * (q - 1) // 2).sum())
+
+
 def mla_ragged_paged_attention(
     ql_nope: torch.Tensor,  # [max_num_tokens, num_q_heads, lkv_dim]
     q_pe: torch.Tensor,  # [max_num_tokens, num_q_heads, r_dim]
@@ -139,7 +152,10 @@ def mla_ragged_paged_attention(
     p.pages_per_seq = (page_d.numel() // max(kv_lens_d.shape[0], 1)) if cu_kv_d is None else 0
     p.max_kv_len = int(max_kv_len) if max_kv_len is not None else _host_max(kv_lens)
     p.num_splits = int(num_splits)
-    p.sum_kv_len = int(sum_kv_len) if sum_kv_len is not None else _host_decode_sum(kv_lens, k)
+    if sum_kv_len is not None:
+        p.sum_kv_len = int(sum_kv_len)
+    else:
+        p.sum_kv_len = 0 if static_shapes else _host_visible_sum(kv_lens, cu_q_lens, k, decode_only)
     p.sliding_window = int(sliding_window) if sliding_window else 0
     p.sm_scale = float(sm_scale)
     p.soft_cap = float(soft_cap) if soft_cap else 0.0

@@ -10,6 +10,7 @@ import sys
 
 import numpy as np
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -804,6 +805,23 @@ def test_mla_chunks_of_few_tokens_run_a_wave_per_tile(pkg, monkeypatch):
         assert ("a wave per tile" in pkg._lib.describe_mla_plan(p, False)) == waves, (tokens, kw)
     monkeypatch.setenv("RPA_MLA_WAVES", "0")
     assert "token_groups=wide" in plan(16, 100, 250)
+
+
+def test_mla_chunk_tokens_are_counted_as_rows(pkg):
+    """Lengths on the host and no sum from the caller: the operator adds up what every query token sees, which is what the plans go by.  With the
+    sequences' lengths in its place 2048 tokens on 4096 would run eight sibling workgroups each, 300 on 1000 in sixteen pieces."""
+    total = pkg.mla._host_visible_sum
+    rng = np.random.default_rng(3)
+    q, old = rng.integers(0, 40, 9), rng.integers(0, 300, 9)
+    cu, kv = np.concatenate([[0], np.cumsum(q)]).astype(np.int32), (q + old).astype(np.int32)
+    want = sum(int(o) + j + 1 for n, o in zip(q[:7], old) for j in range(n))
+    assert total(kv, cu, 7, False) == want and total(torch.from_numpy(kv), torch.from_numpy(cu), 7, False) == want
+    assert total(kv, cu, 7, True) == int(kv[:7].sum()) and total(kv, None, 7, False) == 0 and total(None, cu, 7, False) == 0
+    for n, each, kv_len, fp8, P in ((4, 512, 4608, True, 64), (4, 512, 4608, False, 16), (1, 300, 1300, False, 64)):
+        kv, cu = np.full(n, kv_len, np.int32), np.arange(n + 1, dtype=np.int32) * each
+        p = _mla_params(pkg, 128, P=P, fp8=fp8, S=n, T=n * each, max_kv=kv_len, sum_kv=total(kv, cu, n, False))
+        d = pkg._lib.describe_mla_plan(p, True)
+        assert "a wave per tile" not in d and "pieces_per_row=1 " in d and " workspace=0" in d, d
 
 
 def test_mla_chunk_tokens_are_cut_by_the_longest(pkg, monkeypatch):
