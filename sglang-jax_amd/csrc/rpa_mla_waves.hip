@@ -287,7 +287,7 @@ __device__ __forceinline__ void mla_segment_waves(const MlaDecodeArgs& a, const 
 #pragma unroll
       for (int i = 1; i < 4 * kHalves; ++i) mx = fmaxf(mx, x[i]);
       mx = swap_max(swap16_max(mx));
-      if (k == 0) m = mx;
+      if (k == 0) m = fmaxf(mx, -3.0e38f);  // (scores that overflow to -infinity count nothing, also where they are all of a tile)
       raise = mx;
       if (__builtin_amdgcn_ballot_w64(mx > m + 60.0f) != 0) break;
       u32x4_t pB = {0u, 0u, 0u, 0u}, pR = {0u, 0u, 0u, 0u};  // rounded, and what rounding left of them
@@ -365,7 +365,7 @@ __device__ __forceinline__ void mla_segment_waves(const MlaDecodeArgs& a, const 
     f[w] = fast_exp2(refs[w][0][c] - top);
     sum += refs[w][1][c] * f[w];
   }
-  const float inv = (dest.final_rows ? a.out_scale : 1.0f) / sum;
+  const float inv = dest.final_rows ? a.out_scale / sum : sum == 0.f ? 0.f : 1.0f / sum;  // (a piece of nothing but -infinity weighs nothing)
   __syncthreads();
   f32x4_t own[8];
 #pragma unroll
@@ -385,8 +385,8 @@ __device__ __forceinline__ void mla_segment_waves(const MlaDecodeArgs& a, const 
 #pragma unroll
     for (int j = 0; j < 8; j += 2) st16(row + (wave * 8 + j) * 16 + g * 8, out[j / 2]);
     if (!dest.final_rows && wave == 0 && g == 0) {
-      a.ws_ml[(dest.base + head) * 2 + 0] = top + __builtin_amdgcn_logf(sum);
-      a.ws_ml[(dest.base + head) * 2 + 1] = 1.0f;
+      a.ws_ml[(dest.base + head) * 2 + 0] = sum == 0.f ? top : top + __builtin_amdgcn_logf(sum);
+      a.ws_ml[(dest.base + head) * 2 + 1] = sum == 0.f ? 0.f : 1.0f;
     }
   }
   __syncthreads();  // (the next piece's copies land where this one's rows met)
