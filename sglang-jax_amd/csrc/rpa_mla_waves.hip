@@ -396,20 +396,27 @@ __device__ __forceinline__ void mla_segment_waves(const MlaDecodeArgs& a, const 
 struct NewToken {
   int begin, row;
 };
+// Copies into LDS move aligned chunks of 16 bytes: rows of the caller's that begin elsewhere go through registers into the cache, and come from there.
+__device__ __forceinline__ bool in_chunks(const char* kv_c, const char* k_pe) {
+  return ((reinterpret_cast<uint64_t>(kv_c) | reinterpret_cast<uint64_t>(k_pe)) & 15) == 0;
+}
 template <bool FP8>
-__device__ __forceinline__ NewToken new_token(const MlaDecodeArgs& a, const MlaRow& mr, bool& put) {
+__device__ __forceinline__ NewToken new_token(const MlaDecodeArgs& a, const MlaRow& mr, int t_end, bool& put) {
   if (!a.new_kv_c) {
     put = false;
     return {mr.kv_len, 0};
   }
   const int q0 = scalar_load_i32(a.pt.cu_q_lens + mr.seq), count = scalar_load_i32(a.pt.cu_q_lens + mr.seq + 1) - q0;
-  if (count != 1) {  // (not a decode row: every token in front of everything)
+  const bool direct = in_chunks(a.new_kv_c, a.new_k_pe);
+  if (!direct) put = t_end > mr.kv_len - count;  // (by every workgroup that reads a new token, the same bytes: each follows its own stores)
+  if (!direct || count != 1) {  // (not a decode row: every token in front of everything)
     if (put) {
       put_new_row<FP8>(a, mr.seq, mr.kv_len);
+      if (!direct) wait_all_loads();  // (and stores)
       put = false;
     }
   }
-  return {mr.kv_len - count, q0};
+  return {direct ? mr.kv_len - count : mr.kv_len, q0};
 }
 
 // ---- fixed plan: workgroups (piece, sibling), pieces of a row one after the other.  SPARSE: the rows' page tables are written here first.
@@ -434,7 +441,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void rpa_mla_waves_kernel(const Mla
     // (behind the table's barrier: page ids are read as what nobody writes, and could be asked for in front of it)
     asm volatile("" : "+s"(b.pt.page_indices)::"memory");
     const bool whole_pages = a.sparse.k_pages_max > 0;
-    const int new_begin = a.sparse.new_kv_c ? p.kv_len - 1 : p.kv_len;
+    const int new_begin = a.sparse.new_kv_c && in_chunks(a.sparse.new_kv_c, a.sparse.new_k_pe) ? p.kv_len - 1 : p.kv_len;
     mla_segment_waves<FP8, NT>(b, mr, head_base, p.t_lo, p.t_begin, p.t_end, dest, ring, a.sparse.new_kv_c, a.sparse.new_k_pe, new_begin, row_id, false,
                                whole_pages, p.page_ids);
     return;
@@ -451,7 +458,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void rpa_mla_waves_kernel(const Mla
   const int t_end = (split == a.max_splits - 1) ? kv_len : min(kv_len, t_begin + a.chunk);
   dest.base = ((int64_t)row_id * a.max_splits + split) * a.Hq;
   bool put = sib.unit == 0 && t_end == kv_len;
-  const NewToken nt = new_token<FP8>(a, mr, put);
+  const NewToken nt = new_token<FP8>(a, mr, t_end, put);
   mla_segment_waves<FP8, NT>(a, mr, head_base, t_lo, t_begin, t_end, dest, ring, a.new_kv_c, a.new_k_pe, nt.begin, nt.row, put, false, 0);
 }
 
@@ -463,7 +470,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void rpa_mla_waves_balanced_kernel(
   const int unit = sibling(a).unit;
   mla_balanced_body<FP8, false>(a, [&](const MlaRow& mr, int, int t_lo, int t_begin, int t_end, const MlaDest& dest, int) __attribute__((always_inline)) {
     bool put = unit == 0 && t_end == mr.kv_len;
-    const NewToken nt = new_token<FP8>(a, mr, put);
+    const NewToken nt = new_token<FP8>(a, mr, t_end, put);
     mla_segment_waves<FP8, NT>(a, mr, unit * 16, t_lo, t_begin, t_end, dest, ring, a.new_kv_c, a.new_k_pe, nt.begin, nt.row, put, false, 0);
   });
 }

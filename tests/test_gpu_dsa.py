@@ -242,3 +242,29 @@ def test_a_window_over_a_selection(pkg, wl, gpu, level, P, Hq, dtype, window):
     assert run(ctypes.byref(p), ctypes.byref(s), None, None, torch.cuda.current_stream().cuda_stream) == 0
     torch.cuda.synchronize()
     assert_parity(out.cpu().float(), want.float(), **TOL)
+
+
+@pytest.mark.parametrize("level,P,Hq,dtype", [("page", 64, 16, "bf16"), ("page", 24, 40, "e4m3"), ("token", 64, 16, "bf16"), ("token", 16, 128, "e4m3")])
+def test_selections_with_new_rows_anywhere_in_memory(pkg, wl, gpu, monkeypatch, level, P, Hq, dtype):
+    """New rows that begin 8 bytes behind a multiple of 16 go through registers on a wave per tile as well: the same output and cache, bit for bit."""
+    monkeypatch.setenv("RPA_MLA_WAVES", "1")
+    kv_lens, k = [1, 63, 64, 65, 700, 3001], 512
+    b = batch(wl, kv_lens, P, 86, Hq=Hq)
+    S, pps, dt = len(kv_lens), -(-max(kv_lens) // P), torch.float8_e4m3fn if dtype == "e4m3" else torch.bfloat16
+    g, stored, topk = b.to(gpu), b.cache_kv.to(dt).to(gpu), torch.from_numpy(draw_topk(kv_lens, k, 10)).to(gpu)
+    n, rows, got = 16 // dt.itemsize // 2, torch.randn(S, 576, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).to(dt).to(gpu), []
+    for off in (0, n):
+        parts = []
+        for part in (rows[:, :512], rows[:, 512:]):
+            room = torch.zeros(part.numel() + n, dtype=dt, device=gpu)
+            room[off:off + part.numel()] = part.reshape(-1)
+            parts.append(room[off:off + part.numel()].view(part.shape))
+            assert parts[-1].data_ptr() % 16 == (8 if off else 0)
+        cache = stored.clone()
+        say(f"dsa {level} new rows at +{off} P={P} Hq={Hq} {dtype}")
+        args = (g.ql_nope, g.q_pe, *parts, cache, g.kv_lens, topk, g.page_indices, g.cu_q_lens, g.cu_kv_lens, (S, S, S))
+        common = dict(sm_scale=b.sm_scale, page_size=P, pages_per_seq=pps, kv_lora_rank=512)
+        out = pkg.sparse_mla_via_dense(*args, **common) if level == "token" else pkg.sparse_mla_page_level(*args, k_pages_max=40, **common)[0]
+        torch.cuda.synchronize()
+        got.append((out, cache.view(torch.uint8)))
+    assert torch.isfinite(got[0][0]).all() and torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
