@@ -490,7 +490,10 @@ void launch(const MlaDecodeArgs& a, hipStream_t stream) {
 }  // namespace
 
 hipError_t launch_mla_waves(const MlaDecodeArgs& a, hipStream_t stream) {
-  const bool alone = a.siblings <= 1;
+  // Rows of sequences and selections of 16 heads are one workgroup's and pass through the caches once (NT of mla_segment_waves).  A chunk's tokens all read
+  // the same prefix, out of L2: 116 calls of 40..1000 tokens on up to 8000 x 16 heads, non-temporal -> plain, 1.026 x in the geometric mean, 4 chunks of
+  // 86..326 on 441..882 98.7 -> 90.3 us, e4m3 4 of 63..292 on 463 83.6 -> 78.7; what loses most are prefixes larger than an L2, 142 on 6400 137 -> 140.
+  const bool alone = a.siblings <= 1 && !a.rows_are_tokens;
   if (a.fp8) alone ? launch<true, true>(a, stream) : launch<true, false>(a, stream);
   else alone ? launch<false, true>(a, stream) : launch<false, false>(a, stream);
   return hipGetLastError();
