@@ -1356,17 +1356,23 @@ struct MlaPlan {
 // batches of rows and chunk tokens, best limit 0.75 .. 0.9 rounds for 32 heads, 0.6 .. 0.75 (pages under a tile 1.25 .. 1.75) for 64, 1.4 .. 1.7 (e4m3 2.0 .. 2.1)
 // for 128: 128 heads, 78 rows of 67 tokens 20.7 -> 27.2 (2.4 rounds), 130 of 75 21.1 -> 44.3 (4.1), 32 heads 162 of 89 13.9 -> 20.1 (1.3).  So too for e4m3 rows of
 // a few hundred tokens on whole tiles: 82 of 777 x 64 heads 42.8 -> 47.4 (1.3 rounds), 192 of 242 x 32 heads 33.1 -> 37.4 (1.5).
+//
+// 16 heads take it always, but for bf16 selections of whole pages of whole tiles under 4 rounds: there the three tiles that a workgroup has asked for ahead
+// are 111 KB, the eight of four waves arrive behind one another's waits.  200 drawn selections, inputs that change from call to call, shared tiles ->
+// these: 9 rows of 4096 tokens 21.1 -> 23.5 us (2.2 rounds), 11 of 2048..2688 20.4 -> 22.4, 13 of 4096 23.9 -> 25.9 (3.2); around 4 rounds either, 16 of 4096 25.8 ->
+// 27.3, with fewer pages in use 23.1 -> 22.5; 24 of 4096 32.9 -> 32.9 (6), 32 40.7 -> 37.9 (8), 64 of 8192 105 -> 92.7 (32).  Throughout: e4m3 0.75 .. 1.03 x the
+// time, single tokens 0.86 .. 1.01, pages of 16 0.86 .. 1.03.
 static bool mla_takes_waves(const RpaMlaParams* p, int64_t rows, bool sparse) {
   const int blocks = (p->num_q_heads + 15) / 16;
-  if (blocks == 1) return true;
   const int64_t longest = mla_longest(p);
   const int64_t tokens = p->sum_kv_len > 0 ? std::min(p->sum_kv_len, rows * longest) : rows * longest;
+  const int64_t rounds = tokens * blocks / (64 * (int64_t)mla_wgs());
   const bool fp8 = p->cache_dtype == RPA_KV_FP8_E4M3, whole = p->page_size % 32 == 0;  // (pages of whole tiles: where the other kernels are at their best)
+  if (blocks == 1) return !sparse || fp8 || !whole || rounds >= 4;
   if (longest <= kMlaWholeRow && !sparse) {
     const int eighths = blocks > 4 ? (fp8 ? 16 : 12) : blocks > 2 ? (whole ? 6 : 10) : (fp8 ? 7 : 6);
     return 8 * rows * blocks <= (int64_t)eighths * mla_wgs();
   }
-  const int64_t rounds = tokens * blocks / (64 * (int64_t)mla_wgs());
   const bool one_round = sparse || rows * blocks <= mla_wgs();
   if (blocks <= 2) return fp8 ? one_round || !whole || tokens >= 512 * rows : rounds < (sparse ? 20 : whole ? 6 : 24);
   if (blocks <= 4) return rounds < (fp8 ? whole ? (one_round ? 32 : 0) : 200 : sparse || !whole ? 14 : 6);
@@ -1461,7 +1467,7 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
       }
       // Longer pieces of bf16 rows on pages of whole tiles: shared tiles have less of a start than the waves' 16-token tiles and keep it up to 15 rounds
       // of 64 tokens per CU (113 drawn batches x 16 heads, shared -> waves: 12 of 5800..23203 37.4 -> 40.0, 41 of 472..7560 40.6 -> 43.6, 13.2 rounds 48.3 ->
-      // 50.6; 16.3 rounds 60.3 -> 59.3, 17.2 and more 1.11 .. 1.14 x; pages of 16 1.03 .. 1.14 x, e4m3 1.11 .. 1.64 x throughout; selections level).
+      // 50.6; 16.3 rounds 60.3 -> 59.3, 17.2 and more 1.11 .. 1.14 x; pages of 16 1.03 .. 1.14 x, e4m3 1.11 .. 1.64 x throughout; selections: see mla_takes_waves).
       const int64_t tokens = p->sum_kv_len > 0 ? std::min(p->sum_kv_len, rows * longest) : rows * longest;
       if (blocks == 1 && !sparse && !token_rows && tune.mla_waves < 0 && p->cache_dtype == RPA_KV_BF16 && p->page_size % 32 == 0 &&
           tokens < 15 * 64 * (int64_t)mla_wgs())

@@ -268,3 +268,24 @@ def test_selections_with_new_rows_anywhere_in_memory(pkg, wl, gpu, monkeypatch, 
         torch.cuda.synchronize()
         got.append((out, cache.view(torch.uint8)))
     assert torch.isfinite(got[0][0]).all() and torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("level,P,dtype,S,waves", [("page", 64, "bf16", 15, "0"), ("page", 64, "bf16", 16, "1"), ("page", 64, "e4m3", 3, "1"), ("page", 16, "bf16", 3, "1"),
+                                                   ("token", 64, "bf16", 3, "1")])
+def test_few_selections_of_whole_pages_share_tiles(pkg, wl, gpu, monkeypatch, level, P, dtype, S, waves):
+    """16 heads, bf16, pages of whole tiles: under four rounds of 64 tokens per CU the waves of a workgroup share its tiles, from there on, and for every
+    other selection, each has its own.  Which one ran shows in the bits, and both are near the oracle."""
+    kv_lens, k = [4100] + [100 + 37 * i for i in range(S - 1)], 256
+    b = batch(wl, kv_lens, P, 87)
+    pps, dt = -(-max(kv_lens) // P), torch.float8_e4m3fn if dtype == "e4m3" else torch.bfloat16
+    g, cache, topk_np, got = b.to(gpu), b.cache_kv.to(dt).to(gpu), draw_topk(kv_lens, k, 11), {}
+    args = (g.ql_nope, g.q_pe, None, None, cache, g.kv_lens, torch.from_numpy(topk_np).to(gpu), g.page_indices, g.cu_q_lens, g.cu_kv_lens, (S, S, S))
+    common = dict(sm_scale=b.sm_scale, page_size=P, pages_per_seq=pps, kv_lora_rank=512)
+    for way in (None, "0", "1"):
+        monkeypatch.setenv("RPA_MLA_WAVES", way) if way else monkeypatch.delenv("RPA_MLA_WAVES", raising=False)
+        say(f"dsa {level} P={P} {dtype} S={S} RPA_MLA_WAVES={way}")
+        out = pkg.sparse_mla_via_dense(*args, **common) if level == "token" else pkg.sparse_mla_page_level(*args, k_pages_max=64, **common)[0]
+        torch.cuda.synchronize()
+        got[way] = out.cpu()
+    assert torch.equal(got[None], got[waves]) and not torch.equal(got["0"], got["1"])
+    assert_parity(got["0"].float(), got["1"].float(), **TOL)
