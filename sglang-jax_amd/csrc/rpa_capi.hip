@@ -1244,8 +1244,9 @@ int rpa_describe_plan(const RpaParams* given, char* buf, size_t len) {
                            : r.kernel == rpa::kKernelPrefillWide   ? "rpa_prefill_async_kernel_wide"
                                                                    : "rpa_prefill_async_kernel";
       const PrefillWorkspace w = prefill_workspace(p_in, a);
+      // (a launch that reads the mask's words has the room for bits all the same: new tokens that are not on 16 bytes may send it elsewhere)
       put("prefill: shape=%s kernel=%s tile=%dx%dx%d kv_pieces_with_workspace=%d mask_bits=%s optional_workspace=%zu\n",
-          r.name, kernel, r.tile_q, r.tile_heads, r.tile_kv, w.splits, w.bits_bytes ? "yes" : "no", w.total);
+          r.name, kernel, r.tile_q, r.tile_heads, r.tile_kv, w.splits, w.bits_bytes && !a.mask_words ? "yes" : "no", w.total);
       if (rpa::prefill_by_streams(a)) put("prefill, long sequences: one after the other\n");
       if (a.packed)
         put("prefill, small launch: kernel=rpa_prefill_packed_kernel instead, columns=%d tile=%dx%dx32\n", 32, 32 / a.G, a.G);
@@ -1334,13 +1335,13 @@ static rpa::MlaDecodeArgs mla_key_args(const RpaMlaParams* p, int64_t rows, bool
   return a;
 }
 
-// How a call is cut.  wgs: pieces or shares that run at once; head_blocks > 0: the kernels of a wave per tile (rpa_mla_waves.hip), so many
-// blocks of 16 heads per workgroup and `siblings` workgroups per piece.
+// How a call is cut.  wgs: pieces or shares that run at once; waves: the kernels of a wave per tile (rpa_mla_waves.hip), `siblings` workgroups of
+// 16 heads per piece.
 struct MlaPlan {
   SplitPlan sp;
   const rpa::ShapeRule* rule;
-  int wgs, head_blocks, siblings, token_groups;
-  bool balanced;
+  int wgs, siblings, token_groups;
+  bool waves, balanced;
 };
 
 // Whether a call runs on a wave per tile, with 16 heads a workgroup.  What a piece costs besides its tiles is half of the other kernels', what
@@ -1404,7 +1405,7 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
   MlaPlan m;
   m.rule = &rpa::select_shape(rpa::mla_shape_key(a), rpa::mla_shape_skip(a, tune));
   m.wgs = mla_wgs();
-  m.head_blocks = 0;
+  m.waves = false;
   m.siblings = 1;
   // one workgroup per (row, split, 128 heads) and per CU; every split costs a 256 KiB
   // partial write per 128 heads, so splits are kept as few as fill the CUs once
@@ -1430,7 +1431,7 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
   const int blocks = (p->num_q_heads + 15) / 16;
   if (m.token_groups && waves && tune.mla_waves != 0 && tune.mla_shared_tiles != 0 && (tune.mla_waves > 0 || mla_groups_as_waves(p, rows))) {
     m.token_groups = 0;
-    m.head_blocks = 1;
+    m.waves = true;
     m.siblings = blocks;
     m.balanced = false;
     return m;
@@ -1439,7 +1440,7 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
   if (waves && blocks <= 8 && tune.mla_waves != 0 && !m.token_groups && p->soft_cap == 0.f && tune.mla_shared_tiles != 0 &&
       (tune.mla_waves > 0 || mla_takes_waves(p, rows, sparse))) {
     const MlaPlan other = m;
-    m.head_blocks = 1;
+    m.waves = true;
     m.siblings = blocks;
     m.wgs = std::max(1, m.wgs / m.siblings);
     if (m.siblings > 1 && m.wgs > 8) m.wgs &= ~7;  // (whole eights of workgroups, see Sibling)
@@ -1510,7 +1511,7 @@ static bool mla_use_balanced(const RpaMlaParams* p, const MlaPlan& plan, bool to
   const SplitPlan& fixed = plan.sp;
   const bool on = rpa::tuning().mla_balanced != 0;
   if (!on || token_rows || p->num_splits == 1) return false;
-  if (plan.head_blocks > 0 && mla_min_piece(p) >= kMlaWholeRow) return false;  // (rows of up to 256 tokens stay whole: see there)
+  if (plan.waves && mla_min_piece(p) >= kMlaWholeRow) return false;  // (rows of up to 256 tokens stay whole: see there)
   // Rows the fixed plan leaves whole: one workgroup job per row.  With many more jobs than
   // workgroup slots the dispatcher evens them out by itself; with up to two per slot the kernel
   // ends with the longest rows, and dealing the tiles out evenly pays (300 rows of 1000..8000
@@ -1565,7 +1566,7 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const v
   if (rows <= 0) return RPA_OK;
   MlaPlan plan = mla_plan(p, rows, token_rows, sparse != nullptr);
   // (a call that brings the room of the plan that stood here before stays on it)
-  if (plan.head_blocks > 0 && mla_workspace(p, rows, plan) > (p->workspace ? p->workspace_bytes : 0)) plan = mla_plan(p, rows, token_rows, sparse != nullptr, false);
+  if (plan.waves && mla_workspace(p, rows, plan) > (p->workspace ? p->workspace_bytes : 0)) plan = mla_plan(p, rows, token_rows, sparse != nullptr, false);
   const SplitPlan& sp = plan.sp;
   rpa::MlaDecodeArgs a;
   a.sparse = {};
@@ -1602,13 +1603,13 @@ static int mla_run(const RpaMlaParams* p, void* stream, bool token_rows, const v
   a.cu_tiles = nullptr;
   a.balanced = plan.balanced ? 1 : 0;
   a.num_wgs = plan.wgs;
-  a.head_blocks = plan.head_blocks;
+  a.waves = plan.waves ? 1 : 0;
   a.siblings = plan.siblings;
   a.min_tiles_per_wg = std::max(1, mla_min_piece(p) / 32);
   a.forced_tiles_per_wg = 0;
   a.piece_pad = rpa::tuning().mla_piece_pad >= 0
                     ? rpa::tuning().mla_piece_pad
-                    : plan.head_blocks > 0
+                    : plan.waves
                           ? 8  // (a wave per tile: 6 .. 14 within 1 %; 3 loses 3 % on 64 rows of 2047..16383 e4m3 tokens, 10 % on short rows)
                     : rpa::mla_takes_wide_p16(a, true)
                           ? 12  // (the wide kernels' in the shape table)
@@ -1647,12 +1648,12 @@ int rpa_mla_describe_plan(const RpaMlaParams* p, int token_rows, char* buf, size
   const bool bal = rows > 0 && plan.balanced;
   static const char* const kGroups[] = {"off", "eight_waves_compiled", "eight_waves", "wide"};
   const int tg = plan.token_groups;
-  const bool p16 = !tg && plan.head_blocks == 0 && rpa::mla_takes_wide_p16(mla_key_args(p, rows, token_rows != 0), true);
+  const bool waves = plan.waves, p16 = !tg && !waves && rpa::mla_takes_wide_p16(mla_key_args(p, rows, token_rows != 0), true);
   return snprintf(buf, len, "mla: shape=%s rows=%lld waves_per_wg=%d heads_per_wg=%d share=%d token_groups=%s plan=%s "
                   "pieces_per_row=%d workgroups=%d workspace=%zu%s\n",
-                  r.name, (long long)rows, tg == 3 || p16 ? 4 : r.waves_per_wg, tg ? 128 : r.tile_heads, tg ? 1 : r.share, kGroups[tg],
-                  bal ? "balanced" : "fixed", bal ? 0 : plan.sp.splits, bal ? plan.wgs * plan.siblings : 0,
-                  mla_workspace(p, rows, token_rows != 0), plan.head_blocks > 0 ? " (a wave per tile, 16 heads per workgroup)" : p16 ? " (the wide loop of pages of 16 tokens)" : "");
+                  waves ? "mla_waves" : r.name, (long long)rows, waves || tg == 3 || p16 ? 4 : r.waves_per_wg, waves ? 16 : tg ? 128 : r.tile_heads,
+                  waves || tg ? 1 : r.share, kGroups[tg], bal ? "balanced" : "fixed", bal ? 0 : plan.sp.splits, bal ? plan.wgs * plan.siblings : 0,
+                  mla_workspace(p, rows, token_rows != 0), waves ? " (a wave per tile, 16 heads per workgroup)" : p16 ? " (the wide loop of pages of 16 tokens)" : "");
 }
 
 int rpa_mla_decode(const RpaMlaParams* p, void* stream) {

@@ -218,7 +218,7 @@ struct MlaDecodeArgs {
   int32_t num_wgs;
   int32_t min_tiles_per_wg;
   int32_t forced_tiles_per_wg;
-  int32_t head_blocks;  // > 0: the kernels of a wave per tile (rpa_mla_waves.hip), so many blocks of 16 heads per workgroup
+  int32_t waves;      // the kernels of a wave per tile (rpa_mla_waves.hip), 16 heads per workgroup
   int32_t siblings;   // workgroups that take the same share or piece, each for heads of its own (rpa_mla_waves.hip); 1 elsewhere
   int32_t piece_pad;  // balanced plan: what starting one more (row, head group) costs a workgroup, in tiles
   int32_t* cu_tiles;  // [num_rows + 1] prefix sum of tiles, written by the kernel

@@ -290,7 +290,9 @@ __device__ __forceinline__ void expand_f8_tile(const char* stage, char* slot, in
 // So a wave keeps its own k-steps' queries alone, asks for its K operands before it works out the copies' addresses, and for the partial
 // scores and the V^T operands together behind the barrier; page ids come from a register and the lanes' offsets stay in some.  With
 // the reads two at a time, each waited for, and a scalar load among them: 32 rows of 1000..4000 tokens x 32 heads 40.1 -> 32.1 us,
-// 64 of 2048..16384 x 64 heads 192 -> 170.  16 heads, and little work of more, run a wave per tile (rpa_mla_waves.hip).
+// 64 of 2048..16384 x 64 heads 192 -> 170.  16 heads for the most part, and little work of more, run a wave per tile (rpa_mla_waves.hip); those that do
+// not share a tile four ways too, half the waves only copying: eight ways were 0.5 % slower over 46 ragged batches of up to 16 rounds (three sets
+// of inputs in turn), 0 .. 4 % on selections.
 // TG (token group): with 16 / 32 / 64 heads, the eight waves hold 8 / 4 / 2 CONSECUTIVE QUERY TOKENS of one
 // sequence instead of one token's heads, `group_tokens` of them real (a chunk's tail may leave fewer): wave w
 // owns token (16 w) / Hq of the group and the block of 16 heads (16 w) % Hq.  mr.tq is the group's first token,
@@ -1554,7 +1556,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   const ShapeRule& shape = select_shape(mla_shape_key(a), mla_shape_skip(a, tune));
   const bool pipe = shape.kernel == kKernelMlaWide || shape.kernel == kKernelMlaPipe;
   const int ds = shape.kernel == kKernelMlaShared ? shape.share : 1;
-  if (a.head_blocks > 0) {
+  if (a.waves) {
     hipError_t ew = launch_mla_waves(a, stream);
     if (ew != hipSuccess) return ew;
     if (a.balanced || a.max_splits > 1) launch_mla_combine(a, stream);
@@ -1583,7 +1585,7 @@ hipError_t launch_mla_decode(const MlaDecodeArgs& a, hipStream_t stream) {
   if (ds != 1) {
 #define RPA_MLA_DS_U(LAUNCH, U, F8)                         \
   do {                                                      \
-    if (ds >= 4) LAUNCH<U, false, false, F8, 4>(a, stream); \
+    if (ds == 4) LAUNCH<U, false, false, F8, 4>(a, stream); \
     else LAUNCH<U, false, false, F8, 2>(a, stream);         \
   } while (0)
 #define RPA_MLA_DS(LAUNCH, F8)                    \

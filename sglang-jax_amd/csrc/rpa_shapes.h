@@ -7,6 +7,8 @@
 // query heads a workgroup owns, how many waves walk neighbouring heads together, how many waves stay resident --
 // and this table is their one home: every launcher selects its row here, rpa_describe_plan() prints it, and
 // the RPA_* switches (rpa_tuning.h) only override a row's fields to repeat the measurements behind it.
+// (Absorbed MLA has one choice more, whether a call runs a wave per tile instead, rpa_mla_waves.hip: it goes by how much work the call has and
+// how that would be cut, and is made by mla_plan in rpa_capi.hip.)
 // What varies continuously with the lengths of a batch (how many pieces a row or a K/V range is cut into) is
 // computed from the row's fields by the planners in rpa_capi.hip (plan_splits, the balanced plans) and
 // kv_pieces() (rpa_prefill_common.h).
@@ -119,7 +121,7 @@ constexpr ShapeRule kShapeRules[] = {
   {"mla_pipe", kStageMla, 0, 576, 128, 0, 128, 0, 0, kOptSoftCap | kOptAsmPages,
    kKernelMlaPipe, 1, 128, 32, 8, 8, 1, 12, "e4m3 latents (bytes staged and expanded once per tile) and RPA_MLA_WIDE=0"},
   {"mla_shared_16", kStageMla, 0, 576, 1, 16, 0, 0, 0, kOptSoftCap,
-   kKernelMlaShared, 1, 16, 32, 8, 8, 8, 8, "a tensor-parallel share of the heads; a wave per tile unless RPA_MLA_WAVES=0: 64 rows of 2047..16383 tokens 128 -> 113 us"},
+   kKernelMlaShared, 1, 16, 32, 8, 8, 4, 8, "a tensor-parallel share of the heads: bf16 rows of several lengths, pieces over 512 tokens and up to 15 rounds; few selections of whole pages"},
   {"mla_shared_32", kStageMla, 0, 576, 17, 32, 0, 0, 0, kOptSoftCap,
    kKernelMlaShared, 1, 32, 32, 8, 8, 4, 8, "144 -> 126 us"},
   {"mla_shared_64", kStageMla, 0, 576, 33, 64, 0, 0, 0, kOptSoftCap,

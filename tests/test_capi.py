@@ -871,7 +871,11 @@ def test_mla_shape_table_rows(pkg, monkeypatch):
     c5 = d(params(128), False)
     assert "shape=mla_wide" in c5 and "waves_per_wg=4" in c5 and "plan=balanced" in c5 and "workgroups=256" in c5
     assert "shape=mla_pipe" in d(params(128, fp8=True), False)
-    assert "shape=mla_shared_16" in d(params(16), False) and "share=8" in d(params(16), False)
+    ragged = params(16, S=20, T=20, max_kv=16000, sum_kv=200000)
+    assert "shape=mla_shared_16" in d(ragged, False) and "share=4" in d(ragged, False)
+    for Hq, plan in ((16, "balanced"), (128, "fixed")):  # a wave per tile: four waves, 16 heads
+        text = d(params(16) if Hq == 16 else params(128, S=1, T=1, max_kv=500, sum_kv=500), False)
+        assert "shape=mla_waves" in text and " waves_per_wg=4 heads_per_wg=16 share=1 " in text and f"plan={plan}" in text, text
     assert "shape=mla_shared_64" in d(params(48), False)
     assert "shape=mla_compiled" in d(params(128, P=16), False)
     assert "shape=mla_compiled" in d(params(128, soft_cap=30.0), False)
