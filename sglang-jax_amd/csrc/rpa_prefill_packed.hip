@@ -253,7 +253,7 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_packed_kernel(const Prefil
     mc.mode = 1;
     mc.kv_len = w.kv_len;
   } else if constexpr (EXT) {
-    mc = make_mask_ctx(a, w, row);
+    mc = make_mask_ctx(a, w, min(row, r_hi));
   }
   int t_hi = causal ? min(w.kv_len, w.prefix + r_hi + 1) : w.kv_len;  // exclusive
   int t_lo = 0;
@@ -269,6 +269,9 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_packed_kernel(const Prefil
   const uint32_t vt_at = FP8 ? k_at + 2 * Feed::kTileBytes : v_at;  // V rows as bf16
   const uint32_t ids_at = lds_at + kIdsAt + wave * 256, mask_at = lds_at + kMaskAt + wave * kMaskB;
   const bool has_bits = EXT && !WORDS && mc.mode == 1 && mc.bits;  // (else the caller's words, one load per score)
+  // Columns that are not written see what the last row does: all columns of a wave have their references raised together, so what any of them sees is
+  // part of how the others' probabilities are rounded (and nothing may depend on what LDS holds behind the rows that were copied).
+  const int mask_row = min(pos, r_hi - r_lo);
   const int my_rows = r_hi - r_lo + 1, pairs = WORDS ? __builtin_amdgcn_readfirstlane((my_rows + 1) >> 1) : 0;
   uint64_t mask = 0;   // WORDS: this workgroup's first row
   uint32_t pitch = 0;  // bytes of a row
@@ -392,8 +395,8 @@ __global__ __launch_bounds__(512, 2) void rpa_prefill_packed_kernel(const Prefil
 #pragma unroll
         for (int i = 0; i < decltype(tag)::value; ++i) {
           const uint64_t keep = __ballot(x[i] >= 1);
-          const uint32_t mine = (pos & 1) ? (uint32_t)(keep >> 32) : (uint32_t)keep;
-          mask_word = (pos >> 1) == i ? mine : mask_word;
+          const uint32_t mine = (mask_row & 1) ? (uint32_t)(keep >> 32) : (uint32_t)keep;
+          mask_word = (mask_row >> 1) == i ? mine : mask_word;
         }
       };
       if (pairs <= 2) take(std::integral_constant<int, 2>{});

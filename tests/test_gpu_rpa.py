@@ -1693,6 +1693,41 @@ def test_masks_are_read_as_words(pkg, wl, gpu, monkeypatch, Hq, Hkv, P, fp8, seq
     assert torch.equal(run(), words)
 
 
+@pytest.mark.parametrize("Hq,Hkv,P,fp8", [(32, 8, 64, False), (32, 8, 16, True), (40, 8, 64, False), (16, 8, 48, False)])
+def test_masks_as_words_leave_no_trace(pkg, wl, gpu, monkeypatch, Hq, Hkv, P, fp8):
+    """Workgroups with fewer mask rows than they have room for (1, 9 and 17 tokens where 4, 6, 8 or 16 fit), after launches that left ones and zeros in the
+    room behind them: the same bits every time, and those of a load per score (RPA_MASK_BITS=0)."""
+    rng, window = np.random.default_rng(7), 900
+    monkeypatch.setenv("RPA_PREFILL_PACKED", "1")
+
+    def call(q_lens, kv_lens, density, seed, scale):
+        masks = [(rng.random((ql, kv)) < density).astype(np.int32) for ql, kv in zip(q_lens, kv_lens)]
+        for m in masks:
+            m[:, -1] = 1
+        b = wl.make_batch("mask_trace", q_lens, kv_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=128, page_size=P, seed=seed, sliding_window=window,
+                          kv_dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16)
+        g, mask = b.to(gpu), flat_mask(masks).to(gpu)
+
+        def run():
+            out, _ = pkg.ragged_paged_attention(g.q, None, None, g.kv_cache, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, b.distribution.numpy(),
+                                                mask, sm_scale=scale * b.sm_scale, causal=0, sliding_window=window, k_scale=g.k_scale, v_scale=g.v_scale,
+                                                max_kv_len=max(kv_lens), max_q_len=max(q_lens))
+            torch.cuda.synchronize()
+            return out[: sum(q_lens)].cpu()
+        return run
+
+    fill = [call([16] * 16, [800] * 16, density, 98, 1) for density in (2.0, -1.0)]  # (every token, and the newest alone)
+    target = call([1, 9, 1, 17, 1], [1500, 1300, 3009, 700, 65], 0.1, 99, 4)
+    say(f"masks as words leave no trace Hq={Hq} Hkv={Hkv} P={P} fp8={fp8}")
+    got = []
+    for run in (*fill, *fill):
+        run()
+        got.append(target())
+    monkeypatch.setenv("RPA_MASK_BITS", "0")
+    got.append(target())
+    assert all(torch.equal(x, got[0]) for x in got), [int((x != got[0]).sum()) for x in got]
+
+
 @pytest.mark.parametrize("Hkv,P,fp8,q_lens,old,window,splits", [
     (2, 64, False, [33, 1, 20], [100, 64, 0], None, 0), (2, 16, False, [40, 5], [17, 400], 50, 0), (4, 48, True, [9, 31], [95, 200], None, 0),
     (1, 128, True, [64, 64], [31, 1], None, 0), (2, 64, False, [20], [3000], None, 3), (2, 16, True, [3] * 70, [5 * i for i in range(70)], None, 0)])
