@@ -19,6 +19,16 @@ pytestmark = pytest.mark.gpu
 TOL = dict(rtol=2e-2, atol=2e-2)
 
 
+@pytest.fixture(autouse=True)
+def no_waves(request, monkeypatch):
+    if getattr(request, "param", False):
+        monkeypatch.setenv("RPA_MLA_WAVES", "0")
+
+
+# With the kernels that the plans choose, and without those of a wave per tile.
+both_ways = pytest.mark.parametrize("no_waves", [False, True], ids=["by_call", "no_waves"], indirect=True)
+
+
 def say(*a):
     print(*a, flush=True)
     sys.stdout.flush()
@@ -54,6 +64,7 @@ def test_topk_pages_on_the_device(pkg, gpu, P):
         assert np.array_equal(got.cpu().numpy(), topk_pages_ref(topk, P, pps, kp))
 
 
+@both_ways
 @pytest.mark.parametrize("with_new_token", [False, True])
 def test_token_level_selection_through_the_dense_kernel(pkg, wl, gpu, with_new_token):
     kv_lens, P, k = [40, 300, 64, 1000, 130], 16, 64
@@ -87,6 +98,7 @@ def test_token_level_selection_through_the_dense_kernel(pkg, wl, gpu, with_new_t
     assert_parity(got.cpu().float(), want.float(), **TOL)
 
 
+@both_ways
 @pytest.mark.parametrize("precomputed", [False, True])
 def test_page_level_selection(pkg, wl, gpu, precomputed):
     kv_lens, P, k, kp = [40, 300, 64, 1000, 130], 16, 24, 32
@@ -124,6 +136,7 @@ def test_page_level_selection(pkg, wl, gpu, precomputed):
     assert torch.equal(cache_out.cpu(), b.cache_kv)  # every new row back in its slot, nothing else touched
 
 
+@both_ways
 @pytest.mark.parametrize("level", ["page", "token"])
 @pytest.mark.parametrize("P,Hq,k,dtype", [(16, 16, 2048, "bf16"), (64, 64, 300, "bf16"), (16, 128, 33, "bf16"), (24, 40, 65, "bf16"),
                                           (128, 32, 512, "e4m3"), (16, 128, 96, "e4m3")])
@@ -133,6 +146,7 @@ def test_selections_of_every_shape(pkg, wl, gpu, level, P, Hq, k, dtype):
     check_selections(pkg, wl, gpu, level, P, Hq, k, dtype, [1, 2, 31, P, P + 1, 700, 5003], 40)
 
 
+@both_ways
 @pytest.mark.parametrize("level,P,Hq,k,dtype,kv_lens,kp", [
     # sequences of 2048 pages (whose ids wait in LDS) and of more, and more of them than a wave has lanes
     ("page", 16, 16, 300, "bf16", [32768, 5, 900], 40), ("page", 16, 16, 300, "bf16", [32769, 40000, 5, 900], 40),
@@ -194,6 +208,7 @@ class SparseParams(ctypes.Structure):  # RpaMlaSparse of include/rpa.h
         "topk_count", "topk_stride", "topk_is_pages", "pages_per_seq", "k_pages_max", "num_page_indices")]
 
 
+@both_ways
 @pytest.mark.parametrize("window", [1, 33, 700])
 @pytest.mark.parametrize("level,P,Hq,dtype", [
     ("page", 64, 16, "bf16"), ("page", 64, 128, "bf16"), ("page", 16, 128, "bf16"), ("page", 24, 96, "bf16"), ("page", 32, 64, "e4m3"),

@@ -1595,6 +1595,12 @@ def test_custom_mask_as_bits_equals_the_callers_words(pkg, wl, gpu, monkeypatch,
         monkeypatch.delenv("RPA_PREFILL_SPLITS")
 
 
+def _masked_call(pkg, b, g, q, mask, **kw):
+    return sys.modules["sglang_jax_amd.ragged_paged_attention"].RpaCall(
+        q, g.kv_cache, None, g.kv_lens, g.page_indices, g.cu_q_lens, g.cu_kv_lens, num_seqs=len(b.kv_lens), decode_end=0, sm_scale=b.sm_scale,
+        k_scale=g.k_scale, v_scale=g.v_scale, causal=False, custom_mask=mask, own_workspace=True, **kw)
+
+
 @pytest.mark.parametrize("seqs", [1, 62, 63, 64, 130])
 @pytest.mark.parametrize("bound", [5000, 400000])
 def test_mask_bits_of_many_sequences_and_long_rows(pkg, wl, gpu, monkeypatch, seqs, bound):
@@ -1616,6 +1622,9 @@ def test_mask_bits_of_many_sequences_and_long_rows(pkg, wl, gpu, monkeypatch, se
         torch.cuda.synchronize()
         return out[: sum(q_lens)].cpu()
 
+    monkeypatch.setenv("RPA_PREFILL_PACKED", "0")  # (small launches read the words themselves)
+    text = pkg._lib.describe_plan(_masked_call(pkg, b, g, g.q, mask, max_kv_len=bound, max_q_len=4).params)
+    assert "mask_bits=yes" in text and "rpa_prefill_packed_kernel" not in text, text
     monkeypatch.setenv("RPA_MASK_BITS", "0")
     words = run()
     monkeypatch.delenv("RPA_MASK_BITS")
@@ -1626,9 +1635,9 @@ def test_mask_bits_of_many_sequences_and_long_rows(pkg, wl, gpu, monkeypatch, se
 @pytest.mark.parametrize("D,Hkv,P,fp8", [(128, 2, 16, False), (128, 20, 64, True), (64, 3, 48, False)])
 @pytest.mark.parametrize("on_device", [False, True])
 def test_masked_calls_bring_their_tokens(pkg, wl, gpu, monkeypatch, seqs, D, Hkv, P, fp8, on_device):
-    """The launch that makes bits of a mask puts the new tokens into the cache as well: same rows and the same cache, byte for byte, as
-    the launch in front of it leaves where the mask stays words.  Both searches, rows shorter and longer than a workgroup,
-    narrow heads, and a padded batch whose size is on the device."""
+    """The launch that makes bits of a mask puts the new tokens into the cache as well, and so does a small launch that reads the mask's words: the same rows as
+    where the launch in front leaves the tokens and the mask stays words, and, byte for byte, the cache with the tokens put into it here.  Both searches,
+    rows shorter and longer than a workgroup and than a KiB, narrow heads, and a padded batch whose size is on the device."""
     q_lens = [[3, 1, 17, 4][i % 4] for i in range(seqs)]
     kv_lens = [q + [0, 61, 300][i % 3] for i, q in enumerate(q_lens)]
     rng = np.random.default_rng(seqs)
@@ -1655,12 +1664,34 @@ def test_masked_calls_bring_their_tokens(pkg, wl, gpu, monkeypatch, seqs, D, Hkv
         torch.cuda.synchronize()
         return out[:T].cpu(), cache.cpu().view(torch.uint8)
 
-    monkeypatch.setenv("RPA_MASK_BITS", "0")
-    words = run()
-    monkeypatch.delenv("RPA_MASK_BITS")
+    want, table, t = b.kv_cache.clone().view(torch.uint8), b.padded_page_table(), 0
+    rows = torch.zeros(T, 2 * Hkv, 128, dtype=b.kv_cache.dtype).view(torch.uint8)  # (narrow heads: zeros behind them)
+    for half, x in enumerate((k, v)):
+        rows[:, half::2, :x[:T].cpu().view(torch.uint8).shape[-1]] = x[:T].cpu().view(torch.uint8)
+    for i, (n, kv) in enumerate(zip(q_lens, kv_lens)):
+        for at in range(kv - n, kv):
+            want[int(table[i, at // P]), at % P] = rows[t]
+            t += 1
+    assert not torch.equal(want, b.kv_cache.view(torch.uint8))
+
+    def writer():
+        call = _masked_call(pkg, b, g, g.q, mask, max_kv_len=max(kv_lens), max_q_len=17, **(dict(distribution_d=dist) if on_device else {}))
+        call.params.q_head_dim, call.params.layout = D, call.params.layout | pkg._lib.RPA_PARAMS_TAIL
+        return pkg._lib.describe_plan(call.params)
+
+    small = run()
+    by_small = "workgroups of the prefill launch" in writer()
+    assert by_small == (D == 128 and not on_device)
+    monkeypatch.setenv("RPA_PREFILL_PACKED", "0")
+    assert "written by the launch that makes bits of the mask" in writer()
     bits = run()
-    assert torch.equal(bits[1], words[1]) and not torch.equal(bits[1], g.kv_cache.cpu().view(torch.uint8))
+    monkeypatch.setenv("RPA_MASK_BITS", "0")
+    assert "rpa_kv_write_kernel, in front" in writer()
+    words = run()
+    for _, cache in (small, bits, words):
+        assert torch.equal(cache.view(want.shape), want)
     assert torch.equal(bits[0], words[0])
+    assert_parity(small[0].float(), words[0].float(), **(FP8_TOL if fp8 else BF16_TOL))
 
 
 @pytest.mark.parametrize("Hq,Hkv,P,fp8,seqs,aligned,window", [
