@@ -344,6 +344,10 @@ RPA_API int rpa_kv_write(const RpaParams* p, const void* keys, const void* value
  * rpa_kv_write and rpa_attention as one call: ragged_paged_attention as the reference's layers call it
  * (ragged_paged_attention_v3.py:1667-2097 writes the new tokens and attends to them in one kernel).  keys / values:
  * [T, Hkv, D] in the cache dtype, or both NULL when the cache already holds every token.
+ *
+ * Every sequence sees its own new tokens.  Whether it sees those that another sequence of the same call brings into a page that
+ * both tables name is not defined: the cache is written in front of the attention, beside it or by it, by what the call is.  A call
+ * behind this one on the stream finds all of them.
  */
 RPA_API int rpa_attention_update(const RpaParams* p, const void* keys, const void* values, void* stream);
 
@@ -380,7 +384,8 @@ RPA_API int rpa_mla_kv_write(const RpaMlaParams* p, const void* new_kv_c, const 
 
 /*
  * rpa_mla_kv_write and rpa_mla_decode (token_rows = 0) or rpa_mla_attention (token_rows = 1) as one call; the new rows
- * may both be NULL when the cache already holds every token.
+ * may both be NULL when the cache already holds every token.  New tokens in pages of several sequences: as
+ * rpa_attention_update has it.
  */
 RPA_API int rpa_mla_attention_update(const RpaMlaParams* p, const void* new_kv_c, const void* new_k_pe, int token_rows,
                              void* stream);
