@@ -375,17 +375,22 @@ __device__ __forceinline__ void pipe_loop_masked(RowBlock<64> (&b)[1], const Sha
 // long context) cut every workgroup's run of K/V tiles into a.kv_splits pieces, blockIdx.y picks the piece,
 // and the workgroup leaves unnormalised rows with their (reference, sum) in the workspace for
 // rpa_prefill_combine_kernel instead of finished rows.
-template <bool WIN, int NQ, bool HEADS4 = false, bool SPLIT = false, int HD = 128>
+//
+// DYN: the composition may be on the device.  A kernel of its own: with the early way out in every one the compiler read the arguments behind it, one
+// trip more per workgroup: 6 chunks of 176..353 tokens on up to 945, 64 / 8 heads, 57.3 -> 59.5 us.
+template <bool WIN, int NQ, bool HEADS4 = false, bool SPLIT = false, int HD = 128, bool DYN = false>
 __global__ __launch_bounds__(256, (HD == 64 ? 3 : NQ == 1 ? 2 : 1)) void rpa_prefill_pipe_kernel(const PrefillArgs a_in, int tiles, int nseq,
                                                                                  bool by_level, float row_sum_limit,
                                                                                  bool masked_steps) {
-  PrefillArgs a = a_in;  // static-shape mode: the sequences to process come from the device
-  if (a.dist) {
-    a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
-    a.seq_end = min(a.seq_end, scalar_load_i32(a.dist + 2));
-    // A step of decode rows: the grid of the bounds finds nothing.  Its workgroups go through the few places that their LDS leaves, so what one does
-    // before it leaves is paid once a round (1024 of them 3.3 -> 2.1 us, 4096 behind 112 us of decode 5.9 -> 4.8, 3072 of the compiled loop's 5.2 -> 2.6).
-    if (a.seq_begin >= a.seq_end) return;
+  PrefillArgs a = a_in;
+  if constexpr (DYN) {
+    if (a.dist) {  // static-shape mode: the sequences to process come from the device
+      a.seq_begin = (a.sm.mask_mode == 1) ? 0 : scalar_load_i32(a.dist);
+      a.seq_end = min(a.seq_end, scalar_load_i32(a.dist + 2));
+      // A step of decode rows: the grid of the bounds finds nothing.  Its workgroups go through the few places that their LDS leaves, so what one does
+      // before it leaves is paid once a round (1024 of them 3.3 -> 2.1 us, 4096 behind 112 us of decode 5.9 -> 4.8, 3072 of the compiled loop's 5.2 -> 2.6).
+      if (a.seq_begin >= a.seq_end) return;
+    }
   }
   static_assert((!HEADS4 && HD == 128) || NQ == 1, "the short-chunk tile and narrow heads have one block of rows per wave");
   typedef Head<HD> HL;
@@ -667,12 +672,14 @@ hipError_t launch_prefill_pipe(const PrefillArgs& call, int nseq, bool level_ord
   const dim3 g((unsigned)(grid + a.write_blocks)), blk(256);
   const bool win = a.sm.window > 0;
   const bool narrow = narrow_heads(a, nq);
-#define RPA_LAUNCH(GRID, W, H4, SPLIT, HD) \
-  hipLaunchKernelGGL((rpa_prefill_pipe_kernel<W, 1, H4, SPLIT, HD>), GRID, blk, 0, stream, a, tiles, nseq, by_level, limit, masked)
-#define RPA_LAUNCH_W(GRID, H4, SPLIT, HD)             \
-  do {                                                \
-    if (win) RPA_LAUNCH(GRID, true, H4, SPLIT, HD);   \
-    else RPA_LAUNCH(GRID, false, H4, SPLIT, HD);      \
+#define RPA_LAUNCH(GRID, W, H4, SPLIT, HD, DYN) \
+  hipLaunchKernelGGL((rpa_prefill_pipe_kernel<W, 1, H4, SPLIT, HD, DYN>), GRID, blk, 0, stream, a, tiles, nseq, by_level, limit, masked)
+#define RPA_LAUNCH_W(GRID, H4, SPLIT, HD)                           \
+  do {                                                              \
+    if (win && a.dist) RPA_LAUNCH(GRID, true, H4, SPLIT, HD, true); \
+    else if (win) RPA_LAUNCH(GRID, true, H4, SPLIT, HD, false);     \
+    else if (a.dist) RPA_LAUNCH(GRID, false, H4, SPLIT, HD, true);  \
+    else RPA_LAUNCH(GRID, false, H4, SPLIT, HD, false);             \
   } while (0)
 #define RPA_LAUNCH_D(GRID, H4, SPLIT)                 \
   do {                                                \
@@ -691,8 +698,8 @@ hipError_t launch_prefill_pipe(const PrefillArgs& call, int nseq, bool level_ord
   } else if (nq == 1) {
     RPA_LAUNCH_D(g, false, false);
   } else {
-    if (win) hipLaunchKernelGGL((rpa_prefill_pipe_kernel<true, 2>), g, blk, 0, stream, a, tiles, nseq, by_level, limit, masked);
-    else hipLaunchKernelGGL((rpa_prefill_pipe_kernel<false, 2>), g, blk, 0, stream, a, tiles, nseq, by_level, limit, masked);
+    if (win) hipLaunchKernelGGL((rpa_prefill_pipe_kernel<true, 2, false, false, 128, true>), g, blk, 0, stream, a, tiles, nseq, by_level, limit, masked);
+    else hipLaunchKernelGGL((rpa_prefill_pipe_kernel<false, 2, false, false, 128, true>), g, blk, 0, stream, a, tiles, nseq, by_level, limit, masked);
   }
 #undef RPA_LAUNCH_D
 #undef RPA_LAUNCH_W
