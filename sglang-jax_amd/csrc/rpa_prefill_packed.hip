@@ -94,15 +94,21 @@ struct PackedFeed {
     first = tb;
     last = s.last_tok;
     if constexpr (PG == 0) {
-      fresh = 0;
 #pragma unroll
       for (int n = 0; n < N; ++n) {
         const int tok = min(tb + row_of(n, lane), s.last_tok), ps = page_slot(s, tok);
         const int id = *(__attribute__((address_space(3))) const int32_t*)(lds_t)(uintptr_t)(ids + 4u * (uint32_t)(ps - page_slot(s, tb)));
         row[n] = (int64_t)id * kv.page_stride + (int64_t)(tok - ps * s.page_size) * kv.tok_stride;
-        if (tok >= new_from) {
-          row[n] = (int64_t)(tok - new_from) * new_stride;
-          fresh |= 1u << n;
+      }
+      fresh = 0;
+      if (tb + kTok > new_from) {  // (the same in every lane)
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+          const int past = min(tb + row_of(n, lane), s.last_tok) - new_from;
+          if (past >= 0) {
+            row[n] = (int64_t)past * new_stride;
+            fresh |= 1u << n;
+          }
         }
       }
     } else {
@@ -153,11 +159,17 @@ struct PackedFeed {
       }
     } else {
       const int cp = lane % kPerRow;
-#pragma unroll
-      for (int n = 0; n < N; ++n) {
+      auto put = [&](int n, const char* from) __attribute__((always_inline)) {
         const int t = row_of(n, lane);
-        const char* g = ((fresh >> n) & 1 ? new_head : head) + row[n] + ((IS_V ? chunk_v(t, cp) : chunk_k(t, cp)) << 4);
+        const char* g = from + row[n] + ((IS_V ? chunk_v(t, cp) : chunk_k(t, cp)) << 4);
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at + n * 1024), "v"(g) : "memory", "m0");
+      };
+      if (first + kTok <= new_from) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) put(n, head);
+      } else {
+#pragma unroll
+        for (int n = 0; n < N; ++n) put(n, (fresh >> n) & 1 ? new_head : head);
       }
     }
   }
