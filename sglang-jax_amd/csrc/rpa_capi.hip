@@ -937,9 +937,16 @@ static bool takes_fresh_prompts(const RpaParams* p) {
 // Whether the launch of small chunks behind prefixes (rpa_prefill_packed_kernel) may take the new tokens from the caller's rows and write them into
 // the cache beside the attention.  Not with decode rows in the call, whose launch in front writes the chunks' tokens too.  A call that says
 // nothing of a prefix may be all new, an address per lane and row: up to 512 tokens.
+// On pages of 16 tokens and whole tiles a tile with new tokens takes twice as long as one of cached rows (an address per lane in place of one per tile), which
+// outweighs the 3 us of the launch in front once the workgroups of a CU go through some of them: tokens x query heads x longest chunk in bytes of an element,
+// 12 M of them being three such tiles per wave.  The call, in front -> beside, with that number: bf16 1056 tokens x 8 / 2 heads 19.1 -> 15.8 us (10 M), 1361 of up
+// to 1470 on pages of 48 30.6 -> 26.3, but 1672 x 8 / 1 40.5 -> 43.3 (23 M), 1951 x 8 / 1 35.0 -> 38.6 (37 M), 1628 x 8 / 2 36.5 -> 43.2 (36 M); e4m3 1170 x 8 / 4
+// 20.7 -> 18.5 (8 M), 2354 x 8 / 1 37.4 -> 39.3 (28 M).
 static bool chunks_bring_tokens(const RpaParams* p, const void* keys, const void* values) {
+  const int64_t longest = p->max_q_len > 0 ? p->max_q_len : p->num_tokens;
   return !p->distribution && (p->decode_end == 0 || p->mask_mode == RPA_MASK_CUSTOM) && p->head_dim == 128 && q_dim_of(p) == p->head_dim &&
          (p->max_kv_len > p->max_q_len || p->num_tokens <= 512) && ((reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(values)) & 15) == 0 &&
+         ((p->page_size % 32 != 0 && p->page_size != 16) || longest * p->num_tokens * p->num_q_heads * esize_of(p->kv_dtype) <= 12'000'000) &&
          (int64_t)p->num_tokens * p->num_kv_heads * p->head_dim * esize_of(p->kv_dtype) < (int64_t(1) << 31);
 }
 

@@ -634,8 +634,9 @@ int prefill_packed_pieces(const PrefillArgs& a) {
       const bool long_grid = wgs > 3 * compute_units();
       other = (long_grid ? std::min(margin, 0.65) : margin) * (8.0 + other);
       // The launch that writes the new tokens is spared: 3 prompts of 47 tokens e4m3 x 8 / 4 heads 11.7 -> 7.9, 2 chunks of 21 on 2661 x 8 / 2 18.2 -> 13.9.
-      // Counted in one round of workgroups (6 chunks of 80 on 490 x 40 / 8 19.3, here 24.9), and not for e4m3 pieces (230 tokens on 4277 x 8 / 4 23.0 and 28.1).
-      if (a.saves_launch && wgs <= compute_units()) spared = 3.0;
+      // Counted in one round of workgroups (6 chunks of 80 on 490 x 40 / 8 19.3, here 24.9), and not for e4m3 pieces (230 tokens on 4277 x 8 / 4 23.0 and 28.1)
+      // nor where a tile's rows have an address each (pages of 48: 136 tokens on 3100 x 16 / 8 23.3 and 28.2, 510 on 2894 x 8 / 4 30.0 and 34.5).
+      if (a.saves_launch && wgs <= compute_units() && (a.pt.page_size % kTok == 0 || a.pt.page_size == 16)) spared = 3.0;
       if (a.seq_begin > 0 && a.max_q_len < a.max_kv_len) {
         PrefillArgs own = a;
         own.max_kv_len = a.max_q_len;

@@ -713,6 +713,23 @@ def test_plans_on_both_sides_of_their_rules(pkg, monkeypatch):
     assert "pieces_per_row=4 " in rows(180, 3000, D=256, sum_dec=270000)  # rows that differ: twice the slots
 
 
+def test_small_chunks_bring_their_tokens_where_that_is_less_work(pkg):
+    """The launch of small chunks reads the new tokens from the caller's rows up to 12 M of tokens x query heads x longest chunk x bytes, on pages that are no
+    multiple of a tile whatever they are; the launch in front is not counted as spared there."""
+    def plan(T, q, Hq, Hkv, kv, P=64, S=2, **kw):
+        d = pkg._lib.describe_plan(_shape_params(pkg, S=S, decode_end=0, T=T, Hq=Hq, Hkv=Hkv, P=P, max_q=q, max_kv=kv, **kw))
+        return "rpa_prefill_packed_kernel" in d, "workgroups of the prefill launch, which reads the caller's rows" in d
+
+    assert plan(1056, 603, 8, 2, 684) == (True, True) and plan(1170, 843, 8, 4, 881, fp8=True, P=16) == (True, True)
+    assert plan(1951, 1175, 8, 1, 1512, P=128) == (True, False) and plan(1628, 1383, 8, 2, 1618, P=16) == (True, False)
+    assert plan(2354, 1478, 8, 1, 1640, P=128, fp8=True) == (True, False)
+    for P, beside in ((64, False), (32, False), (16, False), (48, True), (24, True)):
+        assert plan(1951, 1175, 8, 1, 1512, P=P) == (True, beside), P
+    for T, beside in ((1000, True), (1001, False)):
+        assert plan(T, 750, 8, 1, 1512, S=2) == (True, beside), T
+    assert plan(136, 74, 16, 8, 3174, P=16)[0] and not plan(136, 74, 16, 8, 3174, P=48)[0] and not plan(510, 182, 8, 4, 2894, P=48, S=3)[0]
+
+
 def test_shape_table_environment_overrides(pkg, monkeypatch):
     d = pkg._lib.describe_plan
     p = _shape_params(pkg, S=64, decode_end=56, T=8760, Hq=32, Hkv=8, max_q=2048, max_kv=4096, sum_dec=130000)
