@@ -1011,6 +1011,18 @@ static bool prefill_args(const RpaParams* p, rpa::PrefillArgs& a, const void* ke
   if (!a.packed || rpa::tuning().mask_bits == 0) a.mask_words = 0;
   if (a.packed && keys && !a.rows_are_new && chunks_bring_tokens(p, keys, values)) {
     write_beside();
+    // A workgroup has a CU to itself here: those that write, which stand behind the attention's of every piece, are as few as those leave CUs for in their
+    // last round, or one more is waited for (144 tokens on up to 1859, 16 / 8 heads, e4m3, 240 workgroups in three pieces: of 8 tokens each 26.4 us, of 32
+    // 18.8; in front 21.7).  Where they leave none, eight tokens each (121 on up to 4098, 256 workgroups: 22.5, of 64 tokens 26.3).
+    const int per = 32 / a.G, cus = rpa::compute_units();
+    const int64_t wgs = (int64_t)(a.seq_end - a.seq_begin) * ((a.max_q_len + per - 1) / per) * a.Hkv * a.packed;
+    for (int tokens = 8; tokens <= 64; tokens *= 2) {
+      const int blocks = (p->num_tokens + tokens - 1) / tokens;
+      if (wgs % cus + (int64_t)blocks * a.packed > cus) continue;
+      a.write_tokens = tokens;
+      a.write_blocks = blocks;
+      break;
+    }
     a.tail_is_new = 1;
   }
   return true;

@@ -1761,7 +1761,10 @@ def test_masks_as_words_leave_no_trace(pkg, wl, gpu, monkeypatch, Hq, Hkv, P, fp
 
 @pytest.mark.parametrize("Hkv,P,fp8,q_lens,old,window,splits", [
     (2, 64, False, [33, 1, 20], [100, 64, 0], None, 0), (2, 16, False, [40, 5], [17, 400], 50, 0), (4, 48, True, [9, 31], [95, 200], None, 0),
-    (1, 128, True, [64, 64], [31, 1], None, 0), (2, 64, False, [20], [3000], None, 3), (2, 16, True, [3] * 70, [5 * i for i in range(70)], None, 0)])
+    (1, 128, True, [64, 64], [31, 1], None, 0), (2, 64, False, [20], [3000], None, 3), (2, 16, True, [3] * 70, [5 * i for i in range(70)], None, 0),
+    # workgroups that write 16, 32 and 64 tokens each (224, 480 - 256 and 248 of attention)
+    (4, 64, False, [64] * 7, [33 * i for i in range(7)], None, 0), (4, 16, True, [62] * 15, [40 * i for i in range(15)], None, 0),
+    (4, 48, False, [16] * 31, [7 * i for i in range(31)], None, 0)])
 def test_small_chunks_bring_their_tokens(pkg, wl, gpu, monkeypatch, Hkv, P, fp8, q_lens, old, window, splits):
     """Chunks behind prefixes whose new tokens are not in the cache: tiles with old and new rows, new ones alone, the last one short; pages of a tile,
     of half a one and odd ones; a window; pieces; sequences beyond a wavefront's lanes.  The same bits as with the tokens in the cache,
