@@ -1365,11 +1365,15 @@ struct MlaPlan {
 
 // Whether a call runs on a wave per tile, with 16 heads a workgroup.  What a piece costs besides its tiles is half of the other kernels', what
 // a tile costs grows with every 16 heads: so by the work, in rounds of 64 tokens x 16 heads per CU.  us, other kernels -> these, and the rounds:
-//   16 heads           64 rows of 2047..16383 bf16 128 -> 113, e4m3 119 -> 76, on pages of 16 130 -> 114 and 137 -> 78; small ones level to 1.2 x
+//   16 heads           64 rows of 2047..16383 bf16 128 -> 113, e4m3 119 -> 76, on pages of 16 130 -> 114 and 137 -> 78; small ones on pages of 16 1.05 .. 1.4 x, on whole
+//                      tiles level, e4m3 under a round 1.0 .. 0.93 x (2 of 559..1861 12.6 -> 13.6) but for whole rows (5 of 115..210 16.0 -> 12.3)
 //   32 heads, e4m3     the same rows 125 -> 105 (72), 128 of 500 28.2 -> 18.5 (8); bf16 133 -> 141 (72), 30.5 -> 32.0 (9.8), 128 of 500 26.9 -> 21.4 (7.8), on
-//                      pages of 16 35.3 -> 31.9 (9.8), 141 -> 145 (72); selections of 32 rows x 64 pages 39.6 -> 37.8 (16), of 50 rows 47.9 -> 54.4 (25)
+//                      pages of 16 35.3 -> 31.9 (9.8), 141 -> 145 (72); e4m3 in between 23 of 177..6038 29.3 -> 30.7 (8), 12 of 7548..9184 34.8 -> 37.1 (12), 32 of 2133..14199
+//                      61.7 -> 58.9 (30); bf16 selections of 9 rows x 64 pages 22.1 -> 21.6 (4), of 23 32.5 -> 34.1 (12)
 //   64 heads, bf16     20 rows of 300..1500 28.0 -> 24.5 (4.4), 54 of 300..800 31.0 -> 31.8 (7.3), on pages of 16 33.4 -> 31.7; 32 of 1000..4000 41.9 -> 45.0 (20);
-//                      e4m3 44.3 -> 42.6 (20), 157 -> 165 (144); selections of 12 rows x 64 pages 35.3 -> 33.8 (12), of 32 52.2 -> 57.2 (32)
+//                      e4m3 5 of 2829..6230 28.6 -> 23.1 (6), 11 of 4297..4690 33.8 -> 35.1 (12), 49 of 873..1449 37.7 -> 41.8 (14), on pages of 16 17 of 399..8919
+//                      47.4 -> 46.1 (21), 77 of 435..3187 66.4 -> 73.6 (36); selections of 12 rows x 64 pages 35.3 -> 33.8 (12), of 32 52.2 -> 57.2 (32), single tokens 31 of 1024
+//                      28.2 -> 25.9 (8), 24 of 2048 34.7 -> 37.1 (12)
 //   128 heads          one row of 4000 25.1 -> 15.8 (2), 8 of 300..1500 26.7 -> 22.8 (3.5), 20 33.1 -> 34.1 (8.8), on pages of 16 36.9 -> 34.1, e4m3 39.7 -> 33.1;
 //                      54 of 300..800 37.6 -> 45.8 (14.5); selections of 4 rows x 64 pages 33.3 -> 26.3 (8), 12 of 2048 tokens 39.9 -> 39.4 (12)
 // Rows that stay whole (up to 256 tokens) are short beside what a workgroup costs anyway: there by the workgroups, in rounds of the CUs.  351 drawn
@@ -1388,14 +1392,17 @@ static bool mla_takes_waves(const RpaMlaParams* p, int64_t rows, bool sparse) {
   const int64_t tokens = p->sum_kv_len > 0 ? std::min(p->sum_kv_len, rows * longest) : rows * longest;
   const int64_t rounds = tokens * blocks / (64 * (int64_t)mla_wgs());
   const bool fp8 = p->cache_dtype == RPA_KV_FP8_E4M3, whole = p->page_size % 32 == 0;  // (pages of whole tiles: where the other kernels are at their best)
-  if (blocks == 1) return !sparse || fp8 || !whole || rounds >= 4;
+  if (blocks == 1) return !whole || (fp8 ? rounds >= 1 || longest <= kMlaWholeRow : !sparse || rounds >= 4);
   if (longest <= kMlaWholeRow && !sparse) {
     const int eighths = blocks > 4 ? (fp8 ? 16 : 12) : blocks > 2 ? (whole ? 6 : 10) : (fp8 ? 7 : 6);
     return 8 * rows * blocks <= (int64_t)eighths * mla_wgs();
   }
   const bool one_round = sparse || rows * blocks <= mla_wgs();
-  if (blocks <= 2) return fp8 ? one_round || !whole || tokens >= 512 * rows : rounds < (sparse ? 20 : whole ? 6 : 24);
-  if (blocks <= 4) return rounds < (fp8 ? whole ? (one_round ? 32 : 0) : 200 : sparse || !whole ? 14 : 6);
+  if (blocks <= 2) {
+    if (!fp8) return rounds < (sparse ? whole ? 9 : 20 : whole ? 6 : 24);
+    return !whole || sparse || ((one_round || tokens >= 512 * rows) && (rounds < 5 || rounds >= 15));
+  }
+  if (blocks <= 4) return rounds < (fp8 ? !whole ? 22 : sparse ? 14 : one_round ? 9 : 0 : sparse ? whole ? 14 : 11 : whole ? 6 : 14);
   // (selections, one workgroup more than the CUs: 33 rows of 512 tokens 34.5 -> 42)
   return rounds < (fp8 || sparse || !whole ? 10 : 6) && (!sparse || rows * blocks <= mla_wgs());
 }
@@ -1476,10 +1483,14 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
     // of 128, 8 of 1000..8000 22.5 -> 20.0 of 256, 100 of 200..1000 e4m3 25.9 -> 22.7 of 512, 20 of 300..1500 x 32 heads 19.2 -> 17.4; beyond, 100 of
     // 200..1000 in pieces of 256 26.3 -> 33.4.
     const int64_t longest = mla_longest(p);
+    const bool tiles16 = !sparse && !token_rows && tune.mla_waves < 0 && p->cache_dtype == RPA_KV_BF16 && p->page_size % 32 == 0;
     if (p->num_splits == 0 && !(p->sum_kv_len > 0 && p->sum_kv_len == rows * longest)) {
+      bool coarse = false;
       for (int64_t chunk = mla_min_piece(p); chunk <= 512; chunk *= 2) {
         const int64_t pieces = (longest + chunk - 1) / chunk;
         if (rows * pieces > m.wgs) continue;
+        // (pieces of 512 of long bf16 rows leave too many CUs idle: 31 of 137..2231 x 16 heads 20.6 -> 23.0, 7 of 5427..11524 23.2 -> 25.3, 3 of 179..14794 x 32 19.8 -> 22.3)
+        if ((coarse = chunk > 256 && longest > 1024 && blocks <= 2 && tiles16)) break;
         m.sp.splits = (int)pieces;
         m.sp.chunk = (int)((longest + pieces - 1) / pieces + 31) / 32 * 32;
         m.balanced = false;
@@ -1489,9 +1500,7 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
       // of 64 tokens per CU (113 drawn batches x 16 heads, shared -> waves: 12 of 5800..23203 37.4 -> 40.0, 41 of 472..7560 40.6 -> 43.6, 13.2 rounds 48.3 ->
       // 50.6; 16.3 rounds 60.3 -> 59.3, 17.2 and more 1.11 .. 1.14 x; pages of 16 1.03 .. 1.14 x, e4m3 1.11 .. 1.64 x throughout; selections: see mla_takes_waves).
       const int64_t tokens = p->sum_kv_len > 0 ? std::min(p->sum_kv_len, rows * longest) : rows * longest;
-      if (blocks == 1 && !sparse && !token_rows && tune.mla_waves < 0 && p->cache_dtype == RPA_KV_BF16 && p->page_size % 32 == 0 &&
-          tokens < 15 * 64 * (int64_t)mla_wgs())
-        m = other;
+      if (coarse || (blocks == 1 && tiles16 && tokens < 15 * 64 * (int64_t)mla_wgs())) m = other;
     }
   }
   m.balanced = !sparse && mla_use_balanced(p, m, token_rows);

@@ -781,8 +781,20 @@ def test_mla_little_work_runs_a_wave_per_tile(pkg, monkeypatch):
         _mla_params(pkg, Hq, S=S, T=S, max_kv=longest, sum_kv=S * longest * 3 // 4, **kw), False)
     assert takes(16, 64, 16384) and takes(16, 1, 40, P=1, fp8=True) and takes(5, 300, 3000) and not takes(16, 64, 16384, soft_cap=30.0)
     assert takes(32, 64, 16384, fp8=True) and not takes(32, 64, 16384) and takes(24, 8, 1500)
-    assert takes(64, 20, 1000) and not takes(64, 40, 4000) and takes(64, 40, 4000, fp8=True) and takes(64, 30, 2000, P=16)
+    assert takes(64, 20, 1000) and not takes(64, 40, 4000) and takes(64, 10, 4000, fp8=True) and takes(64, 30, 2000, P=16)
     assert takes(128, 3, 4000) and takes(128, 16, 1000, fp8=True) and not takes(128, 64, 1000) and not takes(160, 1, 100)
+    # both sides of the limits, in tokens of the rows; whole rows of e4m3, pieces of 512 of long bf16 rows
+    def sums(Hq, S, longest, tokens, **kw):
+        return "a wave per tile" in pkg._lib.describe_mla_plan(_mla_params(pkg, Hq, S=S, T=S, max_kv=longest, sum_kv=tokens, **kw), False)
+
+    assert not sums(16, 3, 8000, 16383, fp8=True) and sums(16, 3, 8000, 16384, fp8=True) and sums(16, 3, 8000, 16383, fp8=True, P=16)
+    assert sums(16, 5, 256, 700, fp8=True) and not sums(16, 5, 257, 700, fp8=True) and sums(16, 1, 600, 500)
+    for rounds, waves in ((4.9, True), (5, False), (14.9, False), (15, True)):
+        assert sums(32, 20, 9000, int(rounds * 8192), fp8=True) == waves and sums(32, 20, 9000, int(rounds * 8192), fp8=True, P=16), rounds
+    for P, limit in ((64, 9), (16, 22)):
+        assert sums(64, 20, 9000, limit * 4096 - 1, fp8=True, P=P) and not sums(64, 20, 9000, limit * 4096, fp8=True, P=P)
+    assert not sums(16, 31, 2200, 40000) and sums(16, 31, 1000, 20000) and sums(16, 31, 2200, 40000, P=16) and sums(16, 31, 2200, 40000, fp8=True)
+    assert not sums(32, 3, 12200, 18000) and sums(32, 6, 4800, 22000)
     p = _mla_params(pkg, 16, S=20, T=20, max_kv=1500, sum_kv=18000)
     assert "plan=fixed pieces_per_row=12" in pkg._lib.describe_mla_plan(p, False)  # one round of pieces of 128 tokens
     monkeypatch.setenv("RPA_MLA_WAVES", "0")

@@ -285,11 +285,11 @@ def test_selections_with_new_rows_anywhere_in_memory(pkg, wl, gpu, monkeypatch, 
     assert torch.isfinite(got[0][0]).all() and torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
-@pytest.mark.parametrize("level,P,dtype,S,waves", [("page", 64, "bf16", 15, "0"), ("page", 64, "bf16", 16, "1"), ("page", 64, "e4m3", 3, "1"), ("page", 16, "bf16", 3, "1"),
+@pytest.mark.parametrize("level,P,dtype,S,waves", [("page", 64, "bf16", 15, "0"), ("page", 64, "bf16", 16, "1"), ("page", 64, "e4m3", 3, "0"), ("page", 64, "e4m3", 4, "1"), ("page", 16, "bf16", 3, "1"),
                                                    ("token", 64, "bf16", 3, "1")])
 def test_few_selections_of_whole_pages_share_tiles(pkg, wl, gpu, monkeypatch, level, P, dtype, S, waves):
-    """16 heads, bf16, pages of whole tiles: under four rounds of 64 tokens per CU the waves of a workgroup share its tiles, from there on, and for every
-    other selection, each has its own.  Which one ran shows in the bits, and both are near the oracle."""
+    """16 heads, pages of whole tiles: under four rounds of 64 tokens per CU (e4m3: one) the waves of a workgroup share its tiles, from there on, and for
+    every other selection, each has its own.  Which one ran shows in the bits, and both are near the oracle."""
     kv_lens, k = [4100] + [100 + 37 * i for i in range(S - 1)], 256
     b = batch(wl, kv_lens, P, 87)
     pps, dt = -(-max(kv_lens) // P), torch.float8_e4m3fn if dtype == "e4m3" else torch.bfloat16
