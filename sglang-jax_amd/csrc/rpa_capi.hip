@@ -1386,13 +1386,15 @@ struct MlaPlan {
 // these: 9 rows of 4096 tokens 21.1 -> 23.5 us (2.2 rounds), 11 of 2048..2688 20.4 -> 22.4, 13 of 4096 23.9 -> 25.9 (3.2); around 4 rounds either, 16 of 4096 25.8 ->
 // 27.3, with fewer pages in use 23.1 -> 22.5; 24 of 4096 32.9 -> 32.9 (6), 32 40.7 -> 37.9 (8), 64 of 8192 105 -> 92.7 (32).  Throughout: e4m3 0.75 .. 1.03 x the
 // time, single tokens 0.86 .. 1.01, pages of 16 0.86 .. 1.03.
-static bool mla_takes_waves(const RpaMlaParams* p, int64_t rows, bool sparse) {
+static bool mla_takes_waves(const RpaMlaParams* p, int64_t rows, bool token_rows, bool sparse) {
   const int blocks = (p->num_q_heads + 15) / 16;
   const int64_t longest = mla_longest(p);
   const int64_t tokens = p->sum_kv_len > 0 ? std::min(p->sum_kv_len, rows * longest) : rows * longest;
   const int64_t rounds = tokens * blocks / (64 * (int64_t)mla_wgs());
   const bool fp8 = p->cache_dtype == RPA_KV_FP8_E4M3, whole = p->page_size % 32 == 0;  // (pages of whole tiles: where the other kernels are at their best)
   if (blocks == 1) return !whole || (fp8 ? rounds >= 1 || longest <= kMlaWholeRow : !sparse || rounds >= 4);
+  // (a chunk's tokens where their heads form no groups: 177 on 267 x 40 heads 26.7 -> 34.1, e4m3 on pages of 16 465 on 341 50.1 -> 69.9; 75 on 247 23.5 -> 15.6)
+  if (token_rows && rows * blocks > 2 * (int64_t)mla_wgs()) return false;
   if (longest <= kMlaWholeRow && !sparse) {
     const int eighths = blocks > 4 ? (fp8 ? 16 : 12) : blocks > 2 ? (whole ? 6 : 10) : (fp8 ? 7 : 6);
     return 8 * rows * blocks <= (int64_t)eighths * mla_wgs();
@@ -1464,7 +1466,7 @@ static MlaPlan mla_plan(const RpaMlaParams* p, int64_t rows, bool token_rows, bo
   }
   // (at most 128 heads, whatever the switch says: a share's slots in the workspace hold so many, and its line has one unit per row)
   if (waves && blocks <= 8 && tune.mla_waves != 0 && !m.token_groups && p->soft_cap == 0.f && tune.mla_shared_tiles != 0 &&
-      (tune.mla_waves > 0 || mla_takes_waves(p, rows, sparse))) {
+      (tune.mla_waves > 0 || mla_takes_waves(p, rows, token_rows, sparse))) {
     const MlaPlan other = m;
     m.waves = true;
     m.siblings = blocks;

@@ -824,6 +824,8 @@ def test_mla_chunks_of_few_tokens_run_a_wave_per_tile(pkg, monkeypatch):
             d = plan(Hq, T, 250, **kw)
             assert ("a wave per tile" in d) == waves and ("token_groups=off" in d) == waves and "pieces_per_row=1 " in d and " workspace=0" in d, (Hq, T, kw, d)
     assert "token_groups=off" not in plan(16, 300, 4000, window=1000) and "a wave per tile" in plan(16, 300, 4000)
+    for T, waves in ((170, True), (171, False)):  # heads that form no groups: up to two rounds of workgroups
+        assert ("a wave per tile" in plan(40, T, 340, fp8=True, P=16)) == waves, T
     p = _mla_params(pkg, 16, S=1, T=137, max_kv=4610, sum_kv=137 * 4542)  # rows of nearly one length: no tail in a round of its own
     assert "pieces_per_row=1 " in pkg._lib.describe_mla_plan(p, True)
     for Hq, S, longest, waves, kw in ((128, 48, 100, True, {}), (128, 49, 100, False, {}), (128, 64, 100, True, dict(fp8=True)), (128, 65, 100, False, dict(fp8=True)),
