@@ -16,6 +16,9 @@
 // Small calls are a chain: one row of 500 tokens in eight pieces, us: arguments 0.5, lengths 0.6, page ids 0.8, queries and tiles 2, a tile 1.2, the waves'
 // merge 1.7, rows out 0.8; 13.3 -> 12.0 with the launches for 16 heads, 17.6 -> 12.3 for 64, 20.4 -> 13.0 for 128.
 //
+// All 512 registers of a lane are taken.  e4m3 rows spill 18 (balanced) or 4 (fixed pieces) more, 76 or 20 bytes of scratch: what the loop over
+// tiles does not touch, written before it and read behind it.  bf16 rows spill none.
+//
 // A row of a tile has a copy instruction of its own (e4m3: two rows), so pages of any size, the row's last token in place of those past its
 // end and the new token out of the caller's rows are a matter of addresses; tiles that lie in one page have one address for all.
 
