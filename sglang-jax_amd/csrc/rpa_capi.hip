@@ -1381,11 +1381,12 @@ struct MlaPlan {
 // for 128: 128 heads, 78 rows of 67 tokens 20.7 -> 27.2 (2.4 rounds), 130 of 75 21.1 -> 44.3 (4.1), 32 heads 162 of 89 13.9 -> 20.1 (1.3).  So too for e4m3 rows of
 // a few hundred tokens on whole tiles: 82 of 777 x 64 heads 42.8 -> 47.4 (1.3 rounds), 192 of 242 x 32 heads 33.1 -> 37.4 (1.5).
 //
-// 16 heads take it always, but for bf16 selections of whole pages of whole tiles under 4 rounds: there the three tiles that a workgroup has asked for ahead
-// are 111 KB, the eight of four waves arrive behind one another's waits.  200 drawn selections, inputs that change from call to call, shared tiles ->
-// these: 9 rows of 4096 tokens 21.1 -> 23.5 us (2.2 rounds), 11 of 2048..2688 20.4 -> 22.4, 13 of 4096 23.9 -> 25.9 (3.2); around 4 rounds either, 16 of 4096 25.8 ->
-// 27.3, with fewer pages in use 23.1 -> 22.5; 24 of 4096 32.9 -> 32.9 (6), 32 40.7 -> 37.9 (8), 64 of 8192 105 -> 92.7 (32).  Throughout: e4m3 0.75 .. 1.03 x the
-// time, single tokens 0.86 .. 1.01, pages of 16 0.86 .. 1.03.
+// 16 heads take it on pages under a tile, and on whole tiles but for e4m3 rows cut into pieces under a round (above) and bf16 selections of whole pages under 4
+// rounds (bf16 rows of several lengths: see mla_plan).  Selections: the three tiles that a workgroup of the other kernel has asked for ahead are 111 KB, the
+// eight of four waves arrive behind one another's waits.  200 drawn selections, inputs that change from call to call, shared tiles -> these: 9 rows of
+// 4096 tokens 21.1 -> 23.5 us (2.2 rounds), 11 of 2048..2688 20.4 -> 22.4, 13 of 4096 23.9 -> 25.9 (3.2); around 4 rounds either, 16 of 4096 25.8 -> 27.3, with
+// fewer pages in use 23.1 -> 22.5; 24 of 4096 32.9 -> 32.9 (6), 32 40.7 -> 37.9 (8), 64 of 8192 105 -> 92.7 (32).  Throughout: e4m3 0.75 .. 1.03 x the time,
+// single tokens 0.86 .. 1.01, pages of 16 0.86 .. 1.03.
 static bool mla_takes_waves(const RpaMlaParams* p, int64_t rows, bool token_rows, bool sparse) {
   const int blocks = (p->num_q_heads + 15) / 16;
   const int64_t longest = mla_longest(p);

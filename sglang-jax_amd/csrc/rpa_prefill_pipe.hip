@@ -364,8 +364,9 @@ __device__ __forceinline__ void pipe_loop_masked(RowBlock<64> (&b)[1], const Sha
 // HD = 64: narrow heads.  With the zeros of their rows copied and multiplied, 4 chunks of 1500..2048 tokens on prefixes of up to
 // 4096, 32 / 8 heads, took 391 us, as long as heads of 128 dims but for the writes.  Half the copies and matrix instructions at two
 // workgroups per CU: 268 us; 168 registers (8 to 10 more are spilled outside the loop over tiles, 36 to 44 bytes of scratch a lane) and
-// 32 KiB of LDS leave room for a third, whose wavefronts fill what the others wait for (operands two instead of three fragments ahead): 253, 2 x 2000 tokens on 16000 832 -> 539, 3 prompts of 200..1400 34.6 -> 25.9.  What
-// bounds it now is the rate at which a CU's copies land (32 bytes per ns) and the exponentials, which are as many as of wide heads.
+// 32 KiB of LDS leave room for a third, whose wavefronts fill what the others wait for (operands two instead of three fragments ahead):
+// 253, 2 x 2000 tokens on 16000 832 -> 539, 3 prompts of 200..1400 34.6 -> 25.9.  What bounds it now is the rate at which a CU's copies
+// land (32 bytes per ns) and the exponentials, which are as many as of wide heads.
 //
 // HEADS4: the short-chunk tile.  A workgroup owns 32 query positions of FOUR query heads of a kv head, one
 // head per wave, instead of 128 positions of one head: chunks of a few dozen tokens (a verify step, a short

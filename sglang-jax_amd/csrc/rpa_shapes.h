@@ -121,7 +121,7 @@ constexpr ShapeRule kShapeRules[] = {
   {"mla_pipe", kStageMla, 0, 576, 128, 0, 128, 0, 0, kOptSoftCap | kOptAsmPages,
    kKernelMlaPipe, 1, 128, 32, 8, 8, 1, 12, "e4m3 latents (bytes staged and expanded once per tile) and RPA_MLA_WIDE=0"},
   {"mla_shared_16", kStageMla, 0, 576, 1, 16, 0, 0, 0, kOptSoftCap,
-   kKernelMlaShared, 1, 16, 32, 8, 8, 4, 8, "a tensor-parallel share of the heads: bf16 rows of several lengths, pieces over 512 tokens and up to 15 rounds; few selections of whole pages"},
+   kKernelMlaShared, 1, 16, 32, 8, 8, 4, 8, "a tensor-parallel share of the heads: bf16 rows of several lengths, pieces over 512 tokens and up to 15 rounds; few selections of whole pages; e4m3 pieces under a round"},
   {"mla_shared_32", kStageMla, 0, 576, 17, 32, 0, 0, 0, kOptSoftCap,
    kKernelMlaShared, 1, 32, 32, 8, 8, 4, 8, "144 -> 126 us"},
   {"mla_shared_64", kStageMla, 0, 576, 33, 64, 0, 0, 0, kOptSoftCap,
